@@ -1,4 +1,4 @@
-// Attention over the paged cache, general kernel: any value size up to 512, any key size up to 4096, any number
+// Attention over the paged cache, general kernel (the shapes that attention_mfma.hip and attention_f32.hip do not take): any value size up to 512, any key size up to 4096, any number
 // of heads and groups, any page size, optional window or chunks, float32 or bfloat16.
 //
 // One wave per (query token, head).  Keys are taken 64 at a time: each lane scores one
@@ -119,6 +119,13 @@ int tp_paged_attention_fast(const void* q, const void* k_cache, const void* v_ca
                             int bias_len, int keep_first, const float* sink, int value_dim, int chunk, float softcap,
                             hipStream_t s);
 
+// Defined in attention_f32.hip; -1 for shapes that are not its own.
+int tp_paged_attention_f32(const float* q, const float* k_cache, const float* v_cache, const int* block_tables, int table_width,
+                           const int* cu_seqlens, const int* context_lens, float* out, int n_tokens, int n_req, int n_heads, int n_kv,
+                           int head_dim, int value_dim, int page_size, float scale, int window, int max_q_len, int num_splits,
+                           float* scratch, const float* dist_bias, int bias_len, int keep_first, const float* sink, int chunk,
+                           float softcap, hipStream_t s);
+
 extern "C" int tp_paged_attention(const void* q, int dt, const void* k_cache, const void* v_cache,
                                   const int* block_tables, int table_width, const int* cu_seqlens,
                                   const int* context_lens, const int* token_req, void* out, int n_tokens,
@@ -157,6 +164,13 @@ extern "C" int tp_paged_attention(const void* q, int dt, const void* k_cache, co
                                            page_size, scale, window, max_q_len, num_single, num_splits, scratch, token_req,
                                            portion_splits, portion_min_steps, portion_scratch, dist_bias, bias_len, keep_first, sink, value_dim, chunk,
                                            softcap, s);
+    if (rc >= 0) return rc;
+  }
+  if (dt == TP_F32 && allow_fast) {
+    const int rc = tp_paged_attention_f32((const float*)q, (const float*)k_cache, (const float*)v_cache, block_tables, table_width,
+                                          cu_seqlens, context_lens, (float*)out, n_tokens, n_req, n_heads, n_kv, head_dim, value_dim,
+                                          page_size, scale, window, max_q_len, num_splits, scratch, dist_bias, bias_len, keep_first,
+                                          sink, chunk, softcap, s);
     if (rc >= 0) return rc;
   }
   const dim3 grid(n_tokens, n_heads);

@@ -4,7 +4,8 @@
 // plain FMA in float32 (no reduced-precision matrix mode), LDS-tiled 64x64x16 with a
 // 4x4 register block per thread.  The k loop runs in ascending order for every output
 // element, so a row's result does not depend on how many rows are in the batch.
-// bfloat16 products at model sizes go to the MFMA kernels in gemm_mfma.hip.
+// bfloat16 products at model sizes go to the MFMA kernels in gemm_mfma.hip, float32 products whose rows are whole 16-byte
+// pieces to gemm_f32.hip.
 #include "common.h"
 
 #define BM 64
@@ -146,6 +147,10 @@ int tp_linear_mfma(const void* x, const void* w, void* out, int out_dt, int accu
                    const void* post_w, void* post_xg, float* post_ss, int layout, int defer_reduce, int* splits_out,
                    GateAct gate, hipStream_t s);
 
+// Defined in gemm_f32.hip; 0 when it took the product, -1 when the rows are no whole 16-byte pieces.
+int tp_linear_f32(const float* x, const float* w, float* out, int accumulate, int M, int N, int K, float* scratch,
+                  size_t scratch_floats, hipStream_t s);
+
 int tp_linear_rope_mfma(const void* x, const void* w, int w_tiled, int M, int N, int K, const float* pre_ss, int pre_count,
                         float pre_eps, const int* positions, const int* slots, const double* inv_freq, int rotary_dim,
                         float factor, int n_heads, int n_kv, int head_dim, void* q_out, void* k_cache, void* v_cache,
@@ -246,6 +251,10 @@ extern "C" int tp_linear_fused(const void* x, const void* w, int in_dt, void* ou
   }
   TP_REQUIRE(!(layout & 4), "linear: no kernel for tiled weights at M=%d N=%d K=%d", M, N, K);
   TP_REQUIRE(!split_norm, "linear: sizes M=%d N=%d K=%d do not fit the split norm or the k-blocked layout", M, N, K);
+  if (in_dt == TP_F32 && out_dt == TP_F32 && allow_mfma) {
+    const int r = tp_linear_f32((const float*)x, (const float*)w, (float*)out, accumulate, M, N, K, scratch, scratch_floats, s);
+    if (r >= 0) return r;
+  }
   if (in_dt == TP_F32 && out_dt == TP_F32) {
     if (accumulate)
       launch_generic<float, float, true>(x, w, out, M, N, K, s);

@@ -1,0 +1,295 @@
+// Float32 products, out[M, N] (+)= x[M, K] * w[N, K]^T, every multiply-add in float32: 16-byte loads, K % 4 == 0.
+//
+// Up to 16 rows (gemm_f32_rows_kernel) the weight matrix is read once and bounds the product: a block of four waves owns a few
+// weight rows and cuts K between its waves, a lane takes four neighbouring k of every weight row at a time (a wave's load is
+// 1 KB of one row) and multiplies them with all rows of x; lanes and then waves are added in a fixed tree.  Two rows: 3,072 x 8,192 18.8 us (5.4 TB/s),
+// 16,384 x 3,072 33 us (6.1), 128,256 x 3,072 234 us (6.7).  The general kernel, which stages x through LDS between barriers and has
+// one weight element a lane in flight, takes 263, 124 (5,120 x 3,072; here 12.6) and 569 us.  At 16 rows the multiply-adds and the
+// reads of x bound it (16,384 x 3,072: 70 us), still a quarter less than the blocks of 64 rows below.
+//
+// From 17 rows on (gemm_f32_mfma_kernel) the matrix cores take float32 operands at 157 TFLOP/s, twice the rate of the vector unit
+// without packed instructions, and need one LDS read for four of them, so one pipeline of two LDS stages is enough.  611 rows:
+// 3,072 x 3,072 119 us, 16,384 x 3,072 594 us (97 and 104 TFLOP/s; the general kernel 477 and 2,060 us); 2,048 rows of the latter 1,650 us (125).
+#include "common.h"
+
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+
+// ---- up to 16 rows --------------------------------------------------------------------------------------------------------------
+// Adds v[i] over the lanes of a wave for NV values at once: each step halves the values a lane still carries, NV - 1 exchanges
+// (and single ones below NV lanes) instead of 6 NV.  The pairs added are those of an ordinary exchange tree from distance 32
+// down, so a sum's bits do not depend on NV.  The lanes with equal lane / (64 / NV) then hold the sum of value lane / (64 / NV).
+template <int N, int W>
+__device__ inline void lanes_transpose_step(float* v, int lane) {
+  if constexpr (N > 1) {
+    const bool hi = lane & W;
+#pragma unroll
+    for (int i = 0; i < N / 2; ++i) {
+      const float keep = hi ? v[i + N / 2] : v[i], send = hi ? v[i] : v[i + N / 2];
+      v[i] = keep + __shfl_xor(send, W, TP_WAVE);
+    }
+  } else {
+    v[0] += __shfl_xor(v[0], W, TP_WAVE);
+  }
+  if constexpr (W > 1) lanes_transpose_step<(N > 1 ? N / 2 : 1), W / 2>(v, lane);
+}
+template <int NV>
+__device__ inline float lanes_transpose_sum(float (&v)[NV], int lane) {
+  lanes_transpose_step<NV, TP_WAVE / 2>(v, lane);
+  return v[0];
+}
+
+#define FR_WAVES 4
+
+// MC: rows of the block's registers (M <= MC), C: weight rows a block owns.
+template <int MC, int C, bool ACC>
+__global__ __launch_bounds__(256) void gemm_f32_rows_kernel(const float* __restrict__ x, const float* __restrict__ w,
+                                                            float* __restrict__ out, int M, int N, int K) {
+  __shared__ float part[FR_WAVES][MC * C];
+  const int lane = threadIdx.x % TP_WAVE, wave = threadIdx.x / TP_WAVE;
+  const int n0 = blockIdx.x * C;
+  // K in steps of 256 (a wave's load); the steps are dealt to the waves in runs
+  const int steps = (K + 255) / 256, per = (steps + FR_WAVES - 1) / FR_WAVES;
+  const int s0 = wave * per, s1 = min(steps, s0 + per);
+  float acc[C * MC];
+#pragma unroll
+  for (int i = 0; i < C * MC; ++i) acc[i] = 0.f;
+  const float* wr[C];
+#pragma unroll
+  for (int c = 0; c < C; ++c) wr[c] = w + (size_t)min(n0 + c, N - 1) * K;
+  f32x4 nw[C];
+  auto fetch = [&](int s) {
+    const int k = s * 256 + lane * 4;
+    const bool in = s < s1 && k < K;
+#pragma unroll
+    for (int c = 0; c < C; ++c) nw[c] = in ? __builtin_nontemporal_load((const f32x4*)(wr[c] + k)) : (f32x4)(0.f);
+  };
+  fetch(s0);
+  for (int s = s0; s < s1; ++s) {
+    f32x4 cw[C];
+#pragma unroll
+    for (int c = 0; c < C; ++c) cw[c] = nw[c];
+    fetch(s + 1);
+    const int k = s * 256 + lane * 4;
+    if (k < K) {
+#pragma unroll
+      for (int m = 0; m < MC; ++m) {
+        const f32x4 xv = *(const f32x4*)(x + (size_t)min(m, M - 1) * K + k);
+#pragma unroll
+        for (int c = 0; c < C; ++c)
+#pragma unroll
+          for (int j = 0; j < 4; ++j) acc[c * MC + m] = fmaf(cw[c][j], xv[j], acc[c * MC + m]);
+      }
+    }
+  }
+  constexpr int NV = C * MC > 64 ? 64 : C * MC;
+#pragma unroll
+  for (int g = 0; g < C * MC / NV; ++g) {
+    float v[NV];
+#pragma unroll
+    for (int i = 0; i < NV; ++i) v[i] = acc[g * NV + i];
+    const float t = lanes_transpose_sum<NV>(v, lane);
+    if (lane % (TP_WAVE / NV) == 0) part[wave][g * NV + lane / (TP_WAVE / NV)] = t;
+  }
+  __syncthreads();
+  for (int i = threadIdx.x; i < C * MC; i += 256) {
+    const int c = i % C, m = i / C, n = n0 + c;
+    if (m >= M || n >= N) continue;
+    float t = part[0][c * MC + m];
+#pragma unroll
+    for (int v = 1; v < FR_WAVES; ++v) t += part[v][c * MC + m];
+    float* o = out + (size_t)m * N + n;
+    *o = ACC ? *o + t : t;
+  }
+}
+
+// ---- from 17 rows on --------------------------------------------------------------------------------------------------------------
+#define FM_K 32           // K of a stage
+#define FM_LD (FM_K + 4)  // floats of a row in LDS: rows four banks apart, so that eight lanes' 16-byte reads cover all banks
+
+// A block of T x T results, four waves of T/2 x T/2.  v_mfma_f32_32x32x2_f32 takes k = 0 from lanes 0..31 and k = 1 from lanes
+// 32..63; a lane reads four neighbouring k at once and feeds them to four instructions, so instruction j of a run of eight k
+// multiplies k = j and k = 4 + j.
+// splits > 1: blockIdx.y takes a run of K's stages and writes its sums to part [splits, M, N].
+template <int T, bool ACC>
+__global__ __launch_bounds__(256, 2) void gemm_f32_mfma_kernel(const float* __restrict__ x, const float* __restrict__ w,
+                                                            float* __restrict__ out, float* __restrict__ part, int M, int N, int K,
+                                                            int row_tiles, int tiles) {
+  constexpr int W = T / 2, R = W / 32;                 // a wave's side, 32 x 32 tiles a side
+  constexpr int LOADS = T * FM_K / 4 / 256;            // 16-byte loads a thread and operand
+  __shared__ float xs[2][T * FM_LD], ws[2][T * FM_LD];
+  // XCD j (blocks go to the XCDs in turn) takes the j-th eighth of the tiles, row tiles fastest: the blocks that share weight
+  // rows then share an L2
+  const int per = (tiles + 7) / 8;
+  const int tile = (blockIdx.x % 8) * per + blockIdx.x / 8;
+  if ((int)(blockIdx.x / 8) >= per || tile >= tiles) return;
+  const int m0 = tile % row_tiles * T, n0 = tile / row_tiles * T;
+  const int tid = threadIdx.x, lane = tid % TP_WAVE, wave = tid / TP_WAVE;
+  const int wm = wave / 2 * W, wn = wave % 2 * W;
+  const int stages = (K + FM_K - 1) / FM_K, sper = (stages + gridDim.y - 1) / gridDim.y;
+  const int s0 = blockIdx.y * sper, s1 = min(stages, s0 + sper);
+
+  const int lr = tid / 8, lk = tid % 8 * 4;            // loader: 32 rows a pass, eight threads a row
+  f32x4 gx[LOADS], gw[LOADS];
+  auto fetch = [&](int s) {
+    const int k = s * FM_K + lk;
+    const bool in = k < K;
+#pragma unroll
+    for (int i = 0; i < LOADS; ++i) {
+      const int r = lr + 32 * i;
+      gx[i] = in ? *(const f32x4*)(x + (size_t)min(m0 + r, M - 1) * K + k) : (f32x4)(0.f);
+      gw[i] = in ? *(const f32x4*)(w + (size_t)min(n0 + r, N - 1) * K + k) : (f32x4)(0.f);
+    }
+  };
+  auto stage = [&](int b) {
+#pragma unroll
+    for (int i = 0; i < LOADS; ++i) {
+      *(f32x4*)&xs[b][(lr + 32 * i) * FM_LD + lk] = gx[i];
+      *(f32x4*)&ws[b][(lr + 32 * i) * FM_LD + lk] = gw[i];
+    }
+  };
+  // (two sums a result, over alternate runs of eight k: shorter chains of roundings than one sum in ascending order)
+  f32x16 acc[2][R][R];
+#pragma unroll
+  for (int i = 0; i < R; ++i)
+#pragma unroll
+    for (int j = 0; j < R; ++j) acc[0][i][j] = acc[1][i][j] = (f32x16)(0.f);
+  if (s0 < s1) {
+    fetch(s0);
+    stage(0);
+  }
+  __syncthreads();
+  for (int s = s0; s < s1; ++s) {
+    const int b = (s - s0) & 1;
+    if (s + 1 < s1) fetch(s + 1);
+#pragma unroll
+    for (int kk = 0; kk < FM_K; kk += 8) {
+      f32x4 a[R], c[R];
+      const int k = kk + lane / 32 * 4;
+#pragma unroll
+      for (int i = 0; i < R; ++i) {
+        a[i] = *(const f32x4*)&xs[b][(wm + i * 32 + lane % 32) * FM_LD + k];
+        c[i] = *(const f32x4*)&ws[b][(wn + i * 32 + lane % 32) * FM_LD + k];
+      }
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+#pragma unroll
+        for (int i = 0; i < R; ++i)
+#pragma unroll
+          for (int j = 0; j < R; ++j)
+            acc[kk / 8 % 2][i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[i][q], c[j][q], acc[kk / 8 % 2][i][j], 0, 0, 0);
+    }
+    if (s + 1 < s1) stage(b ^ 1);
+    __syncthreads();
+  }
+  // a lane holds column lane % 32 and rows 8 (e / 4) + 4 (lane / 32) + e % 4 of a 32 x 32 tile
+  const bool partial = gridDim.y > 1;
+  float* o0 = partial ? part + (size_t)blockIdx.y * M * N : out;
+#pragma unroll
+  for (int i = 0; i < R; ++i)
+#pragma unroll
+    for (int j = 0; j < R; ++j) {
+      const int n = n0 + wn + j * 32 + lane % 32;
+      const f32x16 sum = acc[0][i][j] + acc[1][i][j];
+#pragma unroll
+      for (int e = 0; e < 16; ++e) {
+        const int m = m0 + wm + i * 32 + 8 * (e / 4) + 4 * (lane / 32) + e % 4;
+        if (m < M && n < N) {
+          float* o = o0 + (size_t)m * N + n;
+          *o = ACC && !partial ? *o + sum[e] : sum[e];
+        }
+      }
+    }
+}
+
+// out (+)= the parts in ascending order.
+template <bool ACC>
+__global__ __launch_bounds__(256) void gemm_f32_parts_kernel(const float* __restrict__ part, float* __restrict__ out, size_t count, int splits) {
+  const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
+  if (i >= count) return;
+  float t = part[i];
+  for (int s = 1; s < splits; ++s) t += part[(size_t)s * count + i];
+  out[i] = ACC ? out[i] + t : t;
+}
+
+template <int MC, int C>
+static void launch_rows(const float* x, const float* w, float* out, bool acc, int M, int N, int K, hipStream_t s) {
+  const dim3 grid((N + C - 1) / C);
+  if (acc)
+    hipLaunchKernelGGL((gemm_f32_rows_kernel<MC, C, true>), grid, dim3(256), 0, s, x, w, out, M, N, K);
+  else
+    hipLaunchKernelGGL((gemm_f32_rows_kernel<MC, C, false>), grid, dim3(256), 0, s, x, w, out, M, N, K);
+}
+
+template <int T>
+static void launch_mfma(const float* x, const float* w, float* out, float* part, bool acc, int M, int N, int K, int splits, hipStream_t s) {
+  const int row_tiles = (M + T - 1) / T, tiles = row_tiles * ((N + T - 1) / T);
+  const dim3 grid((tiles + 7) / 8 * 8, splits);
+  if (acc)
+    hipLaunchKernelGGL((gemm_f32_mfma_kernel<T, true>), grid, dim3(256), 0, s, x, w, out, part, M, N, K, row_tiles, tiles);
+  else
+    hipLaunchKernelGGL((gemm_f32_mfma_kernel<T, false>), grid, dim3(256), 0, s, x, w, out, part, M, N, K, row_tiles, tiles);
+}
+
+// How the product of more than 16 rows is cut: blocks of 128 or 64 a side, K in up to eight parts.  The matrix cores bound it, so
+// the time is the work of the fullest CU: rounds of 256 blocks times a block's results and its share of K; every part costs 3 % for
+// writing and adding its sums and keeps 256 of K.  The parts, which a result's bits depend on, are chosen for rows counted in
+// blocks of 128 (up to 64: 64), so that a step whose rows are padded to the next power of two, or multiple of 128, is cut alike;
+// the block (which they do not depend on) for the rows there are.  3,072 x 3,072 at 64 rows in 1 / 4 / 5 parts: 41 / 25.7 / 23 us;
+// 16,384 x 3,072 at 2,048 rows in blocks of 128 / 64: 1,650 / 1,790 us, 3,072 x 3,072 there 429 / 359 us (one and a half rounds of
+// the large blocks).
+static void f32_plan(int M, int N, int K, bool parts_ok, int* tile, int* splits) {
+  const long rows = M <= 64 ? 64 : (long)(M + 127) / 128 * 128, cols = (N + 63) / 64;
+  *splits = 1;
+  double best = 1e30;
+  for (int p = 1; p <= (parts_ok ? 8 : 1) && (p == 1 || K / p >= 256); ++p) {
+    const double cost = (double)((rows / 64 * cols * p + 255) / 256) / p * (1.0 + 0.03 * (p - 1));
+    if (cost < best) best = cost, *splits = p;
+  }
+  const long t128 = (long)(M + 127) / 128 * ((N + 127) / 128) * *splits, t64 = (long)(M + 63) / 64 * cols * *splits;
+  *tile = 4.0 * ((t128 + 255) / 256) <= 1.08 * ((t64 + 255) / 256) ? 128 : 64;
+}
+
+// Floats of scratch that the product uses for parts of K (0: none).
+extern "C" size_t tp_linear_f32_scratch(int M, int N, int K) {
+  if (M <= 16 || N <= 0 || K <= 0) return 0;
+  int tile, splits;
+  f32_plan(M, N, K, true, &tile, &splits);
+  return splits > 1 ? (size_t)splits * M * N : 0;
+}
+
+// Takes a product whose rows are whole 16-byte pieces (K % 4 == 0, aligned operands); -1: not its own, the general kernel runs.
+int tp_linear_f32(const float* x, const float* w, float* out, int accumulate, int M, int N, int K, float* scratch,
+                  size_t scratch_floats, hipStream_t s) {
+  if (K % 4 != 0 || ((uintptr_t)x | (uintptr_t)w) % 16 != 0) return -1;
+  const bool acc = accumulate != 0;
+  if (M == 1)
+    launch_rows<1, 4>(x, w, out, acc, M, N, K, s);
+  else if (M == 2)
+    launch_rows<2, 4>(x, w, out, acc, M, N, K, s);
+  else if (M <= 4)
+    launch_rows<4, 4>(x, w, out, acc, M, N, K, s);
+  else if (M <= 8)
+    launch_rows<8, 4>(x, w, out, acc, M, N, K, s);
+  else if (M <= 16)
+    launch_rows<16, 4>(x, w, out, acc, M, N, K, s);
+  else {
+    int tile, splits;
+    f32_plan(M, N, K, true, &tile, &splits);
+    if (splits > 1 && (scratch == nullptr || scratch_floats < (size_t)splits * M * N)) f32_plan(M, N, K, false, &tile, &splits);
+    if (tile == 128)
+      launch_mfma<128>(x, w, out, scratch, acc, M, N, K, splits, s);
+    else
+      launch_mfma<64>(x, w, out, scratch, acc, M, N, K, splits, s);
+    if (splits > 1) {
+      const size_t count = (size_t)M * N;
+      const dim3 grid((unsigned)((count + 255) / 256));
+      if (acc)
+        hipLaunchKernelGGL((gemm_f32_parts_kernel<true>), grid, dim3(256), 0, s, scratch, out, count, splits);
+      else
+        hipLaunchKernelGGL((gemm_f32_parts_kernel<false>), grid, dim3(256), 0, s, scratch, out, count, splits);
+    }
+  }
+  TP_CHECK_LAUNCH("linear (float32)");
+  return 0;
+}

@@ -48,6 +48,7 @@ class _Library:
             except OSError as e:
                 raise KernelError(f"cannot load the kernel library {path}: {e}") from e
             lib.tp_last_error.restype = ctypes.c_char_p
+            lib.tp_linear_f32_scratch.restype = ctypes.c_size_t
             cls._lib = lib
             cls.path = path
         return cls._lib
@@ -693,9 +694,12 @@ def linear(x, w: torch.Tensor, out_dtype: torch.dtype, residual: Optional[torch.
         if hand_blocked:
             layout |= 8
     scratch, nscratch = _splitk_scratch(x, m, n) if allow_mfma else (None, 0)
+    if allow_mfma and x.dtype == torch.float32 and m > 16:      # (parts of K where a float32 product has few result tiles)
+        nscratch = int(library().tp_linear_f32_scratch(m, n, k))
+        scratch = torch.empty((nscratch,), dtype=torch.float32, device=x.device) if nscratch else None
     # from 17 rows on: the partial sums of a split K may stay unadded for the kernel that consumes the rows
     layout |= wl
-    defer = scratch is not None and 16 < m and (layout & 3) == 0 and \
+    defer = scratch is not None and x.dtype == torch.bfloat16 and 16 < m and (layout & 3) == 0 and \
         ((next_norm is not None and residual is not None and split_norm_ok(m, n, x.dtype) and n % 4 == 0 and n <= 16384) or
          (partial_ok and residual is None and out_dtype == torch.float32))
     splits = ctypes.c_int(1)
@@ -988,6 +992,16 @@ def paged_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tenso
         splits = max(1, min(64, want, bound // 128))
         if splits > 1:
             scratch = torch.empty((r * heads * splits * (vd + 2),), dtype=torch.float32, device=q.device)
+    fast_f32 = allow_fast_attention and q.dtype == torch.float32 and d == vd and d in (32, 64, 96, 128) and page_size % 16 == 0
+    if fast_f32 and max_q_len == 1 and n == r:
+        # (float32: at least 128 keys a block of four waves, by the same bound on the context as above, until there are
+        # two blocks a CU)
+        bound = 256
+        while bound < max_context_len:
+            bound *= 2
+        splits = max(1, min(64, bound // 128, 512 // (decode_rows_padded(r) * kvh)))
+        if splits > 1:
+            scratch = torch.empty((r * heads * splits * (vd + 2),), dtype=torch.float32, device=q.device)
     parts, part_scratch = 1, None
     # (the kernel with a distance bias does not split a portion's keys)
     if fast and dist_bias is None and not keep_first and num_single < r and d in (32, 64, 128, 192) and (d + vd) % 64 == 0 and page_size & (page_size - 1) == 0 and page_size >= max(8, 512 // d):
@@ -1004,7 +1018,7 @@ def paged_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tenso
             part_scratch = torch.empty((n * heads * parts * (vd + 4),), dtype=torch.float32, device=q.device)
     _call("tp_paged_attention", _ptr(q), _dt(q), _ptr(k_cache), _ptr(v_cache), _ptr(block_tables), width,
           _ptr(cu_seqlens), _ptr(context_lens), _ptr(token_req), _ptr(out), n, r, heads, kvh, d, page_size,
-          ctypes.c_float(scale), int(window), int(max_q_len), int(max_context_len), int(fast),
+          ctypes.c_float(scale), int(window), int(max_q_len), int(max_context_len), int(fast or fast_f32),
           int(num_single), int(splits), _ptr(scratch), int(parts), max(1, portion_min_keys // 32), _ptr(part_scratch),
           _ptr(dist_bias), 0 if dist_bias is None else dist_bias.shape[1], int(vd), int(keep_first), _ptr(sink), int(chunk),
           ctypes.c_float(softcap), _stream())

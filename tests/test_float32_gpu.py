@@ -1,0 +1,118 @@
+"""The float32 products and the float32 attention on the matrix cores against float64 and against the general kernels."""
+import math
+
+import pytest
+import torch
+
+from emu_ops import EmuOps
+
+pytestmark = pytest.mark.gpu
+emu = EmuOps()
+DEV = "cuda:0"
+
+
+def _rel(got, ref):
+    got, ref = got.double().cpu(), ref.double().cpu()
+    return float((got - ref).norm() / ref.norm())
+
+
+# rows: the edges of the few-row kernels (1, 2, 4, 8, 16) and of the 64- and 128-row blocks; K: no whole 256, 32 or 8; N: no whole
+# block, and few enough columns that K is cut into parts
+@pytest.mark.parametrize("m,n,k", [(1, 5, 4), (2, 130, 1028), (3, 64, 260), (5, 67, 2052), (9, 12, 96), (16, 1030, 516), (17, 100, 36),
+                                   (40, 200, 4100), (64, 384, 96), (65, 130, 2048), (129, 257, 132), (300, 1000, 68), (611, 3072, 256)])
+def test_float32_products(m, n, k):
+    """Against float64: a sum of k products, each rounded once and added in float32, is off by at most about k / 2 units of 2^-24 of
+    the sum of magnitudes, and by the root of that in the mean: 2^-24 sqrt(k) of the norm is four times what is seen."""
+    from tempura_amd.kernels import ops
+    g = torch.Generator().manual_seed(m + n + k)
+    x, w, res = torch.randn(m, k, generator=g), torch.randn(n, k, generator=g), torch.randn(m, n, generator=g)
+    ref = x.double() @ w.double().T
+    xd, wd = x.to(DEV), w.to(DEV)
+    got = ops.linear(xd, wd, torch.float32)
+    tol = 2.0 ** -24 * max(2.0, math.sqrt(k))
+    assert _rel(got, ref) < tol
+    assert _rel(ops.linear(xd, wd, torch.float32, residual=res.to(DEV)), ref + res.double()) < tol + 2.0 ** -23
+    assert torch.equal(got, ops.linear(xd, wd, torch.float32))
+    ops.allow_mfma = False
+    try:
+        general = ops.linear(xd, wd, torch.float32)
+    finally:
+        ops.allow_mfma = True
+    assert _rel(got, ref) <= max(_rel(general, ref), 2.0 ** -24 * 2)
+    # a row's bits do not depend on the rows beside it, up to 16 rows
+    if m <= 16:
+        assert torch.equal(ops.linear(xd[: m // 2 + 1].contiguous(), wd, torch.float32), got[: m // 2 + 1])
+    # rows that are no whole 16-byte pieces (an odd K, an operand that starts off such a place) run the general kernel
+    flat = torch.zeros(m * k + 1, device=DEV)
+    off = flat[1:].view(m, k).copy_(xd)
+    assert off.data_ptr() % 16 != 0 and _rel(ops.linear(off, wd, torch.float32), ref) < tol
+
+
+@pytest.mark.parametrize("what", ["plain", "window", "kept", "chunk", "cap", "bias", "sink"])
+@pytest.mark.parametrize("heads,kv,d,page,q_lens,ctx_lens", [
+    (6, 2, 64, 16, [37, 1, 20], [37, 90, 200]),                    # portions beside a single token
+    (4, 4, 32, 32, [1, 1, 1], [1, 16, 17]),                        # single tokens at the edges of a tile
+    (24, 8, 128, 16, [1, 1], [700, 300]),                          # keys split over blocks
+    (3, 1, 96, 48, [5], [260]),
+])
+def test_float32_attention(heads, kv, d, page, q_lens, ctx_lens, what):
+    """Every form against float64 (2e-6: sums of a few hundred float32 terms) and against the general kernel; every cache place that
+    holds no key of its request is NaN."""
+    from tempura_amd.kernels import ops
+    g = torch.Generator().manual_seed(heads * 1000 + d)
+    R, n = len(q_lens), sum(q_lens)
+    pages = sum((c + page - 1) // page for c in ctx_lens) + 2
+    perm = torch.randperm(pages, generator=g).tolist()
+    width = max((c + page - 1) // page for c in ctx_lens) + 1
+    bt = torch.full((R, width), perm[-1], dtype=torch.int32)
+    it = iter(perm)
+    used = torch.zeros(pages, page, dtype=torch.bool)
+    for r, c in enumerate(ctx_lens):
+        for i in range((c + page - 1) // page):
+            bt[r, i] = next(it)
+        for i in range(c):
+            used[bt[r, i // page], i % page] = True
+    kc, vc = torch.randn(pages, kv, page, d, generator=g) * 1.5, torch.randn(pages, kv, d, page, generator=g)
+    q = torch.randn(n, heads, d, generator=g) * 1.5
+    cu = torch.tensor([0] + list(torch.tensor(q_lens).cumsum(0)), dtype=torch.int32)
+    cl, tr = torch.tensor(ctx_lens, dtype=torch.int32), torch.repeat_interleave(torch.arange(R, dtype=torch.int32), torch.tensor(q_lens))
+    scale, window, more = d ** -0.5, 0, {}
+    if what == "window":
+        window = 19
+    elif what == "kept":
+        window, more = 33, {"keep_first": 21}
+    elif what == "chunk":
+        more = {"chunk": 50}
+    elif what == "cap":
+        more = {"softcap": 3.0}
+    elif what == "bias":
+        more = {"dist_bias": torch.randn(heads, 40, generator=g)}
+    elif what == "sink":
+        more = {"sink": torch.randn(heads, generator=g) * 3}
+    ref = emu.paged_attention(q.double(), kc.double(), vc.double(), bt, cu, cl, tr, scale, window, max(q_lens), max(ctx_lens),
+                              **{a: b.double() if torch.is_tensor(b) else b for a, b in more.items()})
+    bad = ~used[:, None, :].expand(pages, kv, page)
+    kc, vc = kc.clone(), vc.clone()
+    kc[bad] = float("nan")
+    vc.transpose(2, 3)[bad] = float("nan")
+    more = {a: b.to(DEV) if torch.is_tensor(b) else b for a, b in more.items()}
+
+    def run(values):
+        return ops.paged_attention(q.to(DEV), kc.to(DEV), values.to(DEV), bt.to(DEV), cu.to(DEV), cl.to(DEV), tr.to(DEV), scale, window,
+                                   max(q_lens), max(ctx_lens), **more)
+    got = run(vc)
+    assert _rel(got, ref) < 2e-6
+    ops.allow_fast_attention = False
+    try:
+        general = run(vc)
+    finally:
+        ops.allow_fast_attention = True
+    assert _rel(got, ref) <= max(2.0 * _rel(general, ref), 3e-7)
+    # a last key whose values are infinite is its own token's matter: rows in front of it keep their bits
+    if q_lens[0] > 1 and what == "plain":
+        inf = vc.clone()
+        last = ctx_lens[0] - 1
+        inf[bt[0, last // page], :, :, last % page] = float("inf")
+        other = run(inf)
+        assert torch.equal(other[: q_lens[0] - 1], got[: q_lens[0] - 1])
+        assert not torch.isfinite(other[q_lens[0] - 1]).any()

@@ -54,6 +54,14 @@ __device__ inline void from_float4(bf16_t* p, float a, float b, float c, float d
   *(uint2*)p = u;
 }
 
+// four neighbouring elements as one load (p aligned to four elements)
+__device__ inline float4 load_float4(const float* p) { return *(const float4*)p; }
+__device__ inline float4 load_float4(const bf16_t* p) {
+  const uint2 u = *(const uint2*)p;
+  return make_float4(bf16_to_float(bf16_t{(uint16_t)(u.x & 0xffff)}), bf16_to_float(bf16_t{(uint16_t)(u.x >> 16)}),
+                     bf16_to_float(bf16_t{(uint16_t)(u.y & 0xffff)}), bf16_to_float(bf16_t{(uint16_t)(u.y >> 16)}));
+}
+
 // cosine and sine (times factor) of pos * inv_freq: the product in float64, reduced to [0, 2 pi) there,
 // sine and cosine of the small rest in float32 (every kernel that rotates uses this one routine)
 __device__ inline void rope_cos_sin(int pos, double inv_freq, float factor, float& c, float& sn) {

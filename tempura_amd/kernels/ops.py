@@ -286,13 +286,13 @@ def qk_store(rows: torch.Tensor, q_bias: Optional[torch.Tensor], k_bias: Optiona
 
 def causal_conv(proj: torch.Tensor, col0: int, channels: int, weight: torch.Tensor, bias: Optional[torch.Tensor], state: torch.Tensor,
                 cu_seqlens: torch.Tensor, token_req: torch.Tensor, state_slots: torch.Tensor, num_requests: int,
-                state_off: int = 0, act: bool = True) -> torch.Tensor:
+                state_off: int = 0, act: bool = True, max_run: int = 0) -> torch.Tensor:
     """Causal convolution per channel over each request's run of tokens, then SiLU (``act`` False: the sums
     themselves).  ``proj`` float32 [n, width] holds the inputs at columns col0 .. col0 + channels; ``weight``
     [taps, channels] (tap-major; the last tap is the current token's), ``bias`` [channels] or None; ``state`` float32
     [slots, row] whose rows hold, from element ``state_off`` on, the carried inputs [taps - 1, channels] (oldest
     first) of the request in that slot: they are read for the first tokens of a run and replaced by the run's last
-    inputs.  Returns float32 [n, channels]."""
+    inputs.  ``max_run``: the longest run (0: not known); runs of one token are one launch.  Returns float32 [n, channels]."""
     if _backend is not None:
         if state_off == 0 and act and bias is not None:
             return _backend.causal_conv(proj, col0, channels, weight, bias, state, cu_seqlens, token_req, state_slots, num_requests)
@@ -312,7 +312,7 @@ def causal_conv(proj: torch.Tensor, col0: int, channels: int, weight: torch.Tens
     out = torch.empty((n, channels), dtype=torch.float32, device=proj.device)
     _call("tp_causal_conv", _ptr(proj), proj.shape[1], int(col0), _ptr(weight), _ptr(bias), _ptr(state),
           ctypes.c_size_t(state.shape[1]), ctypes.c_size_t(state_off), _ptr(cu_seqlens), _ptr(token_req), _ptr(state_slots), _ptr(out),
-          n, int(num_requests), channels, taps, int(bool(act)), _stream())
+          n, int(num_requests), channels, taps, int(bool(act)), int(max_run), _stream())
     return out
 
 
@@ -1779,11 +1779,12 @@ def rmsnorm_cols(x: torch.Tensor, col0: int, width: int, weight: torch.Tensor, e
 
 
 def residual_conv(x: torch.Tensor, weight: torch.Tensor, state: torch.Tensor, state_off: int, cu_seqlens: torch.Tensor,
-                  token_req: torch.Tensor, state_slots: torch.Tensor, num_requests: int, out_dtype: torch.dtype):
+                  token_req: torch.Tensor, state_slots: torch.Tensor, num_requests: int, out_dtype: torch.dtype, max_run: int = 0):
     """What sublayers read of rows ``x`` (float32 [n, width]): for each of the ``weight`` [subs, taps, width] (tap-major,
     the last tap the current token's) x + conv(x) over each request's run of tokens, as ``out_dtype``; a list of
     ``subs`` tensors [n, width].  ``state`` float32 [slots, row]: from element ``state_off`` on a request's carried
-    rows [taps - 1, width] (oldest first), read for the first tokens of a run and replaced by the run's last rows."""
+    rows [taps - 1, width] (oldest first), read for the first tokens of a run and replaced by the run's last rows.  ``max_run``: the longest run
+    (0: not known); runs of one token are one launch."""
     if _backend is not None:
         return _backend.residual_conv(x, weight, state, state_off, cu_seqlens, token_req, state_slots, num_requests, out_dtype)
     _dev_ok(x, weight, state, cu_seqlens, token_req, state_slots)
@@ -1800,7 +1801,7 @@ def residual_conv(x: torch.Tensor, weight: torch.Tensor, state: torch.Tensor, st
     out = torch.empty((subs, n, width), dtype=out_dtype, device=x.device)
     _call("tp_residual_conv", _ptr(x), _ptr(weight), _ptr(state), ctypes.c_size_t(0 if state is None else state.shape[1]), ctypes.c_size_t(state_off),
           _ptr(cu_seqlens), _ptr(token_req), _ptr(state_slots), _ptr(out), _dtcode(out_dtype), n, int(num_requests), width, taps, subs,
-          _stream())
+          int(max_run), _stream())
     return [out[i] for i in range(subs)]
 
 

@@ -518,7 +518,7 @@ class ConvAttention(BranchMixer):
         if self.taps:
             qkv_col0 = 0
             qkv = ops.causal_conv(proj, col0, self.channels, self.conv_w, None, cache.state, ctx.cu_seqlens, ctx.token_req,
-                                  ctx.state_slots, ctx.num_requests, state_off=self.state_off, act=False)
+                                  ctx.state_slots, ctx.num_requests, state_off=self.state_off, act=False, max_run=ctx.max_q_len)
         rot = self.position.rotary()
         inv_freq, rotary_dim, factor, table = None, 0, 1.0, None
         if rot is not None:

@@ -87,7 +87,7 @@ class GatedDeltaMixer(BranchMixer):
 
     def run(self, proj, col0, ctx, cache, out, out_col0, scale):
         qkv = ops.causal_conv(proj, col0, self.channels, self.conv_w, None, cache.state, ctx.cu_seqlens, ctx.token_req,
-                              ctx.state_slots, ctx.num_requests, state_off=self.state_off, act=True)
+                              ctx.state_slots, ctx.num_requests, state_off=self.state_off, act=True, max_run=ctx.max_q_len)
         decay = ops.lowrank_up(proj, col0 + self.a1_col, self.a2_t, "decay", self.a_log, self.dt_bias, self.head_dim)
         gate = ops.lowrank_up(proj, col0 + self.g1_col, self.g2_t, "sigmoid")
         o = ops.delta_scan(qkv, decay, proj, col0 + self.beta_col, cache.state, self.state_off + self.conv_floats, ctx.cu_seqlens,

@@ -45,7 +45,7 @@ class ResidualConv(Part):
     def forward(self, n, ctx, cache):
         """float32 rows [tokens, hidden] -> a list of compute-dtype rows, one per sublayer."""
         return ops.residual_conv(n, self.weight, cache.state, self.state_off, ctx.cu_seqlens, ctx.token_req, ctx.state_slots,
-                                 ctx.num_requests, self.dtype)
+                                 ctx.num_requests, self.dtype, max_run=ctx.max_q_len)
 
 
 register_part("input", "residual_conv", ResidualConv)

@@ -84,7 +84,7 @@ class Mamba2Mixer(Mixer):
     def forward(self, x, ctx, cache, residual=None):
         proj = ops.linear(x, self.w_in, torch.float32)                  # [n, z | x | B | C | dt (| padding)]
         xbc = ops.causal_conv(proj, self.inner, self.channels, self.conv_w, self.conv_b, cache.state, ctx.cu_seqlens,
-                              ctx.token_req, ctx.state_slots, ctx.num_requests)
+                              ctx.token_req, ctx.state_slots, ctx.num_requests, max_run=ctx.max_q_len)
         y = ops.ssm_scan(xbc, proj, self.inner + self.channels, self.dt_bias, self.a_log, self.d_skip, cache.state,
                          self.conv_state, ctx.cu_seqlens, ctx.state_slots, ctx.num_requests, self.num_heads, self.head_dim,
                          self.state_size, self.groups, max_run=ctx.max_q_len)

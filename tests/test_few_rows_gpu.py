@@ -1,0 +1,143 @@
+"""Row kernels that read their rows once in 16-byte pieces, against the plain operations and against the kernels that take any size
+and place (reached by columns that start off a 16-byte place); single-token steps against the general ones."""
+import pytest
+import torch
+
+from emu_ops import EmuOps
+
+pytestmark = pytest.mark.gpu
+emu = EmuOps()
+DEV = "cuda:0"
+
+
+def _close(got, ref, tol):
+    got, ref = got.double().cpu(), ref.double().cpu()
+    assert float((got - ref).abs().max()) <= tol * float(ref.abs().max())
+
+
+def _runs(lens, g):
+    cu = torch.tensor([0] + list(torch.tensor(lens).cumsum(0)), dtype=torch.int32)
+    req = torch.repeat_interleave(torch.arange(len(lens), dtype=torch.int32), torch.tensor(lens))
+    slots = torch.randperm(len(lens) + 2, generator=g)[: len(lens)].to(torch.int32)
+    return cu.to(DEV), req.to(DEV), slots.to(DEV)
+
+
+@pytest.mark.parametrize("channels,taps", [(4, 2), (1024, 4), (2052, 3), (6144, 4)])
+@pytest.mark.parametrize("lens", [[1, 1, 1], [70], [1, 2, 3, 60, 1, 17], [8, 56, 64]])
+def test_causal_conv_paths_agree(channels, taps, lens):
+    """Every path forms a channel's sum in the same order: the same bits, outputs and states alike."""
+    from tempura_amd.kernels import ops
+    g = torch.Generator().manual_seed(channels + len(lens))
+    n = sum(lens)
+    proj = torch.randn(n, channels + 8, generator=g).to(DEV)
+    off = torch.cat([torch.zeros(n, 1, device=DEV), proj], dim=1).contiguous()         # rows off the 16-byte places
+    w, b = torch.randn(taps, channels, generator=g).to(DEV), torch.randn(channels, generator=g).to(DEV)
+    cu, req, slots = _runs(lens, g)
+    state = torch.randn(len(lens) + 2, 5 + (taps - 1) * channels, generator=g).to(DEV)
+    for act in (True, False):
+        s0, s1, s2 = state.clone(), state.clone(), state.clone()
+        want = ops.causal_conv(off, 5, channels, w, b, s0, cu, req, slots, len(lens), 5, act)
+        got = ops.causal_conv(proj, 4, channels, w, b, s1, cu, req, slots, len(lens), 5, act)
+        assert torch.equal(got, want) and torch.equal(s1, s0)
+        got = ops.causal_conv(proj, 4, channels, w, b, s2, cu, req, slots, len(lens), 5, act, max_run=max(lens))
+        assert torch.equal(got, want) and torch.equal(s2, s0)
+
+
+@pytest.mark.parametrize("width,subs,taps", [(8, 1, 2), (1024, 2, 4), (4100, 3, 3)])
+def test_residual_conv_of_single_tokens(width, subs, taps):
+    from tempura_amd.kernels import ops
+    g = torch.Generator().manual_seed(width)
+    lens = [1, 1, 1, 1]
+    cu, req, slots = _runs(lens, g)
+    x, w = torch.randn(4, width, generator=g).to(DEV), torch.randn(subs, taps, width, generator=g).to(DEV)
+    state = torch.randn(6, 3 + (taps - 1) * width, generator=g).to(DEV)
+    s0, s1 = state.clone(), state.clone()
+    want = ops.residual_conv(x, w, s0, 3, cu, req, slots, 4, torch.bfloat16)
+    got = ops.residual_conv(x, w, s1, 3, cu, req, slots, 4, torch.bfloat16, max_run=1)
+    assert all(torch.equal(a, b) for a, b in zip(got, want)) and torch.equal(s0, s1)
+
+
+@pytest.mark.parametrize("streams", [2, 4])
+@pytest.mark.parametrize("width", [4, 260, 4096, 4100, 8192])
+def test_stream_step_in_registers(streams, width):
+    from tempura_amd.kernels import ops
+    g = torch.Generator().manual_seed(width + streams)
+    n = 3
+    h, y = torch.randn(n, streams * width, generator=g), torch.randn(n, width, generator=g)
+    mix, oc, ic, w = torch.randn(streams, streams, generator=g), torch.randn(streams, generator=g), torch.randn(streams, generator=g), torch.randn(width, generator=g)
+    for kw in (dict(y=y, mix=mix, out_coef=oc, in_coef=ic, norm_weight=w, eps=1e-6, out_dtype=torch.float32),
+               dict(y=y, mix=mix, out_coef=oc), dict(out_dtype=torch.float32, write_back=False),
+               dict(norm_weight=w, eps=1e-6, out_dtype=torch.bfloat16, rows=torch.tensor([2, 0], dtype=torch.int32), write_back=False)):
+        h0, h1 = h.clone(), h.to(DEV)
+        want = emu.stream_step(h0, streams, **kw)
+        got = ops.stream_step(h1, streams, **{k: v.to(DEV) if torch.is_tensor(v) else v for k, v in kw.items()})
+        _close(h1, h0, 1e-6)
+        if want is not None:
+            _close(got, want, 2e-6 if want.dtype == torch.float32 else 8e-3)
+
+
+@pytest.mark.parametrize("width,groups", [(256, 1), (1024, 4), (2048, 4), (4096, 8), (1028, 1), (4100, 1), (8192, 1), (24, 6)])
+def test_group_rmsnorm_in_registers(width, groups):
+    from tempura_amd.kernels import ops
+    g = torch.Generator().manual_seed(width)
+    x, w = torch.randn(5, width + 8, generator=g) * 3, torch.randn(width, generator=g)
+    for dt, tol in ((torch.float32, 2e-6), (torch.bfloat16, 8e-3)):
+        want = emu.rmsnorm_cols(x, 4, width, w, 1e-6, dt, groups)
+        _close(ops.rmsnorm_cols(x.to(DEV), 4, width, w.to(DEV), 1e-6, dt, groups), want, tol)
+
+
+@pytest.mark.parametrize("hidden", [4, 1028, 4096, 4100])
+@pytest.mark.parametrize("lens", [[1, 1, 1], [5, 1, 9]])
+def test_embed_bigram_leaves_the_last_tokens(hidden, lens):
+    from tempura_amd.kernels import ops
+    g = torch.Generator().manual_seed(hidden)
+    n, vocab, buckets = sum(lens), 50, 37
+    cu, req, slots = _runs(lens, g)
+    toks = torch.randint(0, vocab, (n,), generator=g, dtype=torch.int32)
+    pos = torch.arange(n, dtype=torch.int32)                     # (the first run begins its request, the others go on)
+    table, bigram, ptab = torch.randn(vocab, hidden, generator=g), torch.randn(buckets + 1, hidden, generator=g), torch.randn(n, hidden, generator=g)
+    prev = torch.randint(0, vocab, (len(lens) + 2, 1), generator=g, dtype=torch.int32)
+    for dt in (torch.float32, torch.bfloat16):
+        a, b, p = (t.to(dt) for t in (table, bigram, ptab))
+        p0, p1 = prev.clone(), prev.to(DEV)
+        want = emu.embed_bigram(toks, a, b, pos, req.cpu(), cu.cpu(), slots.cpu(), p0, len(lens), 31, 7, buckets, 0.5, p)
+        got = ops.embed_bigram(toks.to(DEV), a.to(DEV), b.to(DEV), pos.to(DEV), req, cu, slots, p1, len(lens), 31, 7, buckets, 0.5, p.to(DEV))
+        _close(got, want, 1e-6)
+        assert torch.equal(p1.cpu(), p0)
+
+
+@pytest.mark.parametrize("dims", [(32, 96, 32, 128), (3, 8, 4, 12), (2, 6, 2, 5)])
+def test_latent_rows_in_pieces(dims):
+    from tempura_amd.kernels import ops
+    heads, dim, rot, vdim = dims
+    g = torch.Generator().manual_seed(heads)
+    proj, up = torch.randn(3, 4 + heads * (rot + dim) + rot + 4, generator=g), torch.randn(3, heads * (dim + vdim), generator=g)
+    want = emu.latent_rows(proj, 4, 4 + heads * (rot + dim), up, heads, dim, rot, vdim)
+    assert torch.equal(ops.latent_rows(proj.to(DEV), 4, 4 + heads * (rot + dim), up.to(DEV), heads, dim, rot, vdim).cpu(), want)
+
+
+@pytest.mark.parametrize("experts,groups,keep", [(8, 4, 2), (64, 1, 1), (65, 1, 1), (128, 8, 3), (130, 2, 1)])
+def test_moe_route_by_experts_a_lane(experts, groups, keep):
+    from tempura_amd.kernels import ops
+    g = torch.Generator().manual_seed(experts)
+    logits = torch.randn(9, experts, generator=g)
+    want = emu.moe_route(logits, None, experts, 2, groups, keep)
+    got = ops.moe_route(logits.to(DEV), None, experts, 2, groups, keep)
+    assert torch.equal(got[1].cpu(), want[1])
+    _close(got[0], want[0], 2e-6)
+
+
+@pytest.mark.parametrize("width", [4, 6, 1028, 4096])
+def test_moe_rows_there_and_back(width):
+    from tempura_amd.kernels import ops
+    g = torch.Generator().manual_seed(width)
+    n, experts, top = 33, 5, 2
+    x, ids = torch.randn(n, width, generator=g), torch.stack([torch.randperm(experts, generator=g)[:top] for _ in range(n)]).to(torch.int32)
+    wts, y = torch.randn(n, top, generator=g), torch.randn(n, width, generator=g)
+    counts, offsets, rank = ops.moe_plan(ids.to(DEV), experts)
+    xg, row_of = ops.moe_gather(x.to(DEV), ids.to(DEV), rank, offsets)
+    order = sorted(range(n * top), key=lambda p: (int(ids.view(-1)[p]), p))
+    assert torch.equal(xg.cpu(), x[torch.tensor(order) // top])
+    want = (x.double()[:, None] * wts.double()[:, :, None]).sum(1)
+    _close(ops.moe_scatter(xg, row_of, wts.to(DEV)), want, 1e-6)
+    _close(ops.moe_scatter(xg, row_of, wts.to(DEV), y.to(DEV)), want + y.double(), 1e-6)

@@ -2010,6 +2010,104 @@ def linear_scan(q, k, v, decay: torch.Tensor, state: torch.Tensor, state_off: in
 
 
 # ---------------------------------------------------------------------------------
+# One token a request through a whole recurrent mixer.
+
+#: steps of up to this many requests take a recurrent mixer as one launch (0: never)
+mixer_step_rows = 128
+
+
+def mixer_step_ok(n: int, max_run: int, heads: int, dim: int, vdim: int, ranks, state: torch.Tensor, state_off: int, out: torch.Tensor, out_col0: int,
+                  gate_col0: int = 0, gate_width: int = 0) -> bool:
+    """Whether the one-launch steps below take ``n`` requests of ``max_run`` tokens each, at most: ``heads`` heads of ``dim`` by
+    ``vdim`` elements, low-rank projections of ``ranks``, the head's state at ``state_off`` of the rows of ``state``, results from
+    column ``out_col0`` of ``out``, a raw gate from column ``gate_col0`` of rows ``gate_width`` wide."""
+    # (a head's block has a fixed part that a small state does not pay for once there are more than four blocks a CU: 64 heads of
+    # 64 x 64, a captured chain, separate kernels / one launch: 8 requests 12.8 / 9.0 us, 16: 17.3 / 15.5, 64: 44 / 53; 32 heads of
+    # 128 x 128, 8 requests 26 / 14 us, 64: 85 / 68, 128: 205 / 154)
+    if dim * vdim < 8192 and n * heads > 1024:
+        return False
+    return _backend is None and max_run == 1 and 0 < n <= mixer_step_rows and 32 < dim <= 128 and dim % 4 == 0 and 0 < vdim <= 128 and \
+        vdim % 4 == 0 and all(0 < r <= 128 for r in ranks) and state.shape[1] % 4 == 0 and state_off % 4 == 0 and state.data_ptr() % 16 == 0 and \
+        out.shape[1] % 4 == 0 and out_col0 % 4 == 0 and out.data_ptr() % 16 == 0 and gate_col0 % 4 == 0 and gate_width % 4 == 0
+
+
+def _step_state(n, state, token_req, state_slots, out, out_col0, columns, what):
+    _need(state.dtype == torch.float32 and state.dim() == 2 and out.dim() == 2 and out.shape[0] == n and 0 <= out_col0
+          and out_col0 + columns <= out.shape[1], f"{what}: bad state or output rows")
+    _i32(token_req, n, "token_req")
+    _i32(state_slots, n, "state_slots")
+
+
+def delta_step(proj: torch.Tensor, col0: int, beta_col0: int, a_col0: int, g_col0: int, conv_w: torch.Tensor, a2_t: torch.Tensor,
+               g2_t: torch.Tensor, a_log: torch.Tensor, dt_bias: torch.Tensor, norm_w: torch.Tensor, state: torch.Tensor, conv_off: int,
+               state_off: int, token_req: torch.Tensor, state_slots: torch.Tensor, heads: int, dim: int, vdim: int, q_scale: float,
+               unit_eps: float, norm_eps: float, scale: float, out: torch.Tensor, out_col0: int) -> None:
+    """One token a request of a gated delta rule with as many key heads as heads: ``causal_conv`` (with SiLU) over the columns
+    q | k | v from ``col0`` on, ``lowrank_up`` for the decay and the gate, ``delta_scan`` and ``head_norm_gate``, in one launch and
+    with the same bits (``mixer_step_ok`` says for which sizes)."""
+    _dev_ok(proj, conv_w, a2_t, g2_t, a_log, dt_bias, norm_w, state, token_req, state_slots, out)
+    n, taps = proj.shape[0], conv_w.shape[0]
+    _step_state(n, state, token_req, state_slots, out, out_col0, heads * vdim, "delta_step")
+    _need(proj.dtype == torch.float32 and proj.dim() == 2 and col0 >= 0 and col0 + heads * (2 * dim + vdim) <= proj.shape[1]
+          and 0 <= beta_col0 and beta_col0 + heads <= proj.shape[1] and 0 <= a_col0 and a_col0 + a2_t.shape[0] <= proj.shape[1]
+          and 0 <= g_col0 and g_col0 + g2_t.shape[0] <= proj.shape[1], "delta_step: bad projection rows")
+    _need(conv_w.dtype == a2_t.dtype == g2_t.dtype == a_log.dtype == dt_bias.dtype == norm_w.dtype == torch.float32
+          and conv_w.shape[1] == heads * (2 * dim + vdim) and a2_t.shape[1] == heads * dim and g2_t.shape[1] == heads * vdim
+          and a_log.numel() == heads and dt_bias.numel() == heads * dim and norm_w.numel() == vdim, "delta_step: bad weights")
+    _call("tp_delta_step", _ptr(proj), ctypes.c_size_t(proj.shape[1]), int(col0), int(beta_col0), int(a_col0), a2_t.shape[0], int(g_col0),
+          g2_t.shape[0], _ptr(conv_w), taps, _ptr(a2_t), _ptr(g2_t), _ptr(a_log), _ptr(dt_bias), _ptr(norm_w), _ptr(state),
+          ctypes.c_size_t(state.shape[1]), ctypes.c_size_t(conv_off), ctypes.c_size_t(state_off), _ptr(token_req), _ptr(state_slots), _ptr(out),
+          _dt(out), ctypes.c_size_t(out.shape[1]), int(out_col0), n, int(heads), int(dim), int(vdim), ctypes.c_float(q_scale),
+          ctypes.c_float(unit_eps), ctypes.c_float(norm_eps), ctypes.c_float(scale), _stream())
+
+
+def general_delta_step(proj: torch.Tensor, col0: int, gate_col0: int, w_col0: int, w2_t: torch.Tensor, w0: torch.Tensor, rate: float,
+                       a_bias: torch.Tensor, norm_w: torch.Tensor, state: torch.Tensor, state_off: int, token_req: torch.Tensor,
+                       state_slots: torch.Tensor, heads: int, dim: int, unit_eps: float, norm_eps: float, scale: float, out: torch.Tensor,
+                       out_col0: int) -> None:
+    """One token a request of a generalized delta rule: ``lowrank_up`` for the decay, ``general_delta_scan`` and
+    ``head_norm_gate`` with the raw gate columns, in one launch and with the same bits."""
+    _dev_ok(proj, w2_t, w0, a_bias, norm_w, state, token_req, state_slots, out)
+    n, hd = proj.shape[0], heads * dim
+    _step_state(n, state, token_req, state_slots, out, out_col0, hd, "general_delta_step")
+    _need(proj.dtype == torch.float32 and proj.dim() == 2 and col0 >= 0 and col0 + 4 * hd <= proj.shape[1] and 0 <= gate_col0
+          and gate_col0 + hd <= proj.shape[1] and 0 <= w_col0 and w_col0 + w2_t.shape[0] <= proj.shape[1], "general_delta_step: bad projection rows")
+    _need(w2_t.dtype == w0.dtype == a_bias.dtype == norm_w.dtype == torch.float32 and w2_t.shape[1] == hd and w0.numel() == hd
+          and a_bias.numel() == hd and norm_w.numel() == hd, "general_delta_step: bad weights")
+    _call("tp_general_delta_step", _ptr(proj), ctypes.c_size_t(proj.shape[1]), int(col0), int(gate_col0), int(w_col0), w2_t.shape[0], _ptr(w2_t),
+          _ptr(w0), ctypes.c_float(rate), _ptr(a_bias), _ptr(norm_w), _ptr(state), ctypes.c_size_t(state.shape[1]), ctypes.c_size_t(state_off),
+          _ptr(token_req), _ptr(state_slots), _ptr(out), _dt(out), ctypes.c_size_t(out.shape[1]), int(out_col0), n, int(heads), int(dim),
+          ctypes.c_float(unit_eps), ctypes.c_float(norm_eps), ctypes.c_float(scale), _stream())
+
+
+def linear_step(q, k, v, x, w2_t: torch.Tensor, mode: str, bias: torch.Tensor, rate: float, in_act: Optional[str],
+                bonus: Optional[torch.Tensor], q_scale: float, gate, norm_w: torch.Tensor, norm_eps: float, scale: float, state: torch.Tensor,
+                state_off: int, token_req: torch.Tensor, state_slots: torch.Tensor, heads: int, dim: int, vdim: int, out: torch.Tensor,
+                out_col0: int) -> None:
+    """One token a request of a linear recurrence: ``lowrank_up`` (``mode`` of rows ``x``) for the decay, ``linear_scan`` and
+    ``head_norm_gate`` with the SiLU of the raw gate columns, in one launch and with the same bits.  ``q``, ``k``, ``v``, ``x`` and
+    ``gate`` are pairs (float32 rows, first column)."""
+    _need(mode in ("rate_sigmoid", "exp_exp", "root_sigmoid") and in_act in (None, "tanh"), "linear_step: bad decay")
+    _dev_ok(q[0], k[0], v[0], x[0], gate[0], w2_t, bias, bonus, norm_w, state, token_req, state_slots, out)
+    n = q[0].shape[0]
+    _step_state(n, state, token_req, state_slots, out, out_col0, heads * vdim, "linear_step")
+    for (rows, col), width, what in ((q, heads * dim, "q"), (k, heads * dim, "k"), (v, heads * vdim, "v"), (x, w2_t.shape[0], "decay"),
+                                     (gate, heads * vdim, "gate")):
+        _need(rows.dtype == torch.float32 and rows.dim() == 2 and rows.shape[0] == n and 0 <= col and col + width <= rows.shape[1],
+              f"linear_step: bad {what} rows")
+    _need(w2_t.dtype == bias.dtype == norm_w.dtype == torch.float32 and w2_t.shape[1] == heads * dim and bias.numel() == heads * dim
+          and norm_w.numel() in (vdim, heads * vdim) and (bonus is None or (bonus.dtype == torch.float32 and bonus.numel() == heads * dim)),
+          "linear_step: bad weights")
+    at = lambda rows: ctypes.c_void_p(rows[0].data_ptr() + 4 * int(rows[1]))
+    wide = lambda rows: ctypes.c_size_t(rows[0].shape[1])
+    _call("tp_linear_step", at(q), wide(q), at(k), wide(k), at(v), wide(v), at(x), wide(x), w2_t.shape[0], _ptr(w2_t), _ptr(bias),
+          LOWRANK_MODES[mode], 1 if in_act == "tanh" else 0, ctypes.c_float(rate), _ptr(bonus), ctypes.c_float(q_scale), at(gate), wide(gate),
+          GATE_ACTS["silu"], _ptr(norm_w), int(norm_w.numel() == heads * vdim and heads > 1), _ptr(state), ctypes.c_size_t(state.shape[1]),
+          ctypes.c_size_t(state_off), _ptr(token_req), _ptr(state_slots), _ptr(out), _dt(out), ctypes.c_size_t(out.shape[1]), int(out_col0), n,
+          int(heads), int(dim), int(vdim), ctypes.c_float(norm_eps), ctypes.c_float(scale), _stream())
+
+
+# ---------------------------------------------------------------------------------
 # Products of decode steps that come in groups.
 
 def few_rows_ok(m: int, width: int, dtype: torch.dtype) -> bool:

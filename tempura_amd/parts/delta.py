@@ -86,6 +86,14 @@ class GatedDeltaMixer(BranchMixer):
         return torch.cat([self._to_device(t) for t in rows], dim=0).contiguous(), self._to_device(get(w["o"]))
 
     def run(self, proj, col0, ctx, cache, out, out_col0, scale):
+        if self.num_heads == self.num_kv_heads and ops.mixer_step_ok(
+                proj.shape[0], ctx.max_q_len, self.num_heads, self.head_dim, self.value_dim, (self.a2_t.shape[0], self.g2_t.shape[0]), cache.state,
+                self.state_off + self.conv_floats, out, out_col0):
+            ops.delta_step(proj, col0, col0 + self.beta_col, col0 + self.a1_col, col0 + self.g1_col, self.conv_w, self.a2_t, self.g2_t,
+                           self.a_log, self.dt_bias, self.norm_w, cache.state, self.state_off, self.state_off + self.conv_floats,
+                           ctx.token_req, ctx.state_slots, self.num_heads, self.head_dim, self.value_dim, self.q_scale, self.unit_eps,
+                           self.norm_eps, scale, out, out_col0)
+            return
         qkv = ops.causal_conv(proj, col0, self.channels, self.conv_w, None, cache.state, ctx.cu_seqlens, ctx.token_req,
                               ctx.state_slots, ctx.num_requests, state_off=self.state_off, act=True, max_run=ctx.max_q_len)
         decay = ops.lowrank_up(proj, col0 + self.a1_col, self.a2_t, "decay", self.a_log, self.dt_bias, self.head_dim)
@@ -150,6 +158,12 @@ class GeneralDeltaMixer(BranchMixer):
         return torch.cat([self._to_device(t) for t in rows], dim=0).contiguous(), self._to_device(get(w["o"]))
 
     def run(self, proj, col0, ctx, cache, out, out_col0, scale):
+        if ops.mixer_step_ok(proj.shape[0], ctx.max_q_len, self.num_heads, self.head_dim, self.head_dim, (self.w2_t.shape[0],), cache.state, self.state_off,
+                             out, out_col0, col0 + self.gate_col, proj.shape[1]):
+            ops.general_delta_step(proj, col0, col0 + self.gate_col, col0 + self.w1_col, self.w2_t, self.w0, self.decay_rate, self.a_bias,
+                                   self.norm_w, cache.state, self.state_off, ctx.token_req, ctx.state_slots, self.num_heads, self.head_dim,
+                                   self.unit_eps, self.norm_eps, scale, out, out_col0)
+            return
         decay = ops.lowrank_up(proj, col0 + self.w1_col, self.w2_t, "rate_sigmoid", bias=self.w0, rate=self.decay_rate, in_act="tanh")
         o = ops.general_delta_scan(proj, col0, decay, self.a_bias, cache.state, self.state_off, ctx.cu_seqlens, ctx.state_slots,
                                    ctx.num_requests, self.num_heads, self.head_dim, self.unit_eps)

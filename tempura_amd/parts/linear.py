@@ -82,10 +82,16 @@ class WkvMixer(Mixer):
             r, k, v, (g, g_col), (w, w_col) = ((proj, col) for col in self.cols)
         else:
             r, k, v, (g, g_col), (w, w_col) = ((ops.linear(m, wt, torch.float32), 0) for m, wt in zip(mixes, self.w_in))
+        act = torch.empty((g.shape[0], self.inner), dtype=self.dtype, device=g.device)
+        if ops.mixer_step_ok(g.shape[0], ctx.max_q_len, self.num_heads, self.head_dim, self.head_dim, (self.w2_t.shape[0],), cache.state, 0, act, 0, g_col,
+                             g.shape[1]):
+            ops.linear_step(r, k, v, (w, w_col), self.w2_t, "exp_exp", self.w0, 0.0, "tanh", self.bonus, 1.0, (g, g_col), self.norm_w,
+                            self.norm_eps, 1.0, cache.state, 0, ctx.token_req, ctx.state_slots, self.num_heads, self.head_dim, self.head_dim,
+                            act, 0)
+            return ops.linear(act, self.w_out, torch.float32, residual=residual)
         decay = ops.lowrank_up(w, w_col, self.w2_t, "exp_exp", bias=self.w0, in_act="tanh")
         o = ops.linear_scan(r, k, v, decay, cache.state, 0, ctx.cu_seqlens, ctx.state_slots, ctx.num_requests,
                             self.num_heads, self.head_dim, self.head_dim, bonus=self.bonus, max_run=ctx.max_q_len)
-        act = torch.empty((o.shape[0], self.inner), dtype=self.dtype, device=o.device)
         ops.head_norm_gate(o, self.norm_w, None, self.norm_eps, 1.0, self.num_heads, act, 0, gate_rows=g, gate_col0=g_col, gate_act="silu")
         return ops.linear(act, self.w_out, torch.float32, residual=residual)
 
@@ -144,6 +150,13 @@ class GatedLinearMixer(BranchMixer):
         return torch.cat([self._to_device(t) for t in rows], dim=0).contiguous(), self._to_device(get(w["o"]))
 
     def run(self, proj, col0, ctx, cache, out, out_col0, scale):
+        if ops.mixer_step_ok(proj.shape[0], ctx.max_q_len, self.num_heads, self.head_dim, self.value_dim, (self.a2_t.shape[0],), cache.state, self.state_off,
+                             out, out_col0, col0 + self.gate_col, proj.shape[1]):
+            ops.linear_step((proj, col0), (proj, col0 + self.qk_dim), (proj, col0 + self.v_col), (proj, col0 + self.a1_col), self.a2_t,
+                            "root_sigmoid", self.a2_bias, 1.0 / self.decay_root, None, None, self.q_scale, (proj, col0 + self.gate_col),
+                            self.norm_w, self.norm_eps, scale, cache.state, self.state_off, ctx.token_req, ctx.state_slots, self.num_heads,
+                            self.head_dim, self.value_dim, out, out_col0)
+            return
         decay = ops.lowrank_up(proj, col0 + self.a1_col, self.a2_t, "root_sigmoid", bias=self.a2_bias, rate=1.0 / self.decay_root)
         o = ops.linear_scan((proj, col0), (proj, col0 + self.qk_dim), (proj, col0 + self.v_col), decay, cache.state, self.state_off,
                             ctx.cu_seqlens, ctx.state_slots, ctx.num_requests, self.num_heads, self.head_dim, self.value_dim,

@@ -1715,6 +1715,34 @@ def moe_plan(ids: torch.Tensor, experts: int):
     return counts, offsets, rank
 
 
+def moe_linear_ok(experts: int, n: int, k: int, w, pairs: int = 0) -> bool:
+    """Whether ``moe_linear`` takes the experts' stacked weight ``w`` (each [n, k]) and is the better way for ``pairs`` rows."""
+    # (its tiles are 128 x 128; from some thousand rows an expert on, a product for each with tiles of 256 columns is faster.  Both
+    # products of eight experts, 16,384 pairs / 32,768 pairs, a product an expert against one launch: 4,096 x 4,096 gated and 4,096 x
+    # 2,048 1,095 / 1,776 us against 1,097 / 2,284; 2,048 x 4,096 and 4,096 x 2,048 870 / 1,340 against 766 / 1,640)
+    if pairs > 2048 * experts:
+        return False
+    return _backend is None and allow_mfma and w is not None and w.dtype == torch.bfloat16 and 0 < experts <= 64 and n % 16 == 0 and k % 64 == 0 and \
+        tuple(w.shape) == (experts * n, k)
+
+
+def moe_linear(x: torch.Tensor, w, offsets: torch.Tensor, experts: int, output: str = "float32") -> torch.Tensor:
+    """bfloat16 rows sorted by expert (``moe_gather``; ``offsets`` int32 [experts + 1] of ``moe_plan``) times the stacked weights
+    ``w`` [experts * n, k], a row with its expert's, in one launch and without the counts on the host.  ``output``: ``float32``
+    [pairs, n]; ``swiglu``: bfloat16 [pairs, n / 2], the gated activation of interleaved gate/up rows; ``relu2``: bfloat16 [pairs, n],
+    max(v, 0)^2.  Sizes: ``moe_linear_ok`` (``relu2``: n a multiple of 128)."""
+    wd, wl = _w_args(w)
+    _dev_ok(x, wd, offsets)
+    pairs, k = x.shape
+    n = w.shape[0] // experts
+    _need(x.dtype == torch.bfloat16 and x.dim() == 2 and w.shape[1] == k and moe_linear_ok(experts, n, k, w), "moe_linear: bad operands")
+    _i32(offsets, experts + 1, "offsets")
+    mode = {"float32": 0, "swiglu": 2, "relu2": 3}[output]
+    out = torch.empty((pairs, n // 2 if mode == 2 else n), dtype=torch.float32 if mode == 0 else torch.bfloat16, device=x.device)
+    _call("tp_moe_linear", _ptr(x), _ptr(wd), int(bool(wl)), _ptr(out), mode, pairs, int(experts), _ptr(offsets), n, k, _stream(), tag=(pairs, n, k))
+    return out
+
+
 def moe_gather(x: torch.Tensor, ids: torch.Tensor, rank: torch.Tensor, offsets: torch.Tensor):
     """(rows [n * top, width] of ``x`` [n, width] in the order of the experts, row_of int32 [n, top]: the row of pair (t, k))."""
     if _backend is not None:

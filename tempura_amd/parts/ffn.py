@@ -168,9 +168,11 @@ class RoutedExperts(FeedForward):
     where the expert was not chosen; ``ops.moe_spread``), then the experts' down products one after the other into
     one sum, ascending; nothing of the batch is read on the host, and at a few rows with several experts each
     nearly every expert's weights are read anyway.  A step with portions of prompts: the
-    chosen (token, expert) pairs are brought into the order of the experts, the host reads how many rows each expert
-    has (the one wait of the layer), every expert with rows is one pair of products over its rows, and a token's
-    sum adds its experts' rows in the order of its choice.  Either way a row's result does not depend on what else
+    chosen (token, expert) pairs are brought into the order of the experts, one product over the rows of all experts takes the
+    up weights and one the down weights (``ops.moe_linear``, which reads on the device where an expert's rows begin), and a
+    token's sum adds its experts' rows in the order of its choice.  (In float32, or at sizes which that product does not take,
+    the host reads how many rows each expert has, the one wait of the layer, and every expert with rows is one pair of
+    products over its rows.)  Either way a row's result does not depend on what else
     is in the batch; the ways differ in rounding only.  Tensor roles: ``router``,
     ``correction``, and ``gate`` / ``up`` / ``down`` as name patterns with ``{}`` for the expert's number.
 
@@ -363,6 +365,15 @@ class RoutedExperts(FeedForward):
             return y if residual is None else None
         counts, offsets, rank = ops.moe_plan(ids, self.experts)
         xg, row_of = ops.moe_gather(x, ids, rank, offsets)
+        up_rows = (2 if self.expert_kind == "gated" else 1) * self.intermediate_size
+        if (self.fused or self.expert_kind == "plain") and ops.moe_linear_ok(self.experts, up_rows, self.hidden_size, self.w13_all, xg.shape[0]) and \
+                ops.moe_linear_ok(self.experts, self.hidden_size, self.intermediate_size, self.w2_all, xg.shape[0]):
+            if self.fused or self.fused_relu2:
+                a = ops.moe_linear(xg, self.w13_all, offsets, self.experts, "swiglu" if self.fused else "relu2")
+            else:
+                a = ops.activation(ops.moe_linear(xg, self.w13_all, offsets, self.experts), self.activation, self.dtype)
+            y = ops.moe_scatter(ops.moe_linear(a, self.w2_all, offsets, self.experts), row_of, weights, residual)
+            return y if residual is None else None
         yg = torch.zeros((xg.shape[0], self.hidden_size), dtype=torch.float32, device=xg.device)
         at = 0
         for n, m in enumerate(counts.tolist()):      # (the host waits here for the router)

@@ -141,3 +141,31 @@ def test_moe_rows_there_and_back(width):
     want = (x.double()[:, None] * wts.double()[:, :, None]).sum(1)
     _close(ops.moe_scatter(xg, row_of, wts.to(DEV)), want, 1e-6)
     _close(ops.moe_scatter(xg, row_of, wts.to(DEV), y.to(DEV)), want + y.double(), 1e-6)
+
+
+@pytest.mark.parametrize("counts,n,k", [([0, 5, 0, 300, 128, 1], 256, 64), ([129, 127, 255, 257], 400, 192), ([1], 128, 320), ([0, 0, 3], 16, 64)])
+@pytest.mark.parametrize("tiled", [True, False])
+@pytest.mark.parametrize("output", ["float32", "swiglu", "relu2"])
+def test_moe_linear(counts, n, k, tiled, output):
+    """Rows of several experts in one launch: experts without rows, tiles that end inside an expert, weights whose columns are no whole
+    tile; float64 of the bfloat16 operands, float32 sums of k products within 2^-24 k of their magnitudes (2e-6 of the largest here)."""
+    from tempura_amd.kernels import ops
+    if output == "relu2" and n % 128:
+        pytest.skip("whole tiles of activated columns only")
+    g = torch.Generator().manual_seed(sum(counts) + n)
+    E, pairs = len(counts), sum(counts)
+    x, w = torch.randn(pairs, k, generator=g).to(torch.bfloat16), (torch.randn(E * n, k, generator=g) * 0.2).to(torch.bfloat16)
+    offsets = torch.tensor([0] + list(torch.tensor(counts).cumsum(0)), dtype=torch.int32)
+    want = torch.cat([x[offsets[e]: offsets[e + 1]].double() @ w[e * n: (e + 1) * n].double().T for e in range(E)])
+    wd = ops.tile_weight(w.to(DEV)) if tiled else w.to(DEV)
+    assert isinstance(wd, ops.TiledWeight) == tiled and ops.moe_linear_ok(E, n, k, wd)
+    got = ops.moe_linear(x.to(DEV), wd, offsets.to(DEV), E, output)
+    if output == "float32":
+        _close(got, want, 2e-6)
+    elif output == "relu2":
+        _close(got, want.clamp(min=0.0) ** 2, 8e-3)
+    else:
+        pair = want.view(pairs, -1, 2, 8)
+        gate, up = pair[:, :, 0].reshape(pairs, -1), pair[:, :, 1].reshape(pairs, -1)
+        _close(got, gate * torch.sigmoid(gate) * up, 8e-3)
+    assert torch.equal(got, ops.moe_linear(x.to(DEV), wd, offsets.to(DEV), E, output))

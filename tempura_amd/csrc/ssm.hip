@@ -197,15 +197,16 @@ extern "C" int tp_causal_conv(const float* in, int in_stride, int col0, const fl
 // permutes up to 16 lanes, which cost an instruction each and no trip through LDS).
 //
 // Long runs are cut into pieces of `piece` tokens that run side by side (a recurrence is a chain, and a prompt of
-// thousands of tokens on a chain leaves most of the chip idle).  Three launches of the same kernel:
+// thousands of tokens on a chain leaves most of the chip idle).  Three launches:
 //   SCAN_LOCAL   every piece from a zero state: its end state and its total decay, to scratch;
-//   SCAN_CARRY   per (request, head, columns), piece by piece: the state a piece starts from is
+//   the carry    per state entry, piece by piece (ssm_carry_kernel): the state a piece starts from is
 //                decay(previous piece) * (state the previous piece started from) + (its end state from zero);
 //                the state after the last piece is the request's new state;
 //   SCAN_OUTPUT  every piece again from the state it starts from, now writing y.
+// Where the sizes fit, the first and the last of them are products on the matrix cores (ssm_chunk_kernel).
 // Short runs (single tokens above all) take SCAN_DIRECT: one launch, from the request's state to its new state.
 // How a run is cut changes rounding only.
-enum { SCAN_DIRECT = 0, SCAN_LOCAL = 1, SCAN_CARRY = 2, SCAN_OUTPUT = 3 };
+enum { SCAN_DIRECT = 0, SCAN_LOCAL = 1, SCAN_OUTPUT = 2 };
 
 struct ScanArgs {
   const float* xbc;
@@ -266,33 +267,6 @@ __global__ __launch_bounds__(256) void ssm_scan_kernel(ScanArgs a) {
 #define SCAN_HAS(i, j) (n0 + (i) < N && p0 + (j) < P)
 #define SCAN_AT(i, j) ((size_t)(n0 + (i)) * P + p0 + (j))
 
-  if (a.mode == SCAN_CARRY) {
-    // the state each piece starts from, in place of what it ended with from zero; then the request's new state
-    float cur[TN][TP];
-#pragma unroll
-    for (int i = 0; i < TN; ++i)
-#pragma unroll
-      for (int j = 0; j < TP; ++j) cur[i][j] = SCAN_HAS(i, j) ? S[SCAN_AT(i, j)] : 0.f;
-    for (int c = 0; c < pieces; ++c) {
-      const float decay = PD[c];
-      float* ps = PS + (size_t)c * N * P;
-#pragma unroll
-      for (int i = 0; i < TN; ++i)
-#pragma unroll
-        for (int j = 0; j < TP; ++j)
-          if (SCAN_HAS(i, j)) {
-            const float local = ps[SCAN_AT(i, j)];
-            ps[SCAN_AT(i, j)] = cur[i][j];
-            cur[i][j] = fmaf(decay, cur[i][j], local);
-          }
-    }
-#pragma unroll
-    for (int i = 0; i < TN; ++i)
-#pragma unroll
-      for (int j = 0; j < TP; ++j)
-        if (SCAN_HAS(i, j)) S[SCAN_AT(i, j)] = cur[i][j];
-    return;
-  }
   if (pc >= pieces) return;
   const int start = a.mode == SCAN_DIRECT ? run0 : run0 + pc * a.piece;
   const int len = a.mode == SCAN_DIRECT ? run_len : min(a.piece, run_len - pc * a.piece);
@@ -388,6 +362,259 @@ __global__ __launch_bounds__(256) void ssm_scan_kernel(ScanArgs a) {
 #undef SCAN_AT
 }
 
+// ---- pieces of a long run on the matrix cores -----------------------------------------------------
+// The same two passes over a piece (SCAN_LOCAL, SCAN_OUTPUT) for states of 16 x NT entries, 32 tokens at a time as four products with
+// v_mfma_f32_16x16x4_f32.  With c_t the sum of dt up to token t of the 32 and S the state before them:
+//   y_t = exp(A c_t) S^T C_t + sum over s <= t of (C_t . B_s) exp(A (c_t - c_s)) dt_s x_s + d_skip x_t
+//   S  <- exp(A c_31) S + sum over s of exp(A (c_31 - c_s)) dt_s B_s x_s^T
+// The sums c are float64 and every exponent is at most zero, so a decay over many tokens is one exponential of a difference: its error
+// does not grow with the distance, as that of a product of steps does.
+// A block owns one request, head, piece and 64 value columns; a wave keeps the state of 16 columns in accumulators, which lie as the
+// next product's operand wants them (a lane holds four entries of one column), so the state never leaves the registers.  C_t . B_s is
+// worked out once a block (one 16 x 16 tile a wave) and passed through LDS with its weights; the tile above the diagonal is left out.
+// Sums over the state are added in runs of eight products: longer chains of roundings would lose to the walk's, which adds 16 a lane
+// and then the lanes in a tree.
+// Items go to the XCDs in contiguous shares, heads fastest: what shares B and C of a piece is on one L2.
+//
+// Bound by the matrix cores: 2,048 tokens of 128 heads of 64 with a state of 128 are 14.5 GFLOP in both passes, 100 us at the float32
+// rate; with the carry 220 us, token by token 656 (257 tokens 72 / 206 us; 32 heads of 64 with a state of 16, 2,048 tokens, 34 / 125).
+// (Two blocks a CU for a state of 128: held to three the last pass spills, 248 us.)
+#define SC_T 32     // tokens at a time
+#define SC_P 64     // value columns a block
+typedef float f32x4_s __attribute__((ext_vector_type(4)));
+
+template <int NT, bool OUT>
+__global__ __launch_bounds__(256, OUT && NT == 8 ? 2 : 3) void ssm_chunk_kernel(ScanArgs a, int requests) {
+  constexpr int N = 16 * NT, LD = N + 4, NV = (SC_T * N / 4 + 255) / 256;
+  __shared__ __attribute__((aligned(16))) float Bs[SC_T][LD];
+  __shared__ __attribute__((aligned(16))) float Cs[OUT ? SC_T : 1][LD];
+  __shared__ __attribute__((aligned(16))) float xs[SC_T][SC_P + 4];
+  __shared__ __attribute__((aligned(16))) float Gs[OUT ? SC_T : 1][SC_T + 4];
+  __shared__ double cs[SC_T];
+  __shared__ float dts[SC_T], from_start[SC_T], to_end[SC_T];
+  const int P = a.head_dim, slices = (P + SC_P - 1) / SC_P;
+  const long total = (long)requests * a.heads * slices * a.max_pieces, share = (total + 7) / 8;
+  long item = (long)(blockIdx.x & 7) * share + (blockIdx.x >> 3);
+  if ((long)(blockIdx.x >> 3) >= share || item >= total) return;
+  const int h = (int)(item % a.heads);
+  item /= a.heads;
+  const int slice = (int)(item % slices);
+  item /= slices;
+  const int pc = (int)(item % a.max_pieces), r = (int)(item / a.max_pieces);
+  const int run0 = a.cu_seqlens[r], run_len = a.cu_seqlens[r + 1] - run0;
+  const int start = run0 + pc * a.piece, len = min(a.piece, run_len - pc * a.piece);
+  if (len <= 0) return;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, col = lane & 15, quad = lane >> 4;
+  const int g = h / (a.heads / a.groups), inner = a.heads * P;
+  const int p = slice * SC_P + wave * 16 + col;      // this lane's value column
+  const bool live = p < P;                           // (P is a multiple of 16: a wave's columns are all there or none is)
+  float* state = a.piece_state + (((size_t)r * a.heads + h) * a.max_pieces + pc) * N * P;
+  const float A = -expf(a.a_log[h]), dtb = a.dt_bias[h], Dh = a.d_skip[h];
+  f32x4_s S[NT];
+#pragma unroll
+  for (int j = 0; j < NT; ++j)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) S[j][i] = (OUT && live) ? state[(size_t)(16 * j + 4 * quad + i) * P + p] : 0.f;
+
+  f32x4_s br[NV], cr[OUT ? NV : 1], xr[2];
+  float dt_raw = 0.f;
+  auto fetch = [&](int t0) {     // the next tokens on their way (rows past the piece's last: zeros)
+#pragma unroll
+    for (int v = 0; v < NV; ++v) {
+      const int idx = tid + 256 * v, t = idx / (N / 4), n = idx % (N / 4) * 4;
+      const bool ok = t < SC_T && t0 + t < len;
+      const float* row = a.xbc + (size_t)(start + (ok ? t0 + t : 0)) * a.channels + inner;
+      br[v] = ok ? *(const f32x4_s*)(row + g * N + n) : (f32x4_s)(0.f);
+      if constexpr (OUT) cr[v] = ok ? *(const f32x4_s*)(row + (a.groups + g) * N + n) : (f32x4_s)(0.f);
+    }
+#pragma unroll
+    for (int v = 0; v < 2; ++v) {
+      const int t = (tid >> 4) + 16 * v, c = slice * SC_P + (tid & 15) * 4;
+      xr[v] = (t0 + t < len && c < P) ? *(const f32x4_s*)(a.xbc + (size_t)(start + t0 + t) * a.channels + (size_t)h * P + c) : (f32x4_s)(0.f);
+    }
+    if (wave == 0 && lane < SC_T && t0 + lane < len) dt_raw = a.proj[(size_t)(start + t0 + lane) * a.proj_stride + a.dt_col0 + h];
+  };
+  double dt_sum = 0.0;
+  fetch(0);
+  for (int t0 = 0; t0 < len; t0 += SC_T) {
+    __syncthreads();
+#pragma unroll
+    for (int v = 0; v < NV; ++v) {
+      const int idx = tid + 256 * v, t = idx / (N / 4), n = idx % (N / 4) * 4;
+      if (t < SC_T) {
+        *(f32x4_s*)&Bs[t][n] = br[v];
+        if constexpr (OUT) *(f32x4_s*)&Cs[t][n] = cr[v];
+      }
+    }
+#pragma unroll
+    for (int v = 0; v < 2; ++v) *(f32x4_s*)&xs[(tid >> 4) + 16 * v][(tid & 15) * 4] = xr[v];
+    if (wave == 0) {
+      const float dt = (lane < SC_T && t0 + lane < len) ? softplus_f(dt_raw + dtb) : 0.f;
+      double c = dt;
+#pragma unroll
+      for (int d = 1; d < SC_T; d *= 2) {
+        const double below = __shfl_up(c, d, SC_T);
+        if ((lane & (SC_T - 1)) >= d) c += below;
+      }
+      const double all = __shfl(c, SC_T - 1, TP_WAVE);
+      dt_sum += all;
+      if (lane < SC_T) {
+        // (a difference of zero is a decay of one, whatever A is)
+        cs[lane] = c;
+        dts[lane] = dt;
+        from_start[lane] = c == 0.0 ? 1.f : expf((float)(A * c));
+        to_end[lane] = all == c ? 1.f : expf((float)(A * (all - c)));
+      }
+    }
+    __syncthreads();
+    if (t0 + SC_T < len) fetch(t0 + SC_T);
+
+    if constexpr (OUT) {
+      // C_t . B_s with its weight, rows t of 16 and columns s of 16 a wave: (0, 0), (16, 0), (16, 16)
+      if (wave < 3) {
+        const int tt = wave > 0 ? 16 : 0, ss = wave > 1 ? 16 : 0, t = tt + col;
+        f32x4_s cb = (f32x4_s)(0.f);
+#pragma unroll
+        for (int j0 = 0; j0 < NT; j0 += 2) {
+          f32x4_s sum[4];
+#pragma unroll
+          for (int j = j0; j < j0 + 2 && j < NT; ++j) {
+            const f32x4_s b4 = *(const f32x4_s*)&Bs[ss + col][16 * j + 4 * quad], c4 = *(const f32x4_s*)&Cs[t][16 * j + 4 * quad];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) sum[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(b4[i], c4[i], j == j0 ? (f32x4_s)(0.f) : sum[i], 0, 0, 0);
+          }
+          cb += (sum[0] + sum[1]) + (sum[2] + sum[3]);
+        }
+        const double ct = cs[t];
+        f32x4_s w;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int s = ss + 4 * quad + i;
+          const double d = ct - cs[s];
+          const float decay = d == 0.0 ? 1.f : expf((float)(A * d));
+          w[i] = s <= t ? cb[i] * decay * dts[s] : 0.f;
+        }
+        *(f32x4_s*)&Gs[t][ss + 4 * quad] = w;
+      }
+    }
+    // this lane's x: tokens 16 k + 4 quad + i of its column
+    f32x4_s xv[2];
+#pragma unroll
+    for (int k = 0; k < 2; ++k)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) xv[k][i] = xs[16 * k + 4 * quad + i][wave * 16 + col];
+    if constexpr (OUT) {
+      f32x4_s y[2];
+#pragma unroll
+      for (int k = 0; k < 2; ++k) {
+        y[k] = (f32x4_s)(0.f);
+#pragma unroll
+        for (int j0 = 0; j0 < NT; j0 += 2) {
+          f32x4_s sum[4];
+#pragma unroll
+          for (int j = j0; j < j0 + 2 && j < NT; ++j) {
+            const f32x4_s c4 = *(const f32x4_s*)&Cs[16 * k + col][16 * j + 4 * quad];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) sum[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(c4[i], S[j][i], j == j0 ? (f32x4_s)(0.f) : sum[i], 0, 0, 0);
+          }
+          y[k] += (sum[0] + sum[1]) + (sum[2] + sum[3]);
+        }
+      }
+      __syncthreads();
+      // A zero of the weights times an x that is not finite would reach tokens before it: those columns are added one by one.
+      float odd = 0.f;
+#pragma unroll
+      for (int k = 0; k < 2; ++k)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) odd = fmaf(xv[k][i], 0.f, odd);
+      if (__any(!(odd == 0.f))) {
+#pragma unroll
+        for (int k = 0; k < 2; ++k)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const int t = 16 * k + 4 * quad + i;
+            y[k][i] *= from_start[t];
+            for (int s = 0; s <= t; ++s) y[k][i] = fmaf(Gs[t][s], xs[s][wave * 16 + col], y[k][i]);
+          }
+      } else {
+        f32x4_s z[3];
+#pragma unroll
+        for (int u = 0; u < 3; ++u) {      // (tokens 0..15 of themselves; tokens 16..31 of these and of themselves)
+          f32x4_s sum[2];
+          const f32x4_s g4 = *(const f32x4_s*)&Gs[u > 0 ? 16 + col : col][u > 1 ? 16 + 4 * quad : 4 * quad];
+#pragma unroll
+          for (int i = 0; i < 4; ++i) sum[i % 2] = __builtin_amdgcn_mfma_f32_16x16x4f32(g4[i], xv[u > 1][i], i < 2 ? (f32x4_s)(0.f) : sum[i % 2], 0, 0, 0);
+          z[u] = sum[0] + sum[1];
+        }
+        z[1] += z[2];
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+          const f32x4_s e = *(const f32x4_s*)&from_start[16 * k + 4 * quad];
+#pragma unroll
+          for (int i = 0; i < 4; ++i) y[k][i] = fmaf(y[k][i], e[i], z[k][i]);
+        }
+      }
+#pragma unroll
+      for (int k = 0; k < 2; ++k)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int t = 16 * k + 4 * quad + i;
+          if (live && t0 + t < len) a.y[(size_t)(start + t0 + t) * inner + (size_t)h * P + p] = fmaf(Dh, xv[k][i], y[k][i]);
+        }
+    }
+    if (!OUT || t0 + SC_T < len) {
+      const float decay = from_start[SC_T - 1];
+#pragma unroll
+      for (int j = 0; j < NT; ++j) S[j] *= decay;
+#pragma unroll
+      for (int k = 0; k < 2; ++k) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int s = 16 * k + 4 * quad + i;
+          const float w = xv[k][i] * (to_end[s] * dts[s]);
+#pragma unroll
+          for (int j = 0; j < NT; ++j) S[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(Bs[s][16 * j + col], w, S[j], 0, 0, 0);
+        }
+      }
+    }
+  }
+  if constexpr (!OUT) {
+    if (live)
+#pragma unroll
+      for (int j = 0; j < NT; ++j)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) state[(size_t)(16 * j + 4 * quad + i) * P + p] = S[j][i];
+    if (slice == 0 && tid == 0) a.piece_decay[((size_t)r * a.heads + h) * a.max_pieces + pc] = dt_sum == 0.0 ? 1.f : expf((float)(A * dt_sum));
+  }
+}
+
+// The carry between the passes: a thread owns one entry of a head's state and walks the pieces, four of them on their way at a time.
+// Bound by memory (each piece's state is read and written once).
+__global__ __launch_bounds__(256) void ssm_carry_kernel(ScanArgs a) {
+  const size_t size = (size_t)a.n_state * a.head_dim;
+  const int blocks = (int)((size + 255) / 256), r = blockIdx.x / blocks, h = blockIdx.y;
+  const int run_len = a.cu_seqlens[r + 1] - a.cu_seqlens[r];
+  const size_t e = (size_t)(blockIdx.x % blocks) * 256 + threadIdx.x;
+  if (run_len <= 0 || e >= size) return;
+  const int pieces = (run_len + a.piece - 1) / a.piece;
+  float* S = a.state + (size_t)a.state_slots[r] * a.state_stride + a.state_off + (size_t)h * size + e;
+  float* PS = a.piece_state + ((size_t)r * a.heads + h) * a.max_pieces * size + e;
+  const float* PD = a.piece_decay + ((size_t)r * a.heads + h) * a.max_pieces;
+  float cur = *S;
+  for (int c0 = 0; c0 < pieces; c0 += 4) {
+    float local[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) local[i] = c0 + i < pieces ? PS[(size_t)(c0 + i) * size] : 0.f;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      if (c0 + i < pieces) {
+        PS[(size_t)(c0 + i) * size] = cur;
+        cur = fmaf(PD[c0 + i], cur, local[i]);
+      }
+  }
+  *S = cur;
+}
+
 // scratch floats a scan of n_req requests whose longest run has max_run tokens needs (0: it runs in one launch)
 extern "C" size_t tp_ssm_scan_scratch(int n_req, int max_run, int heads, int head_dim, int n_state, int* piece_out) {
   int piece = 0;
@@ -469,12 +696,30 @@ extern "C" int tp_ssm_scan(const float* xbc, const float* proj, int proj_stride,
     a.mode = SCAN_DIRECT;
     SCAN_DISPATCH(dim3(n_req, heads, slices));
   } else {
+    // The matrix cores' form reads x, B and C in 16-byte pieces and has whole tiles of 16 columns and 16, 32, 64 or 128 state entries.
+    const bool chunked = head_dim % 16 == 0 && (n_state == 16 || n_state == 32 || n_state == 64 || n_state == 128) &&
+                         ((uintptr_t)xbc & 15) == 0;      // (then every column offset and the rows' stride are multiples of 16 floats)
+    const size_t entries = (size_t)n_state * head_dim;
+    const size_t carry_blocks = (entries + 255) / 256 * n_req;
+    TP_REQUIRE(carry_blocks < 0x7fffffffUL, "ssm_scan: too many requests");
+    const long items = (long)n_req * heads * ((head_dim + SC_P - 1) / SC_P) * a.max_pieces;
+    const dim3 chunk_grid((unsigned)((items + 7) / 8 * 8));
+    TP_REQUIRE(items < 0x7ffffff0L, "ssm_scan: too many pieces");
+#define CHUNK_DISPATCH(OUT_)                                                                                                          \
+  do {                                                                                                                                \
+    if (n_state == 16) hipLaunchKernelGGL((ssm_chunk_kernel<1, OUT_>), chunk_grid, dim3(256), 0, s, a, n_req);                        \
+    else if (n_state == 32) hipLaunchKernelGGL((ssm_chunk_kernel<2, OUT_>), chunk_grid, dim3(256), 0, s, a, n_req);                   \
+    else if (n_state == 64) hipLaunchKernelGGL((ssm_chunk_kernel<4, OUT_>), chunk_grid, dim3(256), 0, s, a, n_req);                   \
+    else hipLaunchKernelGGL((ssm_chunk_kernel<8, OUT_>), chunk_grid, dim3(256), 0, s, a, n_req);                                      \
+  } while (0)
     a.mode = SCAN_LOCAL;
-    SCAN_DISPATCH(dim3(n_req, heads, slices * a.max_pieces));
-    a.mode = SCAN_CARRY;
-    SCAN_DISPATCH(dim3(n_req, heads, slices));
+    if (chunked) CHUNK_DISPATCH(false);
+    else SCAN_DISPATCH(dim3(n_req, heads, slices * a.max_pieces));
+    hipLaunchKernelGGL(ssm_carry_kernel, dim3((unsigned)carry_blocks, heads), dim3(256), 0, s, a);
     a.mode = SCAN_OUTPUT;
-    SCAN_DISPATCH(dim3(n_req, heads, slices * a.max_pieces));
+    if (chunked) CHUNK_DISPATCH(true);
+    else SCAN_DISPATCH(dim3(n_req, heads, slices * a.max_pieces));
+#undef CHUNK_DISPATCH
   }
 #undef SCAN_DISPATCH
 #undef SCAN_LAUNCH

@@ -5,7 +5,7 @@
 // 1 KB of one row) and multiplies them with all rows of x; lanes and then waves are added in a fixed tree.  Two rows: 3,072 x 8,192 18.8 us (5.4 TB/s),
 // 16,384 x 3,072 33 us (6.1), 128,256 x 3,072 234 us (6.7).  The general kernel, which stages x through LDS between barriers and has
 // one weight element a lane in flight, takes 263, 124 (5,120 x 3,072; here 12.6) and 569 us.  At 16 rows the multiply-adds and the
-// reads of x bound it (16,384 x 3,072: 70 us), still a quarter less than the blocks of 64 rows below.
+// reads of x bound it (16,384 x 3,072: 56 us), still a quarter less than the blocks of 64 rows below.
 //
 // From 17 rows on (gemm_f32_mfma_kernel) the matrix cores take float32 operands at 157 TFLOP/s, twice the rate of the vector unit
 // without packed instructions, and need one LDS read for four of them, so one pipeline of two LDS stages is enough.  611 rows:
@@ -42,12 +42,23 @@ __device__ inline float lanes_transpose_sum(float (&v)[NV], int lane) {
 #define FR_WAVES 4
 
 // MC: rows of the block's registers (M <= MC), C: weight rows a block owns.
-template <int MC, int C, bool ACC>
+// NORM: x holds rows before their root-mean-square norm (weight norm_w): the block multiplies them with the norm's weight as it reads
+// them, adds their squares beside the products (it sees every row whole) and scales its sums.
+// GATE: N is the columns of each half of w [gate; up], and out is silu(gate) * up: the block owns C / 2 rows of each half.
+// Decode steps of two rows are a chain of small kernels beside the products, each 5 us of launch and dependent reads, and this work
+// costs the products, which wait for memory, little.  Two rows in a captured chain, separate kernels / here: 16,384 x 3,072 with norm
+// and gate 36.3 / 34.1 us, 5,120 x 3,072 with the norm 15.4 / 13.5; 16 rows 73.9 / 63.2 and 35.3 / 27.3 (with eight weight rows a block,
+// which halve what is read of x: without norm and gate 68.2 -> 56.3 and 28.9 -> 24.7; eight rows of x gain at 16,384 weight rows, 48 ->
+// 40, and lose at 3,072 x 8,192, 24 -> 28: they stay at four).
+template <int MC, int C, bool ACC, bool NORM, bool GATE>
 __global__ __launch_bounds__(256) void gemm_f32_rows_kernel(const float* __restrict__ x, const float* __restrict__ w,
-                                                            float* __restrict__ out, int M, int N, int K) {
+                                                            float* __restrict__ out, int M, int N, int K,
+                                                            const float* __restrict__ norm_w, float eps) {
+  constexpr int OWN = GATE ? C / 2 : C;                // columns of the result a block makes
   __shared__ float part[FR_WAVES][MC * C];
+  __shared__ float squares[FR_WAVES][NORM ? MC : 1];
   const int lane = threadIdx.x % TP_WAVE, wave = threadIdx.x / TP_WAVE;
-  const int n0 = blockIdx.x * C;
+  const int n0 = blockIdx.x * OWN;
   // K in steps of 256 (a wave's load); the steps are dealt to the waves in runs
   const int steps = (K + 255) / 256, per = (steps + FR_WAVES - 1) / FR_WAVES;
   const int s0 = wave * per, s1 = min(steps, s0 + per);
@@ -56,7 +67,10 @@ __global__ __launch_bounds__(256) void gemm_f32_rows_kernel(const float* __restr
   for (int i = 0; i < C * MC; ++i) acc[i] = 0.f;
   const float* wr[C];
 #pragma unroll
-  for (int c = 0; c < C; ++c) wr[c] = w + (size_t)min(n0 + c, N - 1) * K;
+  for (int c = 0; c < C; ++c) wr[c] = w + ((size_t)min(n0 + c % OWN, N - 1) + (GATE && c >= OWN ? N : 0)) * K;
+  float ss[NORM ? MC : 1];
+#pragma unroll
+  for (int m = 0; m < (NORM ? MC : 1); ++m) ss[m] = 0.f;
   f32x4 nw[C];
   auto fetch = [&](int s) {
     const int k = s * 256 + lane * 4;
@@ -72,9 +86,16 @@ __global__ __launch_bounds__(256) void gemm_f32_rows_kernel(const float* __restr
     fetch(s + 1);
     const int k = s * 256 + lane * 4;
     if (k < K) {
+      f32x4 wn = (f32x4)(1.f);
+      if constexpr (NORM) wn = *(const f32x4*)(norm_w + k);
 #pragma unroll
       for (int m = 0; m < MC; ++m) {
-        const f32x4 xv = *(const f32x4*)(x + (size_t)min(m, M - 1) * K + k);
+        f32x4 xv = *(const f32x4*)(x + (size_t)min(m, M - 1) * K + k);
+        if constexpr (NORM) {
+#pragma unroll
+          for (int j = 0; j < 4; ++j) ss[m] = fmaf(xv[j], xv[j], ss[m]);
+          xv *= wn;
+        }
 #pragma unroll
         for (int c = 0; c < C; ++c)
 #pragma unroll
@@ -91,13 +112,29 @@ __global__ __launch_bounds__(256) void gemm_f32_rows_kernel(const float* __restr
     const float t = lanes_transpose_sum<NV>(v, lane);
     if (lane % (TP_WAVE / NV) == 0) part[wave][g * NV + lane / (TP_WAVE / NV)] = t;
   }
+  if constexpr (NORM) {
+    const float t = lanes_transpose_sum<MC>(ss, lane);
+    if (lane % (TP_WAVE / MC) == 0) squares[wave][lane / (TP_WAVE / MC)] = t;
+  }
   __syncthreads();
-  for (int i = threadIdx.x; i < C * MC; i += 256) {
-    const int c = i % C, m = i / C, n = n0 + c;
+  for (int i = threadIdx.x; i < OWN * MC; i += 256) {
+    const int c = i % OWN, m = i / OWN, n = n0 + c;
     if (m >= M || n >= N) continue;
-    float t = part[0][c * MC + m];
+    float rstd = 1.f;
+    if constexpr (NORM) {
+      float t = squares[0][m];
 #pragma unroll
-    for (int v = 1; v < FR_WAVES; ++v) t += part[v][c * MC + m];
+      for (int v = 1; v < FR_WAVES; ++v) t += squares[v][m];
+      rstd = 1.0f / sqrtf(t / (float)K + eps);
+    }
+    auto sum_of = [&](int r) {
+      float t = part[0][r * MC + m];
+#pragma unroll
+      for (int v = 1; v < FR_WAVES; ++v) t += part[v][r * MC + m];
+      return NORM ? t * rstd : t;
+    };
+    float t = sum_of(c);
+    if constexpr (GATE) t = t / (1.0f + expf(-t)) * sum_of(OWN + c);
     float* o = out + (size_t)m * N + n;
     *o = ACC ? *o + t : t;
   }
@@ -213,12 +250,32 @@ __global__ __launch_bounds__(256) void gemm_f32_parts_kernel(const float* __rest
 }
 
 template <int MC, int C>
-static void launch_rows(const float* x, const float* w, float* out, bool acc, int M, int N, int K, hipStream_t s) {
-  const dim3 grid((N + C - 1) / C);
-  if (acc)
-    hipLaunchKernelGGL((gemm_f32_rows_kernel<MC, C, true>), grid, dim3(256), 0, s, x, w, out, M, N, K);
+static void launch_rows(const float* x, const float* w, float* out, bool acc, int M, int N, int K, const float* norm_w, float eps, bool gate,
+                        hipStream_t s) {
+  const int own = gate ? C / 2 : C;
+  const dim3 grid((N + own - 1) / own);
+#define FR_LAUNCH(ACC_, NORM_, GATE_) \
+  hipLaunchKernelGGL((gemm_f32_rows_kernel<MC, C, ACC_, NORM_, GATE_>), grid, dim3(256), 0, s, x, w, out, M, N, K, norm_w, eps)
+  if (norm_w != nullptr && gate) FR_LAUNCH(false, true, true);
+  else if (norm_w != nullptr) FR_LAUNCH(false, true, false);
+  else if (gate) FR_LAUNCH(false, false, true);
+  else if (acc) FR_LAUNCH(true, false, false);
+  else FR_LAUNCH(false, false, false);
+#undef FR_LAUNCH
+}
+
+static void launch_rows(const float* x, const float* w, float* out, bool acc, int M, int N, int K, const float* norm_w, float eps, bool gate,
+                        hipStream_t s) {
+  if (M == 1)
+    launch_rows<1, 4>(x, w, out, acc, M, N, K, norm_w, eps, gate, s);
+  else if (M == 2)
+    launch_rows<2, 4>(x, w, out, acc, M, N, K, norm_w, eps, gate, s);
+  else if (M <= 4)
+    launch_rows<4, 4>(x, w, out, acc, M, N, K, norm_w, eps, gate, s);
+  else if (M <= 8)
+    launch_rows<8, 4>(x, w, out, acc, M, N, K, norm_w, eps, gate, s);
   else
-    hipLaunchKernelGGL((gemm_f32_rows_kernel<MC, C, false>), grid, dim3(256), 0, s, x, w, out, M, N, K);
+    launch_rows<16, 8>(x, w, out, acc, M, N, K, norm_w, eps, gate, s);
 }
 
 template <int T>
@@ -263,16 +320,8 @@ int tp_linear_f32(const float* x, const float* w, float* out, int accumulate, in
                   size_t scratch_floats, hipStream_t s) {
   if (K % 4 != 0 || ((uintptr_t)x | (uintptr_t)w) % 16 != 0) return -1;
   const bool acc = accumulate != 0;
-  if (M == 1)
-    launch_rows<1, 4>(x, w, out, acc, M, N, K, s);
-  else if (M == 2)
-    launch_rows<2, 4>(x, w, out, acc, M, N, K, s);
-  else if (M <= 4)
-    launch_rows<4, 4>(x, w, out, acc, M, N, K, s);
-  else if (M <= 8)
-    launch_rows<8, 4>(x, w, out, acc, M, N, K, s);
-  else if (M <= 16)
-    launch_rows<16, 4>(x, w, out, acc, M, N, K, s);
+  if (M <= 16)
+    launch_rows(x, w, out, acc, M, N, K, nullptr, 0.f, false, s);
   else {
     int tile, splits;
     f32_plan(M, N, K, true, &tile, &splits);
@@ -291,5 +340,16 @@ int tp_linear_f32(const float* x, const float* w, float* out, int accumulate, in
     }
   }
   TP_CHECK_LAUNCH("linear (float32)");
+  return 0;
+}
+
+// A product of at most 16 rows with what stands around it: x [M, K] before its norm (norm_w [K], eps; null: as it is); gate != 0: w [2 N, K] holds gate rows and then up rows, and out [M, N] is silu(gate) * up.
+extern "C" int tp_linear_f32_rows(const float* x, const float* w, float* out, int M, int N, int K, const float* norm_w, float eps, int gate,
+                                  hipStream_t s) {
+  TP_REQUIRE(M >= 0 && M <= 16 && N > 0 && K > 0 && K % 4 == 0, "linear_f32_rows: bad sizes (%d x %d x %d)", M, N, K);
+  TP_REQUIRE((((uintptr_t)x | (uintptr_t)w | (uintptr_t)norm_w) & 15) == 0, "linear_f32_rows: misaligned operand");
+  if (M == 0) return 0;
+  launch_rows(x, w, out, false, M, N, K, norm_w, eps, gate != 0, s);
+  TP_CHECK_LAUNCH("linear_f32_rows");
   return 0;
 }

@@ -443,6 +443,20 @@ class Prenormed:
         return self.x.permute(1, 0, 2).reshape(m, k)
 
 
+class Unnormed:
+    """float32 rows whose root-mean-square norm is left to the products that consume them: ``x`` [m, k] as it stands, the norm's
+    ``weight`` [k] and ``eps`` (``norm_in_product_ok`` says for which sizes).  ``x`` must not change before they have run."""
+    __slots__ = ("x", "weight", "eps")
+    dtype = torch.float32
+
+    def __init__(self, x, weight, eps):
+        self.x, self.weight, self.eps = x, weight, float(eps)
+
+    @property
+    def shape(self):
+        return self.x.shape
+
+
 class KBlocked:
     """bfloat16 activations of at most 16 rows stored k-blocked, ``data`` [k / 8, m, 8]: eight consecutive
     columns of all rows side by side.  A product of a few rows that reads its activations straight from
@@ -643,9 +657,43 @@ def _splitk_scratch(x: torch.Tensor, m: int, n: int):
     return torch.empty((count,), dtype=torch.float32, device=x.device), count
 
 
+def norm_in_product_ok(x: torch.Tensor, dtype: torch.dtype) -> bool:
+    """Whether the products behind a norm of the rows ``x`` may norm them themselves (``Unnormed``)."""
+    # (float32, all rows that the product reading each weight once takes, so that a row's bits do not depend on the rows beside it.
+    # 5,120 x 3,072, a captured chain, norm and product apart / together: 1 row 14.8 / 12.7 us, 4 rows 17.4 / 15.6, 16 rows 28.4 / 27.3)
+    return _backend is None and allow_mfma and dtype == x.dtype == torch.float32 and x.dim() == 2 and 0 < x.shape[0] <= 16 and \
+        x.shape[1] % 4 == 0 and x.data_ptr() % 16 == 0 and x.is_contiguous()
+
+
+def linear_gate_f32_ok(x, w) -> bool:
+    """Whether ``linear_gate_f32`` takes the rows ``x`` and the weight ``w`` [gate; up]."""
+    return _backend is None and allow_mfma and isinstance(w, torch.Tensor) and x.dtype == w.dtype == torch.float32 and \
+        0 < x.shape[0] <= 16 and x.shape[1] % 4 == 0 and w.shape[0] % 2 == 0 and w.data_ptr() % 16 == 0 and \
+        (isinstance(x, Unnormed) or (x.data_ptr() % 16 == 0 and x.is_contiguous()))
+
+
+def _f32_rows(x, w: torch.Tensor, gate: bool) -> torch.Tensor:
+    rows, weight, eps = (x.x, x.weight, x.eps) if isinstance(x, Unnormed) else (x, None, 0.0)
+    _dev_ok(rows, weight, w)
+    (m, k), n = rows.shape, w.shape[0] // (2 if gate else 1)
+    _need(w.dim() == 2 and w.shape[1] == k and w.dtype == torch.float32, f"linear: shapes {(m, k)} x {tuple(w.shape)}")
+    _need(weight is None or (weight.dtype == torch.float32 and weight.numel() == k), "linear: norm weight must be float32 [k]")
+    out = torch.empty((m, n), dtype=torch.float32, device=rows.device)
+    _call("tp_linear_f32_rows", _ptr(rows), _ptr(w), _ptr(out), m, n, k, _ptr(weight), ctypes.c_float(eps), int(gate), _stream(),
+          tag=(m, w.shape[0], k))
+    return out
+
+
+def linear_gate_f32(x, w: torch.Tensor) -> torch.Tensor:
+    """float32 x [m, k] (or ``Unnormed``), weight [2 i, k] of gate rows and then up rows -> float32 [m, i] = silu(x g^T) * (x u^T):
+    ``swiglu`` of ``linear`` in one launch for at most 16 rows (``linear_gate_f32_ok``)."""
+    _need(linear_gate_f32_ok(x, w), "linear_gate_f32: needs float32 operands of at most 16 rows")
+    return _f32_rows(x, w, True)
+
+
 def linear(x, w: torch.Tensor, out_dtype: torch.dtype, residual: Optional[torch.Tensor] = None, next_norm=None,
            partial_ok: bool = False):
-    """x [m, k] (or ``Prenormed`` / ``KBlocked``) @ w[n, k]^T -> out_dtype [m, n]; with ``residual`` (float32
+    """x [m, k] (or ``Prenormed`` / ``KBlocked`` / ``Unnormed`` without a residual) @ w[n, k]^T -> out_dtype [m, n]; with ``residual`` (float32
     [m, n]) the product is added into it in place and it is returned.
     With ``next_norm`` = (float32 weight [n], eps) (needs ``residual``) the result is the pair (residual, rows
     for the part behind that norm): ``Prenormed`` rows up to 16 rows of bfloat16, the normed rows themselves
@@ -658,6 +706,10 @@ def linear(x, w: torch.Tensor, out_dtype: torch.dtype, residual: Optional[torch.
         return _backend.linear(x, w, out_dtype, residual)
     layout = 0
     wd, wl = _w_args(w)
+    if isinstance(x, Unnormed):
+        if isinstance(w, torch.Tensor) and residual is None and next_norm is None and out_dtype == torch.float32 and w.data_ptr() % 16 == 0:
+            return _f32_rows(x, w, False)
+        x = rmsnorm(x.x, x.weight, x.eps, torch.float32)
     if isinstance(x, KBlocked):
         _need(allow_mfma and x.data.dtype == torch.bfloat16 and tuple(x.data.shape) == (x.width // 8, x.rows, 8)
               and x.width % 32 == 0, "linear: malformed k-blocked rows")

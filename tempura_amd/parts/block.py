@@ -78,7 +78,7 @@ class PreNormBlock(ArrangedBlock):
         """``x``: rows handed over by the block before (its last product prepared ``mixer_norm``);
         ``next_norm``: the ``entry_norm`` of the block after.  Returns the rows handed to that block, or None."""
         if x is None:
-            x = self.mixer_norm.forward(h)
+            x = self._normed(self.mixer_norm, self.mixer, h)
         x2 = None
         if getattr(self.mixer, "split_norm", False):
             mid = None
@@ -88,11 +88,20 @@ class PreNormBlock(ArrangedBlock):
         else:
             self.mixer.forward(x, ctx, cache, h)
         if x2 is None:
-            x2 = self.ffn_norm.forward(h)
+            x2 = self._normed(self.ffn_norm, self.ffn, h)
         if next_norm is not None and getattr(self.ffn, "split_norm", False):
             return self.ffn.forward(x2, ctx, h, next_norm=next_norm)
         self.ffn.forward(x2, ctx, h)
         return None
+
+    @staticmethod
+    def _normed(norm, part, h):
+        """The rows for ``part``: normed, or with their norm left to its first products (which read them before it adds to ``h``)."""
+        if getattr(part, "split_norm", False) and hasattr(norm, "unapplied"):
+            x = norm.unapplied(h)
+            if x is not None:
+                return x
+        return norm.forward(h)
 
 
 register_part("block", "prenorm", PreNormBlock)

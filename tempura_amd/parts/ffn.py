@@ -45,6 +45,8 @@ class SwiGLU(FeedForward):
         if self.fused:
             # (a few rows go to the next product k-blocked: it reads them straight from global memory)
             a = ops.linear_swiglu(x, self.w13, blocked_out=True)
+        elif self.dtype == torch.float32 and ops.linear_gate_f32_ok(x, self.w13):
+            a = ops.linear_gate_f32(x, self.w13)
         else:
             gu = ops.linear(x, self.w13, torch.float32)
             a = ops.swiglu(gu, self.dtype)

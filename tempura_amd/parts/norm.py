@@ -64,5 +64,11 @@ class RMSNorm(Norm):
             return self.weight, self.eps
         return None
 
+    def unapplied(self, h):
+        """The rows ``h`` with this norm left to the products that read them (``ops.Unnormed``), or None."""
+        if self.groups == 1 and ops.norm_in_product_ok(h, self.dtype):
+            return ops.Unnormed(h, self.weight, self.eps)
+        return None
+
 
 register_part("norm", "rmsnorm", RMSNorm)

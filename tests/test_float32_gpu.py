@@ -48,6 +48,35 @@ def test_float32_products(m, n, k):
     assert off.data_ptr() % 16 != 0 and _rel(ops.linear(off, wd, torch.float32), ref) < tol
 
 
+@pytest.mark.parametrize("m", [1, 2, 3, 4, 5, 8, 9, 16])
+@pytest.mark.parametrize("n,k", [(3, 4), (130, 260), (1026, 3072)])
+def test_float32_products_norm_and_gate_their_rows(m, n, k):
+    """Rows before their norm and gate/up sums of a few rows: against float64 with the bound above (the norm and the gate add a few
+    roundings), no further from it than the separate kernels, and a row's bits the same whatever rows stand beside it."""
+    from tempura_amd.kernels import ops
+    g = torch.Generator().manual_seed(m + n + k)
+    x, w, wn = torch.randn(m, k, generator=g) * 3, torch.randn(2 * n, k, generator=g) * k ** -0.5, torch.rand(k, generator=g) + 0.5
+    xd, wd, nd = x.to(DEV), w.to(DEV), wn.to(DEV)
+    normed = x.double() / (x.double().pow(2).mean(-1, keepdim=True) + 1e-5).sqrt() * wn.double()
+    rows = ops.Unnormed(xd, nd, 1e-5)
+    assert ops.norm_in_product_ok(xd, torch.float32) and ops.linear_gate_f32_ok(rows, wd) and ops.linear_gate_f32_ok(xd, wd)
+    tol = 2.0 ** -24 * max(8.0, math.sqrt(k))      # (a silu of a gate's sum, their product and the norm: up to eight roundings at few k)
+
+    def gated(v):
+        return torch.nn.functional.silu(v[:, :n]) * v[:, n:]
+
+    apart = ops.linear(ops.rmsnorm(xd, nd, 1e-5, torch.float32), wd, torch.float32)
+    for got, ref, old in ((ops.linear(rows, wd, torch.float32), normed @ w.double().T, apart),
+                          (ops.linear_gate_f32(rows, wd), gated(normed @ w.double().T), ops.swiglu(apart, torch.float32))):
+        assert _rel(got, ref) < tol
+        if k > 4:      # (a few results of four terms, which share their row's scale, say little about which way is nearer)
+            assert _rel(got, ref) <= 1.2 * _rel(old, ref) + 2.0 ** -25
+    assert torch.equal(ops.linear_gate_f32(xd, wd), ops.swiglu(ops.linear(xd, wd, torch.float32), torch.float32))
+    few = ops.Unnormed(xd[: m // 2 + 1].contiguous(), nd, 1e-5)
+    assert torch.equal(ops.linear(few, wd, torch.float32), ops.linear(rows, wd, torch.float32)[: m // 2 + 1])
+    assert torch.equal(ops.linear_gate_f32(few, wd), ops.linear_gate_f32(rows, wd)[: m // 2 + 1])
+
+
 @pytest.mark.parametrize("what", ["plain", "window", "kept", "chunk", "cap", "bias", "sink"])
 @pytest.mark.parametrize("heads,kv,d,page,q_lens,ctx_lens", [
     (6, 2, 64, 16, [37, 1, 20], [37, 90, 200]),                    # portions beside a single token

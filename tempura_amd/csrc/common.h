@@ -86,6 +86,7 @@ struct GateAct {
   // activated output, and where the other columns go
   int act_cols, act_ld, side_ld;
   float* side;
+  int act_kind1;             // (products of at most 16 rows: one more than another activation's kind, activations.h; 0: max(v, 0)^2)
 };
 
 struct RopeOut {

@@ -194,7 +194,8 @@ extern "C" int tp_linear_rope(const void* x, const void* w, int w_tiled, int M, 
 //
 // accumulate == 3 (bfloat16, K % 64 == 0): the first act_cols columns (a multiple of 128) become max(v, 0)^2, bfloat16
 // [M, act_cols] in `out` (bit 1 of `layout`, at most 16 rows: k-blocked [act_cols / 8, M, 8]), the others float32
-// [M, N - act_cols] in `side`.
+// [M, N - act_cols] in `side`.  Bits 8 to 10 of `layout` (at most 16 rows): one more than the kind of another activation
+// (activations.h) in place of the squared ReLU.
 //
 // `defer_reduce` (products of more than 16 rows whose K is split over blocks): the partial sums stay in `scratch`
 // as [*splits_out, M, N] float32 and `out` is not touched; the caller's next kernel adds them (ascending).
@@ -207,6 +208,8 @@ extern "C" int tp_linear_fused(const void* x, const void* w, int in_dt, void* ou
   if (splits_out) *splits_out = 1;
   TP_REQUIRE(M >= 0 && N > 0 && K > 0, "linear: bad sizes M=%d N=%d K=%d", M, N, K);
   TP_REQUIRE(accumulate != 1 || out_dt == TP_F32, "linear: accumulating output must be float32");
+  const int act_kind1 = layout >> 8;      // (see accumulate == 3)
+  layout &= 255;
   const bool split_norm = pre_ss != nullptr || post_w != nullptr || (layout & 3) != 0;
   TP_REQUIRE((layout & ~15) == 0 && (!(layout & 2) || accumulate == 2 || accumulate == 3) && (!(layout & 8) || post_w != nullptr),
              "linear: bad layout flags %d", layout);
@@ -236,6 +239,8 @@ extern "C" int tp_linear_fused(const void* x, const void* w, int in_dt, void* ou
     gate.act_ld = act_cols;
     gate.side = side;
     gate.side_ld = N - act_cols;
+    gate.act_kind1 = act_kind1;
+    TP_REQUIRE(act_kind1 >= 0 && act_kind1 <= 4 && (act_kind1 == 0 || M <= 16), "linear: unknown activation %d at %d rows", act_kind1 - 1, M);
     if (M == 0) return 0;
     const int r = tp_linear_mfma(x, w, out, out_dt, 3, M, N, K, scratch, scratch_floats, pre_ss, pre_count, pre_eps, nullptr, nullptr,
                                  nullptr, layout, 0, nullptr, gate, s);

@@ -15,6 +15,7 @@
 // Fragment layout of the 16x16x32 instruction: lane l holds row (l % 16) of its operand
 // and 8 consecutive k at (l / 16) * 8; the result lane l holds rows (l / 16) * 4 + r,
 // r = 0..3, of column l % 16.
+#include "activations.h"
 #include "common.h"
 
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
@@ -28,8 +29,9 @@ enum { OUT_F32 = 0, OUT_BF16 = 1, OUT_ACC_F32 = 2, OUT_SWIGLU = 3 };
 
 __device__ inline bf16x8_t as_frag(u32x4_t v) { return __builtin_bit_cast(bf16x8_t, v); }
 
-// the gated SiLU without constants: the products of a few rows have only this gate (their time is the weights'
-// stream, and the general gate's constants in their epilogue cost them half a microsecond a call, measured)
+// the gated SiLU without constants: the products of a few rows have only this gate in their common kernels (their time is the weights'
+// stream, and the general gate's constants in the epilogue cost every one of them half a microsecond, measured); with constants they take
+// the kernels of the split epilogue
 __device__ inline float silu_mul(float g, float u) {
   return g * u * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(g * -1.4426950408889634f));
 }
@@ -70,7 +72,7 @@ __device__ inline void store_out(void* out, int mode, size_t idx, float v) {
 // mode OUT_SPLIT (see GateAct); layout OUT_KBLOCKED: the activated columns k-blocked
 __device__ inline void store_split(void* out, int layout, const GateAct& ga, int M, int m, int n, float v) {
   if (n < ga.act_cols)
-    store_gated(out, layout, M, ga.act_ld, m, n, relu_squared(v));
+    store_gated(out, layout, M, ga.act_ld, m, n, ga.act_kind1 == 0 ? relu_squared(v) : act_f(v, ga.act_kind1 - 1));
   else
     ga.side[(size_t)m * ga.side_ld + n - ga.act_cols] = v;
 }
@@ -169,7 +171,10 @@ __device__ inline void row_scale_finish(const RowScale& pre, const RowScaleLoads
 // MT: 16-row tiles of activations; NT: 16-row tiles of weights per block; WAVES: waves that
 // split K.  A wave takes K in runs of four consecutive 32-wide steps (256 contiguous bytes of
 // each weight row), run r going to wave r % WAVES.
-// SPLIT: mode OUT_SPLIT, in kernels of its own (its branch in the others' epilogue costs every short product half a microsecond)
+// SPLIT: mode OUT_SPLIT, or OUT_SWIGLU with a gate that has constants, in kernels of their own (these branches in the others' epilogue
+// cost every short product half a microsecond).  The activation's own launch and trip through memory, 4.9 us behind a product of one
+// row, is gone: both products of a feed-forward, 16,384 x 4,096, one row 48.1 -> 46.0 us (gate with constants 66.9 -> 64.8), 16 rows
+// 56.4 -> 53.5 (83.9 -> 74.7: the down product takes k-blocked rows as well).
 template <int MT, int NT, int WAVES, int DEPTH, bool WT, bool SPLIT>
 __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_mfma_kernel(const bf16_t* __restrict__ x,
                                                                       const bf16_t* __restrict__ w,
@@ -256,15 +261,15 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_mfma_kernel(const bf16
     const int n = n0 + j * 16 + (l >> 4) * 4 + r;   // weight row = output column
     const int m = t * 16 + (l & 15);
     if (MT == 1) v *= rstd[l & 15];
-    if constexpr (SPLIT) {
+    if (SPLIT && mode == OUT_SPLIT) {
       if (n < N && m < M) store_split(out, layout, rp.gate, M, m, n, v);
-    } else if (mode == OUT_SWIGLU) {
+    } else if (SPLIT || mode == OUT_SWIGLU) {
       if ((l >> 4) < 2 && n + 8 < N && m < M) {       // a gate row: its up row is eight further on
         float u = 0.f;
 #pragma unroll
         for (int i = 0; i < WAVES; ++i) u += red[i][jt][q + 128];
         if (MT == 1) u *= rstd[l & 15];
-        store_gated(out, layout, M, N / 2, m, (n0 + j * 16) / 2 + (l >> 4) * 4 + r, silu_mul(v, u));
+        store_gated(out, layout, M, N / 2, m, (n0 + j * 16) / 2 + (l >> 4) * 4 + r, SPLIT ? gate_mul(v, u, rp.gate) : silu_mul(v, u));
       }
     } else if (MT == 1 && post.w != nullptr) {
       // residual add, and the next norm's preparation (mode is OUT_ACC_F32)
@@ -415,15 +420,15 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_lds_kernel(const bf16_
     const int n = nt0 + (l >> 4) * 4 + r;
     const int m = l & 15;
     v *= rstd[m];
-    if constexpr (SPLIT) {
+    if (SPLIT && mode == OUT_SPLIT) {
       if (n < N && m < M) store_split(out, layout, rp.gate, M, m, n, v);
-    } else if (mode == OUT_SWIGLU) {
+    } else if (SPLIT || mode == OUT_SWIGLU) {
       if ((l >> 4) < 2 && n + 8 < N && m < M) {
         float u = 0.f;
 #pragma unroll
         for (int i = 0; i < WAVES; ++i) u += red[ge * WAVES + i][j][q + 128];
         u *= rstd[m];
-        store_gated(out, layout, M, N / 2, m, nt0 / 2 + (l >> 4) * 4 + r, silu_mul(v, u));
+        store_gated(out, layout, M, N / 2, m, nt0 / 2 + (l >> 4) * 4 + r, SPLIT ? gate_mul(v, u, rp.gate) : silu_mul(v, u));
       }
     } else if (post.w != nullptr) {
       float sq = 0.f;
@@ -713,6 +718,10 @@ extern "C" void tp_linear_tune(int waves, int nt, int depth) {
   g_tune_depth = depth;
 }
 
+static bool gate_has_constants(const GateAct& g) { return g.extra_slope != 0.f || g.limit > 0.f || g.offset != 0.f; }
+// whether a product of a few rows takes the kernels of the split epilogue (see SPLIT)
+static bool split_epilogue(int mode, const GateAct& g) { return mode == OUT_SPLIT || (mode == OUT_SWIGLU && gate_has_constants(g)); }
+
 template <int MT, int NT, int WAVES, int DEPTH>
 static void launch_skinny4(const bf16_t* x, const bf16_t* w, void* out, int mode, int M, int N, int K, int layout,
                            RowScale pre, NormPrep post, const RopeOut& rp, hipStream_t s) {
@@ -720,7 +729,7 @@ static void launch_skinny4(const bf16_t* x, const bf16_t* w, void* out, int mode
 #define SKINNY(WT_, SPLIT_)                                                                                                              \
   hipLaunchKernelGGL((gemm_skinny_mfma_kernel<MT, NT, WAVES, DEPTH, WT_, SPLIT_>), dim3(blocks), dim3(WAVES * 64), 0, s, x, w, out, mode, \
                      M, N, K, layout, pre, post, rp)
-  if (mode == OUT_SPLIT) {
+  if (split_epilogue(mode, rp.gate)) {
     if (layout & W_TILED) SKINNY(true, true);
     else SKINNY(false, true);
   } else if (layout & W_TILED) {
@@ -757,7 +766,7 @@ static void launch_skinny(const bf16_t* x, const bf16_t* w, void* out, int mode,
       const bool wt = (layout & W_TILED) != 0;
 #define LDS_CASE(NT_, WT_)                                                                                                                     \
   do {                                                                                                                                         \
-    if (mode == OUT_SPLIT)                                                                                                                     \
+    if (split_epilogue(mode, rp.gate))                                                                                                         \
       hipLaunchKernelGGL((gemm_skinny_lds_kernel<NT_, 8, WT_, true>), dim3(blocks), dim3(512), 0, s, x, w, out, mode, M, N, K, layout, pre,    \
                          post, rp);                                                                                                            \
     else                                                                                                                                       \
@@ -856,8 +865,6 @@ int tp_linear_mfma(const void* x, const void* w, void* out, int out_dt, int accu
   RopeOut no_rope = {};
   no_rope.gate = gate;      // (the kernels read the gated epilogue's constants from here)
   if (M <= 16 || (M <= 64 && !mid_ok)) {
-    // (a gate with constants is not these kernels': the caller runs the product and the activation as two steps)
-    if (mode == OUT_SWIGLU && (gate.extra_slope != 0.f || gate.limit > 0.f || gate.offset != 0.f)) return -1;
     if (M <= 16)
       launch_skinny<1>(xb, wb, out, mode, M, N, K, layout, pre, post, no_rope, s);
     else if (M <= 32)

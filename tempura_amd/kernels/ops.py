@@ -402,11 +402,6 @@ def rmsnorm(h: torch.Tensor, weight: torch.Tensor, eps: float, out_dtype: torch.
 allow_mfma = True
 
 
-#: a gate with constants of its own runs in the product's epilogue from this many rows on (the products of fewer
-#: rows stream the weights once and have the plain gated SiLU only)
-gated_epilogue_rows = 17
-
-
 def gated_layout_ok(n_rows: int, k: int) -> bool:
     """Whether ``linear_swiglu`` takes a weight of 2 * n_rows rows and k columns."""
     return n_rows % 8 == 0 and k % 32 == 0
@@ -579,8 +574,7 @@ def linear_swiglu(x, w: torch.Tensor, blocked_out: bool = False, slope: float = 
     silu(x g^T) * (x u^T), the gate applied to the float32 accumulators (no rounding in between).
     With ``blocked_out`` the result comes as ``KBlocked`` when there are at most 16 rows and i % 32 == 0 (else as a tensor).
     ``slope``, ``limit``, ``up_offset``: the general gate of ``gated_act`` (g' * sigmoid(slope g') * (u' + up_offset)
-    with both branches limited when limit > 0) in the same epilogue; the defaults are SwiGLU.  The products of at
-    most 16 rows have the default gate only (``gated_epilogue_rows``)."""
+    with both branches limited when limit > 0) in the same epilogue; the defaults are SwiGLU."""
     if _backend is not None:
         if (slope, limit, up_offset) != (1.0, 0.0, 0.0):
             return _backend.linear_swiglu(x, w, blocked_out, slope, limit, up_offset)
@@ -611,12 +605,19 @@ def linear_relu2_ok(act_cols: int, k: int, dtype: torch.dtype) -> bool:
     return allow_mfma and dtype == torch.bfloat16 and k % 64 == 0 and act_cols % 128 == 0
 
 
-def linear_relu2(x: torch.Tensor, w, act_cols: int, blocked_out: bool = False):
+def linear_act_ok(m: int, act_cols: int, k: int, dtype: torch.dtype) -> bool:
+    """Whether ``linear_relu2`` takes ``m`` rows with another activation than the squared ReLU: the products of at most 16 rows."""
+    return _backend is None and 0 < m <= 16 and linear_relu2_ok(act_cols, k, dtype)
+
+
+def linear_relu2(x: torch.Tensor, w, act_cols: int, blocked_out: bool = False, kind: str = "relu2"):
     """bfloat16 x [m, k], weight [n, k] -> (bfloat16 [m, act_cols] = max(x w^T, 0)^2 of the first ``act_cols`` columns, the
     activation applied to the float32 accumulators; float32 [m, n - act_cols], the other columns as they are).  With
-    ``blocked_out`` the first comes as ``KBlocked`` when there are at most 16 rows.  Sizes: ``linear_relu2_ok``."""
+    ``blocked_out`` the first comes as ``KBlocked`` when there are at most 16 rows.  Sizes: ``linear_relu2_ok``.
+    ``kind``: another of ``ACTIVATIONS`` in its place (``linear_act_ok``)."""
     if _backend is not None:
         return _backend.linear_relu2(x, w, act_cols, blocked_out)
+    _need(kind == "relu2" or linear_act_ok(tuple(x.shape)[0], act_cols, tuple(x.shape)[1], torch.bfloat16), "linear_relu2: another activation takes at most 16 rows")
     wd, wl = _w_args(w)
     shape, xl = tuple(x.shape), 0
     if isinstance(x, KBlocked):
@@ -635,8 +636,8 @@ def linear_relu2(x: torch.Tensor, w, act_cols: int, blocked_out: bool = False):
     side = torch.empty((m, n - act_cols), dtype=torch.float32, device=x.device)
     scratch, nscratch = _splitk_scratch(x, m, n)
     _call("tp_linear_fused", _ptr(x), _ptr(wd), _BF16, _ptr(out.data if blocked_out else out), _BF16, 3, m, n, k, 1, _ptr(scratch),
-          ctypes.c_size_t(nscratch), _ptr(None), 0, ctypes.c_float(0.0), _ptr(None), _ptr(None), _ptr(None), (2 if blocked_out else 0) | wl | xl,
-          0, _ptr(None), ctypes.c_float(1.0), ctypes.c_float(0.0), ctypes.c_float(0.0), int(act_cols), _ptr(side), _stream(), tag=(m, n, k))
+          ctypes.c_size_t(nscratch), _ptr(None), 0, ctypes.c_float(0.0), _ptr(None), _ptr(None), _ptr(None),
+          (2 if blocked_out else 0) | wl | xl | ((0 if kind == "relu2" else ACTIVATIONS[kind] + 1) << 8), 0, _ptr(None), ctypes.c_float(1.0), ctypes.c_float(0.0), ctypes.c_float(0.0), int(act_cols), _ptr(side), _stream(), tag=(m, n, k))
     return out, side
 
 

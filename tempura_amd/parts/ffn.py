@@ -98,10 +98,11 @@ class GatedFFN(FeedForward):
         self.w2 = ops.tile_weight(self._to_device(get(w["down"])))
 
     def forward(self, x, ctx, residual=None):
-        if self.fused and x.shape[0] >= ops.gated_epilogue_rows:
-            a = ops.linear_swiglu(x, self.w13, slope=self.slope, limit=self.limit, up_offset=self.up_offset)
+        if self.fused:
+            # (a few rows go to the down product k-blocked: it reads them straight from global memory)
+            a = ops.linear_swiglu(x, self.w13, blocked_out=True, slope=self.slope, limit=self.limit, up_offset=self.up_offset)
         else:
-            # (a few rows, or sizes the fused product does not take: the product's float32 sums, then the activation)
+            # (sizes the fused product does not take: the product's float32 sums, then the activation)
             gu = ops.linear(x, self.w13, torch.float32)
             a = ops.gated_act(gu, self.dtype, self.slope, self.limit, self.up_offset, interleaved=self.fused)
         return ops.linear(a, self.w2, torch.float32, residual=residual)
@@ -110,7 +111,7 @@ class GatedFFN(FeedForward):
 class DenseMLP(FeedForward):
     """``down(act(up(x)))`` without a gate; ``activation`` names the function (``ops.ACTIVATIONS``: ``gelu_tanh``, ``silu``,
     ``relu2``, ..), which reads the float32 sums of the up product: in the product's own epilogue for ``relu2`` in bfloat16
-    (sizes ``ops.linear_relu2_ok``), else as a kernel of its own."""
+    (sizes ``ops.linear_relu2_ok``) and for every kind in steps of at most 16 rows, else as a kernel of its own."""
     graph_safe = True
     takes_side_rows = True     # (behind the up product's own columns)
     takes_blocked_rows = True
@@ -140,9 +141,9 @@ class DenseMLP(FeedForward):
         self.w_down = ops.tile_weight(self._to_device(get(w["down"])))
 
     def forward(self, x, ctx, residual=None):
-        if self.fused:
+        if self.fused or ops.linear_act_ok(x.shape[0], self.intermediate_size, self.hidden_size, self.dtype):
             # (a few rows go to the down product k-blocked: it reads them straight from global memory)
-            a, side = ops.linear_relu2(x, self.w_up, self.intermediate_size, blocked_out=True)
+            a, side = ops.linear_relu2(x, self.w_up, self.intermediate_size, blocked_out=True, **({} if self.fused else {"kind": self.activation}))
             y = ops.linear(a, self.w_down, torch.float32, residual=residual)
             return y if self.side_rows is None else (y, (side, 0))
         u = ops.linear(x, self.w_up, torch.float32)

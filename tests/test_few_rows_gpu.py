@@ -169,3 +169,39 @@ def test_moe_linear(counts, n, k, tiled, output):
         gate, up = pair[:, :, 0].reshape(pairs, -1), pair[:, :, 1].reshape(pairs, -1)
         _close(got, gate * torch.sigmoid(gate) * up, 8e-3)
     assert torch.equal(got, ops.moe_linear(x.to(DEV), wd, offsets.to(DEV), E, output))
+
+
+@pytest.mark.parametrize("m", [1, 2, 7, 16])
+@pytest.mark.parametrize("act_cols,side,k", [(128, 0, 64), (256, 16, 2048), (384, 48, 8192)])
+@pytest.mark.parametrize("kind", ["gelu_tanh", "silu", "gelu_erf"])
+def test_up_products_of_a_few_rows_leave_activated(m, act_cols, side, k, kind):
+    """The activation in the product's epilogue and the activation's own kernel see the same float32 sums: the same bits."""
+    from tempura_amd.kernels import ops
+    g = torch.Generator().manual_seed(m + k)
+    x = torch.randn(m, k, generator=g).to(torch.bfloat16).to(DEV)
+    w = ops.tile_weight((torch.randn(act_cols + side, k, generator=g) * 2 * k ** -0.5).to(torch.bfloat16).to(DEV))
+    assert ops.linear_act_ok(m, act_cols, k, torch.bfloat16) and not ops.linear_act_ok(17, act_cols, k, torch.bfloat16)
+    sums = ops.linear(x, w, torch.float32)
+    want = ops.activation(sums, kind, torch.bfloat16, 0, act_cols)
+    got, beside = ops.linear_relu2(x, w, act_cols, kind=kind)
+    assert torch.equal(got, want) and torch.equal(beside, sums[:, act_cols:])
+    blocked, _ = ops.linear_relu2(x, w, act_cols, blocked_out=True, kind=kind)
+    assert torch.equal(blocked.data.permute(1, 0, 2).reshape(m, act_cols), want)
+
+
+@pytest.mark.parametrize("m", [1, 3, 16])
+@pytest.mark.parametrize("n,k", [(16, 64), (272, 2048), (528, 8192)])
+@pytest.mark.parametrize("slope,limit,offset", [(1.702, 7.0, 1.0), (1.0, 0.5, 0.0), (1.0, 0.0, 0.5)])
+def test_gated_products_of_a_few_rows_take_the_gates_constants(m, n, k, slope, limit, offset):
+    """Against the activation of the same float32 sums (a rounding to bfloat16 and the hardware's exponential and reciprocal: 2^-8)."""
+    from tempura_amd.kernels import ops
+    g = torch.Generator().manual_seed(m + n)
+    x = torch.randn(m, k, generator=g).to(torch.bfloat16).to(DEV)
+    w = ops.tile_weight((torch.randn(n, k, generator=g) * 3 * k ** -0.5).to(torch.bfloat16).to(DEV))
+    want = ops.gated_act(ops.linear(x, w, torch.float32), torch.float32, slope, limit, offset, interleaved=True)
+    got = ops.linear_swiglu(x, w, slope=slope, limit=limit, up_offset=offset)
+    assert float((got.float() - want).abs().max()) <= 2.0 ** -8 * float(want.abs().max())
+    blocked = ops.linear_swiglu(x, w, True, slope, limit, offset)
+    if isinstance(blocked, ops.KBlocked):
+        blocked = blocked.data.permute(1, 0, 2).reshape(m, n // 2)
+    assert torch.equal(blocked, got)

@@ -223,6 +223,7 @@ struct ScanArgs {
   int heads, head_dim, n_state, groups, channels;
   int R, TC;
   int mode, piece, max_pieces;
+  int unit;             // heads that share B and C and run side by side (ssm_chunk_kernel)
   float* piece_state;   // [request, head, piece, n_state, head_dim]
   float* piece_decay;   // [request, head, piece]
 };
@@ -374,7 +375,7 @@ __global__ __launch_bounds__(256) void ssm_scan_kernel(ScanArgs a) {
 // worked out once a block (one 16 x 16 tile a wave) and passed through LDS with its weights; the tile above the diagonal is left out.
 // Sums over the state are added in runs of eight products: longer chains of roundings would lose to the walk's, which adds 16 a lane
 // and then the lanes in a tree.
-// Items go to the XCDs in contiguous shares, heads fastest: what shares B and C of a piece is on one L2.
+// Up to 16 heads that share B and C of a piece are a unit and go to one XCD and its L2, the units to the XCDs in turn.
 //
 // Bound by the matrix cores: 2,048 tokens of 128 heads of 64 with a state of 128 are 14.5 GFLOP in both passes, 100 us at the float32
 // rate; with the carry 220 us, token by token 656 (257 tokens 72 / 206 us; 32 heads of 64 with a state of 16, 2,048 tokens, 34 / 125).
@@ -393,14 +394,14 @@ __global__ __launch_bounds__(256, OUT && NT == 8 ? 2 : 3) void ssm_chunk_kernel(
   __shared__ double cs[SC_T];
   __shared__ float dts[SC_T], from_start[SC_T], to_end[SC_T];
   const int P = a.head_dim, slices = (P + SC_P - 1) / SC_P;
-  const long total = (long)requests * a.heads * slices * a.max_pieces, share = (total + 7) / 8;
-  long item = (long)(blockIdx.x & 7) * share + (blockIdx.x >> 3);
-  if ((long)(blockIdx.x >> 3) >= share || item >= total) return;
-  const int h = (int)(item % a.heads);
-  item /= a.heads;
+  long item = (long)(blockIdx.x >> 3) / a.unit * 8 + (blockIdx.x & 7);      // (units go to the XCDs in turn)
+  const int units = a.heads / a.unit;
+  const int h = (int)(item % units) * a.unit + (int)(blockIdx.x >> 3) % a.unit;
+  item /= units;
   const int slice = (int)(item % slices);
   item /= slices;
   const int pc = (int)(item % a.max_pieces), r = (int)(item / a.max_pieces);
+  if (r >= requests) return;
   const int run0 = a.cu_seqlens[r], run_len = a.cu_seqlens[r + 1] - run0;
   const int start = run0 + pc * a.piece, len = min(a.piece, run_len - pc * a.piece);
   if (len <= 0) return;
@@ -702,8 +703,10 @@ extern "C" int tp_ssm_scan(const float* xbc, const float* proj, int proj_stride,
     const size_t entries = (size_t)n_state * head_dim;
     const size_t carry_blocks = (entries + 255) / 256 * n_req;
     TP_REQUIRE(carry_blocks < 0x7fffffffUL, "ssm_scan: too many requests");
-    const long items = (long)n_req * heads * ((head_dim + SC_P - 1) / SC_P) * a.max_pieces;
-    const dim3 chunk_grid((unsigned)((items + 7) / 8 * 8));
+    a.unit = heads / groups;
+    while (a.unit > 16 && a.unit % 2 == 0) a.unit /= 2;
+    const long items = ((long)n_req * (heads / a.unit) * ((head_dim + SC_P - 1) / SC_P) * a.max_pieces + 7) / 8 * 8 * a.unit;
+    const dim3 chunk_grid((unsigned)items);
     TP_REQUIRE(items < 0x7ffffff0L, "ssm_scan: too many pieces");
 #define CHUNK_DISPATCH(OUT_)                                                                                                          \
   do {                                                                                                                                \

@@ -117,7 +117,7 @@ int tp_paged_attention_fast(const void* q, const void* k_cache, const void* v_ca
                             int max_q_len, int num_single, int num_splits, float* scratch, const int* token_req,
                             int portion_splits, int portion_min_steps, float* portion_scratch, const float* dist_bias,
                             int bias_len, int keep_first, const float* sink, int value_dim, int chunk, float softcap,
-                            hipStream_t s);
+                            int keep_parts, hipStream_t s);
 
 // Defined in attention_f32.hip; -1 for shapes that are not its own.
 int tp_paged_attention_f32(const float* q, const float* k_cache, const float* v_cache, const int* block_tables, int table_width,
@@ -141,6 +141,8 @@ extern "C" int tp_paged_attention(const void* q, int dt, const void* k_cache, co
   // which, with more than one split, needs `scratch` of n_req * n_heads * num_splits * (head_dim + 2)
   // floats).  portion_splits > 1: the keys of every longer request are split over that many blocks,
   // which needs `portion_scratch` of n_tokens * n_heads * portion_splits * (head_dim + 4) floats.
+  // allow_fast 2 (single tokens only, more than one split): their partial results stay in `scratch` for
+  // tp_attention_combine_gate and `out` is not written.
   TP_REQUIRE(n_tokens >= 0 && n_req >= 0 && n_heads > 0 && n_kv > 0 && head_dim > 0 && page_size > 0,
              "paged_attention: bad sizes");
   TP_REQUIRE(n_heads % n_kv == 0, "paged_attention: %d heads is not a multiple of %d kv heads", n_heads, n_kv);
@@ -163,9 +165,10 @@ extern "C" int tp_paged_attention(const void* q, int dt, const void* k_cache, co
                                            context_lens, out, n_tokens, n_req, n_heads, n_kv, head_dim,
                                            page_size, scale, window, max_q_len, num_single, num_splits, scratch, token_req,
                                            portion_splits, portion_min_steps, portion_scratch, dist_bias, bias_len, keep_first, sink, value_dim, chunk,
-                                           softcap, s);
+                                           softcap, allow_fast == 2, s);
     if (rc >= 0) return rc;
   }
+  TP_REQUIRE(allow_fast != 2, "paged_attention: no parts to keep for these sizes");
   if (dt == TP_F32 && allow_fast) {
     const int rc = tp_paged_attention_f32((const float*)q, (const float*)k_cache, (const float*)v_cache, block_tables, table_width,
                                           cu_seqlens, context_lens, (float*)out, n_tokens, n_req, n_heads, n_kv, head_dim, value_dim,

@@ -90,6 +90,7 @@ struct AttnArgs {
   int portion_min_steps;   // a query block is split into at most (its steps / this) parts
   float* portion_scratch;
   const int* token_req;
+  bool keep_parts;  // the caller combines the single tokens' splits itself (tp_attention_combine_gate)
   // a bias by distance, added to the scaled score (the scale does not multiply it): dist_bias [heads, bias_len]
   // float32, entry min(query position - key position, bias_len - 1); nullptr: none
   const float* dist_bias;
@@ -1321,10 +1322,20 @@ __global__ __launch_bounds__(256) void attn_decode_kernel(AttnArgs a) {
 // (Combining inside the decode kernel by whichever block finishes last was tried and is far
 // slower: the L2 caches of the eight XCDs are not coherent with each other, so partial results
 // would have to travel through memory with device-scope fences.)
+// GATED: a sublayer's gate over the heads' outputs in the same launch, in the order of its own kernel: the row rounded to bfloat16,
+// times sigmoid(gate column) (per columns in a row share one), times a scale, into columns of a wider row (the same bits; a launch
+// of 2.5 to 4 us behind a chain of such: Bomotar's decode step with four
+// of them 387 -> 377 us, Tokatar's with two 282 -> 278).
+struct CombineGate {
+  const float* rows;      // [n, stride] float32, or nullptr: the scale alone
+  int stride, col0, per, out_stride, out_col0;
+  float scale;
+};
+template <bool GATED>
 __global__ __launch_bounds__(64) void attn_combine_kernel(const float* __restrict__ scratch,
                                                           const int* __restrict__ cu_seqlens,
                                                           bf16_t* __restrict__ out, int n_heads, int D,
-                                                          int num_splits, const float* __restrict__ sink) {
+                                                          int num_splits, const float* __restrict__ sink, CombineGate gate) {
   const int r = blockIdx.x, h = blockIdx.y, lane = threadIdx.x;
   const int q_start = cu_seqlens[r];
   if (cu_seqlens[r + 1] - q_start != 1) return;
@@ -1343,6 +1354,8 @@ __global__ __launch_bounds__(64) void attn_combine_kernel(const float* __restric
   // 32 or 96 the lanes that hold the later splits' weights would sit out)
   for (int d0 = 0; d0 < D; d0 += 64) {
     const int d = min(d0 + lane, D - 1);
+    float raw = 0.f;
+    if (GATED && gate.rows != nullptr) raw = gate.rows[(size_t)q_start * gate.stride + gate.col0 + (h * D + d) / gate.per];
     float acc = 0.f;
     int s = 0;
     for (; s + 8 <= num_splits; s += 8) {   // eight independent loads in flight
@@ -1353,8 +1366,29 @@ __global__ __launch_bounds__(64) void attn_combine_kernel(const float* __restric
       for (int u = 0; u < 8; ++u) acc = fmaf(__shfl(ws, s + u, 64), v[u], acc);
     }
     for (; s < num_splits; ++s) acc = fmaf(__shfl(ws, s, 64), base[(size_t)s * (D + 2) + d], acc);
-    if (d0 + lane < D) out[((size_t)q_start * n_heads + h) * D + d] = float_to_bf16(acc * inv);
+    const bf16_t y = float_to_bf16(acc * inv);
+    if constexpr (GATED) {
+      float v = bf16_to_float(y);
+      if (gate.rows != nullptr) v *= 1.0f / (1.0f + expf(-raw));
+      if (d0 + lane < D) out[(size_t)q_start * gate.out_stride + gate.out_col0 + h * D + d] = float_to_bf16(v * gate.scale);
+    } else if (d0 + lane < D) {
+      out[((size_t)q_start * n_heads + h) * D + d] = y;
+    }
   }
+}
+
+extern "C" int tp_attention_combine_gate(const float* scratch, const int* cu_seqlens, void* out, int n_req, int n_heads, int value_dim,
+                                         int num_splits, const float* sink, const float* gate, int gate_stride, int gate_col0, int per,
+                                         float scale, int out_stride, int out_col0, hipStream_t s) {
+  TP_REQUIRE(n_req >= 0 && n_heads > 0 && n_heads <= 65535 && value_dim > 0 && num_splits >= 1 && num_splits <= 64 && scratch && out, "attention_combine_gate: bad sizes");
+  const int width = n_heads * value_dim;
+  TP_REQUIRE(out_col0 >= 0 && out_stride >= out_col0 + width && per >= 1 && width % per == 0, "attention_combine_gate: bad output rows");
+  TP_REQUIRE(gate == nullptr || (gate_col0 >= 0 && gate_stride >= gate_col0 + width / per), "attention_combine_gate: gate rows too short");
+  if (n_req == 0) return 0;
+  hipLaunchKernelGGL(attn_combine_kernel<true>, dim3(n_req, n_heads), dim3(64), 0, s, scratch, cu_seqlens, (bf16_t*)out, n_heads, value_dim,
+                     num_splits, sink, CombineGate{gate, gate_stride, gate_col0, per, out_stride, out_col0, scale});
+  TP_CHECK_LAUNCH("attention_combine_gate");
+  return 0;
 }
 
 // The same for the rows of portions whose keys were split over blocks: out[token, head, :] from the parts
@@ -1422,10 +1456,10 @@ static int launch_all(AttnArgs a, int n_tokens, int n_req, int max_q_len, int nu
       if (bias) hipLaunchKernelGGL((attn_decode_kernel<D, DV, MODE_BIAS>), grid, dim3(256), 0, s, a);
     }
     if (!bias) hipLaunchKernelGGL((attn_decode_kernel<D, DV, MODE>), grid, dim3(256), 0, s, a);
-    if (a.num_splits > 1) {
+    if (a.num_splits > 1 && !a.keep_parts) {
       const dim3 cgrid(n_req, a.n_heads);
-      hipLaunchKernelGGL(attn_combine_kernel, cgrid, dim3(64), 0, s, a.scratch, a.cu_seqlens, a.out, a.n_heads, DV,
-                         a.num_splits, a.sink);
+      hipLaunchKernelGGL(attn_combine_kernel<false>, cgrid, dim3(64), 0, s, a.scratch, a.cu_seqlens, a.out, a.n_heads, DV,
+                         a.num_splits, a.sink, CombineGate{});
     }
   }
   if (has_multi) {
@@ -1543,7 +1577,7 @@ int tp_paged_attention_fast(const void* q, const void* k_cache, const void* v_ca
                             int max_q_len, int num_single, int num_splits, float* scratch, const int* token_req,
                             int portion_splits, int portion_min_steps, float* portion_scratch, const float* dist_bias,
                             int bias_len, int keep_first, const float* sink, int value_dim, int chunk, float softcap,
-                            hipStream_t s) {
+                            int keep_parts, hipStream_t s) {
   if (head_dim % 32 != 0 || page_size % 8 != 0) return -1;
   if (dist_bias != nullptr && (value_dim != head_dim || softcap > 0.f)) return -1;
   if (chunk < 0 || chunk == 1 || (chunk > 0 && (window > 0 || keep_first > 0))) return -1;
@@ -1572,6 +1606,7 @@ int tp_paged_attention_fast(const void* q, const void* k_cache, const void* v_ca
     if ((1 << b) == page_size) a.page_shift = b;
   a.window = window;
   a.num_splits = num_splits;
+  a.keep_parts = keep_parts != 0;
   a.portion_splits = portion_splits;
   a.portion_min_steps = portion_min_steps;
   a.portion_scratch = portion_scratch;

@@ -952,7 +952,8 @@ def paged_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tenso
                     cu_seqlens: torch.Tensor, context_lens: torch.Tensor, token_req: torch.Tensor,
                     scale: float, window: int, max_q_len: int, max_context_len: int,
                     num_single: Optional[int] = None, dist_bias: Optional[torch.Tensor] = None,
-                    sink: Optional[torch.Tensor] = None, keep_first: int = 0, chunk: int = 0, softcap: float = 0.0) -> torch.Tensor:
+                    sink: Optional[torch.Tensor] = None, keep_first: int = 0, chunk: int = 0, softcap: float = 0.0,
+                    into: Optional[tuple] = None) -> Optional[torch.Tensor]:
     """q [n, heads, head_dim] over k [pages, kv_heads, page_size, head_dim] and transposed
     v [pages, kv_heads, value_dim, page_size] -> [n, heads * value_dim] (value_dim is the value cache's own; the
     matrix-core kernels take the pairs of sizes in ``FAST_PAIRS``, other sizes run the general kernel).
@@ -961,7 +962,13 @@ def paged_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tenso
     ``sink`` (float32 [heads]): the softmax's denominator holds one more term, exp(sink[head]), without key or value.
     ``keep_first``: under a window, the request's first ``keep_first`` keys stay visible as well.
     ``chunk`` (instead of a window): a query sees the keys of its own aligned chunk of that many positions only.
-    ``softcap`` > 0: a scaled score s becomes softcap * tanh(s / softcap) before the softmax (no distance bias then)."""
+    ``softcap`` > 0: a scaled score s becomes softcap * tanh(s / softcap) before the softmax (no distance bias then).
+    ``into``: the last six arguments of ``sigmoid_gate`` (gate rows or None, their column, scale, output rows, their column, columns
+    that share a gate): the result goes there and None comes back."""
+    if into is not None and not (_backend is None and num_single == block_tables.shape[0] == q.shape[0]):
+        sigmoid_gate(paged_attention(q, k_cache, v_cache, block_tables, cu_seqlens, context_lens, token_req, scale, window, max_q_len,
+                                     max_context_len, num_single, dist_bias, sink, keep_first, chunk, softcap), *into)
+        return None
     if _backend is not None:
         if chunk or softcap:
             return _backend.paged_attention(q, k_cache, v_cache, block_tables, cu_seqlens, context_lens,
@@ -1069,13 +1076,28 @@ def paged_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tenso
             parts = 1
         if parts > 1:
             part_scratch = torch.empty((n * heads * parts * (vd + 4),), dtype=torch.float32, device=q.device)
+    # (single tokens whose keys are split: the kernel that adds the splits also gates them)
+    keep_parts = into is not None and fast and splits > 1 and num_single == r and n > 0
     _call("tp_paged_attention", _ptr(q), _dt(q), _ptr(k_cache), _ptr(v_cache), _ptr(block_tables), width,
           _ptr(cu_seqlens), _ptr(context_lens), _ptr(token_req), _ptr(out), n, r, heads, kvh, d, page_size,
-          ctypes.c_float(scale), int(window), int(max_q_len), int(max_context_len), int(fast or fast_f32),
+          ctypes.c_float(scale), int(window), int(max_q_len), int(max_context_len), 2 if keep_parts else int(fast or fast_f32),
           int(num_single), int(splits), _ptr(scratch), int(parts), max(1, portion_min_keys // 32), _ptr(part_scratch),
           _ptr(dist_bias), 0 if dist_bias is None else dist_bias.shape[1], int(vd), int(keep_first), _ptr(sink), int(chunk),
           ctypes.c_float(softcap), _stream())
-    return out
+    if into is None:
+        return out
+    if keep_parts:
+        gate, gate_col0, factor, dest, dest_col0, per = into
+        _dev_ok(gate, dest)
+        _need(dest.dim() == 2 and dest.dtype == q.dtype and dest.shape[0] == n and 0 <= dest_col0 and dest_col0 + heads * vd <= dest.shape[1]
+              and per >= 1 and (heads * vd) % per == 0, "paged_attention: bad output rows")
+        _need(gate is None or (gate.dtype == torch.float32 and gate.dim() == 2 and gate.shape[0] == n and 0 <= gate_col0
+                               and gate_col0 + heads * vd // per <= gate.shape[1]), "paged_attention: bad gate rows")
+        _call("tp_attention_combine_gate", _ptr(scratch), _ptr(cu_seqlens), _ptr(dest), r, heads, vd, int(splits), _ptr(sink), _ptr(gate),
+              0 if gate is None else gate.shape[1], int(gate_col0), int(per), ctypes.c_float(factor), dest.shape[1], int(dest_col0), _stream())
+    else:
+        sigmoid_gate(out, *into)
+    return None
 
 
 def swiglu(gu: torch.Tensor, out_dtype: torch.dtype) -> torch.Tensor:

@@ -278,27 +278,30 @@ class PagedAttention(Mixer):
             q = self._project_and_rotate(x, ctx, cache, rot)
         if self.w_gates is not None:
             gates = ops.linear(x, self.w_gates, torch.float32)
+        # (a gate over the heads' outputs: of single tokens the kernel that adds the splits of their keys applies it)
+        into, gated = {}, None
+        if self.gate and self.value_position is None:
+            gated = torch.empty((q.shape[0], self.num_heads * self.value_dim), dtype=q.dtype, device=q.device)
+            into = {"into": (gates, self.gate_col0, 1.0, gated, 0, 1)}
         if self.extended or self.chunk or self.softcap:
             a = ops.paged_attention(
                 q, cache.k, cache.v, ctx.block_tables[cache.group], ctx.cu_seqlens, ctx.context_lens,
                 ctx.token_req, self.scale, int(self.window or 0), ctx.max_q_len, ctx.max_context_len,
-                ctx.num_single, sink=self.sink_w, keep_first=self.keep_first, chunk=self.chunk, softcap=self.softcap)
+                ctx.num_single, sink=self.sink_w, keep_first=self.keep_first, chunk=self.chunk, softcap=self.softcap, **into)
         elif self.dist_table is not None:
             a = ops.paged_attention(
                 q, cache.k, cache.v, ctx.block_tables[cache.group], ctx.cu_seqlens, ctx.context_lens,
                 ctx.token_req, self.scale, int(self.window or 0), ctx.max_q_len, ctx.max_context_len,
-                ctx.num_single, dist_bias=self.dist_table)
+                ctx.num_single, dist_bias=self.dist_table, **into)
         else:
             a = ops.paged_attention(
                 q, cache.k, cache.v, ctx.block_tables[cache.group], ctx.cu_seqlens, ctx.context_lens,
                 ctx.token_req, self.scale, int(self.window or 0), ctx.max_q_len, ctx.max_context_len,
-                ctx.num_single)
+                ctx.num_single, **into)
         if self.value_position is not None:
             vp = self.value_position
             a = ops.turn_gate(a, ctx.positions, vp.inv_freq, self.value_dim, gates if self.gate else None, self.gate_col0, vp.table(ctx))
         elif self.gate:
-            gated = torch.empty_like(a)
-            ops.sigmoid_gate(a, gates, self.gate_col0, 1.0, gated, 0)
             a = gated
         if self.side_rows is not None:
             if residual is not None:
@@ -533,9 +536,9 @@ class ConvAttention(BranchMixer):
             q = ops.rope_kv_write(qkv, ctx.positions, ctx.slot_mapping[cache.group], inv_freq, rotary_dim, factor, self.num_heads,
                                   self.num_kv_heads, self.head_dim, cache.k, cache.v, self.dtype, table, value_dim=self.value_dim,
                                   pad_dim=self.key_dim)
-        a = ops.paged_attention(q, cache.k, cache.v, ctx.block_tables[cache.group], ctx.cu_seqlens, ctx.context_lens,
-                                ctx.token_req, self.scale, int(self.window or 0), ctx.max_q_len, ctx.max_context_len, ctx.num_single)
-        ops.sigmoid_gate(a, proj if self.gate else None, col0 + self.channels, scale, out, out_col0, self.gate_per if self.gate else 1)
+        ops.paged_attention(q, cache.k, cache.v, ctx.block_tables[cache.group], ctx.cu_seqlens, ctx.context_lens,
+                            ctx.token_req, self.scale, int(self.window or 0), ctx.max_q_len, ctx.max_context_len, ctx.num_single,
+                            into=(proj if self.gate else None, col0 + self.channels, scale, out, out_col0, self.gate_per if self.gate else 1))
 
 
 register_part("mixer", "conv_attention", ConvAttention)
@@ -624,9 +627,9 @@ class LatentAttention(BranchMixer):
         table = self.position.table(ctx) if hasattr(self.position, "table") else None
         q = ops.rope_kv_write(rows, ctx.positions, ctx.slot_mapping[cache.group], inv_freq, rotary_dim, factor, H, H, self.key_dim,
                               cache.k, cache.v, self.dtype, table, value_dim=self.value_dim)
-        a = ops.paged_attention(q, cache.k, cache.v, ctx.block_tables[cache.group], ctx.cu_seqlens, ctx.context_lens,
-                                ctx.token_req, self.scale, int(self.window or 0), ctx.max_q_len, ctx.max_context_len, ctx.num_single)
-        ops.sigmoid_gate(a, proj if self.gate else None, col0 + self.q_dim + self.down_dim, scale, out, out_col0)
+        ops.paged_attention(q, cache.k, cache.v, ctx.block_tables[cache.group], ctx.cu_seqlens, ctx.context_lens,
+                            ctx.token_req, self.scale, int(self.window or 0), ctx.max_q_len, ctx.max_context_len, ctx.num_single,
+                            into=(proj if self.gate else None, col0 + self.q_dim + self.down_dim, scale, out, out_col0, 1))
 
 
 register_part("mixer", "latent_attention", LatentAttention)
@@ -722,9 +725,9 @@ class LatentCacheAttention(BranchMixer):
             ops.vector_store(c, ctx.slot_mapping[cache.group], cache.k, cache.v)
         cq = ops.rmsnorm_cols(proj, col0, self.query_rank, self.dq_norm_w, self.norm_eps, self.dtype)
         q = ops.linear(cq, self.w_q, self.dtype).view(n, self.num_heads, self.latent_dim)
-        a = ops.paged_attention(q, cache.k, cache.v, ctx.block_tables[cache.group], ctx.cu_seqlens, ctx.context_lens, ctx.token_req,
-                                self.scale, int(self.window or 0), ctx.max_q_len, ctx.max_context_len, ctx.num_single, sink=self.sink_w)
-        ops.sigmoid_gate(a, None, 0, scale, out, out_col0)
+        ops.paged_attention(q, cache.k, cache.v, ctx.block_tables[cache.group], ctx.cu_seqlens, ctx.context_lens, ctx.token_req,
+                            self.scale, int(self.window or 0), ctx.max_q_len, ctx.max_context_len, ctx.num_single, sink=self.sink_w,
+                            into=(None, 0, scale, out, out_col0, 1))
 
 
 register_part("mixer", "latent_cache_attention", LatentCacheAttention)
@@ -849,12 +852,11 @@ class RotaryLatentAttention(BranchMixer):
         n, gate_col0 = proj.shape[0], d_col0 + self.latent_dim + self.rotary_dim
         if not self.folded:
             ops.head_linear(proj, col0, self.head_dim + self.rotary_dim, self.w_uk, q.view(n, -1), self.rotary_dim, self.cached_key)
+        into = {} if not self.folded else {"into": (proj if self.gate else None, gate_col0, scale, out, out_col0, self.cached_value if self.gate else 1)}
         a = ops.paged_attention(q, cache.k, cache.v, ctx.block_tables[cache.group], ctx.cu_seqlens, ctx.context_lens, ctx.token_req,
-                                self.scale, int(self.window or 0), ctx.max_q_len, ctx.max_context_len, ctx.num_single)
+                                self.scale, int(self.window or 0), ctx.max_q_len, ctx.max_context_len, ctx.num_single, **into)
         if not self.folded:
             ops.head_linear(a, 0, self.cached_value, self.w_uv, out, out_col0, self.value_dim, proj if self.gate else None, gate_col0, scale)
-            return
-        ops.sigmoid_gate(a, proj if self.gate else None, gate_col0, scale, out, out_col0, self.cached_value if self.gate else 1)
 
 
 register_part("mixer", "rotary_latent_attention", RotaryLatentAttention)

@@ -205,3 +205,28 @@ def test_gated_products_of_a_few_rows_take_the_gates_constants(m, n, k, slope, l
     if isinstance(blocked, ops.KBlocked):
         blocked = blocked.data.permute(1, 0, 2).reshape(m, n // 2)
     assert torch.equal(blocked, got)
+
+
+@pytest.mark.parametrize("heads,kv,d,vd", [(4, 2, 64, 64), (3, 1, 96, 96), (8, 8, 32, 32), (16, 1, 576, 512), (2, 2, 160, 96)])
+@pytest.mark.parametrize("ctx", [[700], [1, 40, 1500], [3, 260]])
+@pytest.mark.parametrize("how", ["columns", "heads", "scale", "sink", "portions"])
+def test_attention_gates_what_it_combines(heads, kv, d, vd, ctx, how):
+    """The kernel that adds the splits of single tokens gates them in the order of the gate's own kernel: the same bits, also where
+    keys are not split or a portion is among the requests (the two kernels then)."""
+    from tempura_amd.kernels import ops
+    g = torch.Generator().manual_seed(heads + ctx[-1])
+    page, r = 16, len(ctx)
+    q_lens = [1] * r if how != "portions" else [min(3, ctx[0])] + [1] * (r - 1)
+    n, width, per = sum(q_lens), -(-max(ctx) // page), vd if how == "heads" else 1
+    kc = (torch.randn(r * width, kv, page, d, generator=g)).to(torch.bfloat16).to(DEV)
+    vc = (torch.randn(r * width, kv, vd, page, generator=g)).to(torch.bfloat16).to(DEV)
+    tables = torch.randperm(r * width, generator=g).to(torch.int32).view(r, width).to(DEV)
+    q = torch.randn(n, heads, d, generator=g).to(torch.bfloat16).to(DEV)
+    cu, req, _ = _runs(q_lens, g)
+    args = (q, kc, vc, tables, cu, torch.tensor(ctx, dtype=torch.int32, device=DEV), req, d ** -0.5, 0, max(q_lens), max(ctx), q_lens.count(1))
+    sink = torch.randn(heads, generator=g).to(DEV) if how == "sink" else None
+    rows = None if how == "scale" else torch.randn(n, 5 + heads * vd // per + 2, generator=g).to(DEV)
+    want, got = (torch.full((n, heads * vd + 9), 7.0, dtype=torch.bfloat16, device=DEV) for _ in range(2))
+    ops.sigmoid_gate(ops.paged_attention(*args, sink=sink), rows, 5, 0.75, want, 4, per)
+    assert ops.paged_attention(*args, sink=sink, into=(rows, 5, 0.75, got, 4, per)) is None
+    assert torch.isfinite(got.float()).all() and torch.equal(got, want)

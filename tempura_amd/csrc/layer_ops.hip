@@ -950,7 +950,7 @@ template <typename TO, bool SINGLE>
 __global__ void residual_conv4_kernel(const float* __restrict__ x, const float* __restrict__ w, float* __restrict__ state,
                                       size_t state_stride, size_t state_off, const int* __restrict__ cu_seqlens,
                                       const int* __restrict__ token_req, const int* __restrict__ state_slots, TO* __restrict__ out,
-                                      size_t out_stride_sub, int width, int taps, int subs, int channel_blocks) {
+                                      size_t out_stride_sub, int width, int taps, int subs, int channel_blocks, int blocked) {
   const int t = blockIdx.x / channel_blocks;
   const int c = ((blockIdx.x % channel_blocks) * blockDim.x + threadIdx.x) * 4;
   if (c >= width) return;
@@ -990,9 +990,10 @@ __global__ void residual_conv4_kernel(const float* __restrict__ x, const float* 
   }
 #pragma unroll
   for (int sub = 0; sub < RCONV_MAX_SUBS; ++sub)
-    if (sub < subs)
-      from_float4(out + (size_t)sub * out_stride_sub + (size_t)t * width + c, cur.x + acc[sub].x, cur.y + acc[sub].y,
-                  cur.z + acc[sub].z, cur.w + acc[sub].w);
+    if (sub < subs) {
+      const size_t place = (SINGLE && (blocked >> sub & 1)) ? ((size_t)(c >> 3) * (gridDim.x / channel_blocks) + t) * 8 + (c & 7) : (size_t)t * width + c;
+      from_float4(out + (size_t)sub * out_stride_sub + place, cur.x + acc[sub].x, cur.y + acc[sub].y, cur.z + acc[sub].z, cur.w + acc[sub].w);
+    }
 }
 
 __global__ void residual_conv_state_kernel(const float* __restrict__ x, float* __restrict__ state, size_t state_stride,
@@ -1013,8 +1014,9 @@ __global__ void residual_conv_state_kernel(const float* __restrict__ x, float* _
 
 extern "C" int tp_residual_conv(const float* x, const float* w, float* state, size_t state_stride, size_t state_off,
                                 const int* cu_seqlens, const int* token_req, const int* state_slots, void* out, int out_dt, int n,
-                                int n_req, int width, int taps, int subs, int max_run, hipStream_t s) {
-  // (max_run: the longest run of the step, 0: not known)
+                                int n_req, int width, int taps, int subs, int max_run, int blocked, hipStream_t s) {
+  // max_run: the longest run of the step, 0: not known.  blocked (runs of one token): bit i, sublayer i's rows leave k-blocked,
+  // [width / 8, n, 8]
   TP_REQUIRE(n >= 0 && n_req >= 0 && width > 0 && taps >= 1 && subs >= 1, "residual_conv: bad sizes");
   TP_REQUIRE(state_stride >= state_off + (size_t)(taps - 1) * width, "residual_conv: state rows too short");
   if (n == 0) return 0;
@@ -1030,17 +1032,20 @@ extern "C" int tp_residual_conv(const float* x, const float* w, float* state, si
     const dim3 grid((unsigned)((long)n * qb));
 #define RCONV(TO, SINGLE)                                                                                                           \
   hipLaunchKernelGGL((residual_conv4_kernel<TO, SINGLE>), grid, dim3(qthreads), 0, s, x, w, state, state_stride, state_off, cu_seqlens, \
-                     token_req, state_slots, (TO*)out, sub_stride, width, taps, subs, qb)
+                     token_req, state_slots, (TO*)out, sub_stride, width, taps, subs, qb, blocked)
     if (max_run == 1) {
       if (out_dt == TP_F32) RCONV(float, true);
       else RCONV(bf16_t, true);
       TP_CHECK_LAUNCH("residual_conv");
       return 0;
     }
+    TP_REQUIRE(blocked == 0, "residual_conv: only runs of one token leave k-blocked");
     if (out_dt == TP_F32) RCONV(float, false);
     else RCONV(bf16_t, false);
 #undef RCONV
-  } else if (out_dt == TP_F32)
+  } else if (blocked != 0)
+    TP_REQUIRE(false, "residual_conv: rows of these sizes do not leave k-blocked");
+  else if (out_dt == TP_F32)
     hipLaunchKernelGGL(residual_conv_kernel<float>, dim3((unsigned)((long)n * cb)), dim3(threads), 0, s, x, w, state, state_stride,
                        state_off, cu_seqlens, token_req, state_slots, (float*)out, sub_stride, width, taps, subs, cb);
   else if (out_dt == TP_BF16)

@@ -1882,12 +1882,14 @@ def rmsnorm_cols(x: torch.Tensor, col0: int, width: int, weight: torch.Tensor, e
 
 
 def residual_conv(x: torch.Tensor, weight: torch.Tensor, state: torch.Tensor, state_off: int, cu_seqlens: torch.Tensor,
-                  token_req: torch.Tensor, state_slots: torch.Tensor, num_requests: int, out_dtype: torch.dtype, max_run: int = 0):
+                  token_req: torch.Tensor, state_slots: torch.Tensor, num_requests: int, out_dtype: torch.dtype, max_run: int = 0,
+                  blocked=()):
     """What sublayers read of rows ``x`` (float32 [n, width]): for each of the ``weight`` [subs, taps, width] (tap-major,
     the last tap the current token's) x + conv(x) over each request's run of tokens, as ``out_dtype``; a list of
     ``subs`` tensors [n, width].  ``state`` float32 [slots, row]: from element ``state_off`` on a request's carried
     rows [taps - 1, width] (oldest first), read for the first tokens of a run and replaced by the run's last rows.  ``max_run``: the longest run
-    (0: not known); runs of one token are one launch."""
+    (0: not known); runs of one token are one launch, which gives the sublayers named in ``blocked`` their rows as ``KBlocked``
+    (``few_rows_ok``, at most four sublayers)."""
     if _backend is not None:
         return _backend.residual_conv(x, weight, state, state_off, cu_seqlens, token_req, state_slots, num_requests, out_dtype)
     _dev_ok(x, weight, state, cu_seqlens, token_req, state_slots)
@@ -1904,8 +1906,8 @@ def residual_conv(x: torch.Tensor, weight: torch.Tensor, state: torch.Tensor, st
     out = torch.empty((subs, n, width), dtype=out_dtype, device=x.device)
     _call("tp_residual_conv", _ptr(x), _ptr(weight), _ptr(state), ctypes.c_size_t(0 if state is None else state.shape[1]), ctypes.c_size_t(state_off),
           _ptr(cu_seqlens), _ptr(token_req), _ptr(state_slots), _ptr(out), _dtcode(out_dtype), n, int(num_requests), width, taps, subs,
-          int(max_run), _stream())
-    return [out[i] for i in range(subs)]
+          int(max_run), sum(1 << i for i in blocked), _stream())
+    return [KBlocked(out[i].view(width // 8, n, 8), n, width) if i in blocked else out[i] for i in range(subs)]
 
 
 def add_row(h: torch.Tensor, table: torch.Tensor, row: int) -> None:

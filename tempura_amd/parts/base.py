@@ -147,6 +147,7 @@ class BranchMixer(Mixer):
     graph_safe = True
     returns_output = True      # with ``residual`` None the output comes back instead of being added
     takes_side_rows = True     # (behind the branch's own columns of the input product)
+    takes_blocked_rows = True
     inner = 0
     state_off = 0
 

@@ -438,7 +438,8 @@ class SharedNormBlock(ArrangedBlock):
 
     def forward(self, h, ctx, cache) -> None:
         if self.inputs is not None:
-            xs = self.inputs.forward(self.norm.forward(h, out_dtype=torch.float32), ctx, cache)
+            parts = [self.mixer] if self.ffn is None else [self.mixer, self.ffn]
+            xs = self.inputs.forward(self.norm.forward(h, out_dtype=torch.float32), ctx, cache, parts)
         else:
             xs = [self.norm.forward(h)] * 2
         self.mixer.forward(xs[0], ctx, cache, h)

@@ -42,10 +42,14 @@ class ResidualConv(Part):
         # [sublayers, taps, hidden]: tap-major, so that neighbouring lanes read neighbouring channels
         self.weight = torch.stack([self._to_device(get(name), torch.float32).t() for name in self.names]).contiguous()
 
-    def forward(self, n, ctx, cache):
-        """float32 rows [tokens, hidden] -> a list of compute-dtype rows, one per sublayer."""
+    def forward(self, n, ctx, cache, parts=()):
+        """float32 rows [tokens, hidden] -> a list of compute-dtype rows, one per sublayer (k-blocked for those of the ``parts``
+        that take them so, in a step of a few single tokens)."""
+        few = {}
+        if ctx.max_q_len == 1 and len(self.names) <= 4 and ops.few_rows_ok(n.shape[0], n.shape[1], self.dtype):
+            few = {"blocked": [i for i, part in enumerate(parts) if getattr(part, "takes_blocked_rows", False)]}
         return ops.residual_conv(n, self.weight, cache.state, self.state_off, ctx.cu_seqlens, ctx.token_req, ctx.state_slots,
-                                 ctx.num_requests, self.dtype, max_run=ctx.max_q_len)
+                                 ctx.num_requests, self.dtype, max_run=ctx.max_q_len, **few)
 
 
 register_part("input", "residual_conv", ResidualConv)

@@ -55,6 +55,10 @@ def test_residual_conv_of_single_tokens(width, subs, taps):
     want = ops.residual_conv(x, w, s0, 3, cu, req, slots, 4, torch.bfloat16)
     got = ops.residual_conv(x, w, s1, 3, cu, req, slots, 4, torch.bfloat16, max_run=1)
     assert all(torch.equal(a, b) for a, b in zip(got, want)) and torch.equal(s0, s1)
+    if ops.few_rows_ok(4, width, torch.bfloat16):
+        got = ops.residual_conv(x, w, state.clone(), 3, cu, req, slots, 4, torch.bfloat16, max_run=1, blocked=[subs - 1])
+        assert torch.equal(got[-1].data.permute(1, 0, 2).reshape(4, width), want[-1])
+        assert subs == 1 or torch.equal(got[0], want[0])
 
 
 @pytest.mark.parametrize("streams", [2, 4])

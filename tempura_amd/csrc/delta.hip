@@ -5,8 +5,8 @@
 //
 // A request r of the batch owns tokens cu_seqlens[r] .. cu_seqlens[r + 1] - 1 and the state row state_slots[r];
 // everything is read from device memory, so the same launches serve prompt portions, single decoded tokens and
-// captured steps.  A token's result does not depend on how its run was cut: every token is one step of the same
-// chain, in the same order of operations.
+// captured steps.  In short runs a token's result does not depend on how its run was cut: every token is one step of the
+// same chain, in the same order of operations; long runs go by groups of tokens (delta_chunks.hip), which changes rounding only.
 #include <math.h>
 
 #include "common.h"
@@ -246,10 +246,17 @@ __global__ __launch_bounds__(256) void delta_scan_kernel(DeltaArgs a) {
   }
 }
 
+// Defined in delta_chunks.hip: 0 when it took the runs, -1 when they are not its own.
+int tp_delta_chunks(const float* qkv, int row_stride, const float* decay, const float* proj, int proj_stride, int beta_col0, float* state,
+                    size_t state_stride, size_t state_off, const int* cu_seqlens, const int* state_slots, float* y, int n_req, int heads,
+                    int kv_heads, int dim, int vdim, float q_scale, float unit_eps, int max_run, float* scratch, size_t scratch_floats,
+                    hipStream_t s);
+
+// max_run: the longest run, 0: not known (scratch of tp_delta_scan_scratch floats lets long runs go by groups of tokens).
 extern "C" int tp_delta_scan(float* qkv, int row_stride, const float* decay, const float* proj, int proj_stride,
                              int beta_col0, float* state, size_t state_stride, size_t state_off, const int* cu_seqlens,
                              const int* state_slots, float* y, float* kq, int n, int n_req, int heads, int kv_heads, int dim,
-                             int vdim, float q_scale, float unit_eps, hipStream_t s) {
+                             int vdim, float q_scale, float unit_eps, int max_run, float* scratch, size_t scratch_floats, hipStream_t s) {
   TP_REQUIRE(n >= 0 && n_req >= 0 && heads > 0 && kv_heads > 0 && dim > 0 && vdim > 0, "delta_scan: bad sizes");
   TP_REQUIRE(heads % kv_heads == 0, "delta_scan: %d heads is not a multiple of %d key heads", heads, kv_heads);
   TP_REQUIRE(dim <= 1024, "delta_scan: key size %d exceeds 1024", dim);
@@ -257,6 +264,11 @@ extern "C" int tp_delta_scan(float* qkv, int row_stride, const float* decay, con
   TP_REQUIRE(state_stride >= state_off + (size_t)heads * dim * vdim, "delta_scan: state rows too short");
   TP_REQUIRE(heads <= 65535, "delta_scan: too many heads");
   if (n == 0 || n_req == 0) return 0;
+  if (tp_delta_chunks(qkv, row_stride, decay, proj, proj_stride, beta_col0, state, state_stride, state_off, cu_seqlens, state_slots, y, n_req,
+                      heads, kv_heads, dim, vdim, q_scale, unit_eps, max_run, scratch, scratch_floats, s) == 0) {
+    TP_CHECK_LAUNCH("delta_scan (groups)");
+    return 0;
+  }
   DeltaArgs a{qkv, row_stride, decay, proj, proj_stride, beta_col0, state, state_stride, state_off, cu_seqlens, state_slots, y, kq,
               heads, kv_heads, dim, vdim, q_scale, unit_eps};
   const long pairs = (long)n * kv_heads;

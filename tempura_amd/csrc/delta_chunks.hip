@@ -1,0 +1,372 @@
+// The gated delta rule over long runs, 16 tokens at a time on the matrix cores (v_mfma_f32_16x16x4_f32), for key sizes of 64 and 128 and
+// value sizes of a multiple of 16; delta.hip has the recurrence, and the chain of single tokens that short runs and other sizes take.
+//
+// Within 16 tokens, with G_t the product of the decays up to token t and S the state before them, the rule is a small linear system:
+//   A[t, s] = sum_c k_t k_s (G_t / G_s)  (s < t),  B[t, s] the same with q_t (s <= t),  T = (I + diag(beta) A)^-1 diag(beta)
+//   U = T V - (T K~) S  with K~_t = G_t k_t;   o = Q~ S + B U  with Q~_t = G_t q_t;   S <- G_16 S + K^T U  with K^_s = (G_16 / G_s) k_s
+// Everything but the three products with S is independent of the state: delta_chunk_prep_kernel works it out for all groups of 16 side by
+// side, a wave each, and leaves W = T K~, Q~, K^, B and T V in scratch; the ratios of decays are running products, never quotients, so
+// nothing overflows.  delta_chunk_scan_kernel is the chain over the groups: a block of four waves owns 16 value columns of a head, a wave
+// a quarter of the key channels in accumulators, which lie as the next product's operand wants them; the waves' parts of W S and Q~ S meet
+// in LDS once a group.
+//
+// The chain of single tokens is bound by what a wave issues and waits for a token, 0.25 to 0.55 us; here a group of 16 takes 1.3 us (its
+// products, a meeting in LDS and the update, each waiting for the one before).  16 heads of 128 x 128, single tokens / groups: one run of
+// 128 tokens 41 / 31 us, 256 75 / 42, 2,048 512 / 202; four runs of 451 tokens 171 / 94 (a third of it the first kernel).
+#include <math.h>
+
+#include "common.h"
+#include "column_sum.h"
+
+typedef float f32x4_d __attribute__((ext_vector_type(4)));
+
+#define DC_T 16      // tokens of a group
+
+struct DeltaChunkArgs {
+  const float* qkv;
+  const float* decay;
+  const float* proj;
+  float* state;
+  const int* cu_seqlens;
+  const int* state_slots;
+  float* y;
+  float* scratch;
+  size_t state_stride, state_off;
+  int row_stride, proj_stride, beta_col0, heads, kv_heads, vdim, requests;
+  int first;       // first token of a run that this launch takes
+  int groups;      // groups of a run that this launch takes, at most
+  float q_scale, unit_eps;
+};
+
+// floats of scratch for one group of one head: W, Q~ [16, dim], K^ [dim, 16], G_16 [dim], B [16, 16] without its diagonal, that [16],
+// T V [16, vdim]
+__host__ __device__ inline size_t dc_item_floats(int dim, int vdim) { return (size_t)49 * dim + 272 + (size_t)16 * vdim; }
+
+// places of the sums: for s B(s, s), then A(t, s), B(t, s) of t = s + 1 .. 15
+#define DC_B(t, s) (32 * (s) - (s) * (s) + 2 * ((t) - (s)))
+#define DC_A(t, s) (DC_B(t, s) - 1)
+
+// (a recursion: every place of v is then known to the compiler, which keeps v in registers)
+template <int S, int PER>
+__device__ inline void dc_dots(const float (&q)[DC_T][PER], const float (&k)[DC_T][PER], const float (&gd)[DC_T][PER], float (&v)[64],
+                               float* dots, int lane) {
+  float w[PER];
+#pragma unroll
+  for (int p = 0; p < PER; ++p) w[p] = k[S][p];
+#pragma unroll
+  for (int t = S; t < DC_T; ++t) {
+    float da = 0.f, db = 0.f;
+#pragma unroll
+    for (int p = 0; p < PER; ++p) {
+      if (t > S) w[p] *= gd[t][p];
+      da = fmaf(w[p], k[t][p], da);
+      db = fmaf(w[p], q[t][p], db);
+    }
+    if (t > S) {
+      v[DC_A(t, S) % 64] = da;
+      if (DC_A(t, S) % 64 == 63) dots[DC_A(t, S) - 63 + lane] = lanes_transpose_sum<64>(v, lane);
+    }
+    v[DC_B(t, S) % 64] = db;
+    if (DC_B(t, S) % 64 == 63) dots[DC_B(t, S) - 63 + lane] = lanes_transpose_sum<64>(v, lane);
+  }
+  if constexpr (S + 1 < DC_T) dc_dots<S + 1, PER>(q, k, gd, v, dots, lane);
+}
+
+template <int PER>
+__global__ __launch_bounds__(64) void delta_chunk_prep_kernel(DeltaChunkArgs a) {
+  constexpr int K = 64 * PER;
+  __shared__ float dots[256];
+  __shared__ __attribute__((aligned(16))) float Ts[DC_T][DC_T];
+  __shared__ float bs[DC_T];
+  const int lane = threadIdx.x;
+  const int h = blockIdx.x % a.heads, rest = blockIdx.x / a.heads, c = rest % a.groups, r = rest / a.groups;
+  const int run0 = a.cu_seqlens[r], t0 = a.first + c * DC_T, len = min(DC_T, a.cu_seqlens[r + 1] - run0 - t0);
+  if (len <= 0) return;
+  const size_t row0 = (size_t)(run0 + t0);
+  const int g = h / (a.heads / a.kv_heads);
+  const float* qp = a.qkv + row0 * a.row_stride + (size_t)g * K;
+  const float* kp = qp + (size_t)a.kv_heads * K;
+  const float* gp = a.decay + (row0 * a.heads + h) * K;
+  float q[DC_T][PER], k[DC_T][PER], gd[DC_T][PER];      // (channels lane + 64 p)
+#pragma unroll
+  for (int t = 0; t < DC_T; ++t)
+#pragma unroll
+    for (int p = 0; p < PER; ++p) {
+      const int ch = lane + 64 * p;
+      const bool in = t < len;
+      q[t][p] = in ? qp[(size_t)t * a.row_stride + ch] : 0.f;
+      k[t][p] = in ? kp[(size_t)t * a.row_stride + ch] : 0.f;
+      gd[t][p] = in ? gp[(size_t)t * a.heads * K + ch] : 1.f;
+    }
+  if (lane < DC_T) bs[lane] = lane < len ? 1.0f / (1.0f + expf(-a.proj[(row0 + lane) * a.proj_stride + a.beta_col0 + h])) : 0.f;
+  // unit vectors: the 16 sums of squares of q and of k at once, lane 2 i the i-th
+  {
+    float sq[2 * DC_T];
+#pragma unroll
+    for (int t = 0; t < DC_T; ++t) {
+      float x = 0.f, y = 0.f;
+#pragma unroll
+      for (int p = 0; p < PER; ++p) {
+        x = fmaf(q[t][p], q[t][p], x);
+        y = fmaf(k[t][p], k[t][p], y);
+      }
+      sq[t] = x;
+      sq[DC_T + t] = y;
+    }
+    const float total = lanes_transpose_sum<2 * DC_T>(sq, lane);
+    const float unit = (lane < 32 ? a.q_scale : 1.0f) / sqrtf(total + a.unit_eps);
+#pragma unroll
+    for (int t = 0; t < DC_T; ++t) {
+      const float rq = __shfl(unit, 2 * t, TP_WAVE), rk = __shfl(unit, 2 * (DC_T + t), TP_WAVE);
+#pragma unroll
+      for (int p = 0; p < PER; ++p) {
+        q[t][p] *= rq;
+        k[t][p] *= rk;
+      }
+    }
+  }
+  // A and B, 64 of their sums over the channels at a time
+  {
+    float v[64];
+    dc_dots<0, PER>(q, k, gd, v, dots, lane);
+  }
+  float* item = a.scratch + (((size_t)r * a.groups + c) * a.heads + h) * dc_item_floats(K, a.vdim);
+  float *W = item, *Q = W + DC_T * K, *KT = Q + DC_T * K, *G = KT + DC_T * K, *B = G + K, *U0 = B + 272;
+  // G_16, Q~, K~ (in k's place, after K^ has been made of it)
+#pragma unroll
+  for (int p = 0; p < PER; ++p) {
+    const int ch = lane + 64 * p;
+    float tail = 1.f, kt[DC_T];
+#pragma unroll
+    for (int s = DC_T - 1; s >= 0; --s) {
+      kt[s] = k[s][p] * tail;
+      tail *= gd[s][p];
+    }
+    G[ch] = tail;
+#pragma unroll
+    for (int s = 0; s < DC_T; s += 4) *(f32x4_d*)(KT + (size_t)ch * DC_T + s) = (f32x4_d){kt[s], kt[s + 1], kt[s + 2], kt[s + 3]};
+    float head = 1.f;
+#pragma unroll
+    for (int t = 0; t < DC_T; ++t) {
+      head *= gd[t][p];
+      Q[t * K + ch] = q[t][p] * head;
+      k[t][p] *= head;
+    }
+  }
+  __syncthreads();
+  // lane j: column j of T
+  if (lane < DC_T) {
+    float col[DC_T];
+#pragma unroll
+    for (int t = 0; t < DC_T; ++t) {
+      float sum = 0.f;
+#pragma unroll
+      for (int s = 0; s < t; ++s) sum = fmaf(dots[DC_A(t, s)], col[s], sum);
+      col[t] = t == lane ? bs[t] : t > lane ? -bs[t] * sum : 0.f;
+      Ts[t][lane] = col[t];
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int e = lane + 64 * i, t = e / DC_T, s = e % DC_T;
+    B[e] = s < t ? dots[DC_B(t, s)] : 0.f;
+  }
+  if (lane < DC_T) B[256 + lane] = dots[DC_B(lane, lane)];
+  __syncthreads();
+#pragma unroll
+  for (int t = 0; t < DC_T; ++t) {
+    float w[PER];
+#pragma unroll
+    for (int p = 0; p < PER; ++p) w[p] = 0.f;
+#pragma unroll
+    for (int s = 0; s <= t; ++s)
+#pragma unroll
+      for (int p = 0; p < PER; ++p) w[p] = fmaf(Ts[t][s], k[s][p], w[p]);
+#pragma unroll
+    for (int p = 0; p < PER; ++p) W[t * K + lane + 64 * p] = w[p];
+  }
+  const float* vp = a.qkv + row0 * a.row_stride + 2 * (size_t)a.kv_heads * K + (size_t)h * a.vdim;
+  for (int col = lane; col < a.vdim; col += 64) {
+    float v[DC_T];
+#pragma unroll
+    for (int t = 0; t < DC_T; ++t) v[t] = t < len ? vp[(size_t)t * a.row_stride + col] : 0.f;
+#pragma unroll
+    for (int t = 0; t < DC_T; ++t) {
+      float u = 0.f;
+#pragma unroll
+      for (int s = 0; s <= t; ++s) u = fmaf(Ts[t][s], v[s], u);
+      U0[(size_t)t * a.vdim + col] = u;
+    }
+  }
+}
+
+// CT: tiles of 16 value columns a block.
+template <int KT, int CT>
+__global__ __launch_bounds__(256) void delta_chunk_scan_kernel(DeltaChunkArgs a) {
+  constexpr int K = 16 * KT, TILES = KT / 4;      // 16-channel tiles of a wave
+  __shared__ f32x4_d part[2][4][2 * CT][TP_WAVE];
+  const int lane = threadIdx.x % TP_WAVE, wave = threadIdx.x / TP_WAVE, col = lane % 16, quad = lane / 16;
+  // The blocks of a head read the same W, Q~ and K^: they go side by side to one XCD and its L2, and the heads to the XCDs in turn.
+  const int strips = a.vdim / (16 * CT), pairs = a.requests * a.heads;
+  const int rest = blockIdx.x >> 3, pair = rest / strips * 8 + (blockIdx.x & 7), strip = rest % strips;
+  if (pair >= pairs) return;
+  const int h = pair % a.heads, r = pair / a.heads;
+  const int run0 = a.cu_seqlens[r], left = a.cu_seqlens[r + 1] - run0 - a.first;
+  const int groups = min(a.groups, (left + DC_T - 1) / DC_T);
+  if (groups <= 0) return;
+  const int j0 = strip * 16 * CT + col, i0 = wave * TILES * 16;      // (this lane's columns: j0 + 16 n)
+  const size_t size = dc_item_floats(K, a.vdim);
+  const float* item = a.scratch + ((size_t)r * a.groups * a.heads + h) * size;
+  float* Sm = a.state + (size_t)a.state_slots[r] * a.state_stride + a.state_off + ((size_t)h * a.vdim + j0) * K;
+  f32x4_d S[CT][TILES];
+#pragma unroll
+  for (int n = 0; n < CT; ++n)
+#pragma unroll
+    for (int m = 0; m < TILES; ++m)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) S[n][m][i] = Sm[(size_t)16 * n * K + i0 + 16 * m + 4 * quad + i];
+  struct Group {
+    f32x4_d w[TILES], q[TILES], k[TILES], g[TILES], b, d, u[CT];
+  };
+  auto fetch = [&](Group& x, int c) {
+    const float* p = item + (size_t)c * a.heads * size;
+#pragma unroll
+    for (int m = 0; m < TILES; ++m) {
+      x.w[m] = *(const f32x4_d*)(p + (size_t)col * K + i0 + 16 * m + 4 * quad);
+      x.q[m] = *(const f32x4_d*)(p + (size_t)(DC_T + col) * K + i0 + 16 * m + 4 * quad);
+      x.k[m] = *(const f32x4_d*)(p + (size_t)2 * DC_T * K + (size_t)(i0 + 16 * m + col) * DC_T + 4 * quad);
+      x.g[m] = *(const f32x4_d*)(p + (size_t)3 * DC_T * K + i0 + 16 * m + 4 * quad);
+    }
+    x.b = *(const f32x4_d*)(p + (size_t)49 * K + col * DC_T + 4 * quad);
+    x.d = *(const f32x4_d*)(p + (size_t)49 * K + 256 + 4 * quad);
+#pragma unroll
+    for (int n = 0; n < CT; ++n)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) x.u[n][i] = p[(size_t)49 * K + 272 + (size_t)(4 * quad + i) * a.vdim + j0 + 16 * n];
+  };
+  auto step = [&](const Group& x, int c) {
+    f32x4_d(*buf)[2 * CT][TP_WAVE] = part[c & 1];
+#pragma unroll
+    for (int n = 0; n < CT; ++n) {
+      f32x4_d ws[2], qs[2];
+#pragma unroll
+      for (int m = 0; m < TILES; ++m)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const bool first = m == 0 && i < 2;
+          ws[i % 2] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.w[m][i], S[n][m][i], first ? (f32x4_d)(0.f) : ws[i % 2], 0, 0, 0);
+          qs[i % 2] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.q[m][i], S[n][m][i], first ? (f32x4_d)(0.f) : qs[i % 2], 0, 0, 0);
+        }
+      buf[wave][2 * n][lane] = ws[0] + ws[1];
+      buf[wave][2 * n + 1][lane] = qs[0] + qs[1];
+    }
+#pragma unroll
+    for (int n = 0; n < CT; ++n)
+#pragma unroll
+      for (int m = 0; m < TILES; ++m) S[n][m] *= x.g[m];
+    __syncthreads();      // (the buffer of the group before is free again behind this one)
+#pragma unroll
+    for (int n = 0; n < CT; ++n) {
+      const f32x4_d u = x.u[n] - ((buf[0][2 * n][lane] + buf[1][2 * n][lane]) + (buf[2][2 * n][lane] + buf[3][2 * n][lane]));
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int m = 0; m < TILES; ++m) S[n][m] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.k[m][i], u[i], S[n][m], 0, 0, 0);
+      if (wave == ((c + n) & 3)) {      // (the waves write the rows in turn)
+        const int q0 = 2 * n + 1;
+        f32x4_d o = (buf[0][q0][lane] + buf[1][q0][lane]) + (buf[2][q0][lane] + buf[3][q0][lane]);
+        float odd = 0.f;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) odd = fmaf(u[i], 0.f, odd);
+        if (__any(!(odd == 0.f))) {
+          // (a zero of B times a u that is not finite would reach tokens before it: added one by one)
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            for (int s = 0; s < DC_T; ++s) {
+              const float v0 = __shfl(u[0], (s / 4) * 16 + col, TP_WAVE), v1 = __shfl(u[1], (s / 4) * 16 + col, TP_WAVE);
+              const float v2 = __shfl(u[2], (s / 4) * 16 + col, TP_WAVE), v3 = __shfl(u[3], (s / 4) * 16 + col, TP_WAVE);
+              const float us = s % 4 == 0 ? v0 : s % 4 == 1 ? v1 : s % 4 == 2 ? v2 : v3;
+              if (s < 4 * quad + i) o[i] = fmaf(item[(size_t)c * a.heads * size + (size_t)49 * K + (4 * quad + i) * DC_T + s], us, o[i]);
+            }
+        } else {
+          f32x4_d bu = (f32x4_d)(0.f);
+#pragma unroll
+          for (int i = 0; i < 4; ++i) bu = __builtin_amdgcn_mfma_f32_16x16x4f32(x.b[i], u[i], bu, 0, 0, 0);
+          o += bu;
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int t = c * DC_T + 4 * quad + i;
+          // (a token's own part, most of the sum where decays are strong, is added last: one rounding at its size)
+          if (t < left) a.y[((size_t)(run0 + a.first + t) * a.heads + h) * a.vdim + j0 + 16 * n] = fmaf(u[i], x.d[i], o[i]);
+        }
+      }
+    }
+  };
+  Group x, y;
+  fetch(x, 0);
+  for (int c = 0; c < groups; c += 2) {
+    if (c + 1 < groups) fetch(y, c + 1);
+    step(x, c);
+    if (c + 1 < groups) {
+      if (c + 2 < groups) fetch(x, c + 2);
+      step(y, c + 1);
+    }
+  }
+#pragma unroll
+  for (int n = 0; n < CT; ++n)
+#pragma unroll
+    for (int m = 0; m < TILES; ++m)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) Sm[(size_t)16 * n * K + i0 + 16 * m + 4 * quad + i] = S[n][m][i];
+}
+
+// Groups of a run that one pair of launches takes, 0: the runs are not these kernels'.  The scratch is held to a quarter of a GB: longer
+// runs of many heads and requests take several pairs, each from the state that the one before left.
+static int dc_groups(int n_req, int max_run, int heads, int dim, int vdim) {
+  // (16 heads of 128 x 128, one run, single tokens / groups: 64 tokens 25 / 28 us, 96 33 / 32, 128 41 / 31)
+  if (max_run <= 96 || (dim != 64 && dim != 128) || vdim % 16 != 0) return 0;
+  const size_t group = (size_t)n_req * heads * dc_item_floats(dim, vdim), limit = (size_t)64 << 20;
+  const long all = (max_run + DC_T - 1) / DC_T, fit = (long)(limit / group);
+  if (fit < 1 || (long)n_req * heads * (fit < all ? fit : all) >= 0x7fffffffL || ((long)n_req * heads + 8) * (vdim / 16) >= 0x7fffffffL) return 0;
+  return (int)(fit < all ? fit : all);
+}
+
+// Floats of scratch for runs of up to max_run tokens (0: they go token by token).
+extern "C" size_t tp_delta_scan_scratch(int n_req, int max_run, int heads, int dim, int vdim) {
+  if (n_req <= 0 || heads <= 0 || dim <= 0 || vdim <= 0) return 0;
+  return (size_t)dc_groups(n_req, max_run, heads, dim, vdim) * n_req * heads * dc_item_floats(dim, vdim);
+}
+
+// Returns 0 when it took the runs, -1 when they are not its own.  q and k of qkv are read as they come, before they are unit vectors.
+int tp_delta_chunks(const float* qkv, int row_stride, const float* decay, const float* proj, int proj_stride, int beta_col0, float* state,
+                    size_t state_stride, size_t state_off, const int* cu_seqlens, const int* state_slots, float* y, int n_req, int heads,
+                    int kv_heads, int dim, int vdim, float q_scale, float unit_eps, int max_run, float* scratch, size_t scratch_floats,
+                    hipStream_t s) {
+  const int groups = dc_groups(n_req, max_run, heads, dim, vdim);
+  if (groups == 0 || scratch == nullptr || ((uintptr_t)scratch & 15) || scratch_floats < tp_delta_scan_scratch(n_req, max_run, heads, dim, vdim)) return -1;
+  DeltaChunkArgs a{qkv, decay, proj, state, cu_seqlens, state_slots, y, scratch, state_stride, state_off, row_stride, proj_stride, beta_col0,
+                   heads, kv_heads, vdim, n_req, 0, groups, q_scale, unit_eps};
+  const long pairs = ((long)n_req * heads + 7) / 8 * 8;
+  // (32 columns a block read W, Q~ and K^ half as often, which bounds the chain once there are more blocks of 16 columns than the two
+  // a CU that run at a time: 16 heads of 128 x 128, four runs of 451 tokens, 512 blocks of 16 columns or half as many of 32: 94 / 102 us;
+  // 32 heads, eight runs of 256, 2,048 blocks: 202 / 174)
+  const bool wide = vdim % 32 == 0 && pairs * (vdim / 16) > 512;
+  const dim3 prep((unsigned)((long)n_req * groups * heads)), scan((unsigned)(pairs * (vdim / (wide ? 32 : 16))));
+#define DC_SCAN(KT_)                                                                                                 \
+  do {                                                                                                               \
+    if (wide) hipLaunchKernelGGL((delta_chunk_scan_kernel<KT_, 2>), scan, dim3(256), 0, s, a);                       \
+    else hipLaunchKernelGGL((delta_chunk_scan_kernel<KT_, 1>), scan, dim3(256), 0, s, a);                            \
+  } while (0)
+  for (; a.first < max_run; a.first += groups * DC_T) {
+    if (dim == 128) {
+      hipLaunchKernelGGL(delta_chunk_prep_kernel<2>, prep, dim3(64), 0, s, a);
+      DC_SCAN(8);
+    } else {
+      hipLaunchKernelGGL(delta_chunk_prep_kernel<1>, prep, dim3(64), 0, s, a);
+      DC_SCAN(4);
+    }
+  }
+#undef DC_SCAN
+  return 0;
+}

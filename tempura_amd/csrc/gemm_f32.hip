@@ -11,34 +11,12 @@
 // without packed instructions, and need one LDS read for four of them, so one pipeline of two LDS stages is enough.  611 rows:
 // 3,072 x 3,072 119 us, 16,384 x 3,072 594 us (97 and 104 TFLOP/s; the general kernel 477 and 2,060 us); 2,048 rows of the latter 1,650 us (125).
 #include "common.h"
+#include "column_sum.h"
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 // ---- up to 16 rows --------------------------------------------------------------------------------------------------------------
-// Adds v[i] over the lanes of a wave for NV values at once: each step halves the values a lane still carries, NV - 1 exchanges
-// (and single ones below NV lanes) instead of 6 NV.  The pairs added are those of an ordinary exchange tree from distance 32
-// down, so a sum's bits do not depend on NV.  The lanes with equal lane / (64 / NV) then hold the sum of value lane / (64 / NV).
-template <int N, int W>
-__device__ inline void lanes_transpose_step(float* v, int lane) {
-  if constexpr (N > 1) {
-    const bool hi = lane & W;
-#pragma unroll
-    for (int i = 0; i < N / 2; ++i) {
-      const float keep = hi ? v[i + N / 2] : v[i], send = hi ? v[i] : v[i + N / 2];
-      v[i] = keep + __shfl_xor(send, W, TP_WAVE);
-    }
-  } else {
-    v[0] += __shfl_xor(v[0], W, TP_WAVE);
-  }
-  if constexpr (W > 1) lanes_transpose_step<(N > 1 ? N / 2 : 1), W / 2>(v, lane);
-}
-template <int NV>
-__device__ inline float lanes_transpose_sum(float (&v)[NV], int lane) {
-  lanes_transpose_step<NV, TP_WAVE / 2>(v, lane);
-  return v[0];
-}
-
 #define FR_WAVES 4
 
 // MC: rows of the block's registers (M <= MC), C: weight rows a block owns.

@@ -1712,13 +1712,14 @@ def lowrank_up(x: torch.Tensor, col0: int, weight_t: torch.Tensor, mode: str = "
 
 def delta_scan(qkv: torch.Tensor, decay: torch.Tensor, proj: torch.Tensor, beta_col0: int, state: torch.Tensor, state_off: int,
                cu_seqlens: torch.Tensor, state_slots: torch.Tensor, num_requests: int, heads: int, kv_heads: int, dim: int,
-               vdim: int, q_scale: float, unit_eps: float) -> torch.Tensor:
+               vdim: int, q_scale: float, unit_eps: float, max_run: int = 0) -> torch.Tensor:
     """The gated delta rule per head over each request's run.  ``qkv`` float32 [n, q | k | v] with q and k
     [kv_heads * dim] and v [heads * vdim]; q and k are made unit vectors per head (x / sqrt(sum x^2 + unit_eps), q times
     ``q_scale``); beta = sigmoid(proj[:, beta_col0 + h]); ``decay`` float32 [n, heads * dim].  Per head, with S
     [dim, vdim] (kept at ``state[slot, state_off:]`` column by column, [heads, vdim, dim]):  S <- decay * S;  u = beta (v - S^T k);  S <- S + k u^T;  o = S^T q.
-    Returns o float32 [n, heads * vdim]; the state is left as the run leaves it.  (q and k of ``qkv`` are left as
-    unit vectors: the rows are a temporary of the caller's.)"""
+    Returns o float32 [n, heads * vdim]; the state is left as the run leaves it.  (q and k of ``qkv`` may be left as
+    unit vectors: the rows are a temporary of the caller's.)  ``max_run``: the longest run (0: not known); long runs go by groups of
+    tokens, which changes rounding only."""
     if _backend is not None:
         return _backend.delta_scan(qkv, decay, proj, beta_col0, state, state_off, cu_seqlens, state_slots, num_requests, heads,
                                    kv_heads, dim, vdim, q_scale, unit_eps)
@@ -1734,9 +1735,15 @@ def delta_scan(qkv: torch.Tensor, decay: torch.Tensor, proj: torch.Tensor, beta_
     _i32(state_slots, num_requests, "state_slots")
     y = torch.empty((n, heads * vdim), dtype=torch.float32, device=qkv.device)
     kq = torch.empty((n, kv_heads), dtype=torch.float32, device=qkv.device)      # k . q per token and key head
+    max_run = min(int(max_run), n)
+    lib = _Library.get()
+    lib.tp_delta_scan_scratch.restype = ctypes.c_size_t
+    need = lib.tp_delta_scan_scratch(int(num_requests), max_run, int(heads), int(dim), int(vdim)) if allow_mfma else 0
+    scratch = torch.empty((need,), dtype=torch.float32, device=qkv.device) if need else None
     _call("tp_delta_scan", _ptr(qkv), qkv.shape[1], _ptr(decay), _ptr(proj), proj.shape[1], int(beta_col0), _ptr(state),
           ctypes.c_size_t(state.shape[1]), ctypes.c_size_t(state_off), _ptr(cu_seqlens), _ptr(state_slots), _ptr(y), _ptr(kq), n,
-          int(num_requests), int(heads), int(kv_heads), int(dim), int(vdim), ctypes.c_float(q_scale), ctypes.c_float(unit_eps), _stream())
+          int(num_requests), int(heads), int(kv_heads), int(dim), int(vdim), ctypes.c_float(q_scale), ctypes.c_float(unit_eps),
+          max_run, _ptr(scratch), ctypes.c_size_t(need), _stream())
     return y
 
 

@@ -100,7 +100,7 @@ class GatedDeltaMixer(BranchMixer):
         gate = ops.lowrank_up(proj, col0 + self.g1_col, self.g2_t, "sigmoid")
         o = ops.delta_scan(qkv, decay, proj, col0 + self.beta_col, cache.state, self.state_off + self.conv_floats, ctx.cu_seqlens,
                            ctx.state_slots, ctx.num_requests, self.num_heads, self.num_kv_heads, self.head_dim, self.value_dim,
-                           self.q_scale, self.unit_eps)
+                           self.q_scale, self.unit_eps, max_run=ctx.max_q_len)
         ops.head_norm_gate(o, self.norm_w, gate, self.norm_eps, scale, self.num_heads, out, out_col0)
 
 

@@ -72,3 +72,72 @@ def test_selective_scan_keeps_what_is_not_finite_where_it_belongs(bad, where):
     finite = [torch.isfinite(y) for y in res]
     assert not finite[0].all() and torch.equal(finite[0][:t], torch.ones_like(finite[0][:t])) and torch.equal(finite[0], finite[1])
     assert float((res[0] - res[1])[finite[0]].abs().max()) <= 2e-5 * float(res[1][finite[0]].abs().max())
+
+
+def _delta_inputs(lens, H, G, D, Dv, seed, low):
+    g = torch.Generator().manual_seed(seed)
+    n = sum(lens)
+    cu = torch.tensor([0] + list(torch.tensor(lens).cumsum(0)), dtype=torch.int32)
+    slots = torch.randperm(len(lens) + 2, generator=g)[: len(lens)].to(torch.int32)
+    state = torch.randn(len(lens) + 2, 5 + H * D * Dv, generator=g) * 0.3
+    qkv = torch.randn(n, 2 * G * D + H * Dv, generator=g)
+    qkv[:, G * D: 2 * G * D] += 0.8 * torch.randn(1, G * D, generator=g)      # (keys that share a direction: the system is not near the identity)
+    decay, proj = low + (1.0 - low) * torch.rand(n, H * D, generator=g), torch.randn(n, H + 3, generator=g) * 2
+    return qkv, decay, proj, state, cu, slots
+
+
+@pytest.mark.parametrize("H,G,D,Dv", [(2, 2, 64, 16), (4, 2, 128, 48), (3, 1, 64, 128), (2, 2, 128, 128)])
+@pytest.mark.parametrize("lens,low", [([97], 0.9), ([300, 1, 15, 16, 17], 0.99), ([65, 129], 0.0), ([1000], 0.98)])
+def test_delta_rule_by_groups_of_tokens(H, G, D, Dv, lens, low):
+    from tempura_amd.kernels import ops
+    qkv, decay, proj, state, cu, slots = _delta_inputs(lens, H, G, D, Dv, H * D + len(lens), low)
+    s_ref = state.clone()
+    want = emu.delta_scan(qkv, decay, proj, 2, s_ref, 5, cu, slots, len(lens), H, G, D, Dv, D ** -0.5, 1e-6)
+    dev = [t.to(DEV) for t in (decay, proj, cu, slots)]
+    out = []
+    for max_run in (max(lens), 0):
+        s = state.to(DEV)
+        y = ops.delta_scan(qkv.to(DEV), dev[0], dev[1], 2, s, 5, dev[2], dev[3], len(lens), H, G, D, Dv, D ** -0.5, 1e-6, max_run=max_run)
+        spare = [i for i in range(len(lens) + 2) if i not in slots.tolist()]
+        assert torch.equal(s.cpu()[:, :5], state[:, :5]) and torch.equal(s.cpu()[spare], state[spare])
+        out.append((y, s))
+    for i, ref in enumerate((want, s_ref)):
+        groups, walk = _error(out[0][i], ref), _error(out[1][i], ref)
+        # (root mean squares; a group's sums are no longer chains of roundings than the same tokens' one after the other)
+        assert groups <= 1.25 * walk and groups <= 2e-6, (i, groups, walk)
+
+
+def test_delta_rule_in_several_pairs_of_launches():
+    """More tokens, heads and requests than the scratch holds at a time: each pair of launches goes on from the state of the one before."""
+    from tempura_amd.kernels import ops
+    H, D, Dv, lens = 32, 128, 128, [1200, 700, 3] + [1] * 21
+    lib = ops.library()
+    lib.tp_delta_scan_scratch.restype = __import__("ctypes").c_size_t
+    item = 49 * D + 272 + 16 * Dv
+    groups = lib.tp_delta_scan_scratch(len(lens), max(lens), H, D, Dv) // (item * H * len(lens))
+    assert 1 <= groups < -(-max(lens) // 16) and groups * item * H * len(lens) <= 64 << 20
+    qkv, decay, proj, state, cu, slots = _delta_inputs(lens, H, H, D, Dv, 5, 0.9)
+    dev = [t.to(DEV) for t in (decay, proj, cu, slots)]
+    out = []
+    for max_run in (max(lens), 0):
+        s = state.to(DEV)
+        out.append((ops.delta_scan(qkv.to(DEV), dev[0], dev[1], 2, s, 5, dev[2], dev[3], len(lens), H, H, D, Dv, D ** -0.5, 1e-6, max_run=max_run), s))
+    assert _error(out[0][0], out[1][0].cpu()) <= 1e-6 and _error(out[0][1], out[1][1].cpu()) <= 1e-6
+
+
+@pytest.mark.parametrize("bad", [float("inf"), float("nan")])
+@pytest.mark.parametrize("where", ["q", "k", "v", "beta"])
+def test_delta_rule_keeps_what_is_not_finite_where_it_belongs(bad, where):
+    from tempura_amd.kernels import ops
+    H, D, Dv, t = 2, 64, 32, 77
+    qkv, decay, proj, state, cu, slots = _delta_inputs([200], H, H, D, Dv, 9, 0.9)
+    if where == "beta":
+        proj[t, 2 + 1] = float("nan")
+    else:
+        qkv[t, {"q": D + 3, "k": 3 * D + 3, "v": 4 * D + Dv + 3}[where]] = bad
+    dev = [v.to(DEV) for v in (decay, proj, cu, slots)]
+    res = [ops.delta_scan(qkv.to(DEV), dev[0], dev[1], 2, state.to(DEV), 5, dev[2], dev[3], 1, H, H, D, Dv, D ** -0.5, 1e-6, max_run=m).cpu()
+           for m in (200, 0)]
+    finite = [torch.isfinite(y) for y in res]
+    assert not finite[0].all() and finite[0][:t].all() and torch.equal(finite[0], finite[1])
+    assert float((res[0] - res[1])[finite[0]].abs().max()) <= 2e-6 * float(res[1][finite[0]].abs().max())

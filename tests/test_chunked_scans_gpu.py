@@ -141,3 +141,19 @@ def test_delta_rule_keeps_what_is_not_finite_where_it_belongs(bad, where):
     finite = [torch.isfinite(y) for y in res]
     assert not finite[0].all() and finite[0][:t].all() and torch.equal(finite[0], finite[1])
     assert float((res[0] - res[1])[finite[0]].abs().max()) <= 2e-6 * float(res[1][finite[0]].abs().max())
+
+
+@pytest.mark.parametrize("H,P,N,G", [(4, 8, 16, 2), (2, 24, 5, 1), (6, 40, 56, 2), (3, 64, 128, 3), (1, 41, 600, 1), (2, 16, 1100, 1), (8, 16, 30, 1)])
+@pytest.mark.parametrize("off", [7, 8])
+def test_selective_scan_of_single_tokens(H, P, N, G, off):
+    """A kernel of its own, with the sums of the one that walks runs: the same bits, outputs and states; a request without a token is left alone."""
+    from tempura_amd.kernels import ops
+    xbc, proj, consts, state, _, slots = _scan_inputs([1, 1, 1], H, P, N, G, H + N)
+    cu = torch.tensor([0, 1, 1, 2, 3], dtype=torch.int32)
+    slots, state = torch.tensor([2, 0, 4, 1], dtype=torch.int32), torch.cat([torch.zeros(5, off - 7), state], dim=1).contiguous()
+    dev, dc, out = [t.to(DEV) for t in (xbc, proj, cu, slots)], [c.to(DEV) for c in consts], []
+    for max_run in (1, 2):
+        s = state.to(DEV)
+        out.append((ops.ssm_scan(dev[0], dev[1], 2, *dc, s, off, dev[2], dev[3], 4, H, P, N, G, max_run=max_run), s))
+    assert torch.equal(out[0][0], out[1][0]) and torch.equal(out[0][1], out[1][1])
+    assert torch.equal(out[0][1][0].cpu(), state[0]) and not torch.equal(out[0][1][2].cpu(), state[2])

@@ -1366,13 +1366,12 @@ __global__ __launch_bounds__(64) void attn_combine_kernel(const float* __restric
       for (int u = 0; u < 8; ++u) acc = fmaf(__shfl(ws, s + u, 64), v[u], acc);
     }
     for (; s < num_splits; ++s) acc = fmaf(__shfl(ws, s, 64), base[(size_t)s * (D + 2) + d], acc);
-    const bf16_t y = float_to_bf16(acc * inv);
     if constexpr (GATED) {
-      float v = bf16_to_float(y);
+      float v = bf16_to_float(float_to_bf16(acc * inv));
       if (gate.rows != nullptr) v *= 1.0f / (1.0f + expf(-raw));
       if (d0 + lane < D) out[(size_t)q_start * gate.out_stride + gate.out_col0 + h * D + d] = float_to_bf16(v * gate.scale);
     } else if (d0 + lane < D) {
-      out[((size_t)q_start * n_heads + h) * D + d] = y;
+      out[((size_t)q_start * n_heads + h) * D + d] = float_to_bf16(acc * inv);
     }
   }
 }

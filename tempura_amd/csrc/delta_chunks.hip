@@ -3,16 +3,24 @@
 //
 // Within 16 tokens, with G_t the product of the decays up to token t and S the state before them, the rule is a small linear system:
 //   A[t, s] = sum_c k_t k_s (G_t / G_s)  (s < t),  B[t, s] the same with q_t (s <= t),  T = (I + diag(beta) A)^-1 diag(beta)
-//   U = T V - (T K~) S  with K~_t = G_t k_t;   o = Q~ S + B U  with Q~_t = G_t q_t;   S <- G_16 S + K^T U  with K^_s = (G_16 / G_s) k_s
-// Everything but the three products with S is independent of the state: delta_chunk_prep_kernel works it out for all groups of 16 side by
-// side, a wave each, and leaves W = T K~, Q~, K^, B and T V in scratch; the ratios of decays are running products, never quotients, so
+//   U = T (V - K~ S)  with K~_t = G_t k_t;   o = Q~ S + B U  with Q~_t = G_t q_t;   S <- G_16 S + K^T U  with K^_s = (G_16 / G_s) k_s
+// Everything but the products with S and U is independent of the state: delta_chunk_prep_kernel works it out for all groups of 16 side by
+// side, a wave each, and leaves K~, Q~, K^, T and B in scratch; the ratios of decays are running products, never quotients, so
 // nothing overflows.  delta_chunk_scan_kernel is the chain over the groups: a block of four waves owns 16 value columns of a head, a wave
-// a quarter of the key channels in accumulators, which lie as the next product's operand wants them; the waves' parts of W S and Q~ S meet
+// a quarter of the key channels in accumulators, which lie as the next product's operand wants them; the waves' parts of K~ S and Q~ S meet
 // in LDS once a group.
+//
+// The rounding is held to that of the chain of single tokens: the products of decays that act on the state (G, K~, Q~, K^) run in float64,
+// the sums A and B over the channels are added in float64 from the second level of their tree on, and a group's tokens lie so that every
+// matrix-core product adds them in ascending order (DC_PLACE): the tokens nearest to a result, which strong decays leave as most of it,
+// are added last, where a sum's roundings are few.  Root mean square error against float64 over that of the chain, runs of 112, 300 and
+// 1,000 tokens: decays of 0 to 1 a token 0.91 (states 0.99), 0.5 to 1 0.93 (0.97), 0.8 to 1 0.96 (0.95), 0.9 to 1 0.94 (0.92), 0.99 to 1
+// 0.82 (0.81).  (In float32 throughout, tokens in the order of the rows and U = T V - (T K~) S it was 1.03, 1.06, 1.08, 1.06 and 0.94;
+// one run of 2,048 tokens then took 204 us, now 223, four of 450 tokens 94 and 95.)
 //
 // The chain of single tokens is bound by what a wave issues and waits for a token, 0.25 to 0.55 us; here a group of 16 takes 1.3 us (its
 // products, a meeting in LDS and the update, each waiting for the one before).  16 heads of 128 x 128, single tokens / groups: one run of
-// 128 tokens 41 / 31 us, 256 75 / 42, 2,048 512 / 202; four runs of 451 tokens 171 / 94 (a third of it the first kernel).
+// 128 tokens 41 / 31 us, 256 75 / 42, 2,048 500 / 223; four runs of 450 tokens 160 / 95 (a third of it the first kernel).
 #include <math.h>
 
 #include "common.h"
@@ -38,13 +46,45 @@ struct DeltaChunkArgs {
   float q_scale, unit_eps;
 };
 
-// floats of scratch for one group of one head: W, Q~ [16, dim], K^ [dim, 16], G_16 [dim], B [16, 16] without its diagonal, that [16],
-// T V [16, vdim]
-__host__ __device__ inline size_t dc_item_floats(int dim, int vdim) { return (size_t)49 * dim + 272 + (size_t)16 * vdim; }
+// Where a token of the group lies among the rows and columns of the operands: instruction i of a product over the tokens takes element i
+// of each lane, from lanes quad = 0 .. 3, so with token 4 i + quad at place 4 quad + i the instructions run through the tokens in order.
+// (Its own inverse.)
+#define DC_PLACE(t) (4 * ((t) % 4) + (t) / 4)
+
+// floats of scratch for one group of one head: K~, Q~ [16, dim], K^ [dim, 16], G_16 [dim], T [16, 16], B [16, 16] without its diagonal,
+// that [16]; tokens at their places
+__host__ __device__ inline size_t dc_item_floats(int dim) { return (size_t)49 * dim + 528; }
 
 // places of the sums: for s B(s, s), then A(t, s), B(t, s) of t = s + 1 .. 15
 #define DC_B(t, s) (32 * (s) - (s) * (s) + 2 * ((t) - (s)))
 #define DC_A(t, s) (DC_B(t, s) - 1)
+
+// The sums over the lanes of a wave of 64 values, lane i the i-th's: lanes_transpose_sum's tree (distance 32 down to 1), in float64 behind
+// its first level.  The two widest levels are the instructions that swap halves or odd rows with even ones.
+__device__ inline float dc_sum64(const float (&v)[64], int lane) {
+  double d[32];
+#pragma unroll
+  for (int i = 0; i < 32; ++i) {
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v[i]), __float_as_uint(v[i + 32]), false, false);
+    d[i] = (double)(__uint_as_float(r[0]) + __uint_as_float(r[1]));
+  }
+#pragma unroll
+  for (int i = 0; i < 16; ++i) {
+    const auto lo = __builtin_amdgcn_permlane16_swap(__double2loint(d[i]), __double2loint(d[i + 16]), false, false);
+    const auto hi = __builtin_amdgcn_permlane16_swap(__double2hiint(d[i]), __double2hiint(d[i + 16]), false, false);
+    d[i] = __hiloint2double(hi[0], lo[0]) + __hiloint2double(hi[1], lo[1]);
+  }
+#pragma unroll
+  for (int w = 8; w > 0; w /= 2) {
+    const bool up = lane & w;
+#pragma unroll
+    for (int i = 0; i < w; ++i) {
+      const double keep = up ? d[i + w] : d[i], send = up ? d[i] : d[i + w];
+      d[i] = keep + __shfl_xor(send, w, TP_WAVE);
+    }
+  }
+  return (float)d[0];
+}
 
 // (a recursion: every place of v is then known to the compiler, which keeps v in registers)
 template <int S, int PER>
@@ -64,10 +104,10 @@ __device__ inline void dc_dots(const float (&q)[DC_T][PER], const float (&k)[DC_
     }
     if (t > S) {
       v[DC_A(t, S) % 64] = da;
-      if (DC_A(t, S) % 64 == 63) dots[DC_A(t, S) - 63 + lane] = lanes_transpose_sum<64>(v, lane);
+      if (DC_A(t, S) % 64 == 63) dots[DC_A(t, S) - 63 + lane] = dc_sum64(v, lane);
     }
     v[DC_B(t, S) % 64] = db;
-    if (DC_B(t, S) % 64 == 63) dots[DC_B(t, S) - 63 + lane] = lanes_transpose_sum<64>(v, lane);
+    if (DC_B(t, S) % 64 == 63) dots[DC_B(t, S) - 63 + lane] = dc_sum64(v, lane);
   }
   if constexpr (S + 1 < DC_T) dc_dots<S + 1, PER>(q, k, gd, v, dots, lane);
 }
@@ -76,7 +116,6 @@ template <int PER>
 __global__ __launch_bounds__(64) void delta_chunk_prep_kernel(DeltaChunkArgs a) {
   constexpr int K = 64 * PER;
   __shared__ float dots[256];
-  __shared__ __attribute__((aligned(16))) float Ts[DC_T][DC_T];
   __shared__ float bs[DC_T];
   const int lane = threadIdx.x;
   const int h = blockIdx.x % a.heads, rest = blockIdx.x / a.heads, c = rest % a.groups, r = rest / a.groups;
@@ -130,27 +169,27 @@ __global__ __launch_bounds__(64) void delta_chunk_prep_kernel(DeltaChunkArgs a) 
     float v[64];
     dc_dots<0, PER>(q, k, gd, v, dots, lane);
   }
-  float* item = a.scratch + (((size_t)r * a.groups + c) * a.heads + h) * dc_item_floats(K, a.vdim);
-  float *W = item, *Q = W + DC_T * K, *KT = Q + DC_T * K, *G = KT + DC_T * K, *B = G + K, *U0 = B + 272;
-  // G_16, Q~, K~ (in k's place, after K^ has been made of it)
+  float* item = a.scratch + (((size_t)r * a.groups + c) * a.heads + h) * dc_item_floats(K);
+  float *Kt = item, *Q = Kt + DC_T * K, *KT = Q + DC_T * K, *G = KT + DC_T * K, *T = G + K, *B = T + 256, *diag = B + 256;
 #pragma unroll
   for (int p = 0; p < PER; ++p) {
     const int ch = lane + 64 * p;
-    float tail = 1.f, kt[DC_T];
+    double tail = 1.0;
+    float kt[DC_T];
 #pragma unroll
     for (int s = DC_T - 1; s >= 0; --s) {
-      kt[s] = k[s][p] * tail;
-      tail *= gd[s][p];
+      kt[DC_PLACE(s)] = (float)((double)k[s][p] * tail);
+      tail *= (double)gd[s][p];
     }
-    G[ch] = tail;
+    G[ch] = (float)tail;
 #pragma unroll
     for (int s = 0; s < DC_T; s += 4) *(f32x4_d*)(KT + (size_t)ch * DC_T + s) = (f32x4_d){kt[s], kt[s + 1], kt[s + 2], kt[s + 3]};
-    float head = 1.f;
+    double head = 1.0;
 #pragma unroll
     for (int t = 0; t < DC_T; ++t) {
-      head *= gd[t][p];
-      Q[t * K + ch] = q[t][p] * head;
-      k[t][p] *= head;
+      head *= (double)gd[t][p];
+      Q[DC_PLACE(t) * K + ch] = (float)((double)q[t][p] * head);
+      Kt[DC_PLACE(t) * K + ch] = (float)((double)k[t][p] * head);
     }
   }
   __syncthreads();
@@ -163,41 +202,36 @@ __global__ __launch_bounds__(64) void delta_chunk_prep_kernel(DeltaChunkArgs a) 
 #pragma unroll
       for (int s = 0; s < t; ++s) sum = fmaf(dots[DC_A(t, s)], col[s], sum);
       col[t] = t == lane ? bs[t] : t > lane ? -bs[t] * sum : 0.f;
-      Ts[t][lane] = col[t];
+      T[DC_PLACE(t) * DC_T + DC_PLACE(lane)] = col[t];
     }
+    diag[DC_PLACE(lane)] = dots[DC_B(lane, lane)];
   }
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
-    const int e = lane + 64 * i, t = e / DC_T, s = e % DC_T;
+    const int e = lane + 64 * i, t = DC_PLACE(e / DC_T), s = DC_PLACE(e % DC_T);
     B[e] = s < t ? dots[DC_B(t, s)] : 0.f;
   }
-  if (lane < DC_T) B[256 + lane] = dots[DC_B(lane, lane)];
-  __syncthreads();
+}
+
+// sum over s of M[token, s] x_s for this lane's four tokens (place 4 quad + i) and its column, one product after the other, M [16, 16] in
+// scratch; s <= t, or s < t.  For values that are not finite: a matrix-core product multiplies them with zeros as well.
+template <bool OWN>
+__device__ inline f32x4_d dc_lower(const float* M, const f32x4_d& x, f32x4_d sum, int col, int quad) {
 #pragma unroll
-  for (int t = 0; t < DC_T; ++t) {
-    float w[PER];
+  for (int s = 0; s < DC_T; ++s) {
+    const float xs = __shfl(x[s / 4], (s % 4) * 16 + col, TP_WAVE);
 #pragma unroll
-    for (int p = 0; p < PER; ++p) w[p] = 0.f;
-#pragma unroll
-    for (int s = 0; s <= t; ++s)
-#pragma unroll
-      for (int p = 0; p < PER; ++p) w[p] = fmaf(Ts[t][s], k[s][p], w[p]);
-#pragma unroll
-    for (int p = 0; p < PER; ++p) W[t * K + lane + 64 * p] = w[p];
+    for (int i = 0; i < 4; ++i)
+      if (OWN ? s <= 4 * i + quad : s < 4 * i + quad) sum[i] = fmaf(M[(4 * quad + i) * DC_T + DC_PLACE(s)], xs, sum[i]);
   }
-  const float* vp = a.qkv + row0 * a.row_stride + 2 * (size_t)a.kv_heads * K + (size_t)h * a.vdim;
-  for (int col = lane; col < a.vdim; col += 64) {
-    float v[DC_T];
+  return sum;
+}
+
+__device__ inline bool dc_finite(const f32x4_d& x) {
+  float odd = 0.f;
 #pragma unroll
-    for (int t = 0; t < DC_T; ++t) v[t] = t < len ? vp[(size_t)t * a.row_stride + col] : 0.f;
-#pragma unroll
-    for (int t = 0; t < DC_T; ++t) {
-      float u = 0.f;
-#pragma unroll
-      for (int s = 0; s <= t; ++s) u = fmaf(Ts[t][s], v[s], u);
-      U0[(size_t)t * a.vdim + col] = u;
-    }
-  }
+  for (int i = 0; i < 4; ++i) odd = fmaf(x[i], 0.f, odd);
+  return !__any(!(odd == 0.f));
 }
 
 // CT: tiles of 16 value columns a block.
@@ -215,7 +249,8 @@ __global__ __launch_bounds__(256) void delta_chunk_scan_kernel(DeltaChunkArgs a)
   const int groups = min(a.groups, (left + DC_T - 1) / DC_T);
   if (groups <= 0) return;
   const int j0 = strip * 16 * CT + col, i0 = wave * TILES * 16;      // (this lane's columns: j0 + 16 n)
-  const size_t size = dc_item_floats(K, a.vdim);
+  const size_t size = dc_item_floats(K);
+  const float* vcol = a.qkv + (size_t)(run0 + a.first) * a.row_stride + 2 * (size_t)a.kv_heads * K + (size_t)h * a.vdim + j0;
   const float* item = a.scratch + ((size_t)r * a.groups * a.heads + h) * size;
   float* Sm = a.state + (size_t)a.state_slots[r] * a.state_stride + a.state_off + ((size_t)h * a.vdim + j0) * K;
   f32x4_d S[CT][TILES];
@@ -226,7 +261,7 @@ __global__ __launch_bounds__(256) void delta_chunk_scan_kernel(DeltaChunkArgs a)
 #pragma unroll
       for (int i = 0; i < 4; ++i) S[n][m][i] = Sm[(size_t)16 * n * K + i0 + 16 * m + 4 * quad + i];
   struct Group {
-    f32x4_d w[TILES], q[TILES], k[TILES], g[TILES], b, d, u[CT];
+    f32x4_d w[TILES], q[TILES], k[TILES], g[TILES], t, b, d, v[CT];
   };
   auto fetch = [&](Group& x, int c) {
     const float* p = item + (size_t)c * a.heads * size;
@@ -237,12 +272,15 @@ __global__ __launch_bounds__(256) void delta_chunk_scan_kernel(DeltaChunkArgs a)
       x.k[m] = *(const f32x4_d*)(p + (size_t)2 * DC_T * K + (size_t)(i0 + 16 * m + col) * DC_T + 4 * quad);
       x.g[m] = *(const f32x4_d*)(p + (size_t)3 * DC_T * K + i0 + 16 * m + 4 * quad);
     }
-    x.b = *(const f32x4_d*)(p + (size_t)49 * K + col * DC_T + 4 * quad);
-    x.d = *(const f32x4_d*)(p + (size_t)49 * K + 256 + 4 * quad);
+    x.t = *(const f32x4_d*)(p + (size_t)49 * K + col * DC_T + 4 * quad);
+    x.b = *(const f32x4_d*)(p + (size_t)49 * K + 256 + col * DC_T + 4 * quad);
+    x.d = *(const f32x4_d*)(p + (size_t)49 * K + 512 + 4 * quad);
 #pragma unroll
-    for (int n = 0; n < CT; ++n)
+    for (int i = 0; i < 4; ++i) {
+      const int t = c * DC_T + 4 * i + quad;
 #pragma unroll
-      for (int i = 0; i < 4; ++i) x.u[n][i] = p[(size_t)49 * K + 272 + (size_t)(4 * quad + i) * a.vdim + j0 + 16 * n];
+      for (int n = 0; n < CT; ++n) x.v[n][i] = t < left ? vcol[(size_t)t * a.row_stride + 16 * n] : 0.f;
+    }
   };
   auto step = [&](const Group& x, int c) {
     f32x4_d(*buf)[2 * CT][TP_WAVE] = part[c & 1];
@@ -267,7 +305,15 @@ __global__ __launch_bounds__(256) void delta_chunk_scan_kernel(DeltaChunkArgs a)
     __syncthreads();      // (the buffer of the group before is free again behind this one)
 #pragma unroll
     for (int n = 0; n < CT; ++n) {
-      const f32x4_d u = x.u[n] - ((buf[0][2 * n][lane] + buf[1][2 * n][lane]) + (buf[2][2 * n][lane] + buf[3][2 * n][lane]));
+      const f32x4_d e = x.v[n] - ((buf[0][2 * n][lane] + buf[1][2 * n][lane]) + (buf[2][2 * n][lane] + buf[3][2 * n][lane]));
+      const float* M = item + (size_t)c * a.heads * size + (size_t)49 * K;
+      f32x4_d u = (f32x4_d)(0.f);
+      if (dc_finite(e)) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) u = __builtin_amdgcn_mfma_f32_16x16x4f32(x.t[i], e[i], u, 0, 0, 0);
+      } else {
+        u = dc_lower<true>(M, e, u, col, quad);
+      }
 #pragma unroll
       for (int i = 0; i < 4; ++i)
 #pragma unroll
@@ -275,28 +321,17 @@ __global__ __launch_bounds__(256) void delta_chunk_scan_kernel(DeltaChunkArgs a)
       if (wave == ((c + n) & 3)) {      // (the waves write the rows in turn)
         const int q0 = 2 * n + 1;
         f32x4_d o = (buf[0][q0][lane] + buf[1][q0][lane]) + (buf[2][q0][lane] + buf[3][q0][lane]);
-        float odd = 0.f;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) odd = fmaf(u[i], 0.f, odd);
-        if (__any(!(odd == 0.f))) {
-          // (a zero of B times a u that is not finite would reach tokens before it: added one by one)
-#pragma unroll
-          for (int i = 0; i < 4; ++i)
-            for (int s = 0; s < DC_T; ++s) {
-              const float v0 = __shfl(u[0], (s / 4) * 16 + col, TP_WAVE), v1 = __shfl(u[1], (s / 4) * 16 + col, TP_WAVE);
-              const float v2 = __shfl(u[2], (s / 4) * 16 + col, TP_WAVE), v3 = __shfl(u[3], (s / 4) * 16 + col, TP_WAVE);
-              const float us = s % 4 == 0 ? v0 : s % 4 == 1 ? v1 : s % 4 == 2 ? v2 : v3;
-              if (s < 4 * quad + i) o[i] = fmaf(item[(size_t)c * a.heads * size + (size_t)49 * K + (4 * quad + i) * DC_T + s], us, o[i]);
-            }
-        } else {
+        if (dc_finite(u)) {
           f32x4_d bu = (f32x4_d)(0.f);
 #pragma unroll
           for (int i = 0; i < 4; ++i) bu = __builtin_amdgcn_mfma_f32_16x16x4f32(x.b[i], u[i], bu, 0, 0, 0);
           o += bu;
+        } else {
+          o = dc_lower<false>(M + 256, u, o, col, quad);
         }
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-          const int t = c * DC_T + 4 * quad + i;
+          const int t = c * DC_T + 4 * i + quad;
           // (a token's own part, most of the sum where decays are strong, is added last: one rounding at its size)
           if (t < left) a.y[((size_t)(run0 + a.first + t) * a.heads + h) * a.vdim + j0 + 16 * n] = fmaf(u[i], x.d[i], o[i]);
         }
@@ -326,7 +361,7 @@ __global__ __launch_bounds__(256) void delta_chunk_scan_kernel(DeltaChunkArgs a)
 static int dc_groups(int n_req, int max_run, int heads, int dim, int vdim) {
   // (16 heads of 128 x 128, one run, single tokens / groups: 64 tokens 25 / 28 us, 96 33 / 32, 128 41 / 31)
   if (max_run <= 96 || (dim != 64 && dim != 128) || vdim % 16 != 0) return 0;
-  const size_t group = (size_t)n_req * heads * dc_item_floats(dim, vdim), limit = (size_t)64 << 20;
+  const size_t group = (size_t)n_req * heads * dc_item_floats(dim), limit = (size_t)64 << 20;
   const long all = (max_run + DC_T - 1) / DC_T, fit = (long)(limit / group);
   if (fit < 1 || (long)n_req * heads * (fit < all ? fit : all) >= 0x7fffffffL || ((long)n_req * heads + 8) * (vdim / 16) >= 0x7fffffffL) return 0;
   return (int)(fit < all ? fit : all);
@@ -335,7 +370,7 @@ static int dc_groups(int n_req, int max_run, int heads, int dim, int vdim) {
 // Floats of scratch for runs of up to max_run tokens (0: they go token by token).
 extern "C" size_t tp_delta_scan_scratch(int n_req, int max_run, int heads, int dim, int vdim) {
   if (n_req <= 0 || heads <= 0 || dim <= 0 || vdim <= 0) return 0;
-  return (size_t)dc_groups(n_req, max_run, heads, dim, vdim) * n_req * heads * dc_item_floats(dim, vdim);
+  return (size_t)dc_groups(n_req, max_run, heads, dim, vdim) * n_req * heads * dc_item_floats(dim);
 }
 
 // Returns 0 when it took the runs, -1 when they are not its own.  q and k of qkv are read as they come, before they are unit vectors.

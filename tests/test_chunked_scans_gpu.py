@@ -107,6 +107,39 @@ def test_delta_rule_by_groups_of_tokens(H, G, D, Dv, lens, low):
         assert groups <= 1.25 * walk and groups <= 2e-6, (i, groups, walk)
 
 
+def _delta_rule_64(qkv, decay, proj, b0, state, off, H, G, D, Dv, q_scale, eps):
+    """One run from the state rows' first slot on, in float64 and not rounded: outputs and the state."""
+    x, n, unit = qkv.double(), qkv.shape[0], lambda v: v / torch.sqrt((v * v).sum(-1, keepdim=True) + eps)
+    q, k = ((unit(x[:, i * G * D: (i + 1) * G * D].view(n, G, D)) * f).repeat_interleave(H // G, dim=1) for i, f in ((0, q_scale), (1, 1.0)))
+    v, g, beta = x[:, 2 * G * D:].view(n, H, Dv), decay.double().view(n, H, D), torch.sigmoid(proj.double()[:, b0: b0 + H])
+    S, y = state[0, off: off + H * D * Dv].double().view(H, Dv, D), []
+    for t in range(n):
+        S = g[t][:, None, :] * S
+        S = S + (beta[t][:, None] * (v[t] - (S * k[t][:, None, :]).sum(-1)))[:, :, None] * k[t][:, None, :]
+        y.append((S * q[t][:, None, :]).sum(-1))
+    return torch.stack(y).view(n, H * Dv), S.reshape(-1)
+
+
+@pytest.mark.parametrize("low", [0.0, 0.5, 0.8, 0.9, 0.99])
+def test_delta_rule_by_groups_rounds_no_more_than_token_by_token(low):
+    """Against float64 from strong decays to weak ones, the mean (of logarithms) over sizes and inputs of the error's ratio to that of the
+    chain of single tokens: a single ratio scatters by some percent, the mean over 24 by one (states by two)."""
+    from tempura_amd.kernels import ops
+    ratios = []
+    for H, G, D, Dv in ((2, 2, 64, 16), (3, 1, 64, 128), (4, 2, 128, 48), (2, 2, 128, 128)):
+        for seed in range(6):
+            qkv, decay, proj, state, cu, slots = (t.to(DEV) for t in _delta_inputs([97 + 31 * seed], H, G, D, Dv, 100 * seed + H * D, low))
+            y64, s64 = _delta_rule_64(qkv, decay, proj, 2, state[int(slots[0]):], 5, H, G, D, Dv, D ** -0.5, 1e-6)
+            err = []
+            for max_run in (qkv.shape[0], 0):
+                s = state.clone()
+                y = ops.delta_scan(qkv.clone(), decay, proj, 2, s, 5, cu, slots, 1, H, G, D, Dv, D ** -0.5, 1e-6, max_run=max_run)
+                err.append(((y - y64).norm(), (s[int(slots[0]), 5: 5 + s64.numel()] - s64).norm()))
+            ratios.append([float(torch.log(a / b)) for a, b in zip(*err)])
+    y, s = torch.tensor(ratios).mean(0).exp().tolist()
+    assert y <= 1.01 and s <= 1.02, (y, s)
+
+
 def test_delta_rule_in_several_pairs_of_launches():
     """More tokens, heads and requests than the scratch holds at a time: each pair of launches goes on from the state of the one before."""
     from tempura_amd.kernels import ops

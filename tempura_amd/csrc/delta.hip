@@ -7,6 +7,7 @@
 // everything is read from device memory, so the same launches serve prompt portions, single decoded tokens and
 // captured steps.  In short runs a token's result does not depend on how its run was cut: every token is one step of the
 // same chain, in the same order of operations; long runs go by groups of tokens (delta_chunks.hip), which changes rounding only.
+// What other requests bring does not matter to either.
 #include <math.h>
 
 #include "common.h"
@@ -49,13 +50,27 @@ struct DeltaArgs {
   float* kq;   // [n, kv_heads]
   int heads, kv_heads, dim, vdim;
   float q_scale, unit_eps;
+  int n_req;
+  int longest;   // runs of more tokens have been taken by groups (delta_chunks.hip); 0: none has
 };
+
+// Whether token t belongs to a run of more than `longest` tokens (the same in every lane of a wave; all of them come here).
+__device__ inline bool in_longer_run(const int* cu_seqlens, int n_req, int t, int longest, int lane) {
+  for (int r0 = 0; r0 < n_req; r0 += TP_WAVE) {
+    const int r = r0 + lane;
+    const int a = r < n_req ? cu_seqlens[r] : 0, b = r < n_req ? cu_seqlens[r + 1] : 0;
+    const bool own = a <= t && t < b;
+    if (__any(own)) return __any(own && b - a > longest);
+  }
+  return false;
+}
 
 __global__ __launch_bounds__(256) void delta_prep_kernel(DeltaArgs a, long pairs) {
   const long p = (long)blockIdx.x * 4 + threadIdx.x / TP_WAVE;
   const int lane = threadIdx.x % TP_WAVE;
   if (p >= pairs) return;
   const long t = p / a.kv_heads;
+  if (a.longest > 0 && in_longer_run(a.cu_seqlens, a.n_req, (int)t, a.longest, lane)) return;
   const int g = (int)(p % a.kv_heads);
   float* q = a.qkv + (size_t)t * a.row_stride + (size_t)g * a.dim;
   float* k = q + (size_t)a.kv_heads * a.dim;
@@ -91,7 +106,7 @@ __global__ __launch_bounds__(256) void delta_scan_kernel(DeltaArgs a) {
   __shared__ float kqs[TC];
   const int r = blockIdx.x, h = blockIdx.y;
   const int start = a.cu_seqlens[r], len = a.cu_seqlens[r + 1] - start;
-  if (len <= 0) return;
+  if (len <= 0 || (a.longest > 0 && len > a.longest)) return;
   const int tid = threadIdx.x, wave = tid / TP_WAVE, lane = tid % TP_WAVE;
   const int ks = lane % KS, jl = wave * CW + lane / KS;
   const int j = blockIdx.z * CB + jl;
@@ -246,7 +261,7 @@ __global__ __launch_bounds__(256) void delta_scan_kernel(DeltaArgs a) {
   }
 }
 
-// Defined in delta_chunks.hip: 0 when it took the runs, -1 when they are not its own.
+// Defined in delta_chunks.hip: takes the runs of more than the returned number of tokens; -1: none.
 int tp_delta_chunks(const float* qkv, int row_stride, const float* decay, const float* proj, int proj_stride, int beta_col0, float* state,
                     size_t state_stride, size_t state_off, const int* cu_seqlens, const int* state_slots, float* y, int n_req, int heads,
                     int kv_heads, int dim, int vdim, float q_scale, float unit_eps, int max_run, float* scratch, size_t scratch_floats,
@@ -264,13 +279,14 @@ extern "C" int tp_delta_scan(float* qkv, int row_stride, const float* decay, con
   TP_REQUIRE(state_stride >= state_off + (size_t)heads * dim * vdim, "delta_scan: state rows too short");
   TP_REQUIRE(heads <= 65535, "delta_scan: too many heads");
   if (n == 0 || n_req == 0) return 0;
-  if (tp_delta_chunks(qkv, row_stride, decay, proj, proj_stride, beta_col0, state, state_stride, state_off, cu_seqlens, state_slots, y, n_req,
-                      heads, kv_heads, dim, vdim, q_scale, unit_eps, max_run, scratch, scratch_floats, s) == 0) {
+  const int longest = tp_delta_chunks(qkv, row_stride, decay, proj, proj_stride, beta_col0, state, state_stride, state_off, cu_seqlens, state_slots,
+                                      y, n_req, heads, kv_heads, dim, vdim, q_scale, unit_eps, max_run, scratch, scratch_floats, s);
+  if (longest >= 0) {
     TP_CHECK_LAUNCH("delta_scan (groups)");
-    return 0;
+    if ((long)n_req * max_run == n) return 0;      // (every run is as long as the longest)
   }
   DeltaArgs a{qkv, row_stride, decay, proj, proj_stride, beta_col0, state, state_stride, state_off, cu_seqlens, state_slots, y, kq,
-              heads, kv_heads, dim, vdim, q_scale, unit_eps};
+              heads, kv_heads, dim, vdim, q_scale, unit_eps, n_req, longest < 0 ? 0 : longest};
   const long pairs = (long)n * kv_heads;
   TP_REQUIRE((pairs + 3) / 4 < 0x7fffffffL, "delta_scan: too many rows");
   hipLaunchKernelGGL(delta_prep_kernel, dim3((unsigned)((pairs + 3) / 4)), dim3(256), 0, s, a, pairs);

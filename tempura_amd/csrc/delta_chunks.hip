@@ -29,6 +29,9 @@
 typedef float f32x4_d __attribute__((ext_vector_type(4)));
 
 #define DC_T 16      // tokens of a group
+// Runs of up to this many tokens are left to the chain of single tokens, whatever runs stand beside them: a request's bits do not depend
+// on its neighbours.  (16 heads of 128 x 128, one run, single tokens / groups: 64 tokens 25 / 28 us, 96 33 / 32, 128 41 / 31.)
+#define DC_SHORT 96
 
 struct DeltaChunkArgs {
   const float* qkv;
@@ -119,8 +122,8 @@ __global__ __launch_bounds__(64) void delta_chunk_prep_kernel(DeltaChunkArgs a) 
   __shared__ float bs[DC_T];
   const int lane = threadIdx.x;
   const int h = blockIdx.x % a.heads, rest = blockIdx.x / a.heads, c = rest % a.groups, r = rest / a.groups;
-  const int run0 = a.cu_seqlens[r], t0 = a.first + c * DC_T, len = min(DC_T, a.cu_seqlens[r + 1] - run0 - t0);
-  if (len <= 0) return;
+  const int run0 = a.cu_seqlens[r], run = a.cu_seqlens[r + 1] - run0, t0 = a.first + c * DC_T, len = min(DC_T, run - t0);
+  if (run <= DC_SHORT || len <= 0) return;
   const size_t row0 = (size_t)(run0 + t0);
   const int g = h / (a.heads / a.kv_heads);
   const float* qp = a.qkv + row0 * a.row_stride + (size_t)g * K;
@@ -245,9 +248,9 @@ __global__ __launch_bounds__(256) void delta_chunk_scan_kernel(DeltaChunkArgs a)
   const int rest = blockIdx.x >> 3, pair = rest / strips * 8 + (blockIdx.x & 7), strip = rest % strips;
   if (pair >= pairs) return;
   const int h = pair % a.heads, r = pair / a.heads;
-  const int run0 = a.cu_seqlens[r], left = a.cu_seqlens[r + 1] - run0 - a.first;
+  const int run0 = a.cu_seqlens[r], run = a.cu_seqlens[r + 1] - run0, left = run - a.first;
   const int groups = min(a.groups, (left + DC_T - 1) / DC_T);
-  if (groups <= 0) return;
+  if (run <= DC_SHORT || groups <= 0) return;
   const int j0 = strip * 16 * CT + col, i0 = wave * TILES * 16;      // (this lane's columns: j0 + 16 n)
   const size_t size = dc_item_floats(K);
   const float* vcol = a.qkv + (size_t)(run0 + a.first) * a.row_stride + 2 * (size_t)a.kv_heads * K + (size_t)h * a.vdim + j0;
@@ -359,21 +362,21 @@ __global__ __launch_bounds__(256) void delta_chunk_scan_kernel(DeltaChunkArgs a)
 // Groups of a run that one pair of launches takes, 0: the runs are not these kernels'.  The scratch is held to a quarter of a GB: longer
 // runs of many heads and requests take several pairs, each from the state that the one before left.
 static int dc_groups(int n_req, int max_run, int heads, int dim, int vdim) {
-  // (16 heads of 128 x 128, one run, single tokens / groups: 64 tokens 25 / 28 us, 96 33 / 32, 128 41 / 31)
-  if (max_run <= 96 || (dim != 64 && dim != 128) || vdim % 16 != 0) return 0;
+  if (max_run <= DC_SHORT || (dim != 64 && dim != 128) || vdim % 16 != 0) return 0;
   const size_t group = (size_t)n_req * heads * dc_item_floats(dim), limit = (size_t)64 << 20;
   const long all = (max_run + DC_T - 1) / DC_T, fit = (long)(limit / group);
   if (fit < 1 || (long)n_req * heads * (fit < all ? fit : all) >= 0x7fffffffL || ((long)n_req * heads + 8) * (vdim / 16) >= 0x7fffffffL) return 0;
   return (int)(fit < all ? fit : all);
 }
 
-// Floats of scratch for runs of up to max_run tokens (0: they go token by token).
+// Floats of scratch for runs of up to max_run tokens (0: all go token by token).
 extern "C" size_t tp_delta_scan_scratch(int n_req, int max_run, int heads, int dim, int vdim) {
   if (n_req <= 0 || heads <= 0 || dim <= 0 || vdim <= 0) return 0;
   return (size_t)dc_groups(n_req, max_run, heads, dim, vdim) * n_req * heads * dc_item_floats(dim);
 }
 
-// Returns 0 when it took the runs, -1 when they are not its own.  q and k of qkv are read as they come, before they are unit vectors.
+// Takes the runs of more than the returned number of tokens (-1: none of them are its own).  q and k of qkv are read as they come, before
+// they are unit vectors, and left alone.
 int tp_delta_chunks(const float* qkv, int row_stride, const float* decay, const float* proj, int proj_stride, int beta_col0, float* state,
                     size_t state_stride, size_t state_off, const int* cu_seqlens, const int* state_slots, float* y, int n_req, int heads,
                     int kv_heads, int dim, int vdim, float q_scale, float unit_eps, int max_run, float* scratch, size_t scratch_floats,
@@ -403,5 +406,5 @@ int tp_delta_chunks(const float* qkv, int row_stride, const float* decay, const 
     }
   }
 #undef DC_SCAN
-  return 0;
+  return DC_SHORT;
 }

@@ -140,6 +140,31 @@ def test_delta_rule_by_groups_rounds_no_more_than_token_by_token(low):
     assert y <= 1.01 and s <= 1.02, (y, s)
 
 
+@pytest.mark.parametrize("H,G,D,Dv", [(4, 2, 64, 16), (2, 2, 128, 128)])
+def test_delta_rule_of_a_run_does_not_depend_on_its_neighbours(H, G, D, Dv):
+    """Decoded tokens and short portions beside long ones: the bits, outputs and states, that every run has alone."""
+    from tempura_amd.kernels import ops
+    lens = [300, 1, 96, 0, 20, 97] + [1] * 70 + [50, 257]
+    qkv, decay, proj, state, cu, slots = (t.to(DEV) for t in _delta_inputs(lens, H, G, D, Dv, 31, 0.8))
+    together = state.clone()
+    y = ops.delta_scan(qkv.clone(), decay, proj, 2, together, 5, cu, slots, len(lens), H, G, D, Dv, D ** -0.5, 1e-6, max_run=max(lens))
+    for i, n in enumerate(lens):
+        rows, alone = slice(int(cu[i]), int(cu[i + 1])), state.clone()
+        if n:
+            one = torch.tensor([0, n], dtype=torch.int32, device=DEV)
+            got = ops.delta_scan(qkv[rows].clone(), decay[rows].contiguous(), proj[rows].contiguous(), 2, alone, 5, one, slots[i: i + 1], 1, H, G, D, Dv,
+                                 D ** -0.5, 1e-6, max_run=n)
+            assert torch.equal(y[rows], got), n
+        assert torch.equal(together[int(slots[i])], alone[int(slots[i])]), n
+        if n in (20, 96):      # (and those that its tokens have one a step)
+            alone, one = state.clone(), torch.tensor([0, 1], dtype=torch.int32, device=DEV)
+            for t in range(int(cu[i]), int(cu[i + 1])):
+                got = ops.delta_scan(qkv[t: t + 1].clone(), decay[t: t + 1].contiguous(), proj[t: t + 1].contiguous(), 2, alone, 5, one, slots[i: i + 1],
+                                     1, H, G, D, Dv, D ** -0.5, 1e-6, max_run=1)
+                assert torch.equal(y[t: t + 1], got), (n, t)
+            assert torch.equal(together[int(slots[i])], alone[int(slots[i])]), n
+
+
 def test_delta_rule_in_several_pairs_of_launches():
     """More tokens, heads and requests than the scratch holds at a time: each pair of launches goes on from the state of the one before."""
     from tempura_amd.kernels import ops

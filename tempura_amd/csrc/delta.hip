@@ -263,7 +263,7 @@ __global__ __launch_bounds__(256) void delta_scan_kernel(DeltaArgs a) {
 
 // Defined in delta_chunks.hip: takes the runs of more than the returned number of tokens; -1: none.
 int tp_delta_chunks(const float* qkv, int row_stride, const float* decay, const float* proj, int proj_stride, int beta_col0, float* state,
-                    size_t state_stride, size_t state_off, const int* cu_seqlens, const int* state_slots, float* y, int n_req, int heads,
+                    size_t state_stride, size_t state_off, const int* cu_seqlens, const int* state_slots, float* y, int n, int n_req, int heads,
                     int kv_heads, int dim, int vdim, float q_scale, float unit_eps, int max_run, float* scratch, size_t scratch_floats,
                     hipStream_t s);
 
@@ -280,7 +280,7 @@ extern "C" int tp_delta_scan(float* qkv, int row_stride, const float* decay, con
   TP_REQUIRE(heads <= 65535, "delta_scan: too many heads");
   if (n == 0 || n_req == 0) return 0;
   const int longest = tp_delta_chunks(qkv, row_stride, decay, proj, proj_stride, beta_col0, state, state_stride, state_off, cu_seqlens, state_slots,
-                                      y, n_req, heads, kv_heads, dim, vdim, q_scale, unit_eps, max_run, scratch, scratch_floats, s);
+                                      y, n, n_req, heads, kv_heads, dim, vdim, q_scale, unit_eps, max_run, scratch, scratch_floats, s);
   if (longest >= 0) {
     TP_CHECK_LAUNCH("delta_scan (groups)");
     if ((long)n_req * max_run == n) return 0;      // (every run is as long as the longest)

@@ -16,11 +16,13 @@
 // are added last, where a sum's roundings are few.  Root mean square error against float64 over that of the chain, runs of 112, 300 and
 // 1,000 tokens: decays of 0 to 1 a token 0.91 (states 0.99), 0.5 to 1 0.93 (0.97), 0.8 to 1 0.96 (0.95), 0.9 to 1 0.94 (0.92), 0.99 to 1
 // 0.82 (0.81).  (In float32 throughout, tokens in the order of the rows and U = T V - (T K~) S it was 1.03, 1.06, 1.08, 1.06 and 0.94;
-// one run of 2,048 tokens then took 204 us, now 223, four of 450 tokens 94 and 95.)
+// one run of 2,048 tokens then took 204 us, now 228, four of 450 tokens 94 and 97.)
 //
-// The chain of single tokens is bound by what a wave issues and waits for a token, 0.25 to 0.55 us; here a group of 16 takes 1.3 us (its
+// The chain of single tokens is bound by what a wave issues and waits for a token, 0.25 to 0.55 us; here a group of 16 takes 1.5 us (its
 // products, a meeting in LDS and the update, each waiting for the one before).  16 heads of 128 x 128, single tokens / groups: one run of
-// 128 tokens 41 / 31 us, 256 75 / 42, 2,048 500 / 223; four runs of 450 tokens 160 / 95 (a third of it the first kernel).
+// 128 tokens 41 / 31 us, 256 75 / 42, 2,048 495 / 228; four runs of 450 tokens 162 / 97 (a third of it the first kernel); a long run and
+// single tokens beside it, with the chain that takes these: 700 and 31 1,329 / 115, 1,800 and 63 3,411 / 243, 1,800 and 247 1,304 / 378;
+// the other way about, 200 and ten of 90, 123 / 135 (the two kinds run one behind the other).
 #include <math.h>
 
 #include "common.h"
@@ -44,8 +46,7 @@ struct DeltaChunkArgs {
   float* scratch;
   size_t state_stride, state_off;
   int row_stride, proj_stride, beta_col0, heads, kv_heads, vdim, requests;
-  int first;       // first token of a run that this launch takes
-  int groups;      // groups of a run that this launch takes, at most
+  int first, groups;      // the groups that this launch takes, among those of all long runs one behind the other
   float q_scale, unit_eps;
 };
 
@@ -61,6 +62,46 @@ __host__ __device__ inline size_t dc_item_floats(int dim) { return (size_t)49 * 
 // places of the sums: for s B(s, s), then A(t, s), B(t, s) of t = s + 1 .. 15
 #define DC_B(t, s) (32 * (s) - (s) * (s) + 2 * ((t) - (s)))
 #define DC_A(t, s) (DC_B(t, s) - 1)
+
+// The groups of all long runs are numbered one behind the other, so that scratch and launches are sized by the step's tokens and not by
+// its requests times their longest run; where a run's groups begin is read from the runs' bounds here, 64 of them at a time.
+__device__ inline int dc_run_groups(const int* cu_seqlens, int r, int requests) {
+  const int len = r < requests ? cu_seqlens[r + 1] - cu_seqlens[r] : 0;
+  return len > DC_SHORT ? (len + DC_T - 1) / DC_T : 0;
+}
+
+__device__ inline int dc_first_group(const int* cu_seqlens, int r, int lane) {
+  int sum = 0;
+  for (int r0 = 0; r0 < r; r0 += TP_WAVE) {
+    int v = dc_run_groups(cu_seqlens, r0 + lane, r);
+#pragma unroll
+    for (int d = TP_WAVE / 2; d > 0; d /= 2) v += __shfl_xor(v, d, TP_WAVE);
+    sum += v;
+  }
+  return __builtin_amdgcn_readfirstlane(sum);
+}
+
+// The run that group i belongs to, and its number there; false: there are fewer groups.
+__device__ inline bool dc_find_group(const int* cu_seqlens, int requests, int i, int lane, int& run, int& number) {
+  for (int r0 = 0; r0 < requests; r0 += TP_WAVE) {
+    const int own = dc_run_groups(cu_seqlens, r0 + lane, requests);
+    int upto = own;
+#pragma unroll
+    for (int d = 1; d < TP_WAVE; d *= 2) {
+      const int below = __shfl_up(upto, d, TP_WAVE);
+      if (lane >= d) upto += below;
+    }
+    const unsigned long long behind = __ballot(upto > i);
+    if (behind != 0) {
+      const int at = __ffsll(behind) - 1;
+      run = __builtin_amdgcn_readfirstlane(r0 + at);
+      number = __builtin_amdgcn_readfirstlane(i - __shfl(upto - own, at, TP_WAVE));
+      return true;
+    }
+    i -= __shfl(upto, TP_WAVE - 1, TP_WAVE);
+  }
+  return false;
+}
 
 // The sums over the lanes of a wave of 64 values, lane i the i-th's: lanes_transpose_sum's tree (distance 32 down to 1), in float64 behind
 // its first level.  The two widest levels are the instructions that swap halves or odd rows with even ones.
@@ -121,9 +162,10 @@ __global__ __launch_bounds__(64) void delta_chunk_prep_kernel(DeltaChunkArgs a) 
   __shared__ float dots[256];
   __shared__ float bs[DC_T];
   const int lane = threadIdx.x;
-  const int h = blockIdx.x % a.heads, rest = blockIdx.x / a.heads, c = rest % a.groups, r = rest / a.groups;
-  const int run0 = a.cu_seqlens[r], run = a.cu_seqlens[r + 1] - run0, t0 = a.first + c * DC_T, len = min(DC_T, run - t0);
-  if (run <= DC_SHORT || len <= 0) return;
+  const int h = blockIdx.x % a.heads, at = blockIdx.x / a.heads;
+  int r, c;
+  if (!dc_find_group(a.cu_seqlens, a.requests, a.first + at, lane, r, c)) return;
+  const int run0 = a.cu_seqlens[r], t0 = c * DC_T, len = min(DC_T, a.cu_seqlens[r + 1] - run0 - t0);
   const size_t row0 = (size_t)(run0 + t0);
   const int g = h / (a.heads / a.kv_heads);
   const float* qp = a.qkv + row0 * a.row_stride + (size_t)g * K;
@@ -172,7 +214,7 @@ __global__ __launch_bounds__(64) void delta_chunk_prep_kernel(DeltaChunkArgs a) 
     float v[64];
     dc_dots<0, PER>(q, k, gd, v, dots, lane);
   }
-  float* item = a.scratch + (((size_t)r * a.groups + c) * a.heads + h) * dc_item_floats(K);
+  float* item = a.scratch + ((size_t)at * a.heads + h) * dc_item_floats(K);
   float *Kt = item, *Q = Kt + DC_T * K, *KT = Q + DC_T * K, *G = KT + DC_T * K, *T = G + K, *B = T + 256, *diag = B + 256;
 #pragma unroll
   for (int p = 0; p < PER; ++p) {
@@ -248,13 +290,17 @@ __global__ __launch_bounds__(256) void delta_chunk_scan_kernel(DeltaChunkArgs a)
   const int rest = blockIdx.x >> 3, pair = rest / strips * 8 + (blockIdx.x & 7), strip = rest % strips;
   if (pair >= pairs) return;
   const int h = pair % a.heads, r = pair / a.heads;
-  const int run0 = a.cu_seqlens[r], run = a.cu_seqlens[r + 1] - run0, left = run - a.first;
-  const int groups = min(a.groups, (left + DC_T - 1) / DC_T);
-  if (run <= DC_SHORT || groups <= 0) return;
+  const int run = a.cu_seqlens[r + 1] - a.cu_seqlens[r];
+  if (run <= DC_SHORT) return;
+  // this run's groups that the launch holds: from its c0-th on, where `begin` is the launch's first for this run
+  const int begin = dc_first_group(a.cu_seqlens, r, lane) - a.first, c0 = max(0, -begin);
+  const int groups = min(a.groups - begin, (run + DC_T - 1) / DC_T) - c0;
+  if (groups <= 0) return;
+  const int run0 = a.cu_seqlens[r] + c0 * DC_T, left = run - c0 * DC_T;      // (the run from there on)
   const int j0 = strip * 16 * CT + col, i0 = wave * TILES * 16;      // (this lane's columns: j0 + 16 n)
   const size_t size = dc_item_floats(K);
-  const float* vcol = a.qkv + (size_t)(run0 + a.first) * a.row_stride + 2 * (size_t)a.kv_heads * K + (size_t)h * a.vdim + j0;
-  const float* item = a.scratch + ((size_t)r * a.groups * a.heads + h) * size;
+  const float* vcol = a.qkv + (size_t)run0 * a.row_stride + 2 * (size_t)a.kv_heads * K + (size_t)h * a.vdim + j0;
+  const float* item = a.scratch + ((size_t)(begin + c0) * a.heads + h) * size;
   float* Sm = a.state + (size_t)a.state_slots[r] * a.state_stride + a.state_off + ((size_t)h * a.vdim + j0) * K;
   f32x4_d S[CT][TILES];
 #pragma unroll
@@ -336,7 +382,7 @@ __global__ __launch_bounds__(256) void delta_chunk_scan_kernel(DeltaChunkArgs a)
         for (int i = 0; i < 4; ++i) {
           const int t = c * DC_T + 4 * i + quad;
           // (a token's own part, most of the sum where decays are strong, is added last: one rounding at its size)
-          if (t < left) a.y[((size_t)(run0 + a.first + t) * a.heads + h) * a.vdim + j0 + 16 * n] = fmaf(u[i], x.d[i], o[i]);
+          if (t < left) a.y[((size_t)(run0 + t) * a.heads + h) * a.vdim + j0 + 16 * n] = fmaf(u[i], x.d[i], o[i]);
         }
       }
     }
@@ -359,44 +405,51 @@ __global__ __launch_bounds__(256) void delta_chunk_scan_kernel(DeltaChunkArgs a)
       for (int i = 0; i < 4; ++i) Sm[(size_t)16 * n * K + i0 + 16 * m + 4 * quad + i] = S[n][m][i];
 }
 
-// Groups of a run that one pair of launches takes, 0: the runs are not these kernels'.  The scratch is held to a quarter of a GB: longer
-// runs of many heads and requests take several pairs, each from the state that the one before left.
-static int dc_groups(int n_req, int max_run, int heads, int dim, int vdim) {
+// Groups that one pair of launches takes, 0: the runs are not these kernels'; *all: groups of the step, at most (a long run has more than
+// DC_SHORT tokens, and one group that is not full).  The scratch is held to a quarter of a GB: longer steps take several pairs, each from
+// the states that the one before left.  A pair then writes and reads that much, beside which its launches and the states are little.
+static int dc_groups(int n, int n_req, int max_run, int heads, int dim, int vdim, int* all) {
+  *all = 0;
   if (max_run <= DC_SHORT || (dim != 64 && dim != 128) || vdim % 16 != 0) return 0;
-  const size_t group = (size_t)n_req * heads * dc_item_floats(dim), limit = (size_t)64 << 20;
-  const long all = (max_run + DC_T - 1) / DC_T, fit = (long)(limit / group);
-  if (fit < 1 || (long)n_req * heads * (fit < all ? fit : all) >= 0x7fffffffL || ((long)n_req * heads + 8) * (vdim / 16) >= 0x7fffffffL) return 0;
-  return (int)(fit < all ? fit : all);
+  const size_t fit = ((size_t)64 << 20) / ((size_t)heads * dc_item_floats(dim));
+  if (fit < 1 || ((long)n_req * heads + 8) * (vdim / 16) >= 0x7fffffffL) return 0;
+  const int runs = n / (DC_SHORT + 1);
+  *all = n / DC_T + (runs < n_req ? runs : n_req);
+  return (size_t)*all < fit ? *all : (int)fit;
 }
 
-// Floats of scratch for runs of up to max_run tokens (0: all go token by token).
-extern "C" size_t tp_delta_scan_scratch(int n_req, int max_run, int heads, int dim, int vdim) {
-  if (n_req <= 0 || heads <= 0 || dim <= 0 || vdim <= 0) return 0;
-  return (size_t)dc_groups(n_req, max_run, heads, dim, vdim) * n_req * heads * dc_item_floats(dim);
+// Floats of scratch for n tokens in n_req runs of up to max_run (0: all go token by token).
+extern "C" size_t tp_delta_scan_scratch(int n, int n_req, int max_run, int heads, int dim, int vdim) {
+  if (n <= 0 || n_req <= 0 || heads <= 0 || dim <= 0 || vdim <= 0) return 0;
+  int all;
+  return (size_t)dc_groups(n, n_req, max_run, heads, dim, vdim, &all) * heads * dc_item_floats(dim);
 }
 
 // Takes the runs of more than the returned number of tokens (-1: none of them are its own).  q and k of qkv are read as they come, before
 // they are unit vectors, and left alone.
 int tp_delta_chunks(const float* qkv, int row_stride, const float* decay, const float* proj, int proj_stride, int beta_col0, float* state,
-                    size_t state_stride, size_t state_off, const int* cu_seqlens, const int* state_slots, float* y, int n_req, int heads,
+                    size_t state_stride, size_t state_off, const int* cu_seqlens, const int* state_slots, float* y, int n, int n_req, int heads,
                     int kv_heads, int dim, int vdim, float q_scale, float unit_eps, int max_run, float* scratch, size_t scratch_floats,
                     hipStream_t s) {
-  const int groups = dc_groups(n_req, max_run, heads, dim, vdim);
-  if (groups == 0 || scratch == nullptr || ((uintptr_t)scratch & 15) || scratch_floats < tp_delta_scan_scratch(n_req, max_run, heads, dim, vdim)) return -1;
+  int all;
+  const int groups = dc_groups(n, n_req, max_run, heads, dim, vdim, &all);
+  if (groups == 0 || scratch == nullptr || ((uintptr_t)scratch & 15) || scratch_floats < (size_t)groups * heads * dc_item_floats(dim)) return -1;
   DeltaChunkArgs a{qkv, decay, proj, state, cu_seqlens, state_slots, y, scratch, state_stride, state_off, row_stride, proj_stride, beta_col0,
                    heads, kv_heads, vdim, n_req, 0, groups, q_scale, unit_eps};
   const long pairs = ((long)n_req * heads + 7) / 8 * 8;
-  // (32 columns a block read W, Q~ and K^ half as often, which bounds the chain once there are more blocks of 16 columns than the two
+  // (32 columns a block read K~, Q~ and K^ half as often, which bounds the chain once there are more blocks of 16 columns than the two
   // a CU that run at a time: 16 heads of 128 x 128, four runs of 451 tokens, 512 blocks of 16 columns or half as many of 32: 94 / 102 us;
-  // 32 heads, eight runs of 256, 2,048 blocks: 202 / 174)
-  const bool wide = vdim % 32 == 0 && pairs * (vdim / 16) > 512;
-  const dim3 prep((unsigned)((long)n_req * groups * heads)), scan((unsigned)(pairs * (vdim / (wide ? 32 : 16))));
+  // 32 heads, eight runs of 256, 2,048 blocks: 202 / 174.  Blocks of short runs end at once and do not count.)
+  const long others = max_run < n ? (n - max_run) / (DC_SHORT + 1) : 0, long_runs = 1 + (others < n_req - 1 ? others : n_req - 1);
+  const bool wide = vdim % 32 == 0 && long_runs * heads * (vdim / 16) > 512;
+  const dim3 scan((unsigned)(pairs * (vdim / (wide ? 32 : 16))));
 #define DC_SCAN(KT_)                                                                                                 \
   do {                                                                                                               \
     if (wide) hipLaunchKernelGGL((delta_chunk_scan_kernel<KT_, 2>), scan, dim3(256), 0, s, a);                       \
     else hipLaunchKernelGGL((delta_chunk_scan_kernel<KT_, 1>), scan, dim3(256), 0, s, a);                            \
   } while (0)
-  for (; a.first < max_run; a.first += groups * DC_T) {
+  for (; a.first < all; a.first += groups) {
+    const dim3 prep((unsigned)((long)(groups < all - a.first ? groups : all - a.first) * heads));
     if (dim == 128) {
       hipLaunchKernelGGL(delta_chunk_prep_kernel<2>, prep, dim3(64), 0, s, a);
       DC_SCAN(8);

@@ -49,6 +49,7 @@ class _Library:
                 raise KernelError(f"cannot load the kernel library {path}: {e}") from e
             lib.tp_last_error.restype = ctypes.c_char_p
             lib.tp_linear_f32_scratch.restype = ctypes.c_size_t
+            lib.tp_delta_scan_scratch.restype = ctypes.c_size_t
             cls._lib = lib
             cls.path = path
         return cls._lib
@@ -1736,9 +1737,7 @@ def delta_scan(qkv: torch.Tensor, decay: torch.Tensor, proj: torch.Tensor, beta_
     y = torch.empty((n, heads * vdim), dtype=torch.float32, device=qkv.device)
     kq = torch.empty((n, kv_heads), dtype=torch.float32, device=qkv.device)      # k . q per token and key head
     max_run = min(int(max_run), n)
-    lib = _Library.get()
-    lib.tp_delta_scan_scratch.restype = ctypes.c_size_t
-    need = lib.tp_delta_scan_scratch(int(num_requests), max_run, int(heads), int(dim), int(vdim)) if allow_mfma else 0
+    need = library().tp_delta_scan_scratch(n, int(num_requests), max_run, int(heads), int(dim), int(vdim)) if allow_mfma else 0
     scratch = torch.empty((need,), dtype=torch.float32, device=qkv.device) if need else None
     _call("tp_delta_scan", _ptr(qkv), qkv.shape[1], _ptr(decay), _ptr(proj), proj.shape[1], int(beta_col0), _ptr(state),
           ctypes.c_size_t(state.shape[1]), ctypes.c_size_t(state_off), _ptr(cu_seqlens), _ptr(state_slots), _ptr(y), _ptr(kq), n,

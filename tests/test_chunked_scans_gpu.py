@@ -165,15 +165,21 @@ def test_delta_rule_of_a_run_does_not_depend_on_its_neighbours(H, G, D, Dv):
             assert torch.equal(together[int(slots[i])], alone[int(slots[i])]), n
 
 
-def test_delta_rule_in_several_pairs_of_launches():
-    """More tokens, heads and requests than the scratch holds at a time: each pair of launches goes on from the state of the one before."""
+def _held_groups(lens, H, D, Dv):
+    """Groups of 16 tokens that the scratch holds for these runs."""
     from tempura_amd.kernels import ops
-    H, D, Dv, lens = 32, 128, 128, [1200, 700, 3] + [1] * 21
-    lib = ops.library()
-    lib.tp_delta_scan_scratch.restype = __import__("ctypes").c_size_t
-    item = 49 * D + 272 + 16 * Dv
-    groups = lib.tp_delta_scan_scratch(len(lens), max(lens), H, D, Dv) // (item * H * len(lens))
-    assert 1 <= groups < -(-max(lens) // 16) and groups * item * H * len(lens) <= 64 << 20
+    floats = ops.library().tp_delta_scan_scratch(sum(lens), len(lens), max(lens), H, D, Dv)
+    assert floats <= 64 << 20 and floats % (H * (49 * D + 528)) == 0
+    return floats // (H * (49 * D + 528))
+
+
+@pytest.mark.parametrize("lens", [[1200, 700, 3] + [1] * 21, [1] * 70 + [97, 450, 96] + [1, 0] * 70 + [520, 100]])
+def test_delta_rule_in_several_pairs_of_launches(lens):
+    """More tokens and heads than the scratch holds at a time: each pair of launches goes on from the states that the one before left, also
+    in the middle of a run; runs whose groups begin behind those of more than 64 others."""
+    from tempura_amd.kernels import ops
+    H, D, Dv = 160, 128, 16
+    assert 1 <= _held_groups(lens, H, D, Dv) < sum(-(-n // 16) for n in lens if n > 96)
     qkv, decay, proj, state, cu, slots = _delta_inputs(lens, H, H, D, Dv, 5, 0.9)
     dev = [t.to(DEV) for t in (decay, proj, cu, slots)]
     out = []
@@ -181,6 +187,13 @@ def test_delta_rule_in_several_pairs_of_launches():
         s = state.to(DEV)
         out.append((ops.delta_scan(qkv.to(DEV), dev[0], dev[1], 2, s, 5, dev[2], dev[3], len(lens), H, H, D, Dv, D ** -0.5, 1e-6, max_run=max_run), s))
     assert _error(out[0][0], out[1][0].cpu()) <= 1e-6 and _error(out[0][1], out[1][1].cpu()) <= 1e-6
+
+
+@pytest.mark.parametrize("lens", [[1800] + [1] * 63, [1800] + [1] * 299, [97] * 11, [2000]])
+def test_delta_rule_scratch_is_sized_by_tokens(lens):
+    """A long run beside many single tokens needs the room of its own groups, and one more a run that could be long."""
+    need = sum(-(-n // 16) for n in lens if n > 96)
+    assert need <= _held_groups(lens, 16, 128, 128) <= sum(lens) // 16 + sum(lens) // 97
 
 
 @pytest.mark.parametrize("bad", [float("inf"), float("nan")])

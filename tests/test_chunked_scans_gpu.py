@@ -56,6 +56,42 @@ def test_selective_scan_in_chunks(H, P, N, G, lens):
         assert chunks <= 1.25 * walk and chunks <= 1e-6, (i, chunks, walk)
 
 
+def _selective_scan_64(xbc, proj, c0, dt_bias, a_log, d_skip, state, off, H, P, N, G):
+    """One run from the state rows' first slot on, in float64 and not rounded: outputs and the state."""
+    n, X = xbc.shape[0], xbc.double()
+    x = X[:, : H * P].view(n, H, P)
+    B, C = (X[:, H * P + i * G * N: H * P + (i + 1) * G * N].view(n, G, N).repeat_interleave(H // G, dim=1) for i in (0, 1))
+    dt = torch.nn.functional.softplus(proj.double()[:, c0: c0 + H] + dt_bias.double())
+    decay, S, y = torch.exp(-torch.exp(a_log.double()) * dt), state[0, off: off + H * N * P].double().view(H, N, P), []
+    for t in range(n):
+        S = decay[t, :, None, None] * S + dt[t, :, None, None] * B[t, :, :, None] * x[t, :, None, :]
+        y.append((S * C[t, :, :, None]).sum(1) + d_skip.double()[:, None] * x[t])
+    return torch.stack(y).view(n, H * P), S.reshape(-1)
+
+
+@pytest.mark.parametrize("H,P,N,G", [(4, 16, 16, 2), (2, 48, 32, 1), (3, 64, 64, 3), (8, 64, 128, 4)])
+def test_selective_scan_in_chunks_rounds_no_more_than_the_walk(H, P, N, G):
+    """Against float64 with weak decays, strong ones, and strong ones of small steps: the mean (of logarithms) over inputs of the error's
+    ratio to that of the token-by-token walk.  A single ratio scatters by some percent, the mean over 16 by one (states of few heads, the
+    sum of a few tokens where decays are strong, by three)."""
+    from tempura_amd.kernels import ops
+    for bias, rate in ((0.0, 0.0), (2.5, 2.0), (0.0, 4.0)):
+        ratios = []
+        for seed in range(16):
+            xbc, proj, consts, state, cu, slots = _scan_inputs([270 + 17 * seed], H, P, N, G, 1000 * seed + H * N)
+            xbc, proj, state, cu, slots = (t.to(DEV) for t in (xbc, proj, state, cu, slots))
+            consts = [c.to(DEV) for c in (consts[0] + bias, consts[1] + rate, consts[2])]
+            y64, s64 = _selective_scan_64(xbc, proj, 2, *consts, state[int(slots[0]):], 7, H, P, N, G)
+            err = []
+            for x in (xbc, _off(xbc)):
+                s = state.clone()
+                y = ops.ssm_scan(x, proj, 2, *consts, s, 7, cu, slots, 1, H, P, N, G, max_run=xbc.shape[0])
+                err.append(((y - y64).norm(), (s[int(slots[0]), 7: 7 + s64.numel()] - s64).norm()))
+            ratios.append([float(torch.log(a / b)) for a, b in zip(*err)])
+        y, s = torch.tensor(ratios).mean(0).exp().tolist()
+        assert y <= 1.01 and s <= 1.03, (bias, rate, y, s)
+
+
 @pytest.mark.parametrize("bad", [float("inf"), float("nan")])
 @pytest.mark.parametrize("where", ["x", "b", "c", "dt"])
 def test_selective_scan_keeps_what_is_not_finite_where_it_belongs(bad, where):

@@ -87,6 +87,7 @@ struct GateAct {
   int act_cols, act_ld, side_ld;
   float* side;
   int act_kind1;             // (products of at most 16 rows: one more than another activation's kind, activations.h; 0: max(v, 0)^2)
+  float slope;               // (1 + extra_slope as the caller gave it)
 };
 
 struct RopeOut {
@@ -113,7 +114,8 @@ __device__ inline float relu_squared(float v) {
 }
 
 // g * sigmoid(slope g) * (u + offset) with the hardware's exp2 and reciprocal (one ulp each; the result is rounded to
-// bfloat16), the same arithmetic in every bfloat16 product, whatever the number of rows
+// bfloat16), the same arithmetic in every bfloat16 product of more than 16 rows; up to 16 the gate without constants has it too
+// (silu_mul), one with constants gated_value's
 __device__ inline float gate_mul(float g, float u, const GateAct& a) {
   if (a.limit > 0.f) {
     g = fminf(g, a.limit);

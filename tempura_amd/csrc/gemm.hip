@@ -225,7 +225,8 @@ extern "C" int tp_linear_fused(const void* x, const void* w, int in_dt, void* ou
   if (accumulate == 2) {  // gated-SiLU epilogue: only the matrix-core kernels have it
     TP_REQUIRE(in_dt == TP_BF16 && allow_mfma, "linear: the gated epilogue needs bfloat16 operands");
     // (the epilogue's activation: slope of the sigmoid, limit of both branches (<= 0: none), what is added to the up branch)
-    const GateAct gate = {gate_slope - 1.0f, gate_limit > 0.f ? gate_limit : 0.f, gate_offset};
+    GateAct gate = {gate_slope - 1.0f, gate_limit > 0.f ? gate_limit : 0.f, gate_offset};
+    gate.slope = gate_slope;
     const int r = tp_linear_mfma(x, w, out, out_dt, 2, M, N, K, scratch, scratch_floats, pre_ss, pre_count, pre_eps,
                                  nullptr, nullptr, nullptr, layout, 0, nullptr, gate, s);
     TP_REQUIRE(r >= 0, "linear: sizes M=%d N=%d K=%d do not fit the gated epilogue", M, N, K);

@@ -36,6 +36,9 @@ __device__ inline float silu_mul(float g, float u) {
   return g * u * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(g * -1.4426950408889634f));
 }
 
+// the same with constants, as the activation's own kernel has it: the same bits as the product and that kernel
+__device__ inline float gated_few(float g, float u, const GateAct& a) { return gated_value(g, u, a.slope, a.limit, a.offset); }
+
 // A decode product reads every weight once per step and never again before the whole model has streamed through
 // the caches: the loads say so (nontemporal), which leaves the cache lines to the activations and measures faster
 // on a chain of streaming kernels (5.7 -> 6.4 TB/s on products of these sizes).
@@ -269,7 +272,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_mfma_kernel(const bf16
 #pragma unroll
         for (int i = 0; i < WAVES; ++i) u += red[i][jt][q + 128];
         if (MT == 1) u *= rstd[l & 15];
-        store_gated(out, layout, M, N / 2, m, (n0 + j * 16) / 2 + (l >> 4) * 4 + r, SPLIT ? gate_mul(v, u, rp.gate) : silu_mul(v, u));
+        store_gated(out, layout, M, N / 2, m, (n0 + j * 16) / 2 + (l >> 4) * 4 + r, SPLIT ? gated_few(v, u, rp.gate) : silu_mul(v, u));
       }
     } else if (MT == 1 && post.w != nullptr) {
       // residual add, and the next norm's preparation (mode is OUT_ACC_F32)
@@ -428,7 +431,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_lds_kernel(const bf16_
 #pragma unroll
         for (int i = 0; i < WAVES; ++i) u += red[ge * WAVES + i][j][q + 128];
         u *= rstd[m];
-        store_gated(out, layout, M, N / 2, m, nt0 / 2 + (l >> 4) * 4 + r, SPLIT ? gate_mul(v, u, rp.gate) : silu_mul(v, u));
+        store_gated(out, layout, M, N / 2, m, nt0 / 2 + (l >> 4) * 4 + r, SPLIT ? gated_few(v, u, rp.gate) : silu_mul(v, u));
       }
     } else if (post.w != nullptr) {
       float sq = 0.f;

@@ -3,6 +3,7 @@
 // Everything is float32 arithmetic; only stored activations may be bfloat16.
 #include <math.h>
 
+#include "activations.h"
 #include "common.h"
 
 // ---- embedding + sinusoidal position, written to every stream ---------------------------------
@@ -286,13 +287,7 @@ __global__ void gated_act_kernel(const TI* __restrict__ gu, TO* __restrict__ out
   const int i = (int)(idx % inter);
   const int gc = interleaved ? (i / 8) * 16 + i % 8 : i;
   const int uc = interleaved ? gc + 8 : inter + i;
-  float g = to_float(gu[m * 2 * inter + gc]);
-  float u = to_float(gu[m * 2 * inter + uc]);
-  if (limit > 0.f) {
-    g = fminf(g, limit);
-    u = fminf(fmaxf(u, -limit), limit);
-  }
-  from_float(out + idx, g / (1.0f + expf(-slope * g)) * (u + up_offset));
+  from_float(out + idx, gated_value(to_float(gu[m * 2 * inter + gc]), to_float(gu[m * 2 * inter + uc]), slope, limit, up_offset));
 }
 
 extern "C" int tp_gated_act(const void* gu, int in_dt, void* out, int out_dt, int m, int inter, float slope, float limit,

@@ -211,6 +211,28 @@ def test_gated_products_of_a_few_rows_take_the_gates_constants(m, n, k, slope, l
     assert torch.equal(blocked, got)
 
 
+@pytest.mark.parametrize("m,n,k", [(1, 16, 64), (3, 528, 8192), (16, 272, 2048), (16, 65536, 64)])
+@pytest.mark.parametrize("slope,limit,offset", [(1.702, 7.0, 1.0), (0.3, 0.0, 0.0), (3.0, 0.5, 0.5)])
+def test_gates_with_constants_have_the_bits_of_the_activations_kernel(m, n, k, slope, limit, offset):
+    """What a decoded row's gate is as a kernel of its own: float32 exponential and division, not the hardware's short forms (which round
+    one bfloat16 in some ten thousand the other way)."""
+    from tempura_amd.kernels import ops
+    g = torch.Generator().manual_seed(m + n)
+    x = torch.randn(m, k, generator=g).to(torch.bfloat16).to(DEV)
+    w = ops.tile_weight((torch.randn(n, k, generator=g) * 3 * k ** -0.5).to(torch.bfloat16).to(DEV))
+    want = ops.gated_act(ops.linear(x, w, torch.float32), torch.bfloat16, slope, limit, offset, interleaved=True)
+    assert torch.equal(ops.linear_swiglu(x, w, slope=slope, limit=limit, up_offset=offset), want)
+
+
+def test_a_closed_gate_leaves_zero_of_a_huge_value():
+    """gate -200, up 2^121: their product overflows, the gated value does not."""
+    from tempura_amd.kernels import ops
+    x, w = torch.zeros(1, 64), torch.zeros(16, 64)
+    x[0, 0], x[0, 1], w[:8, 0], w[8:, 1] = 1.0, 2.0 ** 60, -200.0, 2.0 ** 61
+    got = ops.linear_swiglu(x.to(torch.bfloat16).to(DEV), w.to(torch.bfloat16).to(DEV), slope=1.0, limit=0.0, up_offset=0.5)
+    assert torch.equal(got, torch.zeros_like(got))
+
+
 @pytest.mark.parametrize("heads,kv,d,vd", [(4, 2, 64, 64), (3, 1, 96, 96), (8, 8, 32, 32), (16, 1, 576, 512), (2, 2, 160, 96)])
 @pytest.mark.parametrize("ctx", [[700], [1, 40, 1500], [3, 260]])
 @pytest.mark.parametrize("how", ["columns", "heads", "scale", "sink", "portions"])

@@ -211,7 +211,7 @@ extern "C" int tp_linear_fused(const void* x, const void* w, int in_dt, void* ou
   const int act_kind1 = layout >> 8;      // (see accumulate == 3)
   layout &= 255;
   const bool split_norm = pre_ss != nullptr || post_w != nullptr || (layout & 3) != 0;
-  TP_REQUIRE((layout & ~15) == 0 && (!(layout & 2) || accumulate == 2 || accumulate == 3) && (!(layout & 8) || post_w != nullptr),
+  TP_REQUIRE((layout & ~15) == 0 && (act_kind1 == 0 || accumulate == 3) && (!(layout & 2) || accumulate == 2 || accumulate == 3) && (!(layout & 8) || post_w != nullptr),
              "linear: bad layout flags %d", layout);
   TP_REQUIRE(!(layout & 4) || (in_dt == TP_BF16 && allow_mfma && N % 16 == 0 && K % 64 == 0),
              "linear: tiled weights are bfloat16 with N %% 16 == 0 and K %% 64 == 0 (N=%d K=%d)", N, K);

@@ -224,6 +224,22 @@ def test_gates_with_constants_have_the_bits_of_the_activations_kernel(m, n, k, s
     assert torch.equal(ops.linear_swiglu(x, w, slope=slope, limit=limit, up_offset=offset), want)
 
 
+def test_layout_bits_of_an_activation_belong_to_its_epilogue():
+    """Refused, as every unknown bit is, by a product that has no such epilogue (nothing is launched)."""
+    import ctypes
+    from tempura_amd.kernels import ops
+    x, w, out = (torch.zeros(16, 64, dtype=torch.bfloat16, device=DEV) for _ in range(3))
+    none, zero, ptr = ctypes.c_void_p(None), ctypes.c_float(0.0), lambda t: ctypes.c_void_p(t.data_ptr())
+    def call(layout, accumulate):
+        splits = ctypes.c_int(1)
+        return ops.library().tp_linear_fused(ptr(x), ptr(w), 1, ptr(out), 1, accumulate, 16, 16, 64, 1, none, ctypes.c_size_t(0), none, 0, zero,
+                                             none, none, none, layout, 0, ctypes.byref(splits), ctypes.c_float(1.0), zero, zero, 0, none, none)
+    for layout in (256, 1024, 1 << 12):
+        for accumulate in (0, 2):
+            assert call(layout, accumulate) == 1 and b"layout" in ops.library().tp_last_error()
+    assert call(0, 0) == 0
+
+
 def test_a_closed_gate_leaves_zero_of_a_huge_value():
     """gate -200, up 2^121: their product overflows, the gated value does not."""
     from tempura_amd.kernels import ops

@@ -165,7 +165,11 @@ extern "C" int tp_causal_conv(const float* in, int in_stride, int col0, const fl
   }
   const bool four = taps >= 2 && taps <= CONV_TAPS && channels % 4 == 0 && in_stride % 4 == 0 && col0 % 4 == 0 &&
                     (((uintptr_t)in | (uintptr_t)w | (uintptr_t)b | (uintptr_t)out) & 15) == 0;
-  if (four && n >= 64) {   // (shorter steps: too few blocks of CONV_RUN tokens)
+  // (a thread's run is a chain of three dependent trips to memory, 9 us whatever the step: the grid of single tokens is faster until it
+  // reads some megabytes four times over.  Four taps, single tokens / runs: 64 tokens of 10,240 channels 6.9 / 9.3 us, 130 9.9 / 9.7, 500
+  // 26 / 17; 300 of 3,072 8.2 / 9.3, 500 10.7 / 9.7; 700 of 2,048 10.2 / 9.6; 2,000 of 512 8.8 / 9.0; two
+  // taps, 500 of 3,072 8.9 / 9.1, 700 11.3 / 10.6)
+  if (four && (long)n * channels >= (taps > 2 ? 1300000 : 1600000)) {
     const int qb = (channels / 4 + 255) / 256;
     hipLaunchKernelGGL(causal_conv_run_kernel, dim3((unsigned)((n + CONV_RUN - 1) / CONV_RUN * qb)), dim3(256), 0, s, in, in_stride, col0,
                        w, b, state, state_stride, cu_seqlens, token_req, state_slots, out, n, channels, taps, qb, state_off, act);

@@ -43,6 +43,13 @@ def test_causal_conv_paths_agree(channels, taps, lens):
         assert torch.equal(got, want) and torch.equal(s2, s0)
 
 
+@pytest.mark.parametrize("channels,taps,lens", [(20480, 4, [70]), (10244, 4, [1, 2, 3, 60, 1, 70]), (2052, 3, [8, 56, 64, 1, 700]),
+                                                (1028, 2, [1600]), (12, 4, [100003, 9])])
+def test_causal_conv_of_steps_large_enough_for_runs(channels, taps, lens):
+    """Steps of some more than a million inputs go by runs of tokens a thread: the same bits as by single tokens."""
+    test_causal_conv_paths_agree(channels, taps, lens)
+
+
 @pytest.mark.parametrize("width,subs,taps", [(8, 1, 2), (1024, 2, 4), (4100, 3, 3)])
 def test_residual_conv_of_single_tokens(width, subs, taps):
     from tempura_amd.kernels import ops

@@ -293,6 +293,14 @@ extern "C" size_t tp_linear_f32_scratch(int M, int N, int K) {
   return splits > 1 ? (size_t)splits * M * N : 0;
 }
 
+// The side of the blocks that the product takes with that scratch (0: it is one of few rows); for tests that mean a certain one.
+extern "C" int tp_linear_f32_block(int M, int N, int K) {
+  if (M <= 16 || N <= 0 || K <= 0) return 0;
+  int tile, splits;
+  f32_plan(M, N, K, true, &tile, &splits);
+  return tile;
+}
+
 // Takes a product whose rows are whole 16-byte pieces (K % 4 == 0, aligned operands); -1: not its own, the general kernel runs.
 int tp_linear_f32(const float* x, const float* w, float* out, int accumulate, int M, int N, int K, float* scratch,
                   size_t scratch_floats, hipStream_t s) {

@@ -48,6 +48,26 @@ def test_float32_products(m, n, k):
     assert off.data_ptr() % 16 != 0 and _rel(ops.linear(off, wd, torch.float32), ref) < tol
 
 
+@pytest.mark.parametrize("small,large,n,k,parts", [(385, 449, 6150, 68, 1), (257, 383, 8198, 132, 1), (513, 577, 4100, 1028, 3)])
+def test_float32_products_in_blocks_of_128_and_64(small, large, n, k, parts):
+    """Rows, columns and k that fill no block, with and without K in parts, plain and added into rows: against float64 with the bound above,
+    and the bits of a row are the same in either block."""
+    from tempura_amd.kernels import ops
+    lib = ops.library()
+    assert lib.tp_linear_f32_block(large, n, k) == 128 and lib.tp_linear_f32_block(small, n, k) == 64
+    assert [lib.tp_linear_f32_scratch(m, n, k) for m in (small, large)] == [parts * m * n if parts > 1 else 0 for m in (small, large)]
+    g = torch.Generator().manual_seed(large + n + k)
+    x, w, res = (torch.randn(*s, generator=g).to(DEV) for s in ((large, k), (n, k), (large, n)))
+    ref, tol = x.double() @ w.double().T, 2.0 ** -24 * math.sqrt(k)
+    got, added = ops.linear(x, w, torch.float32), ops.linear(x, w, torch.float32, residual=res.clone())
+    assert _rel(got, ref) < tol and _rel(added, ref + res.double()) < tol + 2.0 ** -23
+    worst = ((got.double() - ref).abs() / (x.double().abs() @ w.double().abs().T)).max()      # (no result of a wrong place among the others)
+    assert float(worst) < 2.0 ** -24 * k / 2
+    few = x[:small].contiguous()
+    assert torch.equal(ops.linear(few, w, torch.float32), got[:small])
+    assert torch.equal(ops.linear(few, w, torch.float32, residual=res[:small].clone()), added[:small])
+
+
 @pytest.mark.parametrize("m", [1, 2, 3, 4, 5, 8, 9, 16])
 @pytest.mark.parametrize("n,k", [(3, 4), (130, 260), (1026, 3072)])
 def test_float32_products_norm_and_gate_their_rows(m, n, k):

@@ -283,7 +283,7 @@ extern "C" int tp_delta_scan(float* qkv, int row_stride, const float* decay, con
                                       y, n, n_req, heads, kv_heads, dim, vdim, q_scale, unit_eps, max_run, scratch, scratch_floats, s);
   if (longest >= 0) {
     TP_CHECK_LAUNCH("delta_scan (groups)");
-    if ((long)n_req * max_run == n) return 0;      // (every run is as long as the longest)
+    if ((long)n - (long)(n_req - 1) * max_run > longest) return 0;      // (the shortest run that such tokens can leave is a long one)
   }
   DeltaArgs a{qkv, row_stride, decay, proj, proj_stride, beta_col0, state, state_stride, state_off, cu_seqlens, state_slots, y, kq,
               heads, kv_heads, dim, vdim, q_scale, unit_eps, n_req, longest < 0 ? 0 : longest};

@@ -16,11 +16,11 @@
 // are added last, where a sum's roundings are few.  Root mean square error against float64 over that of the chain, runs of 112, 300 and
 // 1,000 tokens: decays of 0 to 1 a token 0.91 (states 0.99), 0.5 to 1 0.93 (0.97), 0.8 to 1 0.96 (0.95), 0.9 to 1 0.94 (0.92), 0.99 to 1
 // 0.82 (0.81).  (In float32 throughout, tokens in the order of the rows and U = T V - (T K~) S it was 1.03, 1.06, 1.08, 1.06 and 0.94;
-// one run of 2,048 tokens then took 204 us, now 228, four of 450 tokens 94 and 97.)
+// one run of 2,048 tokens then took 201 us, now 219, four of 451 tokens 92 and 91, with 32 heads eight of 256 159 and 175.)
 //
-// The chain of single tokens is bound by what a wave issues and waits for a token, 0.25 to 0.55 us; here a group of 16 takes 1.5 us (its
+// The chain of single tokens is bound by what a wave issues and waits for a token, 0.25 to 0.55 us; here a group of 16 takes 1.4 us (its
 // products, a meeting in LDS and the update, each waiting for the one before).  16 heads of 128 x 128, single tokens / groups: one run of
-// 128 tokens 41 / 31 us, 256 75 / 42, 2,048 495 / 228; four runs of 450 tokens 162 / 97 (a third of it the first kernel); a long run and
+// 128 tokens 41 / 31 us, 256 75 / 42, 2,048 495 / 219; four runs of 451 tokens 162 / 91 (a third of it the first kernel); a long run and
 // single tokens beside it, with the chain that takes these: 700 and 31 1,329 / 115, 1,800 and 63 3,411 / 243, 1,800 and 247 1,304 / 378;
 // the other way about, 200 and ten of 90, 123 / 135 (the two kinds run one behind the other).
 #include <math.h>
@@ -357,12 +357,9 @@ __global__ __launch_bounds__(256) void delta_chunk_scan_kernel(DeltaChunkArgs a)
       const f32x4_d e = x.v[n] - ((buf[0][2 * n][lane] + buf[1][2 * n][lane]) + (buf[2][2 * n][lane] + buf[3][2 * n][lane]));
       const float* M = item + (size_t)c * a.heads * size + (size_t)49 * K;
       f32x4_d u = (f32x4_d)(0.f);
-      if (dc_finite(e)) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) u = __builtin_amdgcn_mfma_f32_16x16x4f32(x.t[i], e[i], u, 0, 0, 0);
-      } else {
-        u = dc_lower<true>(M, e, u, col, quad);
-      }
+      for (int i = 0; i < 4; ++i) u = __builtin_amdgcn_mfma_f32_16x16x4f32(x.t[i], e[i], u, 0, 0, 0);
+      if (!dc_finite(e)) u = dc_lower<true>(M, e, (f32x4_d)(0.f), col, quad);      // (looked at while the products run)
 #pragma unroll
       for (int i = 0; i < 4; ++i)
 #pragma unroll
@@ -439,7 +436,7 @@ int tp_delta_chunks(const float* qkv, int row_stride, const float* decay, const 
   const long pairs = ((long)n_req * heads + 7) / 8 * 8;
   // (32 columns a block read K~, Q~ and K^ half as often, which bounds the chain once there are more blocks of 16 columns than the two
   // a CU that run at a time: 16 heads of 128 x 128, four runs of 451 tokens, 512 blocks of 16 columns or half as many of 32: 94 / 102 us;
-  // 32 heads, eight runs of 256, 2,048 blocks: 202 / 174.  Blocks of short runs end at once and do not count.)
+  // 32 heads, eight runs of 256, 2,048 blocks: 202 / 174 when the rule was made.  Blocks of short runs end at once and do not count.)
   const long others = max_run < n ? (n - max_run) / (DC_SHORT + 1) : 0, long_runs = 1 + (others < n_req - 1 ? others : n_req - 1);
   const bool wide = vdim % 32 == 0 && long_runs * heads * (vdim / 16) > 512;
   const dim3 scan((unsigned)(pairs * (vdim / (wide ? 32 : 16))));

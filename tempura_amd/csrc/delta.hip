@@ -6,266 +6,31 @@
 // A request r of the batch owns tokens cu_seqlens[r] .. cu_seqlens[r + 1] - 1 and the state row state_slots[r];
 // everything is read from device memory, so the same launches serve prompt portions, single decoded tokens and
 // captured steps.  In short runs a token's result does not depend on how its run was cut: every token is one step of the
-// same chain, in the same order of operations; long runs go by groups of tokens (delta_chunks.hip), which changes rounding only.
+// same chain, in the same order of operations; runs of 64 tokens and more go by groups of tokens (delta_chunks.hip), which changes rounding only.
 // What other requests bring does not matter to either.
 #include <math.h>
 
 #include "common.h"
 #include "column_sum.h"
+#include "delta_chain.h"
 
-__device__ inline float d_sigmoid(float v) { return 1.0f / (1.0f + expf(-v)); }
 // ln(1 + e^v) without overflow: max(v, 0) + ln(1 + e^-|v|)
 __device__ inline float d_softplus(float v) { return fmaxf(v, 0.f) + log1pf(expf(-fabsf(v))); }
 
-// ---- the recurrence ---------------------------------------------------------------------------
-// Per head h (its q and k are those of key head h / (heads / kv_heads)), with q and k made unit vectors
-// (x / sqrt(sum x^2 + unit_eps); q also times q_scale), beta = sigmoid(beta_raw) and a decay g per key channel:
-//   S <- g * S (rows are key channels);  u = beta (v - S^T k);  S <- S + k u^T;  o = S^T q.
-// With P = (g * S_old)^T k and R = (g * S_old)^T q the read-out is o = R + u (k . q), so one pass over a thread's
-// state entries forms both sums, one reduction over the lanes that share a column adds them, and a second pass
-// writes k u^T.
-//
-// qkv [n, row_stride] float32 holds, per token, q [kv_heads * dim] | k [kv_heads * dim] | v [heads * vdim] (after the
-// convolution and its activation); decay [n, heads * dim]; beta_raw is column beta_col0 + h of `proj`.
-//
-// Two kernels.  delta_prep (a wave per token and key head, all tokens side by side) makes q and k unit vectors in
-// place and leaves k . q per token and key head.  delta_scan is the chain: a block owns one request, one head and
-// CB = 256 / KS value columns; a thread holds PER consecutive key channels of one column in registers, and the KS
-// neighbouring lanes that share a column split the key channels among them (their sums meet by row permutes, no
-// trip through LDS up to 16 lanes).  A wave has one instruction stream, so the time of a token is the number of
-// instructions a wave issues for it: few state entries a lane (8 up to a key size of 128) keep that near 60.
-// Tokens are taken TC at a time through LDS (rows padded to KS * PER channels with q = k = 0 and decay 1, so the
-// run itself needs no bounds); the next chunk's values travel from memory into registers while this chunk runs.
-struct DeltaArgs {
-  float* qkv;
-  int row_stride;
-  const float* decay;
-  const float* proj;
-  int proj_stride, beta_col0;
-  float* state;
-  size_t state_stride, state_off;
-  const int* cu_seqlens;
-  const int* state_slots;
-  float* y;
-  float* kq;   // [n, kv_heads]
-  int heads, kv_heads, dim, vdim;
-  float q_scale, unit_eps;
-  int n_req;
-  int longest;   // runs of more tokens have been taken by groups (delta_chunks.hip); 0: none has
-};
-
-// Whether token t belongs to a run of more than `longest` tokens (the same in every lane of a wave; all of them come here).
-__device__ inline bool in_longer_run(const int* cu_seqlens, int n_req, int t, int longest, int lane) {
-  for (int r0 = 0; r0 < n_req; r0 += TP_WAVE) {
-    const int r = r0 + lane;
-    const int a = r < n_req ? cu_seqlens[r] : 0, b = r < n_req ? cu_seqlens[r + 1] : 0;
-    const bool own = a <= t && t < b;
-    if (__any(own)) return __any(own && b - a > longest);
-  }
-  return false;
-}
-
+// ---- the recurrence: delta_chain.h ------------------------------------------------------------
 __global__ __launch_bounds__(256) void delta_prep_kernel(DeltaArgs a, long pairs) {
   const long p = (long)blockIdx.x * 4 + threadIdx.x / TP_WAVE;
-  const int lane = threadIdx.x % TP_WAVE;
-  if (p >= pairs) return;
-  const long t = p / a.kv_heads;
-  if (a.longest > 0 && in_longer_run(a.cu_seqlens, a.n_req, (int)t, a.longest, lane)) return;
-  const int g = (int)(p % a.kv_heads);
-  float* q = a.qkv + (size_t)t * a.row_stride + (size_t)g * a.dim;
-  float* k = q + (size_t)a.kv_heads * a.dim;
-  float sq = 0.f, sk = 0.f;
-  for (int i = lane; i < a.dim; i += TP_WAVE) {
-    sq = fmaf(q[i], q[i], sq);
-    sk = fmaf(k[i], k[i], sk);
-  }
-  sq = wave_sum(sq);
-  sk = wave_sum(sk);
-  const float rq = a.q_scale / sqrtf(sq + a.unit_eps), rk = 1.0f / sqrtf(sk + a.unit_eps);
-  float dot = 0.f;
-  for (int i = lane; i < a.dim; i += TP_WAVE) {
-    const float qv = q[i] * rq, kv = k[i] * rk;
-    q[i] = qv;
-    k[i] = kv;
-    dot = fmaf(qv, kv, dot);
-  }
-  dot = wave_sum(dot);
-  if (lane == 0) a.kq[p] = dot;
+  if (p < pairs) delta_unit_rows(a, p / a.kv_heads, (int)(p % a.kv_heads), threadIdx.x % TP_WAVE);
 }
 
 template <int PER, int KS>
 __global__ __launch_bounds__(256) void delta_scan_kernel(DeltaArgs a) {
-  constexpr int DP = PER * KS, CW = TP_WAVE / KS, CB = 4 * CW;
-  constexpr int TC = DP <= 256 ? 16 : 4096 / DP;
-  constexpr int NI = (TC * DP + 255) / 256, NV = (TC * CB + 255) / 256;
-  __shared__ __attribute__((aligned(16))) float qs[TC * DP];
-  __shared__ __attribute__((aligned(16))) float kk[TC * DP];
-  __shared__ __attribute__((aligned(16))) float gs[TC * DP];
-  __shared__ float vs[TC * CB];
-  __shared__ float bs[TC];
-  __shared__ float kqs[TC];
-  const int r = blockIdx.x, h = blockIdx.y;
-  const int start = a.cu_seqlens[r], len = a.cu_seqlens[r + 1] - start;
-  if (len <= 0 || (a.longest > 0 && len > a.longest)) return;
-  const int tid = threadIdx.x, wave = tid / TP_WAVE, lane = tid % TP_WAVE;
-  const int ks = lane % KS, jl = wave * CW + lane / KS;
-  const int j = blockIdx.z * CB + jl;
-  const bool col_ok = j < a.vdim;
-  const int kvh = h / (a.heads / a.kv_heads);
-
-  // a head's state lies in memory column by column, [vdim][dim]: the key channels of one value column are
-  // neighbours, so a lane's entries are one or two 16-byte pieces and a wave's columns one contiguous run
-  float* S_mem = a.state + (size_t)a.state_slots[r] * a.state_stride + a.state_off + ((size_t)h * a.vdim + (col_ok ? j : 0)) * a.dim;
-  const bool vec = a.dim % 4 == 0 && ((uintptr_t)S_mem % 16) == 0;
-  float S[PER];
-#pragma unroll
-  for (int e4 = 0; e4 < PER / 4; ++e4) {
-    const int i = ks * PER + e4 * 4;
-    if (vec && col_ok && i < a.dim) {
-      const float4 v = *(const float4*)(S_mem + i);
-      S[e4 * 4 + 0] = v.x; S[e4 * 4 + 1] = v.y; S[e4 * 4 + 2] = v.z; S[e4 * 4 + 3] = v.w;
-    } else {
-#pragma unroll
-      for (int c = 0; c < 4; ++c) S[e4 * 4 + c] = (col_ok && i + c < a.dim) ? S_mem[i + c] : 0.f;
-    }
-  }
-  const int q_col = kvh * a.dim, k_col = (a.kv_heads + kvh) * a.dim, v_col = 2 * a.kv_heads * a.dim + h * a.vdim;
-  const int out_width = a.heads * a.vdim;
-  const size_t decay_stride = (size_t)a.heads * a.dim;
-
-  float rq[NI], rk[NI], rg[NI], rv[NV], rb = 0.f, rkq = 0.f;
-  auto fetch = [&](int t0) {
-#pragma unroll
-    for (int it = 0; it < NI; ++it) {
-      const int idx = it * 256 + tid;
-      const int t = idx / DP, i = idx % DP;
-      const bool in = idx < TC * DP && t0 + t < len && i < a.dim;
-      const size_t row = (size_t)(start + t0 + t);
-      rq[it] = in ? a.qkv[row * a.row_stride + q_col + i] : 0.f;
-      rk[it] = in ? a.qkv[row * a.row_stride + k_col + i] : 0.f;
-      rg[it] = in ? a.decay[row * decay_stride + (size_t)h * a.dim + i] : 1.f;
-    }
-#pragma unroll
-    for (int it = 0; it < NV; ++it) {
-      const int idx = it * 256 + tid;
-      const int t = idx / CB, c = idx % CB;
-      const int col = blockIdx.z * CB + c;
-      rv[it] = (idx < TC * CB && t0 + t < len && col < a.vdim) ? a.qkv[(size_t)(start + t0 + t) * a.row_stride + v_col + col] : 0.f;
-    }
-    if (tid < TC && t0 + tid < len) {
-      const size_t row = (size_t)(start + t0 + tid);
-      rb = d_sigmoid(a.proj[row * a.proj_stride + a.beta_col0 + h]);
-      rkq = a.kq[row * a.kv_heads + kvh];
-    }
-  };
-  struct Tok {
-    float4 q[PER / 4], k[PER / 4], g[PER / 4];
-    float b, v, kq;
-  };
-  auto take = [&](Tok& x, int t) {
-    const float4* q4 = (const float4*)(qs + t * DP + ks * PER);
-    const float4* k4 = (const float4*)(kk + t * DP + ks * PER);
-    const float4* g4 = (const float4*)(gs + t * DP + ks * PER);
-#pragma unroll
-    for (int e4 = 0; e4 < PER / 4; ++e4) {
-      x.q[e4] = q4[e4];
-      x.k[e4] = k4[e4];
-      x.g[e4] = g4[e4];
-    }
-    x.b = bs[t];
-    x.v = vs[t * CB + jl];
-    x.kq = kqs[t];
-  };
-  auto step = [&](const Tok& x, int t_run) {
-    float pred[PER / 4], read[PER / 4];
-#pragma unroll
-    for (int e4 = 0; e4 < PER / 4; ++e4) {
-      const float qa[4] = {x.q[e4].x, x.q[e4].y, x.q[e4].z, x.q[e4].w}, ka[4] = {x.k[e4].x, x.k[e4].y, x.k[e4].z, x.k[e4].w},
-                  ga[4] = {x.g[e4].x, x.g[e4].y, x.g[e4].z, x.g[e4].w};
-      float p = 0.f, rd = 0.f;
-#pragma unroll
-      for (int c = 0; c < 4; ++c) {
-        const int e = e4 * 4 + c;
-        S[e] *= ga[c];
-        p = fmaf(S[e], ka[c], p);
-        rd = fmaf(S[e], qa[c], rd);
-      }
-      pred[e4] = p;
-      read[e4] = rd;
-    }
-    float ps = pred[0], rs = read[0];
-#pragma unroll
-    for (int e4 = 1; e4 < PER / 4; ++e4) {   // (a fixed order: the same sums wherever the token stands)
-      ps += pred[e4];
-      rs += read[e4];
-    }
-    ps = column_sum<KS>(ps);
-    rs = column_sum<KS>(rs);
-    const float u = x.b * (x.v - ps);
-#pragma unroll
-    for (int e4 = 0; e4 < PER / 4; ++e4) {
-      S[e4 * 4 + 0] = fmaf(x.k[e4].x, u, S[e4 * 4 + 0]);
-      S[e4 * 4 + 1] = fmaf(x.k[e4].y, u, S[e4 * 4 + 1]);
-      S[e4 * 4 + 2] = fmaf(x.k[e4].z, u, S[e4 * 4 + 2]);
-      S[e4 * 4 + 3] = fmaf(x.k[e4].w, u, S[e4 * 4 + 3]);
-    }
-    if (ks == 0 && col_ok) a.y[(size_t)(start + t_run) * out_width + (size_t)h * a.vdim + j] = fmaf(u, x.kq, rs);
-  };
-  fetch(0);
-  for (int t0 = 0; t0 < len; t0 += TC) {
-    const int tc = min(TC, len - t0);
-    __syncthreads();   // the chunk before has been consumed
-#pragma unroll
-    for (int it = 0; it < NI; ++it) {
-      const int idx = it * 256 + tid;
-      if (idx < TC * DP) {
-        qs[idx] = rq[it];
-        kk[idx] = rk[it];
-        gs[idx] = rg[it];
-      }
-    }
-#pragma unroll
-    for (int it = 0; it < NV; ++it) {
-      const int idx = it * 256 + tid;
-      if (idx < TC * CB) vs[idx] = rv[it];
-    }
-    if (tid < TC) {
-      bs[tid] = rb;
-      kqs[tid] = rkq;
-    }
-    __syncthreads();
-    if (t0 + TC < len) fetch(t0 + TC);   // on its way while this chunk runs
-    // two tokens a turn, each token's LDS reads issued before the token ahead of it is worked on: a wave issues in
-    // order, and reads that start only when the chain reaches them would add their whole latency to every token
-    Tok A, B;
-    take(A, 0);
-    for (int t = 0; t < tc; t += 2) {
-      if (t + 1 < tc) take(B, t + 1);
-      step(A, t0 + t);
-      if (t + 1 < tc) {
-        if (t + 2 < tc) take(A, t + 2);
-        step(B, t0 + t + 1);
-      }
-    }
-  }
-#pragma unroll
-  for (int e4 = 0; e4 < PER / 4; ++e4) {
-    const int i = ks * PER + e4 * 4;
-    if (vec && col_ok && i < a.dim) {
-      *(float4*)(S_mem + i) = make_float4(S[e4 * 4 + 0], S[e4 * 4 + 1], S[e4 * 4 + 2], S[e4 * 4 + 3]);
-    } else {
-#pragma unroll
-      for (int c = 0; c < 4; ++c)
-        if (col_ok && i + c < a.dim) S_mem[i + c] = S[e4 * 4 + c];
-    }
-  }
+  delta_chain<PER, KS>(a, blockIdx.x, blockIdx.y, blockIdx.z);
 }
 
-// Defined in delta_chunks.hip: takes the runs of more than the returned number of tokens; -1: none.
-int tp_delta_chunks(const float* qkv, int row_stride, const float* decay, const float* proj, int proj_stride, int beta_col0, float* state,
-                    size_t state_stride, size_t state_off, const int* cu_seqlens, const int* state_slots, float* y, int n, int n_req, int heads,
-                    int kv_heads, int dim, int vdim, float q_scale, float unit_eps, int max_run, float* scratch, size_t scratch_floats,
-                    hipStream_t s);
+// Defined in delta_chunks.hip: 0 when it took the runs (long ones by groups of tokens, the others by the chain), -1 when none is a long one
+// of its own.
+int tp_delta_chunks(const DeltaArgs& chain, int n, int n_req, int max_run, float* scratch, size_t scratch_floats, hipStream_t s);
 
 // max_run: the longest run, 0: not known (scratch of tp_delta_scan_scratch floats lets long runs go by groups of tokens).
 extern "C" int tp_delta_scan(float* qkv, int row_stride, const float* decay, const float* proj, int proj_stride,
@@ -279,14 +44,12 @@ extern "C" int tp_delta_scan(float* qkv, int row_stride, const float* decay, con
   TP_REQUIRE(state_stride >= state_off + (size_t)heads * dim * vdim, "delta_scan: state rows too short");
   TP_REQUIRE(heads <= 65535, "delta_scan: too many heads");
   if (n == 0 || n_req == 0) return 0;
-  const int longest = tp_delta_chunks(qkv, row_stride, decay, proj, proj_stride, beta_col0, state, state_stride, state_off, cu_seqlens, state_slots,
-                                      y, n, n_req, heads, kv_heads, dim, vdim, q_scale, unit_eps, max_run, scratch, scratch_floats, s);
-  if (longest >= 0) {
+  const DeltaArgs a{qkv, row_stride, decay, proj, proj_stride, beta_col0, state, state_stride, state_off, cu_seqlens, state_slots, y, kq,
+                    heads, kv_heads, dim, vdim, q_scale, unit_eps};
+  if (tp_delta_chunks(a, n, n_req, max_run, scratch, scratch_floats, s) == 0) {
     TP_CHECK_LAUNCH("delta_scan (groups)");
-    if ((long)n - (long)(n_req - 1) * max_run > longest) return 0;      // (the shortest run that such tokens can leave is a long one)
+    return 0;
   }
-  DeltaArgs a{qkv, row_stride, decay, proj, proj_stride, beta_col0, state, state_stride, state_off, cu_seqlens, state_slots, y, kq,
-              heads, kv_heads, dim, vdim, q_scale, unit_eps, n_req, longest < 0 ? 0 : longest};
   const long pairs = (long)n * kv_heads;
   TP_REQUIRE((pairs + 3) / 4 < 0x7fffffffL, "delta_scan: too many rows");
   hipLaunchKernelGGL(delta_prep_kernel, dim3((unsigned)((pairs + 3) / 4)), dim3(256), 0, s, a, pairs);

@@ -16,38 +16,39 @@
 // are added last, where a sum's roundings are few.  Root mean square error against float64 over that of the chain, runs of 112, 300 and
 // 1,000 tokens: decays of 0 to 1 a token 0.91 (states 0.99), 0.5 to 1 0.93 (0.97), 0.8 to 1 0.96 (0.95), 0.9 to 1 0.94 (0.92), 0.99 to 1
 // 0.82 (0.81).  (In float32 throughout, tokens in the order of the rows and U = T V - (T K~) S it was 1.03, 1.06, 1.08, 1.06 and 0.94;
-// one run of 2,048 tokens then took 201 us, now 219, four of 451 tokens 92 and 91, with 32 heads eight of 256 159 and 175.)
+// one run of 2,048 tokens then took 201 us, now 198, four of 451 tokens 92 and 93, with 32 heads eight of 256 160 and 177.)
 //
-// The chain of single tokens is bound by what a wave issues and waits for a token, 0.25 to 0.55 us; here a group of 16 takes 1.4 us (its
-// products, a meeting in LDS and the update, each waiting for the one before).  16 heads of 128 x 128, single tokens / groups: one run of
-// 128 tokens 41 / 31 us, 256 75 / 42, 2,048 495 / 219; four runs of 451 tokens 162 / 91 (a third of it the first kernel); a long run and
-// single tokens beside it, with the chain that takes these: 700 and 31 1,329 / 115, 1,800 and 63 3,411 / 243, 1,800 and 247 1,304 / 378;
-// the other way about, 200 and ten of 90, 123 / 135 (the two kinds run one behind the other).
+// Runs of fewer than 64 tokens (DC_SHORT) go by the chain (delta_chain.h) in further blocks of the same two launches, so that a step's
+// long and short runs take the time of the longer way and not of both.
+//
+// The chain of single tokens is bound by what a wave issues and waits for a token, 0.25 to 0.55 us; here a group of 16 takes 1.3 us (its
+// products, a meeting in LDS and the update, each waiting for the one before).  16 heads of 128 x 128, all by single tokens / as here: one
+// run of 128 tokens 37 / 28 us, 2,048 486 / 198; four runs of 451 tokens 162 / 93 (a third of it the first kernel); runs of 82, 327, 573 and
+// 821 tokens 262 / 118; 700 tokens beside 31 single ones 1,327 / 85, 1,800 beside 63 3,412 / 190, beside 247 1,316 / 324; 200 beside ten of
+// 63 105 / 87.  What loses: short runs whose work is most of the step, which the registers of the groups' kernel hold to two blocks a CU
+// (64 tokens beside seven of 63 56 / 63, beside 100 single ones 70 / 100).
 #include <math.h>
 
 #include "common.h"
 #include "column_sum.h"
+#include "delta_chain.h"
 
 typedef float f32x4_d __attribute__((ext_vector_type(4)));
 
 #define DC_T 16      // tokens of a group
-// Runs of up to this many tokens are left to the chain of single tokens, whatever runs stand beside them: a request's bits do not depend
-// on its neighbours.  (16 heads of 128 x 128, one run, single tokens / groups: 64 tokens 25 / 28 us, 96 33 / 32, 128 41 / 31.)
-#define DC_SHORT 96
+// Runs of up to this many tokens go by the chain of single tokens, whatever runs stand beside them: a request's bits do not depend on its
+// neighbours.  (Alone the two ways meet at 64 tokens, several runs sooner.  16 heads of 128 x 128, single tokens / groups: one run of 48
+// tokens 18 / 20 us, 64 22 / 21, 96 29 / 24; three of 48 22 / 24, 64 28 / 27; eight of 32 29 / 27, 64 49 / 36.  Eight heads of 64 x 64: one
+// of 48 16 / 17, 64 19 / 18; 24 of 48 22 / 25, 64 28 / 28.)
+#define DC_SHORT 63
+#define DC_HEADS 4    // key heads a wave makes unit vectors of, for those runs
 
 struct DeltaChunkArgs {
-  const float* qkv;
-  const float* decay;
-  const float* proj;
-  float* state;
-  const int* cu_seqlens;
-  const int* state_slots;
-  float* y;
+  DeltaArgs in;           // (its q and k as they come: a group makes unit vectors of its own)
   float* scratch;
-  size_t state_stride, state_off;
-  int row_stride, proj_stride, beta_col0, heads, kv_heads, vdim, requests;
+  int requests;
   int first, groups;      // the groups that this launch takes, among those of all long runs one behind the other
-  float q_scale, unit_eps;
+  int blocks;             // that many blocks take groups; those behind them the runs of up to DC_SHORT tokens (all in the first launch)
 };
 
 // Where a token of the group lies among the rows and columns of the operands: instruction i of a product over the tokens takes element i
@@ -99,6 +100,15 @@ __device__ inline bool dc_find_group(const int* cu_seqlens, int requests, int i,
       return true;
     }
     i -= __shfl(upto, TP_WAVE - 1, TP_WAVE);
+  }
+  return false;
+}
+
+// Whether token t belongs to a run that goes by groups (the same in every lane).
+__device__ inline bool dc_in_long_run(const int* cu_seqlens, int requests, int t, int lane) {
+  for (int r0 = 0; r0 < requests; r0 += TP_WAVE) {
+    const int r = r0 + lane, a = r < requests ? cu_seqlens[r] : 0, b = r < requests ? cu_seqlens[r + 1] : 0;
+    if (__any(a <= t && t < b)) return __any(a <= t && t < b && b - a > DC_SHORT);
   }
   return false;
 }
@@ -157,15 +167,22 @@ __device__ inline void dc_dots(const float (&q)[DC_T][PER], const float (&k)[DC_
 }
 
 template <int PER>
-__global__ __launch_bounds__(64) void delta_chunk_prep_kernel(DeltaChunkArgs a) {
+__global__ __launch_bounds__(64) void delta_chunk_prep_kernel(DeltaChunkArgs c) {
   constexpr int K = 64 * PER;
   __shared__ float dots[256];
   __shared__ float bs[DC_T];
   const int lane = threadIdx.x;
+  const DeltaArgs& a = c.in;
+  if ((int)blockIdx.x >= c.blocks) {      // unit vectors of the chain's tokens, DC_HEADS key heads a wave
+    const int parts = (a.kv_heads + DC_HEADS - 1) / DC_HEADS, i = blockIdx.x - c.blocks, t = i / parts, g0 = i % parts * DC_HEADS;
+    if (dc_in_long_run(a.cu_seqlens, c.requests, t, lane)) return;
+    for (int g = g0; g < min(g0 + DC_HEADS, a.kv_heads); ++g) delta_unit_rows(a, t, g, lane);
+    return;
+  }
   const int h = blockIdx.x % a.heads, at = blockIdx.x / a.heads;
-  int r, c;
-  if (!dc_find_group(a.cu_seqlens, a.requests, a.first + at, lane, r, c)) return;
-  const int run0 = a.cu_seqlens[r], t0 = c * DC_T, len = min(DC_T, a.cu_seqlens[r + 1] - run0 - t0);
+  int r, number;
+  if (!dc_find_group(a.cu_seqlens, c.requests, c.first + at, lane, r, number)) return;
+  const int run0 = a.cu_seqlens[r], t0 = number * DC_T, len = min(DC_T, a.cu_seqlens[r + 1] - run0 - t0);
   const size_t row0 = (size_t)(run0 + t0);
   const int g = h / (a.heads / a.kv_heads);
   const float* qp = a.qkv + row0 * a.row_stride + (size_t)g * K;
@@ -214,7 +231,7 @@ __global__ __launch_bounds__(64) void delta_chunk_prep_kernel(DeltaChunkArgs a) 
     float v[64];
     dc_dots<0, PER>(q, k, gd, v, dots, lane);
   }
-  float* item = a.scratch + ((size_t)at * a.heads + h) * dc_item_floats(K);
+  float* item = c.scratch + ((size_t)at * a.heads + h) * dc_item_floats(K);
   float *Kt = item, *Q = Kt + DC_T * K, *KT = Q + DC_T * K, *G = KT + DC_T * K, *T = G + K, *B = T + 256, *diag = B + 256;
 #pragma unroll
   for (int p = 0; p < PER; ++p) {
@@ -281,26 +298,33 @@ __device__ inline bool dc_finite(const f32x4_d& x) {
 
 // CT: tiles of 16 value columns a block.
 template <int KT, int CT>
-__global__ __launch_bounds__(256) void delta_chunk_scan_kernel(DeltaChunkArgs a) {
+__global__ __launch_bounds__(256) void delta_chunk_scan_kernel(DeltaChunkArgs x) {
   constexpr int K = 16 * KT, TILES = KT / 4;      // 16-channel tiles of a wave
+  const DeltaArgs& a = x.in;
+  if ((int)blockIdx.x >= x.blocks) {      // the chain: as many lanes a column as in delta.hip's kernel of this key size
+    constexpr int KS = K / 8, CB = 4 * TP_WAVE / KS;
+    const int i = blockIdx.x - x.blocks, strips = (a.vdim + CB - 1) / CB, r = i / (a.heads * strips);
+    if (a.cu_seqlens[r + 1] - a.cu_seqlens[r] <= DC_SHORT) delta_chain<8, KS>(a, r, i / strips % a.heads, i % strips);
+    return;
+  }
   __shared__ f32x4_d part[2][4][2 * CT][TP_WAVE];
   const int lane = threadIdx.x % TP_WAVE, wave = threadIdx.x / TP_WAVE, col = lane % 16, quad = lane / 16;
   // The blocks of a head read the same W, Q~ and K^: they go side by side to one XCD and its L2, and the heads to the XCDs in turn.
-  const int strips = a.vdim / (16 * CT), pairs = a.requests * a.heads;
+  const int strips = a.vdim / (16 * CT), pairs = x.requests * a.heads;
   const int rest = blockIdx.x >> 3, pair = rest / strips * 8 + (blockIdx.x & 7), strip = rest % strips;
   if (pair >= pairs) return;
   const int h = pair % a.heads, r = pair / a.heads;
   const int run = a.cu_seqlens[r + 1] - a.cu_seqlens[r];
   if (run <= DC_SHORT) return;
   // this run's groups that the launch holds: from its c0-th on, where `begin` is the launch's first for this run
-  const int begin = dc_first_group(a.cu_seqlens, r, lane) - a.first, c0 = max(0, -begin);
-  const int groups = min(a.groups - begin, (run + DC_T - 1) / DC_T) - c0;
+  const int begin = dc_first_group(a.cu_seqlens, r, lane) - x.first, c0 = max(0, -begin);
+  const int groups = min(x.groups - begin, (run + DC_T - 1) / DC_T) - c0;
   if (groups <= 0) return;
   const int run0 = a.cu_seqlens[r] + c0 * DC_T, left = run - c0 * DC_T;      // (the run from there on)
   const int j0 = strip * 16 * CT + col, i0 = wave * TILES * 16;      // (this lane's columns: j0 + 16 n)
   const size_t size = dc_item_floats(K);
   const float* vcol = a.qkv + (size_t)run0 * a.row_stride + 2 * (size_t)a.kv_heads * K + (size_t)h * a.vdim + j0;
-  const float* item = a.scratch + ((size_t)(begin + c0) * a.heads + h) * size;
+  const float* item = x.scratch + ((size_t)(begin + c0) * a.heads + h) * size;
   float* Sm = a.state + (size_t)a.state_slots[r] * a.state_stride + a.state_off + ((size_t)h * a.vdim + j0) * K;
   f32x4_d S[CT][TILES];
 #pragma unroll
@@ -384,14 +408,14 @@ __global__ __launch_bounds__(256) void delta_chunk_scan_kernel(DeltaChunkArgs a)
       }
     }
   };
-  Group x, y;
-  fetch(x, 0);
+  Group even, odd;
+  fetch(even, 0);
   for (int c = 0; c < groups; c += 2) {
-    if (c + 1 < groups) fetch(y, c + 1);
-    step(x, c);
+    if (c + 1 < groups) fetch(odd, c + 1);
+    step(even, c);
     if (c + 1 < groups) {
-      if (c + 2 < groups) fetch(x, c + 2);
-      step(y, c + 1);
+      if (c + 2 < groups) fetch(even, c + 2);
+      step(odd, c + 1);
     }
   }
 #pragma unroll
@@ -422,39 +446,41 @@ extern "C" size_t tp_delta_scan_scratch(int n, int n_req, int max_run, int heads
   return (size_t)dc_groups(n, n_req, max_run, heads, dim, vdim, &all) * heads * dc_item_floats(dim);
 }
 
-// Takes the runs of more than the returned number of tokens (-1: none of them are its own).  q and k of qkv are read as they come, before
-// they are unit vectors, and left alone.
-int tp_delta_chunks(const float* qkv, int row_stride, const float* decay, const float* proj, int proj_stride, int beta_col0, float* state,
-                    size_t state_stride, size_t state_off, const int* cu_seqlens, const int* state_slots, float* y, int n, int n_req, int heads,
-                    int kv_heads, int dim, int vdim, float q_scale, float unit_eps, int max_run, float* scratch, size_t scratch_floats,
-                    hipStream_t s) {
+// Returns 0 when it took the step's runs, -1 when none of them is a long one of its own.
+int tp_delta_chunks(const DeltaArgs& in, int n, int n_req, int max_run, float* scratch, size_t scratch_floats, hipStream_t s) {
+  const int heads = in.heads, dim = in.dim, vdim = in.vdim;
   int all;
   const int groups = dc_groups(n, n_req, max_run, heads, dim, vdim, &all);
   if (groups == 0 || scratch == nullptr || ((uintptr_t)scratch & 15) || scratch_floats < (size_t)groups * heads * dc_item_floats(dim)) return -1;
-  DeltaChunkArgs a{qkv, decay, proj, state, cu_seqlens, state_slots, y, scratch, state_stride, state_off, row_stride, proj_stride, beta_col0,
-                   heads, kv_heads, vdim, n_req, 0, groups, q_scale, unit_eps};
-  const long pairs = ((long)n_req * heads + 7) / 8 * 8;
   // (32 columns a block read K~, Q~ and K^ half as often, which bounds the chain once there are more blocks of 16 columns than the two
   // a CU that run at a time: 16 heads of 128 x 128, four runs of 451 tokens, 512 blocks of 16 columns or half as many of 32: 94 / 102 us;
   // 32 heads, eight runs of 256, 2,048 blocks: 202 / 174 when the rule was made.  Blocks of short runs end at once and do not count.)
   const long others = max_run < n ? (n - max_run) / (DC_SHORT + 1) : 0, long_runs = 1 + (others < n_req - 1 ? others : n_req - 1);
   const bool wide = vdim % 32 == 0 && long_runs * heads * (vdim / 16) > 512;
-  const dim3 scan((unsigned)(pairs * (vdim / (wide ? 32 : 16))));
+  // Short runs go beside the long ones, in blocks behind theirs (one behind the other the two kinds would add their chains), unless the
+  // shortest run that such a step can have is a long one.
+  const bool short_runs = (long)n - (long)(n_req - 1) * max_run <= DC_SHORT;
+  const int column_block = dim == 128 ? 16 : 32;
+  const long unit_blocks = short_runs ? (long)n * ((in.kv_heads + DC_HEADS - 1) / DC_HEADS) : 0;
+  const long chain_blocks = short_runs ? (long)n_req * heads * ((vdim + column_block - 1) / column_block) : 0;
+  const long scan_blocks = ((long)n_req * heads + 7) / 8 * 8 * (vdim / (wide ? 32 : 16));
+  if ((long)groups * heads + unit_blocks >= 0x7fffffffL || scan_blocks + chain_blocks >= 0x7fffffffL) return -1;
+  DeltaChunkArgs a{in, scratch, n_req, 0, groups, 0};
+  for (; a.first < all; a.first += groups) {
+    const long prep_blocks = (long)(groups < all - a.first ? groups : all - a.first) * heads;
+    const dim3 prep((unsigned)(prep_blocks + (a.first == 0 ? unit_blocks : 0))), scan((unsigned)(scan_blocks + (a.first == 0 ? chain_blocks : 0)));
+    a.blocks = (int)prep_blocks;
+    if (dim == 128) hipLaunchKernelGGL(delta_chunk_prep_kernel<2>, prep, dim3(64), 0, s, a);
+    else hipLaunchKernelGGL(delta_chunk_prep_kernel<1>, prep, dim3(64), 0, s, a);
+    a.blocks = (int)scan_blocks;
 #define DC_SCAN(KT_)                                                                                                 \
   do {                                                                                                               \
     if (wide) hipLaunchKernelGGL((delta_chunk_scan_kernel<KT_, 2>), scan, dim3(256), 0, s, a);                       \
     else hipLaunchKernelGGL((delta_chunk_scan_kernel<KT_, 1>), scan, dim3(256), 0, s, a);                            \
   } while (0)
-  for (; a.first < all; a.first += groups) {
-    const dim3 prep((unsigned)((long)(groups < all - a.first ? groups : all - a.first) * heads));
-    if (dim == 128) {
-      hipLaunchKernelGGL(delta_chunk_prep_kernel<2>, prep, dim3(64), 0, s, a);
-      DC_SCAN(8);
-    } else {
-      hipLaunchKernelGGL(delta_chunk_prep_kernel<1>, prep, dim3(64), 0, s, a);
-      DC_SCAN(4);
-    }
-  }
+    if (dim == 128) DC_SCAN(8);
+    else DC_SCAN(4);
 #undef DC_SCAN
-  return DC_SHORT;
+  }
+  return 0;
 }

@@ -1719,8 +1719,8 @@ def delta_scan(qkv: torch.Tensor, decay: torch.Tensor, proj: torch.Tensor, beta_
     ``q_scale``); beta = sigmoid(proj[:, beta_col0 + h]); ``decay`` float32 [n, heads * dim].  Per head, with S
     [dim, vdim] (kept at ``state[slot, state_off:]`` column by column, [heads, vdim, dim]):  S <- decay * S;  u = beta (v - S^T k);  S <- S + k u^T;  o = S^T q.
     Returns o float32 [n, heads * vdim]; the state is left as the run leaves it.  (q and k of ``qkv`` may be left as
-    unit vectors: the rows are a temporary of the caller's.)  ``max_run``: the longest run (0: not known); runs of some
-    hundred tokens go by groups of tokens, which changes rounding only, whatever runs stand beside them."""
+    unit vectors: the rows are a temporary of the caller's.)  ``max_run``: the longest run (0: not known); runs of 64
+    tokens and more go by groups of tokens, which changes rounding only, whatever runs stand beside them."""
     if _backend is not None:
         return _backend.delta_scan(qkv, decay, proj, beta_col0, state, state_off, cu_seqlens, state_slots, num_requests, heads,
                                    kv_heads, dim, vdim, q_scale, unit_eps)

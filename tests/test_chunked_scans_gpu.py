@@ -180,7 +180,7 @@ def test_delta_rule_by_groups_rounds_no_more_than_token_by_token(low):
 def test_delta_rule_of_a_run_does_not_depend_on_its_neighbours(H, G, D, Dv):
     """Decoded tokens and short portions beside long ones: the bits, outputs and states, that every run has alone."""
     from tempura_amd.kernels import ops
-    lens = [300, 1, 96, 0, 20, 97] + [1] * 70 + [50, 257]
+    lens = [300, 1, 63, 0, 20, 64] + [1] * 70 + [50, 257]
     qkv, decay, proj, state, cu, slots = (t.to(DEV) for t in _delta_inputs(lens, H, G, D, Dv, 31, 0.8))
     together = state.clone()
     y = ops.delta_scan(qkv.clone(), decay, proj, 2, together, 5, cu, slots, len(lens), H, G, D, Dv, D ** -0.5, 1e-6, max_run=max(lens))
@@ -192,7 +192,7 @@ def test_delta_rule_of_a_run_does_not_depend_on_its_neighbours(H, G, D, Dv):
                                  D ** -0.5, 1e-6, max_run=n)
             assert torch.equal(y[rows], got), n
         assert torch.equal(together[int(slots[i])], alone[int(slots[i])]), n
-        if n in (20, 96):      # (and those that its tokens have one a step)
+        if n in (20, 63):      # (and those that its tokens have one a step)
             alone, one = state.clone(), torch.tensor([0, 1], dtype=torch.int32, device=DEV)
             for t in range(int(cu[i]), int(cu[i + 1])):
                 got = ops.delta_scan(qkv[t: t + 1].clone(), decay[t: t + 1].contiguous(), proj[t: t + 1].contiguous(), 2, alone, 5, one, slots[i: i + 1],
@@ -209,13 +209,13 @@ def _held_groups(lens, H, D, Dv):
     return floats // (H * (49 * D + 528))
 
 
-@pytest.mark.parametrize("lens", [[1200, 700, 3] + [1] * 21, [1] * 70 + [97, 450, 96] + [1, 0] * 70 + [520, 100]])
+@pytest.mark.parametrize("lens", [[1200, 700, 3] + [1] * 21, [1] * 70 + [64, 450, 63] + [1, 0] * 70 + [520, 100]])
 def test_delta_rule_in_several_pairs_of_launches(lens):
     """More tokens and heads than the scratch holds at a time: each pair of launches goes on from the states that the one before left, also
     in the middle of a run; runs whose groups begin behind those of more than 64 others."""
     from tempura_amd.kernels import ops
     H, D, Dv = 160, 128, 16
-    assert 1 <= _held_groups(lens, H, D, Dv) < sum(-(-n // 16) for n in lens if n > 96)
+    assert 1 <= _held_groups(lens, H, D, Dv) < sum(-(-n // 16) for n in lens if n > 63)
     qkv, decay, proj, state, cu, slots = _delta_inputs(lens, H, H, D, Dv, 5, 0.9)
     dev = [t.to(DEV) for t in (decay, proj, cu, slots)]
     out = []
@@ -225,11 +225,11 @@ def test_delta_rule_in_several_pairs_of_launches(lens):
     assert _error(out[0][0], out[1][0].cpu()) <= 1e-6 and _error(out[0][1], out[1][1].cpu()) <= 1e-6
 
 
-@pytest.mark.parametrize("lens", [[1800] + [1] * 63, [1800] + [1] * 299, [97] * 11, [2000]])
+@pytest.mark.parametrize("lens", [[1800] + [1] * 63, [1800] + [1] * 299, [64] * 11, [2000]])
 def test_delta_rule_scratch_is_sized_by_tokens(lens):
     """A long run beside many single tokens needs the room of its own groups, and one more a run that could be long."""
-    need = sum(-(-n // 16) for n in lens if n > 96)
-    assert need <= _held_groups(lens, 16, 128, 128) <= sum(lens) // 16 + sum(lens) // 97
+    need = sum(-(-n // 16) for n in lens if n > 63)
+    assert need <= _held_groups(lens, 16, 128, 128) <= sum(lens) // 16 + sum(lens) // 64
 
 
 @pytest.mark.parametrize("bad", [float("inf"), float("nan")])

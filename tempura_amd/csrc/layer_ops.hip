@@ -12,8 +12,7 @@ __device__ inline float l_sigmoid(float v) { return 1.0f / (1.0f + expf(-v)); }
 // ---- embedding plus a row of a hashed bigram table --------------------------------------------
 // out[t] = table[token] * scale + bigram[row] (+ pos_table[position], a learned row per position), row = (previous * mul_prev + token * mul_cur) mod buckets, and row `buckets`
 // (the table's last) for the token at position 0.  The previous token is the one before it in the step's run, or,
-// for a run's first token, what the request's state row holds; a second kernel leaves each run's last token there.
-// (the previous token of the run's first token: read by that token's block alone, which then leaves the run's last token there)
+// for a run's first token, what the request's state row holds: that token's block alone reads it, and then leaves the run's last token there.
 template <typename T>
 __global__ void embed_bigram_kernel(const int* __restrict__ tokens, const int* __restrict__ positions,
                                     const int* __restrict__ token_req, const int* __restrict__ cu_seqlens,

@@ -7,7 +7,8 @@
 // threads owns one request and one head: it requests its state first (32 entries a thread), works out the head's inputs from LDS
 // while those loads travel, takes the step, norms its own read-out and writes the output columns.  It needs every head's inputs to be
 // its own: as many key heads as heads, keys of 33 to 128 and values of up to 128 elements, ranks of up to 128.
-// Sums are formed in the order of the kernels that serve runs of tokens (delta.hip, general_delta.hip, linear_scan.hip): the same bits.
+// Sums are formed in the order of the kernels that serve runs of tokens (delta.hip, general_delta.hip, linear_scan.hip): the same bits up
+// to 64 requests (of more rows tp_lowrank_up adds its products in ascending order, here as of up to 64 in eight shares).
 // Bound by those dependent trips up to a block a CU, by the state's 128 KB a head (read and written) beyond.  Gated delta rule, a
 // captured chain, separate kernels / one launch: 16 heads of 128 x 128, one request 17.8 / 8.8 us, four 19.2 / 9.4; 32 heads, eight
 // requests 26 / 14 us, 64 requests 85 / 68 us.  (At 128 registers a thread, two blocks a CU: 136 without the bound are 0.3 us less

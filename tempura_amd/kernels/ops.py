@@ -239,8 +239,9 @@ def scale_(x: torch.Tensor, scale: float) -> torch.Tensor:
 def gated_act(gu: torch.Tensor, out_dtype: torch.dtype, slope: float = 1.0, limit: float = 0.0, up_offset: float = 0.0,
               interleaved: bool = False) -> torch.Tensor:
     """[m, 2i] (gate columns then up columns; ``interleaved``: eight gate and eight up columns in turn, the layout of
-    ``interleave_gate_up``) -> out_dtype [m, i]: g = min(gate, limit), u = clamp(up, -limit, limit)
-    (limit <= 0: none), g * sigmoid(slope * g) * (u + up_offset)."""
+    ``interleave_gate_up``; no part asks for it, it is what the products that gate their own sums are tested against)
+    -> out_dtype [m, i]: g = min(gate, limit), u = clamp(up, -limit, limit) (limit <= 0: none),
+    g * sigmoid(slope * g) * (u + up_offset)."""
     if _backend is not None:
         return _backend.gated_act(gu, out_dtype, slope, limit, up_offset, interleaved)
     _dev_ok(gu)
@@ -575,7 +576,7 @@ def linear_swiglu(x, w: torch.Tensor, blocked_out: bool = False, slope: float = 
     silu(x g^T) * (x u^T), the gate applied to the float32 accumulators (no rounding in between).
     With ``blocked_out`` the result comes as ``KBlocked`` when there are at most 16 rows and i % 32 == 0 (else as a tensor).
     ``slope``, ``limit``, ``up_offset``: the general gate of ``gated_act`` (g' * sigmoid(slope g') * (u' + up_offset)
-    with both branches limited when limit > 0) in the same epilogue; the defaults are SwiGLU."""
+    with both branches limited when limit > 0) in the same epilogue (of up to 16 rows with that kernel's bits); the defaults are SwiGLU."""
     if _backend is not None:
         if (slope, limit, up_offset) != (1.0, 0.0, 0.0):
             return _backend.linear_swiglu(x, w, blocked_out, slope, limit, up_offset)
@@ -2123,7 +2124,8 @@ def linear_scan(q, k, v, decay: torch.Tensor, state: torch.Tensor, state_off: in
 # ---------------------------------------------------------------------------------
 # One token a request through a whole recurrent mixer.
 
-#: steps of up to this many requests take a recurrent mixer as one launch (0: never)
+#: steps of up to this many requests take a recurrent mixer as one launch (0: never): up to 64 with the bits of the separate kernels,
+#: beyond, where ``lowrank_up`` adds its products in another order, with the same rounding
 mixer_step_rows = 128
 
 

@@ -104,7 +104,7 @@ class GatedFFN(FeedForward):
         else:
             # (sizes the fused product does not take: the product's float32 sums, then the activation)
             gu = ops.linear(x, self.w13, torch.float32)
-            a = ops.gated_act(gu, self.dtype, self.slope, self.limit, self.up_offset, interleaved=self.fused)
+            a = ops.gated_act(gu, self.dtype, self.slope, self.limit, self.up_offset)
         return ops.linear(a, self.w2, torch.float32, residual=residual)
 
 

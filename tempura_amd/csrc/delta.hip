@@ -23,13 +23,15 @@ __global__ __launch_bounds__(256) void delta_prep_kernel(DeltaArgs a, long pairs
   if (p < pairs) delta_unit_rows(a, p / a.kv_heads, (int)(p % a.kv_heads), threadIdx.x % TP_WAVE);
 }
 
+// longest > 0: runs of more tokens have been taken by groups.
 template <int PER, int KS>
-__global__ __launch_bounds__(256) void delta_scan_kernel(DeltaArgs a) {
+__global__ __launch_bounds__(256) void delta_scan_kernel(DeltaArgs a, int longest) {
+  if (longest > 0 && a.cu_seqlens[blockIdx.x + 1] - a.cu_seqlens[blockIdx.x] > longest) return;
   delta_chain<PER, KS>(a, blockIdx.x, blockIdx.y, blockIdx.z);
 }
 
 // Defined in delta_chunks.hip: 0 when it took the runs (long ones by groups of tokens, the others by the chain), -1 when none is a long one
-// of its own.
+// of its own; else it took the runs of more tokens than it returns.
 int tp_delta_chunks(const DeltaArgs& chain, int n, int n_req, int max_run, float* scratch, size_t scratch_floats, hipStream_t s);
 
 // max_run: the longest run, 0: not known (scratch of tp_delta_scan_scratch floats lets long runs go by groups of tokens).
@@ -46,10 +48,9 @@ extern "C" int tp_delta_scan(float* qkv, int row_stride, const float* decay, con
   if (n == 0 || n_req == 0) return 0;
   const DeltaArgs a{qkv, row_stride, decay, proj, proj_stride, beta_col0, state, state_stride, state_off, cu_seqlens, state_slots, y, kq,
                     heads, kv_heads, dim, vdim, q_scale, unit_eps};
-  if (tp_delta_chunks(a, n, n_req, max_run, scratch, scratch_floats, s) == 0) {
-    TP_CHECK_LAUNCH("delta_scan (groups)");
-    return 0;
-  }
+  const int longest = tp_delta_chunks(a, n, n_req, max_run, scratch, scratch_floats, s);
+  if (longest >= 0) TP_CHECK_LAUNCH("delta_scan (groups)");
+  if (longest == 0) return 0;
   const long pairs = (long)n * kv_heads;
   TP_REQUIRE((pairs + 3) / 4 < 0x7fffffffL, "delta_scan: too many rows");
   hipLaunchKernelGGL(delta_prep_kernel, dim3((unsigned)((pairs + 3) / 4)), dim3(256), 0, s, a, pairs);
@@ -60,7 +61,7 @@ extern "C" int tp_delta_scan(float* qkv, int row_stride, const float* decay, con
   const int cb = 4 * (TP_WAVE / ks);
   const dim3 grid(n_req, heads, (vdim + cb - 1) / cb);
   TP_REQUIRE(grid.z <= 65535, "delta_scan: too many value columns");
-#define SCAN(P, K) hipLaunchKernelGGL((delta_scan_kernel<P, K>), grid, dim3(256), 0, s, a)
+#define SCAN(P, K) hipLaunchKernelGGL((delta_scan_kernel<P, K>), grid, dim3(256), 0, s, a, longest)
   if (per == 8) {
     if (ks == 1) SCAN(8, 1);
     else if (ks == 2) SCAN(8, 2);

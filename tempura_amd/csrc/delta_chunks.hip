@@ -25,8 +25,8 @@
 // products, a meeting in LDS and the update, each waiting for the one before).  16 heads of 128 x 128, all by single tokens / as here: one
 // run of 128 tokens 37 / 28 us, 2,048 486 / 198; four runs of 451 tokens 162 / 93 (a third of it the first kernel); runs of 82, 327, 573 and
 // 821 tokens 262 / 118; 700 tokens beside 31 single ones 1,327 / 85, 1,800 beside 63 3,412 / 190, beside 247 1,316 / 324; 200 beside ten of
-// 63 105 / 87.  What loses: short runs whose work is most of the step, which the registers of the groups' kernel hold to two blocks a CU
-// (64 tokens beside seven of 63 56 / 63, beside 100 single ones 70 / 100).
+// 63 105 / 87.  What loses is a run of hardly more than 64 tokens beside many that stay with the chain: 64 beside seven of 63 56 / 63, beside
+// 100 single ones 70 / 88.
 #include <math.h>
 
 #include "common.h"
@@ -446,7 +446,7 @@ extern "C" size_t tp_delta_scan_scratch(int n, int n_req, int max_run, int heads
   return (size_t)dc_groups(n, n_req, max_run, heads, dim, vdim, &all) * heads * dc_item_floats(dim);
 }
 
-// Returns 0 when it took the step's runs, -1 when none of them is a long one of its own.
+// Returns 0 when it took the step's runs, -1 when none of them is a long one of its own, DC_SHORT when it took those alone that are longer.
 int tp_delta_chunks(const DeltaArgs& in, int n, int n_req, int max_run, float* scratch, size_t scratch_floats, hipStream_t s) {
   const int heads = in.heads, dim = in.dim, vdim = in.vdim;
   int all;
@@ -461,8 +461,13 @@ int tp_delta_chunks(const DeltaArgs& in, int n, int n_req, int max_run, float* s
   // shortest run that such a step can have is a long one.
   const bool short_runs = (long)n - (long)(n_req - 1) * max_run <= DC_SHORT;
   const int column_block = dim == 128 ? 16 : 32;
-  const long unit_blocks = short_runs ? (long)n * ((in.kv_heads + DC_HEADS - 1) / DC_HEADS) : 0;
-  const long chain_blocks = short_runs ? (long)n_req * heads * ((vdim + column_block - 1) / column_block) : 0;
+  // (Where their blocks are many beside a long run that ends soon, they are left to delta.hip's kernels, which hold five blocks a CU where
+  // the registers of the groups' kernel hold two.  128 x 128, in the same launches / apart: 16 heads, 64 tokens beside 100 single ones 101 /
+  // 88 us, 128 beside 127 123 / 103, 128 beside 31 47 / 52, 700 beside 127 145 / 156; 32 heads, 300 beside 100 213 / 188, 1,800 beside 247
+  // 601 / 705.)
+  const bool apart = short_runs && (long)n_req * heads * ((vdim + column_block - 1) / column_block) > 40L * max_run;
+  const long unit_blocks = short_runs && !apart ? (long)n * ((in.kv_heads + DC_HEADS - 1) / DC_HEADS) : 0;
+  const long chain_blocks = short_runs && !apart ? (long)n_req * heads * ((vdim + column_block - 1) / column_block) : 0;
   const long scan_blocks = ((long)n_req * heads + 7) / 8 * 8 * (vdim / (wide ? 32 : 16));
   if ((long)groups * heads + unit_blocks >= 0x7fffffffL || scan_blocks + chain_blocks >= 0x7fffffffL) return -1;
   DeltaChunkArgs a{in, scratch, n_req, 0, groups, 0};
@@ -482,5 +487,5 @@ int tp_delta_chunks(const DeltaArgs& in, int n, int n_req, int max_run, float* s
     else DC_SCAN(4);
 #undef DC_SCAN
   }
-  return 0;
+  return apart ? DC_SHORT : 0;
 }

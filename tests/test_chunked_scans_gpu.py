@@ -176,11 +176,12 @@ def test_delta_rule_by_groups_rounds_no_more_than_token_by_token(low):
     assert y <= 1.01 and s <= 1.02, (y, s)
 
 
-@pytest.mark.parametrize("H,G,D,Dv", [(4, 2, 64, 16), (2, 2, 128, 128)])
-def test_delta_rule_of_a_run_does_not_depend_on_its_neighbours(H, G, D, Dv):
-    """Decoded tokens and short portions beside long ones: the bits, outputs and states, that every run has alone."""
+@pytest.mark.parametrize("H,G,D,Dv,lens", [(4, 2, 64, 16, [300, 1, 63, 0, 20, 64] + [1] * 70 + [50, 257]), (2, 2, 128, 128, [300, 1, 63, 0, 20, 64, 50, 257]),
+                                           (16, 8, 128, 128, [20, 1, 0, 64, 63] + [1] * 40), (8, 8, 64, 32, [1] * 300 + [64, 63])])
+def test_delta_rule_of_a_run_does_not_depend_on_its_neighbours(H, G, D, Dv, lens):
+    """Decoded tokens and short portions beside long ones, in their launches or (many blocks of short runs) behind them: the bits, outputs
+    and states, that every run has alone."""
     from tempura_amd.kernels import ops
-    lens = [300, 1, 63, 0, 20, 64] + [1] * 70 + [50, 257]
     qkv, decay, proj, state, cu, slots = (t.to(DEV) for t in _delta_inputs(lens, H, G, D, Dv, 31, 0.8))
     together = state.clone()
     y = ops.delta_scan(qkv.clone(), decay, proj, 2, together, 5, cu, slots, len(lens), H, G, D, Dv, D ** -0.5, 1e-6, max_run=max(lens))

@@ -981,11 +981,27 @@ __global__ __launch_bounds__(256) void gemm_pipe_big_kernel(const bf16_t* __rest
 // Here the weights are the traffic and the matrix core has little to do: a block owns 64 x 128 of the
 // result (a wave 32 x 64), three stages of (64 + 128) rows (72 KB: two blocks per CU), K split over
 // blockIdx.y until there are about two blocks for every CU.  Loads, LDS reads and MFMAs interleave as above.
+// NST: stages of LDS, NS with two blocks a CU, more with one.
 // NJ = 2 instead of 4: 64 x 64 blocks (a wave 32 x 32, 48 KB of stages), for products whose N gives too few blocks
 // of 128 columns to put one on every CU without cutting K into short pieces.
 namespace {
 
 constexpr int BM64 = 64;
+
+// waits until at most `n` (uniform, 0..7) of the stages requested last are still on their way, LPW loads each
+template <int LPW_>
+__device__ inline void wait_stages(int n) {
+  switch (n) {
+    case 0: WAIT_VM(0); break;
+    case 1: WAIT_VM(LPW_); break;
+    case 2: WAIT_VM(2 * LPW_); break;
+    case 3: WAIT_VM(3 * LPW_); break;
+    case 4: WAIT_VM(4 * LPW_); break;
+    case 5: WAIT_VM(5 * LPW_); break;
+    case 6: WAIT_VM(6 * LPW_); break;
+    default: WAIT_VM(7 * LPW_); break;
+  }
+}
 
 template <int NJ>
 struct Frags64 {
@@ -1042,12 +1058,12 @@ __device__ inline void half_step64(f32x4_t (&acc)[2][NJ], const Frags64<NJ>& cur
 
 }  // namespace
 
-template <int NJ>
-__global__ __launch_bounds__(256, 2) void gemm_pipe64_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w,
+template <int NJ, int NST>
+__global__ __launch_bounds__(256, NST == NS ? 2 : 1) void gemm_pipe64_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w,
                                                              void* __restrict__ out, float* __restrict__ partial,
                                                              int mode, int M, int N, int K, int wt, GateAct ga) {
   constexpr int BNT = 32 * NJ, STAGE = (BM64 + BNT) * ROWB, LPWT = 2 + NJ;
-  __shared__ __attribute__((aligned(1024))) unsigned char stages[NS * STAGE];
+  __shared__ __attribute__((aligned(1024))) unsigned char stages[NST * STAGE];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave >> 1, wn = wave & 1;
   const int MB = (M + BM64 - 1) / BM64;
@@ -1098,12 +1114,12 @@ __global__ __launch_bounds__(256, 2) void gemm_pipe64_kernel(const bf16_t* __res
     }
   };
 #pragma unroll
-  for (int p = 0; p < NS; ++p)
+  for (int p = 0; p < NST; ++p)
     if (p < KT) issue_stage64(stages + p * STAGE, xk + p * BK * 2, wk + p * wkstep);
-  xk += NS * BK * 2;
-  wk += NS * wkstep;
+  xk += NST * BK * 2;
+  wk += NST * wkstep;
   Frags64<NJ> fa, fb;
-  if (KT > 2) WAIT_VM(2 * LPWT); else WAIT_VM(0);
+  wait_stages<LPWT>(min(KT, NST) - 1);
   __builtin_amdgcn_s_barrier();
   auto read_all = [&](Frags64<NJ>& f, unsigned aaddr, unsigned baddr) {
     read_one<0, NJ>(f, aaddr, baddr); read_one<1, NJ>(f, aaddr, baddr); read_one<2, NJ>(f, aaddr, baddr);
@@ -1115,12 +1131,12 @@ __global__ __launch_bounds__(256, 2) void gemm_pipe64_kernel(const bf16_t* __res
   read_all(fa, lds0 + arow + off0, lds0 + brow + boff0);
   wait_frags<NJ>(fa);
   int st = 0, kt = 0;
-  for (; kt + NS < KT; ++kt) {
-    const int sn = st + 1 == NS ? 0 : st + 1;
+  for (; kt + NST < KT; ++kt) {
+    const int sn = st + 1 == NST ? 0 : st + 1;
     const unsigned cur = lds0 + st * STAGE, nxt = lds0 + sn * STAGE;
     half_step64<true, false, NJ>(acc, fa, fb, cur + arow + off1, cur + brow + boff1, nullptr, nullptr, nullptr, voff, wave);
     wait_frags<NJ>(fb);
-    WAIT_VM(LPWT);
+    WAIT_VM((NST - 2) * LPWT);
     __builtin_amdgcn_s_barrier();
     half_step64<true, true, NJ>(acc, fb, fa, nxt + arow + off0, nxt + brow + boff0, stages + st * STAGE, xk, wk, voff, wave);
     wait_frags<NJ>(fa);
@@ -1129,11 +1145,11 @@ __global__ __launch_bounds__(256, 2) void gemm_pipe64_kernel(const bf16_t* __res
     st = sn;
   }
   for (; kt + 1 < KT; ++kt) {
-    const int sn = st + 1 == NS ? 0 : st + 1;
+    const int sn = st + 1 == NST ? 0 : st + 1;
     const unsigned cur = lds0 + st * STAGE, nxt = lds0 + sn * STAGE;
     half_step64<true, false, NJ>(acc, fa, fb, cur + arow + off1, cur + brow + boff1, nullptr, nullptr, nullptr, voff, wave);
     wait_frags<NJ>(fb);
-    WAIT_VM(0);
+    wait_stages<LPWT>(KT - kt - 2);
     __builtin_amdgcn_s_barrier();
     half_step64<true, false, NJ>(acc, fb, fa, nxt + arow + off0, nxt + brow + boff0, nullptr, nullptr, nullptr, voff, wave);
     wait_frags<NJ>(fa);
@@ -1645,12 +1661,19 @@ int tp_linear_pipe64(const bf16_t* x, const bf16_t* w, int w_tiled, void* out, i
     splits = splits_narrow;
   }
   const bool leave = defer && splits > 1 && splits_out != nullptr && mode != OUT_SWIGLU && mode != OUT_SPLIT;
-  if (narrow)
-    hipLaunchKernelGGL(gemm_pipe64_kernel<2>, dim3((unsigned)tiles, splits), dim3(256), 0, s, x, w, out,
-                       splits > 1 ? scratch : nullptr, mode, M, N, K, w_tiled, gate);
-  else
-    hipLaunchKernelGGL(gemm_pipe64_kernel<4>, dim3((unsigned)tiles, splits), dim3(256), 0, s, x, w, out,
-                       splits > 1 ? scratch : nullptr, mode, M, N, K, w_tiled, gate);
+  // one block of 64 columns a CU that walks all of K: eight stages of 16 KB instead of three (64 KB of weights on their way
+  // instead of 24).  16,384 x 3,072 gated, 24 / 48 / 64 rows 23.1 / 22.9 / 23.4 -> 19.6 / 20.4 / 21.5 us; 12,288 x 4,096 29.6 -> 22.5
+  // (24 rows) and 30.1 -> 27.4 (64); 9,216 x 2,048 13.1 -> 11.1 and 13.2 -> 12.5.  Under 32 steps of K it gains nothing (1,024 of K:
+  // 9.2 / 9.7 at 64 rows), nor do blocks that walk a part of K, nor those of 128 columns (28,672 x 4,096 with six stages of 24 KB
+  // 42.1 -> 43.1).
+  const bool deep = narrow && splits == 1 && tiles <= 256 && KT >= 32;
+#define PIPE64(NJ_, NST_)                                                                                           \
+  hipLaunchKernelGGL((gemm_pipe64_kernel<NJ_, NST_>), dim3((unsigned)tiles, splits), dim3(256), 0, s, x, w, out,     \
+                     splits > 1 ? scratch : nullptr, mode, M, N, K, w_tiled, gate)
+  if (deep) PIPE64(2, 8);
+  else if (narrow) PIPE64(2, NS);
+  else PIPE64(4, NS);
+#undef PIPE64
   if (leave) {
     *splits_out = splits;
   } else if (splits > 1) {

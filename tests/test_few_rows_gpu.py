@@ -279,3 +279,21 @@ def test_attention_gates_what_it_combines(heads, kv, d, vd, ctx, how):
     ops.sigmoid_gate(ops.paged_attention(*args, sink=sink), rows, 5, 0.75, want, 4, per)
     assert ops.paged_attention(*args, sink=sink, into=(rows, 5, 0.75, got, 4, per)) is None
     assert torch.isfinite(got.float()).all() and torch.equal(got, want)
+
+
+@pytest.mark.parametrize("m", [17, 40, 64])
+@pytest.mark.parametrize("n,k", [(8256, 2048), (16384, 2112), (9216, 2624)])
+def test_products_of_one_deep_block_a_cu(m, n, k):
+    """17 to 64 rows onto 129 to 256 blocks of 64 columns, 32 steps of K and more: eight stages of LDS, the last of them
+    drained one by one.  Float32 sums of k products against float32 sums in another order: an error of sqrt(k) roundings."""
+    from tempura_amd.kernels import ops
+    g = torch.Generator().manual_seed(m + n + k)
+    x = torch.randn(m, k, generator=g).to(DEV).bfloat16()
+    w = torch.randn(n, k, generator=g).to(DEV).bfloat16()
+    want = x.float() @ w.float().t()
+    for weight in (w, ops.tile_weight(w)):
+        got = ops.linear(x, weight, torch.float32)
+        assert float((got - want).norm()) <= 4 * k ** 0.5 * 2.0 ** -24 * float(want.norm())
+        h = torch.ones(m, n, device=DEV)
+        ops.linear(x, weight, torch.float32, residual=h)
+        assert torch.equal(h, got + 1.0)

@@ -117,7 +117,8 @@ int tp_paged_attention_fast(const void* q, const void* k_cache, const void* v_ca
                             int max_q_len, int num_single, int num_splits, float* scratch, const int* token_req,
                             int portion_splits, int portion_min_steps, float* portion_scratch, const float* dist_bias,
                             int bias_len, int keep_first, const float* sink, int value_dim, int chunk, float softcap,
-                            int keep_parts, hipStream_t s);
+                            int gated, const float* gate, int gate_stride, int gate_col0, int gate_per, float gate_scale, int out_stride,
+                            int out_col0, hipStream_t s);
 
 // Defined in attention_f32.hip; -1 for shapes that are not its own.
 int tp_paged_attention_f32(const float* q, const float* k_cache, const float* v_cache, const int* block_tables, int table_width,
@@ -133,7 +134,8 @@ extern "C" int tp_paged_attention(const void* q, int dt, const void* k_cache, co
                                   int window, int max_q_len, int max_ctx, int allow_fast, int num_single,
                                   int num_splits, float* scratch, int portion_splits, int portion_min_steps,
                                   float* portion_scratch, const float* dist_bias, int bias_len, int value_dim,
-                                  int keep_first, const float* sink, int chunk, float softcap, hipStream_t s) {
+                                  int keep_first, const float* sink, int chunk, float softcap, const float* gate, int gate_stride,
+                                  int gate_col0, int gate_per, float gate_scale, int out_stride, int out_col0, hipStream_t s) {
   // value_dim: the size of a value head (0: head_dim): v_cache is [page, kv_head, value_dim, page_size] and out
   // [n, heads * value_dim]; the matrix-core kernels take equal sizes and a few pairs with wider keys.
   if (value_dim <= 0) value_dim = head_dim;
@@ -141,8 +143,9 @@ extern "C" int tp_paged_attention(const void* q, int dt, const void* k_cache, co
   // which, with more than one split, needs `scratch` of n_req * n_heads * num_splits * (head_dim + 2)
   // floats).  portion_splits > 1: the keys of every longer request are split over that many blocks,
   // which needs `portion_scratch` of n_tokens * n_heads * portion_splits * (head_dim + 4) floats.
-  // allow_fast 2 (single tokens only, more than one split): their partial results stay in `scratch` for
-  // tp_attention_combine_gate and `out` is not written.
+  // allow_fast 2 (single tokens only, sizes that the matrix-core kernels take): `out` is rows of out_stride columns, and the heads'
+  // outputs go to its columns from out_col0 on, rounded to bfloat16, times sigmoid(gate[:, gate_col0 + column / gate_per]) (gate
+  // float32 rows of gate_stride; nullptr: none) and gate_scale.
   TP_REQUIRE(n_tokens >= 0 && n_req >= 0 && n_heads > 0 && n_kv > 0 && head_dim > 0 && page_size > 0,
              "paged_attention: bad sizes");
   TP_REQUIRE(n_heads % n_kv == 0, "paged_attention: %d heads is not a multiple of %d kv heads", n_heads, n_kv);
@@ -158,6 +161,11 @@ extern "C" int tp_paged_attention(const void* q, int dt, const void* k_cache, co
   }
   if (window == 0) keep_first = 0;   // (without a window every key is seen anyway)
   TP_REQUIRE(n_heads <= 65535, "paged_attention: too many heads");
+  if (allow_fast == 2) {
+    const int width = n_heads * value_dim;
+    TP_REQUIRE(out_col0 >= 0 && out_stride >= out_col0 + width && gate_per >= 1 && width % gate_per == 0, "paged_attention: bad output rows");
+    TP_REQUIRE(gate == nullptr || (gate_col0 >= 0 && gate_stride >= gate_col0 + width / gate_per), "paged_attention: gate rows too short");
+  }
   if (n_tokens == 0) return 0;
   TP_REQUIRE(dist_bias == nullptr || bias_len > 0, "paged_attention: empty distance bias table");
   if (dt == TP_BF16 && allow_fast) {
@@ -165,10 +173,10 @@ extern "C" int tp_paged_attention(const void* q, int dt, const void* k_cache, co
                                            context_lens, out, n_tokens, n_req, n_heads, n_kv, head_dim,
                                            page_size, scale, window, max_q_len, num_single, num_splits, scratch, token_req,
                                            portion_splits, portion_min_steps, portion_scratch, dist_bias, bias_len, keep_first, sink, value_dim, chunk,
-                                           softcap, allow_fast == 2, s);
+                                           softcap, allow_fast == 2, gate, gate_stride, gate_col0, gate_per, gate_scale, out_stride, out_col0, s);
     if (rc >= 0) return rc;
   }
-  TP_REQUIRE(allow_fast != 2, "paged_attention: no parts to keep for these sizes");
+  TP_REQUIRE(allow_fast != 2, "paged_attention: no gate over the heads' outputs for these sizes");
   if (dt == TP_F32 && allow_fast) {
     const int rc = tp_paged_attention_f32((const float*)q, (const float*)k_cache, (const float*)v_cache, block_tables, table_width,
                                           cu_seqlens, context_lens, (float*)out, n_tokens, n_req, n_heads, n_kv, head_dim, value_dim,

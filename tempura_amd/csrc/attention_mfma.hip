@@ -70,6 +70,24 @@ __device__ inline float quad_rows_max(float x) {
   return max_raw(x, y);
 }
 
+// A sublayer's gate over the heads' outputs, by whichever kernel writes a single token's row, in the order of the gate's own kernel:
+// the row rounded to bfloat16, times sigmoid(gate column) (per columns in a row share one), times a scale, into columns of a wider
+// row (the same bits; a launch of 2.5 to 4 us behind a chain of such: Bomotar's decode step with four of them 387 -> 377 us,
+// Tokatar's with two 282 -> 278).
+struct CombineGate {
+  const float* rows;      // [n, stride] float32, or nullptr: the scale alone
+  int stride, col0, per, out_stride, out_col0;
+  float scale;
+};
+__device__ inline void store_gated_head(const CombineGate& gate, bf16_t* out, int row, int col, float v, float raw) {
+  v = bf16_to_float(float_to_bf16(v));
+  if (gate.rows != nullptr) v *= 1.0f / (1.0f + expf(-raw));
+  out[(size_t)row * gate.out_stride + gate.out_col0 + col] = float_to_bf16(v * gate.scale);
+}
+__device__ inline float gate_of(const CombineGate& gate, int row, int col) {
+  return gate.rows != nullptr ? gate.rows[(size_t)row * gate.stride + gate.col0 + col / gate.per] : 0.f;
+}
+
 struct AttnArgs {
   const bf16_t* q;
   const bf16_t* k_cache;
@@ -90,7 +108,9 @@ struct AttnArgs {
   int portion_min_steps;   // a query block is split into at most (its steps / this) parts
   float* portion_scratch;
   const int* token_req;
-  bool keep_parts;  // the caller combines the single tokens' splits itself (tp_attention_combine_gate)
+  bool all_single;  // (every request brings one token: request r's row is row r)
+  bool gated;       // (every request brings one token: the rows go through `gate`)
+  CombineGate gate;
   // a bias by distance, added to the scaled score (the scale does not multiply it): dist_bias [heads, bias_len]
   // float32, entry min(query position - key position, bias_len - 1); nullptr: none
   const float* dist_bias;
@@ -1228,87 +1248,54 @@ __global__ __launch_bounds__(256, 1) void attn_prefill_latent_kernel(AttnArgs a,
 }
 
 // ---- decode -----------------------------------------------------------------------------
-// grid: (kv_heads * ceil(group / 16), requests, splits); block: 4 waves.  Handles requests
-// with exactly one new token.  Scratch per (request, head, split): DV floats of O, then max, sum.
-// (The kv heads run fastest: consecutive blocks go to the eight XCDs in turn, so the heads of every request are
-// spread over all of them and each XCD reads about the same number of bytes however the contexts differ.  With
-// the requests fastest, 60 requests of 128 to 2,304 keys took 77 us where 60 of their mean took 54: the XCD
-// with the longest requests set the time, and more splits changed nothing, since the splits of a (request, head)
-// pair fell to the same XCD.)
-template <int D, int DV, int MODE = MODE_PLAIN>
-__global__ __launch_bounds__(256) void attn_decode_kernel(AttnArgs a) {
-  __shared__ float red_o[4][DV][16];
-  __shared__ float red_m[4][16], red_l[4][16];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+// The steps of 32 keys that a single token at position ctx - 1 sees: those of the kept first keys that lie before the window's first
+// step, then the window's, which begin at key `first`.
+__device__ inline int decode_steps(const AttnArgs& a, int ctx, int& first, int& kept_steps) {
+  first = max(0, attn_first_key(a, ctx - 1)) & ~31;
+  kept_steps = min(first, (a.keep_first + 31) & ~31) / 32;
+  return kept_steps + (ctx - first + 31) / 32;
+}
+// The waves' sums of a block, added in their order through LDS (red: WAVES * (DV * 17 + 32) floats; 17: rows of 16 columns a
+// bank apart): the answer where the keys are not split, else the split's partial result.  h0: the first head, ncols: how many.
+template <int DV, int WAVES>
+__device__ inline void decode_merge(const AttnArgs& a, float* red, int wave, int lane, float m, float l, const f32x4_t (&o)[DV / 16],
+                                    int r, int q_start, int h0, int ncols) {
   const int g = lane >> 4, c = lane & 15;
-  const int r = blockIdx.y;
-  const int q_start = a.cu_seqlens[r];
-  if (a.cu_seqlens[r + 1] - q_start != 1) return;
-  const int group = a.n_heads / a.n_kv;
-  const int hblocks = (group + 15) / 16;
-  const int kvh = blockIdx.x / hblocks;
-  const int h0 = (blockIdx.x % hblocks) * 16;            // first head (within the group) of this block
-  const int ncols = min(16, group - h0);
-  const int head = kvh * group + h0 + min(c, ncols - 1);  // spare columns repeat the last head
-  const int ctx = a.context_lens[r];
-  const int pos = ctx - 1;
-  const int* table = a.block_tables + (size_t)r * a.table_width;
-
-  bf16x8_t qf[1][D / 32];
-  int qpos[1] = {pos};
-  float m[1] = {-INFINITY}, l[1] = {0.f};
-  f32x4_t o[1][DV / 16];
-  const bf16_t* qr = a.q + ((size_t)q_start * a.n_heads + head) * D + g * 8;
-#pragma unroll
-  for (int dk = 0; dk < D / 32; ++dk) qf[0][dk] = frag_of(*(const u32x4_t*)(qr + dk * 32));
-#pragma unroll
-  for (int dt = 0; dt < DV / 16; ++dt) o[0][dt] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
-
-  const int first = max(0, attn_first_key(a, pos)) & ~31;
-  // steps of 32 keys: those of the kept first keys that lie before the window's first step, then the window's
-  const int kept_steps = min(first, (a.keep_first + 31) & ~31) / 32;
-  const int steps = kept_steps + (ctx - first + 31) / 32;
-  const int per_split = (steps + a.num_splits - 1) / a.num_splits;
-  const int s_begin = blockIdx.z * per_split, s_end = min(steps, s_begin + per_split);
-  // (Fetching the next step's fragments while this one is computed was measured: the doubled
-  // fragment registers halve the occupancy and the kernel gets slower, not faster.)
-  const float* bias_row = MODE == MODE_BIAS ? a.dist_bias + (size_t)head * a.bias_len : nullptr;   // (a column is a head)
-  for (int s = s_begin + wave; s < s_end; s += 4)
-    attn_step<D, DV, 1, MODE>(a, table, kvh, ctx, s < kept_steps ? s * 32 : first + (s - kept_steps) * 32, qf, qpos, m, l, o, bias_row);
-
-  // merge the four waves (fixed order), then write this split's partial
-  float lt = l[0];
-  lt += __shfl_xor(lt, 16, 64);
-  lt += __shfl_xor(lt, 32, 64);
+  float* stat = red + WAVES * DV * 17;
+  l += __shfl_xor(l, 16, 64);
+  l += __shfl_xor(l, 32, 64);
   if (g == 0) {
-    red_m[wave][c] = m[0];
-    red_l[wave][c] = lt;
+    stat[wave * 32 + c] = m;
+    stat[wave * 32 + 16 + c] = l;
   }
 #pragma unroll
   for (int dt = 0; dt < DV / 16; ++dt)
 #pragma unroll
-    for (int rr = 0; rr < 4; ++rr) red_o[wave][dt * 16 + 4 * g + rr][c] = o[0][dt][rr];
+    for (int rr = 0; rr < 4; ++rr) red[(wave * DV + dt * 16 + 4 * g + rr) * 17 + c] = o[dt][rr];
   __syncthreads();
-  for (int e = threadIdx.x; e < DV * 16; e += 256) {
-    const int d = e / 16, col = e % 16;
-    if (col >= ncols) continue;
-    float mg = red_m[0][col];
+  for (int e = threadIdx.x; e < DV * ncols; e += WAVES * 64) {
+    const int d = e % DV, col = e / DV;
+    float mg = stat[col];
 #pragma unroll
-    for (int w = 1; w < 4; ++w) mg = fmaxf(mg, red_m[w][col]);
+    for (int w = 1; w < WAVES; ++w) mg = fmaxf(mg, stat[w * 32 + col]);
     const float mu = (mg == -INFINITY) ? 0.f : mg;
     float acc = 0.f, lsum = 0.f;
 #pragma unroll
-    for (int w = 0; w < 4; ++w) {
-      const float f = __builtin_amdgcn_exp2f(red_m[w][col] - mu);
-      acc += f * red_o[w][d][col];
-      lsum += f * red_l[w][col];
+    for (int w = 0; w < WAVES; ++w) {
+      const float f = __builtin_amdgcn_exp2f(stat[w * 32 + col] - mu);
+      acc += f * red[(w * DV + d) * 17 + col];
+      lsum += f * stat[w * 32 + 16 + col];
     }
+    const int hd = h0 + col;
     if (a.num_splits == 1) {  // nothing to combine: this is the answer
-      lsum += sink_term(a.sink, kvh * group + h0 + col, mu);
-      a.out[((size_t)q_start * a.n_heads + (kvh * group + h0 + col)) * DV + d] = float_to_bf16(acc / lsum);
+      lsum += sink_term(a.sink, hd, mu);
+      if (a.gated)
+        store_gated_head(a.gate, a.out, q_start, hd * DV + d, acc / lsum, gate_of(a.gate, q_start, hd * DV + d));
+      else
+        a.out[((size_t)q_start * a.n_heads + hd) * DV + d] = float_to_bf16(acc / lsum);
       continue;
     }
-    float* part = a.scratch + (((size_t)r * a.n_heads + (kvh * group + h0 + col)) * a.num_splits + blockIdx.z) * (DV + 2);
+    float* part = a.scratch + (((size_t)r * a.n_heads + hd) * a.num_splits + blockIdx.z) * (DV + 2);
     part[d] = acc;
     if (d == 0) {
       part[DV] = mg;
@@ -1317,20 +1304,229 @@ __global__ __launch_bounds__(256) void attn_decode_kernel(AttnArgs a) {
   }
 }
 
+// grid: (kv_heads * ceil(group / 16), requests, splits); block: 4 waves.  Handles requests
+// with exactly one new token.  Scratch per (request, head, split): DV floats of O, then max, sum.
+// (The kv heads run fastest: consecutive blocks go to the eight XCDs in turn, so the heads of every request are
+// spread over all of them and each XCD reads about the same number of bytes however the contexts differ.  With
+// the requests fastest, 60 requests of 128 to 2,304 keys took 77 us where 60 of their mean took 54: the XCD
+// with the longest requests set the time, and more splits changed nothing, since the splits of a (request, head)
+// pair fell to the same XCD.)
+// This kernel loads keys and values into registers, a step at a time: the sizes and pages that attn_decode_lds_kernel does not take.
+template <int D, int DV, int MODE = MODE_PLAIN>
+__global__ __launch_bounds__(256) void attn_decode_kernel(AttnArgs a) {
+  __shared__ float red[4 * (DV * 17 + 32)];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int g = lane >> 4, c = lane & 15;
+  const int group = a.n_heads / a.n_kv;
+  const int hblocks = (group + 15) / 16;
+  const int kvh = blockIdx.x / hblocks;
+  const int h0 = (blockIdx.x % hblocks) * 16;            // first head (within the group) of this block
+  const int ncols = min(16, group - h0);
+  const int head = kvh * group + h0 + min(c, ncols - 1);  // spare columns repeat the last head
+  const float* bias_row = MODE == MODE_BIAS ? a.dist_bias + (size_t)head * a.bias_len : nullptr;   // (a column is a head)
+  const int r = blockIdx.y, q_start = a.all_single ? r : a.cu_seqlens[r];
+  if (!a.all_single && a.cu_seqlens[r + 1] - q_start != 1) return;
+  const int ctx = a.context_lens[r];
+  const int* table = a.block_tables + (size_t)r * a.table_width;
+
+  bf16x8_t qf[1][D / 32];
+  int qpos[1] = {ctx - 1};
+  float m[1] = {-INFINITY}, l[1] = {0.f};
+  f32x4_t o[1][DV / 16];
+  const bf16_t* qr = a.q + ((size_t)q_start * a.n_heads + head) * D + g * 8;
+#pragma unroll
+  for (int dk = 0; dk < D / 32; ++dk) qf[0][dk] = frag_of(*(const u32x4_t*)(qr + dk * 32));
+#pragma unroll
+  for (int dt = 0; dt < DV / 16; ++dt) o[0][dt] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+
+  int first, kept_steps;
+  const int steps = decode_steps(a, ctx, first, kept_steps);
+  const int per_split = (steps + a.num_splits - 1) / a.num_splits;
+  const int s_begin = blockIdx.z * per_split, s_end = min(steps, s_begin + per_split);
+  // (Fetching the next step's fragments while this one is computed was measured: the doubled
+  // fragment registers halve the occupancy and the kernel gets slower, not faster.)
+  for (int s = s_begin + wave; s < s_end; s += 4)
+    attn_step<D, DV, 1, MODE>(a, table, kvh, ctx, s < kept_steps ? s * 32 : first + (s - kept_steps) * 32, qf, qpos, m, l, o, bias_row);
+  decode_merge<DV, 4>(a, red, wave, lane, m[0], l[0], o[0], r, q_start, kvh * group + h0, ncols);
+}
+
+// The same with keys and values on their way to LDS instead of registers (the sizes and pages of attn_prefill_lds_kernel, whose
+// layout of a step in LDS this is).  Every wave has a ring of NB steps of its own, filled by direct global-to-LDS loads of whole
+// kilobytes (a key fragment loaded into its registers is 64-byte pieces of sixteen rows, which the address path of a CU takes at
+// half the rate) and emptied without a barrier: a step's keys go on their way NB steps ahead, as soon as the fragments of the keys
+// they replace are in registers, its values likewise, its pages before that.
+// (a wait that stays in its place among the assembly that reads LDS behind it)
+#define ATTN_WAIT_VM_ORDERED(n) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(n) : "memory")
+template <int D, int DV, int MODE, int WAVES, int NB>
+__global__ __launch_bounds__(WAVES * 64) void attn_decode_lds_kernel(AttnArgs a) {
+  constexpr int C = D / 8;             // 16-byte chunks per key row
+  constexpr int SH = C == 16 ? 0 : (C == 8 || C == 24 ? 1 : 2);
+  constexpr int KI = D / 16, VI = DV / 16, STAGE = (KI + VI) * 1024;
+  static_assert((D == 32 || D == 64 || D == 128 || D == 192) && VI <= 8, "sizes");
+  static_assert(NB * STAGE >= (DV * 17 + 32) * 4, "room for the merge");
+  static_assert((NB == 1 || NB == 2) && 2 * VI + KI <= 63 && 2 * KI + VI <= 63, "the waits below");
+  __shared__ __attribute__((aligned(1024))) unsigned char stages[WAVES * NB * STAGE];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int g = lane >> 4, c = lane & 15;
+  const int group = a.n_heads / a.n_kv;
+  const int hblocks = (group + 15) / 16;
+  const int kvh = blockIdx.x / hblocks;
+  const int h0 = (blockIdx.x % hblocks) * 16;
+  const int ncols = min(16, group - h0);
+  const int head = kvh * group + h0 + min(c, ncols - 1);
+  static_assert(MODE != MODE_BIAS, "a table read inside the loop would wait for the copies into LDS");
+  const int r = blockIdx.y, q_start = a.all_single ? r : a.cu_seqlens[r];
+  if (!a.all_single && a.cu_seqlens[r + 1] - q_start != 1) return;
+  const int ctx = a.context_lens[r];
+  u32x4_t qv[D / 32];
+  const bf16_t* qr = a.q + ((size_t)q_start * a.n_heads + head) * D + g * 8;
+#pragma unroll
+  for (int dk = 0; dk < D / 32; ++dk) qv[dk] = *(const u32x4_t*)(qr + dk * 32);
+  // this lane's offset in each load of a step, and its addresses in LDS (see attn_prefill_lds_kernel)
+  const int ps = a.page_size, psh = a.page_shift, pmask = ps - 1;
+  unsigned koff[KI];
+#pragma unroll
+  for (int t = 0; t < KI; ++t) {
+    const int row = (64 * t + lane) / C, pc = (64 * t + lane) % C;
+    const int f = (((row >> 3) << 2) | (row & 3)) >> SH;
+    koff[t] = (unsigned)((row - 8 * (((64 * t) / C) >> 3)) * D * 2 + ((pc - f + C) % C) * 16);
+  }
+  const unsigned voff = (unsigned)(((lane & 31) * ps + 8 * (lane >> 5)) * 2);
+  const unsigned page_bytes = (unsigned)(a.n_kv * D * ps * 2), vpage_bytes = (unsigned)(a.n_kv * DV * ps * 2);
+  const unsigned char* kbase = (const unsigned char*)a.k_cache + (size_t)kvh * ps * D * 2;
+  const unsigned char* vbase = (const unsigned char*)a.v_cache + (size_t)kvh * DV * ps * 2;
+  unsigned char* ring = stages + wave * (NB * STAGE);
+  const unsigned lds0 = (unsigned)(size_t)(__attribute__((address_space(3))) const unsigned char*)ring;
+  unsigned kaddr[2][D / 32];
+#pragma unroll
+  for (int t2 = 0; t2 < 2; ++t2) {
+    const int row = 8 * (c >> 2) + 4 * t2 + (c & 3);
+#pragma unroll
+    for (int dk = 0; dk < D / 32; ++dk) kaddr[t2][dk] = (row * C + (dk * 4 + g + (c >> SH)) % C) * 16;
+  }
+  const unsigned vaddr = KI * 1024 + (g >> 1) * 1024 + (g & 1) * 512 + c * 16;
+
+  const int* table = a.block_tables + (size_t)r * a.table_width;
+  // (the block table through the constant address space: uniform loads from it are scalar loads)
+  const __attribute__((address_space(4))) int* ctab = (const __attribute__((address_space(4))) int*)(uintptr_t)table;
+  int first, kept_steps;
+  const int steps = decode_steps(a, ctx, first, kept_steps);
+  const int per_split = (steps + a.num_splits - 1) / a.num_splits;
+  const int s_begin = blockIdx.z * per_split, s_end = min(steps, s_begin + per_split);
+  const int n = max(0, (s_end - s_begin - wave + WAVES - 1) / WAVES);      // this wave's steps
+  auto key0 = [&](int i) {
+    const int s = s_begin + wave + i * WAVES;
+    return s < kept_steps ? s * 32 : first + (s - kept_steps) * 32;
+  };
+  // the pages of the two halves of a step's keys (the second clamped to the last key that exists).  What a page holds behind the
+  // last key is fetched with it: its scores are masked, its values cleared when they are read.
+  int pp0 = 0, pp1 = 0;
+  auto pages_of = [&](int i) {
+    const int j0 = key0(i);
+    pp0 = ctab[j0 >> psh];
+    pp1 = ctab[min(j0 + 16, (ctx - 1) & ~7) >> psh];
+  };
+  auto issue_keys = [&](int i, int st) __attribute__((always_inline)) {
+    const int j0 = key0(i);
+#pragma unroll
+    for (int t = 0; t < KI; ++t) {
+      const int gr = ((64 * t) / C) >> 3;
+      const unsigned char* src = kbase + (size_t)(unsigned)(gr >= 2 ? pp1 : pp0) * page_bytes + (unsigned)(((j0 + 8 * gr) & pmask) * D * 2);
+      __builtin_amdgcn_global_load_lds(GPTR(src + koff[t]), LPTR(ring + st * STAGE + t * 1024), 16, 0, 2);
+    }
+  };
+  auto issue_values = [&](int i, int st) __attribute__((always_inline)) {
+    const int j0 = key0(i);
+#pragma unroll
+    for (int t = 0; t < VI; ++t) {
+      const unsigned char* src = vbase + (size_t)(unsigned)((t & 1) ? pp1 : pp0) * vpage_bytes +
+                                 (unsigned)(((j0 + ((t & 1) ? 16 : 0)) & pmask) * 2 + 32 * (t >> 1) * ps * 2);
+      __builtin_amdgcn_global_load_lds(GPTR(src + voff), LPTR(ring + st * STAGE + (KI + t) * 1024), 16, 0, 2);
+    }
+  };
+#pragma unroll
+  for (int i = 0; i < NB; ++i)
+    if (i < n) {
+      pages_of(i);
+      issue_keys(i, i);
+      issue_values(i, i);
+    }
+  if (NB < n) pages_of(NB);
+  bf16x8_t qf[1][D / 32];
+  int qpos[1] = {ctx - 1};
+  float m[1] = {-INFINITY}, l[1] = {0.f};
+  f32x4_t o[1][DV / 16];
+#pragma unroll
+  for (int dk = 0; dk < D / 32; ++dk) qf[0][dk] = frag_of(qv[dk]);
+#pragma unroll
+  for (int dt = 0; dt < DV / 16; ++dt) o[0][dt] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+
+  int st = 0;
+  for (int i = 0; i < n; ++i) {
+    const unsigned base = lds0 + st * STAGE;
+    const bool behind = NB > 1 && i + 1 < n;      // (a whole step on its way behind this one)
+    const bool more = i + NB < n;
+    if (behind) ATTN_WAIT_VM_ORDERED(VI + KI + VI);
+    else ATTN_WAIT_VM_ORDERED(VI);
+    u32x4_t kk[2][D / 32];
+#pragma unroll
+    for (int t2 = 0; t2 < 2; ++t2)
+#pragma unroll
+      for (int dk = 0; dk < D / 32; ++dk) kk[t2][dk] = attn_lds_read<0>(base + kaddr[t2][dk]);
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    bf16x8_t kf[2][D / 32];
+#pragma unroll
+    for (int t2 = 0; t2 < 2; ++t2)
+#pragma unroll
+      for (int dk = 0; dk < D / 32; ++dk) {
+        asm volatile("" : "+v"(kk[t2][dk]));
+        kf[t2][dk] = frag_of(kk[t2][dk]);
+      }
+    if (more) issue_keys(i + NB, st);
+    f32x4_t sc[1][2];
+    attn_scores<D, 1>(kf, qf, sc);
+    bf16x8_t pf[1];
+    float alpha[1];
+    bool moved[1];
+    const int j0 = key0(i);
+    attn_softmax<1, true, MODE>(a, j0, sc, qpos, m, l, pf, alpha, moved);
+    if (more && behind) ATTN_WAIT_VM_ORDERED(KI + KI + VI);
+    else if (more) ATTN_WAIT_VM_ORDERED(KI);
+    else if (behind) ATTN_WAIT_VM_ORDERED(KI + VI);
+    else ATTN_WAIT_VM_ORDERED(0);
+    u32x4_t vv[DV / 16];
+#define ATTN_RV(dt) if constexpr (dt < DV / 16) vv[dt] = attn_lds_read<(dt >> 1) * 2048 + (dt & 1) * 256>(base + vaddr)
+    ATTN_RV(0); ATTN_RV(1); ATTN_RV(2); ATTN_RV(3); ATTN_RV(4); ATTN_RV(5); ATTN_RV(6); ATTN_RV(7);
+#undef ATTN_RV
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    bf16x8_t vf[DV / 16];
+#pragma unroll
+    for (int dt = 0; dt < DV / 16; ++dt) {
+      asm volatile("" : "+v"(vv[dt]));
+      vf[dt] = frag_of(vv[dt]);
+    }
+    if (more) {
+      issue_values(i + NB, st);
+      if (i + NB + 1 < n) pages_of(i + NB + 1);
+    }
+    if (j0 + 32 > ctx) {     // the step that holds the last key: places past it are cleared (see attn_existing_keys)
+      const u32x4_t keep = attn_existing_keys(ctx - (j0 + 8 * g));
+#pragma unroll
+      for (int dt = 0; dt < DV / 16; ++dt) vf[dt] = frag_of(__builtin_bit_cast(u32x4_t, vf[dt]) & keep);
+    }
+    attn_pv<DV, 1>(vf, pf, alpha, moved, o);
+    st = st + 1 == NB ? 0 : st + 1;
+  }
+  __syncthreads();     // (every wave's ring is empty)
+  decode_merge<DV, WAVES>(a, (float*)stages, wave, lane, m[0], l[0], o[0], r, q_start, kvh * group + h0, ncols);
+}
+
 // out[token, head, :] = sum_s 2^(m_s - m) O_s / sum_s 2^(m_s - m) l_s, splits in ascending order.
 // grid: (requests, heads); block: one wave.  Lane s holds split s's statistics (num_splits <= 64).
 // (Combining inside the decode kernel by whichever block finishes last was tried and is far
 // slower: the L2 caches of the eight XCDs are not coherent with each other, so partial results
 // would have to travel through memory with device-scope fences.)
-// GATED: a sublayer's gate over the heads' outputs in the same launch, in the order of its own kernel: the row rounded to bfloat16,
-// times sigmoid(gate column) (per columns in a row share one), times a scale, into columns of a wider row (the same bits; a launch
-// of 2.5 to 4 us behind a chain of such: Bomotar's decode step with four
-// of them 387 -> 377 us, Tokatar's with two 282 -> 278).
-struct CombineGate {
-  const float* rows;      // [n, stride] float32, or nullptr: the scale alone
-  int stride, col0, per, out_stride, out_col0;
-  float scale;
-};
+// GATED: with the gate over the heads' outputs (AttnArgs::gate).
 template <bool GATED>
 __global__ __launch_bounds__(64) void attn_combine_kernel(const float* __restrict__ scratch,
                                                           const int* __restrict__ cu_seqlens,
@@ -1355,7 +1551,7 @@ __global__ __launch_bounds__(64) void attn_combine_kernel(const float* __restric
   for (int d0 = 0; d0 < D; d0 += 64) {
     const int d = min(d0 + lane, D - 1);
     float raw = 0.f;
-    if (GATED && gate.rows != nullptr) raw = gate.rows[(size_t)q_start * gate.stride + gate.col0 + (h * D + d) / gate.per];
+    if (GATED) raw = gate_of(gate, q_start, h * D + d);
     float acc = 0.f;
     int s = 0;
     for (; s + 8 <= num_splits; s += 8) {   // eight independent loads in flight
@@ -1367,27 +1563,11 @@ __global__ __launch_bounds__(64) void attn_combine_kernel(const float* __restric
     }
     for (; s < num_splits; ++s) acc = fmaf(__shfl(ws, s, 64), base[(size_t)s * (D + 2) + d], acc);
     if constexpr (GATED) {
-      float v = bf16_to_float(float_to_bf16(acc * inv));
-      if (gate.rows != nullptr) v *= 1.0f / (1.0f + expf(-raw));
-      if (d0 + lane < D) out[(size_t)q_start * gate.out_stride + gate.out_col0 + h * D + d] = float_to_bf16(v * gate.scale);
+      if (d0 + lane < D) store_gated_head(gate, out, q_start, h * D + d, acc * inv, raw);
     } else if (d0 + lane < D) {
       out[((size_t)q_start * n_heads + h) * D + d] = float_to_bf16(acc * inv);
     }
   }
-}
-
-extern "C" int tp_attention_combine_gate(const float* scratch, const int* cu_seqlens, void* out, int n_req, int n_heads, int value_dim,
-                                         int num_splits, const float* sink, const float* gate, int gate_stride, int gate_col0, int per,
-                                         float scale, int out_stride, int out_col0, hipStream_t s) {
-  TP_REQUIRE(n_req >= 0 && n_heads > 0 && n_heads <= 65535 && value_dim > 0 && num_splits >= 1 && num_splits <= 64 && scratch && out, "attention_combine_gate: bad sizes");
-  const int width = n_heads * value_dim;
-  TP_REQUIRE(out_col0 >= 0 && out_stride >= out_col0 + width && per >= 1 && width % per == 0, "attention_combine_gate: bad output rows");
-  TP_REQUIRE(gate == nullptr || (gate_col0 >= 0 && gate_stride >= gate_col0 + width / per), "attention_combine_gate: gate rows too short");
-  if (n_req == 0) return 0;
-  hipLaunchKernelGGL(attn_combine_kernel<true>, dim3(n_req, n_heads), dim3(64), 0, s, scratch, cu_seqlens, (bf16_t*)out, n_heads, value_dim,
-                     num_splits, sink, CombineGate{gate, gate_stride, gate_col0, per, out_stride, out_col0, scale});
-  TP_CHECK_LAUNCH("attention_combine_gate");
-  return 0;
 }
 
 // The same for the rows of portions whose keys were split over blocks: out[token, head, :] from the parts
@@ -1454,11 +1634,28 @@ static int launch_all(AttnArgs a, int n_tokens, int n_req, int max_q_len, int nu
     if constexpr (WITH_BIAS) {
       if (bias) hipLaunchKernelGGL((attn_decode_kernel<D, DV, MODE_BIAS>), grid, dim3(256), 0, s, a);
     }
-    if (!bias) hipLaunchKernelGGL((attn_decode_kernel<D, DV, MODE>), grid, dim3(256), 0, s, a);
-    if (a.num_splits > 1 && !a.keep_parts) {
+    bool done = bias;
+    if constexpr (LDS && DV <= 128) {
+      // rings of 64 KB a block, two blocks a CU; where the keys are not split and every block has a CU of its own, twice the waves
+      // (one request of 500 keys of 64 elements 7.2 -> 6.4 us, 32 of 3,000 36.1 -> 35.6; 48 requests, 384 blocks, 20.6 -> 22.7)
+      constexpr int NB = (D + DV) * 64 > 8192 ? 1 : 2;
+      if (!bias && a.page_shift >= 4 && g_attn_tune != 1) {
+        if (a.num_splits == 1 && grid.x * grid.y <= 256)
+          hipLaunchKernelGGL((attn_decode_lds_kernel<D, DV, MODE, 8, NB>), grid, dim3(512), 0, s, a);
+        else
+          hipLaunchKernelGGL((attn_decode_lds_kernel<D, DV, MODE, 4, NB>), grid, dim3(256), 0, s, a);
+        done = true;
+      }
+    }
+    if (!done) hipLaunchKernelGGL((attn_decode_kernel<D, DV, MODE>), grid, dim3(256), 0, s, a);
+    if (a.num_splits > 1) {
       const dim3 cgrid(n_req, a.n_heads);
-      hipLaunchKernelGGL(attn_combine_kernel<false>, cgrid, dim3(64), 0, s, a.scratch, a.cu_seqlens, a.out, a.n_heads, DV,
-                         a.num_splits, a.sink, CombineGate{});
+      if (a.gated)
+        hipLaunchKernelGGL(attn_combine_kernel<true>, cgrid, dim3(64), 0, s, a.scratch, a.cu_seqlens, a.out, a.n_heads, DV,
+                           a.num_splits, a.sink, a.gate);
+      else
+        hipLaunchKernelGGL(attn_combine_kernel<false>, cgrid, dim3(64), 0, s, a.scratch, a.cu_seqlens, a.out, a.n_heads, DV,
+                           a.num_splits, a.sink, CombineGate{});
     }
   }
   if (has_multi) {
@@ -1576,7 +1773,8 @@ int tp_paged_attention_fast(const void* q, const void* k_cache, const void* v_ca
                             int max_q_len, int num_single, int num_splits, float* scratch, const int* token_req,
                             int portion_splits, int portion_min_steps, float* portion_scratch, const float* dist_bias,
                             int bias_len, int keep_first, const float* sink, int value_dim, int chunk, float softcap,
-                            int keep_parts, hipStream_t s) {
+                            int gated, const float* gate, int gate_stride, int gate_col0, int gate_per, float gate_scale, int out_stride,
+                            int out_col0, hipStream_t s) {
   if (head_dim % 32 != 0 || page_size % 8 != 0) return -1;
   if (dist_bias != nullptr && (value_dim != head_dim || softcap > 0.f)) return -1;
   if (chunk < 0 || chunk == 1 || (chunk > 0 && (window > 0 || keep_first > 0))) return -1;
@@ -1587,6 +1785,7 @@ int tp_paged_attention_fast(const void* q, const void* k_cache, const void* v_ca
   if (n_req > 65535 || n_req <= 0) return -1;
   if (num_single > 0 && (num_splits < 1 || num_splits > 64)) return -1;
   if (num_single > 0 && num_splits > 1 && scratch == nullptr) return -1;
+  if (gated && num_single != n_req) return -1;
   AttnArgs a;
   a.q = (const bf16_t*)q;
   a.k_cache = (const bf16_t*)k_cache;
@@ -1605,7 +1804,9 @@ int tp_paged_attention_fast(const void* q, const void* k_cache, const void* v_ca
     if ((1 << b) == page_size) a.page_shift = b;
   a.window = window;
   a.num_splits = num_splits;
-  a.keep_parts = keep_parts != 0;
+  a.all_single = num_single == n_req;
+  a.gated = gated != 0;
+  a.gate = CombineGate{gate, gate_stride, gate_col0, gate_per, out_stride, out_col0, gate_scale};
   a.portion_splits = portion_splits;
   a.portion_min_steps = portion_min_steps;
   a.portion_scratch = portion_scratch;

@@ -943,6 +943,11 @@ def fast_pair(key_dim: int, value_dim: int, exact_values: bool = True):
     return min(fit, key=lambda p: (p[0] + p[1], p)) if fit else None
 
 
+def decode_rings(key_dim: int, value_dim: int, page_size: int) -> bool:
+    """Whether single tokens take the kernel whose waves have their keys and values on the way to LDS."""
+    return key_dim in (32, 64, 128, 192) and (key_dim + value_dim) % 64 == 0 and value_dim <= 128 and page_size >= 16 and page_size & (page_size - 1) == 0
+
+
 def fast_attention_takes(has_sink: bool, keep_first: int) -> bool:
     """Whether the matrix-core attention kernels take a softmax with a sink and kept first keys (else the general
     kernel runs, and no splits or partial results are prepared for them): both (kept first keys by the kernels that
@@ -1002,7 +1007,6 @@ def paged_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tenso
     _i32(token_req, n, "token_req") if n else None
     _need(pages * kvh * page_size < 2 ** 31, "paged_attention: cache pool too large for 32-bit row indices")
     _need(max_context_len <= width * page_size, "paged_attention: block table narrower than the longest context")
-    out = torch.empty((n, heads * vd), dtype=q.dtype, device=q.device)
     if num_single is None:
         num_single = r if max_q_len == 1 else 0
     _need(0 <= num_single <= r, "paged_attention: num_single out of range")
@@ -1051,7 +1055,19 @@ def paged_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tenso
         bound = 256
         while bound < max_context_len:
             bound *= 2
-        splits = max(1, min(64, want, bound // 128))
+        seen = min(bound, window + keep_first + 31) if window else min(bound, chunk) if chunk else bound
+        if decode_force_splits == 0 and dist_bias is None and decode_rings(d, vd, page_size):
+            # (a launch and a trip through memory for the kernel that adds the splits, 4 us, against the keys that one block walks
+            # alone, 5 us for 512 of 128 elements: 8 key heads of 128, not split / as above, one request of 120 / 500 / 1,000 keys
+            # 4.6 / 8.6 / 13.4 against 8.0 / 10.4 / 8.8 us, 8 requests 5.8 / 9.4 / 14.2 against 9.0 / 12.0 / 12.5.  From 65 blocks a
+            # split on: 16 requests of 1,000 keys 15.8 against 19.5 us, of 3,000 41.9 against 39.8 and in two splits 38.4, of 600 to
+            # 6,000 59 and 43.5; from 129 on: 32 requests of 500 / 1,000 / 3,000 keys 13.9 / 23.6 / 64 against 18.1 / 28.5 / 68,
+            # of 600 to 6,000 73.8 against 82.)
+            if seen <= 512 or blocks_per_split > 128:
+                want = 1
+            elif blocks_per_split > 64:
+                want = 1 if seen <= 1024 else 2
+        splits = max(1, min(64, want, max(1, seen // 128)))
         if splits > 1:
             scratch = torch.empty((r * heads * splits * (vd + 2),), dtype=torch.float32, device=q.device)
     fast_f32 = allow_fast_attention and q.dtype == torch.float32 and d == vd and d in (32, 64, 96, 128) and page_size % 16 == 0
@@ -1078,27 +1094,29 @@ def paged_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tenso
             parts = 1
         if parts > 1:
             part_scratch = torch.empty((n * heads * parts * (vd + 4),), dtype=torch.float32, device=q.device)
-    # (single tokens whose keys are split: the kernel that adds the splits also gates them)
-    keep_parts = into is not None and fast and splits > 1 and num_single == r and n > 0
-    _call("tp_paged_attention", _ptr(q), _dt(q), _ptr(k_cache), _ptr(v_cache), _ptr(block_tables), width,
-          _ptr(cu_seqlens), _ptr(context_lens), _ptr(token_req), _ptr(out), n, r, heads, kvh, d, page_size,
-          ctypes.c_float(scale), int(window), int(max_q_len), int(max_context_len), 2 if keep_parts else int(fast or fast_f32),
-          int(num_single), int(splits), _ptr(scratch), int(parts), max(1, portion_min_keys // 32), _ptr(part_scratch),
-          _ptr(dist_bias), 0 if dist_bias is None else dist_bias.shape[1], int(vd), int(keep_first), _ptr(sink), int(chunk),
-          ctypes.c_float(softcap), _stream())
-    if into is None:
-        return out
-    if keep_parts:
+    # (single tokens: the kernel that writes a row also gates it)
+    gated = into is not None and fast and num_single == r == n and 0 < n <= 65535
+    if not gated:
+        gate, gate_col0, factor, dest_col0, per = None, 0, 1.0, 0, 1
+        dest = torch.empty((n, heads * vd), dtype=q.dtype, device=q.device)
+    else:
         gate, gate_col0, factor, dest, dest_col0, per = into
         _dev_ok(gate, dest)
         _need(dest.dim() == 2 and dest.dtype == q.dtype and dest.shape[0] == n and 0 <= dest_col0 and dest_col0 + heads * vd <= dest.shape[1]
               and per >= 1 and (heads * vd) % per == 0, "paged_attention: bad output rows")
         _need(gate is None or (gate.dtype == torch.float32 and gate.dim() == 2 and gate.shape[0] == n and 0 <= gate_col0
                                and gate_col0 + heads * vd // per <= gate.shape[1]), "paged_attention: bad gate rows")
-        _call("tp_attention_combine_gate", _ptr(scratch), _ptr(cu_seqlens), _ptr(dest), r, heads, vd, int(splits), _ptr(sink), _ptr(gate),
-              0 if gate is None else gate.shape[1], int(gate_col0), int(per), ctypes.c_float(factor), dest.shape[1], int(dest_col0), _stream())
-    else:
-        sigmoid_gate(out, *into)
+    _call("tp_paged_attention", _ptr(q), _dt(q), _ptr(k_cache), _ptr(v_cache), _ptr(block_tables), width,
+          _ptr(cu_seqlens), _ptr(context_lens), _ptr(token_req), _ptr(dest), n, r, heads, kvh, d, page_size,
+          ctypes.c_float(scale), int(window), int(max_q_len), int(max_context_len), 2 if gated else int(fast or fast_f32),
+          int(num_single), int(splits), _ptr(scratch), int(parts), max(1, portion_min_keys // 32), _ptr(part_scratch),
+          _ptr(dist_bias), 0 if dist_bias is None else dist_bias.shape[1], int(vd), int(keep_first), _ptr(sink), int(chunk),
+          ctypes.c_float(softcap), _ptr(gate), 0 if gate is None else gate.shape[1], int(gate_col0), int(per), ctypes.c_float(factor),
+          dest.shape[1], int(dest_col0), _stream())
+    if into is None:
+        return dest
+    if not gated:
+        sigmoid_gate(dest, *into)
     return None
 
 

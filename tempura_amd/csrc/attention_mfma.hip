@@ -147,6 +147,31 @@ __device__ inline int attn_first_key(const AttnArgs& a, int pos) {
 __device__ inline float attn_capped(const AttnArgs& a, float dot) {
   return fmaf(-2.0f * a.cap_log2, __builtin_amdgcn_rcpf(__builtin_amdgcn_exp2f(dot * a.cap_in) + 1.0f), a.cap_log2);
 }
+// What stands between a projection's float32 rows and the attention of single tokens, for the decode kernel that takes the rows
+// themselves (ROWS): rows [n, stride] of q | k | v heads (parts > 1: the partial sums of a product whose K was split, part_stride
+// apart, added in ascending order), a causal convolution per channel (conv_w [taps, channels] or nullptr; its carried inputs
+// [taps - 1, channels] in the request's state row, moved on here), a norm per head of q and k (weights [D] or nullptr), the rotation
+// of neighbouring pairs, and the places of k and v in the cache.
+struct RowsIn {
+  const float* rows;
+  size_t part_stride;
+  int stride, parts;
+  const float* conv_w;
+  float* state;
+  size_t state_stride, state_off;
+  const int* state_slots;
+  int taps, channels;
+  const float *q_norm, *k_norm;
+  float norm_eps, factor;
+  const float2* cos_sin;      // [n, rotary_dim / 2] this step's table, or nullptr
+  const int* positions;
+  const double* inv_freq;
+  int rotary_dim;
+  const int* slots;
+  bf16_t *k_cache, *v_cache;
+};
+#define ROWS_PARTS 8
+#define ROWS_TAPS 4
 #define PART_STRIDE(D) ((D) + 4)
 // the sink's share of a denominator that is relative to the maximum m (scores and m are in units of log 2): 2^(sink *
 // log2(e) - m); a sink far above m makes the sum infinite and the row zero, which is its limit
@@ -1357,8 +1382,13 @@ __global__ __launch_bounds__(256) void attn_decode_kernel(AttnArgs a) {
 // they replace are in registers, its values likewise, its pages before that.
 // (a wait that stays in its place among the assembly that reads LDS behind it)
 #define ATTN_WAIT_VM_ORDERED(n) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(n) : "memory")
-template <int D, int DV, int MODE, int WAVES, int NB>
-__global__ __launch_bounds__(WAVES * 64) void attn_decode_lds_kernel(AttnArgs a) {
+// ROWS: q, k and v come as the projection's float32 rows (RowsIn): a wave takes a head (of q, or the new key, or the new value), the
+// block's heads go to LDS, the new key and value to the cache and, since the cache's own copy may not have arrived when the step
+// that holds it is read, into that step's place in LDS.  The rows travel beside the first keys; a launch or two between the
+// projection and the attention are gone: Bomotar's decode step, four layers with a convolution, 377 -> 361 us; 28 layers of the 3B
+// shape with 48 requests, three parts of K, 3,219 -> 3,187.
+template <int D, int DV, int MODE, int WAVES, int NB, bool ROWS = false>
+__global__ __launch_bounds__(WAVES * 64) void attn_decode_lds_kernel(AttnArgs a, RowsIn in) {
   constexpr int C = D / 8;             // 16-byte chunks per key row
   constexpr int SH = C == 16 ? 0 : (C == 8 || C == 24 ? 1 : 2);
   constexpr int KI = D / 16, VI = DV / 16, STAGE = (KI + VI) * 1024;
@@ -1366,6 +1396,7 @@ __global__ __launch_bounds__(WAVES * 64) void attn_decode_lds_kernel(AttnArgs a)
   static_assert(NB * STAGE >= (DV * 17 + 32) * 4, "room for the merge");
   static_assert((NB == 1 || NB == 2) && 2 * VI + KI <= 63 && 2 * KI + VI <= 63, "the waits below");
   __shared__ __attribute__((aligned(1024))) unsigned char stages[WAVES * NB * STAGE];
+  __shared__ __attribute__((aligned(16))) bf16_t heads_lds[ROWS ? 18 * D : 8];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int g = lane >> 4, c = lane & 15;
   const int group = a.n_heads / a.n_kv;
@@ -1379,9 +1410,41 @@ __global__ __launch_bounds__(WAVES * 64) void attn_decode_lds_kernel(AttnArgs a)
   if (!a.all_single && a.cu_seqlens[r + 1] - q_start != 1) return;
   const int ctx = a.context_lens[r];
   u32x4_t qv[D / 32];
-  const bf16_t* qr = a.q + ((size_t)q_start * a.n_heads + head) * D + g * 8;
+  if constexpr (!ROWS) {
+    const bf16_t* qr = a.q + ((size_t)q_start * a.n_heads + head) * D + g * 8;
 #pragma unroll
-  for (int dk = 0; dk < D / 32; ++dk) qv[dk] = *(const u32x4_t*)(qr + dk * 32);
+    for (int dk = 0; dk < D / 32; ++dk) qv[dk] = *(const u32x4_t*)(qr + dk * 32);
+  }
+  // (ROWS; r is the token's row) item i: head i of q, then the new key, then the new value; a lane has the elements 2 lane, 2 lane + 1
+  const int items = ncols + 2;
+  float2 raw[ROWS ? ROWS_PARTS : 1], turn = make_float2(1.f, 0.f);
+  int place = 0;
+  auto fetch_row = [&](int i) __attribute__((always_inline)) {
+    if constexpr (ROWS) {
+      const int e = 2 * lane;
+      if (e >= (i == ncols + 1 ? DV : D)) return;
+      const int qd = a.n_heads * D, kd = a.n_kv * D;
+      const int col = (i < ncols ? (kvh * group + i) * D : i == ncols ? qd + kvh * D : qd + kd + kvh * DV) + e;
+      const float* row = in.rows + (size_t)r * in.stride + col;
+      if (in.conv_w != nullptr) {     // this token's input, the carried ones, the weights
+        raw[0] = *(const float2*)row;
+        const float* st = in.state + (size_t)in.state_slots[r] * in.state_stride + in.state_off + col;
+#pragma unroll
+        for (int t = 0; t < ROWS_TAPS - 1; ++t)
+          if (t < in.taps - 1) raw[1 + t] = *(const float2*)(st + (size_t)t * in.channels);
+#pragma unroll
+        for (int t = 0; t < ROWS_TAPS; ++t)
+          if (t < in.taps) raw[ROWS_TAPS + t] = *(const float2*)(in.conv_w + (size_t)t * in.channels + col);
+      } else {
+#pragma unroll
+        for (int t = 0; t < ROWS_PARTS; ++t)
+          if (t < in.parts) raw[t] = *(const float2*)(row + (size_t)t * in.part_stride);
+      }
+      if (i <= ncols && e < in.rotary_dim && in.cos_sin != nullptr) turn = in.cos_sin[(size_t)r * (in.rotary_dim >> 1) + lane];
+      if (i >= ncols) place = in.slots[r];
+    }
+  };
+  if (ROWS && wave < items) fetch_row(wave);
   // this lane's offset in each load of a step, and its addresses in LDS (see attn_prefill_lds_kernel)
   const int ps = a.page_size, psh = a.page_shift, pmask = ps - 1;
   unsigned koff[KI];
@@ -1452,6 +1515,75 @@ __global__ __launch_bounds__(WAVES * 64) void attn_decode_lds_kernel(AttnArgs a)
       issue_values(i, i);
     }
   if (NB < n) pages_of(NB);
+  const unsigned hl0 = (unsigned)(size_t)(__attribute__((address_space(3))) const bf16_t*)heads_lds;
+  if constexpr (ROWS) {
+    const bool newest = s_begin < s_end && s_end == steps;      // this block's keys end with the token's own
+    for (int i = wave; i < items; i += WAVES) {
+      if (i != wave) fetch_row(i);
+      if (i >= ncols && !newest) continue;
+      const int e = 2 * lane, width = i == ncols + 1 ? DV : D;
+      float x0 = 0.f, x1 = 0.f;
+      if (e < width) {
+        if (in.conv_w != nullptr) {
+          const int qd = a.n_heads * D, kd = a.n_kv * D;
+          const int col = (i < ncols ? (kvh * group + i) * D : i == ncols ? qd + kvh * D : qd + kd + kvh * DV) + e;
+          float* st = in.state + (size_t)in.state_slots[r] * in.state_stride + in.state_off + col;
+#pragma unroll
+          for (int t = 0; t < ROWS_TAPS; ++t)
+            if (t < in.taps) {
+              const float2 v = t == in.taps - 1 ? raw[0] : raw[1 + t];
+              if (t > 0) *(float2*)(st + (size_t)(t - 1) * in.channels) = v;
+              x0 = fmaf(raw[ROWS_TAPS + t].x, v.x, x0);
+              x1 = fmaf(raw[ROWS_TAPS + t].y, v.y, x1);
+            }
+        } else {
+#pragma unroll
+          for (int t = 0; t < ROWS_PARTS; ++t)
+            if (t < in.parts) {
+              x0 += raw[t].x;
+              x1 += raw[t].y;
+            }
+        }
+      }
+      if (i <= ncols && in.q_norm != nullptr) {
+        const float* w = i < ncols ? in.q_norm : in.k_norm;
+        const float rstd = 1.0f / sqrtf(wave_sum(fmaf(x0, x0, x1 * x1)) / (float)D + in.norm_eps);
+        if (e < D) {
+          x0 = x0 * rstd * w[e];
+          x1 = x1 * rstd * w[e + 1];
+        }
+      }
+      if (e >= width) continue;
+      if (i <= ncols && e < in.rotary_dim) {
+        float2 cs = turn;
+        if (in.cos_sin == nullptr) rope_cos_sin(in.positions[r], in.inv_freq[lane], in.factor, cs.x, cs.y);
+        const float y0 = x0, y1 = x1;
+        x0 = y0 * cs.x - y1 * cs.y;
+        x1 = y0 * cs.y + y1 * cs.x;
+      }
+      const unsigned pk = pack_bf16(x0, x1);
+      const unsigned to = hl0 + (i < ncols ? i : 16 + i - ncols) * (D * 2) + e * 2;
+      asm volatile("ds_write_b32 %0, %1" ::"v"(to), "v"(pk) : "memory");
+      if (i >= ncols) {
+        const size_t page = (size_t)(place >> psh), off = (size_t)(place & pmask);
+        if (i == ncols) {
+          *(unsigned*)(in.k_cache + ((page * a.n_kv + kvh) * ps + off) * D + e) = pk;
+        } else {
+          bf16_t* o = in.v_cache + ((page * a.n_kv + kvh) * DV + e) * ps + off;
+          o[0] = bf16_t{(uint16_t)(pk & 0xffff)};
+          o[ps] = bf16_t{(uint16_t)(pk >> 16)};
+        }
+      }
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    const unsigned qa = hl0 + min(c, ncols - 1) * (D * 2) + g * 16;
+#pragma unroll
+    for (int dk = 0; dk < D / 32; ++dk) qv[dk] = attn_lds_read<0>(qa + dk * 64);
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+#pragma unroll
+    for (int dk = 0; dk < D / 32; ++dk) asm volatile("" : "+v"(qv[dk]));
+  }
   bf16x8_t qf[1][D / 32];
   int qpos[1] = {ctx - 1};
   float m[1] = {-INFINITY}, l[1] = {0.f};
@@ -1466,8 +1598,24 @@ __global__ __launch_bounds__(WAVES * 64) void attn_decode_lds_kernel(AttnArgs a)
     const unsigned base = lds0 + st * STAGE;
     const bool behind = NB > 1 && i + 1 < n;      // (a whole step on its way behind this one)
     const bool more = i + NB < n;
-    if (behind) ATTN_WAIT_VM_ORDERED(VI + KI + VI);
+    // (ROWS: the stores of the new key, value and carried inputs are behind the first loads, and the waits count them as well: a
+    // step that should have waited for its loads alone waits for less than it could, never for less than it needs, so the first
+    // steps wait for everything)
+    if (ROWS && i < NB) ATTN_WAIT_VM_ORDERED(0);
+    else if (behind) ATTN_WAIT_VM_ORDERED(VI + KI + VI);
     else ATTN_WAIT_VM_ORDERED(VI);
+    const int j0 = key0(i);
+    const bool own = ROWS && ctx - 1 - j0 < 32 && ctx - 1 >= j0;   // the step that holds the token's own key and value
+    const int kr = ctx - 1 - j0;
+    if (own) {
+      const int f = ((((kr >> 3) << 2) | (kr & 3)) >> SH);
+      if (lane < C) {
+        const u32x4_t kv = attn_lds_read<0>(hl0 + 16 * (D * 2) + lane * 16);
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        asm volatile("ds_write_b128 %0, %1" ::"v"(base + (kr * C + (lane + f) % C) * 16), "v"(kv) : "memory");
+      }
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    }
     u32x4_t kk[2][D / 32];
 #pragma unroll
     for (int t2 = 0; t2 < 2; ++t2)
@@ -1488,12 +1636,23 @@ __global__ __launch_bounds__(WAVES * 64) void attn_decode_lds_kernel(AttnArgs a)
     bf16x8_t pf[1];
     float alpha[1];
     bool moved[1];
-    const int j0 = key0(i);
     attn_softmax<1, true, MODE>(a, j0, sc, qpos, m, l, pf, alpha, moved);
     if (more && behind) ATTN_WAIT_VM_ORDERED(KI + KI + VI);
     else if (more) ATTN_WAIT_VM_ORDERED(KI);
     else if (behind) ATTN_WAIT_VM_ORDERED(KI + VI);
     else ATTN_WAIT_VM_ORDERED(0);
+    if (own) {
+#pragma unroll
+      for (int d = lane; d < DV; d += 64) {
+        unsigned v;
+        asm volatile("ds_read_u16 %0, %1\n\ts_waitcnt lgkmcnt(0)" : "=v"(v) : "v"(hl0 + 17 * (D * 2) + d * 2));
+        asm volatile("ds_write_b16 %0, %1" ::"v"(base + KI * 1024 + (d >> 5) * 2048 + ((d >> 4) & 1) * 256 + (d & 15) * 16 + (kr >> 4) * 1024 +
+                                                 ((kr >> 3) & 1) * 512 + (kr & 7) * 2),
+                     "v"(v)
+                     : "memory");
+      }
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    }
     u32x4_t vv[DV / 16];
 #define ATTN_RV(dt) if constexpr (dt < DV / 16) vv[dt] = attn_lds_read<(dt >> 1) * 2048 + (dt & 1) * 256>(base + vaddr)
     ATTN_RV(0); ATTN_RV(1); ATTN_RV(2); ATTN_RV(3); ATTN_RV(4); ATTN_RV(5); ATTN_RV(6); ATTN_RV(7);
@@ -1615,6 +1774,15 @@ __global__ __launch_bounds__(64) void attn_combine_rows_kernel(const float* __re
 static int g_attn_tune = 0;   // 1: portions take the kernel that loads keys and values per wave; 2 / 3: 32 / 16 query rows per wave
 extern "C" void tp_attention_tune(int v) { g_attn_tune = v; }
 
+static void launch_combine(const AttnArgs& a, int n_req, int value_dim, hipStream_t s) {
+  const dim3 grid(n_req, a.n_heads);
+  if (a.gated)
+    hipLaunchKernelGGL(attn_combine_kernel<true>, grid, dim3(64), 0, s, a.scratch, a.cu_seqlens, a.out, a.n_heads, value_dim, a.num_splits, a.sink, a.gate);
+  else
+    hipLaunchKernelGGL(attn_combine_kernel<false>, grid, dim3(64), 0, s, a.scratch, a.cu_seqlens, a.out, a.n_heads, value_dim, a.num_splits, a.sink,
+                       CombineGate{});
+}
+
 // MODE: MODE_PLAIN, or MODE_CAP where the scores are capped; a bias by distance (square sizes only) is chosen inside.
 template <int D, int DV, int MODE>
 static int launch_all(AttnArgs a, int n_tokens, int n_req, int max_q_len, int num_single, hipStream_t s) {
@@ -1641,22 +1809,14 @@ static int launch_all(AttnArgs a, int n_tokens, int n_req, int max_q_len, int nu
       constexpr int NB = (D + DV) * 64 > 8192 ? 1 : 2;
       if (!bias && a.page_shift >= 4 && g_attn_tune != 1) {
         if (a.num_splits == 1 && grid.x * grid.y <= 256)
-          hipLaunchKernelGGL((attn_decode_lds_kernel<D, DV, MODE, 8, NB>), grid, dim3(512), 0, s, a);
+          hipLaunchKernelGGL((attn_decode_lds_kernel<D, DV, MODE, 8, NB>), grid, dim3(512), 0, s, a, RowsIn{});
         else
-          hipLaunchKernelGGL((attn_decode_lds_kernel<D, DV, MODE, 4, NB>), grid, dim3(256), 0, s, a);
+          hipLaunchKernelGGL((attn_decode_lds_kernel<D, DV, MODE, 4, NB>), grid, dim3(256), 0, s, a, RowsIn{});
         done = true;
       }
     }
     if (!done) hipLaunchKernelGGL((attn_decode_kernel<D, DV, MODE>), grid, dim3(256), 0, s, a);
-    if (a.num_splits > 1) {
-      const dim3 cgrid(n_req, a.n_heads);
-      if (a.gated)
-        hipLaunchKernelGGL(attn_combine_kernel<true>, cgrid, dim3(64), 0, s, a.scratch, a.cu_seqlens, a.out, a.n_heads, DV,
-                           a.num_splits, a.sink, a.gate);
-      else
-        hipLaunchKernelGGL(attn_combine_kernel<false>, cgrid, dim3(64), 0, s, a.scratch, a.cu_seqlens, a.out, a.n_heads, DV,
-                           a.num_splits, a.sink, CombineGate{});
-    }
+    if (a.num_splits > 1) launch_combine(a, n_req, DV, s);
   }
   if (has_multi) {
     // A wave owns 16 query rows, three blocks to a CU, or 32 rows (two tiles: half the key and value reads per
@@ -1767,6 +1927,91 @@ static int launch_sizes(const AttnArgs& a, int d, int dv, int n_tokens, int n_re
   }
 }
 
+static AttnArgs decode_args(const bf16_t* k_cache, const bf16_t* v_cache, const int* block_tables, int table_width, const int* cu_seqlens,
+                            const int* context_lens, bf16_t* out, int n_heads, int n_kv, int page_size, float scale, int window, int num_splits,
+                            float* scratch, int keep_first, const float* sink, int chunk) {
+  AttnArgs a = {};
+  a.k_cache = k_cache;
+  a.v_cache = v_cache;
+  a.block_tables = block_tables;
+  a.table_width = table_width;
+  a.cu_seqlens = cu_seqlens;
+  a.context_lens = context_lens;
+  a.out = out;
+  a.scratch = scratch;
+  a.n_heads = n_heads;
+  a.n_kv = n_kv;
+  a.page_size = page_size;
+  a.page_shift = -1;
+  for (int b = 0; b < 30; ++b)
+    if ((1 << b) == page_size) a.page_shift = b;
+  a.window = window;
+  a.num_splits = num_splits;
+  a.portion_splits = 1;
+  a.portion_min_steps = 1;
+  a.heads_per_block = 4;
+  a.sink = sink;
+  a.keep_first = window > 0 ? keep_first : 0;
+  a.scale_log2 = scale * 1.4426950408889634f;
+  a.chunk = chunk;
+  if (chunk > 0) {
+    while ((2u << a.chunk_shift) < (unsigned)chunk) ++a.chunk_shift;      // ceil(log2(chunk)) - 1
+    a.chunk_mul = (unsigned)((((unsigned long long)1 << (32 + a.chunk_shift)) + (unsigned)chunk - 1) / (unsigned)chunk);
+  }
+  return a;
+}
+
+// Single tokens from their projection's rows (see RowsIn and attn_decode_lds_kernel): n requests of one token each, heads of 64 or 128
+// elements, values alike, at most 16 heads a key head, pages of a power of two from 16 on.  With num_splits > 1 scratch of n * n_heads *
+// num_splits * (dim + 2) floats, and no convolution (a channel's carried inputs have one block).  gated: out as of tp_paged_attention
+// with allow_fast 2.
+extern "C" int tp_attention_rows(const float* rows, size_t part_stride, int stride, int parts, const float* conv_w, int taps, int channels,
+                                 float* state, size_t state_stride, size_t state_off, const int* state_slots, const float* q_norm,
+                                 const float* k_norm, float norm_eps, const int* positions, const double* inv_freq, int rotary_dim, float factor,
+                                 const float* cos_sin, const int* slots, void* k_cache, void* v_cache, const int* block_tables, int table_width,
+                                 const int* cu_seqlens, const int* context_lens, void* out, int n, int n_heads, int n_kv, int dim, int page_size,
+                                 float scale, int window, int keep_first, int chunk, const float* sink, int num_splits, float* scratch, int gated,
+                                 const float* gate, int gate_stride, int gate_col0, int gate_per, float gate_scale, int out_stride, int out_col0,
+                                 hipStream_t s) {
+  TP_REQUIRE(n >= 0 && n <= 65535 && n_kv > 0 && n_heads > 0 && n_heads <= 65535 && n_heads % n_kv == 0 && n_heads / n_kv <= 16 && (dim == 64 || dim == 128),
+             "attention_rows: bad heads (%d of %d, %d key heads)", n_heads, dim, n_kv);
+  TP_REQUIRE(page_size >= 16 && (page_size & (page_size - 1)) == 0 && parts >= 1 && parts <= ROWS_PARTS && stride % 2 == 0 && part_stride % 2 == 0 &&
+                 stride >= (n_heads + 2 * n_kv) * dim && ((uintptr_t)rows & 7) == 0,
+             "attention_rows: bad rows or pages");
+  TP_REQUIRE(rotary_dim >= 0 && rotary_dim <= dim && rotary_dim % 2 == 0 && (rotary_dim == 0 || cos_sin != nullptr || (positions && inv_freq)) && slots,
+             "attention_rows: bad rotation");
+  TP_REQUIRE(conv_w == nullptr || (taps >= 1 && taps <= ROWS_TAPS && parts == 1 && num_splits == 1 && channels == (n_heads + 2 * n_kv) * dim && state &&
+                                   state_slots && state_stride % 2 == 0 && state_off % 2 == 0 && (((uintptr_t)state | (uintptr_t)conv_w) & 7) == 0 &&
+                                   state_stride >= state_off + (size_t)(taps - 1) * channels),
+             "attention_rows: bad convolution");
+  TP_REQUIRE((q_norm == nullptr) == (k_norm == nullptr), "attention_rows: a norm needs both weights");
+  TP_REQUIRE(num_splits >= 1 && num_splits <= 64 && (num_splits == 1 || scratch), "attention_rows: bad splits");
+  TP_REQUIRE(window >= 0 && keep_first >= 0 && chunk >= 0 && chunk != 1 && (chunk == 0 || window == 0), "attention_rows: bad mask");
+  const int width = n_heads * dim;
+  TP_REQUIRE(!gated || (out_col0 >= 0 && out_stride >= out_col0 + width && gate_per >= 1 && width % gate_per == 0 &&
+                        (gate == nullptr || (gate_col0 >= 0 && gate_stride >= gate_col0 + width / gate_per))),
+             "attention_rows: bad gate or output rows");
+  if (n == 0) return 0;
+  AttnArgs a = decode_args((const bf16_t*)k_cache, (const bf16_t*)v_cache, block_tables, table_width, cu_seqlens, context_lens, (bf16_t*)out, n_heads,
+                           n_kv, page_size, scale, window, num_splits, scratch, keep_first, sink, chunk);
+  a.all_single = true;
+  a.gated = gated != 0;
+  a.gate = CombineGate{gate, gate_stride, gate_col0, gate_per, out_stride, out_col0, gate_scale};
+  const RowsIn in = {rows, part_stride, stride, parts, conv_w, state, state_stride, state_off, state_slots, taps, channels, q_norm, k_norm, norm_eps,
+                     factor, (const float2*)cos_sin, positions, inv_freq, rotary_dim, slots, (bf16_t*)k_cache, (bf16_t*)v_cache};
+  const dim3 grid(n_kv, n, num_splits);
+  const bool wide = num_splits == 1 && (long)n_kv * n <= 256;
+#define ROWS_KERNEL(D_, W_, NB_) hipLaunchKernelGGL((attn_decode_lds_kernel<D_, D_, MODE_PLAIN, W_, NB_, true>), grid, dim3(W_ * 64), 0, s, a, in)
+  if (dim == 128 && wide) ROWS_KERNEL(128, 8, 1);
+  else if (dim == 128) ROWS_KERNEL(128, 4, 1);
+  else if (wide) ROWS_KERNEL(64, 8, 2);
+  else ROWS_KERNEL(64, 4, 2);
+#undef ROWS_KERNEL
+  if (num_splits > 1) launch_combine(a, n, dim, s);
+  TP_CHECK_LAUNCH("attention_rows");
+  return 0;
+}
+
 int tp_paged_attention_fast(const void* q, const void* k_cache, const void* v_cache, const int* block_tables,
                             int table_width, const int* cu_seqlens, const int* context_lens, void* out, int n_tokens,
                             int n_req, int n_heads, int n_kv, int head_dim, int page_size, float scale, int window,
@@ -1786,24 +2031,10 @@ int tp_paged_attention_fast(const void* q, const void* k_cache, const void* v_ca
   if (num_single > 0 && (num_splits < 1 || num_splits > 64)) return -1;
   if (num_single > 0 && num_splits > 1 && scratch == nullptr) return -1;
   if (gated && num_single != n_req) return -1;
-  AttnArgs a;
+  if (dist_bias != nullptr && bias_len <= 0) return -1;
+  AttnArgs a = decode_args((const bf16_t*)k_cache, (const bf16_t*)v_cache, block_tables, table_width, cu_seqlens, context_lens, (bf16_t*)out, n_heads,
+                           n_kv, page_size, scale, window, num_splits, scratch, keep_first, sink, chunk);
   a.q = (const bf16_t*)q;
-  a.k_cache = (const bf16_t*)k_cache;
-  a.v_cache = (const bf16_t*)v_cache;
-  a.block_tables = block_tables;
-  a.table_width = table_width;
-  a.cu_seqlens = cu_seqlens;
-  a.context_lens = context_lens;
-  a.out = (bf16_t*)out;
-  a.scratch = scratch;
-  a.n_heads = n_heads;
-  a.n_kv = n_kv;
-  a.page_size = page_size;
-  a.page_shift = -1;
-  for (int b = 0; b < 30; ++b)
-    if ((1 << b) == page_size) a.page_shift = b;
-  a.window = window;
-  a.num_splits = num_splits;
   a.all_single = num_single == n_req;
   a.gated = gated != 0;
   a.gate = CombineGate{gate, gate_stride, gate_col0, gate_per, out_stride, out_col0, gate_scale};
@@ -1813,18 +2044,6 @@ int tp_paged_attention_fast(const void* q, const void* k_cache, const void* v_ca
   a.token_req = token_req;
   a.dist_bias = dist_bias;
   a.bias_len = bias_len;
-  a.heads_per_block = 4;
-  a.sink = sink;
-  a.keep_first = window > 0 ? keep_first : 0;
-  if (dist_bias != nullptr && bias_len <= 0) return -1;
-  a.scale_log2 = scale * 1.4426950408889634f;
-  a.chunk = chunk;
-  a.chunk_shift = 0;
-  a.chunk_mul = 0;
-  if (chunk > 0) {
-    while ((2u << a.chunk_shift) < (unsigned)chunk) ++a.chunk_shift;      // ceil(log2(chunk)) - 1
-    a.chunk_mul = (unsigned)((((unsigned long long)1 << (32 + a.chunk_shift)) + (unsigned)chunk - 1) / (unsigned)chunk);
-  }
   a.cap_log2 = softcap * 1.4426950408889634f;
   a.cap_in = softcap > 0.f ? 2.0f * 1.4426950408889634f * scale / softcap : 0.f;
   const int rc = softcap > 0.f ? launch_sizes<MODE_CAP>(a, head_dim, value_dim, n_tokens, n_req, max_q_len, num_single, s)

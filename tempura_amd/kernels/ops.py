@@ -924,6 +924,8 @@ def decode_rows_padded(rows: int) -> int:
 decode_min_splits = 8
 #: measurements: this many splits whatever the batch (0: chosen by the rules below)
 decode_force_splits = 0
+#: steps of single tokens take their attention from the projection's rows where its kernel allows it
+rows_attention = True
 #: portions of prompts with fewer query blocks than this have their keys split over blocks (1: never)
 portion_target_blocks = 1024
 #: in parts of at least this many keys
@@ -953,6 +955,49 @@ def fast_attention_takes(has_sink: bool, keep_first: int) -> bool:
     kernel runs, and no splits or partial results are prepared for them): both (kept first keys by the kernels that
     load keys and values per wave, whose portions are never split over blocks)."""
     return True
+
+
+def _decode_splits(requests: int, heads: int, kvh: int, max_context_len: int, window: int, keep_first: int, chunk: int, rings: bool) -> int:
+    """Into how many splits the keys of a step's single tokens are cut (``rings``: by the kernel of ``decode_rings``)."""
+    # enough blocks to fill 256 CUs, but at least 128 keys per block
+    blocks_per_split = decode_rows_padded(requests) * kvh * ((heads // kvh + 15) // 16)
+    # (two blocks fit a CU, 512 the chip.  From 65 to 256 blocks per split, as many splits as fill it once: measured
+    # alone at 2,100 keys, 16 requests 35.8 -> 33.5 us, 20 requests 47.2 -> 38.5, 32 requests 54.3 -> 52.7, and more
+    # for contexts that differ; through the engine 16 requests of the 8B shape 4.33 -> 4.25 ms a step, 32 requests
+    # 5.27 -> 5.20; 12 requests in five splits against three 4.11 / 4.27, 20 in three against two 4.77 / 4.92, 24 in
+    # two against three 4.97 / 5.21.)
+    if blocks_per_split <= 64:
+        want = -(-decode_target_blocks // blocks_per_split)
+    elif blocks_per_split <= decode_target_blocks:
+        want = max(1, 2 * decode_target_blocks // blocks_per_split)
+    else:
+        # (more blocks than half the chip's places: no split.  Through the engine, requests of 2,048+ keys of the 8B
+        # shape, one split against two: 36 requests 6.06 / 5.97 ms a step, 40: 6.14 / 6.04, 48: 6.27 / 6.49,
+        # 56: 6.42 / 6.68, 64: 6.62 / 6.89; three splits at 36 and 40 requests, which the kernel timed alone
+        # prefers, 6.07 and 6.13)
+        want = 1
+    if blocks_per_split <= 64:
+        want = max(want, decode_min_splits)     # (batch 8 of the 8B shape: eight splits 3.87 ms a step, four 3.94)
+    if decode_force_splits > 0:
+        want = decode_force_splits
+    # (at least 128 keys a split, by the longest context rounded up to a power of two from 256: a step captured
+    # for a bound on the context and an eager step at the actual length then cut alike and give the same bits)
+    bound = 256
+    while bound < max_context_len:
+        bound *= 2
+    seen = min(bound, window + keep_first + 31) if window else min(bound, chunk) if chunk else bound
+    if decode_force_splits == 0 and rings:
+        # (a launch and a trip through memory for the kernel that adds the splits, 4 us, against the keys that one block walks
+        # alone, 5 us for 512 of 128 elements: 8 key heads of 128, not split / as above, one request of 120 / 500 / 1,000 keys
+        # 4.6 / 8.6 / 13.4 against 8.0 / 10.4 / 8.8 us, 8 requests 5.8 / 9.4 / 14.2 against 9.0 / 12.0 / 12.5.  From 65 blocks a
+        # split on: 16 requests of 1,000 keys 15.8 against 19.5 us, of 3,000 41.9 against 39.8 and in two splits 38.4, of 600 to
+        # 6,000 59 and 43.5; from 129 on: 32 requests of 500 / 1,000 / 3,000 keys 13.9 / 23.6 / 64 against 18.1 / 28.5 / 68,
+        # of 600 to 6,000 73.8 against 82.)
+        if seen <= 512 or blocks_per_split > 128:
+            want = 1
+        elif blocks_per_split > 64:
+            want = 1 if seen <= 1024 else 2
+    return max(1, min(64, want, max(1, seen // 128)))
 
 
 def paged_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, block_tables: torch.Tensor,
@@ -1029,45 +1074,7 @@ def paged_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tenso
     fast = fast and fast_attention_takes(sink is not None, keep_first) and not (keep_first and dist_bias is not None)
     splits, scratch = 1, None
     if fast and num_single > 0:
-        # enough blocks to fill 256 CUs, but at least 128 keys per block
-        blocks_per_split = decode_rows_padded(num_single) * kvh * ((heads // kvh + 15) // 16)
-        # (two blocks fit a CU, 512 the chip.  From 65 to 256 blocks per split, as many splits as fill it once: measured
-        # alone at 2,100 keys, 16 requests 35.8 -> 33.5 us, 20 requests 47.2 -> 38.5, 32 requests 54.3 -> 52.7, and more
-        # for contexts that differ; through the engine 16 requests of the 8B shape 4.33 -> 4.25 ms a step, 32 requests
-        # 5.27 -> 5.20; 12 requests in five splits against three 4.11 / 4.27, 20 in three against two 4.77 / 4.92, 24 in
-        # two against three 4.97 / 5.21.)
-        if blocks_per_split <= 64:
-            want = -(-decode_target_blocks // blocks_per_split)
-        elif blocks_per_split <= decode_target_blocks:
-            want = max(1, 2 * decode_target_blocks // blocks_per_split)
-        else:
-            # (more blocks than half the chip's places: no split.  Through the engine, requests of 2,048+ keys of the 8B
-            # shape, one split against two: 36 requests 6.06 / 5.97 ms a step, 40: 6.14 / 6.04, 48: 6.27 / 6.49,
-            # 56: 6.42 / 6.68, 64: 6.62 / 6.89; three splits at 36 and 40 requests, which the kernel timed alone
-            # prefers, 6.07 and 6.13)
-            want = 1
-        if blocks_per_split <= 64:
-            want = max(want, decode_min_splits)     # (batch 8 of the 8B shape: eight splits 3.87 ms a step, four 3.94)
-        if decode_force_splits > 0:
-            want = decode_force_splits
-        # (at least 128 keys a split, by the longest context rounded up to a power of two from 256: a step captured
-        # for a bound on the context and an eager step at the actual length then cut alike and give the same bits)
-        bound = 256
-        while bound < max_context_len:
-            bound *= 2
-        seen = min(bound, window + keep_first + 31) if window else min(bound, chunk) if chunk else bound
-        if decode_force_splits == 0 and dist_bias is None and decode_rings(d, vd, page_size):
-            # (a launch and a trip through memory for the kernel that adds the splits, 4 us, against the keys that one block walks
-            # alone, 5 us for 512 of 128 elements: 8 key heads of 128, not split / as above, one request of 120 / 500 / 1,000 keys
-            # 4.6 / 8.6 / 13.4 against 8.0 / 10.4 / 8.8 us, 8 requests 5.8 / 9.4 / 14.2 against 9.0 / 12.0 / 12.5.  From 65 blocks a
-            # split on: 16 requests of 1,000 keys 15.8 against 19.5 us, of 3,000 41.9 against 39.8 and in two splits 38.4, of 600 to
-            # 6,000 59 and 43.5; from 129 on: 32 requests of 500 / 1,000 / 3,000 keys 13.9 / 23.6 / 64 against 18.1 / 28.5 / 68,
-            # of 600 to 6,000 73.8 against 82.)
-            if seen <= 512 or blocks_per_split > 128:
-                want = 1
-            elif blocks_per_split > 64:
-                want = 1 if seen <= 1024 else 2
-        splits = max(1, min(64, want, max(1, seen // 128)))
+        splits = _decode_splits(num_single, heads, kvh, max_context_len, window, keep_first, chunk, dist_bias is None and decode_rings(d, vd, page_size))
         if splits > 1:
             scratch = torch.empty((r * heads * splits * (vd + 2),), dtype=torch.float32, device=q.device)
     fast_f32 = allow_fast_attention and q.dtype == torch.float32 and d == vd and d in (32, 64, 96, 128) and page_size % 16 == 0
@@ -1118,6 +1125,89 @@ def paged_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tenso
     if not gated:
         sigmoid_gate(dest, *into)
     return None
+
+
+def attention_rows_ok(rows, ctx, heads: int, kvh: int, dim: int, value_dim: int, k_cache: torch.Tensor, conv_taps: int = 0, window: int = 0) -> bool:
+    """Whether ``attention_rows`` takes a projection's float32 ``rows`` (or ``Partials``): a step of single tokens, bfloat16 caches."""
+    data = rows.data if isinstance(rows, Partials) else rows
+    page_size = k_cache.shape[2]
+    if not (_backend is None and allow_fast_attention and rows_attention and k_cache.dtype == torch.bfloat16 and k_cache.shape[3] == dim == value_dim
+            and dim in (64, 128) and decode_rings(dim, dim, page_size) and heads // kvh <= 16 and ctx.num_requests == ctx.num_single == ctx.num_tokens
+            and data.dtype == torch.float32 and data.shape[-1] % 2 == 0 and data.data_ptr() % 8 == 0 and (data.dim() == 2 or data.shape[0] <= 8)):
+        return False
+    # (a channel's carried inputs have one block: with a convolution the keys are not split, for which 1,024 keys are a microsecond more
+    # than split, and the two launches in front of the attention 5)
+    if conv_taps:
+        bound = 256
+        while bound < ctx.max_context_len:
+            bound *= 2
+        seen = min(bound, window) if window else bound
+        return conv_taps <= 4 and data.dim() == 2 and (seen <= 1024 or decode_rows_padded(ctx.num_tokens) * kvh > 64)
+    return True
+
+
+def attention_rows(rows, col0: int, ctx, group: int, heads: int, kvh: int, dim: int, k_cache: torch.Tensor, v_cache: torch.Tensor, scale: float,
+                   inv_freq: Optional[torch.Tensor], rotary_dim: int, factor: float, cos_sin: Optional[torch.Tensor], window: int = 0,
+                   keep_first: int = 0, chunk: int = 0, sink: Optional[torch.Tensor] = None, norms=None, norm_eps: float = 0.0, conv=None,
+                   into: Optional[tuple] = None) -> Optional[torch.Tensor]:
+    """A step of single tokens from their projection's rows (q | k | v from column ``col0`` on, or ``Partials``) to the heads' outputs:
+    ``causal_conv`` without activation (``conv`` = (weights [taps, channels], state, its column)), a norm per head of q and k (``norms``),
+    ``rope_kv_write`` and ``paged_attention`` in one launch.  ``ctx``: the step; ``group``: its cache group.  Sizes: ``attention_rows_ok``."""
+    parts, data = 1, rows
+    if isinstance(rows, Partials):
+        parts, data = rows.data.shape[0], rows.data.view(-1, rows.data.shape[2])
+    n, stride = ctx.num_tokens, data.shape[1]
+    bt = ctx.block_tables[group]
+    slots = ctx.slot_mapping[group]
+    _dev_ok(data, k_cache, v_cache, bt, ctx.context_lens, ctx.positions, slots, inv_freq, cos_sin, sink)
+    _need(attention_rows_ok(rows, ctx, heads, kvh, dim, v_cache.shape[2], k_cache, 0 if conv is None else conv[0].shape[0], window),
+          "attention_rows: sizes that it does not take")
+    _need(data.shape[0] == parts * n and col0 >= 0 and col0 % 2 == 0 and col0 + (heads + 2 * kvh) * dim <= stride, "attention_rows: bad rows")
+    pages, _, page_size, _ = k_cache.shape
+    _need(k_cache.shape[1] == kvh and tuple(v_cache.shape) == (pages, kvh, dim, page_size) and v_cache.dtype == torch.bfloat16, "attention_rows: bad caches")
+    _need(pages * kvh * page_size < 2 ** 31, "paged_attention: cache pool too large for 32-bit row indices")
+    _need(bt.dtype == torch.int32 and bt.shape[0] == n and ctx.max_context_len <= bt.shape[1] * page_size, "attention_rows: bad block table")
+    _i32(ctx.context_lens, n, "context_lens")
+    _i32(ctx.positions, n, "positions")
+    _i32(slots, n, "slots")
+    if rotary_dim:
+        _need(inv_freq is not None and inv_freq.dtype == torch.float64 and inv_freq.numel() == rotary_dim // 2, "attention_rows: inv_freq must be float64 [rotary_dim / 2]")
+    if cos_sin is not None:
+        _need(cos_sin.dtype == torch.float32 and tuple(cos_sin.shape) == (n, rotary_dim // 2, 2), "attention_rows: table must be float32 [n, rotary_dim / 2, 2]")
+    if sink is not None:
+        _need(sink.dtype == torch.float32 and sink.numel() == heads, "attention_rows: sink must be float32 [heads]")
+    if norms is not None:
+        _dev_ok(*norms)
+        _need(all(w.dtype == torch.float32 and w.numel() == dim for w in norms), "attention_rows: norm weights must be float32 [dim]")
+    conv_w, state, state_off = conv if conv is not None else (None, None, 0)
+    if conv is not None:
+        _dev_ok(conv_w, state)
+        _need(conv_w.dtype == state.dtype == torch.float32 and conv_w.dim() == state.dim() == 2 and conv_w.shape[1] == (heads + 2 * kvh) * dim,
+              "attention_rows: bad convolution")
+        _i32(ctx.state_slots, n, "state_slots")
+    if chunk == 1:
+        chunk, window = 0, 1
+    splits = 1 if conv is not None else _decode_splits(n, heads, kvh, ctx.max_context_len, window, keep_first, chunk, True)
+    scratch = torch.empty((n * heads * splits * (dim + 2),), dtype=torch.float32, device=data.device) if splits > 1 else None
+    if into is not None:
+        gate, gate_col0, gate_scale, out, out_col0, per = into
+        _dev_ok(gate, out)
+        _need(out.dim() == 2 and out.dtype == torch.bfloat16 and out.shape[0] == n and 0 <= out_col0 and out_col0 + heads * dim <= out.shape[1]
+              and per >= 1 and (heads * dim) % per == 0, "attention_rows: bad output rows")
+        _need(gate is None or (gate.dtype == torch.float32 and gate.dim() == 2 and gate.shape[0] == n and 0 <= gate_col0
+                               and gate_col0 + heads * dim // per <= gate.shape[1]), "attention_rows: bad gate rows")
+    else:
+        gate, gate_col0, gate_scale, out_col0, per = None, 0, 1.0, 0, 1
+        out = torch.empty((n, heads * dim), dtype=torch.bfloat16, device=data.device)
+    _call("tp_attention_rows", ctypes.c_void_p(data.data_ptr() + 4 * col0), ctypes.c_size_t(n * stride), stride, parts,
+          _ptr(conv_w), 0 if conv_w is None else conv_w.shape[0], 0 if conv_w is None else conv_w.shape[1], _ptr(state),
+          ctypes.c_size_t(0 if state is None else state.shape[1]), ctypes.c_size_t(state_off), _ptr(ctx.state_slots if conv is not None else None),
+          _ptr(None if norms is None else norms[0]), _ptr(None if norms is None else norms[1]), ctypes.c_float(norm_eps), _ptr(ctx.positions),
+          _ptr(inv_freq), int(rotary_dim), ctypes.c_float(factor), _ptr(cos_sin), _ptr(slots), _ptr(k_cache), _ptr(v_cache), _ptr(bt), bt.shape[1],
+          _ptr(ctx.cu_seqlens), _ptr(ctx.context_lens), _ptr(out), n, heads, kvh, dim, page_size, ctypes.c_float(scale), int(window), int(keep_first),
+          int(chunk), _ptr(sink), int(splits), _ptr(scratch), int(into is not None), _ptr(gate), 0 if gate is None else gate.shape[1], int(gate_col0),
+          int(per), ctypes.c_float(gate_scale), out.shape[1], int(out_col0), _stream())
+    return None if into is not None else out
 
 
 def swiglu(gu: torch.Tensor, out_dtype: torch.dtype) -> torch.Tensor:

@@ -274,16 +274,31 @@ class PagedAttention(Mixer):
                 table = self.position.table(ctx, always=True) if hasattr(self.position, "table") else None
                 q = ops.linear_rope_kv(x, self.wqkv, ctx.positions, ctx.slot_mapping[cache.group], rot[0], rot[1], rot[2],
                                        self.num_heads, self.num_kv_heads, self.head_dim, cache.k, cache.v, table)
-        if q is None:
-            q = self._project_and_rotate(x, ctx, cache, rot)
         if self.w_gates is not None:
             gates = ops.linear(x, self.w_gates, torch.float32)
-        # (a gate over the heads' outputs: of single tokens the kernel that adds the splits of their keys applies it)
+        # (a gate over the heads' outputs: of single tokens the kernel that writes their rows applies it)
         into, gated = {}, None
         if self.gate and self.value_position is None:
-            gated = torch.empty((q.shape[0], self.num_heads * self.value_dim), dtype=q.dtype, device=q.device)
+            gated = torch.empty((x.shape[0], self.num_heads * self.value_dim), dtype=self.dtype, device=self.device)
             into = {"into": (gates, self.gate_col0, 1.0, gated, 0, 1)}
-        if self.extended or self.chunk or self.softcap:
+        a, attended = None, False
+        if q is None:
+            rows = self._project(x, cache, rot)
+            if cache.writes and (rot is not None or type(self.position).__name__ == "NoPosition") and not self.softcap and self.dist_table is None \
+                    and ops.attention_rows_ok(rows, ctx, self.num_heads, self.num_kv_heads, self.head_dim, self.value_dim, cache.k):
+                # single tokens: the attention takes the projection's rows itself
+                inv_freq, rotary_dim, factor = rot if rot is not None else (None, 0, 1.0)
+                table = self.position.table(ctx) if hasattr(self.position, "table") else None
+                norms = {} if self.qk_norm is None else {"norms": (self.q_norm_w, self.k_norm_w), "norm_eps": float(self.qk_norm["eps"])}
+                a = ops.attention_rows(rows, 0, ctx, cache.group, self.num_heads, self.num_kv_heads, self.head_dim, cache.k, cache.v, self.scale,
+                                       inv_freq, rotary_dim, factor, table, int(self.window or 0), self.keep_first, self.chunk, self.sink_w,
+                                       **norms, **into)
+                attended = True
+            else:
+                q = self._rotate(rows, ctx, cache, rot)
+        if attended:
+            pass
+        elif self.extended or self.chunk or self.softcap:
             a = ops.paged_attention(
                 q, cache.k, cache.v, ctx.block_tables[cache.group], ctx.cu_seqlens, ctx.context_lens,
                 ctx.token_req, self.scale, int(self.window or 0), ctx.max_q_len, ctx.max_context_len,
@@ -341,52 +356,32 @@ class PagedAttention(Mixer):
         rows = ops.linear(x, ops.weight_rows(self.wqkv, 0, self.q_dim), torch.float32)
         return ops.qk_store(rows, self.q_bias, None, None, self.num_heads, self.num_kv_heads, self.head_dim, None, None, self.dtype)
 
-    def _project_extended(self, x, ctx, cache, rot):
-        """q of a projection with a norm per head and/or values of their own size: the float32 rows are normed in
-        place, then rotated (if the position part rotates) and stored by the cache-write kernel."""
-        if rot is None and type(self.position).__name__ != "NoPosition":
+    def _project(self, x, cache, rot):
+        """The projection's float32 rows q | k | v (of a call that reads another call's cache q alone), or their ``Partials`` where a
+        rotation follows that adds them."""
+        if self.extended and rot is None and type(self.position).__name__ != "NoPosition":
             raise ValueError("attention: qk_norm, value_dim, sink and keep_first need a rotary position part or none")
+        w = self.wqkv if cache.writes else ops.weight_rows(self.wqkv, 0, self.q_dim)
+        return ops.linear(x, w, torch.float32, partial_ok=rot is not None and not self.extended)
+
+    def _rotate(self, qkv, ctx, cache, rot):
+        """q (rotated, [n, heads, head_dim]) of the projection's rows; k and v go to the cache.  With a norm per head the rows are
+        normed in place first; values may have a size of their own."""
         writes = cache.writes
-        w = self.wqkv if writes else ops.weight_rows(self.wqkv, 0, self.q_dim)
-        qkv = ops.linear(x, w, torch.float32)
-        if self.qk_norm is not None:
+        if self.extended and self.qk_norm is not None:
             ops.head_rmsnorm(qkv, 0, self.num_heads, self.q_norm_w, self.q_dim, self.num_kv_heads if writes else 0, self.k_norm_w,
                              self.head_dim, float(self.qk_norm["eps"]))
         inv_freq, rotary_dim, factor, table = None, 0, 1.0, None
         if rot is not None:
             inv_freq, rotary_dim, factor = rot
             table = self.position.table(ctx) if hasattr(self.position, "table") else None
+        elif not self.extended:
+            q2, k2 = self.position.apply(qkv[:, : self.q_dim], qkv[:, self.q_dim: self.q_dim + self.kv_dim] if writes else None, ctx.positions)
+            qkv = torch.cat([q2, k2, qkv[:, self.q_dim + self.kv_dim:]], dim=1).contiguous() if writes else q2.contiguous()
+        sizes = {"value_dim": self.value_dim, "pad_dim": self.key_dim} if self.extended else {}
         return ops.rope_kv_write(qkv, ctx.positions, ctx.slot_mapping[cache.group] if writes else None, inv_freq, rotary_dim, factor,
                                  self.num_heads, self.num_kv_heads, self.head_dim, cache.k if writes else None,
-                                 cache.v if writes else None, self.dtype, table, value_dim=self.value_dim, pad_dim=self.key_dim)
-
-    def _project_and_rotate(self, x, ctx, cache, rot):
-        """q (rotated, [n, heads, head_dim]) of the projection; k and v go to the cache."""
-        # (with a rotary position the next kernel may add the projection's partial sums itself)
-        if self.extended:
-            return self._project_extended(x, ctx, cache, rot)
-        if cache.writes:
-            qkv = ops.linear(x, self.wqkv, torch.float32, partial_ok=rot is not None)
-        else:
-            # A call that reads another call's cache needs queries only.
-            qkv = ops.linear(x, ops.weight_rows(self.wqkv, 0, self.q_dim), torch.float32, partial_ok=rot is not None)
-        if rot is None:
-            q = qkv[:, : self.q_dim]
-            k = qkv[:, self.q_dim: self.q_dim + self.kv_dim] if cache.writes else None
-            q2, k2 = self.position.apply(q, k, ctx.positions)
-            if cache.writes:
-                qkv = torch.cat([q2, k2, qkv[:, self.q_dim + self.kv_dim:]], dim=1).contiguous()
-            else:
-                qkv = q2.contiguous()
-            inv_freq, rotary_dim, factor, table = None, 0, 1.0, None
-        else:
-            inv_freq, rotary_dim, factor = rot
-            table = self.position.table(ctx) if hasattr(self.position, "table") else None
-        q = ops.rope_kv_write(
-            qkv, ctx.positions, ctx.slot_mapping[cache.group] if cache.writes else None,
-            inv_freq, rotary_dim, factor, self.num_heads, self.num_kv_heads, self.head_dim,
-            cache.k if cache.writes else None, cache.v if cache.writes else None, self.dtype, table)
-        return q
+                                 cache.v if writes else None, self.dtype, table, **sizes)
 
 
 register_part("mixer", "attention", PagedAttention)
@@ -517,16 +512,24 @@ class ConvAttention(BranchMixer):
     def run(self, proj, col0, ctx, cache, out, out_col0, scale):
         if not cache.writes:
             raise ValueError("conv_attention: a call that reads another call's cache is not supported")
-        qkv, qkv_col0 = proj, col0
-        if self.taps:
-            qkv_col0 = 0
-            qkv = ops.causal_conv(proj, col0, self.channels, self.conv_w, None, cache.state, ctx.cu_seqlens, ctx.token_req,
-                                  ctx.state_slots, ctx.num_requests, state_off=self.state_off, act=False, max_run=ctx.max_q_len)
         rot = self.position.rotary()
         inv_freq, rotary_dim, factor, table = None, 0, 1.0, None
         if rot is not None:
             inv_freq, rotary_dim, factor = rot
             table = self.position.table(ctx) if hasattr(self.position, "table") else None
+        into = (proj if self.gate else None, col0 + self.channels, scale, out, out_col0, self.gate_per if self.gate else 1)
+        if out.dtype == torch.bfloat16 and ops.attention_rows_ok(proj, ctx, self.num_heads, self.num_kv_heads, self.head_dim, self.value_dim,
+                                                                 cache.k, self.taps, int(self.window or 0)):
+            ops.attention_rows(proj, col0, ctx, cache.group, self.num_heads, self.num_kv_heads, self.head_dim, cache.k, cache.v, self.scale,
+                               inv_freq, rotary_dim, factor, table, int(self.window or 0), norms=self.norms,
+                               norm_eps=float(self.qk_norm["eps"]) if self.qk_norm is not None else 0.0,
+                               conv=(self.conv_w, cache.state, self.state_off) if self.taps else None, into=into)
+            return
+        qkv, qkv_col0 = proj, col0
+        if self.taps:
+            qkv_col0 = 0
+            qkv = ops.causal_conv(proj, col0, self.channels, self.conv_w, None, cache.state, ctx.cu_seqlens, ctx.token_req,
+                                  ctx.state_slots, ctx.num_requests, state_off=self.state_off, act=False, max_run=ctx.max_q_len)
         if self.rows_path:
             q = ops.qkv_rows(qkv, ctx.positions, ctx.slot_mapping[cache.group], self.num_heads, self.num_kv_heads, self.head_dim,
                              self.value_dim, cache.k, cache.v, inv_freq, rotary_dim, factor, table, norms=self.norms,
@@ -537,8 +540,7 @@ class ConvAttention(BranchMixer):
                                   self.num_kv_heads, self.head_dim, cache.k, cache.v, self.dtype, table, value_dim=self.value_dim,
                                   pad_dim=self.key_dim)
         ops.paged_attention(q, cache.k, cache.v, ctx.block_tables[cache.group], ctx.cu_seqlens, ctx.context_lens,
-                            ctx.token_req, self.scale, int(self.window or 0), ctx.max_q_len, ctx.max_context_len, ctx.num_single,
-                            into=(proj if self.gate else None, col0 + self.channels, scale, out, out_col0, self.gate_per if self.gate else 1))
+                            ctx.token_req, self.scale, int(self.window or 0), ctx.max_q_len, ctx.max_context_len, ctx.num_single, into=into)
 
 
 register_part("mixer", "conv_attention", ConvAttention)

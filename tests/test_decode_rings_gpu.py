@@ -1,5 +1,7 @@
 """Single tokens' attention with keys and values on their way to LDS: contexts at the edges of steps, waves and rings, keys that are
 split or not, a block or more a CU, masks, and the gate behind the heads, against the plain operation."""
+from types import SimpleNamespace
+
 import pytest
 import torch
 
@@ -48,3 +50,67 @@ def test_gate_behind_the_heads(ctx, page, per):
         ops.sigmoid_gate(plain, gate, 5, 0.75, want, 8, per)
         assert ops.paged_attention(*args, into=(gate, 5, 0.75, got, 8, per)) is None
         assert torch.equal(got, want)
+
+
+def _step(ctx_lens, kv, d, page, g):
+    """A step of one token for each request: what the parts read of it, and caches with every earlier key in place."""
+    n, width = len(ctx_lens), -(-max(ctx_lens) // page) + 1
+    tables = torch.randperm(n * width, generator=g).to(torch.int32).view(n, width)
+    cl = torch.tensor(ctx_lens, dtype=torch.int32)
+    slots = torch.stack([tables[i, (c - 1) // page] * page + (c - 1) % page for i, c in enumerate(ctx_lens)]).to(torch.int32)
+    ctx = SimpleNamespace(num_tokens=n, num_requests=n, num_single=n, max_q_len=1, max_context_len=max(ctx_lens), positions=(cl - 1).to(DEV),
+                          context_lens=cl.to(DEV), cu_seqlens=torch.arange(n + 1, dtype=torch.int32, device=DEV), block_tables=[tables.to(DEV)],
+                          slot_mapping=[slots.to(DEV)], state_slots=torch.randperm(n + 2, generator=g)[:n].to(torch.int32).to(DEV))
+    ctx.token_req = ctx.cu_seqlens[:n]
+    k = torch.randn(n * width, kv, page, d, generator=g).to(DEV).bfloat16()
+    v = torch.randn(n * width, kv, d, page, generator=g).to(DEV).bfloat16()
+    return ctx, k, v
+
+
+@pytest.mark.parametrize("heads,kv,d,page", [(6, 2, 128, 16), (8, 8, 64, 32), (16, 1, 64, 16)])
+@pytest.mark.parametrize("ctx_lens", [[1, 2, 31, 32, 33, 64, 65], [257, 16, 17, 300], [2000, 700, 1]])
+@pytest.mark.parametrize("how", ["plain", "partials", "conv", "norms", "gate", "half"])
+def test_attention_from_the_projections_rows(heads, kv, d, page, ctx_lens, how):
+    """One launch against the kernels it stands for: the same cache, carried inputs and outputs, bit for bit; a norm per head sums its
+    squares in another order, which may move a rounding to bfloat16."""
+    ops = _ops()
+    g = torch.Generator().manual_seed(heads + d + len(ctx_lens))
+    ctx, k, v = _step(ctx_lens, kv, d, page, g)
+    n, width, col0 = len(ctx_lens), (heads + 2 * kv) * d, 0 if how == "partials" else 6
+    rows = torch.randn(3 if how == "partials" else 1, n, width + col0, generator=g).to(DEV)
+    freq = (10000.0 ** -torch.arange(0, 1, 2.0 / d, dtype=torch.float64)).to(DEV)
+    rotary = d // 2 if how == "half" else d
+    freq = freq[: rotary // 2].contiguous()
+    table = ops.rope_table(ctx.positions, freq, rotary, 1.25) if how == "conv" else None
+    taps, norms = 3, tuple(torch.rand(d, generator=g).add(0.5).to(DEV) for _ in "qk") if how == "norms" else None
+    conv_w = torch.randn(taps, width, generator=g).to(DEV)
+    state = torch.randn(n + 2, 4 + (taps - 1) * width, generator=g).to(DEV)
+    gate = torch.randn(n, heads * d, generator=g).to(DEV)
+    if not ops.attention_rows_ok(rows[0], ctx, heads, kv, d, d, k, taps if how == "conv" else 0):
+        assert how == "conv" and max(ctx_lens) > 1024
+        pytest.skip("keys that are split keep the convolution's own launch")
+    k2, v2, state2 = k.clone(), v.clone(), state.clone()
+    if how == "partials":
+        given = ops.Partials(rows)
+        plain = ops.Partials(rows.clone())
+    else:
+        given, plain = rows[0], rows[0, :, col0:].contiguous()
+    if how == "conv":
+        plain = ops.causal_conv(plain, 0, width, conv_w, None, state2, ctx.cu_seqlens, ctx.token_req, ctx.state_slots, n, state_off=4, act=False, max_run=1)
+    if how == "norms":
+        ops.head_rmsnorm(plain, 0, heads, norms[0], heads * d, kv, norms[1], d, 1e-6)
+    q = ops.rope_kv_write(plain, ctx.positions, ctx.slot_mapping[0], freq, rotary, 1.25, heads, kv, d, k2, v2, torch.bfloat16, table)
+    window, scale = (40 if how == "half" else 0), d ** -0.5
+    args = (q, k2, v2, ctx.block_tables[0], ctx.cu_seqlens, ctx.context_lens, ctx.token_req, scale, window, 1, ctx.max_context_len, n)
+    into = [torch.zeros(n, heads * d, dtype=torch.bfloat16, device=DEV) for _ in "ab"]
+    want = ops.paged_attention(*args, into=(gate, 0, 0.5, into[0], 0, 1) if how == "gate" else None)
+    got = ops.attention_rows(given, col0, ctx, 0, heads, kv, d, k, v, scale, freq, rotary, 1.25, table, window, norms=norms, norm_eps=1e-6,
+                             conv=(conv_w, state, 4) if how == "conv" else None, into=(gate, 0, 0.5, into[1], 0, 1) if how == "gate" else None)
+    if how == "gate":
+        want, got = into
+    assert torch.equal(v, v2) and torch.equal(state, state2)
+    if how == "norms":
+        assert float((k.float() - k2.float()).abs().max()) <= 2.0 ** -8 * float(k2.float().abs().max())
+        assert float((got.float() - want.float()).norm()) <= 2.0 ** -8 * float(want.float().norm())
+    else:
+        assert torch.equal(k, k2) and torch.equal(got, want)

@@ -26,6 +26,7 @@
 #include <math.h>
 
 #include "common.h"
+#include "step_mixer.h"
 
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
@@ -1284,7 +1285,7 @@ __device__ inline int decode_steps(const AttnArgs& a, int ctx, int& first, int& 
 // bank apart): the answer where the keys are not split, else the split's partial result.  h0: the first head, ncols: how many.
 template <int DV, int WAVES>
 __device__ inline void decode_merge(const AttnArgs& a, float* red, int wave, int lane, float m, float l, const f32x4_t (&o)[DV / 16],
-                                    int r, int q_start, int h0, int ncols) {
+                                    int r, int q_start, int split, int h0, int ncols) {
   const int g = lane >> 4, c = lane & 15;
   float* stat = red + WAVES * DV * 17;
   l += __shfl_xor(l, 16, 64);
@@ -1320,7 +1321,7 @@ __device__ inline void decode_merge(const AttnArgs& a, float* red, int wave, int
         a.out[((size_t)q_start * a.n_heads + hd) * DV + d] = float_to_bf16(acc / lsum);
       continue;
     }
-    float* part = a.scratch + (((size_t)r * a.n_heads + hd) * a.num_splits + blockIdx.z) * (DV + 2);
+    float* part = a.scratch + (((size_t)r * a.n_heads + hd) * a.num_splits + split) * (DV + 2);
     part[d] = acc;
     if (d == 0) {
       part[DV] = mg;
@@ -1372,7 +1373,7 @@ __global__ __launch_bounds__(256) void attn_decode_kernel(AttnArgs a) {
   // fragment registers halve the occupancy and the kernel gets slower, not faster.)
   for (int s = s_begin + wave; s < s_end; s += 4)
     attn_step<D, DV, 1, MODE>(a, table, kvh, ctx, s < kept_steps ? s * 32 : first + (s - kept_steps) * 32, qf, qpos, m, l, o, bias_row);
-  decode_merge<DV, 4>(a, red, wave, lane, m[0], l[0], o[0], r, q_start, kvh * group + h0, ncols);
+  decode_merge<DV, 4>(a, red, wave, lane, m[0], l[0], o[0], r, q_start, blockIdx.z, kvh * group + h0, ncols);
 }
 
 // The same with keys and values on their way to LDS instead of registers (the sizes and pages of attn_prefill_lds_kernel, whose
@@ -1387,8 +1388,9 @@ __global__ __launch_bounds__(256) void attn_decode_kernel(AttnArgs a) {
 // that holds it is read, into that step's place in LDS.  The rows travel beside the first keys; a launch or two between the
 // projection and the attention are gone: Bomotar's decode step, four layers with a convolution, 377 -> 361 us; 28 layers of the 3B
 // shape with 48 requests, three parts of K, 3,219 -> 3,187.
-template <int D, int DV, int MODE, int WAVES, int NB, bool ROWS = false>
-__global__ __launch_bounds__(WAVES * 64) void attn_decode_lds_kernel(AttnArgs a, RowsIn in) {
+// (bx: key head and block of heads, r: request, split: its part of the keys)
+template <int D, int DV, int MODE, int WAVES, int NB, bool ROWS>
+__device__ inline void attn_decode_lds_block(const AttnArgs& a, const RowsIn& in, int bx, int r, int split) {
   constexpr int C = D / 8;             // 16-byte chunks per key row
   constexpr int SH = C == 16 ? 0 : (C == 8 || C == 24 ? 1 : 2);
   constexpr int KI = D / 16, VI = DV / 16, STAGE = (KI + VI) * 1024;
@@ -1401,12 +1403,12 @@ __global__ __launch_bounds__(WAVES * 64) void attn_decode_lds_kernel(AttnArgs a,
   const int g = lane >> 4, c = lane & 15;
   const int group = a.n_heads / a.n_kv;
   const int hblocks = (group + 15) / 16;
-  const int kvh = blockIdx.x / hblocks;
-  const int h0 = (blockIdx.x % hblocks) * 16;
+  const int kvh = bx / hblocks;
+  const int h0 = (bx % hblocks) * 16;
   const int ncols = min(16, group - h0);
   const int head = kvh * group + h0 + min(c, ncols - 1);
   static_assert(MODE != MODE_BIAS, "a table read inside the loop would wait for the copies into LDS");
-  const int r = blockIdx.y, q_start = a.all_single ? r : a.cu_seqlens[r];
+  const int q_start = a.all_single ? r : a.cu_seqlens[r];
   if (!a.all_single && a.cu_seqlens[r + 1] - q_start != 1) return;
   const int ctx = a.context_lens[r];
   u32x4_t qv[D / 32];
@@ -1475,7 +1477,7 @@ __global__ __launch_bounds__(WAVES * 64) void attn_decode_lds_kernel(AttnArgs a,
   int first, kept_steps;
   const int steps = decode_steps(a, ctx, first, kept_steps);
   const int per_split = (steps + a.num_splits - 1) / a.num_splits;
-  const int s_begin = blockIdx.z * per_split, s_end = min(steps, s_begin + per_split);
+  const int s_begin = split * per_split, s_end = min(steps, s_begin + per_split);
   const int n = max(0, (s_end - s_begin - wave + WAVES - 1) / WAVES);      // this wave's steps
   auto key0 = [&](int i) {
     const int s = s_begin + wave + i * WAVES;
@@ -1677,7 +1679,23 @@ __global__ __launch_bounds__(WAVES * 64) void attn_decode_lds_kernel(AttnArgs a,
     st = st + 1 == NB ? 0 : st + 1;
   }
   __syncthreads();     // (every wave's ring is empty)
-  decode_merge<DV, WAVES>(a, (float*)stages, wave, lane, m[0], l[0], o[0], r, q_start, kvh * group + h0, ncols);
+  decode_merge<DV, WAVES>(a, (float*)stages, wave, lane, m[0], l[0], o[0], r, q_start, split, kvh * group + h0, ncols);
+}
+
+template <int D, int DV, int MODE, int WAVES, int NB, bool ROWS = false>
+__global__ __launch_bounds__(WAVES * 64) void attn_decode_lds_kernel(AttnArgs a, RowsIn in) {
+  attn_decode_lds_block<D, DV, MODE, WAVES, NB, ROWS>(a, in, blockIdx.x, blockIdx.y, blockIdx.z);
+}
+
+// The attention of single tokens and the recurrent mixer that stands beside it in one launch: neither fills the chip (32 and 64 blocks
+// for four requests of Bomotar at width 2,048), and each is a chain of trips to memory.  Blocks of 512 threads, the attention's first.
+template <int D, int NB, int KIND, int KS>
+__global__ __launch_bounds__(512) void attn_beside_step_kernel(AttnArgs a, RowsIn in, StepArgs st, int n, int splits) {
+  const int mine = a.n_kv * n * splits, b = blockIdx.x;
+  if (b < mine)
+    attn_decode_lds_block<D, D, MODE_PLAIN, 8, NB, true>(a, in, b % a.n_kv, b / a.n_kv % n, b / (a.n_kv * n));
+  else
+    mixer_step_block<KIND, KS, bf16_t>(st, (b - mine) % n, (b - mine) / n);
 }
 
 // out[token, head, :] = sum_s 2^(m_s - m) O_s / sum_s 2^(m_s - m) l_s, splits in ascending order.
@@ -1962,7 +1980,8 @@ static AttnArgs decode_args(const bf16_t* k_cache, const bf16_t* v_cache, const 
 }
 
 // Single tokens from their projection's rows (see RowsIn and attn_decode_lds_kernel): n requests of one token each, heads of 64 or 128
-// elements, values alike, at most 16 heads a key head, pages of a power of two from 16 on.  With num_splits > 1 scratch of n * n_heads *
+// elements, values alike, at most 16 heads a key head, pages of a power of two from 16 on.  beside: a step that tp_delta_step or
+// tp_linear_step wrote down, of the same requests, to run in the same launch (nullptr: none).  With num_splits > 1 scratch of n * n_heads *
 // num_splits * (dim + 2) floats, and no convolution (a channel's carried inputs have one block).  gated: out as of tp_paged_attention
 // with allow_fast 2.
 extern "C" int tp_attention_rows(const float* rows, size_t part_stride, int stride, int parts, const float* conv_w, int taps, int channels,
@@ -1972,7 +1991,7 @@ extern "C" int tp_attention_rows(const float* rows, size_t part_stride, int stri
                                  const int* cu_seqlens, const int* context_lens, void* out, int n, int n_heads, int n_kv, int dim, int page_size,
                                  float scale, int window, int keep_first, int chunk, const float* sink, int num_splits, float* scratch, int gated,
                                  const float* gate, int gate_stride, int gate_col0, int gate_per, float gate_scale, int out_stride, int out_col0,
-                                 hipStream_t s) {
+                                 const void* beside, hipStream_t s) {
   TP_REQUIRE(n >= 0 && n <= 65535 && n_kv > 0 && n_heads > 0 && n_heads <= 65535 && n_heads % n_kv == 0 && n_heads / n_kv <= 16 && (dim == 64 || dim == 128),
              "attention_rows: bad heads (%d of %d, %d key heads)", n_heads, dim, n_kv);
   TP_REQUIRE(page_size >= 16 && (page_size & (page_size - 1)) == 0 && parts >= 1 && parts <= ROWS_PARTS && stride % 2 == 0 && part_stride % 2 == 0 &&
@@ -2002,7 +2021,23 @@ extern "C" int tp_attention_rows(const float* rows, size_t part_stride, int stri
   const dim3 grid(n_kv, n, num_splits);
   const bool wide = num_splits == 1 && (long)n_kv * n <= 256;
 #define ROWS_KERNEL(D_, W_, NB_) hipLaunchKernelGGL((attn_decode_lds_kernel<D_, D_, MODE_PLAIN, W_, NB_, true>), grid, dim3(W_ * 64), 0, s, a, in)
-  if (dim == 128 && wide) ROWS_KERNEL(128, 8, 1);
+  if (beside != nullptr) {
+    const PreparedStep* st = (const PreparedStep*)beside;
+    TP_REQUIRE(st->n == n && (st->kind == STEP_DELTA || st->kind == STEP_LINEAR), "attention_rows: a step of other requests beside it");
+    const long blocks = (long)n_kv * n * num_splits + (long)n * st->args.heads;
+    TP_REQUIRE(blocks < 0x7fffffffL, "attention_rows: too many blocks");
+    const bool low = st->args.dim <= 64;
+#define BESIDE(D_, NB_, KIND_)                                                                                                                 \
+  do {                                                                                                                                         \
+    if (low) hipLaunchKernelGGL((attn_beside_step_kernel<D_, NB_, KIND_, 8>), dim3((unsigned)blocks), dim3(512), 0, s, a, in, st->args, n, num_splits); \
+    else hipLaunchKernelGGL((attn_beside_step_kernel<D_, NB_, KIND_, 16>), dim3((unsigned)blocks), dim3(512), 0, s, a, in, st->args, n, num_splits);    \
+  } while (0)
+    if (dim == 128 && st->kind == STEP_DELTA) BESIDE(128, 1, STEP_DELTA);
+    else if (dim == 128) BESIDE(128, 1, STEP_LINEAR);
+    else if (st->kind == STEP_DELTA) BESIDE(64, 2, STEP_DELTA);
+    else BESIDE(64, 2, STEP_LINEAR);
+#undef BESIDE
+  } else if (dim == 128 && wide) ROWS_KERNEL(128, 8, 1);
   else if (dim == 128) ROWS_KERNEL(128, 4, 1);
   else if (wide) ROWS_KERNEL(64, 8, 2);
   else ROWS_KERNEL(64, 4, 2);

@@ -50,6 +50,7 @@ class _Library:
             lib.tp_last_error.restype = ctypes.c_char_p
             lib.tp_linear_f32_scratch.restype = ctypes.c_size_t
             lib.tp_delta_scan_scratch.restype = ctypes.c_size_t
+            lib.tp_step_prepared_size.restype = ctypes.c_size_t
             cls._lib = lib
             cls.path = path
         return cls._lib
@@ -1146,13 +1147,24 @@ def attention_rows_ok(rows, ctx, heads: int, kvh: int, dim: int, value_dim: int,
     return True
 
 
+def _rows_splits(ctx, heads: int, kvh: int, window: int, keep_first: int, chunk: int, conv: bool, beside: bool) -> int:
+    splits = 1 if conv else _decode_splits(ctx.num_tokens, heads, kvh, ctx.max_context_len, window, keep_first, chunk, True)
+    return -(-splits // 2) if beside else splits        # (blocks of eight waves instead of four)
+
+
+def attention_beside_ok(ctx, heads: int, kvh: int, window: int, conv_taps: int, step_heads: int) -> bool:
+    """Whether ``attention_rows`` should run a recurrent mixer's step in its launch: while the blocks of both have a CU each."""
+    return ctx.num_tokens * (kvh * _rows_splits(ctx, heads, kvh, window, 0, 0, conv_taps > 0, True) + step_heads) <= 256
+
+
 def attention_rows(rows, col0: int, ctx, group: int, heads: int, kvh: int, dim: int, k_cache: torch.Tensor, v_cache: torch.Tensor, scale: float,
                    inv_freq: Optional[torch.Tensor], rotary_dim: int, factor: float, cos_sin: Optional[torch.Tensor], window: int = 0,
                    keep_first: int = 0, chunk: int = 0, sink: Optional[torch.Tensor] = None, norms=None, norm_eps: float = 0.0, conv=None,
-                   into: Optional[tuple] = None) -> Optional[torch.Tensor]:
+                   into: Optional[tuple] = None, beside=None) -> Optional[torch.Tensor]:
     """A step of single tokens from their projection's rows (q | k | v from column ``col0`` on, or ``Partials``) to the heads' outputs:
     ``causal_conv`` without activation (``conv`` = (weights [taps, channels], state, its column)), a norm per head of q and k (``norms``),
-    ``rope_kv_write`` and ``paged_attention`` in one launch.  ``ctx``: the step; ``group``: its cache group.  Sizes: ``attention_rows_ok``."""
+    ``rope_kv_write`` and ``paged_attention`` in one launch.  ``beside``: a recurrent mixer's step of the same requests, written down by
+    ``delta_step`` or ``linear_step``, which runs in that launch too.  ``ctx``: the step; ``group``: its cache group.  Sizes: ``attention_rows_ok``."""
     parts, data = 1, rows
     if isinstance(rows, Partials):
         parts, data = rows.data.shape[0], rows.data.view(-1, rows.data.shape[2])
@@ -1187,7 +1199,7 @@ def attention_rows(rows, col0: int, ctx, group: int, heads: int, kvh: int, dim: 
         _i32(ctx.state_slots, n, "state_slots")
     if chunk == 1:
         chunk, window = 0, 1
-    splits = 1 if conv is not None else _decode_splits(n, heads, kvh, ctx.max_context_len, window, keep_first, chunk, True)
+    splits = _rows_splits(ctx, heads, kvh, window, keep_first, chunk, conv is not None, beside is not None)
     scratch = torch.empty((n * heads * splits * (dim + 2),), dtype=torch.float32, device=data.device) if splits > 1 else None
     if into is not None:
         gate, gate_col0, gate_scale, out, out_col0, per = into
@@ -1206,7 +1218,7 @@ def attention_rows(rows, col0: int, ctx, group: int, heads: int, kvh: int, dim: 
           _ptr(inv_freq), int(rotary_dim), ctypes.c_float(factor), _ptr(cos_sin), _ptr(slots), _ptr(k_cache), _ptr(v_cache), _ptr(bt), bt.shape[1],
           _ptr(ctx.cu_seqlens), _ptr(ctx.context_lens), _ptr(out), n, heads, kvh, dim, page_size, ctypes.c_float(scale), int(window), int(keep_first),
           int(chunk), _ptr(sink), int(splits), _ptr(scratch), int(into is not None), _ptr(gate), 0 if gate is None else gate.shape[1], int(gate_col0),
-          int(per), ctypes.c_float(gate_scale), out.shape[1], int(out_col0), _stream())
+          int(per), ctypes.c_float(gate_scale), out.shape[1], int(out_col0), beside, _stream())
     return None if into is not None else out
 
 
@@ -2259,13 +2271,19 @@ def _step_state(n, state, token_req, state_slots, out, out_col0, columns, what):
     _i32(state_slots, n, "state_slots")
 
 
+def step_buffer():
+    """Host memory for a step that is written down (``prepared``)."""
+    return ctypes.create_string_buffer(int(library().tp_step_prepared_size()))
+
+
 def delta_step(proj: torch.Tensor, col0: int, beta_col0: int, a_col0: int, g_col0: int, conv_w: torch.Tensor, a2_t: torch.Tensor,
                g2_t: torch.Tensor, a_log: torch.Tensor, dt_bias: torch.Tensor, norm_w: torch.Tensor, state: torch.Tensor, conv_off: int,
                state_off: int, token_req: torch.Tensor, state_slots: torch.Tensor, heads: int, dim: int, vdim: int, q_scale: float,
-               unit_eps: float, norm_eps: float, scale: float, out: torch.Tensor, out_col0: int) -> None:
+               unit_eps: float, norm_eps: float, scale: float, out: torch.Tensor, out_col0: int, prepared=None) -> None:
     """One token a request of a gated delta rule with as many key heads as heads: ``causal_conv`` (with SiLU) over the columns
     q | k | v from ``col0`` on, ``lowrank_up`` for the decay and the gate, ``delta_scan`` and ``head_norm_gate``, in one launch and
-    with the same bits (``mixer_step_ok`` says for which sizes)."""
+    with the same bits (``mixer_step_ok`` says for which sizes).  ``prepared`` (``step_buffer()``): the step is written down there for
+    ``attention_rows`` instead of launched; its tensors have to live until that call."""
     _dev_ok(proj, conv_w, a2_t, g2_t, a_log, dt_bias, norm_w, state, token_req, state_slots, out)
     n, taps = proj.shape[0], conv_w.shape[0]
     _step_state(n, state, token_req, state_slots, out, out_col0, heads * vdim, "delta_step")
@@ -2279,7 +2297,7 @@ def delta_step(proj: torch.Tensor, col0: int, beta_col0: int, a_col0: int, g_col
           g2_t.shape[0], _ptr(conv_w), taps, _ptr(a2_t), _ptr(g2_t), _ptr(a_log), _ptr(dt_bias), _ptr(norm_w), _ptr(state),
           ctypes.c_size_t(state.shape[1]), ctypes.c_size_t(conv_off), ctypes.c_size_t(state_off), _ptr(token_req), _ptr(state_slots), _ptr(out),
           _dt(out), ctypes.c_size_t(out.shape[1]), int(out_col0), n, int(heads), int(dim), int(vdim), ctypes.c_float(q_scale),
-          ctypes.c_float(unit_eps), ctypes.c_float(norm_eps), ctypes.c_float(scale), _stream())
+          ctypes.c_float(unit_eps), ctypes.c_float(norm_eps), ctypes.c_float(scale), prepared, _stream())
 
 
 def general_delta_step(proj: torch.Tensor, col0: int, gate_col0: int, w_col0: int, w2_t: torch.Tensor, w0: torch.Tensor, rate: float,
@@ -2304,10 +2322,10 @@ def general_delta_step(proj: torch.Tensor, col0: int, gate_col0: int, w_col0: in
 def linear_step(q, k, v, x, w2_t: torch.Tensor, mode: str, bias: torch.Tensor, rate: float, in_act: Optional[str],
                 bonus: Optional[torch.Tensor], q_scale: float, gate, norm_w: torch.Tensor, norm_eps: float, scale: float, state: torch.Tensor,
                 state_off: int, token_req: torch.Tensor, state_slots: torch.Tensor, heads: int, dim: int, vdim: int, out: torch.Tensor,
-                out_col0: int) -> None:
+                out_col0: int, prepared=None) -> None:
     """One token a request of a linear recurrence: ``lowrank_up`` (``mode`` of rows ``x``) for the decay, ``linear_scan`` and
     ``head_norm_gate`` with the SiLU of the raw gate columns, in one launch and with the same bits.  ``q``, ``k``, ``v``, ``x`` and
-    ``gate`` are pairs (float32 rows, first column)."""
+    ``gate`` are pairs (float32 rows, first column).  ``prepared``: as of ``delta_step``."""
     _need(mode in ("rate_sigmoid", "exp_exp", "root_sigmoid") and in_act in (None, "tanh"), "linear_step: bad decay")
     _dev_ok(q[0], k[0], v[0], x[0], gate[0], w2_t, bias, bonus, norm_w, state, token_req, state_slots, out)
     n = q[0].shape[0]
@@ -2325,7 +2343,7 @@ def linear_step(q, k, v, x, w2_t: torch.Tensor, mode: str, bias: torch.Tensor, r
           LOWRANK_MODES[mode], 1 if in_act == "tanh" else 0, ctypes.c_float(rate), _ptr(bonus), ctypes.c_float(q_scale), at(gate), wide(gate),
           GATE_ACTS["silu"], _ptr(norm_w), int(norm_w.numel() == heads * vdim and heads > 1), _ptr(state), ctypes.c_size_t(state.shape[1]),
           ctypes.c_size_t(state_off), _ptr(token_req), _ptr(state_slots), _ptr(out), _dt(out), ctypes.c_size_t(out.shape[1]), int(out_col0), n,
-          int(heads), int(dim), int(vdim), ctypes.c_float(norm_eps), ctypes.c_float(scale), _stream())
+          int(heads), int(dim), int(vdim), ctypes.c_float(norm_eps), ctypes.c_float(scale), prepared, _stream())
 
 
 # ---------------------------------------------------------------------------------

@@ -160,6 +160,14 @@ class BranchMixer(Mixer):
     def run(self, proj, col0, ctx, cache, out, out_col0, scale) -> None:
         raise NotImplementedError
 
+    def takes_beside(self, proj, ctx, cache, out, heads: int) -> bool:
+        """Whether ``run`` would take another branch's prepared step (``beside``), a block for each of ``heads`` heads, into its launch."""
+        return False
+
+    def prepare(self, proj, col0, ctx, cache, out, out_col0, scale):
+        """``run`` as a step written down for another branch's launch, or None where it is no such step (bfloat16 results)."""
+        return None
+
     def state_spec(self):
         n = self.state_floats()
         return StateSpec((n,), torch.float32) if n else None

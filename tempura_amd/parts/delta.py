@@ -85,14 +85,23 @@ class GatedDeltaMixer(BranchMixer):
         self.g1_col = self.a1_col + a1.shape[0]
         return torch.cat([self._to_device(t) for t in rows], dim=0).contiguous(), self._to_device(get(w["o"]))
 
-    def run(self, proj, col0, ctx, cache, out, out_col0, scale):
-        if self.num_heads == self.num_kv_heads and ops.mixer_step_ok(
+    def _step(self, proj, col0, ctx, cache, out, out_col0, scale, prepared=None) -> bool:
+        if not (self.num_heads == self.num_kv_heads and ops.mixer_step_ok(
                 proj.shape[0], ctx.max_q_len, self.num_heads, self.head_dim, self.value_dim, (self.a2_t.shape[0], self.g2_t.shape[0]), cache.state,
-                self.state_off + self.conv_floats, out, out_col0):
-            ops.delta_step(proj, col0, col0 + self.beta_col, col0 + self.a1_col, col0 + self.g1_col, self.conv_w, self.a2_t, self.g2_t,
-                           self.a_log, self.dt_bias, self.norm_w, cache.state, self.state_off, self.state_off + self.conv_floats,
-                           ctx.token_req, ctx.state_slots, self.num_heads, self.head_dim, self.value_dim, self.q_scale, self.unit_eps,
-                           self.norm_eps, scale, out, out_col0)
+                self.state_off + self.conv_floats, out, out_col0)):
+            return False
+        ops.delta_step(proj, col0, col0 + self.beta_col, col0 + self.a1_col, col0 + self.g1_col, self.conv_w, self.a2_t, self.g2_t,
+                       self.a_log, self.dt_bias, self.norm_w, cache.state, self.state_off, self.state_off + self.conv_floats,
+                       ctx.token_req, ctx.state_slots, self.num_heads, self.head_dim, self.value_dim, self.q_scale, self.unit_eps,
+                       self.norm_eps, scale, out, out_col0, prepared)
+        return True
+
+    def prepare(self, proj, col0, ctx, cache, out, out_col0, scale):
+        buffer = ops.step_buffer()
+        return buffer if self._step(proj, col0, ctx, cache, out, out_col0, scale, buffer) else None
+
+    def run(self, proj, col0, ctx, cache, out, out_col0, scale):
+        if self._step(proj, col0, ctx, cache, out, out_col0, scale):
             return
         qkv = ops.causal_conv(proj, col0, self.channels, self.conv_w, None, cache.state, ctx.cu_seqlens, ctx.token_req,
                               ctx.state_slots, ctx.num_requests, state_off=self.state_off, act=True, max_run=ctx.max_q_len)

@@ -149,13 +149,22 @@ class GatedLinearMixer(BranchMixer):
         self.a1_col = self.gate_col + self.inner
         return torch.cat([self._to_device(t) for t in rows], dim=0).contiguous(), self._to_device(get(w["o"]))
 
+    def _step(self, proj, col0, ctx, cache, out, out_col0, scale, prepared=None) -> bool:
+        if not ops.mixer_step_ok(proj.shape[0], ctx.max_q_len, self.num_heads, self.head_dim, self.value_dim, (self.a2_t.shape[0],), cache.state,
+                                 self.state_off, out, out_col0, col0 + self.gate_col, proj.shape[1]):
+            return False
+        ops.linear_step((proj, col0), (proj, col0 + self.qk_dim), (proj, col0 + self.v_col), (proj, col0 + self.a1_col), self.a2_t,
+                        "root_sigmoid", self.a2_bias, 1.0 / self.decay_root, None, None, self.q_scale, (proj, col0 + self.gate_col),
+                        self.norm_w, self.norm_eps, scale, cache.state, self.state_off, ctx.token_req, ctx.state_slots, self.num_heads,
+                        self.head_dim, self.value_dim, out, out_col0, prepared)
+        return True
+
+    def prepare(self, proj, col0, ctx, cache, out, out_col0, scale):
+        buffer = ops.step_buffer()
+        return buffer if self._step(proj, col0, ctx, cache, out, out_col0, scale, buffer) else None
+
     def run(self, proj, col0, ctx, cache, out, out_col0, scale):
-        if ops.mixer_step_ok(proj.shape[0], ctx.max_q_len, self.num_heads, self.head_dim, self.value_dim, (self.a2_t.shape[0],), cache.state, self.state_off,
-                             out, out_col0, col0 + self.gate_col, proj.shape[1]):
-            ops.linear_step((proj, col0), (proj, col0 + self.qk_dim), (proj, col0 + self.v_col), (proj, col0 + self.a1_col), self.a2_t,
-                            "root_sigmoid", self.a2_bias, 1.0 / self.decay_root, None, None, self.q_scale, (proj, col0 + self.gate_col),
-                            self.norm_w, self.norm_eps, scale, cache.state, self.state_off, ctx.token_req, ctx.state_slots, self.num_heads,
-                            self.head_dim, self.value_dim, out, out_col0)
+        if self._step(proj, col0, ctx, cache, out, out_col0, scale):
             return
         decay = ops.lowrank_up(proj, col0 + self.a1_col, self.a2_t, "root_sigmoid", bias=self.a2_bias, rate=1.0 / self.decay_root)
         o = ops.linear_scan((proj, col0), (proj, col0 + self.qk_dim), (proj, col0 + self.v_col), decay, cache.state, self.state_off,

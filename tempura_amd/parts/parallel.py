@@ -77,7 +77,16 @@ class ParallelMixer(Mixer):
     def forward(self, x, ctx, cache, residual=None):
         proj = ops.linear(x, self.w_in, torch.float32)
         act = torch.empty((proj.shape[0], self.inner), dtype=self.dtype, device=proj.device)
-        for b, scale, col, ocol in zip(self.branches, self.scales, self.in_cols, self.out_cols):
+        todo = list(zip(self.branches, self.in_cols, self.out_cols, self.scales))
+        # (single tokens: a recurrent branch's step runs in the launch of the attention beside it)
+        for host in todo:
+            guest = next((t for t in todo if t is not host and host[0].takes_beside(proj, ctx, cache, act, getattr(t[0], "num_heads", 0))), None)
+            step = guest[0].prepare(proj, guest[1], ctx, cache, act, guest[2], guest[3]) if guest is not None else None
+            if step is not None:
+                host[0].run(proj, host[1], ctx, cache, act, host[2], host[3], beside=step)
+                todo = [t for t in todo if t is not host and t is not guest]
+                break
+        for b, col, ocol, scale in todo:
             b.run(proj, col, ctx, cache, act, ocol, scale)
         return ops.linear(act, self.w_out, torch.float32, residual=residual)
 

@@ -114,3 +114,53 @@ def test_attention_from_the_projections_rows(heads, kv, d, page, ctx_lens, how):
         assert float((got.float() - want.float()).norm()) <= 2.0 ** -8 * float(want.float().norm())
     else:
         assert torch.equal(k, k2) and torch.equal(got, want)
+
+
+@pytest.mark.parametrize("d,kv", [(64, 2), (128, 4)])
+@pytest.mark.parametrize("ctx_lens", [[3, 200], [1, 700, 900, 33], [2500]])
+@pytest.mark.parametrize("kind,n_step,dim,vdim", [("delta", 3, 64, 64), ("delta", 2, 128, 100), ("linear", 3, 64, 128), ("linear", 2, 100, 72)])
+def test_a_step_beside_the_attention(d, kv, ctx_lens, kind, n_step, dim, vdim):
+    """A recurrent mixer's step in the attention's launch: the bits of both launches, outputs and states alike."""
+    ops = _ops()
+    g = torch.Generator().manual_seed(d + dim + len(ctx_lens))
+    ctx, k, v = _step(ctx_lens, kv, d, 16, g)
+    n, heads, width = len(ctx_lens), 2 * kv, 4 * kv * d
+    rnd = lambda *s: torch.randn(*s, generator=g).to(DEV)
+    rows, (hd, hv), rank, taps = rnd(n, width), (n_step * dim, n_step * vdim), 33, 4
+    channels = 2 * hd + hv
+    proj = rnd(n, (2 * channels + 2 * rank + 3) // 4 * 4)
+    off = (taps - 1) * channels
+    state = rnd(n + 2, (off + hd * vdim + 3) // 4 * 4)
+    w2, b, nw, a_log, cw = rnd(rank, hd) * 0.3, rnd(hd) - 2.0, rnd(vdim), rnd(n_step), rnd(taps, channels)
+    g2, out_col0 = rnd(rank, hv), heads * d
+
+    def step(state, out, prepared=None):
+        where = (state, 0, off) if kind == "delta" else (state, off)
+        if kind == "delta":
+            ops.delta_step(proj, 0, channels, channels + n_step, channels + n_step + rank, cw, w2, g2, a_log, b, nw, *where, ctx.token_req, ctx.state_slots,
+                           n_step, dim, vdim, dim ** -0.5, 1e-6, 1e-6, 1.3, out, out_col0, prepared)
+        else:
+            ops.linear_step((proj, 0), (proj, hd), (proj, 2 * hd), (proj, 2 * hd + 2 * hv), w2, "root_sigmoid", b, 0.06, None, None, 0.3,
+                            (proj, 2 * hd + hv), nw, 1e-6, 1.3, *where, ctx.token_req, ctx.state_slots, n_step, dim, vdim, out, out_col0, prepared)
+
+    def attend(out, beside=None):
+        kk, vv = k.clone(), v.clone()
+        ops.attention_rows(rows, 0, ctx, 0, heads, kv, d, kk, vv, d ** -0.5, None, 0, 1.0, None, into=(None, 0, 0.75, out, 0, 1), beside=beside)
+        return kk, vv
+    assert ops.attention_beside_ok(ctx, heads, kv, 0, 0, n_step)
+    outs, states, caches = [torch.zeros(n, heads * d + hv, dtype=torch.bfloat16, device=DEV) for _ in "ab"], [state.clone(), state.clone()], []
+    force = ops.decode_force_splits
+    try:
+        ops.decode_force_splits = ops._rows_splits(ctx, heads, kv, 0, 0, 0, False, True)      # (the same parts of the keys both ways)
+        step(states[0], outs[0])
+        caches.append(attend(outs[0]))
+        ops.decode_force_splits = 2 * ops.decode_force_splits if ops.decode_force_splits > 1 else 1
+        buffer = ops.step_buffer()
+        step(states[1], outs[1], buffer)
+        caches.append(attend(outs[1], buffer))
+    finally:
+        ops.decode_force_splits = force
+    assert torch.equal(outs[0][:, out_col0:], outs[1][:, out_col0:]) and torch.equal(states[0], states[1])
+    assert all(torch.equal(a, c) for a, c in zip(*caches))
+    # (the attention's sums by eight waves here and by four there where the keys are split)
+    assert float((outs[0][:, :out_col0].float() - outs[1][:, :out_col0].float()).norm()) <= 2.0 ** -8 * float(outs[0][:, :out_col0].float().norm())

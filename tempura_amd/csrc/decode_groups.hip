@@ -10,6 +10,7 @@
 
 #include "common.h"
 #include "activations.h"
+#include "moe_route.h"
 
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
@@ -132,12 +133,100 @@ __global__ __launch_bounds__(DG_WAVES * 64) void moe_up_kernel(const bf16_t* __r
   a[((size_t)(n >> 3) * M + m) * 8 + (n & 7)] = float_to_bf16(weight == 0.f ? 0.f : y * weight);
 }
 
+// Opens a layer of routed experts: block 0 works out the router's logits and every row's choice, the others are the up product of
+// an expert that every row uses (w tiled [rows >= size, K], activated; with `gated` its row `size` is a gate's, left raw in g [M]),
+// which needs no choice and keeps the memory busy meanwhile.  The logits are formed in the order of the products of a few rows.
+// Router product, choice, shared up product, its activation and its down product were launches of their own, 3 to 6 us each of which
+// half is the chain: a layer of eight experts and a shared one at width 4,096, three rows, 79 -> 60 us of kernels (58 MB of them shared).
+#define DG_OPEN_EXPERTS 64
+__global__ __launch_bounds__(DG_WAVES * 64) void moe_open_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w_router, Route r,
+                                                                  const bf16_t* __restrict__ w, bf16_t* __restrict__ a, float* __restrict__ g,
+                                                                  int M, int K, int size, int kind, int gated) {
+  __shared__ float red[DG_WAVES][256];
+  __shared__ float logits[16][DG_OPEN_EXPERTS];
+  __shared__ float route_lds[DG_WAVES][2 * DG_OPEN_EXPERTS];
+  const int lane = threadIdx.x % 64, wave = threadIdx.x / 64;
+  const int row = min(lane & 15, M - 1);
+  const u32x4_t* xp = (const u32x4_t*)(x + ((size_t)(lane >> 4) * M + row) * 8);
+  const int q = threadIdx.x, l = q / 4, m = l & 15;
+  if (blockIdx.x > 0) {
+    const int n0 = (blockIdx.x - 1) * 16;
+    const f32x4_t acc = dg_tile((const u32x4_t*)(w + (size_t)n0 * K) + lane, xp, 4 * M, K / 32, wave, (f32x4_t){0.f, 0.f, 0.f, 0.f});
+#pragma unroll
+    for (int i = 0; i < 4; ++i) red[wave][lane * 4 + i] = acc[i];
+    __syncthreads();
+    if (q >= 256 || m >= M) return;
+    const float v = dg_sum(red, q);
+    const int n = n0 + (l >> 4) * 4 + q % 4;
+    if (n < size) a[((size_t)(n >> 3) * M + m) * 8 + (n & 7)] = float_to_bf16(act_f(v, kind));
+    else if (gated && n == size) g[m] = v;
+    return;
+  }
+  for (int e0 = 0; e0 < r.experts; e0 += 16) {
+    const u32x4_t* wp = (const u32x4_t*)(w_router + (size_t)e0 * K) + lane;
+    // (rows of the tile past the last expert are not read)
+    const bool mine = e0 + (lane & 15) < r.experts;
+    f32x4_t acc = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+    const int steps = K / 32;
+    for (int s0 = wave * 4; s0 < steps; s0 += DG_WAVES * 8) {
+      u32x4_t av[2][4], bv[2][4];
+#pragma unroll
+      for (int d = 0; d < 2; ++d)
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          const int st = min(s0 + d * DG_WAVES * 4 + u, steps - 1);
+          av[d][u] = (u32x4_t){0u, 0u, 0u, 0u};
+          if (mine) av[d][u] = wp[(size_t)st * 64];
+          bv[d][u] = xp[(size_t)st * 4 * M];
+        }
+#pragma unroll
+      for (int d = 0; d < 2; ++d)
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+          if (s0 + d * DG_WAVES * 4 + u < steps) acc = dg_mfma(av[d][u], bv[d][u], acc);
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) red[wave][lane * 4 + i] = acc[i];
+    __syncthreads();
+    if (q < 256 && e0 + (l >> 4) * 4 + q % 4 < DG_OPEN_EXPERTS) logits[m][e0 + (l >> 4) * 4 + q % 4] = dg_sum(red, q);
+    __syncthreads();
+  }
+  for (int t0 = 0; t0 < M; t0 += DG_WAVES) {
+    const int t = min(t0 + wave, M - 1);
+    route_token<1>(r, logits[t], t, t0 + wave < M, route_lds[wave], route_lds[wave] + DG_OPEN_EXPERTS);
+    __syncthreads();
+  }
+}
+
+// x: bfloat16 [K / 8, M, 8]; w_router: tiled [experts rounded up to 16, K]; the outputs of tp_moe_route; w_shared: tiled [shared_rows, K]
+// (nullptr: none), its first `size` rows activated into a_shared bfloat16 [size / 8, M, 8], row `size` with gate != nullptr into gate [M].
+extern "C" int tp_moe_open(const void* x, const void* w_router, const float* correction, const float* logit_bias, int experts, int top, int groups,
+                           int keep, float* dense, int* ids, float* weights, int M, int K, int score_kind, int group_best, int normalize,
+                           float sum_eps, float scale, const void* w_shared, int shared_rows, int size, int kind, void* a_shared, float* gate,
+                           hipStream_t s) {
+  TP_REQUIRE(M > 0 && M <= 16 && K > 0 && K % 64 == 0, "moe_open: %d rows of %d", M, K);
+  TP_REQUIRE(experts > 0 && experts <= DG_OPEN_EXPERTS && top > 0 && top <= experts && (groups <= 1 || (experts % groups == 0 && keep >= 1 && keep <= groups)) &&
+                 (score_kind == 0 || score_kind == 1) && group_best >= 1,
+             "moe_open: bad router");
+  TP_REQUIRE(w_shared == nullptr || (shared_rows % 16 == 0 && size > 0 && size % 8 == 0 && size + (gate != nullptr ? 1 : 0) <= shared_rows && kind >= 0 &&
+                                     kind <= 3 && a_shared),
+             "moe_open: bad shared expert");
+  TP_REQUIRE((((uintptr_t)x | (uintptr_t)w_router | (uintptr_t)w_shared | (uintptr_t)a_shared) & 15) == 0, "moe_open: operands must be aligned to 16 bytes");
+  const Route r = {correction, logit_bias, experts, top, groups, keep, score_kind, group_best, normalize, sum_eps, scale, dense, ids, weights};
+  hipLaunchKernelGGL(moe_open_kernel, dim3(1 + (w_shared != nullptr ? shared_rows / 16 : 0)), dim3(DG_WAVES * 64), 0, s, (const bf16_t*)x,
+                     (const bf16_t*)w_router, r, (const bf16_t*)w_shared, (bf16_t*)a_shared, gate, M, K, size, kind, gate != nullptr ? 1 : 0);
+  TP_CHECK_LAUNCH("moe_open");
+  return 0;
+}
+
 // Down: y[m] (+)= sum_e a[m][e] . down_e, experts ascending; the same experts are skipped.  w: every expert's tiled [N, ff], one
-// behind the other.
+// behind the other.  ws: then the shared expert's tiled [N, size] (nullptr: none) times a_shared, its sum added on its own, times
+// sigmoid(gate[m]) where there is a gate.
 __global__ __launch_bounds__(DG_WAVES * 64) void moe_down_kernel(const bf16_t* __restrict__ a, const bf16_t* __restrict__ w,
                                                                   const float* __restrict__ dense, float* __restrict__ y, int M, int experts,
-                                                                  int ff, int N, int accumulate) {
-  __shared__ float red[DG_WAVES][256];
+                                                                  int ff, int N, int accumulate, const bf16_t* __restrict__ ws,
+                                                                  const bf16_t* __restrict__ a_shared, const float* __restrict__ gate, int size) {
+  __shared__ float red[DG_WAVES][256], red_s[DG_WAVES][256];
   __shared__ int list[DG_MAX_EXPERTS];
   __shared__ int counts[DG_WAVES];
   const int lane = threadIdx.x % 64, wave = threadIdx.x / 64;
@@ -192,20 +281,35 @@ __global__ __launch_bounds__(DG_WAVES * 64) void moe_down_kernel(const bf16_t* _
   }
 #pragma unroll
   for (int r = 0; r < 4; ++r) red[wave][lane * 4 + r] = acc[r];
+  if (ws != nullptr) {
+    const f32x4_t sum = dg_tile((const u32x4_t*)(ws + (size_t)n0 * size) + lane, (const u32x4_t*)(a_shared + ((size_t)(lane >> 4) * M + row) * 8),
+                                xstep, size / 32, wave, (f32x4_t){0.f, 0.f, 0.f, 0.f});
+#pragma unroll
+    for (int r = 0; r < 4; ++r) red_s[wave][lane * 4 + r] = sum[r];
+  }
   __syncthreads();
   const int q = threadIdx.x;
   if (q >= 256) return;
   const int l = q / 4, m = l & 15;
   if (m >= M) return;
   float* o = y + (size_t)m * N + n0 + (l >> 4) * 4 + q % 4;
-  const float v = dg_sum(red, q);
-  *o = accumulate ? *o + v : v;
+  float v = dg_sum(red, q);
+  if (accumulate) v = *o + v;
+  if (ws != nullptr) {
+    const float sv = dg_sum(red_s, q);
+    v += gate != nullptr ? sv * (1.0f / (1.0f + expf(-gate[m]))) : sv;
+  }
+  *o = v;
 }
 
 // x: bfloat16 [K / 8, M, 8]; w_up: tiled [experts * rows, K], rows = ff, or 2 ff with gated (kind is then not read); w_down: experts
-// tiled [N, ff]; dense float32 [M, experts]; a: bfloat16 scratch [experts * ff / 8, M, 8]; y float32 [M, N].
+// tiled [N, ff]; dense float32 [M, experts]; a: bfloat16 scratch [experts * ff / 8, M, 8]; y float32 [M, N].  w_shared (nullptr: none):
+// tiled [N, size], a_shared and gate (nullptr: none) as tp_moe_open leaves them.
 extern "C" int tp_moe_few(const void* x, const void* w_up, const void* w_down, const float* dense, void* a, float* y, int M, int experts,
-                          int ff, int K, int N, int gated, int kind, int accumulate, hipStream_t s) {
+                          int ff, int K, int N, int gated, int kind, int accumulate, const void* w_shared, const void* a_shared, const float* gate,
+                          int size, hipStream_t s) {
+  TP_REQUIRE(w_shared == nullptr || (size > 0 && size % 64 == 0 && a_shared && (((uintptr_t)w_shared | (uintptr_t)a_shared) & 15) == 0),
+             "moe_few: bad shared expert");
   TP_REQUIRE(M > 0 && M <= 16 && experts > 0 && experts <= DG_MAX_EXPERTS, "moe_few: %d rows, %d experts", M, experts);
   TP_REQUIRE(ff > 0 && ff % 64 == 0 && K > 0 && K % 64 == 0 && N > 0 && N % 16 == 0, "moe_few: sizes ff %d K %d N %d", ff, K, N);
   TP_REQUIRE(gated || (kind >= 0 && kind <= 3), "moe_few: unknown activation %d", kind);
@@ -217,7 +321,8 @@ extern "C" int tp_moe_few(const void* x, const void* w_up, const void* w_down, c
     hipLaunchKernelGGL(moe_up_kernel<true>, up, block, 0, s, (const bf16_t*)x, (const bf16_t*)w_up, dense, (bf16_t*)a, M, experts, rows, K, 0);
   else
     hipLaunchKernelGGL(moe_up_kernel<false>, up, block, 0, s, (const bf16_t*)x, (const bf16_t*)w_up, dense, (bf16_t*)a, M, experts, rows, K, kind);
-  hipLaunchKernelGGL(moe_down_kernel, dim3(N / 16), block, 0, s, (const bf16_t*)a, (const bf16_t*)w_down, dense, y, M, experts, ff, N, accumulate);
+  hipLaunchKernelGGL(moe_down_kernel, dim3(N / 16), block, 0, s, (const bf16_t*)a, (const bf16_t*)w_down, dense, y, M, experts, ff, N, accumulate,
+                     (const bf16_t*)w_shared, (const bf16_t*)a_shared, gate, size);
   TP_CHECK_LAUNCH("moe_few");
   return 0;
 }

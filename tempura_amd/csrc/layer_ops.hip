@@ -5,6 +5,7 @@
 #include <math.h>
 
 #include "common.h"
+#include "moe_route.h"
 #include "activations.h"
 
 __device__ inline float l_sigmoid(float v) { return 1.0f / (1.0f + expf(-v)); }
@@ -462,166 +463,16 @@ extern "C" int tp_activation(const void* in, int in_dt, void* out, int out_dt, s
   return 0;
 }
 
-// ---- router of a mixture of experts -----------------------------------------------------------
-// logits [n, logit_stride] float32 (the first `experts` columns count).  s = softmax over the experts; the choice
-// score of expert e is s[e] + correction[e]; experts form `groups` equal groups of neighbours, a group's score is
-// its largest choice score, and only experts of the `keep` best groups can be chosen (groups <= 1: all); the `top`
-// allowed experts with the largest choice scores are chosen (ties: the lower index), and a chosen expert's weight
-// is s[e].  dense [n, experts] gets the weight of every chosen expert and 0 elsewhere; ids and weights [n, top]
-// list the chosen experts in the order of choice.  One wave per token; lane l holds experts l, l + 64, ...
-#define ROUTE_PER_LANE 8   // experts <= 64 * ROUTE_PER_LANE
-
-__device__ inline void wave_arg_best(float& v, int& i) {
-#pragma unroll
-  for (int o = TP_WAVE / 2; o > 0; o >>= 1) {
-    const float ov = __shfl_xor(v, o, TP_WAVE);
-    const int oi = __shfl_xor(i, o, TP_WAVE);
-    if (ov > v || (ov == v && oi < i)) {
-      v = ov;
-      i = oi;
-    }
-  }
-}
-
-// score_kind 0: s = softmax over the experts; 1: s = sigmoid of each logit by itself.  The choice score is s plus the
-// correction (none: s).  A group is ranked by the sum of its `group_best` largest choice scores.  The weights are the
-// chosen experts' s, with `normalize` divided by their sum plus sum_eps (added in the order of choice), times `scale`.
+// ---- router of a mixture of experts (see moe_route.h) ------------------------------------------
 template <int ROUTE_LANE>
-__global__ __launch_bounds__(256) void moe_route_kernel(const float* __restrict__ logits, int logit_stride,
-                                                        const float* __restrict__ correction, int experts, int top,
-                                                        int groups, int keep, float* __restrict__ dense,
-                                                        int* __restrict__ ids, float* __restrict__ weights, int n,
-                                                        int score_kind, int group_best, int normalize, float sum_eps,
-                                                        float scale, const float* __restrict__ logit_bias) {
+__global__ __launch_bounds__(256) void moe_route_kernel(Route r, const float* __restrict__ logits, int logit_stride, int n) {
   extern __shared__ float lds[];   // per wave: choice scores [experts], then group scores [groups]
-  const int wave = threadIdx.x / TP_WAVE, lane = threadIdx.x % TP_WAVE;
+  const int wave = threadIdx.x / TP_WAVE;
   // (a wave past the last token works on the last token again and stores nothing: every wave reaches every barrier)
   const bool live = blockIdx.x * 4 + wave < n;
   const int t = live ? blockIdx.x * 4 + wave : n - 1;
-  float* choice_l = lds + (size_t)wave * (experts + max(groups, 1));
-  float* group_l = choice_l + experts;
-  float z[ROUTE_LANE], sc[ROUTE_LANE], ch[ROUTE_LANE];
-  int won[ROUTE_LANE];
-  float mx = -INFINITY;
-#pragma unroll
-  for (int k = 0; k < ROUTE_LANE; ++k) {
-    const int e = lane + k * TP_WAVE;
-    z[k] = e < experts ? logits[(size_t)t * logit_stride + e] + (logit_bias != nullptr ? logit_bias[e] : 0.f) : -INFINITY;
-    mx = fmaxf(mx, z[k]);
-    won[k] = -1;
-  }
-  if (score_kind == 1) {
-#pragma unroll
-    for (int k = 0; k < ROUTE_LANE; ++k) sc[k] = lane + k * TP_WAVE < experts ? l_sigmoid(z[k]) : 0.f;
-  } else {
-    mx = wave_max(mx);
-    float sum = 0.f;
-#pragma unroll
-    for (int k = 0; k < ROUTE_LANE; ++k) {
-      sc[k] = lane + k * TP_WAVE < experts ? expf(z[k] - mx) : 0.f;
-      sum += sc[k];
-    }
-    sum = wave_sum(sum);
-    const float inv = 1.0f / sum;
-#pragma unroll
-    for (int k = 0; k < ROUTE_LANE; ++k) sc[k] *= inv;
-  }
-#pragma unroll
-  for (int k = 0; k < ROUTE_LANE; ++k) {
-    const int e = lane + k * TP_WAVE;
-    ch[k] = e < experts ? (correction != nullptr ? sc[k] + correction[e] : sc[k]) : -INFINITY;
-    if (e < experts) {
-      choice_l[e] = ch[k];
-      if (live) dense[(size_t)t * experts + e] = 0.f;
-    }
-  }
-  if (groups > 1) {
-    const int per = experts / groups;
-    __syncthreads();
-    for (int g = lane; g < groups; g += TP_WAVE) {
-      // the group's largest scores one after the other (equal scores: the lower index first), added in that order
-      float total = 0.f, pv = INFINITY;
-      int pi = -1;
-      for (int b = 0; b < group_best; ++b) {
-        float best = -INFINITY;
-        int bi = -1;
-        for (int i = 0; i < per; ++i) {
-          const float v = choice_l[g * per + i];
-          if ((v < pv || (v == pv && i > pi)) && (bi < 0 || v > best)) {
-            best = v;
-            bi = i;
-          }
-        }
-        if (bi < 0) break;
-        total = b == 0 ? best : total + best;
-        pv = best;
-        pi = bi;
-      }
-      group_l[g] = total;
-    }
-    __syncthreads();
-    // the `keep` best groups, one after the other; a kept group's score becomes +inf as its mark
-    for (int it = 0; it < keep; ++it) {
-      float bv = -INFINITY;
-      int bi = 0x7fffffff;
-      for (int g = lane; g < groups; g += TP_WAVE) {
-        const float v = group_l[g];
-        if (v != INFINITY && (v > bv || (v == bv && g < bi))) {
-          bv = v;
-          bi = g;
-        }
-      }
-      wave_arg_best(bv, bi);
-      __syncthreads();
-      if (lane == 0 && bi != 0x7fffffff) group_l[bi] = INFINITY;
-      __syncthreads();
-    }
-#pragma unroll
-    for (int k = 0; k < ROUTE_LANE; ++k) {
-      const int e = lane + k * TP_WAVE;
-      if (e < experts && group_l[e / per] != INFINITY) ch[k] = -INFINITY;
-    }
-  }
-  float chosen_sum = 0.f;
-  for (int it = 0; it < top; ++it) {
-    float bv = -INFINITY, bs = 0.f;
-    int bi = 0x7fffffff, bk = -1;
-#pragma unroll
-    for (int k = 0; k < ROUTE_LANE; ++k) {
-      const int e = lane + k * TP_WAVE;
-      if (e < experts && ch[k] > bv) {   // (ascending e within a lane: the lower index wins a tie)
-        bv = ch[k];
-        bi = e;
-        bk = k;
-        bs = sc[k];
-      }
-    }
-    float v = bv;
-    int i = bi;
-    wave_arg_best(v, i);
-    if (i == 0x7fffffff) break;   // fewer allowed experts than `top` (uniform over the wave)
-    chosen_sum += __shfl(bs, i % TP_WAVE, TP_WAVE);   // (the winner's lane holds its score; every lane adds alike)
-    if (i == bi && bk >= 0) {
-      // this lane owns the winner
-#pragma unroll
-      for (int k = 0; k < ROUTE_LANE; ++k)
-        if (k == bk) {
-          ch[k] = -INFINITY;
-          won[k] = it;
-        }
-    }
-  }
-  const float factor = normalize ? scale / (chosen_sum + sum_eps) : scale;
-#pragma unroll
-  for (int k = 0; k < ROUTE_LANE; ++k) {
-    if (won[k] >= 0 && live) {
-      const int e = lane + k * TP_WAVE;
-      const float w = (normalize || scale != 1.0f) ? sc[k] * factor : sc[k];
-      dense[(size_t)t * experts + e] = w;
-      ids[(size_t)t * top + won[k]] = e;
-      weights[(size_t)t * top + won[k]] = w;
-    }
-  }
+  float* choice_l = lds + (size_t)wave * (r.experts + max(r.groups, 1));
+  route_token<ROUTE_LANE>(r, logits + (size_t)t * logit_stride, t, live, choice_l, choice_l + r.experts);
 }
 
 extern "C" int tp_moe_route(const float* logits, int logit_stride, const float* correction, int experts, int top, int groups,
@@ -634,9 +485,8 @@ extern "C" int tp_moe_route(const float* logits, int logit_stride, const float* 
   if (n == 0) return 0;
   const size_t shmem = sizeof(float) * 4 * (size_t)(experts + (groups > 1 ? groups : 1));
   // (as many experts a lane as there are: eight experts in four groups, eight tokens, 7.9 -> 7.5 us with one instead of eight)
-#define ROUTE(L)                                                                                                                        \
-  hipLaunchKernelGGL(moe_route_kernel<L>, dim3((n + 3) / 4), dim3(256), shmem, s, logits, logit_stride, correction, experts, top, groups, \
-                     keep, dense, ids, weights, n, score_kind, group_best, normalize, sum_eps, scale, logit_bias)
+  const Route r = {correction, logit_bias, experts, top, groups, keep, score_kind, group_best, normalize, sum_eps, scale, dense, ids, weights};
+#define ROUTE(L) hipLaunchKernelGGL(moe_route_kernel<L>, dim3((n + 3) / 4), dim3(256), shmem, s, r, logits, logit_stride, n)
   if (experts <= TP_WAVE) ROUTE(1);
   else if (experts <= 2 * TP_WAVE) ROUTE(2);
   else ROUTE(ROUTE_PER_LANE);

@@ -2388,23 +2388,68 @@ def moe_few_ok(m: int, experts: int, ff: int, w_up, w_down) -> bool:
             and few_rows_ok(m, w_up.shape[1], w_up.dtype))
 
 
-def moe_few(x: KBlocked, w_up, w_down, dense: torch.Tensor, ff: int, activation: Optional[str], y: Optional[torch.Tensor] = None) -> torch.Tensor:
+def moe_open_ok(experts: int, w_router, k: int, w_shared_up=None, w_shared_down=None, size: int = 0) -> bool:
+    """Whether ``moe_open`` takes this router and, if there is one, this shared expert (of ``size``, without a gated activation)."""
+    if not (isinstance(w_router, TiledWeight) and experts <= 64 and w_router.shape[0] == -(-experts // 16) * 16 and k % 64 == 0):
+        return False
+    return w_shared_up is None or (isinstance(w_shared_up, TiledWeight) and isinstance(w_shared_down, TiledWeight) and size % 64 == 0)
+
+
+def moe_open(x: KBlocked, w_router, correction: Optional[torch.Tensor], experts: int, top: int, groups: int, keep: int, score: str = "softmax",
+             group_best: int = 1, normalize: bool = False, sum_eps: float = 0.0, scale: float = 1.0, bias: Optional[torch.Tensor] = None,
+             shared: Optional[tuple] = None):
+    """The router of at most 16 rows in one launch: ``moe_route`` of the rows' product with the tiled ``w_router`` (its rows padded to 16),
+    the same bits.  ``shared`` = (tiled up weight, size, activation, whether its row ``size`` is a gate's): the shared expert's up product
+    beside it.  Returns (dense, ids, weights, (activated rows bfloat16 [size / 8, m, 8], raw gate float32 [m] or None) or None)."""
+    m, k = x.shape
+    _dev_ok(x.data, w_router.data, correction, bias)
+    _need(moe_open_ok(experts, w_router, k) and w_router.shape[1] == k and score in ROUTE_SCORES and group_best >= 1, "moe_open: sizes that it does not take")
+    _need(bias is None or (bias.dtype == torch.float32 and bias.numel() == experts), "moe_open: bias must be float32 [experts]")
+    _need(correction is None or (correction.dtype == torch.float32 and correction.numel() == experts), "moe_open: correction must be float32 [experts]")
+    dev = x.data.device
+    dense = torch.empty((m, experts), dtype=torch.float32, device=dev)
+    ids = torch.empty((m, top), dtype=torch.int32, device=dev)
+    weights = torch.empty((m, top), dtype=torch.float32, device=dev)
+    w_shared, size, kind, a, gate = None, 0, 0, None, None
+    if shared is not None:
+        w_shared, size, activation, gated = shared
+        _dev_ok(w_shared.data)
+        _need(w_shared.shape[1] == k and size + int(gated) <= w_shared.shape[0], "moe_open: bad shared expert")
+        kind = ACTIVATIONS[activation]
+        a = torch.empty((size // 8, m, 8), dtype=torch.bfloat16, device=dev)
+        gate = torch.empty((m,), dtype=torch.float32, device=dev) if gated else None
+    _call("tp_moe_open", _ptr(x.data), _ptr(w_router.data), _ptr(correction), _ptr(bias), int(experts), int(top), int(groups), int(keep), _ptr(dense),
+          _ptr(ids), _ptr(weights), m, k, ROUTE_SCORES[score], int(group_best), int(bool(normalize)), ctypes.c_float(sum_eps), ctypes.c_float(scale),
+          _ptr(None if w_shared is None else w_shared.data), 0 if w_shared is None else w_shared.shape[0], int(size), kind, _ptr(a), _ptr(gate), _stream())
+    return dense, ids, weights, None if shared is None else (a, gate)
+
+
+def moe_few(x: KBlocked, w_up, w_down, dense: torch.Tensor, ff: int, activation: Optional[str], y: Optional[torch.Tensor] = None,
+            shared: Optional[tuple] = None) -> torch.Tensor:
     """The routed experts of at most 16 rows: y (+)= sum_e down_e(f(up_e x) * dense[:, e]), skipping the weights of experts
     whose column of ``dense`` (float32 [m, experts]) is zero.  ``w_up``: the experts' tiled up weights stacked
     ([experts * ff, k]; ``activation`` None: gate and up rows interleaved by eights, [2 experts * ff, k], f = silu(gate) * up);
-    ``w_down``: their tiled [n, ff] one behind the other, as a ``TiledWeight`` of [experts * n, ff].  ``y`` float32 [m, n] or None."""
+    ``w_down``: their tiled [n, ff] one behind the other, as a ``TiledWeight`` of [experts * n, ff].  ``y`` float32 [m, n] or None.
+    ``shared`` = (tiled down weight [n, size], activated rows, raw gate or None, as of ``moe_open``): the shared expert's output behind
+    the routed sum, times sigmoid(gate)."""
     m, k = x.shape
     experts = dense.shape[1]
+    w_s, a_s, gate = shared if shared is not None else (None, None, None)
     n = w_down.shape[0] // experts
     _dev_ok(x.data, w_up.data, w_down.data, dense, y)
     rows = ff if activation is not None else 2 * ff
     _need(tuple(w_up.shape) == (experts * rows, k) and tuple(w_down.shape) == (experts * n, ff), "moe_few: weights disagree with the sizes")
     _need(dense.dtype == torch.float32 and tuple(dense.shape) == (m, experts), "moe_few: dense must be float32 [m, experts]")
     _need(y is None or (y.dtype == torch.float32 and tuple(y.shape) == (m, n)), "moe_few: y must be float32 [m, n]")
+    if w_s is not None:
+        _dev_ok(w_s.data, a_s, gate)
+        _need(w_s.shape[0] == n and tuple(a_s.shape) == (w_s.shape[1] // 8, m, 8) and a_s.dtype == torch.bfloat16 and
+              (gate is None or (gate.dtype == torch.float32 and gate.numel() == m)), "moe_few: shared expert disagrees with the sizes")
     acc = y is not None
     if not acc:
         y = torch.empty((m, n), dtype=torch.float32, device=dense.device)
     a = torch.empty((experts * ff // 8, m, 8), dtype=torch.bfloat16, device=dense.device)
     _call("tp_moe_few", _ptr(x.data), _ptr(w_up.data), _ptr(w_down.data), _ptr(dense), _ptr(a), _ptr(y), m, experts, int(ff), k, n,
-          int(activation is None), 0 if activation is None else ACTIVATIONS[activation], int(acc), _stream(), tag=(m, experts, ff, k))
+          int(activation is None), 0 if activation is None else ACTIVATIONS[activation], int(acc), _ptr(None if w_s is None else w_s.data), _ptr(a_s),
+          _ptr(gate), 0 if w_s is None else w_s.shape[1], _stream(), tag=(m, experts, ff, k))
     return y

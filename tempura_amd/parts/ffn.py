@@ -320,7 +320,28 @@ class RoutedExperts(FeedForward):
                            self.shared_size if self.shared_gated else None)
         ops.linear(a, self.w_shared_down, torch.float32, residual=y)
 
+    def _few(self, x, ctx, residual):
+        """A step of at most 16 single tokens in three launches: the choice beside the shared expert's up product, the chosen experts' up
+        products, all down products."""
+        rows = x if isinstance(x, ops.KBlocked) else ops.block_rows(x)
+        up = down = None
+        if self.shared is not None:
+            up = (self.w_shared_up, self.shared_size, str(self.shared.get("activation", "silu")), self.shared_gated)
+        dense, _, _, opened = ops.moe_open(rows, self.w_router, self.correction, self.experts, self.top, self.groups, self.keep, self.score,
+                                           self.group_best, self.normalize, self.sum_eps, self.weight_scale, self.router_bias, up)
+        if opened is not None:
+            down = (self.w_shared_down,) + opened
+        y = ops.moe_few(rows, self.w13_all, self.w2_all, dense, self.intermediate_size, self.activation if self.expert_kind == "plain" else None,
+                        residual, down)
+        return y if residual is None else None
+
+    def _opens(self, m):
+        shared = () if self.shared is None else (self.w_shared_up, self.w_shared_down, self.shared_size)
+        return self._few_ok(m) and ops.moe_open_ok(self.experts, self.w_router, self.hidden_size, *shared)
+
     def forward(self, x, ctx, residual=None):
+        if getattr(ctx, "max_q_len", 1) <= 1 and self._opens(x.shape[0]):
+            return self._few(x, ctx, residual)
         if self.shared is None:
             return self._routed(x, ctx, residual)
         y = self._routed(x, ctx, residual)

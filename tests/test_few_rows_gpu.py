@@ -297,3 +297,39 @@ def test_products_of_one_deep_block_a_cu(m, n, k):
         h = torch.ones(m, n, device=DEV)
         ops.linear(x, weight, torch.float32, residual=h)
         assert torch.equal(h, got + 1.0)
+
+
+@pytest.mark.parametrize("m,experts,top,groups,keep", [(1, 8, 2, 1, 1), (3, 8, 2, 4, 2), (9, 20, 4, 5, 2), (16, 64, 6, 1, 1)])
+@pytest.mark.parametrize("k,ff,size,gated", [(64, 64, 64, True), (1152, 128, 192, False), (2048, 64, 0, False)])
+def test_router_beside_the_shared_expert(m, experts, top, groups, keep, k, ff, size, gated):
+    """Choice, shared up product and down product in the routed experts' launches: the choice and the routed sum bit for bit those of
+    the kernels by themselves, the shared expert's sum with its gate behind the down product instead of in front of it."""
+    from tempura_amd.kernels import ops
+    g = torch.Generator().manual_seed(m * 100 + k + experts)
+    rnd = lambda *s: (torch.randn(*s, generator=g) * 0.1).to(DEV).bfloat16()
+    n, pad = 96, -experts % 16
+    x = rnd(m, k) * 10
+    w_router = torch.cat([rnd(experts, k), torch.zeros(pad, k, dtype=torch.bfloat16, device=DEV)])
+    w_up, w_down = ops.tile_weight(rnd(experts * ff, k)), rnd(experts, n, ff)
+    w_down = ops.TiledWeight(torch.cat([ops.tile_weight(w).data for w in w_down]), experts * n, ff)
+    correction, bias = torch.rand(experts, generator=g).to(DEV) * 0.1, torch.randn(experts, generator=g).to(DEV) * 0.1
+    rest = dict(score="sigmoid" if gated else "softmax", group_best=2 if groups > 1 else 1, normalize=gated, sum_eps=1e-6, scale=1.5, bias=bias)
+    router, rows = ops.tile_weight(w_router), ops.block_rows(x)
+    shared = down = None
+    if size:
+        w_su, w_sd = rnd(size + 16, k), rnd(n, size)
+        shared = (ops.tile_weight(w_su), size, "relu2" if not gated else "silu", gated)
+    assert ops.moe_open_ok(experts, router, k, *([shared[0], ops.tile_weight(w_sd), size] if size else []))
+    want = ops.moe_route(ops.linear(rows, router, torch.float32), correction, experts, top, groups, keep, **rest)
+    *got, opened = ops.moe_open(rows, router, correction, experts, top, groups, keep, shared=shared, **rest)
+    assert all(torch.equal(a, b) for a, b in zip(got, want))
+    plain = ops.moe_few(rows, w_up, w_down, want[0], ff, "silu")
+    if not size:
+        assert opened is None
+        return
+    y = ops.moe_few(rows, w_up, w_down, got[0], ff, "silu", torch.ones(m, n, device=DEV), (ops.tile_weight(w_sd),) + opened)
+    u = x.double() @ w_su.double().t()
+    act = torch.relu(u[:, :size]) ** 2 if not gated else torch.nn.functional.silu(u[:, :size])
+    add = act @ w_sd.double().t() * (torch.sigmoid(u[:, size:size + 1]) if gated else 1.0)
+    # (the activations are rounded to bfloat16: 2^-9 of each term, whose sum over `size` of them is off by that much of its norm)
+    assert float((y.double() - 1.0 - plain.double() - add).norm()) <= 2.0 ** -8 * float(add.norm()) + 1e-5 * float(plain.norm())

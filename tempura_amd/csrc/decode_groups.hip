@@ -96,6 +96,39 @@ extern "C" int tp_group_linear(const void* x, const void* w, float* out, const i
   return 0;
 }
 
+// ---- a product of few column blocks --------------------------------------------------------------
+// out [splits, M, N] float32: partial sums over equal parts of K, for the kernel that consumes the rows to add.  A block of 16 columns
+// pulls at most 57 GB/s, its CU's share of the way to memory, so 128 of them (N = 2,048) stay under the memory's rate however long K is.
+// With the norm behind it, a captured chain, whole / in parts: 2,048 x 8,192 one row 12.8 / 11.0 us, sixteen 16.1 / 12.5; 1,024 x 8,192
+// (four parts) 11.9 / 8.5 and 15.4 / 9.8; 2,048 x 4,096 9.3 / 8.5 and 11.3 / 9.7.
+__global__ __launch_bounds__(DG_WAVES * 64) void split_linear_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w,
+                                                                      float* __restrict__ out, int M, int N, int K) {
+  __shared__ float red[DG_WAVES][256];
+  const int lane = threadIdx.x % 64, wave = threadIdx.x / 64;
+  const int n0 = blockIdx.x * 16, steps = K / 32 / gridDim.y, s0 = blockIdx.y * steps;
+  const int row = min(lane & 15, M - 1);
+  const u32x4_t* wp = (const u32x4_t*)(w + (size_t)n0 * K) + lane + (size_t)s0 * 64;
+  const u32x4_t* xp = (const u32x4_t*)(x + ((size_t)(lane >> 4) * M + row) * 8) + (size_t)s0 * 4 * M;
+  const f32x4_t acc = dg_tile(wp, xp, 4 * M, steps, wave, (f32x4_t){0.f, 0.f, 0.f, 0.f});
+#pragma unroll
+  for (int r = 0; r < 4; ++r) red[wave][lane * 4 + r] = acc[r];
+  __syncthreads();
+  const int q = threadIdx.x;
+  if (q >= 256) return;
+  const int l = q / 4, m = l & 15;
+  if (m < M) out[((size_t)blockIdx.y * M + m) * N + n0 + (l >> 4) * 4 + q % 4] = dg_sum(red, q);
+}
+
+// x: bfloat16 [K / 8, M, 8]; w: tiled [N, K]; K in `splits` equal parts of whole steps of 32
+extern "C" int tp_split_linear(const void* x, const void* w, float* out, int M, int N, int K, int splits, hipStream_t s) {
+  TP_REQUIRE(M > 0 && M <= 16 && N > 0 && N % 16 == 0 && K > 0 && K % 64 == 0 && splits >= 1 && splits <= 16 && K / 32 % splits == 0,
+             "split_linear: sizes M %d N %d K %d in %d parts", M, N, K, splits);
+  TP_REQUIRE((((uintptr_t)x | (uintptr_t)w) & 15) == 0, "split_linear: operands must be aligned to 16 bytes");
+  hipLaunchKernelGGL(split_linear_kernel, dim3(N / 16, splits), dim3(DG_WAVES * 64), 0, s, (const bf16_t*)x, (const bf16_t*)w, out, M, N, K);
+  TP_CHECK_LAUNCH("split_linear");
+  return 0;
+}
+
 // ---- routed experts ---------------------------------------------------------------------------------
 // Up: a[m][e * ff + c] = f(x_m . up_e[c]) * dense[m][e] as bfloat16, k-blocked over the columns of all experts; experts whose
 // column of `dense` is zero for all rows are skipped (their columns stay unwritten).  GATED: the weight's rows alternate
@@ -220,7 +253,8 @@ extern "C" int tp_moe_open(const void* x, const void* w_router, const float* cor
 }
 
 // Down: y[m] (+)= sum_e a[m][e] . down_e, experts ascending; the same experts are skipped.  w: every expert's tiled [N, ff], one
-// behind the other.  ws: then the shared expert's tiled [N, size] (nullptr: none) times a_shared, its sum added on its own, times
+// behind the other.  gridDim.y > 1: every expert's K in that many equal parts of whole runs, y [parts, M, N] (see split_linear_kernel).
+// ws: then the shared expert's tiled [N, size] (nullptr: none) times a_shared, its sum added on its own, times
 // sigmoid(gate[m]) where there is a gate.
 __global__ __launch_bounds__(DG_WAVES * 64) void moe_down_kernel(const bf16_t* __restrict__ a, const bf16_t* __restrict__ w,
                                                                   const float* __restrict__ dense, float* __restrict__ y, int M, int experts,
@@ -246,11 +280,12 @@ __global__ __launch_bounds__(DG_WAVES * 64) void moe_down_kernel(const bf16_t* _
   if (used) list[before + __popcll(mask & ((1ull << lane) - 1ull))] = threadIdx.x;
   __syncthreads();
 
-  const int n0 = blockIdx.x * 16, steps = ff / 32, runs = (steps + 3) / 4;
+  const int n0 = blockIdx.x * 16, steps = ff / 32 / gridDim.y, runs = (steps + 3) / 4;
   const int row = min(lane & 15, M - 1);
   const int xstep = 4 * M;
-  const u32x4_t* w_lane = (const u32x4_t*)(w + (size_t)n0 * ff) + lane;
-  const u32x4_t* x_lane = (const u32x4_t*)(a + ((size_t)(lane >> 4) * M + row) * 8);
+  const size_t first = (size_t)blockIdx.y * steps;
+  const u32x4_t* w_lane = (const u32x4_t*)(w + (size_t)n0 * ff) + lane + first * 64;
+  const u32x4_t* x_lane = (const u32x4_t*)(a + ((size_t)(lane >> 4) * M + row) * 8) + first * xstep;
   const size_t w_expert = (size_t)N * ff / 8, x_expert = (size_t)(ff / 8) * M;   // in pieces of 16 bytes
   // run r of expert e goes to wave (e * runs + r) % 8: `per` turns an expert
   const int per = (runs + DG_WAVES - 1) / DG_WAVES;
@@ -282,8 +317,11 @@ __global__ __launch_bounds__(DG_WAVES * 64) void moe_down_kernel(const bf16_t* _
 #pragma unroll
   for (int r = 0; r < 4; ++r) red[wave][lane * 4 + r] = acc[r];
   if (ws != nullptr) {
-    const f32x4_t sum = dg_tile((const u32x4_t*)(ws + (size_t)n0 * size) + lane, (const u32x4_t*)(a_shared + ((size_t)(lane >> 4) * M + row) * 8),
-                                xstep, size / 32, wave, (f32x4_t){0.f, 0.f, 0.f, 0.f});
+    const int steps_s = size / 32 / gridDim.y;
+    const size_t first_s = (size_t)blockIdx.y * steps_s;
+    const f32x4_t sum = dg_tile((const u32x4_t*)(ws + (size_t)n0 * size) + lane + first_s * 64,
+                                (const u32x4_t*)(a_shared + ((size_t)(lane >> 4) * M + row) * 8) + first_s * xstep, xstep, steps_s, wave,
+                                (f32x4_t){0.f, 0.f, 0.f, 0.f});
 #pragma unroll
     for (int r = 0; r < 4; ++r) red_s[wave][lane * 4 + r] = sum[r];
   }
@@ -292,7 +330,7 @@ __global__ __launch_bounds__(DG_WAVES * 64) void moe_down_kernel(const bf16_t* _
   if (q >= 256) return;
   const int l = q / 4, m = l & 15;
   if (m >= M) return;
-  float* o = y + (size_t)m * N + n0 + (l >> 4) * 4 + q % 4;
+  float* o = y + ((size_t)blockIdx.y * M + m) * N + n0 + (l >> 4) * 4 + q % 4;
   float v = dg_sum(red, q);
   if (accumulate) v = *o + v;
   if (ws != nullptr) {
@@ -304,10 +342,12 @@ __global__ __launch_bounds__(DG_WAVES * 64) void moe_down_kernel(const bf16_t* _
 
 // x: bfloat16 [K / 8, M, 8]; w_up: tiled [experts * rows, K], rows = ff, or 2 ff with gated (kind is then not read); w_down: experts
 // tiled [N, ff]; dense float32 [M, experts]; a: bfloat16 scratch [experts * ff / 8, M, 8]; y float32 [M, N].  w_shared (nullptr: none):
-// tiled [N, size], a_shared and gate (nullptr: none) as tp_moe_open leaves them.
+// tiled [N, size], a_shared and gate (nullptr: none) as tp_moe_open leaves them.  parts > 1: y [parts, M, N], partial sums.
 extern "C" int tp_moe_few(const void* x, const void* w_up, const void* w_down, const float* dense, void* a, float* y, int M, int experts,
                           int ff, int K, int N, int gated, int kind, int accumulate, const void* w_shared, const void* a_shared, const float* gate,
-                          int size, hipStream_t s) {
+                          int size, int parts, hipStream_t s) {
+  TP_REQUIRE(parts >= 1 && parts <= 16 && (parts == 1 || (!accumulate && ff / 32 % parts == 0 && (w_shared == nullptr || size / 32 % parts == 0))),
+             "moe_few: K in %d parts", parts);
   TP_REQUIRE(w_shared == nullptr || (size > 0 && size % 64 == 0 && a_shared && (((uintptr_t)w_shared | (uintptr_t)a_shared) & 15) == 0),
              "moe_few: bad shared expert");
   TP_REQUIRE(M > 0 && M <= 16 && experts > 0 && experts <= DG_MAX_EXPERTS, "moe_few: %d rows, %d experts", M, experts);
@@ -321,7 +361,7 @@ extern "C" int tp_moe_few(const void* x, const void* w_up, const void* w_down, c
     hipLaunchKernelGGL(moe_up_kernel<true>, up, block, 0, s, (const bf16_t*)x, (const bf16_t*)w_up, dense, (bf16_t*)a, M, experts, rows, K, 0);
   else
     hipLaunchKernelGGL(moe_up_kernel<false>, up, block, 0, s, (const bf16_t*)x, (const bf16_t*)w_up, dense, (bf16_t*)a, M, experts, rows, K, kind);
-  hipLaunchKernelGGL(moe_down_kernel, dim3(N / 16), block, 0, s, (const bf16_t*)a, (const bf16_t*)w_down, dense, y, M, experts, ff, N, accumulate,
+  hipLaunchKernelGGL(moe_down_kernel, dim3(N / 16, parts), block, 0, s, (const bf16_t*)a, (const bf16_t*)w_down, dense, y, M, experts, ff, N, accumulate,
                      (const bf16_t*)w_shared, (const bf16_t*)a_shared, gate, size);
   TP_CHECK_LAUNCH("moe_few");
   return 0;

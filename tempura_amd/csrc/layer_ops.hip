@@ -175,12 +175,13 @@ template <typename TO>
 __global__ __launch_bounds__(256) void norm_add_kernel(float* __restrict__ h, const float* __restrict__ y,
                                                        const float* __restrict__ w, float eps,
                                                        const float* __restrict__ w_next, float eps_next,
-                                                       TO* __restrict__ x, int width, InputGate gate, int normed, int blocked) {
+                                                       TO* __restrict__ x, int width, InputGate gate, int normed, int blocked, int parts) {
   __shared__ float scratch[32];
   const size_t base = (size_t)blockIdx.x * width;
   const float* gr = gate.rows != nullptr ? gate.rows + (size_t)blockIdx.x * gate.stride + gate.col0 : nullptr;
   auto value = [&](int c) {
-    const float v = y[base + c];
+    float v = y[base + c];
+    for (int p = 1; p < parts; ++p) v += y[(size_t)p * gridDim.x * width + base + c];
     return gr != nullptr ? v * l_sigmoid(gr[c] + (gate.bias != nullptr ? gate.bias[c] : 0.f)) : v;
   };
   float rstd = 1.0f;
@@ -214,7 +215,7 @@ template <typename TO, int NV, bool GATE>
 __global__ __launch_bounds__(256) void norm_add_reg_kernel(float* __restrict__ h, const float* __restrict__ y,
                                                            const float* __restrict__ w, float eps,
                                                            const float* __restrict__ w_next, float eps_next,
-                                                           TO* __restrict__ x, int width, InputGate gate, int normed, int blocked) {
+                                                           TO* __restrict__ x, int width, InputGate gate, int normed, int blocked, int parts) {
   __shared__ float scratch[32];
   const size_t base = (size_t)blockIdx.x * width;
   const int w4 = width / 4;
@@ -227,6 +228,22 @@ __global__ __launch_bounds__(256) void norm_add_reg_kernel(float* __restrict__ h
       hv[k] = *(const float4*)(h + base + 4 * c);
       wv[k] = *(const float4*)(w + 4 * c);
     }
+  }
+  // (parts > 1: y is that many partial sums of a product, added in ascending order)
+  for (int p = 1; p < parts; ++p) {
+    const float* yp = y + (size_t)p * gridDim.x * width + base;
+    float4 more[NV];
+#pragma unroll
+    for (int k = 0; k < NV; ++k)
+      if (k * 256 + threadIdx.x < w4) more[k] = *(const float4*)(yp + 4 * (k * 256 + threadIdx.x));
+#pragma unroll
+    for (int k = 0; k < NV; ++k)
+      if (k * 256 + threadIdx.x < w4) {
+        yv[k].x += more[k].x;
+        yv[k].y += more[k].y;
+        yv[k].z += more[k].z;
+        yv[k].w += more[k].w;
+      }
   }
   if constexpr (GATE) {
     const float* gr = gate.rows + (size_t)blockIdx.x * gate.stride + gate.col0;
@@ -295,7 +312,8 @@ __global__ __launch_bounds__(256) void norm_add_reg_kernel(float* __restrict__ h
 
 extern "C" int tp_norm_add(float* h, const float* y, const float* w, float eps, const float* w_next, float eps_next, void* x,
                            int x_dt, int n, int width, const float* gate_rows, size_t gate_stride, int gate_col0,
-                           const float* gate_bias, int normed, int blocked, hipStream_t s) {
+                           const float* gate_bias, int normed, int blocked, int parts, hipStream_t s) {
+  TP_REQUIRE(parts >= 1, "norm_add: bad parts");
   TP_REQUIRE(n >= 0 && width > 0, "norm_add: bad sizes");
   TP_REQUIRE(gate_rows == nullptr || (gate_col0 >= 0 && gate_stride >= (size_t)gate_col0 + width), "norm_add: gate rows too short");
   const InputGate gate{gate_rows, gate_bias, gate_stride, gate_col0};
@@ -309,7 +327,7 @@ extern "C" int tp_norm_add(float* h, const float* y, const float* w, float eps, 
   if (width % 4 == 0 && width >= 1024 && width <= 256 * 4 * 8 && aligned) {
     const bool bf = w_next != nullptr && x_dt == TP_BF16;
 #define NA1(TO, NV, G) \
-  hipLaunchKernelGGL((norm_add_reg_kernel<TO, NV, G>), dim3(n), dim3(256), 0, s, h, y, w, eps, w_next, eps_next, (TO*)x, width, gate, normed, blocked)
+  hipLaunchKernelGGL((norm_add_reg_kernel<TO, NV, G>), dim3(n), dim3(256), 0, s, h, y, w, eps, w_next, eps_next, (TO*)x, width, gate, normed, blocked, parts)
 #define NA(NV)                                    \
   do {                                            \
     if (gate_rows != nullptr) {                   \
@@ -330,9 +348,9 @@ extern "C" int tp_norm_add(float* h, const float* y, const float* w, float eps, 
   }
   const int threads = width >= 1024 ? 256 : (width >= 256 ? 128 : 64);
   if (w_next == nullptr || x_dt == TP_F32)
-    hipLaunchKernelGGL(norm_add_kernel<float>, dim3(n), dim3(threads), 0, s, h, y, w, eps, w_next, eps_next, (float*)x, width, gate, normed, blocked);
+    hipLaunchKernelGGL(norm_add_kernel<float>, dim3(n), dim3(threads), 0, s, h, y, w, eps, w_next, eps_next, (float*)x, width, gate, normed, blocked, parts);
   else if (x_dt == TP_BF16)
-    hipLaunchKernelGGL(norm_add_kernel<bf16_t>, dim3(n), dim3(threads), 0, s, h, y, w, eps, w_next, eps_next, (bf16_t*)x, width, gate, normed, blocked);
+    hipLaunchKernelGGL(norm_add_kernel<bf16_t>, dim3(n), dim3(threads), 0, s, h, y, w, eps, w_next, eps_next, (bf16_t*)x, width, gate, normed, blocked, parts);
   else
     TP_REQUIRE(false, "norm_add: unknown dtype %d", x_dt);
   TP_CHECK_LAUNCH("norm_add");

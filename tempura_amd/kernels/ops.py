@@ -539,7 +539,7 @@ def _w_args(w):
 class Partials:
     """The float32 partial sums [splits, m, n] of a product whose K was split over blocks, not yet added:
     the kernel that consumes the rows adds them (in ascending order), which saves the reduction kernel.
-    Made by ``linear(..., partial_ok=True)``, taken by ``rope_kv_write``."""
+    Made by ``linear(..., partial_ok=True)`` and ``moe_few(..., parts)``, taken by ``rope_kv_write``, ``attention_rows`` and ``norm_add``."""
     __slots__ = ("data",)
 
     def __init__(self, data):
@@ -695,6 +695,26 @@ def linear_gate_f32(x, w: torch.Tensor) -> torch.Tensor:
     return _f32_rows(x, w, True)
 
 
+def few_splits(m: int, n: int, k: int) -> int:
+    """Into how many parts the K of a product of ``m`` <= 16 rows onto ``n`` columns is cut where its consumer adds partial sums: until
+    there are 256 blocks of 16 columns, a run of 128 a wave left in each."""
+    # (from 4,096 of K on, 9.3 / 8.5 us at 2,048 columns; a shorter one is a single trip to memory for every wave anyway)
+    splits = 1
+    while allow_mfma and 0 < m <= 16 and k >= 4096 and splits < 4 and 2 * splits * (n // 16) <= 256 and k % (2048 * splits) == 0:
+        splits *= 2
+    return splits
+
+
+def _split_linear(x: KBlocked, w) -> "Partials":
+    m, (n, k) = x.rows, w.shape
+    _dev_ok(x.data, w.data)
+    _need(tuple(x.data.shape) == (k // 8, m, 8) and x.data.dtype == w.dtype == torch.bfloat16, "linear: malformed k-blocked rows")
+    splits = few_splits(m, n, k)
+    out = torch.empty((splits, m, n), dtype=torch.float32, device=x.data.device)
+    _call("tp_split_linear", _ptr(x.data), _ptr(w.data), _ptr(out), m, n, k, splits, _stream(), tag=(m, n, k))
+    return Partials(out)
+
+
 def linear(x, w: torch.Tensor, out_dtype: torch.dtype, residual: Optional[torch.Tensor] = None, next_norm=None,
            partial_ok: bool = False):
     """x [m, k] (or ``Prenormed`` / ``KBlocked`` / ``Unnormed`` without a residual) @ w[n, k]^T -> out_dtype [m, n]; with ``residual`` (float32
@@ -703,7 +723,8 @@ def linear(x, w: torch.Tensor, out_dtype: torch.dtype, residual: Optional[torch.
     for the part behind that norm): ``Prenormed`` rows up to 16 rows of bfloat16, the normed rows themselves
     from 17 rows on when the product's K was split (one kernel adds the partial sums into the residual and norms
     it), or None when the norm has to run on its own.
-    With ``partial_ok`` (float32 output, no residual) the result may be ``Partials``."""
+    With ``partial_ok`` (float32 output, no residual) the result may be ``Partials`` (of up to 16 rows: k-blocked ones and a tiled
+    weight with few column blocks and a long K, ``few_splits``)."""
     if _backend is not None:
         if next_norm is not None:
             return _backend.linear(x, w, out_dtype, residual, next_norm)
@@ -715,6 +736,9 @@ def linear(x, w: torch.Tensor, out_dtype: torch.dtype, residual: Optional[torch.
             return _f32_rows(x, w, False)
         x = rmsnorm(x.x, x.weight, x.eps, torch.float32)
     if isinstance(x, KBlocked):
+        if partial_ok and residual is None and next_norm is None and out_dtype == torch.float32 and isinstance(w, TiledWeight) \
+                and few_splits(x.rows, w.shape[0], w.shape[1]) > 1 and x.width == w.shape[1]:
+            return _split_linear(x, w)
         _need(allow_mfma and x.data.dtype == torch.bfloat16 and tuple(x.data.shape) == (x.width // 8, x.rows, 8)
               and x.width % 32 == 0, "linear: malformed k-blocked rows")
         kb, layout = x, 1
@@ -1693,7 +1717,8 @@ def head_linear(x: torch.Tensor, x_col0: int, x_head: int, w: torch.Tensor, out:
 def norm_add(h: torch.Tensor, y: torch.Tensor, weight: torch.Tensor, eps: float, next_weight: Optional[torch.Tensor] = None,
              next_eps: float = 0.0, out_dtype: Optional[torch.dtype] = None, gate: Optional[torch.Tensor] = None, gate_col0: int = 0,
              gate_bias: Optional[torch.Tensor] = None, normed: bool = True, blocked: bool = False):
-    """h += y / sqrt(mean(y^2) + eps) * weight (not ``normed``: h += y * weight), per row, in place (float32 [n, width]).  With ``next_weight`` the
+    """h += y / sqrt(mean(y^2) + eps) * weight (not ``normed``: h += y * weight), per row, in place (float32 [n, width]; y may be
+    ``Partials``).  With ``next_weight`` the
     rows of the new h normed with it (and ``next_eps``) come back as ``out_dtype``.  With ``gate`` (float32 rows [n,
     wider]) y is first multiplied by sigmoid(gate[:, gate_col0 + c] + gate_bias[c]).  ``blocked``: the rows come back as
     ``KBlocked`` (see ``few_rows_ok``)."""
@@ -1701,8 +1726,12 @@ def norm_add(h: torch.Tensor, y: torch.Tensor, weight: torch.Tensor, eps: float,
         if gate is not None:
             return _backend.norm_add(h, y, weight, eps, next_weight, next_eps, out_dtype, gate, gate_col0, gate_bias)
         return _backend.norm_add(h, y, weight, eps, next_weight, next_eps, out_dtype)
+    parts = 1
+    if isinstance(y, Partials):
+        parts, y = y.data.shape[0], y.data.view(-1, y.data.shape[2])
+        _need(y.shape[0] == parts * h.shape[0] and y.is_contiguous(), "norm_add: malformed partial sums")
     _dev_ok(h, y, weight, next_weight, gate, gate_bias)
-    _need(h.dtype == torch.float32 and h.dim() == 2 and y.dtype == torch.float32 and tuple(y.shape) == tuple(h.shape),
+    _need(h.dtype == torch.float32 and h.dim() == 2 and y.dtype == torch.float32 and tuple(y.shape) == (parts * h.shape[0], h.shape[1]),
           "norm_add: h and y must be float32 [n, width]")
     n, width = h.shape
     _need(weight.dtype == torch.float32 and weight.numel() == width, "norm_add: weight must be float32 [width]")
@@ -1716,7 +1745,7 @@ def norm_add(h: torch.Tensor, y: torch.Tensor, weight: torch.Tensor, eps: float,
         x = torch.empty((width // 8, n, 8) if blocked else (n, width), dtype=out_dtype, device=h.device)
     _call("tp_norm_add", _ptr(h), _ptr(y), _ptr(weight), ctypes.c_float(eps), _ptr(next_weight), ctypes.c_float(next_eps), _ptr(x),
           _dtcode(out_dtype) if x is not None else _F32, n, width, _ptr(gate), ctypes.c_size_t(0 if gate is None else gate.shape[1]),
-          int(gate_col0), _ptr(gate_bias), int(normed), int(blocked), _stream())
+          int(gate_col0), _ptr(gate_bias), int(normed), int(blocked), parts, _stream())
     return KBlocked(x, n, width) if blocked and x is not None else x
 
 
@@ -2425,13 +2454,13 @@ def moe_open(x: KBlocked, w_router, correction: Optional[torch.Tensor], experts:
 
 
 def moe_few(x: KBlocked, w_up, w_down, dense: torch.Tensor, ff: int, activation: Optional[str], y: Optional[torch.Tensor] = None,
-            shared: Optional[tuple] = None) -> torch.Tensor:
+            shared: Optional[tuple] = None, partial_ok: bool = False):
     """The routed experts of at most 16 rows: y (+)= sum_e down_e(f(up_e x) * dense[:, e]), skipping the weights of experts
     whose column of ``dense`` (float32 [m, experts]) is zero.  ``w_up``: the experts' tiled up weights stacked
     ([experts * ff, k]; ``activation`` None: gate and up rows interleaved by eights, [2 experts * ff, k], f = silu(gate) * up);
     ``w_down``: their tiled [n, ff] one behind the other, as a ``TiledWeight`` of [experts * n, ff].  ``y`` float32 [m, n] or None.
     ``shared`` = (tiled down weight [n, size], activated rows, raw gate or None, as of ``moe_open``): the shared expert's output behind
-    the routed sum, times sigmoid(gate)."""
+    the routed sum, times sigmoid(gate).  With ``partial_ok`` and no ``y`` the result may be ``Partials`` (``few_splits``)."""
     m, k = x.shape
     experts = dense.shape[1]
     w_s, a_s, gate = shared if shared is not None else (None, None, None)
@@ -2446,10 +2475,15 @@ def moe_few(x: KBlocked, w_up, w_down, dense: torch.Tensor, ff: int, activation:
         _need(w_s.shape[0] == n and tuple(a_s.shape) == (w_s.shape[1] // 8, m, 8) and a_s.dtype == torch.bfloat16 and
               (gate is None or (gate.dtype == torch.float32 and gate.numel() == m)), "moe_few: shared expert disagrees with the sizes")
     acc = y is not None
+    # (an expert's own K is what is cut, so that a row's sums do not depend on the experts of the rows beside it; whole turns of eight runs)
+    parts = 1
+    while partial_ok and not acc and parts < 4 and 2 * parts * (n // 16) <= 256 and ff % (2048 * parts) == 0 and \
+            (w_s is None or w_s.shape[1] % (64 * parts) == 0):
+        parts *= 2
     if not acc:
-        y = torch.empty((m, n), dtype=torch.float32, device=dense.device)
+        y = torch.empty((parts, m, n) if parts > 1 else (m, n), dtype=torch.float32, device=dense.device)
     a = torch.empty((experts * ff // 8, m, 8), dtype=torch.bfloat16, device=dense.device)
     _call("tp_moe_few", _ptr(x.data), _ptr(w_up.data), _ptr(w_down.data), _ptr(dense), _ptr(a), _ptr(y), m, experts, int(ff), k, n,
           int(activation is None), 0 if activation is None else ACTIVATIONS[activation], int(acc), _ptr(None if w_s is None else w_s.data), _ptr(a_s),
-          _ptr(gate), 0 if w_s is None else w_s.shape[1], _stream(), tag=(m, experts, ff, k))
-    return y
+          _ptr(gate), 0 if w_s is None else w_s.shape[1], parts, _stream(), tag=(m, experts, ff, k))
+    return y if parts == 1 else Partials(y)

@@ -82,6 +82,8 @@ class Part:
     input_dtype: Optional[torch.dtype] = None
     #: True: in a step of a few single tokens the rows may come k-blocked (``ops.KBlocked``), for blocks that ask
     takes_blocked_rows = False
+    #: set by a block whose closing kernel adds partial sums: ``forward`` without a residual may return ``ops.Partials`` for its rows
+    partial_output = False
 
     def __init__(self, spec: PartSpec, hidden_size: int, dtype: torch.dtype, device):
         self.spec = spec
@@ -106,6 +108,9 @@ class Part:
         """Called before ``load_weights`` with rows [r, hidden].  ``forward`` (with ``residual`` None) then returns the pair
         (output, (float32 rows, first column)): the r products of these rows with the input, from that column on."""
         self.side_rows = rows
+
+    def _partial(self, residual) -> dict:
+        return {"partial_ok": True} if self.partial_output and residual is None else {}
 
     def _to_device(self, t: torch.Tensor, dtype: Optional[torch.dtype] = None) -> torch.Tensor:
         return t.to(device=self.device, dtype=dtype or self.dtype).contiguous()

@@ -291,6 +291,8 @@ class SandwichBlock(ArrangedBlock):
         self._check_parts()
         self.hidden_size = hidden_size
         self.dtype = dtype
+        if self.ffn is not None:
+            self.ffn.partial_output = True
 
     def _check_parts(self):
         if len({self.ffn is None, self.ffn_norm is None, self.ffn_post_norm is None}) != 1:

@@ -105,7 +105,7 @@ class GatedFFN(FeedForward):
             # (sizes the fused product does not take: the product's float32 sums, then the activation)
             gu = ops.linear(x, self.w13, torch.float32)
             a = ops.gated_act(gu, self.dtype, self.slope, self.limit, self.up_offset)
-        return ops.linear(a, self.w2, torch.float32, residual=residual)
+        return ops.linear(a, self.w2, torch.float32, residual=residual, **self._partial(residual))
 
 
 class DenseMLP(FeedForward):
@@ -144,7 +144,7 @@ class DenseMLP(FeedForward):
         if self.fused or ops.linear_act_ok(x.shape[0], self.intermediate_size, self.hidden_size, self.dtype):
             # (a few rows go to the down product k-blocked: it reads them straight from global memory)
             a, side = ops.linear_relu2(x, self.w_up, self.intermediate_size, blocked_out=True, **({} if self.fused else {"kind": self.activation}))
-            y = ops.linear(a, self.w_down, torch.float32, residual=residual)
+            y = ops.linear(a, self.w_down, torch.float32, residual=residual, **self._partial(residual))
             return y if self.side_rows is None else (y, (side, 0))
         u = ops.linear(x, self.w_up, torch.float32)
         if self.side_rows is not None:
@@ -332,7 +332,7 @@ class RoutedExperts(FeedForward):
         if opened is not None:
             down = (self.w_shared_down,) + opened
         y = ops.moe_few(rows, self.w13_all, self.w2_all, dense, self.intermediate_size, self.activation if self.expert_kind == "plain" else None,
-                        residual, down)
+                        residual, down, **self._partial(residual))
         return y if residual is None else None
 
     def _opens(self, m):

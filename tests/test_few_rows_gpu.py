@@ -333,3 +333,67 @@ def test_router_beside_the_shared_expert(m, experts, top, groups, keep, k, ff, s
     add = act @ w_sd.double().t() * (torch.sigmoid(u[:, size:size + 1]) if gated else 1.0)
     # (the activations are rounded to bfloat16: 2^-9 of each term, whose sum over `size` of them is off by that much of its norm)
     assert float((y.double() - 1.0 - plain.double() - add).norm()) <= 2.0 ** -8 * float(add.norm()) + 1e-5 * float(plain.norm())
+
+
+@pytest.mark.parametrize("m", [1, 3, 16])
+@pytest.mark.parametrize("n,k,parts", [(16, 4096, 4), (2048, 4096, 2), (1024, 8192, 4), (4096, 8192, 1), (2064, 8192, 1), (272, 6144, 2)])
+@pytest.mark.parametrize("blocked", [True, False])
+def test_few_column_blocks_leave_parts(m, n, k, parts, blocked):
+    """Products of few column blocks against float64, and the norm that adds their parts against the norm of the added rows."""
+    from tempura_amd.kernels import ops
+    g = torch.Generator().manual_seed(m + n + k)
+    x, w = torch.randn(m, k, generator=g).to(DEV).bfloat16(), (torch.randn(n, k, generator=g) * 0.05).to(DEV).bfloat16()
+    assert ops.few_splits(m, n, k) == parts and ops.few_splits(17, n, k) == 1
+    y = ops.linear(ops.block_rows(x), ops.tile_weight(w), torch.float32, partial_ok=True)
+    assert isinstance(y, ops.Partials) == (parts > 1)
+    total = y
+    if parts > 1:
+        total = y.data[0].clone()
+        for p in range(1, parts):
+            total += y.data[p]
+    ref = x.double() @ w.double().t()
+    # (k products of float32 sums: rounding of the running sum, 2^-24 of it each, as a random walk)
+    assert float((total.double() - ref).abs().max()) <= 2.0 ** -24 * k ** 0.5 * 4 * float(ref.abs().max())
+    wide = torch.randn(m, n + 8, generator=g).to(DEV)
+    nw, bias = torch.rand(n, generator=g).to(DEV), torch.rand(n, generator=g).to(DEV)
+    for gate in (None, wide):
+        for normed in (True, False):
+            h0 = torch.randn(m, n, generator=g).to(DEV)
+            h1 = h0.clone()
+            more = dict(gate=gate, gate_col0=4, gate_bias=bias) if gate is not None else {}
+            a = ops.norm_add(h0, y, nw, 1e-5, bias, 1e-6, torch.bfloat16, normed=normed, blocked=blocked and n % 64 == 0, **more)
+            b = ops.norm_add(h1, total, nw, 1e-5, bias, 1e-6, torch.bfloat16, normed=normed, blocked=blocked and n % 64 == 0, **more)
+            assert torch.equal(h0, h1) and torch.equal(getattr(a, "data", a), getattr(b, "data", b))
+
+
+@pytest.mark.parametrize("width", [6, 1028, 20484])
+def test_norm_of_partial_sums(width):
+    """The norm kernels' other widths (no whole vectors, more than the registers hold) with three parts."""
+    from tempura_amd.kernels import ops
+    g = torch.Generator().manual_seed(width)
+    y, h0, w = torch.randn(3, 5, width, generator=g).to(DEV), torch.randn(5, width, generator=g).to(DEV), torch.rand(width, generator=g).to(DEV)
+    h1 = h0.clone()
+    a = ops.norm_add(h0, ops.Partials(y), w, 1e-5, w, 1e-5, torch.bfloat16)
+    b = ops.norm_add(h1, y[0] + y[1] + y[2], w, 1e-5, w, 1e-5, torch.bfloat16)
+    assert torch.equal(h0, h1) and torch.equal(a, b)
+
+
+@pytest.mark.parametrize("m,experts", [(1, 8), (4, 8), (16, 3)])
+@pytest.mark.parametrize("ff,n,parts", [(2048, 96, 2), (4096, 1024, 4), (2112, 96, 1), (2048, 2064, 1)])
+@pytest.mark.parametrize("size", [0, 512])
+def test_experts_down_products_in_parts(m, experts, ff, n, parts, size):
+    from tempura_amd.kernels import ops
+    g = torch.Generator().manual_seed(m + ff + n)
+    rnd = lambda *s: (torch.randn(*s, generator=g) * 0.1).to(DEV).bfloat16()
+    x, w_up, w_down = ops.block_rows(rnd(m, 64)), ops.tile_weight(rnd(experts * ff, 64)), rnd(experts, n, ff)
+    w_down = ops.TiledWeight(torch.cat([ops.tile_weight(w).data for w in w_down]), experts * n, ff)
+    dense = torch.rand(m, experts, generator=g) * (torch.rand(m, experts, generator=g) < 0.5)
+    shared = (ops.tile_weight(rnd(n, size)), ops.block_rows(rnd(m, size)).data, torch.randn(m, generator=g).to(DEV)) if size else None
+    args = (x, w_up, w_down, dense.to(DEV), ff, "silu", None, shared)
+    want, got = ops.moe_few(*args), ops.moe_few(*args, partial_ok=True)
+    assert isinstance(got, ops.Partials) == (parts > 1)
+    if parts > 1:
+        assert got.data.shape == (parts, m, n)
+        got = got.data.double().sum(0)
+    # (the same products added in another order: 2^-24 of the sum of magnitudes at each of some hundred additions, as a random walk)
+    assert float((got - want.double()).abs().max()) <= 2.0 ** -24 * 64 * max(1.0, float(want.abs().max()))

@@ -129,6 +129,91 @@ extern "C" int tp_split_linear(const void* x, const void* w, float* out, int M, 
   return 0;
 }
 
+// ---- a product that closes a sublayer over several copies of the stream ---------------------------
+// y = x w^T, then per row and column, in the order of hc_step_reg_kernel: h'[b] = sum_a mix[a, b] h[a] + outc[b] y, written back into
+// h [M, S, N]; with norm_w also u = sum_a inc[a] h'[a], handed over as xg = bfloat16(u * norm_w), k-blocked [N / 8, M, 8], and ss
+// [N / 16, 16], each block's sums of u^2 per row, for the next product to finish the norm (RowScale in gemm_mfma.hip).  The copies mix
+// column by column, so the block that has a column's sum has all it needs; what it reads besides is requested before the weights.
+// Bound by the weights' stream, as the product alone.  Four copies, a captured chain, product and closing kernel / together, one row and
+// eight: 4,096 x 4,096 11.4 / 8.4 and 12.8 / 8.9 us, 4,096 x 14,336 25.2 / 22.1 and 26.5 / 22.8, 2,048 x 7,168 13.7 / 11.5 and 15.2 / 12.2,
+// 1,024 x 2,048 6.8 / 4.7 and 7.3 / 4.7; sixteen rows of 4,096 x 14,336 28.9 / 25.1.
+struct StreamEnd {
+  const float *mix, *outc, *inc, *norm_w;   // nullptr: identity, ones, ones, no norm behind
+  bf16_t* xg;
+  float* ss;
+};
+
+__global__ __launch_bounds__(DG_WAVES * 64) void stream_linear_kernel(const bf16_t* __restrict__ x, int blocked, const bf16_t* __restrict__ w,
+                                                                       float* __restrict__ h, StreamEnd e, int M, int N, int K) {
+  __shared__ float red[DG_WAVES][256];
+  __shared__ float part[4][16];
+  constexpr int S = 4;
+  const int lane = threadIdx.x % 64, wave = threadIdx.x / 64;
+  const int n0 = blockIdx.x * 16;
+  const int q = threadIdx.x, l = q / 4, m = l & 15, n = n0 + ((l >> 4) & 3) * 4 + q % 4;
+  const bool mine = q < 256 && m < M;
+  float v[S], wn = 0.f, mc[S * S], oc[S], ic[S];
+  float* hp = h + (size_t)m * S * N + n;
+  if (mine) {
+#pragma unroll
+    for (int a = 0; a < S; ++a) v[a] = hp[(size_t)a * N];
+    if (e.norm_w != nullptr) wn = e.norm_w[n];
+  }
+#pragma unroll
+  for (int a = 0; a < S; ++a) {
+#pragma unroll
+    for (int b = 0; b < S; ++b) mc[a * S + b] = e.mix ? e.mix[a * S + b] : (a == b ? 1.f : 0.f);
+    oc[a] = e.outc ? e.outc[a] : 1.f;
+    ic[a] = e.inc ? e.inc[a] : 1.f;
+  }
+  const u32x4_t* wp = (const u32x4_t*)(w + (size_t)n0 * K) + lane;
+  const int row = min(lane & 15, M - 1);
+  const u32x4_t* xp = blocked ? (const u32x4_t*)x + (size_t)(lane >> 4) * M + row : (const u32x4_t*)(x + (size_t)row * K) + (lane >> 4);
+  const f32x4_t acc = dg_tile(wp, xp, blocked ? 4 * M : 4, K / 32, wave, (f32x4_t){0.f, 0.f, 0.f, 0.f});
+#pragma unroll
+  for (int r = 0; r < 4; ++r) red[wave][lane * 4 + r] = acc[r];
+  __syncthreads();
+  if (q < 256) {
+    float sq = 0.f;
+    if (mine) {
+      const float y = dg_sum(red, q);
+      float u = 0.f;
+#pragma unroll
+      for (int b = 0; b < S; ++b) {
+        float t = 0.f;
+#pragma unroll
+        for (int a = 0; a < S; ++a) t = fmaf(mc[a * S + b], v[a], t);
+        t = fmaf(oc[b], y, t);
+        hp[(size_t)b * N] = t;
+        u = fmaf(ic[b], t, u);
+      }
+      if (e.norm_w != nullptr) e.xg[((size_t)(n >> 3) * M + m) * 8 + (n & 7)] = float_to_bf16(u * wn);
+      sq = u * u;
+    }
+    sq += __shfl_xor(sq, 1, 64);      // the four columns of this lane's row
+    sq += __shfl_xor(sq, 2, 64);
+    if (q % 4 == 0) part[l >> 4][m] = sq;
+  }
+  if (e.norm_w == nullptr) return;   // (the same for every thread)
+  __syncthreads();
+  if (threadIdx.x < 16)
+    e.ss[blockIdx.x * 16 + threadIdx.x] = part[0][threadIdx.x] + part[1][threadIdx.x] + part[2][threadIdx.x] + part[3][threadIdx.x];
+}
+
+// x: bfloat16 [K / 8, M, 8] (blocked) or [M, K]; w: tiled [N, K]; h float32 [M, streams, N]; mix float32 [streams, streams], outc and inc
+// [streams], norm_w [N] (each may be nullptr); xg bfloat16 [N / 8, M, 8] and ss [N / 16, 16] with norm_w
+extern "C" int tp_stream_linear(const void* x, int blocked, const void* w, float* h, int streams, const float* mix, const float* outc,
+                                const float* inc, const float* norm_w, void* xg, float* ss, int M, int N, int K, hipStream_t s) {
+  TP_REQUIRE(M > 0 && M <= 16 && N > 0 && N % 16 == 0 && K > 0 && K % 64 == 0, "stream_linear: sizes M %d N %d K %d", M, N, K);
+  TP_REQUIRE((((uintptr_t)x | (uintptr_t)w) & 15) == 0, "stream_linear: operands must be aligned to 16 bytes");
+  TP_REQUIRE(norm_w == nullptr || (xg != nullptr && ss != nullptr), "stream_linear: no room for the rows of the next norm");
+  const StreamEnd e = {mix, outc, inc, norm_w, (bf16_t*)xg, ss};
+  TP_REQUIRE(streams == 4, "stream_linear: %d copies of the stream (takes 4)", streams);
+  hipLaunchKernelGGL(stream_linear_kernel, dim3(N / 16), dim3(DG_WAVES * 64), 0, s, (const bf16_t*)x, blocked, (const bf16_t*)w, h, e, M, N, K);
+  TP_CHECK_LAUNCH("stream_linear");
+  return 0;
+}
+
 // ---- routed experts ---------------------------------------------------------------------------------
 // Up: a[m][e * ff + c] = f(x_m . up_e[c]) * dense[m][e] as bfloat16, k-blocked over the columns of all experts; experts whose
 // column of `dense` is zero for all rows are skipped (their columns stay unwritten).  GATED: the weight's rows alternate

@@ -695,6 +695,51 @@ def linear_gate_f32(x, w: torch.Tensor) -> torch.Tensor:
     return _f32_rows(x, w, True)
 
 
+class StreamClose:
+    """In the place of ``linear``'s residual: the product is a sublayer's output that closes the sublayer over ``streams`` copies of the
+    stream (``stream_step``: h, mix, out_coef); with ``opening`` = (in_coef, norm weight, eps) it also opens the next one, and ``linear``
+    returns that one's rows (``Prenormed`` where the product does it all, see ``stream_linear_ok``), else None."""
+    __slots__ = ("h", "streams", "mix", "out_coef", "opening")
+
+    def __init__(self, h, streams, mix, out_coef, opening=None):
+        self.h, self.streams, self.mix, self.out_coef, self.opening = h, streams, mix, out_coef, opening
+
+
+def stream_linear_ok(m: int, width: int, streams: int, dtype: torch.dtype) -> bool:
+    """Whether a product of ``m`` rows closes a sublayer over the copies itself: few rows (one tile of the matrix cores) and four copies."""
+    # (Two copies stay with the closing kernel.  The rows go on rounded in front of the norm's scale instead of behind it: errors of whole
+    # models are alike, 0.0025 of mifutar at 4,096 either way, but a small model of two copies with a bias that magnifies one score differs
+    # by chance in one token of 400, 0.030 -> 0.054, more than that model is held to.)
+    return _backend is None and allow_mfma and dtype == torch.bfloat16 and 0 < m <= 16 and width % 32 == 0 and streams == 4
+
+
+def _stream_linear(x, w, close: StreamClose):
+    m, k = x.shape
+    n, h = w.shape[0], close.h
+    blocked = isinstance(x, KBlocked)
+    if not (isinstance(w, TiledWeight) and stream_linear_ok(m, n, close.streams, w.dtype) and (blocked or (x.dtype == torch.bfloat16 and x.is_contiguous()))):
+        y = linear(x, w, torch.float32)
+        inc, weight, eps = close.opening or (None, None, 0.0)
+        return stream_step(h, close.streams, y, close.mix, close.out_coef, inc, weight, eps, None if weight is None else w.dtype)
+    data = x.data if blocked else x
+    _dev_ok(data, w.data, h, close.mix, close.out_coef)
+    _need(k == w.shape[1] and (not blocked or tuple(data.shape) == (k // 8, m, 8)), f"linear: shapes {(m, k)} x {tuple(w.shape)}")
+    _need(h.dtype == torch.float32 and tuple(h.shape) == (m, close.streams * n), "linear: the stream must be float32 [m, streams * n]")
+    s = close.streams
+    inc, weight, eps = close.opening or (None, None, 0.0)
+    for t, size in ((close.mix, s * s), (close.out_coef, s), (inc, s), (weight, n)):
+        if t is not None:
+            _dev_ok(t)
+            _need(t.dtype == torch.float32 and t.numel() == size, "linear: malformed coefficients of the streams")
+    handed = None
+    if weight is not None:
+        handed = Prenormed(torch.empty((n // 8, m, 8), dtype=torch.bfloat16, device=h.device),
+                           torch.empty((n // 16, 16), dtype=torch.float32, device=h.device), eps, (m, n))
+    _call("tp_stream_linear", _ptr(data), int(blocked), _ptr(w.data), _ptr(h), s, _ptr(close.mix), _ptr(close.out_coef), _ptr(inc),
+          _ptr(weight), _ptr(None if handed is None else handed.x), _ptr(None if handed is None else handed.ss), m, n, k, _stream(), tag=(m, n, k))
+    return handed
+
+
 def few_splits(m: int, n: int, k: int) -> int:
     """Into how many parts the K of a product of ``m`` <= 16 rows onto ``n`` columns is cut where its consumer adds partial sums: until
     there are 256 blocks of 16 columns, a run of 128 a wave left in each."""
@@ -723,8 +768,11 @@ def linear(x, w: torch.Tensor, out_dtype: torch.dtype, residual: Optional[torch.
     for the part behind that norm): ``Prenormed`` rows up to 16 rows of bfloat16, the normed rows themselves
     from 17 rows on when the product's K was split (one kernel adds the partial sums into the residual and norms
     it), or None when the norm has to run on its own.
+    ``residual`` may be a ``StreamClose``: the product goes into all copies of the stream, and the next sublayer's rows come back.
     With ``partial_ok`` (float32 output, no residual) the result may be ``Partials`` (of up to 16 rows: k-blocked ones and a tiled
     weight with few column blocks and a long K, ``few_splits``)."""
+    if isinstance(residual, StreamClose):
+        return _stream_linear(x, w, residual)
     if _backend is not None:
         if next_norm is not None:
             return _backend.linear(x, w, out_dtype, residual, next_norm)

@@ -78,6 +78,7 @@ class PagedAttention(Mixer):
     preferred_portion_align = 8
     split_norm = True      # takes rows whose norm its first product finishes; prepares the next norm in its last
     returns_output = True  # with ``residual`` None the output comes back instead of being added
+    closes_streams = takes_unfinished = True
     takes_side_rows = True  # (behind the gate's rows, or behind q | k | v where one kernel reads the projection's rows)
 
     def __init__(self, spec, hidden_size, dtype, device):
@@ -322,8 +323,8 @@ class PagedAttention(Mixer):
             if residual is not None:
                 raise ValueError("attention: with side rows the output comes back, it is not added")
             return ops.linear(a, self.wo, torch.float32), (gates, self.side_col0)
-        if residual is None:
-            return ops.linear(a, self.wo, torch.float32)
+        if residual is None or isinstance(residual, ops.StreamClose):
+            return ops.linear(a, self.wo, torch.float32, residual=residual)
         if next_norm is None:
             ops.linear(a, self.wo, torch.float32, residual=residual)
             return None
@@ -347,8 +348,6 @@ class PagedAttention(Mixer):
     def _project_plain(self, x, ctx, cache):
         """q ([n, heads, head_dim]) of a projection without rotation: biases added, k stored as keys and, when the
         values are the keys, as values too (the value cache is transposed, so it is a second store, not a view)."""
-        if isinstance(x, ops.Prenormed):
-            raise ValueError("attention: rows with an unfinished norm need a rotary projection")
         if cache.writes:
             rows = ops.linear(x, self.wqkv, torch.float32)
             return ops.qk_store(rows, self.q_bias, self.k_bias, ctx.slot_mapping[cache.group], self.num_heads,

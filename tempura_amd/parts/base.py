@@ -85,6 +85,11 @@ class Part:
     #: set by a block whose closing kernel adds partial sums: ``forward`` without a residual may return ``ops.Partials`` for its rows
     partial_output = False
 
+    #: True: in a step of few rows ``forward`` takes an ``ops.StreamClose`` as its residual, whose result (the next sublayer's rows) it returns
+    closes_streams = False
+    #: True: ``forward`` takes rows whose norm its first product finishes (``ops.Prenormed``) from such a product
+    takes_unfinished = False
+
     def __init__(self, spec: PartSpec, hidden_size: int, dtype: torch.dtype, device):
         self.spec = spec
         self.hidden_size = hidden_size

@@ -137,11 +137,11 @@ register_part("connection", "hyper_connection", HyperConnection)
 
 class StreamOpening:
     """What the kernel that closes one sublayer needs to open the next: the input coefficients of its connection
-    (None: the plain sum) and the weight and eps of its norm."""
-    __slots__ = ("in_coef", "weight", "eps")
+    (None: the plain sum), the weight and eps of its norm, and whether its part takes rows with that norm unfinished."""
+    __slots__ = ("in_coef", "weight", "eps", "unfinished")
 
-    def __init__(self, in_coef, weight, eps):
-        self.in_coef, self.weight, self.eps = in_coef, weight, eps
+    def __init__(self, in_coef, weight, eps, unfinished=False):
+        self.in_coef, self.weight, self.eps, self.unfinished = in_coef, weight, eps, unfinished
 
 
 class HyperBlock(ArrangedBlock):
@@ -151,7 +151,8 @@ class HyperBlock(ArrangedBlock):
     has the plain residual sum (one copy, x <- x + y).
 
     One kernel closes a sublayer and opens the next (update of the copies, the next input combination and its
-    norm), also across layers: ``entry_norm`` says what the block before needs for that."""
+    norm), also across layers: ``entry_norm`` says what the block before needs for that.  Of few rows that kernel is the
+    sublayer's own last product where its part allows it (``Part.closes_streams``)."""
     ROLES = {"mixer_norm": "norm", "mixer": "mixer", "mixer_link": "connection",
              "ffn_norm": "norm", "ffn": "ffn", "ffn_link": "connection"}
     OPTIONAL = frozenset({"mixer_link", "ffn_norm", "ffn", "ffn_link"})
@@ -169,18 +170,18 @@ class HyperBlock(ArrangedBlock):
         self.dtype = dtype
 
     @staticmethod
-    def _opening(norm, link):
+    def _opening(norm, link, part):
         if hasattr(norm, "weight") and hasattr(norm, "eps") and type(norm).__name__ == "RMSNorm" and getattr(norm, "groups", 1) == 1:
-            return StreamOpening(None if link is None else link.in_coef, norm.weight, norm.eps)
+            return StreamOpening(None if link is None else link.in_coef, norm.weight, norm.eps, getattr(part, "takes_unfinished", False))
         return None
 
     def entry_norm(self, m):
         """What the block before needs to prepare this block's first sublayer input (None: this block does it)."""
-        return self._opening(self.mixer_norm, self.mixer_link)
+        return self._opening(self.mixer_norm, self.mixer_link, self.mixer)
 
-    def _open(self, h, norm, link):
+    def _open(self, h, norm, link, part):
         """The normed input of a sublayer from the copies as they stand."""
-        op = self._opening(norm, link)
+        op = self._opening(norm, link, part)
         if op is not None:
             return ops.stream_step(h, self.streams, in_coef=op.in_coef, norm_weight=op.weight, eps=op.eps, out_dtype=self.dtype)
         u = ops.stream_step(h, self.streams, in_coef=None if link is None else link.in_coef, out_dtype=torch.float32)
@@ -195,29 +196,32 @@ class HyperBlock(ArrangedBlock):
             return None
         return ops.stream_step(h, self.streams, y, mix, out, opening.in_coef, opening.weight, opening.eps, self.dtype)
 
-    def _run(self, part, x, ctx, cache, n, device):
-        """A sublayer's output as a tensor of its own, float32 [tokens, hidden]."""
+    def _sublayer(self, h, part, link, x, ctx, cache, opening):
+        """Run a sublayer and close it; with ``opening`` return the next sublayer's input."""
         args = (x, ctx, cache) if cache is not None else (x, ctx)
+        if getattr(part, "closes_streams", False) and link is not None and getattr(part, "side_rows", None) is None \
+                and ops.stream_linear_ok(h.shape[0], self.hidden_size, self.streams, self.dtype):
+            ends = opening is not None and opening.unfinished
+            handed = part.forward(*args, ops.StreamClose(h, self.streams, link.mix, link.out_coef, (opening.in_coef, opening.weight, opening.eps) if ends else None))
+            if ends or opening is None:
+                return handed
+            return ops.stream_step(h, self.streams, in_coef=opening.in_coef, norm_weight=opening.weight, eps=opening.eps, out_dtype=self.dtype)
         if getattr(part, "returns_output", False):
-            return part.forward(*args, None)
-        y = torch.zeros((n, self.hidden_size), dtype=torch.float32, device=device)
+            return self._close(h, part.forward(*args, None), link, opening)
+        y = torch.zeros((h.shape[0], self.hidden_size), dtype=torch.float32, device=h.device)
         part.forward(*args, y)
-        return y
+        return self._close(h, y, link, opening)
 
     def forward(self, h, ctx, cache, x=None, next_norm=None):
-        n = h.shape[0]
         if x is None:
-            x = self._open(h, self.mixer_norm, self.mixer_link)
-        y = self._run(self.mixer, x, ctx, cache, n, h.device)
+            x = self._open(h, self.mixer_norm, self.mixer_link, self.mixer)
         after = next_norm if isinstance(next_norm, StreamOpening) else None
         if self.ffn is None:
-            return self._close(h, y, self.mixer_link, after)
-        mid = self._opening(self.ffn_norm, self.ffn_link)
-        x2 = self._close(h, y, self.mixer_link, mid)
+            return self._sublayer(h, self.mixer, self.mixer_link, x, ctx, cache, after)
+        x2 = self._sublayer(h, self.mixer, self.mixer_link, x, ctx, cache, self._opening(self.ffn_norm, self.ffn_link, self.ffn))
         if x2 is None:
-            x2 = self._open(h, self.ffn_norm, self.ffn_link)
-        y2 = self._run(self.ffn, x2, ctx, None, n, h.device)
-        return self._close(h, y2, self.ffn_link, after)
+            x2 = self._open(h, self.ffn_norm, self.ffn_link, self.ffn)
+        return self._sublayer(h, self.ffn, self.ffn_link, x2, ctx, None, after)
 
 
 register_part("block", "hyper", HyperBlock)

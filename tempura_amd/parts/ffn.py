@@ -63,6 +63,7 @@ class GatedFFN(FeedForward):
     product, whatever the compute dtype."""
     graph_safe = True
     returns_output = True      # with ``residual`` None the output comes back instead of being added
+    closes_streams = takes_unfinished = True
 
     def __init__(self, spec, hidden_size, dtype, device):
         super().__init__(spec, hidden_size, dtype, device)

@@ -26,6 +26,7 @@ from .base import Mixer, StateSpec, WeightInfo, register_part
 class Mamba2Mixer(Mixer):
     graph_safe = True
     returns_output = True      # with ``residual`` None the output comes back instead of being added
+    closes_streams = takes_unfinished = True
 
     def __init__(self, spec, hidden_size, dtype, device):
         super().__init__(spec, hidden_size, dtype, device)

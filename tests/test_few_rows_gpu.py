@@ -397,3 +397,39 @@ def test_experts_down_products_in_parts(m, experts, ff, n, parts, size):
         got = got.data.double().sum(0)
     # (the same products added in another order: 2^-24 of the sum of magnitudes at each of some hundred additions, as a random walk)
     assert float((got - want.double()).abs().max()) <= 2.0 ** -24 * 64 * max(1.0, float(want.abs().max()))
+
+
+@pytest.mark.parametrize("m", [1, 3, 16])
+@pytest.mark.parametrize("streams,n,k", [(4, 32, 64), (4, 1024, 4160), (4, 4096, 1024), (4, 288, 14336)])
+@pytest.mark.parametrize("coefs", [True, False])
+def test_product_closes_streams(m, streams, n, k, coefs):
+    """The product that closes a sublayer over the copies, and a product behind it that finishes the norm, against float64."""
+    from tempura_amd.kernels import ops
+    g = torch.Generator().manual_seed(m + n + k)
+    rnd = lambda *s: torch.randn(*s, generator=g).to(DEV)
+    x, w, w2 = rnd(m, k).bfloat16(), (rnd(n, k) * k ** -0.5).bfloat16(), (rnd(48, n) * 0.1).bfloat16()
+    mix, out, inc = (rnd(streams, streams), rnd(streams), rnd(streams)) if coefs else (None, None, None)
+    weight, h0 = rnd(n), rnd(m, streams * n)
+    y = x.double() @ w.double().t()
+    mixed = h0.double().view(m, streams, n)
+    if coefs:
+        mixed = torch.einsum("ab,man->mbn", mix.double(), mixed)
+    ref = mixed + (out.double() if coefs else torch.ones(streams, device=DEV).double())[None, :, None] * y[:, None]
+    u = (ref * inc.double()[None, :, None]).sum(1) if coefs else ref.sum(1)
+    normed = u / torch.sqrt((u * u).mean(1, keepdim=True) + 1e-5) * weight.double()
+    assert ops.stream_linear_ok(m, n, streams, torch.bfloat16) and not ops.stream_linear_ok(17, n, streams, torch.bfloat16) and not ops.stream_linear_ok(m, n, 2, torch.bfloat16)
+    got = {}
+    for rows in (x, ops.block_rows(x)):
+        for opening in (None, (inc, weight, 1e-5)):
+            h = h0.clone()
+            x2 = ops.linear(rows, ops.tile_weight(w), torch.float32, residual=ops.StreamClose(h, streams, mix, out, opening))
+            # (y: k products in float32, 2^-24 each as a random walk; then a sum of streams + 1 terms)
+            assert float((h.double().view_as(ref) - ref).norm()) <= (4 * k ** 0.5 + 16) * 2.0 ** -24 * float(ref.norm())
+            assert torch.equal(got.setdefault("h", h), h)
+            if opening is None:
+                assert x2 is None
+                continue
+            z = ops.linear(x2, ops.tile_weight(w2), torch.float32)
+            # (rows and weights in bfloat16: the rows' rounding, 2^-9 of each term of a sum)
+            assert float((z.double() - normed @ w2.double().t()).norm()) <= 2.0 ** -8 * float(z.norm()) + 1e-6
+            assert torch.equal(got.setdefault("z", z), z)

@@ -813,6 +813,7 @@ __global__ void residual_conv_kernel(const float* __restrict__ x, const float* _
 // SINGLE: every request brings one token; a thread is then the only reader of its channels' carried rows and moves them on
 // itself, so that no second kernel follows.
 #define RCONV_MAX_SUBS 4
+#define RCONV_MAX_TAPS 4   // (of norm_residual_conv_kernel)
 template <typename TO, bool SINGLE>
 __global__ void residual_conv4_kernel(const float* __restrict__ x, const float* __restrict__ w, float* __restrict__ state,
                                       size_t state_stride, size_t state_off, const int* __restrict__ cu_seqlens,
@@ -861,6 +862,128 @@ __global__ void residual_conv4_kernel(const float* __restrict__ x, const float* 
       const size_t place = (SINGLE && (blocked >> sub & 1)) ? ((size_t)(c >> 3) * (gridDim.x / channel_blocks) + t) * 8 + (c & 7) : (size_t)t * width + c;
       from_float4(out + (size_t)sub * out_stride_sub + place, cur.x + acc[sub].x, cur.y + acc[sub].y, cur.z + acc[sub].z, cur.w + acc[sub].w);
     }
+}
+
+// The norm of a row's parts and what the sublayers read of it, single tokens: the sums of group_rmsnorm_reg_kernel and, of the same elements
+// in the same thread, those of residual_conv4_kernel (the same bits; the normed rows go nowhere else), the carried rows and the
+// taps requested with the row in front of the sum.  Two trips to memory and a launch instead of two of each; a captured chain, two kernels / one: 4,096 in
+// eight parts, 1 / 8 / 64 rows 6.1 / 4.1, 6.3 / 4.3 and 7.1 / 4.6 us, 2,048 in eight 6.1 / 3.2 of eight rows, 1,024 5.8 / 3.2.  (With the
+// taps loaded behind the sum, sublayer by sublayer, 5.9 of eight rows of 4,096.)
+template <typename TO, int NV, int WAVES, int SUBS>
+__global__ __launch_bounds__(256) void norm_residual_conv_kernel(const float* __restrict__ x, const float* __restrict__ nw, int groups, float eps,
+                                                                 const float* __restrict__ w, float* __restrict__ state, size_t state_stride,
+                                                                 size_t state_off, const int* __restrict__ token_req,
+                                                                 const int* __restrict__ state_slots, TO* __restrict__ out, size_t out_stride_sub,
+                                                                 int width, int taps, int blocked) {
+  __shared__ float scratch[32];
+  constexpr int T = WAVES * TP_WAVE;
+  const int t = blockIdx.x, g = WAVES == 1 ? blockIdx.y * 4 + threadIdx.x / TP_WAVE : blockIdx.y;
+  if (g >= groups) return;       // (a wave of its own: no barrier follows)
+  const int tid = threadIdx.x % T, per = width / groups, p4 = per / 4;
+  const float* p = x + (size_t)t * width + (size_t)g * per;
+  float4 v[NV], wv[NV], old[NV][RCONV_MAX_TAPS], f[NV][SUBS][RCONV_MAX_TAPS];   // (old: the last place is the token's own row)
+  float* st = state + (size_t)state_slots[token_req[t]] * state_stride + state_off + (size_t)g * per;
+  float ss = 0.f;
+#pragma unroll
+  for (int k = 0; k < NV; ++k) {
+    const int c = k * T + tid;
+    if (c < p4) {
+      v[k] = *(const float4*)(p + 4 * c);
+      wv[k] = *(const float4*)(nw + (size_t)g * per + 4 * c);
+#pragma unroll
+      for (int j = 0; j < RCONV_MAX_TAPS; ++j) {
+        // (places and taps beyond the last repeat one that is there and are dropped below: every load is requested before the sum)
+        const float* q = st + (size_t)min(j, taps - 2) * width + 4 * c;
+        old[k][j] = make_float4(q[0], q[1], q[2], q[3]);
+#pragma unroll
+        for (int sub = 0; sub < SUBS; ++sub)
+          f[k][sub][j] = *(const float4*)(w + ((size_t)sub * taps + min(j, taps - 1)) * width + (size_t)g * per + 4 * c);
+      }
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < NV; ++k)
+    if (k * T + tid < p4) {
+      ss = fmaf(v[k].x, v[k].x, ss);
+      ss = fmaf(v[k].y, v[k].y, ss);
+      ss = fmaf(v[k].z, v[k].z, ss);
+      ss = fmaf(v[k].w, v[k].w, ss);
+    }
+  if constexpr (WAVES == 1)
+    ss = wave_sum(ss);
+  else
+    ss = block_sum(ss, scratch);
+  const float scale = 1.0f / sqrtf(ss / (float)per + eps);
+#pragma unroll
+  for (int k = 0; k < NV; ++k) {
+    const int c = k * T + tid;
+    if (c >= p4) continue;
+    const float4 cur = make_float4(v[k].x * scale * wv[k].x, v[k].y * scale * wv[k].y, v[k].z * scale * wv[k].z, v[k].w * scale * wv[k].w);
+    const int col = g * per + 4 * c;
+#pragma unroll
+    for (int j = 1; j < RCONV_MAX_TAPS; ++j) {
+      if (j == taps - 1) old[k][j] = cur;
+      if (j < taps) {
+        float* q = st + (size_t)(j - 1) * width + 4 * c;
+        q[0] = old[k][j].x;
+        q[1] = old[k][j].y;
+        q[2] = old[k][j].z;
+        q[3] = old[k][j].w;
+      }
+    }
+#pragma unroll
+    for (int sub = 0; sub < SUBS; ++sub) {
+      float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+      for (int j = 0; j < RCONV_MAX_TAPS; ++j)
+        if (j < taps) {
+          acc.x = fmaf(f[k][sub][j].x, old[k][j].x, acc.x);
+          acc.y = fmaf(f[k][sub][j].y, old[k][j].y, acc.y);
+          acc.z = fmaf(f[k][sub][j].z, old[k][j].z, acc.z);
+          acc.w = fmaf(f[k][sub][j].w, old[k][j].w, acc.w);
+        }
+      const size_t place = (blocked >> sub & 1) ? ((size_t)(col >> 3) * gridDim.x + t) * 8 + (col & 7) : (size_t)t * width + col;
+      from_float4(out + (size_t)sub * out_stride_sub + place, cur.x + acc.x, cur.y + acc.y, cur.z + acc.z, cur.w + acc.w);
+    }
+  }
+}
+
+// x [n, width]: the norm in `groups` parts (nw, eps), then residual_conv over runs of one token (see tp_residual_conv); width / groups at most
+// 4,096 and a multiple of four, 2 to RCONV_MAX_TAPS taps
+extern "C" int tp_norm_residual_conv(const float* x, const float* nw, int groups, float eps, const float* w, float* state, size_t state_stride,
+                                     size_t state_off, const int* token_req, const int* state_slots, void* out, int out_dt, int n, int width,
+                                     int taps, int subs, int blocked, hipStream_t s) {
+  TP_REQUIRE(n >= 0 && width > 0 && groups > 0 && groups <= 65535 && width % groups == 0 && width / groups % 4 == 0 && width / groups <= 4096 &&
+             taps >= 2 && taps <= RCONV_MAX_TAPS && subs >= 1 && subs <= 2, "norm_residual_conv: bad sizes");
+  TP_REQUIRE((((uintptr_t)x | (uintptr_t)nw | (uintptr_t)w | (uintptr_t)out) & 15) == 0, "norm_residual_conv: operands must be aligned to 16 bytes");
+  TP_REQUIRE(state != nullptr && state_stride >= state_off + (size_t)(taps - 1) * width, "norm_residual_conv: state rows too short");
+  TP_REQUIRE((blocked == 0 || width % 8 == 0) && (out_dt == TP_F32 || out_dt == TP_BF16), "norm_residual_conv: bad output");
+  if (n == 0) return 0;
+  const int per = width / groups;
+  const size_t sub_stride = (size_t)n * width;
+#define NRC(TO, NV, WAVES, GY)                                                                                                      \
+  do {                                                                                                                              \
+    if (subs == 1)                                                                                                                  \
+      hipLaunchKernelGGL((norm_residual_conv_kernel<TO, NV, WAVES, 1>), dim3(n, GY), dim3(256), 0, s, x, nw, groups, eps, w, state, \
+                         state_stride, state_off, token_req, state_slots, (TO*)out, sub_stride, width, taps, blocked);              \
+    else                                                                                                                            \
+      hipLaunchKernelGGL((norm_residual_conv_kernel<TO, NV, WAVES, 2>), dim3(n, GY), dim3(256), 0, s, x, nw, groups, eps, w, state, \
+                         state_stride, state_off, token_req, state_slots, (TO*)out, sub_stride, width, taps, blocked);              \
+  } while (0)
+#define NRC_SIZES(TO)                                            \
+  do {                                                           \
+    if (per <= 256) NRC(TO, 1, 1, (groups + 3) / 4);             \
+    else if (per <= 512) NRC(TO, 2, 1, (groups + 3) / 4);        \
+    else if (per <= 1024) NRC(TO, 1, 4, groups);                 \
+    else if (per <= 2048) NRC(TO, 2, 4, groups);                 \
+    else NRC(TO, 4, 4, groups);                                  \
+  } while (0)
+  if (out_dt == TP_F32) NRC_SIZES(float);
+  else NRC_SIZES(bf16_t);
+#undef NRC_SIZES
+#undef NRC
+  TP_CHECK_LAUNCH("norm_residual_conv");
+  return 0;
 }
 
 __global__ void residual_conv_state_kernel(const float* __restrict__ x, float* __restrict__ state, size_t state_stride,

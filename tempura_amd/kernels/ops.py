@@ -2114,6 +2114,35 @@ def residual_conv(x: torch.Tensor, weight: torch.Tensor, state: torch.Tensor, st
     return [KBlocked(out[i].view(width // 8, n, 8), n, width) if i in blocked else out[i] for i in range(subs)]
 
 
+def norm_residual_conv_ok(n: int, width: int, groups: int, taps: int, subs: int, max_run: int) -> bool:
+    """Whether ``norm_residual_conv`` takes a step of ``n`` tokens: single ones, few enough that a launch counts."""
+    # (several parts: a row normed whole has a kernel that adds its squares in another order.  The gain grows with the rows, 128 of 4,096
+    # 8.5 / 5.2 us; beyond 64 a launch no longer counts beside the products)
+    return _backend is None and max_run == 1 and 0 < n <= 64 and groups > 1 and width % 8 == 0 and width % groups == 0 and width // groups % 4 == 0 and \
+        width // groups <= 4096 and 2 <= taps <= 4 and 1 <= subs <= 2
+
+
+def norm_residual_conv(h: torch.Tensor, norm_weight: torch.Tensor, eps: float, groups: int, weight: torch.Tensor, state: torch.Tensor,
+                       state_off: int, token_req: torch.Tensor, state_slots: torch.Tensor, out_dtype: torch.dtype, blocked=()):
+    """``residual_conv`` of the rows ``rmsnorm(h, norm_weight, eps, float32, groups=groups)`` in one launch, for runs of one token each
+    (``norm_residual_conv_ok``), with the bits of the two."""
+    _dev_ok(h, norm_weight, weight, state, token_req, state_slots)
+    _need(h.dtype == torch.float32 and h.dim() == 2 and weight.dtype == torch.float32 and weight.dim() == 3 and weight.shape[2] == h.shape[1],
+          "norm_residual_conv: rows must be float32 [n, width], weight float32 [subs, taps, width]")
+    (n, width), (subs, taps) = h.shape, weight.shape[:2]
+    _need(norm_residual_conv_ok(n, width, groups, taps, subs, 1), "norm_residual_conv: sizes")
+    _need(norm_weight.dtype == torch.float32 and norm_weight.numel() == width, "norm_residual_conv: norm weight must be float32 [width]")
+    _need(state.dtype == torch.float32 and state.dim() == 2 and state_off >= 0 and state.shape[1] >= state_off + (taps - 1) * width,
+          "norm_residual_conv: state rows too short")
+    _i32(token_req, n, "token_req")
+    _need(state_slots.dtype == torch.int32, "state_slots must be int32")
+    out = torch.empty((subs, n, width), dtype=out_dtype, device=h.device)
+    _call("tp_norm_residual_conv", _ptr(h), _ptr(norm_weight), int(groups), ctypes.c_float(eps), _ptr(weight), _ptr(state),
+          ctypes.c_size_t(state.shape[1]), ctypes.c_size_t(state_off), _ptr(token_req), _ptr(state_slots), _ptr(out), _dtcode(out_dtype), n, width,
+          taps, subs, sum(1 << i for i in blocked), _stream())
+    return [KBlocked(out[i].view(width // 8, n, 8), n, width) if i in blocked else out[i] for i in range(subs)]
+
+
 def add_row(h: torch.Tensor, table: torch.Tensor, row: int) -> None:
     """h[t] += table[row] for every row t, in place (float32)."""
     if _backend is not None:

@@ -445,7 +445,10 @@ class SharedNormBlock(ArrangedBlock):
     def forward(self, h, ctx, cache) -> None:
         if self.inputs is not None:
             parts = [self.mixer] if self.ffn is None else [self.mixer, self.ffn]
-            xs = self.inputs.forward(self.norm.forward(h, out_dtype=torch.float32), ctx, cache, parts)
+            if getattr(self.inputs, "takes_unnormed", None) is not None and self.inputs.takes_unnormed(self.norm, h, ctx):
+                xs = self.inputs.forward(h, ctx, cache, parts, self.norm)
+            else:
+                xs = self.inputs.forward(self.norm.forward(h, out_dtype=torch.float32), ctx, cache, parts)
         else:
             xs = [self.norm.forward(h)] * 2
         self.mixer.forward(xs[0], ctx, cache, h)

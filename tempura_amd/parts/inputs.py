@@ -42,12 +42,20 @@ class ResidualConv(Part):
         # [sublayers, taps, hidden]: tap-major, so that neighbouring lanes read neighbouring channels
         self.weight = torch.stack([self._to_device(get(name), torch.float32).t() for name in self.names]).contiguous()
 
-    def forward(self, n, ctx, cache, parts=()):
+    def takes_unnormed(self, norm, h, ctx) -> bool:
+        """Whether ``forward`` takes the stream ``h`` itself and applies ``norm`` in its launch."""
+        return type(norm).__name__ == "RMSNorm" and \
+            ops.norm_residual_conv_ok(h.shape[0], h.shape[1], norm.groups, self.taps, len(self.names), ctx.max_q_len)
+
+    def forward(self, n, ctx, cache, parts=(), norm=None):
         """float32 rows [tokens, hidden] -> a list of compute-dtype rows, one per sublayer (k-blocked for those of the ``parts``
-        that take them so, in a step of a few single tokens)."""
+        that take them so, in a step of a few single tokens).  ``norm`` (``takes_unnormed``): the rows are the stream, to be normed."""
         few = {}
         if ctx.max_q_len == 1 and len(self.names) <= 4 and ops.few_rows_ok(n.shape[0], n.shape[1], self.dtype):
             few = {"blocked": [i for i, part in enumerate(parts) if getattr(part, "takes_blocked_rows", False)]}
+        if norm is not None:
+            return ops.norm_residual_conv(n, norm.weight, norm.eps, norm.groups, self.weight, cache.state, self.state_off, ctx.token_req,
+                                          ctx.state_slots, self.dtype, **few)
         return ops.residual_conv(n, self.weight, cache.state, self.state_off, ctx.cu_seqlens, ctx.token_req, ctx.state_slots,
                                  ctx.num_requests, self.dtype, max_run=ctx.max_q_len, **few)
 

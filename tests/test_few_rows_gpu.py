@@ -433,3 +433,23 @@ def test_product_closes_streams(m, streams, n, k, coefs):
             # (rows and weights in bfloat16: the rows' rounding, 2^-9 of each term of a sum)
             assert float((z.double() - normed @ w2.double().t()).norm()) <= 2.0 ** -8 * float(z.norm()) + 1e-6
             assert torch.equal(got.setdefault("z", z), z)
+
+
+@pytest.mark.parametrize("n", [1, 5, 64])
+@pytest.mark.parametrize("width,groups,taps,subs", [(8, 2, 2, 1), (264, 11, 4, 2), (4096, 8, 4, 2), (1024, 8, 3, 1), (2048, 2, 4, 2), (8192, 2, 2, 2), (3072, 2, 4, 1)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_norm_in_the_residual_convolution(n, width, groups, taps, subs, dtype):
+    """The norm and the convolution behind it in one launch: the bits of the two kernels, rows and states alike."""
+    from tempura_amd.kernels import ops
+    g = torch.Generator().manual_seed(n + width + taps)
+    h, nw, w = torch.randn(n, width, generator=g).to(DEV), torch.randn(width, generator=g).to(DEV), torch.randn(subs, taps, width, generator=g).to(DEV)
+    cu, req, slots = _runs([1] * n, g)
+    for off in (0, 3):
+        s0 = torch.randn(n + 2, off + (taps - 1) * width + 5, generator=g).to(DEV)
+        s1 = s0.clone()
+        blocked = [subs - 1] if dtype == torch.bfloat16 and n <= 16 and ops.few_rows_ok(n, width, dtype) else []
+        want = ops.residual_conv(ops.rmsnorm(h, nw, 1e-5, torch.float32, groups=groups), w, s0, off, cu, req, slots, n, dtype, max_run=1, blocked=blocked)
+        assert ops.norm_residual_conv_ok(n, width, groups, taps, subs, 1) and not ops.norm_residual_conv_ok(n, width, groups, taps, subs, 2)
+        got = ops.norm_residual_conv(h, nw, 1e-5, groups, w, s1, off, req, slots, dtype, blocked)
+        assert torch.equal(s0, s1)
+        assert all(torch.equal(getattr(a, "data", a), getattr(b, "data", b)) for a, b in zip(got, want))

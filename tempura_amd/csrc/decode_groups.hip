@@ -309,6 +309,10 @@ __global__ __launch_bounds__(DG_WAVES * 64) void moe_open_kernel(const bf16_t* _
     if (q < 256 && e0 + (l >> 4) * 4 + q % 4 < DG_OPEN_EXPERTS) logits[m][e0 + (l >> 4) * 4 + q % 4] = dg_sum(red, q);
     __syncthreads();
   }
+  if (r.experts <= ROUTE_FEW) {
+    if (wave < 4) route_few(r, logits[q / ROUTE_FEW], q / ROUTE_FEW, q / ROUTE_FEW < M);
+    return;
+  }
   for (int t0 = 0; t0 < M; t0 += DG_WAVES) {
     const int t = min(t0 + wave, M - 1);
     route_token<1>(r, logits[t], t, t0 + wave < M, route_lds[wave], route_lds[wave] + DG_OPEN_EXPERTS);

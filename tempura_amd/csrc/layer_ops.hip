@@ -493,6 +493,11 @@ __global__ __launch_bounds__(256) void moe_route_kernel(Route r, const float* __
   route_token<ROUTE_LANE>(r, logits + (size_t)t * logit_stride, t, live, choice_l, choice_l + r.experts);
 }
 
+__global__ __launch_bounds__(256) void moe_route_few_kernel(Route r, const float* __restrict__ logits, int logit_stride, int n) {
+  const int t = blockIdx.x * (256 / ROUTE_FEW) + threadIdx.x / ROUTE_FEW;
+  route_few(r, logits + (size_t)min(t, n - 1) * logit_stride, t, t < n);
+}
+
 extern "C" int tp_moe_route(const float* logits, int logit_stride, const float* correction, int experts, int top, int groups,
                             int keep, float* dense, int* ids, float* weights, int n, int score_kind, int group_best,
                             int normalize, float sum_eps, float scale, const float* logit_bias, hipStream_t s) {
@@ -505,7 +510,9 @@ extern "C" int tp_moe_route(const float* logits, int logit_stride, const float* 
   // (as many experts a lane as there are: eight experts in four groups, eight tokens, 7.9 -> 7.5 us with one instead of eight)
   const Route r = {correction, logit_bias, experts, top, groups, keep, score_kind, group_best, normalize, sum_eps, scale, dense, ids, weights};
 #define ROUTE(L) hipLaunchKernelGGL(moe_route_kernel<L>, dim3((n + 3) / 4), dim3(256), shmem, s, r, logits, logit_stride, n)
-  if (experts <= TP_WAVE) ROUTE(1);
+  if (experts <= ROUTE_FEW)
+    hipLaunchKernelGGL(moe_route_few_kernel, dim3((n + 256 / ROUTE_FEW - 1) / (256 / ROUTE_FEW)), dim3(256), 0, s, r, logits, logit_stride, n);
+  else if (experts <= TP_WAVE) ROUTE(1);
   else if (experts <= 2 * TP_WAVE) ROUTE(2);
   else ROUTE(ROUTE_PER_LANE);
 #undef ROUTE

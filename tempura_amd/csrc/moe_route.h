@@ -168,3 +168,82 @@ __device__ inline void route_token(const Route& r, const float* logits, int t, b
     }
   }
 }
+
+// The same choice of up to 16 experts, bit for bit: lane l of a row of 16 lanes holds expert l, a wave works on four tokens.  The scores of a
+// token are gathered once (sixteen loads from other lanes in flight together) and every lane counts the scores in front of its own; the
+// choice one by one is a chain of reductions through LDS and barriers, some 5 us of a block that everything waits for.  Router and choice of
+// eight experts in four groups at width 4,096 / 2,048, eight rows: 9.8 -> 6.4 and 8.6 -> 5.3 us; without groups 7.2 -> 4.8 and 6.5 -> 3.7; the
+// choice alone of 1,803 rows 6.4 -> 4.2.
+// Of scores that compare with nothing (NaN) none is chosen, and a group whose total is infinite is kept beside the others, as there.
+#define ROUTE_FEW 16
+__device__ inline void route_few(const Route& r, const float* logits, int t, bool live) {
+  const int e = threadIdx.x % ROUTE_FEW, base = threadIdx.x % TP_WAVE - e, experts = r.experts;
+  const bool mine = e < experts;
+  const float correction = mine && r.correction != nullptr ? r.correction[e] : 0.f;
+  const float z = mine ? logits[e] + (r.bias != nullptr ? r.bias[e] : 0.f) : -INFINITY;
+  float sc;
+  if (r.score_kind == 1) {
+    sc = mine ? 1.0f / (1.0f + expf(-z)) : 0.f;
+  } else {
+    const float mx = row_max(z);
+    sc = mine ? expf(z - mx) : 0.f;
+    sc *= 1.0f / row_sum(sc);
+  }
+  float ch = mine ? (r.correction != nullptr ? sc + correction : sc) : -INFINITY;
+  if (r.groups > 1) {
+    const int per = experts / r.groups, first = e / per * per;   // (lanes past the last expert: a group of their own, never looked at)
+    float all[ROUTE_FEW], totals[ROUTE_FEW];
+#pragma unroll
+    for (int j = 0; j < ROUTE_FEW; ++j) all[j] = __shfl(ch, base + j, TP_WAVE);
+    // the group's largest scores one after the other (equal scores: the lower index first), added in that order
+    float total = 0.f, pv = INFINITY;
+    int pi = -1;
+    for (int b = 0; b < r.group_best; ++b) {
+      float best = -INFINITY;
+      int bi = -1;
+#pragma unroll
+      for (int j = 0; j < ROUTE_FEW; ++j)
+        if (j >= first && j < first + per && (all[j] < pv || (all[j] == pv && j > pi)) && (bi < 0 || all[j] > best)) {
+          best = all[j];
+          bi = j;
+        }
+      if (bi >= 0) total = b == 0 ? best : total + best;
+      pv = bi >= 0 ? best : -INFINITY;
+      pi = bi >= 0 ? bi : ROUTE_FEW;
+    }
+#pragma unroll
+    for (int j = 0; j < ROUTE_FEW; ++j) totals[j] = __shfl(total, base + j, TP_WAVE);
+    int in_front = 0;
+#pragma unroll
+    for (int j = 0; j < ROUTE_FEW; ++j)
+      if (j < experts && (j < first || j >= first + per) && totals[j] != INFINITY && (totals[j] > total || (totals[j] == total && j < first))) ++in_front;
+    // (counted member by member: per times the groups in front)
+    if (!(total == INFINITY || (total == total && in_front < r.keep * per))) ch = -INFINITY;
+  }
+  float all[ROUTE_FEW];
+#pragma unroll
+  for (int j = 0; j < ROUTE_FEW; ++j) all[j] = __shfl(ch, base + j, TP_WAVE);
+  int place = 0;
+#pragma unroll
+  for (int j = 0; j < ROUTE_FEW; ++j)
+    if (all[j] > ch || (all[j] == ch && j < e)) ++place;
+  const bool won = mine && ch > -INFINITY && place < r.top;
+  float w = sc;
+  if (r.normalize) {
+    float chosen_sum = 0.f;      // (in the order of choice)
+    for (int it = 0; it < r.top; ++it) {
+      const unsigned there = (unsigned)(__ballot(won && place == it) >> base) & 0xffffu;
+      const float s = __shfl(sc, base + (there != 0 ? __ffs(there) - 1 : 0), TP_WAVE);
+      if (there != 0) chosen_sum += s;
+    }
+    w = sc * (r.scale / (chosen_sum + r.sum_eps));
+  } else if (r.scale != 1.0f) {
+    w = sc * r.scale;
+  }
+  if (!live || !mine) return;
+  r.dense[(size_t)t * experts + e] = won ? w : 0.f;
+  if (won) {
+    r.ids[(size_t)t * r.top + place] = e;
+    r.weights[(size_t)t * r.top + place] = w;
+  }
+}

@@ -453,3 +453,47 @@ def test_norm_in_the_residual_convolution(n, width, groups, taps, subs, dtype):
         got = ops.norm_residual_conv(h, nw, 1e-5, groups, w, s1, off, req, slots, dtype, blocked)
         assert torch.equal(s0, s1)
         assert all(torch.equal(getattr(a, "data", a), getattr(b, "data", b)) for a, b in zip(got, want))
+
+
+@pytest.mark.parametrize("n", [1, 15, 17, 300])
+@pytest.mark.parametrize("experts,top,groups,keep,group_best", [(1, 1, 1, 1, 1), (8, 2, 4, 2, 1), (12, 5, 3, 2, 3), (16, 16, 1, 1, 1), (16, 3, 8, 3, 2), (15, 4, 5, 4, 1)])
+@pytest.mark.parametrize("sigmoid,normalize,scale", [(False, False, 1.0), (True, True, 2.5), (False, True, 1.0)])
+def test_choice_of_few_experts(n, experts, top, groups, keep, group_best, sigmoid, normalize, scale):
+    """Up to 16 experts against the choice one by one of float64 scores, with equal scores, infinite corrections and rows of NaN."""
+    from tempura_amd.kernels import ops
+    g = torch.Generator().manual_seed(n + experts + top)
+    logits = torch.randn(n, experts + 3, generator=g).mul(4).round().div(4)          # (many equal ones)
+    if n > 2:
+        logits[1] = float("nan")
+    bias, correction = torch.randn(experts, generator=g).round(), torch.randn(experts, generator=g).mul(2).round().div(2)
+    if experts > 8:
+        correction[3], correction[5] = float("inf"), -float("inf")
+    dense, ids, weights = ops.moe_route(logits.to(DEV), correction.to(DEV), experts, top, groups, keep, score="sigmoid" if sigmoid else "softmax",
+                                        group_best=group_best, normalize=normalize, sum_eps=1e-6, scale=scale, bias=bias.to(DEV))
+    dense, ids, weights = dense.cpu(), ids.cpu(), weights.cpu()
+    for t in range(n):
+        z = logits[t, :experts] + bias
+        s = torch.sigmoid(z) if sigmoid else torch.softmax(z, 0)
+        # (equal logits give equal scores in any precision, so the order of float32 scores is theirs)
+        ch = (s + correction).tolist()
+        if groups > 1:
+            per, total = experts // groups, []
+            for q in range(groups):
+                best = sorted((c for c in ch[q * per: (q + 1) * per] if c == c), reverse=True)[:group_best]
+                v = torch.tensor(0.0)
+                for i, c in enumerate(best):
+                    v = torch.tensor(c) if i == 0 else v + torch.tensor(c)
+                total.append(float(v))
+            kept = [q for q in range(groups) if total[q] == float("inf")]
+            kept += sorted((q for q in range(groups) if total[q] < float("inf")), key=lambda q: (-total[q], q))[:keep]
+            ch = [c if i // per in kept else -float("inf") for i, c in enumerate(ch)]
+        order = sorted((i for i in range(experts) if ch[i] > -float("inf")), key=lambda i: (-ch[i], i))[:top]
+        near = any(abs(a - b) < 1e-6 and a != b for i, a in enumerate(ch) for b in ch[:i])
+        want = torch.zeros(experts)
+        chosen = sum(float(s[i]) for i in order)
+        for i in order:
+            want[i] = float(s[i]) * (scale / (chosen + 1e-6) if normalize else scale)
+        if near:
+            continue
+        assert ids[t, : len(order)].tolist() == order, t
+        assert torch.allclose(dense[t], want, rtol=1e-5, atol=1e-7) and torch.equal(dense[t][order], weights[t, : len(order)]), t

@@ -1213,3 +1213,81 @@ extern "C" int tp_vector_store(const void* c, int dt, const int* slots, void* k_
   TP_CHECK_LAUNCH("vector_store");
   return 0;
 }
+
+// Of few rows the two norms in front of an attention over latents in one launch: block (t, 0) norms the query's latent into cq, block (t, 1)
+// the key's and puts it into the cache.  The parts, their lanes and the order of their sums are group_rmsnorm_reg_kernel's (up to 512 columns
+// a wave, else the block), so the bits are those of the three launches, each a few trips to memory around
+// some kilobytes.  Latents of 1,024 and 128, a captured chain, three kernels / one: 1 / 4 / 64 rows 5.0 / 2.2, 5.7 / 2.3 and 6.0 / 2.7 us.
+template <typename TO>
+__global__ __launch_bounds__(256) void latent_norms_kernel(const float* __restrict__ rows, size_t stride, int q_col0, int q_dim,
+                                                           const float* __restrict__ q_w, int c_col0, int c_dim, const float* __restrict__ c_w,
+                                                           float eps, TO* __restrict__ cq, const int* __restrict__ slots,
+                                                           TO* __restrict__ k_cache, TO* __restrict__ v_cache, int page_size) {
+  __shared__ float scratch[32];
+  const int t = blockIdx.x, per = blockIdx.y == 0 ? q_dim : c_dim, p4 = per / 4, lanes = per <= 512 ? TP_WAVE : 256, tid = threadIdx.x;
+  if (tid >= lanes) return;      // (a wave by itself: no barrier follows)
+  const float* p = rows + (size_t)t * stride + (blockIdx.y == 0 ? q_col0 : c_col0);
+  const float* w = blockIdx.y == 0 ? q_w : c_w;
+  const int slot = blockIdx.y == 0 ? 0 : slots[t];
+  float4 v[4], wv[4];
+  float ss = 0.f;
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    const int c = k * lanes + tid;
+    if (c < p4) {
+      v[k] = *(const float4*)(p + 4 * c);
+      wv[k] = *(const float4*)(w + 4 * c);
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < 4; ++k)
+    if (k * lanes + tid < p4) {
+      ss = fmaf(v[k].x, v[k].x, ss);
+      ss = fmaf(v[k].y, v[k].y, ss);
+      ss = fmaf(v[k].z, v[k].z, ss);
+      ss = fmaf(v[k].w, v[k].w, ss);
+    }
+  ss = lanes == TP_WAVE ? wave_sum(ss) : block_sum(ss, scratch);
+  const float scale = 1.0f / sqrtf(ss / (float)per + eps);
+  const size_t page = slot / page_size;
+  const int off = slot % page_size;
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    const int c = k * lanes + tid;
+    if (c >= p4) continue;
+    const float4 o = make_float4(v[k].x * scale * wv[k].x, v[k].y * scale * wv[k].y, v[k].z * scale * wv[k].z, v[k].w * scale * wv[k].w);
+    if (blockIdx.y == 0) {
+      from_float4(cq + (size_t)t * per + 4 * c, o.x, o.y, o.z, o.w);
+    } else {
+      from_float4(k_cache + (page * page_size + off) * per + 4 * c, o.x, o.y, o.z, o.w);
+      TO* vp = v_cache + (page * per + 4 * c) * page_size + off;
+      from_float(vp, o.x);
+      from_float(vp + page_size, o.y);
+      from_float(vp + 2 * (size_t)page_size, o.z);
+      from_float(vp + 3 * (size_t)page_size, o.w);
+    }
+  }
+}
+
+// rows float32 [n, stride]: columns q_col0 .. + q_dim normed (q_w, eps) -> cq [n, q_dim]; c_col0 .. + c_dim normed (c_w) -> cache places (see
+// tp_vector_store).  All of type dt; dimensions, columns and stride multiples of four, at most 4,096 columns each.
+extern "C" int tp_latent_norms(const float* rows, size_t stride, int q_col0, int q_dim, const float* q_w, int c_col0, int c_dim, const float* c_w,
+                               float eps, void* cq, const int* slots, void* k_cache, void* v_cache, int dt, int n, int page_size, hipStream_t s) {
+  TP_REQUIRE(n >= 0 && n <= 65535 && q_dim > 0 && c_dim > 0 && q_dim <= 4096 && c_dim <= 4096 && page_size > 0 && q_col0 >= 0 && c_col0 >= 0 &&
+             (q_dim | c_dim | q_col0 | c_col0) % 4 == 0 && stride % 4 == 0 && stride >= (size_t)q_col0 + q_dim && stride >= (size_t)c_col0 + c_dim,
+             "latent_norms: bad sizes");
+  TP_REQUIRE((((uintptr_t)rows | (uintptr_t)q_w | (uintptr_t)c_w | (uintptr_t)cq | (uintptr_t)k_cache) & 15) == 0,
+             "latent_norms: operands must be aligned to 16 bytes");
+  if (n == 0) return 0;
+  const dim3 grid(n, 2);
+  if (dt == TP_F32)
+    hipLaunchKernelGGL(latent_norms_kernel<float>, grid, dim3(256), 0, s, rows, stride, q_col0, q_dim, q_w, c_col0, c_dim, c_w, eps, (float*)cq, slots,
+                       (float*)k_cache, (float*)v_cache, page_size);
+  else if (dt == TP_BF16)
+    hipLaunchKernelGGL(latent_norms_kernel<bf16_t>, grid, dim3(256), 0, s, rows, stride, q_col0, q_dim, q_w, c_col0, c_dim, c_w, eps, (bf16_t*)cq,
+                       slots, (bf16_t*)k_cache, (bf16_t*)v_cache, page_size);
+  else
+    TP_REQUIRE(false, "latent_norms: unknown dtype %d", dt);
+  TP_CHECK_LAUNCH("latent_norms");
+  return 0;
+}

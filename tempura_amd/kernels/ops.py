@@ -2231,6 +2231,33 @@ def vector_store(c: torch.Tensor, slots: torch.Tensor, k_cache: torch.Tensor, v_
     _call("tp_vector_store", _ptr(c), _dt(c), _ptr(slots), _ptr(k_cache), _ptr(v_cache), n, dim, page_size, _stream())
 
 
+def latent_norms_ok(rows: torch.Tensor, q_col0: int, q_dim: int, c_col0: int, c_dim: int, cache_dtype: torch.dtype, dtype: torch.dtype) -> bool:
+    """Whether ``latent_norms`` takes these rows: few of them (a launch counts), both parts in 16-byte pieces and one type for all results."""
+    return _backend is None and 0 < rows.shape[0] <= 64 and dtype == cache_dtype and rows.shape[1] % 4 == 0 and rows.is_contiguous() and \
+        rows.data_ptr() % 16 == 0 and all(v % 4 == 0 for v in (q_col0, q_dim, c_col0, c_dim)) and 0 < q_dim <= 4096 and 0 < c_dim <= 4096 and \
+        c_dim * dtype.itemsize % 16 == 0 and q_dim * dtype.itemsize % 16 == 0
+
+
+def latent_norms(rows: torch.Tensor, q_col0: int, q_dim: int, q_weight: torch.Tensor, c_col0: int, c_dim: int, c_weight: torch.Tensor, eps: float,
+                 slots: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor) -> torch.Tensor:
+    """``vector_store(rmsnorm_cols(rows, c_col0, c_dim, c_weight, eps, k_cache.dtype), slots, k_cache, v_cache)`` and the returned
+    ``rmsnorm_cols(rows, q_col0, q_dim, q_weight, eps, k_cache.dtype)`` in one launch (``latent_norms_ok``), with their bits."""
+    _dev_ok(rows, q_weight, c_weight, slots, k_cache, v_cache)
+    _need(rows.dtype == torch.float32 and rows.dim() == 2 and latent_norms_ok(rows, q_col0, q_dim, c_col0, c_dim, k_cache.dtype, k_cache.dtype)
+          and 0 <= q_col0 and q_col0 + q_dim <= rows.shape[1] and 0 <= c_col0 and c_col0 + c_dim <= rows.shape[1], "latent_norms: bad rows")
+    for w, d in ((q_weight, q_dim), (c_weight, c_dim)):
+        _need(w.dtype == torch.float32 and w.numel() == d, "latent_norms: weights must be float32, one for each column")
+    _need(k_cache.dim() == 4 and k_cache.shape[1] == 1 and k_cache.shape[3] == c_dim and v_cache.dtype == k_cache.dtype
+          and tuple(v_cache.shape) == (k_cache.shape[0], 1, c_dim, k_cache.shape[2]),
+          "latent_norms: caches must be k [pages, 1, page_size, dim], v [pages, 1, dim, page_size]")
+    n = rows.shape[0]
+    _i32(slots, n, "slots")
+    cq = torch.empty((n, q_dim), dtype=k_cache.dtype, device=rows.device)
+    _call("tp_latent_norms", _ptr(rows), ctypes.c_size_t(rows.shape[1]), int(q_col0), int(q_dim), _ptr(q_weight), int(c_col0), int(c_dim),
+          _ptr(c_weight), ctypes.c_float(eps), _ptr(cq), _ptr(slots), _ptr(k_cache), _ptr(v_cache), _dt(k_cache), n, k_cache.shape[2], _stream())
+    return cq
+
+
 def mlstm_scan(proj: torch.Tensor, col0: int, i_bias: torch.Tensor, f_bias: torch.Tensor, cap: float, q_scale: float,
                state: torch.Tensor, state_off: int, cu_seqlens: torch.Tensor, state_slots: torch.Tensor, num_requests: int,
                heads: int, dim: int, vdim: int, norm_weight: torch.Tensor, eps: float, scale: float, out: torch.Tensor,

@@ -728,10 +728,14 @@ class LatentCacheAttention(BranchMixer):
         if cache.writes != self.own_latent:
             raise ValueError("latent_cache_attention: a layer with a latent of its own writes its cache slot, one without reads another's")
         n = proj.shape[0]
-        if cache.writes:
-            c = ops.rmsnorm_cols(proj, col0 + self.query_rank, self.latent_dim, self.dkv_norm_w, self.norm_eps, cache.k.dtype)
-            ops.vector_store(c, ctx.slot_mapping[cache.group], cache.k, cache.v)
-        cq = ops.rmsnorm_cols(proj, col0, self.query_rank, self.dq_norm_w, self.norm_eps, self.dtype)
+        if cache.writes and ops.latent_norms_ok(proj, col0, self.query_rank, col0 + self.query_rank, self.latent_dim, cache.k.dtype, self.dtype):
+            cq = ops.latent_norms(proj, col0, self.query_rank, self.dq_norm_w, col0 + self.query_rank, self.latent_dim, self.dkv_norm_w,
+                                  self.norm_eps, ctx.slot_mapping[cache.group], cache.k, cache.v)
+        else:
+            if cache.writes:
+                c = ops.rmsnorm_cols(proj, col0 + self.query_rank, self.latent_dim, self.dkv_norm_w, self.norm_eps, cache.k.dtype)
+                ops.vector_store(c, ctx.slot_mapping[cache.group], cache.k, cache.v)
+            cq = ops.rmsnorm_cols(proj, col0, self.query_rank, self.dq_norm_w, self.norm_eps, self.dtype)
         q = ops.linear(cq, self.w_q, self.dtype).view(n, self.num_heads, self.latent_dim)
         ops.paged_attention(q, cache.k, cache.v, ctx.block_tables[cache.group], ctx.cu_seqlens, ctx.context_lens, ctx.token_req,
                             self.scale, int(self.window or 0), ctx.max_q_len, ctx.max_context_len, ctx.num_single, sink=self.sink_w,

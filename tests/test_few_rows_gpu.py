@@ -497,3 +497,22 @@ def test_choice_of_few_experts(n, experts, top, groups, keep, group_best, sigmoi
             continue
         assert ids[t, : len(order)].tolist() == order, t
         assert torch.allclose(dense[t], want, rtol=1e-5, atol=1e-7) and torch.equal(dense[t][order], weights[t, : len(order)]), t
+
+
+@pytest.mark.parametrize("n", [1, 5, 64])
+@pytest.mark.parametrize("q_dim,c_dim", [(8, 8), (512, 256), (1024, 128), (520, 516), (4096, 4096), (72, 1032)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_latent_norms_and_store(n, q_dim, c_dim, dtype):
+    """Both norms and the cache write in one launch: the bits of the three."""
+    from tempura_amd.kernels import ops
+    g = torch.Generator().manual_seed(n + q_dim + c_dim)
+    c_dim -= c_dim % (16 // dtype.itemsize)
+    rows, qw, cw = torch.randn(n, 4 + q_dim + c_dim + 8, generator=g).to(DEV), torch.randn(q_dim, generator=g).to(DEV), torch.randn(c_dim, generator=g).to(DEV)
+    slots = torch.randperm(80, generator=g)[:n].to(torch.int32).to(DEV)
+    k0, v0 = torch.randn(5, 1, 16, c_dim, generator=g).to(dtype).to(DEV), torch.randn(5, 1, c_dim, 16, generator=g).to(dtype).to(DEV)
+    k1, v1 = k0.clone(), v0.clone()
+    ops.vector_store(ops.rmsnorm_cols(rows, 4 + q_dim, c_dim, cw, 1e-5, dtype), slots, k0, v0)
+    want = ops.rmsnorm_cols(rows, 4, q_dim, qw, 1e-5, dtype)
+    assert ops.latent_norms_ok(rows, 4, q_dim, 4 + q_dim, c_dim, dtype, dtype) and not ops.latent_norms_ok(rows, 2, q_dim, 4, c_dim, dtype, dtype)
+    got = ops.latent_norms(rows, 4, q_dim, qw, 4 + q_dim, c_dim, cw, 1e-5, slots, k1, v1)
+    assert torch.equal(got, want) and torch.equal(k0, k1) and torch.equal(v0, v1)

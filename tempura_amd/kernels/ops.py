@@ -1200,13 +1200,19 @@ def paged_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tenso
     return None
 
 
-def attention_rows_ok(rows, ctx, heads: int, kvh: int, dim: int, value_dim: int, k_cache: torch.Tensor, conv_taps: int = 0, window: int = 0) -> bool:
-    """Whether ``attention_rows`` takes a projection's float32 ``rows`` (or ``Partials``): a step of single tokens, bfloat16 caches."""
+def attention_rows_ok(rows, ctx, heads: int, kvh: int, dim: int, value_dim: int, k_cache: torch.Tensor, conv_taps: int = 0, window: int = 0,
+                      col0: int = 0, state: Optional[torch.Tensor] = None, state_off: int = 0) -> bool:
+    """Whether ``attention_rows`` takes a projection's float32 ``rows`` (or ``Partials``) from column ``col0`` on: a step of single tokens,
+    bfloat16 caches, and everything read in pairs of floats at even places, the carried inputs of a convolution (from ``state_off`` on in
+    the rows of ``state``) among them."""
     data = rows.data if isinstance(rows, Partials) else rows
     page_size = k_cache.shape[2]
     if not (_backend is None and allow_fast_attention and rows_attention and k_cache.dtype == torch.bfloat16 and k_cache.shape[3] == dim == value_dim
             and dim in (64, 128) and decode_rings(dim, dim, page_size) and heads // kvh <= 16 and ctx.num_requests == ctx.num_single == ctx.num_tokens
-            and data.dtype == torch.float32 and data.shape[-1] % 2 == 0 and data.data_ptr() % 8 == 0 and (data.dim() == 2 or data.shape[0] <= 8)):
+            and ctx.num_tokens <= 65535 and data.dtype == torch.float32 and data.shape[-1] % 2 == 0 and data.data_ptr() % 8 == 0 and col0 % 2 == 0
+            and (data.dim() == 2 or data.shape[0] <= 8)):
+        return False
+    if conv_taps and state is not None and (state.shape[1] % 2 != 0 or state_off % 2 != 0 or state.data_ptr() % 8 != 0):
         return False
     # (a channel's carried inputs have one block: with a convolution the keys are not split, for which 1,024 keys are a microsecond more
     # than split, and the two launches in front of the attention 5)
@@ -1244,9 +1250,9 @@ def attention_rows(rows, col0: int, ctx, group: int, heads: int, kvh: int, dim: 
     bt = ctx.block_tables[group]
     slots = ctx.slot_mapping[group]
     _dev_ok(data, k_cache, v_cache, bt, ctx.context_lens, ctx.positions, slots, inv_freq, cos_sin, sink)
-    _need(attention_rows_ok(rows, ctx, heads, kvh, dim, v_cache.shape[2], k_cache, 0 if conv is None else conv[0].shape[0], window),
-          "attention_rows: sizes that it does not take")
-    _need(data.shape[0] == parts * n and col0 >= 0 and col0 % 2 == 0 and col0 + (heads + 2 * kvh) * dim <= stride, "attention_rows: bad rows")
+    _need(attention_rows_ok(rows, ctx, heads, kvh, dim, v_cache.shape[2], k_cache, 0 if conv is None else conv[0].shape[0], window, col0,
+                            *(() if conv is None else conv[1:])), "attention_rows: sizes that it does not take")
+    _need(data.shape[0] == parts * n and col0 >= 0 and col0 + (heads + 2 * kvh) * dim <= stride, "attention_rows: bad rows")
     pages, _, page_size, _ = k_cache.shape
     _need(k_cache.shape[1] == kvh and tuple(v_cache.shape) == (pages, kvh, dim, page_size) and v_cache.dtype == torch.bfloat16, "attention_rows: bad caches")
     _need(pages * kvh * page_size < 2 ** 31, "paged_attention: cache pool too large for 32-bit row indices")

@@ -508,12 +508,13 @@ class ConvAttention(BranchMixer):
         self.position.load_weights(get)
         return torch.cat([self._to_device(t) for t in rows], dim=0).contiguous(), self._to_device(get(w["o"]))
 
-    def _takes_rows(self, proj, ctx, cache, out) -> bool:
+    def _takes_rows(self, proj, col0, ctx, cache, out) -> bool:
         return cache.writes and out.dtype == torch.bfloat16 and ops.attention_rows_ok(
-            proj, ctx, self.num_heads, self.num_kv_heads, self.head_dim, self.value_dim, cache.k, self.taps, int(self.window or 0))
+            proj, ctx, self.num_heads, self.num_kv_heads, self.head_dim, self.value_dim, cache.k, self.taps, int(self.window or 0), col0,
+            cache.state, self.state_off)
 
-    def takes_beside(self, proj, ctx, cache, out, heads):
-        return heads > 0 and self._takes_rows(proj, ctx, cache, out) and \
+    def takes_beside(self, proj, col0, ctx, cache, out, heads):
+        return heads > 0 and self._takes_rows(proj, col0, ctx, cache, out) and \
             ops.attention_beside_ok(ctx, self.num_heads, self.num_kv_heads, int(self.window or 0), self.taps, heads)
 
     def run(self, proj, col0, ctx, cache, out, out_col0, scale, beside=None):
@@ -525,7 +526,7 @@ class ConvAttention(BranchMixer):
             inv_freq, rotary_dim, factor = rot
             table = self.position.table(ctx) if hasattr(self.position, "table") else None
         into = (proj if self.gate else None, col0 + self.channels, scale, out, out_col0, self.gate_per if self.gate else 1)
-        if self._takes_rows(proj, ctx, cache, out):
+        if self._takes_rows(proj, col0, ctx, cache, out):
             ops.attention_rows(proj, col0, ctx, cache.group, self.num_heads, self.num_kv_heads, self.head_dim, cache.k, cache.v, self.scale,
                                inv_freq, rotary_dim, factor, table, int(self.window or 0), norms=self.norms,
                                norm_eps=float(self.qk_norm["eps"]) if self.qk_norm is not None else 0.0,

@@ -170,7 +170,7 @@ class BranchMixer(Mixer):
     def run(self, proj, col0, ctx, cache, out, out_col0, scale) -> None:
         raise NotImplementedError
 
-    def takes_beside(self, proj, ctx, cache, out, heads: int) -> bool:
+    def takes_beside(self, proj, col0, ctx, cache, out, heads: int) -> bool:
         """Whether ``run`` would take another branch's prepared step (``beside``), a block for each of ``heads`` heads, into its launch."""
         return False
 

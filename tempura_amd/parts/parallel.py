@@ -80,7 +80,7 @@ class ParallelMixer(Mixer):
         todo = list(zip(self.branches, self.in_cols, self.out_cols, self.scales))
         # (single tokens: a recurrent branch's step runs in the launch of the attention beside it)
         for host in todo:
-            guest = next((t for t in todo if t is not host and host[0].takes_beside(proj, ctx, cache, act, getattr(t[0], "num_heads", 0))), None)
+            guest = next((t for t in todo if t is not host and host[0].takes_beside(proj, host[1], ctx, cache, act, getattr(t[0], "num_heads", 0))), None)
             step = guest[0].prepare(proj, guest[1], ctx, cache, act, guest[2], guest[3]) if guest is not None else None
             if step is not None:
                 host[0].run(proj, host[1], ctx, cache, act, host[2], host[3], beside=step)

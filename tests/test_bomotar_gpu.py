@@ -368,6 +368,20 @@ def test_every_cutting_matches_plain(dirs, name, mode, dtype):
     assert runner.cache.free_pages() == [p.num_pages for p in runner.cache.pools]
 
 
+def test_state_rows_of_an_odd_number_of_floats(tmp_path, monkeypatch):
+    """The attention's carried inputs and a recurrence with values of 33 share a state row: 9,321 floats, so that every other request's begins
+    at an odd place.  Decoded steps beside whole prompts, bfloat16."""
+    layer = cases._layer(cases._left(4, 2, 64, 64, 4, rot_dims=32, base=1e4), cases._right(3, 3, 64, 33, 4, 8, 8), cases._dense(128), 0.8, 0.7)
+    monkeypatch.setitem(cases.CASES, "odd", cases._case(90, 128, [layer, layer], 53, 31, 7, mult=0.7))
+    runner = _runner(cases.write_model("odd", str(tmp_path / "odd")), "bfloat16", 192)
+    assert all(t.shape[1] % 2 == 1 for t in runner.pools.state.values())
+    reqs = {r: cases.tokens("odd", n, 70 + n) for r, n in (("a", 40), ("b", 33), ("c", 25))}
+    got = helpers.run_schedule(runner, reqs, helpers.schedule_bulk_tail({r: len(t) for r, t in reqs.items()}, tail=12))
+    for r, toks in reqs.items():
+        err = plain.logit_error(got[r], plain.forward(cases.config_json("odd"), cases.make_weights("odd"), toks))
+        assert err < TOL["bfloat16"], f"request {r}: error {err:.3e}"
+
+
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 def test_cutting_changes_rounding_only(dirs, dtype):
     """The same request whole, in portions and beside others: float32 differs in summation order only; bfloat16 runs

@@ -1,0 +1,27 @@
+"""The rules by which a step of single tokens takes its kernels: what they accept has to be what the kernels take, and a step padded to
+more rows has to be decided as the step itself.  No GPU: the rules read sizes only."""
+from types import SimpleNamespace
+
+import pytest
+import torch
+
+from tempura_amd.kernels import ops
+
+
+def _step(n, longest):
+    return SimpleNamespace(num_tokens=n, num_requests=n, num_single=n, max_context_len=longest)
+
+
+@pytest.mark.parametrize("what,takes", [("plain", True), ("odd state rows", False), ("odd place in the state", False), ("odd first column", False),
+                                        ("odd state rows without a convolution", True), ("more requests than a grid has rows", False)])
+def test_rows_at_odd_places_keep_the_separate_kernels(what, takes):
+    """The kernel that takes a projection's rows reads pairs of floats, and has a request a row of its grid."""
+    heads, kv, d, taps = 4, 2, 64, 4
+    width = (heads + 2 * kv) * d
+    n = 65536 if what.startswith("more") else 3
+    rows = torch.empty((1, width + 8)).expand(n, -1)
+    k = torch.empty((4, kv, 16, d), dtype=torch.bfloat16)
+    state = torch.empty((n if n < 9 else 1, (taps - 1) * width + 10 + ("odd state rows" in what)))
+    got = ops.attention_rows_ok(rows, _step(n, 300), heads, kv, d, d, k, 0 if "without" in what else taps, 0, 3 if "column" in what else 2, state,
+                                5 if "place" in what else 4)
+    assert got is takes

@@ -1232,7 +1232,8 @@ def _rows_splits(ctx, heads: int, kvh: int, window: int, keep_first: int, chunk:
 
 def attention_beside_ok(ctx, heads: int, kvh: int, window: int, conv_taps: int, step_heads: int) -> bool:
     """Whether ``attention_rows`` should run a recurrent mixer's step in its launch: while the blocks of both have a CU each."""
-    return ctx.num_tokens * (kvh * _rows_splits(ctx, heads, kvh, window, 0, 0, conv_taps > 0, True) + step_heads) <= 256
+    # (of the rows that the step is sized for: beside the mixer the keys are cut otherwise, and a captured step has to do as an eager one)
+    return decode_rows_padded(ctx.num_tokens) * (kvh * _rows_splits(ctx, heads, kvh, window, 0, 0, conv_taps > 0, True) + step_heads) <= 256
 
 
 def attention_rows(rows, col0: int, ctx, group: int, heads: int, kvh: int, dim: int, k_cache: torch.Tensor, v_cache: torch.Tensor, scale: float,

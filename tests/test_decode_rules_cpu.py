@@ -25,3 +25,18 @@ def test_rows_at_odd_places_keep_the_separate_kernels(what, takes):
     got = ops.attention_rows_ok(rows, _step(n, 300), heads, kv, d, d, k, 0 if "without" in what else taps, 0, 3 if "column" in what else 2, state,
                                 5 if "place" in what else 4)
     assert got is takes
+
+
+def _same_for_padded(rule):
+    for n in [*range(1, 140), 200, 256, 300]:
+        assert rule(n) == rule(ops.decode_rows_padded(n)), n
+
+
+@pytest.mark.parametrize("longest", [30, 513, 1100, 5000])
+@pytest.mark.parametrize("kvh,window,taps,step_heads", [(8, 1024, 0, 16), (4, 1024, 0, 8), (3, 0, 4, 5), (12, 0, 0, 24)])
+def test_a_padded_step_runs_a_mixer_beside_the_attention_as_the_step_itself(longest, kvh, window, taps, step_heads):
+    def rule(n):
+        ctx = _step(n, longest)
+        beside = ops.attention_beside_ok(ctx, 2 * kvh, kvh, window, taps, step_heads)
+        return beside, ops._rows_splits(ctx, 2 * kvh, kvh, window, 0, 0, taps > 0, beside)
+    _same_for_padded(rule)

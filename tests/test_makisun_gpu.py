@@ -529,6 +529,27 @@ def test_a_captured_step_gives_the_bits_of_the_eager_one(dirs):
     assert torch.equal(runs[0], runs[1])
 
 
+@pytest.mark.parametrize("n,kv,step_heads,context", [(5, 8, 16, 1100)])
+def test_a_captured_step_takes_the_kernels_of_the_eager_one(tmp_path, n, kv, step_heads, context):
+    """Numbers of requests that are no power of two, where the rows that a captured step is padded to would decide otherwise than the
+    requests: whether the recurrence runs beside the attention, whose keys are then cut into other splits.  Bit for bit."""
+    from tempura_amd.engine.runner import StepEntry
+    cfg = cases.config_json("wide")
+    left = cases._left(kv, kv, 64, 64, 0.125, 32, 10000.0)
+    cfg["layers"] = [cases._layer(cases._parallel(left, cases._right(step_heads, 64, 64, 12.0), 0.8, 0.9), cases._dense(128))] * 2
+    folder = cases.write_model("wide", str(tmp_path / "m"), weights=cases.make_weights("wide", 5, cfg=cfg), config=cfg)
+    seqs = [cases.tokens("wide", context + 6 - i % 3, 80 + i) for i in range(n)]
+    runs = []
+    for use_graph in (False, True):
+        runner = _runner(folder, "bfloat16", n * (context + 32), max_requests=n, use_graph=use_graph)
+        for i, toks in enumerate(seqs):
+            runner.add_request(i)
+            runner.step([StepEntry(i, toks[:-4], [])])
+        runs.append(torch.stack([runner.step([StepEntry(i, [toks[len(toks) - 4 + t]], [0]) for i, toks in enumerate(seqs)]).cpu().clone() for t in range(4)]))
+        assert not use_graph or runner.graph_steps == 4
+    assert torch.equal(runs[0], runs[1])
+
+
 @pytest.mark.parametrize("name", ["mix", "wide"])
 @pytest.mark.parametrize("use_graph", [False, True])
 def test_engine_generates_what_plain_greedy_generates(dirs, name, use_graph):

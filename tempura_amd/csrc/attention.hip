@@ -114,7 +114,7 @@ __global__ __launch_bounds__(64) void paged_attention_kernel(
 int tp_paged_attention_fast(const void* q, const void* k_cache, const void* v_cache, const int* block_tables,
                             int table_width, const int* cu_seqlens, const int* context_lens, void* out, int n_tokens,
                             int n_req, int n_heads, int n_kv, int head_dim, int page_size, float scale, int window,
-                            int max_q_len, int num_single, int num_splits, float* scratch, const int* token_req,
+                            int max_q_len, int num_single, int num_splits, int decode_waves, float* scratch, const int* token_req,
                             int portion_splits, int portion_min_steps, float* portion_scratch, const float* dist_bias,
                             int bias_len, int keep_first, const float* sink, int value_dim, int chunk, float softcap,
                             int gated, const float* gate, int gate_stride, int gate_col0, int gate_per, float gate_scale, int out_stride,
@@ -132,7 +132,7 @@ extern "C" int tp_paged_attention(const void* q, int dt, const void* k_cache, co
                                   const int* context_lens, const int* token_req, void* out, int n_tokens,
                                   int n_req, int n_heads, int n_kv, int head_dim, int page_size, float scale,
                                   int window, int max_q_len, int max_ctx, int allow_fast, int num_single,
-                                  int num_splits, float* scratch, int portion_splits, int portion_min_steps,
+                                  int num_splits, int decode_waves, float* scratch, int portion_splits, int portion_min_steps,
                                   float* portion_scratch, const float* dist_bias, int bias_len, int value_dim,
                                   int keep_first, const float* sink, int chunk, float softcap, const float* gate, int gate_stride,
                                   int gate_col0, int gate_per, float gate_scale, int out_stride, int out_col0, hipStream_t s) {
@@ -171,7 +171,7 @@ extern "C" int tp_paged_attention(const void* q, int dt, const void* k_cache, co
   if (dt == TP_BF16 && allow_fast) {
     const int rc = tp_paged_attention_fast(q, k_cache, v_cache, block_tables, table_width, cu_seqlens,
                                            context_lens, out, n_tokens, n_req, n_heads, n_kv, head_dim,
-                                           page_size, scale, window, max_q_len, num_single, num_splits, scratch, token_req,
+                                           page_size, scale, window, max_q_len, num_single, num_splits, decode_waves, scratch, token_req,
                                            portion_splits, portion_min_steps, portion_scratch, dist_bias, bias_len, keep_first, sink, value_dim, chunk,
                                            softcap, allow_fast == 2, gate, gate_stride, gate_col0, gate_per, gate_scale, out_stride, out_col0, s);
     if (rc >= 0) return rc;

@@ -109,6 +109,7 @@ struct AttnArgs {
   int portion_min_steps;   // a query block is split into at most (its steps / this) parts
   float* portion_scratch;
   const int* token_req;
+  int decode_waves;  // of a block of single tokens whose keys go to LDS, 4 or 8
   bool all_single;  // (every request brings one token: request r's row is row r)
   bool gated;       // (every request brings one token: the rows go through `gate`)
   CombineGate gate;
@@ -1827,11 +1828,10 @@ static int launch_all(AttnArgs a, int n_tokens, int n_req, int max_q_len, int nu
     }
     bool done = bias;
     if constexpr (LDS && DV <= 128) {
-      // rings of 64 KB a block, two blocks a CU; where the keys are not split and every block has a CU of its own, twice the waves
-      // (one request of 500 keys of 64 elements 7.2 -> 6.4 us, 32 of 3,000 36.1 -> 35.6; 48 requests, 384 blocks, 20.6 -> 22.7)
+      // rings of 64 KB a block, two blocks a CU; twice the waves where the caller knows that every block has a CU of its own
       constexpr int NB = (D + DV) * 64 > 8192 ? 1 : 2;
       if (!bias && a.page_shift >= 4 && g_attn_tune != 1) {
-        if (a.num_splits == 1 && grid.x * grid.y <= 256)
+        if (a.decode_waves == 8)
           hipLaunchKernelGGL((attn_decode_lds_kernel<D, DV, MODE, 8, NB>), grid, dim3(512), 0, s, a, RowsIn{});
         else
           hipLaunchKernelGGL((attn_decode_lds_kernel<D, DV, MODE, 4, NB>), grid, dim3(256), 0, s, a, RowsIn{});
@@ -1952,7 +1952,7 @@ static int launch_sizes(const AttnArgs& a, int d, int dv, int n_tokens, int n_re
 
 static AttnArgs decode_args(const bf16_t* k_cache, const bf16_t* v_cache, const int* block_tables, int table_width, const int* cu_seqlens,
                             const int* context_lens, bf16_t* out, int n_heads, int n_kv, int page_size, float scale, int window, int num_splits,
-                            float* scratch, int keep_first, const float* sink, int chunk) {
+                            int decode_waves, float* scratch, int keep_first, const float* sink, int chunk) {
   AttnArgs a = {};
   a.k_cache = k_cache;
   a.v_cache = v_cache;
@@ -1970,6 +1970,7 @@ static AttnArgs decode_args(const bf16_t* k_cache, const bf16_t* v_cache, const 
     if ((1 << b) == page_size) a.page_shift = b;
   a.window = window;
   a.num_splits = num_splits;
+  a.decode_waves = decode_waves;
   a.portion_splits = 1;
   a.portion_min_steps = 1;
   a.heads_per_block = 4;
@@ -1986,7 +1987,7 @@ static AttnArgs decode_args(const bf16_t* k_cache, const bf16_t* v_cache, const 
 
 // Single tokens from their projection's rows (see RowsIn and attn_decode_lds_kernel): n requests of one token each, heads of 64 or 128
 // elements, values alike, at most 16 heads a key head, pages of a power of two from 16 on.  beside: a step that tp_delta_step or
-// tp_linear_step wrote down, of the same requests, to run in the same launch (nullptr: none).  With num_splits > 1 scratch of n * n_heads *
+// tp_linear_step wrote down, of the same requests, to run in the same launch (nullptr: none; then decode_waves is 8).  With num_splits > 1 scratch of n * n_heads *
 // num_splits * (dim + 2) floats, and no convolution (a channel's carried inputs have one block).  gated: out as of tp_paged_attention
 // with allow_fast 2.
 extern "C" int tp_attention_rows(const float* rows, size_t part_stride, int stride, int parts, const float* conv_w, int taps, int channels,
@@ -1994,7 +1995,7 @@ extern "C" int tp_attention_rows(const float* rows, size_t part_stride, int stri
                                  const float* k_norm, float norm_eps, const int* positions, const double* inv_freq, int rotary_dim, float factor,
                                  const float* cos_sin, const int* slots, void* k_cache, void* v_cache, const int* block_tables, int table_width,
                                  const int* cu_seqlens, const int* context_lens, void* out, int n, int n_heads, int n_kv, int dim, int page_size,
-                                 float scale, int window, int keep_first, int chunk, const float* sink, int num_splits, float* scratch, int gated,
+                                 float scale, int window, int keep_first, int chunk, const float* sink, int num_splits, int decode_waves, float* scratch, int gated,
                                  const float* gate, int gate_stride, int gate_col0, int gate_per, float gate_scale, int out_stride, int out_col0,
                                  const void* beside, hipStream_t s) {
   TP_REQUIRE(n >= 0 && n <= 65535 && n_kv > 0 && n_heads > 0 && n_heads <= 65535 && n_heads % n_kv == 0 && n_heads / n_kv <= 16 && (dim == 64 || dim == 128),
@@ -2009,7 +2010,8 @@ extern "C" int tp_attention_rows(const float* rows, size_t part_stride, int stri
                                    state_stride >= state_off + (size_t)(taps - 1) * channels),
              "attention_rows: bad convolution");
   TP_REQUIRE((q_norm == nullptr) == (k_norm == nullptr), "attention_rows: a norm needs both weights");
-  TP_REQUIRE(num_splits >= 1 && num_splits <= 64 && (num_splits == 1 || scratch), "attention_rows: bad splits");
+  TP_REQUIRE(num_splits >= 1 && num_splits <= 64 && (num_splits == 1 || scratch) && (decode_waves == 8 || (decode_waves == 4 && beside == nullptr)),
+             "attention_rows: bad splits");
   TP_REQUIRE(window >= 0 && keep_first >= 0 && chunk >= 0 && chunk != 1 && (chunk == 0 || window == 0), "attention_rows: bad mask");
   const int width = n_heads * dim;
   TP_REQUIRE(!gated || (out_col0 >= 0 && out_stride >= out_col0 + width && gate_per >= 1 && width % gate_per == 0 &&
@@ -2017,14 +2019,14 @@ extern "C" int tp_attention_rows(const float* rows, size_t part_stride, int stri
              "attention_rows: bad gate or output rows");
   if (n == 0) return 0;
   AttnArgs a = decode_args((const bf16_t*)k_cache, (const bf16_t*)v_cache, block_tables, table_width, cu_seqlens, context_lens, (bf16_t*)out, n_heads,
-                           n_kv, page_size, scale, window, num_splits, scratch, keep_first, sink, chunk);
+                           n_kv, page_size, scale, window, num_splits, decode_waves, scratch, keep_first, sink, chunk);
   a.all_single = true;
   a.gated = gated != 0;
   a.gate = CombineGate{gate, gate_stride, gate_col0, gate_per, out_stride, out_col0, gate_scale};
   const RowsIn in = {rows, part_stride, stride, parts, conv_w, state, state_stride, state_off, state_slots, taps, channels, q_norm, k_norm, norm_eps,
                      factor, (const float2*)cos_sin, positions, inv_freq, rotary_dim, slots, (bf16_t*)k_cache, (bf16_t*)v_cache};
   const dim3 grid(n_kv, n, num_splits);
-  const bool wide = num_splits == 1 && (long)n_kv * n <= 256;
+  const bool wide = decode_waves == 8;
 #define ROWS_KERNEL(D_, W_, NB_) hipLaunchKernelGGL((attn_decode_lds_kernel<D_, D_, MODE_PLAIN, W_, NB_, true>), grid, dim3(W_ * 64), 0, s, a, in)
   if (beside != nullptr) {
     const PreparedStep* st = (const PreparedStep*)beside;
@@ -2055,7 +2057,7 @@ extern "C" int tp_attention_rows(const float* rows, size_t part_stride, int stri
 int tp_paged_attention_fast(const void* q, const void* k_cache, const void* v_cache, const int* block_tables,
                             int table_width, const int* cu_seqlens, const int* context_lens, void* out, int n_tokens,
                             int n_req, int n_heads, int n_kv, int head_dim, int page_size, float scale, int window,
-                            int max_q_len, int num_single, int num_splits, float* scratch, const int* token_req,
+                            int max_q_len, int num_single, int num_splits, int decode_waves, float* scratch, const int* token_req,
                             int portion_splits, int portion_min_steps, float* portion_scratch, const float* dist_bias,
                             int bias_len, int keep_first, const float* sink, int value_dim, int chunk, float softcap,
                             int gated, const float* gate, int gate_stride, int gate_col0, int gate_per, float gate_scale, int out_stride,
@@ -2068,12 +2070,12 @@ int tp_paged_attention_fast(const void* q, const void* k_cache, const void* v_ca
   if (portion_splits < 1 || portion_splits > 64 || (portion_splits > 1 && (portion_scratch == nullptr || token_req == nullptr))) return -1;
   if ((long)n_req * portion_splits > 65535) return -1;
   if (n_req > 65535 || n_req <= 0) return -1;
-  if (num_single > 0 && (num_splits < 1 || num_splits > 64)) return -1;
+  if (num_single > 0 && (num_splits < 1 || num_splits > 64 || (decode_waves != 4 && decode_waves != 8))) return -1;
   if (num_single > 0 && num_splits > 1 && scratch == nullptr) return -1;
   if (gated && num_single != n_req) return -1;
   if (dist_bias != nullptr && bias_len <= 0) return -1;
   AttnArgs a = decode_args((const bf16_t*)k_cache, (const bf16_t*)v_cache, block_tables, table_width, cu_seqlens, context_lens, (bf16_t*)out, n_heads,
-                           n_kv, page_size, scale, window, num_splits, scratch, keep_first, sink, chunk);
+                           n_kv, page_size, scale, window, num_splits, decode_waves, scratch, keep_first, sink, chunk);
   a.q = (const bf16_t*)q;
   a.all_single = num_single == n_req;
   a.gated = gated != 0;

@@ -40,3 +40,12 @@ def test_a_padded_step_runs_a_mixer_beside_the_attention_as_the_step_itself(long
         beside = ops.attention_beside_ok(ctx, 2 * kvh, kvh, window, taps, step_heads)
         return beside, ops._rows_splits(ctx, 2 * kvh, kvh, window, 0, 0, taps > 0, beside)
     _same_for_padded(rule)
+
+
+@pytest.mark.parametrize("longest", [200, 1000, 3000])
+@pytest.mark.parametrize("heads,kvh", [(8, 8), (24, 12), (6, 3), (80, 5), (32, 1)])
+def test_a_padded_step_has_the_splits_and_waves_of_the_step_itself(longest, heads, kvh):
+    def rule(n):
+        splits = ops._decode_splits(n, heads, kvh, longest, 0, 0, 0, True)
+        return splits, ops._decode_waves(n, heads, kvh, splits)
+    _same_for_padded(rule)

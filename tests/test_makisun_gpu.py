@@ -529,10 +529,11 @@ def test_a_captured_step_gives_the_bits_of_the_eager_one(dirs):
     assert torch.equal(runs[0], runs[1])
 
 
-@pytest.mark.parametrize("n,kv,step_heads,context", [(5, 8, 16, 1100)])
+@pytest.mark.parametrize("n,kv,step_heads,context", [(5, 8, 16, 1100), (17, 12, 5, 200), (9, 3, 8, 300)])
 def test_a_captured_step_takes_the_kernels_of_the_eager_one(tmp_path, n, kv, step_heads, context):
     """Numbers of requests that are no power of two, where the rows that a captured step is padded to would decide otherwise than the
-    requests: whether the recurrence runs beside the attention, whose keys are then cut into other splits.  Bit for bit."""
+    requests: whether the recurrence runs beside the attention, whose keys are then cut into other splits, and how many waves a block of the
+    attention has.  Bit for bit."""
     from tempura_amd.engine.runner import StepEntry
     cfg = cases.config_json("wide")
     left = cases._left(kv, kv, 64, 64, 0.125, 32, 10000.0)

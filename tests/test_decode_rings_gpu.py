@@ -164,3 +164,103 @@ def test_a_step_beside_the_attention(d, kv, ctx_lens, kind, n_step, dim, vdim):
     assert all(torch.equal(a, c) for a, c in zip(*caches))
     # (the attention's sums by eight waves here and by four there where the keys are split)
     assert float((outs[0][:, :out_col0].float() - outs[1][:, :out_col0].float()).norm()) <= 2.0 ** -8 * float(outs[0][:, :out_col0].float().norm())
+
+
+def _from_rows_and_apart(ops, ctx, rows, heads, kv, d, k, v, g, conv_state=None, norms=None, rotary=0, **mask):
+    """(launches apart, one launch): outputs and caches of ``attention_rows`` and of the kernels that it stands for."""
+    width, n = (heads + 2 * kv) * d, ctx.num_tokens
+    freq = (10000.0 ** -torch.arange(0, 1, 2.0 / max(2, rotary), dtype=torch.float64))[: rotary // 2].contiguous().to(DEV)
+    k2, v2, plain, conv = k.clone(), v.clone(), rows.clone(), None
+    if conv_state is not None:
+        state, off, taps = conv_state
+        conv_w, state2 = torch.randn(taps, width, generator=g).to(DEV), state.clone()
+        plain = ops.causal_conv(plain, 0, width, conv_w, None, state2, ctx.cu_seqlens, ctx.token_req, ctx.state_slots, n, state_off=off, act=False, max_run=1)
+        conv = (conv_w, state, off)
+    if norms is not None:
+        ops.head_rmsnorm(plain, 0, heads, norms[0], heads * d, kv, norms[1], d, 1e-6)
+    q = ops.rope_kv_write(plain, ctx.positions, ctx.slot_mapping[0], freq if rotary else None, rotary, 1.0, heads, kv, d, k2, v2, torch.bfloat16)
+    want = ops.paged_attention(q, k2, v2, ctx.block_tables[0], ctx.cu_seqlens, ctx.context_lens, ctx.token_req, d ** -0.5, mask.get("window", 0), 1,
+                               ctx.max_context_len, n, sink=mask.get("sink"), keep_first=mask.get("keep_first", 0), chunk=mask.get("chunk", 0))
+    got = ops.attention_rows(rows, 0, ctx, 0, heads, kv, d, k, v, d ** -0.5, freq if rotary else None, rotary, 1.0, None, norms=norms, norm_eps=1e-6,
+                             conv=conv, **mask)
+    if conv is not None:
+        assert torch.equal(state, state2)
+    return (want, k2, v2), (got, k, v)
+
+
+@pytest.mark.parametrize("heads,kv,d", [(6, 2, 128), (8, 8, 64)])
+@pytest.mark.parametrize("ctx_lens", [[1, 33, 40, 47, 300], [2000, 700, 64, 1]])
+@pytest.mark.parametrize("mask", [{"sink": True}, {"window": 40, "keep_first": 7}, {"window": 700, "keep_first": 40, "sink": True}, {"chunk": 48}, {"chunk": 1},
+                                  {"chunk": 700, "sink": True}])
+def test_masks_from_the_projections_rows(heads, kv, d, ctx_lens, mask):
+    """A sink, kept first keys and chunks, keys split or not: bit for bit."""
+    ops = _ops()
+    g = torch.Generator().manual_seed(heads + d + len(ctx_lens))
+    ctx, k, v = _step(ctx_lens, kv, d, 16, g)
+    rows = torch.randn(len(ctx_lens), (heads + 2 * kv) * d, generator=g).to(DEV)
+    assert ops.attention_rows_ok(rows, ctx, heads, kv, d, d, k)
+    more = {**mask, **({"sink": torch.randn(heads, generator=g).to(DEV)} if "sink" in mask else {})}
+    for want, got in zip(*_from_rows_and_apart(ops, ctx, rows, heads, kv, d, k, v, g, rotary=d, **more)):
+        assert torch.equal(want, got)
+
+
+@pytest.mark.parametrize("n,heads,kv", [(9, 8, 8), (70, 2, 1)])
+def test_a_convolution_in_front_of_many_long_requests(n, heads, kv):
+    """More than 64 blocks and more than 1,024 keys: the keys stay whole, in blocks of eight waves and of four."""
+    ops = _ops()
+    g = torch.Generator().manual_seed(n)
+    d, taps = 64, 4
+    ctx, k, v = _step([1 + i * 1500 // (n - 1) for i in range(n)], kv, d, 16, g)
+    width = (heads + 2 * kv) * d
+    rows = torch.randn(n, width, generator=g).to(DEV)
+    state = torch.randn(n + 2, 6 + (taps - 1) * width, generator=g).to(DEV)
+    assert ops.attention_rows_ok(rows, ctx, heads, kv, d, d, k, taps, 0, 0, state, 6)
+    one = _from_rows_and_apart(ops, ctx, rows, heads, kv, d, k, v, g, conv_state=(state, 6, taps), rotary=32)
+    assert torch.equal(one[0][1], one[1][1]) and torch.equal(one[0][2], one[1][2])
+    # (apart the keys are cut into splits: sums of float32 in another order, then a rounding to bfloat16)
+    assert float((one[0][0].float() - one[1][0].float()).norm()) <= 2.0 ** -8 * float(one[0][0].float().norm())
+
+
+@pytest.mark.parametrize("kind,n_step,dim,vdim", [("delta", 3, 64, 64), ("linear", 2, 100, 72)])
+@pytest.mark.parametrize("how", ["convolution", "norms and rotation"])
+def test_a_step_beside_what_an_attention_brings(kind, n_step, dim, vdim, how):
+    """Beside an attention with a convolution, whose carried inputs lie in the state rows of the step, and beside one with a norm per head and
+    a rotation: outputs, states and caches bit for bit those of two launches."""
+    ops = _ops()
+    d, kv, ctx_lens = 64, 2, [1, 700, 900, 33]
+    g = torch.Generator().manual_seed(dim + len(how))
+    ctx, k, v = _step(ctx_lens, kv, d, 16, g)
+    n, heads, width = len(ctx_lens), 2 * kv, 4 * kv * d
+    rnd = lambda *s: torch.randn(*s, generator=g).to(DEV)
+    rows, (hd, hv), rank, taps = rnd(n, width), (n_step * dim, n_step * vdim), 33, 4
+    channels, front = 2 * hd + hv, 3 * width
+    proj = rnd(n, (2 * channels + 2 * rank + 3) // 4 * 4)
+    off = front + (taps - 1) * channels
+    state0 = rnd(n + 2, (off + hd * vdim + 3) // 4 * 4)
+    w2, b, nw, a_log, cw, g2 = rnd(rank, hd) * 0.3, rnd(hd) - 2.0, rnd(vdim), rnd(n_step), rnd(taps, channels), rnd(rank, hv)
+    conv_w, norms = rnd(4, width), tuple(torch.rand(d, generator=g).add(0.5).to(DEV) for _ in "qk")
+    freq = (10000.0 ** -torch.arange(0, 1, 2.0 / d, dtype=torch.float64)).to(DEV)
+
+    def step(state, out, prepared=None):
+        if kind == "delta":
+            ops.delta_step(proj, 0, channels, channels + n_step, channels + n_step + rank, cw, w2, g2, a_log, b, nw, state, front, off, ctx.token_req,
+                           ctx.state_slots, n_step, dim, vdim, dim ** -0.5, 1e-6, 1e-6, 1.3, out, heads * d, prepared)
+        else:
+            ops.linear_step((proj, 0), (proj, hd), (proj, 2 * hd), (proj, 2 * hd + 2 * hv), w2, "root_sigmoid", b, 0.06, None, None, 0.3,
+                            (proj, 2 * hd + hv), nw, 1e-6, 1.3, state, off, ctx.token_req, ctx.state_slots, n_step, dim, vdim, out, heads * d, prepared)
+    results = []
+    force = ops.decode_force_splits
+    for beside in (False, True):
+        state, out, kk, vv = state0.clone(), torch.zeros(n, heads * d + hv, dtype=torch.bfloat16, device=DEV), k.clone(), v.clone()
+        buffer = ops.step_buffer() if beside else None
+        step(state, out, buffer)
+        conv = (conv_w, state, 0) if how == "convolution" else None
+        try:
+            ops.decode_force_splits = 1      # (whole keys and eight waves both ways)
+            ops.attention_rows(rows, 0, ctx, 0, heads, kv, d, kk, vv, d ** -0.5, freq, d, 1.0, None, norms=None if conv else norms, norm_eps=1e-6, conv=conv,
+                               into=(None, 0, 0.75, out, 0, 1), beside=buffer)
+        finally:
+            ops.decode_force_splits = force
+        results.append((out, state, kk, vv))
+    assert not torch.equal(results[0][1], state0)
+    assert all(torch.equal(a, c) for a, c in zip(*results))

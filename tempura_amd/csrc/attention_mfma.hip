@@ -73,8 +73,7 @@ __device__ inline float quad_rows_max(float x) {
 
 // A sublayer's gate over the heads' outputs, by whichever kernel writes a single token's row, in the order of the gate's own kernel:
 // the row rounded to bfloat16, times sigmoid(gate column) (per columns in a row share one), times a scale, into columns of a wider
-// row (the same bits; a launch of 2.5 to 4 us behind a chain of such: Bomotar's decode step with four of them 387 -> 377 us,
-// Tokatar's with two 282 -> 278).
+// row (the same bits; a launch of 2.5 to 4 us less a layer).
 struct CombineGate {
   const float* rows;      // [n, stride] float32, or nullptr: the scale alone
   int stride, col0, per, out_stride, out_col0;

@@ -97,9 +97,8 @@ extern "C" int tp_group_linear(const void* x, const void* w, float* out, const i
 }
 
 // ---- a product of few column blocks --------------------------------------------------------------
-// out [splits, M, N] float32: partial sums over equal parts of K, for the kernel that consumes the rows to add.  A block of 16 columns
-// pulls at most 57 GB/s, its CU's share of the way to memory, so 128 of them (N = 2,048) stay under the memory's rate however long K is.
-// With the norm behind it, a captured chain, whole / in parts: 2,048 x 8,192 one row 12.8 / 11.0 us, sixteen 16.1 / 12.5; 1,024 x 8,192
+// out [splits, M, N] float32: partial sums over equal parts of K, for the kernel that consumes the rows to add.  A block owns 16 columns:
+// at 2,048 of them half the CUs have no block, and each block walks all of K.  With the norm behind it, a captured chain, whole / in parts: 2,048 x 8,192 one row 12.8 / 11.0 us, sixteen 16.1 / 12.5; 1,024 x 8,192
 // (four parts) 11.9 / 8.5 and 15.4 / 9.8; 2,048 x 4,096 9.3 / 8.5 and 11.3 / 9.7.
 __global__ __launch_bounds__(DG_WAVES * 64) void split_linear_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w,
                                                                       float* __restrict__ out, int M, int N, int K) {

@@ -707,9 +707,11 @@ class StreamClose:
 
 def stream_linear_ok(m: int, width: int, streams: int, dtype: torch.dtype) -> bool:
     """Whether a product of ``m`` rows closes a sublayer over the copies itself: few rows (one tile of the matrix cores) and four copies."""
-    # (Two copies stay with the closing kernel.  The rows go on rounded in front of the norm's scale instead of behind it: errors of whole
-    # models are alike, 0.0025 of mifutar at 4,096 either way, but a small model of two copies with a bias that magnifies one score differs
-    # by chance in one token of 400, 0.030 -> 0.054, more than that model is held to.)
+    # (The kernel is written for four copies.  The rows go on rounded in front of the norm's scale instead of behind it, one rounding to bfloat16
+    # either way.  Against 64 bits: 24 small models of four copies, 2-norm 0.0064 in front and 0.0065 behind, largest difference 0.016 and
+    # 0.016 on average, from 0.006 to 0.09 by model; 4 seeds of mifutar at 4,096 0.00278 and 0.00278.  Two copies came out alike as well, but
+    # one model of two copies that a test holds to a largest difference of 0.05 went from 0.030 to 0.054, which is no more than that measure
+    # moves by rounding alone; so two copies keep the closing kernel.  Three and more than four were not measured.)
     return _backend is None and allow_mfma and dtype == torch.bfloat16 and 0 < m <= 16 and width % 32 == 0 and streams == 4
 
 
@@ -742,8 +744,9 @@ def _stream_linear(x, w, close: StreamClose):
 
 def few_splits(m: int, n: int, k: int) -> int:
     """Into how many parts the K of a product of ``m`` <= 16 rows onto ``n`` columns is cut where its consumer adds partial sums: until
-    there are 256 blocks of 16 columns, a run of 128 a wave left in each."""
-    # (from 4,096 of K on, 9.3 / 8.5 us at 2,048 columns; a shorter one is a single trip to memory for every wave anyway)
+    there are 256 blocks of 16 columns."""
+    # (from 4,096 of K on, 9.3 / 8.5 us at 2,048 columns; a shorter one is a single trip to memory for every wave anyway.  Each part a multiple
+    # of 2,048, which all eight waves of a block walk in the same number of turns; other K were not measured and stay whole)
     splits = 1
     while allow_mfma and 0 < m <= 16 and k >= 4096 and splits < 4 and 2 * splits * (n // 16) <= 256 and k % (2048 * splits) == 0:
         splits *= 2

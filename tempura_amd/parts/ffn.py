@@ -190,8 +190,9 @@ class RoutedExperts(FeedForward):
     function (``ops.ACTIVATIONS``; it reads the float32 sums of the up product).
     ``shared`` (``{"intermediate_size", "activation"}``, tensor roles ``shared_up``, ``shared_down`` and, optionally,
     ``shared_gate`` [1, hidden]): one more plain expert that every token uses, its output, with a gate times
-    sigmoid(w_gate . x), one number a token, added to the routed sum.  The gate row rides along in the shared up product, and the gate multiplies the activations in
-    front of the down product (which is linear), not its result."""
+    sigmoid(w_gate . x), one number a token, added to the routed sum.  The gate row rides along in the shared up product.  In the
+    launches for at most 16 single tokens the gate multiplies the down product's float32 result; in every other step the activations
+    in front of it (the product is linear), before they are rounded to the compute dtype."""
     graph_safe = True
     returns_output = True
 

@@ -1478,14 +1478,16 @@ __device__ inline void attn_decode_lds_block(const AttnArgs& a, const RowsIn& in
   const int steps = decode_steps(a, ctx, first, kept_steps);
   const int per_split = (steps + a.num_splits - 1) / a.num_splits;
   const int s_begin = split * per_split, s_end = min(steps, s_begin + per_split);
-  // A wave's steps are neighbours.  (Every WAVES-th step instead, and all blocks walk pages that were handed out in order side by side:
-  // their reads meet in the same banks of memory.  64 requests of 3,073 to 3,165 keys, 8 key heads of 128, pages as the engine hands them
-  // out 139.4 -> 129.4 us, of one request behind the other 137.9 -> 127.8, at random 128.8 either way; the kernel above 133.6, 131.8 and 131.
-  // A step of 32 layers 7.95 -> 7.85 ms, 128 requests of 3,100 keys 13.75 -> 13.49.)
-  const int run = (s_end - s_begin + WAVES - 1) / WAVES, w_begin = s_begin + wave * run;
-  const int n = max(0, min(s_end - w_begin, run));      // this wave's steps
+  // Of blocks of four waves, two of which share a CU, a wave's steps are neighbours.  (Every fourth step instead, and all blocks walk pages
+  // that were handed out in order side by side: their reads meet in the same banks of memory.  64 requests of 3,073 to 3,165 keys, 8 key
+  // heads of 128, pages as the engine hands them out 139.4 -> 129.4 us, of one request behind the other 137.9 -> 127.8, at random 128.8 either
+  // way; the kernel above 133.6, 131.8 and 131.  A step of 32 layers 7.95 -> 7.85 ms, 128 requests of 3,100 keys 13.75 -> 13.49.)  Of the few
+  // blocks of eight waves a wave takes every eighth: it makes no difference there, 32 requests of 1,000 keys 4.16 ms a step and 4.17 in runs.
+  constexpr bool RUNS = WAVES == 4;
+  const int run = (s_end - s_begin + WAVES - 1) / WAVES, w_begin = s_begin + (RUNS ? wave * run : wave);
+  const int n = max(0, RUNS ? min(s_end - w_begin, run) : (s_end - w_begin + WAVES - 1) / WAVES);      // this wave's steps
   auto key0 = [&](int i) {
-    const int s = w_begin + i;
+    const int s = w_begin + (RUNS ? i : i * WAVES);
     return s < kept_steps ? s * 32 : first + (s - kept_steps) * 32;
   };
   // the pages of the two halves of a step's keys (the second clamped to the last key that exists).  What a page holds behind the

@@ -1033,6 +1033,15 @@ def fast_attention_takes(has_sink: bool, keep_first: int) -> bool:
     return True
 
 
+def _keys_seen(max_context_len: int, window: int, keep_first: int, chunk: int) -> int:
+    """The most keys that a single token sees, by the longest context rounded up to a power of two from 256: a step captured for a bound on
+    the context and an eager step at the actual length then decide alike and give the same bits."""
+    bound = 256
+    while bound < max_context_len:
+        bound *= 2
+    return min(bound, window + keep_first + 31) if window else min(bound, chunk) if chunk else bound
+
+
 def _decode_splits(requests: int, heads: int, kvh: int, max_context_len: int, window: int, keep_first: int, chunk: int, rings: bool) -> int:
     """Into how many splits the keys of a step's single tokens are cut (``rings``: by the kernel of ``decode_rings``)."""
     # enough blocks to fill 256 CUs, but at least 128 keys per block
@@ -1056,12 +1065,7 @@ def _decode_splits(requests: int, heads: int, kvh: int, max_context_len: int, wi
         want = max(want, decode_min_splits)     # (batch 8 of the 8B shape: eight splits 3.87 ms a step, four 3.94)
     if decode_force_splits > 0:
         want = decode_force_splits
-    # (at least 128 keys a split, by the longest context rounded up to a power of two from 256: a step captured
-    # for a bound on the context and an eager step at the actual length then cut alike and give the same bits)
-    bound = 256
-    while bound < max_context_len:
-        bound *= 2
-    seen = min(bound, window + keep_first + 31) if window else min(bound, chunk) if chunk else bound
+    seen = _keys_seen(max_context_len, window, keep_first, chunk)      # (at least 128 keys a split)
     if decode_force_splits == 0 and rings:
         # (a launch and a trip through memory for the kernel that adds the splits, 4 us, against the keys that one block walks
         # alone, 5 us for 512 of 128 elements: 8 key heads of 128, not split / as above, one request of 120 / 500 / 1,000 keys
@@ -1227,12 +1231,20 @@ def attention_rows_ok(rows, ctx, heads: int, kvh: int, dim: int, value_dim: int,
     # (a channel's carried inputs have one block: with a convolution the keys are not split, for which 1,024 keys are a microsecond more
     # than split, and the two launches in front of the attention 5)
     if conv_taps:
-        bound = 256
-        while bound < ctx.max_context_len:
-            bound *= 2
-        seen = min(bound, window) if window else bound
+        seen = min(_keys_seen(ctx.max_context_len, 0, 0, 0), window or 1 << 30)
         return conv_taps <= 4 and data.dim() == 2 and (seen <= 1024 or decode_rows_padded(ctx.num_tokens) * kvh > 64)
     return True
+
+
+def attention_rows_pays(ctx, kvh: int, dim: int, window: int = 0, keep_first: int = 0, chunk: int = 0) -> bool:
+    """Whether ``attention_rows`` is the faster way where it could be taken: its blocks work their rows out before they begin with their keys."""
+    # (A launch of 4 to 5 us saved against that start.  Where two blocks a CU and more share a long stream of keys the start costs more: steps
+    # of 32 layers, 8 key heads of 128, from rows / with the launches apart, 32 requests of 500 / 1,000 / 3,000 keys 3.82 / 3.90, 4.15 / 4.22 and
+    # 5.45 / 5.50 ms, 48 of 500 / 1,800 / 3,000 4.23 / 4.27, 5.53 / 5.56 and 6.69 / 6.68, 64 of 400 / 800 / 3,000 4.25 / 4.29, 4.79 / 4.78 and
+    # 7.69 / 7.53; 128 of 800 / 1,500 / 3,050 7.44 / 7.35, 9.34 / 9.13 and 13.79 / 13.49.  Heads of 64 carry half the bytes a key: the kernels
+    # alone 64 of 3,000 keys 69.3 / 69.5 us, 128 of 800 / 3,000 45.6 / 48.0 and 132.8 / 135.0, with a convolution 55.9 / 57.5 and 152 / 146.)
+    blocks = decode_rows_padded(ctx.num_tokens) * kvh
+    return blocks <= 256 or _keys_seen(ctx.max_context_len, window, keep_first, chunk) * dim <= (2048 if blocks <= 512 else 512) * 128
 
 
 def _rows_splits(ctx, heads: int, kvh: int, window: int, keep_first: int, chunk: int, conv: bool, beside: bool) -> int:

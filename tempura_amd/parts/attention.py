@@ -286,7 +286,8 @@ class PagedAttention(Mixer):
         if q is None:
             rows = self._project(x, cache, rot)
             if cache.writes and (rot is not None or type(self.position).__name__ == "NoPosition") and not self.softcap and self.dist_table is None \
-                    and ops.attention_rows_ok(rows, ctx, self.num_heads, self.num_kv_heads, self.head_dim, self.value_dim, cache.k):
+                    and ops.attention_rows_ok(rows, ctx, self.num_heads, self.num_kv_heads, self.head_dim, self.value_dim, cache.k) \
+                    and ops.attention_rows_pays(ctx, self.num_kv_heads, self.head_dim, int(self.window or 0), self.keep_first, self.chunk):
                 # single tokens: the attention takes the projection's rows itself
                 inv_freq, rotary_dim, factor = rot if rot is not None else (None, 0, 1.0)
                 table = self.position.table(ctx) if hasattr(self.position, "table") else None
@@ -511,7 +512,7 @@ class ConvAttention(BranchMixer):
     def _takes_rows(self, proj, col0, ctx, cache, out) -> bool:
         return cache.writes and out.dtype == torch.bfloat16 and ops.attention_rows_ok(
             proj, ctx, self.num_heads, self.num_kv_heads, self.head_dim, self.value_dim, cache.k, self.taps, int(self.window or 0), col0,
-            cache.state, self.state_off)
+            cache.state, self.state_off) and ops.attention_rows_pays(ctx, self.num_kv_heads, self.head_dim, int(self.window or 0))
 
     def takes_beside(self, proj, col0, ctx, cache, out, heads):
         return heads > 0 and self._takes_rows(proj, col0, ctx, cache, out) and \

@@ -49,3 +49,15 @@ def test_a_padded_step_has_the_splits_and_waves_of_the_step_itself(longest, head
         splits = ops._decode_splits(n, heads, kvh, longest, 0, 0, 0, True)
         return splits, ops._decode_waves(n, heads, kvh, splits)
     _same_for_padded(rule)
+
+
+@pytest.mark.parametrize("longest", [200, 800, 1500, 3000])
+@pytest.mark.parametrize("kvh,dim,window", [(8, 128, 0), (8, 64, 0), (3, 128, 0), (8, 128, 1024), (1, 64, 0)])
+def test_a_padded_step_takes_the_projections_rows_as_the_step_itself(longest, kvh, dim, window):
+    _same_for_padded(lambda n: ops.attention_rows_pays(_step(n, longest), kvh, dim, window))
+
+
+def test_few_blocks_or_short_streams_of_keys_take_the_projections_rows():
+    pays = lambda n, longest, *rest: ops.attention_rows_pays(_step(n, longest), 8, *rest)
+    assert pays(32, 100000, 128) and pays(64, 2000, 128) and not pays(64, 3000, 128) and pays(64, 3000, 64) and not pays(64, 5000, 64)
+    assert pays(128, 500, 128) and not pays(128, 800, 128) and pays(128, 800, 64) and not pays(128, 1500, 64) and pays(64, 100000, 128, 1024)

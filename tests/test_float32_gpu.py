@@ -68,6 +68,56 @@ def test_float32_products_in_blocks_of_128_and_64(small, large, n, k, parts):
     assert torch.equal(ops.linear(few, w, torch.float32, residual=res[:small].clone()), added[:small])
 
 
+# rows and columns at the edges of a block of 128 and of the 16 x 16 tiles; K: whole stages of 32, an odd number of them, a part of one; in parts
+@pytest.mark.parametrize("m,n,k,parts", [(65, 4097, 1536, 6), (128, 4100, 1540, 6), (129, 2050, 1572, 6), (255, 4096, 1568, 4), (300, 3072, 3072, 3),
+                                         (640, 6500, 1600, 1), (700, 5200, 1536, 1)])
+def test_float32_products_in_pieces(m, n, k, parts):
+    """Operands in bfloat16 pieces, plain and added into rows, against float64 with the bound of the products above: of normal operands, of operands
+    over twelve orders of magnitude, of positive ones, and of tiny ones; the same call gives the same bits; a row's bits are the same when rows are
+    added up to the next whole block of 128."""
+    from tempura_amd.kernels import ops
+    lib = ops.library()
+    assert lib.tp_linear_f32_block(m, n, k) == 128 and lib.tp_linear_f32_scratch(m, n, k) == (parts * m * n if parts > 1 else 0)
+    g = torch.Generator().manual_seed(m + n + k)
+    x, w, res = (torch.randn(*s, generator=g).to(DEV) for s in ((m, k), (n, k), (m, n)))
+    tol = 2.0 ** -24 * math.sqrt(k)
+    for a, b in ((x, w), (x * torch.exp(3 * torch.randn(m, k, generator=g)).to(DEV), w * torch.exp(2 * torch.randn(n, k, generator=g)).to(DEV)),
+                 (x.abs(), w.abs()), (x * 2.0 ** -60, w * 2.0 ** -40)):
+        ref, got = a.double() @ b.double().T, ops.linear(a, b, torch.float32)
+        assert _rel(got, ref) < tol
+        assert float(((got.double() - ref).abs() / (a.double().abs() @ b.double().abs().T)).max()) < 2.0 ** -24 * k / 2
+        assert torch.equal(got, ops.linear(a, b, torch.float32))
+    ref, got = x.double() @ w.double().T, ops.linear(x, w, torch.float32)
+    assert _rel(ops.linear(x, w, torch.float32, residual=res.clone()), ref + res.double()) < tol + 2.0 ** -23
+    padded = torch.cat([x, torch.randn((-m) % 128, k, generator=g).to(DEV)])
+    assert torch.equal(ops.linear(padded, w, torch.float32)[:m], got)
+
+
+def test_float32_products_in_pieces_of_extreme_values():
+    """Infinity, NaN and the largest finite values give what the products of whole operands give: infinity of the sign of the factor beside it,
+    NaN for infinity times zero, and finite results of values that bfloat16 would round to infinity."""
+    from tempura_amd.kernels import ops
+    m, n, k = 256, 4096, 1536
+    g = torch.Generator().manual_seed(5)
+    x, w = torch.randn(m, k, generator=g), torch.randn(n, k, generator=g)
+    top = torch.finfo(torch.float32).max
+    x[0, 7], x[1, 100], x[2, 1535], x[3, 0] = math.inf, -math.inf, math.nan, math.inf
+    w[5, 7], w[6, 100] = 0.0, 1000.0 + 1.0 / 3.0
+    w[9, 3] = -math.inf
+    x[4], x[5] = 0.0, 0.0
+    x[4, 11], x[5, 12] = top, -top
+    w[:, 11], w[:, 12] = 0.25, 0.5
+    assert ops.library().tp_linear_f32_block(m, n, k) == 128
+    got = ops.linear(x.to(DEV), w.to(DEV), torch.float32).cpu()
+    ref = x.double() @ w.double().T
+    odd = ~torch.isfinite(ref)
+    assert torch.equal(torch.isnan(got), torch.isnan(ref)) and torch.equal(torch.isinf(got), torch.isinf(ref))
+    assert torch.equal(got[torch.isinf(ref)].double(), ref[torch.isinf(ref)])
+    got, ref = torch.where(odd, 0.0, got.double()), torch.where(odd, 0.0, ref)
+    assert float(((got[4:6] - ref[4:6]).abs() / ref[4:6].abs().clamp_min(1.0)).max()) < 2.0 ** -22
+    assert _rel(got[6:], ref[6:]) < 2.0 ** -24 * math.sqrt(k)
+
+
 @pytest.mark.parametrize("m", [1, 2, 3, 4, 5, 8, 9, 16])
 @pytest.mark.parametrize("n,k", [(3, 4), (130, 260), (1026, 3072)])
 def test_float32_products_norm_and_gate_their_rows(m, n, k):

@@ -583,8 +583,24 @@ __device__ __host__ inline int portion_parts(int steps, int max_parts, int min_s
 }
 
 #define ATTN_BIAS_LDS 1024   // the longest distance table a wave keeps in LDS
-template <int D, int DV, int NQ, int NS = 4, int OCC = 2, int MODE = MODE_PLAIN>
-__global__ __launch_bounds__(256, OCC) void attn_prefill_lds_kernel(AttnArgs a, int skip_single) {
+// The j-th of a step's requests with more than one token (-1: there are fewer).
+__device__ inline int portion_request(const int* __restrict__ cu_seqlens, int n_req, int j) {
+  const int lane = threadIdx.x & 63;
+  for (int base = 0; base < n_req; base += 64) {
+    const int i = base + lane;
+    const bool more = i < n_req && cu_seqlens[i + 1] - cu_seqlens[i] > 1;
+    const unsigned long long b = __ballot(more);
+    const int before = __builtin_amdgcn_mbcnt_hi((unsigned)(b >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)b, 0));
+    const unsigned long long hit = __ballot(more && before == j);
+    if (hit != 0) return base + (int)__builtin_ctzll(hit);
+    j -= (int)__popcll(b);
+  }
+  return -1;
+}
+
+// (stages: NS * (D + DV) * 64 bytes of LDS; lin, gx, gy: the block's number in a grid of gx query blocks, gy head groups and the requests' parts)
+template <int D, int DV, int NQ, int NS, int MODE>
+__device__ inline void attn_prefill_lds_block(const AttnArgs& a, unsigned char* stages, int lin, int gx, int gy, int skip_single, int among) {
   constexpr bool BIAS = MODE == MODE_BIAS, CAP = MODE == MODE_CAP;
   static_assert(!BIAS || NQ == 1, "the distance bias is in the variant of one query tile a wave");
   // (each wave's head has its row of the distance table in LDS: a load from global memory inside the loop would
@@ -598,16 +614,16 @@ __global__ __launch_bounds__(256, OCC) void attn_prefill_lds_kernel(AttnArgs a, 
   constexpr int STAGE = (KI + VI) * 1024;
   static_assert(D == 32 || D == 64 || D == 128 || D == 192, "head size");
   static_assert((KI + VI) % 4 == 0 && VI <= 8, "every wave issues the same number of loads");
-  __shared__ __attribute__((aligned(1024))) unsigned char stages[NS * STAGE];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int g = lane >> 4, c = lane & 15;
   // Blocks go to the eight XCDs in turn, each with an L2 of its own: neighbouring blocks take different
   // kv heads (fastest index), so that one L2 holds the keys and values of few heads, read by all their
   // query blocks; the longest query blocks come first.
-  const int lin = blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z);
-  const int by = lin % gridDim.y, bx = (lin / gridDim.y) % gridDim.x;
-  const int rz = lin / (gridDim.x * gridDim.y);
-  const int r = rz / a.portion_splits, part = rz % a.portion_splits;   // (gridDim.z = requests * parts)
+  const int by = lin % gy, bx = (lin / gy) % gx;
+  const int rz = lin / (gx * gy);
+  const int part = rz % a.portion_splits;                              // (requests * parts)
+  const int r = among > 0 ? portion_request(a.cu_seqlens, among, rz / a.portion_splits) : rz / a.portion_splits;
+  if (r < 0) return;
   const int q_start = a.cu_seqlens[r];
   const int q_len = a.cu_seqlens[r + 1] - q_start;
   if (q_len <= 0 || (skip_single && q_len == 1)) return;
@@ -930,6 +946,12 @@ __global__ __launch_bounds__(256, OCC) void attn_prefill_lds_kernel(AttnArgs a, 
     }
   }
   }
+}
+
+template <int D, int DV, int NQ, int NS = 4, int OCC = 2, int MODE = MODE_PLAIN>
+__global__ __launch_bounds__(256, OCC) void attn_prefill_lds_kernel(AttnArgs a, int skip_single) {
+  __shared__ __attribute__((aligned(1024))) unsigned char stages[NS * (D + DV) * 64];
+  attn_prefill_lds_block<D, DV, NQ, NS, MODE>(a, stages, blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z), gridDim.x, gridDim.y, skip_single, 0);
 }
 
 // ---- prefill, keys of several hundred (latents) -----------------------------------------------
@@ -1388,16 +1410,15 @@ __global__ __launch_bounds__(256) void attn_decode_kernel(AttnArgs a) {
 // that holds it is read, into that step's place in LDS.  The rows travel beside the first keys; a launch or two between the
 // projection and the attention are gone: Bomotar's decode step, four layers with a convolution, 377 -> 361 us; 28 layers of the 3B
 // shape with 48 requests, three parts of K, 3,219 -> 3,187.
-// (bx: key head and block of heads, r: request, split: its part of the keys)
+// (stages: WAVES * NB * (D + DV) * 64 bytes of LDS; bx: key head and block of heads, r: request, split: its part of the keys)
 template <int D, int DV, int MODE, int WAVES, int NB, bool ROWS>
-__device__ inline void attn_decode_lds_block(const AttnArgs& a, const RowsIn& in, int bx, int r, int split) {
+__device__ inline void attn_decode_lds_block(const AttnArgs& a, const RowsIn& in, unsigned char* stages, int bx, int r, int split) {
   constexpr int C = D / 8;             // 16-byte chunks per key row
   constexpr int SH = C == 16 ? 0 : (C == 8 || C == 24 ? 1 : 2);
   constexpr int KI = D / 16, VI = DV / 16, STAGE = (KI + VI) * 1024;
   static_assert((D == 32 || D == 64 || D == 128 || D == 192) && VI <= 8, "sizes");
   static_assert(NB * STAGE >= (DV * 17 + 32) * 4, "room for the merge");
   static_assert((NB == 1 || NB == 2) && 2 * VI + KI <= 63 && 2 * KI + VI <= 63, "the waits below");
-  __shared__ __attribute__((aligned(1024))) unsigned char stages[WAVES * NB * STAGE];
   __shared__ __attribute__((aligned(16))) bf16_t heads_lds[ROWS ? 18 * D : 8];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int g = lane >> 4, c = lane & 15;
@@ -1691,18 +1712,37 @@ __device__ inline void attn_decode_lds_block(const AttnArgs& a, const RowsIn& in
 
 template <int D, int DV, int MODE, int WAVES, int NB, bool ROWS = false>
 __global__ __launch_bounds__(WAVES * 64) void attn_decode_lds_kernel(AttnArgs a, RowsIn in) {
-  attn_decode_lds_block<D, DV, MODE, WAVES, NB, ROWS>(a, in, blockIdx.x, blockIdx.y, blockIdx.z);
+  __shared__ __attribute__((aligned(1024))) unsigned char stages[WAVES * NB * (D + DV) * 64];
+  attn_decode_lds_block<D, DV, MODE, WAVES, NB, ROWS>(a, in, stages, blockIdx.x, blockIdx.y, blockIdx.z);
 }
 
 // The attention of single tokens and the recurrent mixer that stands beside it in one launch: neither fills the chip (32 and 64 blocks
 // for four requests of Bomotar at width 2,048), and each is a chain of trips to memory.  Blocks of 512 threads, the attention's first.
 template <int D, int NB, int KIND, int KS>
 __global__ __launch_bounds__(512) void attn_beside_step_kernel(AttnArgs a, RowsIn in, StepArgs st, int n, int splits) {
+  __shared__ __attribute__((aligned(1024))) unsigned char stages[8 * NB * D * 128];
   const int mine = a.n_kv * n * splits, b = blockIdx.x;
   if (b < mine)
-    attn_decode_lds_block<D, D, MODE_PLAIN, 8, NB, true>(a, in, b % a.n_kv, b / a.n_kv % n, b / (a.n_kv * n));
+    attn_decode_lds_block<D, D, MODE_PLAIN, 8, NB, true>(a, in, stages, b % a.n_kv, b / a.n_kv % n, b / (a.n_kv * n));
   else
     mixer_step_block<KIND, KS, bf16_t>(st, (b - mine) % n, (b - mine) / n);
+}
+
+// The portions of a step and its single tokens in one launch.  Each alone waits for its longest chain of steps and fills neither the chip's
+// waves nor its memory: 700 tokens of a prompt 23.5 us, 31 single tokens with 180 to 1,740 keys 25.6, one after the other 49.6, together 29.2.
+// Blocks of four waves, two a CU by their LDS.  n_req: the requests of the step; single: the decode's blocks, first or (late > 0: their number)
+// behind the portions'; gx, gy: query blocks and head groups.
+template <int D, int DV, int MODE, int NB>
+__global__ __launch_bounds__(256, 2) void attn_both_kernel(AttnArgs a, int n_req, int single, int late, int gx, int gy) {
+  __shared__ __attribute__((aligned(1024))) unsigned char stages[4 * NB * (D + DV) * 64];
+  int b = (int)blockIdx.x - late;
+  if (b >= 0 && b < single) {
+    const int hb = a.n_kv * ((a.n_heads / a.n_kv + 15) / 16);
+    attn_decode_lds_block<D, DV, MODE, 4, NB, false>(a, RowsIn{}, stages, b % hb, b / hb % n_req, b / (hb * n_req));
+  } else {
+    if (b >= single) b -= single;
+    attn_prefill_lds_block<D, DV, 1, 3, MODE>(a, stages, late > 0 ? (int)blockIdx.x : b, gx, gy, 1, n_req);
+  }
 }
 
 // out[token, head, :] = sum_s 2^(m_s - m) O_s / sum_s 2^(m_s - m) l_s, splits in ascending order.
@@ -1822,6 +1862,30 @@ static int launch_all(AttnArgs a, int n_tokens, int n_req, int max_q_len, int nu
   constexpr bool WIDE = D + DV > 256;
   constexpr int OCC2 = WIDE ? 1 : 2;     // 32 query rows a wave
   constexpr int OCC1 = WIDE ? 2 : 3;     // 16 query rows a wave
+  if constexpr (LDS && DV <= 128 && !WIDE) {
+    // single tokens beside portions: one launch where the portions take 16 query rows a wave whole (see below) and make no more
+    // than about 800 blocks; beyond, three blocks a CU instead of two are worth more to them.  24 heads in 8 groups, two launches / one: 700 rows beside
+    // 4 / 16 / 40 requests of 900 keys 34.3 / 39.4 / 56.0 against 26.2 / 24.8 / 34.3 us, 1,600 rows 60.6 / 69.3 / 89.1 against 55.7 / 63.2 /
+    // 75.6, 2,000 rows 72.4 / 82.2 / 107.5 against 76.8 / 83.6 / 94.6.  More than 256 blocks of single tokens fill the chip alone; the portions
+    // then come first (48 requests of 3,000 keys beside 700 rows 135.5 / 135.4).
+    const int kv_groups = a.n_kv * ((group + 3) / 4), portions = n_req - num_single;
+    const long blocks2 = (long)((n_tokens - num_single + 31) / 32 + (portions - 1)) * kv_groups;
+    if (num_single > 0 && has_multi && !bias && g_attn_tune == 0 && a.page_shift >= 4 && a.page_size >= 512 / D && blocks2 <= 400 &&
+        (a.portion_splits == 1 || a.keep_first > 0)) {
+      constexpr int NB = (D + DV) * 64 > 8192 ? 1 : 2;
+      a.portion_splits = 1;
+      const int tiles = group <= 2 ? 4 / group : 1;
+      if (group <= 2) a.heads_per_block = group;
+      const int gx = (max_q_len + 16 * tiles - 1) / (16 * tiles), gy = group <= 2 ? a.n_kv : kv_groups;
+      const long single = (long)a.n_kv * ((group + 15) / 16) * n_req * a.num_splits, most = (long)gx * gy * portions;
+      if (single + most < 0x7fffffffL) {
+        hipLaunchKernelGGL((attn_both_kernel<D, DV, MODE, NB>), dim3((unsigned)(single + most)), dim3(256), 0, s, a, n_req, (int)single,
+                           single > 256 ? (int)most : 0, gx, gy);
+        if (a.num_splits > 1) launch_combine(a, n_req, DV, s);
+        return 0;
+      }
+    }
+  }
   if (num_single > 0) {
     const dim3 grid(a.n_kv * ((group + 15) / 16), n_req, a.num_splits);
     if constexpr (WITH_BIAS) {

@@ -5,6 +5,7 @@ from types import SimpleNamespace
 import pytest
 import torch
 
+from emu_ops import EmuOps
 from test_kernels_gpu import DEV, _attention_case, _ops
 
 pytestmark = pytest.mark.gpu
@@ -264,3 +265,49 @@ def test_a_step_beside_what_an_attention_brings(kind, n_step, dim, vdim, how):
         results.append((out, state, kk, vv))
     assert not torch.equal(results[0][1], state0)
     assert all(torch.equal(a, c) for a, c in zip(*results))
+
+
+@pytest.mark.parametrize("heads,kv,d,vd,page", [(6, 2, 128, 128, 16), (3, 3, 64, 64, 32), (8, 4, 128, 64, 16), (34, 2, 32, 32, 16), (10, 2, 64, 64, 16)])
+@pytest.mark.parametrize("q_lens,ctx_lens", [([1, 40, 1], [700, 40, 33]), ([2, 1], [2, 1]), ([1] * 70 + [17] + [1] * 3 + [130, 1], [50] * 70 + [400] + [9] * 3 + [131, 2000]),
+                                             ([300, 1, 1, 16], [300, 900, 1100, 64])])
+@pytest.mark.parametrize("mask", [{}, {"window": 37}, {"window": 24, "keep_first": 9}, {"chunk": 48, "sink": True}, {"softcap": 4.0}])
+def test_portions_and_single_tokens_in_one_launch(heads, kv, d, vd, page, q_lens, ctx_lens, mask):
+    """Portions anywhere among single tokens, more requests than a wave has lanes, keys split or not, more and fewer than 256 blocks of single
+    tokens: the portions' rows are bit for bit those of a launch of their own, the single tokens' differ by what the sums of four waves
+    instead of eight move a rounding to bfloat16 (2^-8), and both are what the plain operation gives within that rounding (twice: q k and the result)."""
+    ops = _ops()
+    R, n = len(q_lens), sum(q_lens)
+    g = torch.Generator().manual_seed(n + heads)
+    width = max(-(-c // page) for c in ctx_lens)
+    pages = sum(-(-c // page) for c in ctx_lens)
+    order, bt, at = torch.randperm(pages, generator=g), torch.zeros(R, width, dtype=torch.int32), 0
+    for r, c in enumerate(ctx_lens):
+        used = -(-c // page)
+        bt[r, :used] = order[at: at + used]
+        at += used
+    k = torch.randn(pages, kv, page, d, generator=g).bfloat16()
+    v = torch.randn(pages, kv, vd, page, generator=g).bfloat16()
+    q = torch.randn(n, heads, d, generator=g).bfloat16()
+    cu = torch.tensor([0] + list(torch.tensor(q_lens).cumsum(0)), dtype=torch.int32)
+    cl, tr = torch.tensor(ctx_lens, dtype=torch.int32), torch.repeat_interleave(torch.arange(R, dtype=torch.int32), torch.tensor(q_lens))
+    more = dict(mask)
+    window = more.pop("window", 0)
+    if more.get("sink"):
+        more["sink"] = torch.randn(heads, generator=g)
+    args = (d ** -0.5, window, max(q_lens), max(ctx_lens), q_lens.count(1))
+    dev = {a: b.to(DEV) if torch.is_tensor(b) else b for a, b in more.items()}
+    place = [t.to(DEV) for t in (q, k, v, bt, cu, cl, tr)]
+    got = ops.paged_attention(*place, *args, **dev)
+    lib = ops.library()
+    lib.tp_attention_tune(4)      # (no choice of a kernel's variant, and one launch for each kind)
+    try:
+        apart = ops.paged_attention(*place, *args, **dev)
+    finally:
+        lib.tp_attention_tune(0)
+    single = torch.tensor([q_lens[r] == 1 for r in tr.tolist()])
+    assert torch.equal(got.cpu()[~single], apart.cpu()[~single])
+    want = EmuOps().paged_attention(q, k, v, bt, cu, cl, tr, *args, **more)
+    for a, b in ((got, apart), (got, want)):
+        a, b = a.double().cpu(), b.double().cpu()
+        assert float((a - b)[single].norm() / b[single].norm()) < 2.0 ** -8
+        assert float((a - b).abs().max() / b.abs().max()) < 2.0 ** -6

@@ -686,50 +686,50 @@ constexpr int BNB = 256, NSB = 2;
 constexpr int CLDB = 128 + 4;   // padded row of a quarter (32 rows) of a wave's result tile in LDS, in floats
 constexpr int CLDS = 32 + 4;    // padded row of a strip (32 columns) of a wave's result tile in LDS, in floats
 
-// Operand fragments of a half step (32 of K): eight 16-row tiles of x, NJ (eight or six) of w.  The w fragments
-// are double-buffered, and so are the last two x fragments; x fragments 0..5 are used by one row of MFMAs each,
+// Operand fragments of a half step (32 of K): NI (eight or six) 16-row tiles of x, NJ (eight or six) of w.  The w fragments
+// are double-buffered, and so are the last two x fragments; the other x fragments are used by one row of MFMAs each,
 // so the next half step's takes the register as soon as that row has been issued (the LDS read takes far
 // longer than an MFMA needs to fetch its operands).
-template <int NJ>
+template <int NI, int NJ>
 struct FragsBig {
-  u32x4_t a[6], a6[2], a7[2], b[2][NJ];
+  u32x4_t a[NI - 2], late[2][2], b[2][NJ];
 };
-template <int NJ, int p>
-__device__ inline void tie_frags(FragsBig<NJ>& f) {
+template <int NI, int NJ, int p>
+__device__ inline void tie_frags(FragsBig<NI, NJ>& f) {
   asm volatile("s_waitcnt lgkmcnt(0)"
                : "+v"(f.b[p][0]), "+v"(f.b[p][1]), "+v"(f.b[p][2]), "+v"(f.b[p][3]), "+v"(f.b[p][4]), "+v"(f.b[p][5]),
-                 "+v"(f.a[0]), "+v"(f.a[1]), "+v"(f.a[2]), "+v"(f.a[3]), "+v"(f.a[4]), "+v"(f.a[5]), "+v"(f.a6[p]),
-                 "+v"(f.a7[p]));
+                 "+v"(f.a[0]), "+v"(f.a[1]), "+v"(f.a[2]), "+v"(f.a[3]), "+v"(f.late[0][p]), "+v"(f.late[1][p]));
+  if constexpr (NI == 8) asm volatile("" : "+v"(f.a[4]), "+v"(f.a[5]));
   if constexpr (NJ == 8) asm volatile("" : "+v"(f.b[p][6]), "+v"(f.b[p][7]));
 }
-// load I (0..7 + NJ) of this wave into stage `buf`: 0..7 are x rows, the others w rows; one load covers 8 rows
-template <int I, int NJ>
+// load I (0..NI + NJ - 1) of this wave into stage `buf`: the first NI are x rows, the others w rows; one load covers 8 rows
+template <int I, int NI, int NJ>
 __device__ inline void issue_big(unsigned char* buf, const unsigned char* xk, const unsigned char* wk,
-                                 const unsigned (&voff)[8 + NJ], int wave) {
-  if constexpr (I < 8 + NJ) {
-    const int t = I < 8 ? wave * 8 + I : 32 + wave * NJ + (I - 8);
-    load_lds16(I < 8 ? xk : wk, voff[I], buf + t * 1024);
+                                 const unsigned (&voff)[NI + NJ], int wave) {
+  if constexpr (I < NI + NJ) {
+    const int t = I < NI ? wave * NI + I : 4 * NI + wave * NJ + (I - NI);
+    load_lds16(I < NI ? xk : wk, voff[I], buf + t * 1024);
   }
 }
-template <int NJ>
+template <int NI, int NJ>
 __device__ inline void issue_stage_big(unsigned char* buf, const unsigned char* xk, const unsigned char* wk,
-                                       const unsigned (&voff)[8 + NJ], int wave) {
-  issue_big<0, NJ>(buf, xk, wk, voff, wave); issue_big<1, NJ>(buf, xk, wk, voff, wave); issue_big<2, NJ>(buf, xk, wk, voff, wave);
-  issue_big<3, NJ>(buf, xk, wk, voff, wave); issue_big<4, NJ>(buf, xk, wk, voff, wave); issue_big<5, NJ>(buf, xk, wk, voff, wave);
-  issue_big<6, NJ>(buf, xk, wk, voff, wave); issue_big<7, NJ>(buf, xk, wk, voff, wave); issue_big<8, NJ>(buf, xk, wk, voff, wave);
-  issue_big<9, NJ>(buf, xk, wk, voff, wave); issue_big<10, NJ>(buf, xk, wk, voff, wave); issue_big<11, NJ>(buf, xk, wk, voff, wave);
-  issue_big<12, NJ>(buf, xk, wk, voff, wave); issue_big<13, NJ>(buf, xk, wk, voff, wave); issue_big<14, NJ>(buf, xk, wk, voff, wave);
-  issue_big<15, NJ>(buf, xk, wk, voff, wave);
+                                       const unsigned (&voff)[NI + NJ], int wave) {
+  issue_big<0, NI, NJ>(buf, xk, wk, voff, wave); issue_big<1, NI, NJ>(buf, xk, wk, voff, wave); issue_big<2, NI, NJ>(buf, xk, wk, voff, wave);
+  issue_big<3, NI, NJ>(buf, xk, wk, voff, wave); issue_big<4, NI, NJ>(buf, xk, wk, voff, wave); issue_big<5, NI, NJ>(buf, xk, wk, voff, wave);
+  issue_big<6, NI, NJ>(buf, xk, wk, voff, wave); issue_big<7, NI, NJ>(buf, xk, wk, voff, wave); issue_big<8, NI, NJ>(buf, xk, wk, voff, wave);
+  issue_big<9, NI, NJ>(buf, xk, wk, voff, wave); issue_big<10, NI, NJ>(buf, xk, wk, voff, wave); issue_big<11, NI, NJ>(buf, xk, wk, voff, wave);
+  issue_big<12, NI, NJ>(buf, xk, wk, voff, wave); issue_big<13, NI, NJ>(buf, xk, wk, voff, wave); issue_big<14, NI, NJ>(buf, xk, wk, voff, wave);
+  issue_big<15, NI, NJ>(buf, xk, wk, voff, wave);
 }
-// The 8 x NJ MFMAs of a half step with the fragments of parity P, row by row.  READ: the next half step's
+// The NI x NJ MFMAs of a half step with the fragments of parity P, row by row.  READ: the next half step's
 // fragments are requested between them (w and the last two x fragments into the other set, x fragment i into
 // a[i] after row i).  LOAD: one global load per group of MFMAs.
-template <int P, bool READ, bool LOAD, int NJ>
-__device__ inline void half_step_big(f32x4_t (&acc)[8][NJ], FragsBig<NJ>& f, unsigned aaddr, unsigned baddr, unsigned char* buf,
-                                     const unsigned char* xk, const unsigned char* wk, const unsigned (&voff)[8 + NJ],
+template <int P, bool READ, bool LOAD, int NI, int NJ>
+__device__ inline void half_step_big(f32x4_t (&acc)[NI][NJ], FragsBig<NI, NJ>& f, unsigned aaddr, unsigned baddr, unsigned char* buf,
+                                     const unsigned char* xk, const unsigned char* wk, const unsigned (&voff)[NI + NJ],
                                      int wave) {
 #define SB() __builtin_amdgcn_sched_barrier(0)
-#define AF(I) (I < 6 ? f.a[I < 6 ? I : 0] : (I == 6 ? f.a6[P] : f.a7[P]))
+#define AF(I) (I < NI - 2 ? f.a[I < NI - 2 ? I : 0] : f.late[I == NI - 1][P])
 // (written as assembly with the accumulator tied to an AGPR: left to itself the register allocator keeps
 // part of the accumulator registers in VGPRs and copies them back and forth inside the loop)
 #define M1(I, J) \
@@ -741,13 +741,13 @@ __device__ inline void half_step_big(f32x4_t (&acc)[8][NJ], FragsBig<NJ>& f, uns
 #define RA(I) \
   if (READ) f.a[I] = lds_read16<(I) * 16 * ROWB>(aaddr); \
   SB()
-#define R67()                                                  \
-  if (READ) f.a6[P ^ 1] = lds_read16<6 * 16 * ROWB>(aaddr);    \
-  SB();                                                        \
-  if (READ) f.a7[P ^ 1] = lds_read16<7 * 16 * ROWB>(aaddr);    \
+#define RLATE()                                                             \
+  if (READ) f.late[0][P ^ 1] = lds_read16<(NI - 2) * 16 * ROWB>(aaddr);     \
+  SB();                                                                     \
+  if (READ) f.late[1][P ^ 1] = lds_read16<(NI - 1) * 16 * ROWB>(aaddr);     \
   SB()
 #define LD(G) \
-  if (LOAD) issue_big<G, NJ>(buf, xk, wk, voff, wave); \
+  if (LOAD) issue_big<G, NI, NJ>(buf, xk, wk, voff, wave); \
   SB()
   if constexpr (NJ == 8) {
 #define ROW(I, PRE0, PRE1)                             \
@@ -759,13 +759,17 @@ __device__ inline void half_step_big(f32x4_t (&acc)[8][NJ], FragsBig<NJ>& f, uns
     ROW(1, RB(2); RA(0), RB(3));
     ROW(2, RB(4); RA(1), RB(5));
     ROW(3, RB(6); RA(2), RB(7));
-    ROW(4, RA(3), R67());
-    ROW(5, RA(4), (void)0);
-    ROW(6, RA(5), (void)0);
-    ROW(7, (void)0, (void)0);
+    ROW(4, RA(3), RLATE());
+    if constexpr (NI == 8) {
+      ROW(5, RA(4), (void)0);
+      ROW(6, RA(5), (void)0);
+      ROW(7, (void)0, (void)0);
+    } else {
+      ROW(5, LD(12), LD(13));
+    }
 #undef ROW
   } else {
-    static_assert(NJ == 6 || NJ == 8, "w tiles per wave");
+    static_assert(NJ == 6 && NI == 8, "w tiles per wave");
 #define ROW(I, PRE0, PRE1)                   \
   PRE0;                                      \
   M1(I, 0); M1(I, 1); LD(2 * (I)); M1(I, 2); \
@@ -775,59 +779,62 @@ __device__ inline void half_step_big(f32x4_t (&acc)[8][NJ], FragsBig<NJ>& f, uns
     ROW(1, RB(2); RA(0), RB(3));
     ROW(2, RB(4); RA(1), RB(5));
     ROW(3, RA(2), (void)0);
-    ROW(4, RA(3), R67());
+    ROW(4, RA(3), RLATE());
     ROW(5, RA(4), (void)0);
     ROW(6, RA(5), (void)0);
     ROW(7, (void)0, (void)0);
 #undef ROW
   }
   if (READ) {
-    tie_frags<NJ, (P ^ 1)>(f);
+    tie_frags<NI, NJ, (P ^ 1)>(f);
     SB();
   }
 #undef LD
-#undef R67
+#undef RLATE
 #undef RA
 #undef RB
 #undef M1
 #undef AF
 #undef SB
 }
-template <int NJ>
-__device__ inline void read_all_big(FragsBig<NJ>& f, unsigned aaddr, unsigned baddr) {
+template <int NI, int NJ>
+__device__ inline void read_all_big(FragsBig<NI, NJ>& f, unsigned aaddr, unsigned baddr) {
 #define RB0(J) if constexpr (J < NJ) f.b[0][J < NJ ? J : 0] = lds_read16<(J) * 16 * ROWB>(baddr)
 #define RA0(I) f.a[I] = lds_read16<(I) * 16 * ROWB>(aaddr)
   RB0(0); RB0(1); RB0(2); RB0(3); RB0(4); RB0(5); RB0(6); RB0(7);
-  RA0(0); RA0(1); RA0(2); RA0(3); RA0(4); RA0(5);
-  f.a6[0] = lds_read16<6 * 16 * ROWB>(aaddr);
-  f.a7[0] = lds_read16<7 * 16 * ROWB>(aaddr);
+  RA0(0); RA0(1); RA0(2); RA0(3);
+  if constexpr (NI == 8) {
+    RA0(4); RA0(5);
+  }
+  f.late[0][0] = lds_read16<(NI - 2) * 16 * ROWB>(aaddr);
+  f.late[1][0] = lds_read16<(NI - 1) * 16 * ROWB>(aaddr);
 #undef RB0
 #undef RA0
-  tie_frags<NJ, 0>(f);
+  tie_frags<NI, NJ, 0>(f);
 }
 
 }  // namespace
 
-// No split of K here.  A block tile is 256 rows x 32 NJ columns (NJ = 8: 256, a wave owns 128 x 128; NJ = 6: 192, a
-// wave owns 128 x 96: for an N where that many more tiles make whole rounds of the CUs).  N: the columns of this
-// launch (a multiple of the tile's); ldo as above.
-template <int NJ>
+// No split of K here.  A block tile is 32 NI rows x 32 NJ columns (8, 8: 256 x 256, a wave owns 128 x 128; 8, 6: 256 x 192, a
+// wave owns 128 x 96, and 6, 8: 192 x 256, a wave owns 96 x 128: for an N or M where that many more tiles make whole rounds
+// of the CUs).  N: the columns of this launch (a multiple of the tile's); ldo as above.
+template <int NI, int NJ>
 __global__ __launch_bounds__(256) void gemm_pipe_big_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w,
                                                             void* __restrict__ out, int mode, int M, int N, int K,
                                                             int pm, int ldo, RopeOut rp, int wt) {
-  constexpr int BNT = 32 * NJ, WN = 16 * NJ, STAGE = (BM + BNT) * ROWB, LPWT = 8 + NJ;
+  constexpr int BMT = 32 * NI, BNT = 32 * NJ, WM = 16 * NI, WN = 16 * NJ, STAGE = (BMT + BNT) * ROWB, LPWT = NI + NJ;
   __shared__ __attribute__((aligned(1024))) unsigned char stages[NSB * STAGE];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave >> 1, wn = wave & 1;
   int bm, bn;
   {
-    const int MB = (M + BM - 1) / BM, NB = N / BNT;
+    const int MB = (M + BMT - 1) / BMT, NB = N / BNT;
     if (!tile_of_block(blockIdx.x, MB, NB, pm, bm, bn)) return;
   }
-  const int m0 = bm * BM, n0 = bn * BNT;
-  f32x4_t acc[8][NJ];
+  const int m0 = bm * BMT, n0 = bn * BNT;
+  f32x4_t acc[NI][NJ];
 #pragma unroll
-  for (int i = 0; i < 8; ++i)
+  for (int i = 0; i < NI; ++i)
 #pragma unroll
     for (int j = 0; j < NJ; ++j) acc[i][j] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
   const int KT = K / BK;
@@ -835,16 +842,16 @@ __global__ __launch_bounds__(256) void gemm_pipe_big_kernel(const bf16_t* __rest
   const unsigned lds0 = (unsigned)(size_t)(__attribute__((address_space(3))) const unsigned char*)&stages[0];
   const unsigned off0 = c * ROWB + (((0 * 4 + g) ^ ((c >> 1) & 7)) << 4);
   const unsigned off1 = c * ROWB + (((1 * 4 + g) ^ ((c >> 1) & 7)) << 4);
-  const unsigned arow = wm * 128 * ROWB, brow = (BM + wn * WN) * ROWB;
+  const unsigned arow = wm * WM * ROWB, brow = (BMT + wn * WN) * ROWB;
   unsigned voff[LPWT];
 #pragma unroll
   for (int i = 0; i < LPWT; ++i) {
-    const int row = (i < 8 ? wave * 8 + i : wave * NJ + (i - 8)) * 8 + (lane >> 3);
+    const int row = (i < NI ? wave * NI + i : wave * NJ + (i - NI)) * 8 + (lane >> 3);
     const int chunk = (lane & 7) ^ ((row >> 1) & 7);
-    const int grow = i < 8 ? min(row, M - 1 - m0) : row;   // (every w row of the launch exists)
+    const int grow = i < NI ? min(row, M - 1 - m0) : row;   // (every w row of the launch exists)
     voff[i] = (unsigned)grow * (unsigned)K * 2u + chunk * 16;
-    if (wt && i >= 8) {   // block u of the stage's weights: row group u / 2 of the block tile, first or second 32 of k
-      const int u = wave * NJ + (i - 8);
+    if (wt && i >= NI) {   // block u of the stage's weights: row group u / 2 of the block tile, first or second 32 of k
+      const int u = wave * NJ + (i - NI);
       voff[i] = ((unsigned)(u / 2) * (unsigned)(K / 32) + (u & 1)) * 1024u + lane * 16;
     }
   }
@@ -854,13 +861,13 @@ __global__ __launch_bounds__(256) void gemm_pipe_big_kernel(const bf16_t* __rest
   const unsigned char* wk = (const unsigned char*)w + (size_t)n0 * K * 2;
 #pragma unroll
   for (int p = 0; p < NSB; ++p)
-    if (p < KT) issue_stage_big<NJ>(stages + p * STAGE, xk + p * BK * 2, wk + p * wkstep, voff, wave);
+    if (p < KT) issue_stage_big<NI, NJ>(stages + p * STAGE, xk + p * BK * 2, wk + p * wkstep, voff, wave);
   xk += NSB * BK * 2;
   wk += NSB * wkstep;
-  FragsBig<NJ> f;
+  FragsBig<NI, NJ> f;
   if (KT > 1) WAIT_VM(LPWT); else WAIT_VM(0);
   __builtin_amdgcn_s_barrier();
-  read_all_big<NJ>(f, lds0 + arow + off0, lds0 + brow + boff0);
+  read_all_big<NI, NJ>(f, lds0 + arow + off0, lds0 + brow + boff0);
   // Tile kt: the first half step multiplies the fragments of its first 32 of K and reads those of the second;
   // then tile kt + 1 must have landed for every wave (barrier), which also means that every wave is done
   // reading tile kt's stage: the second half step refills it with tile kt + 2 while it multiplies and reads
@@ -868,46 +875,46 @@ __global__ __launch_bounds__(256) void gemm_pipe_big_kernel(const bf16_t* __rest
   int st = 0, kt = 0;
   for (; kt + NSB < KT; ++kt) {
     const unsigned cur = lds0 + st * STAGE, nxt = lds0 + (st ^ 1) * STAGE;
-    half_step_big<0, true, false, NJ>(acc, f, cur + arow + off1, cur + brow + boff1, nullptr, nullptr, nullptr, voff, wave);
+    half_step_big<0, true, false, NI, NJ>(acc, f, cur + arow + off1, cur + brow + boff1, nullptr, nullptr, nullptr, voff, wave);
     WAIT_VM(0);
     __builtin_amdgcn_s_barrier();
-    half_step_big<1, true, true, NJ>(acc, f, nxt + arow + off0, nxt + brow + boff0, stages + st * STAGE, xk, wk, voff, wave);
+    half_step_big<1, true, true, NI, NJ>(acc, f, nxt + arow + off0, nxt + brow + boff0, stages + st * STAGE, xk, wk, voff, wave);
     xk += BK * 2;
     wk += wkstep;
     st ^= 1;
   }
   for (; kt + 1 < KT; ++kt) {  // nothing left to load
     const unsigned cur = lds0 + st * STAGE, nxt = lds0 + (st ^ 1) * STAGE;
-    half_step_big<0, true, false, NJ>(acc, f, cur + arow + off1, cur + brow + boff1, nullptr, nullptr, nullptr, voff, wave);
+    half_step_big<0, true, false, NI, NJ>(acc, f, cur + arow + off1, cur + brow + boff1, nullptr, nullptr, nullptr, voff, wave);
     WAIT_VM(0);
     __builtin_amdgcn_s_barrier();
-    half_step_big<1, true, false, NJ>(acc, f, nxt + arow + off0, nxt + brow + boff0, nullptr, nullptr, nullptr, voff, wave);
+    half_step_big<1, true, false, NI, NJ>(acc, f, nxt + arow + off0, nxt + brow + boff0, nullptr, nullptr, nullptr, voff, wave);
     st ^= 1;
   }
   {
     const unsigned cur = lds0 + st * STAGE;
-    half_step_big<0, true, false, NJ>(acc, f, cur + arow + off1, cur + brow + boff1, nullptr, nullptr, nullptr, voff, wave);
-    half_step_big<1, false, false, NJ>(acc, f, 0, 0, nullptr, nullptr, nullptr, voff, wave);
+    half_step_big<0, true, false, NI, NJ>(acc, f, cur + arow + off1, cur + brow + boff1, nullptr, nullptr, nullptr, voff, wave);
+    half_step_big<1, false, false, NI, NJ>(acc, f, 0, 0, nullptr, nullptr, nullptr, voff, wave);
   }
   // The MFMAs are assembly, so the compiler does not know that their results take time: wait out the last ones
   // (eight passes of the matrix core and the write-back).  The wait is tied to their accumulators, or the
   // compiler may read them (a register copy on the way into the epilogue) before it.
   asm volatile("s_nop 15\n\ts_nop 15\n\ts_nop 15\n\ts_nop 15\n\ts_nop 15\n\ts_nop 15\n\ts_nop 15\n\ts_nop 15"
-               : "+a"(acc[7][0]), "+a"(acc[7][1]), "+a"(acc[7][2]), "+a"(acc[7][3]), "+a"(acc[7][4]), "+a"(acc[7][5])
+               : "+a"(acc[NI - 1][0]), "+a"(acc[NI - 1][1]), "+a"(acc[NI - 1][2]), "+a"(acc[NI - 1][3]), "+a"(acc[NI - 1][4]), "+a"(acc[NI - 1][5])
                :
                : "memory");
-  if constexpr (NJ == 8) asm volatile("" : "+a"(acc[7][6]), "+a"(acc[7][7]));
+  if constexpr (NJ == 8) asm volatile("" : "+a"(acc[NI - 1][6]), "+a"(acc[NI - 1][7]));
   // (and every other accumulator passes through an ordered statement after it)
 #pragma unroll
-  for (int i = 0; i < 7; ++i) {
+  for (int i = 0; i < NI - 1; ++i) {
     asm volatile("" : "+a"(acc[i][0]), "+a"(acc[i][1]), "+a"(acc[i][2]), "+a"(acc[i][3]), "+a"(acc[i][4]), "+a"(acc[i][5]));
     if constexpr (NJ == 8) asm volatile("" : "+a"(acc[i][6]), "+a"(acc[i][7]));
   }
 
   __syncthreads();
-  const int mw = m0 + wm * 128, nw = n0 + wn * WN;
+  const int mw = m0 + wm * WM, nw = n0 + wn * WN;
   if constexpr (NJ == 8) {
-  // ---- the result leaves through LDS, 32 rows of the wave's 128 x 128 at a time ---------------------------
+  // ---- the result leaves through LDS, 32 rows of the wave's 128 (or 96) x 128 at a time ---------------------------
   float* ct = (float*)stages + wave * (32 * CLDB);
   // (written out four times: were the loop over the quarters not unrolled, the accumulators would be indexed at
   // run time and live in scratch memory)
@@ -916,7 +923,7 @@ __global__ __launch_bounds__(256) void gemm_pipe_big_kernel(const bf16_t* __rest
     RopeFetch<32, 128> fetched;   /* the rotating epilogue's loads travel while the quarter goes to LDS */       \
     if (mode == OUT_ROPE) rope_fetch(fetched, lane, mw + (Q) * 32, nw, rp, M);                                  \
     _Pragma("unroll") for (int i = 0; i < 2; ++i) _Pragma("unroll") for (int j = 0; j < 8; ++j)                 \
-        _Pragma("unroll") for (int r = 0; r < 4; ++r) ct[(i * 16 + g * 4 + r) * CLDB + j * 16 + c] = acc[(Q) * 2 + i][j][r]; \
+        _Pragma("unroll") for (int r = 0; r < 4; ++r) ct[(i * 16 + g * 4 + r) * CLDB + j * 16 + c] = acc[(Q) * 2 + i < NI ? (Q) * 2 + i : 0][j][r]; \
     /* this wave's LDS writes before its reads, and the reverse below */                                        \
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");                                                          \
     if (mode == OUT_ROPE)                                                                                       \
@@ -928,7 +935,7 @@ __global__ __launch_bounds__(256) void gemm_pipe_big_kernel(const bf16_t* __rest
   QUARTER(0)
   QUARTER(1)
   QUARTER(2)
-  QUARTER(3)
+  if constexpr (NI == 8) QUARTER(3)
 #undef QUARTER
   } else {
   // ---- the wave's 128 x 96 leaves as a strip of 64 columns (two halves of 64 rows) and one of 32.  A strip
@@ -1519,7 +1526,7 @@ extern "C" int tp_moe_linear(const void* x, const void* w, int w_tiled, void* ou
 
 // Returns 0 when launched, -1 when the sizes are not this kernel's.  `scratch` (optional) is room for
 // float32 partial sums: with few result tiles K is split over blocks until there is work for every CU.
-int g_pipe_big = 0;   // tuning: 1 = 256 x 256 tiles for every whole block of 256 columns, 2 = never; 3 = 256 x 192 wherever N allows, 4 = never
+int g_pipe_big = 0;   // tuning: 1 = 256 x 256 tiles for every whole block of 256 columns, 2 = never; 3 = 256 x 192 wherever N allows, 4 = never; 5 = 192 x 256 wherever N allows
 int tp_linear_pipe(const bf16_t* x, const bf16_t* w, int w_tiled, void* out, int mode, int M, int N, int K, float* scratch,
                    size_t scratch_floats, int tune_splits, const RopeOut* rope, int defer, int* splits_out, GateAct gate,
                    hipStream_t s) {
@@ -1560,6 +1567,7 @@ int tp_linear_pipe(const bf16_t* x, const bf16_t* w, int w_tiled, void* out, int
   // needs the fewest rounds when a big tile is priced at 1.72 small ones (measured: 113 against 65 us at
   // K = 4096).
   int nb_big = 0;
+  bool low = false;    // tiles of 192 rows
   // (with the rotating epilogue a wave's 128 columns of a big tile have to lie inside one of q, k and v: heads
   // of a multiple of 128; the strips of the 192-column tile are ordered for heads of 128)
   const bool big_ok = rope == nullptr || rope->head_dim % 128 == 0;
@@ -1577,6 +1585,17 @@ int tp_linear_pipe(const bf16_t* x, const bf16_t* w, int w_tiled, void* out, int
         nb_big = (int)cand;
       }
     if (g_pipe_big == 1) nb_big = (int)NB2;
+    // Tiles of 192 x 256 for all columns, priced at 1.5 small tiles: where they save a quarter of each round's tile (731 rows of 16,384 x
+    // 3,072 gated are 256 of them in one round instead of 192 of 256 x 256 on three quarters of the CUs: 79.8 -> 75.5 us, 560 rows 77.0 ->
+    // 67.6; 2,048 rows of 5,120 x 3,072 69.0 -> 63.3; at an even number of rounds they lose: 731 rows of 28,672 x 4,096 157 -> 165).
+    const int MB192 = (M + 191) / 192;
+    if (N % BNB == 0 && g_pipe_big != 1) {
+      const double cost = 1.5 * (double)(((long)MB192 * (N / BNB) + 255) / 256);
+      if (cost < best - 1e-9 || g_pipe_big == 5) {
+        best = cost;
+        low = true;
+      }
+    }
     // Tiles of 256 x 192 where N is a multiple of 192 and that many more tiles fill whole rounds: priced at 1.35
     // small tiles (the q/k/v projection of 2,048 rows, N = 6,144: 256 tiles in one round instead of 192 of 256 x 256
     // on three quarters of the CUs, 109 -> 8x us).
@@ -1584,15 +1603,22 @@ int tp_linear_pipe(const bf16_t* x, const bf16_t* w, int w_tiled, void* out, int
       const long t192 = (long)MB * (N / 192);
       if (1.35 * (double)((t192 + 255) / 256) < best - 1e-9 || g_pipe_big == 3) {
         const long blocks3 = blocks_for(N / 192);
-        hipLaunchKernelGGL(gemm_pipe_big_kernel<6>, dim3((unsigned)blocks3), dim3(256), 0, s, x, w, out, mode, M, N, K, pm, ldo,
+        hipLaunchKernelGGL((gemm_pipe_big_kernel<8, 6>), dim3((unsigned)blocks3), dim3(256), 0, s, x, w, out, mode, M, N, K, pm, ldo,
                            rp, w_tiled);
         return 0;
       }
     }
   }
+  if (low) {
+    const int MB192 = (M + 191) / 192, strips192 = (MB192 + 7) / 8;
+    const long blocks4 = 8L * (((long)MB192 * (N / BNB) + 7) / 8);
+    hipLaunchKernelGGL((gemm_pipe_big_kernel<6, 8>), dim3((unsigned)blocks4), dim3(256), 0, s, x, w, out, mode, M, N, K,
+                       (MB192 + strips192 - 1) / strips192, ldo, rp, w_tiled);
+    return 0;
+  }
   if (nb_big > 0) {
     const long blocks2 = blocks_for(nb_big);
-    hipLaunchKernelGGL(gemm_pipe_big_kernel<8>, dim3((unsigned)blocks2), dim3(256), 0, s, x, w, out, mode, M, nb_big * BNB, K,
+    hipLaunchKernelGGL((gemm_pipe_big_kernel<8, 8>), dim3((unsigned)blocks2), dim3(256), 0, s, x, w, out, mode, M, nb_big * BNB, K,
                        pm, ldo, rp, w_tiled);
     const int n_done = nb_big * BNB;
     if (n_done == N) return 0;

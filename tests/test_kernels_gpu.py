@@ -545,6 +545,46 @@ def test_linear_big_tiles(m, n, k):
             lib.tp_linear_tune_tile(0)
 
 
+@pytest.mark.parametrize("m,heads,kv,k", [(191, 4, 2, 64), (192, 6, 1, 128), (193, 12, 2, 192), (577, 12, 4, 320), (1153, 14, 9, 256)])
+def test_linear_tiles_of_192_rows(m, heads, kv, k):
+    """192 x 256 tiles asked for, and the choice that the library makes by itself, at rows that fill no whole tile: the bits of the 256 x 128
+    tiles (every sum runs over K in ascending order) in every output mode, row-major and tiled weights, and through the rotating epilogue."""
+    ops = _ops()
+    lib = ops.library()
+    from tempura_amd.parts.rope import rotary_inv_freq
+    d, page, n = 128, 16, (heads + 2 * kv) * 128
+    assert n % 256 == 0
+    g = torch.Generator().manual_seed(m)
+    x = torch.randn(m, k, generator=g).to(torch.bfloat16).to(DEV)
+    w = (torch.randn(n, k, generator=g) * 0.1).to(torch.bfloat16).to(DEV)
+    res = torch.randn(m, n, generator=g).to(DEV)
+    pages = 3 + -(-m // page)
+    slots = torch.randperm(pages * page, generator=g)[:m].to(torch.int32).to(DEV)
+    pos = torch.arange(m, dtype=torch.int32, device=DEV)
+    inv = rotary_inv_freq(d, 500000.0, None, d).to(DEV)
+    table = ops.rope_table(pos, inv, d, 1.0)
+
+    def every(wv):
+        kc, vc = torch.zeros(pages, kv, page, d, dtype=torch.bfloat16, device=DEV), torch.zeros(pages, kv, d, page, dtype=torch.bfloat16, device=DEV)
+        out = [ops.linear(x, wv, torch.float32), ops.linear(x, wv, torch.bfloat16), ops.linear(x, wv, torch.float32, residual=res.clone()),
+               ops.linear_swiglu(x, wv), *ops.linear_relu2(x, wv, n // 2)]
+        if ops.linear_rope_ok(m, n, k, d, d, page, torch.bfloat16, torch.bfloat16):
+            out += [ops.linear_rope_kv(x, wv, pos, slots, inv, d, 1.0, heads, kv, d, kc, vc, table), kc, vc]
+        return out
+
+    got = {}
+    for mode in (6, 9, 0):
+        lib.tp_linear_tune_tile(mode)
+        lib.tp_linear_tune_mid_tile(2)
+        try:
+            got[mode] = every(w) + every(ops.tile_weight(w))
+        finally:
+            lib.tp_linear_tune_tile(0)
+            lib.tp_linear_tune_mid_tile(0)
+    for mode in (9, 0):
+        assert all(torch.equal(a, b) for a, b in zip(got[mode], got[6])), mode
+
+
 @pytest.mark.parametrize("m,hidden,kp,nc", [(1, 64, 32, 48), (8, 4096, 4096, 6144), (16, 160, 96, 272), (5, 4096, 14336, 1024),
                                              (3, 96, 2048, 40)])
 def test_linear_split_norm(m, hidden, kp, nc):

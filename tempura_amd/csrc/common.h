@@ -191,6 +191,27 @@ __device__ inline float block_sum(float v, float* scratch) {
   return t;
 }
 
+// The same for a block of T threads (64, or a multiple of 256) whose `scratch` (T / 64 floats, aligned to 16 bytes) no earlier sum has used: one barrier, and the
+// waves' sums in 16-byte reads side by side (sixteen dependent reads one after the other take longer than the barrier).
+template <int T>
+__device__ inline float block_sum_once(float v, float* scratch) {
+  static_assert(T == TP_WAVE || T % (4 * TP_WAVE) == 0, "one wave, or whole 16-byte pieces");
+  v = wave_sum(v);
+  if constexpr (T == TP_WAVE) return v;
+  if (threadIdx.x % TP_WAVE == 0) scratch[threadIdx.x / TP_WAVE] = v;
+  __syncthreads();
+  float4 t = *(const float4*)scratch;
+#pragma unroll
+  for (int i = 1; i < T / (4 * TP_WAVE); ++i) {
+    const float4 u = ((const float4*)scratch)[i];
+    t.x += u.x;
+    t.y += u.y;
+    t.z += u.z;
+    t.w += u.w;
+  }
+  return (t.x + t.y) + (t.z + t.w);
+}
+
 __device__ inline float block_max(float v, float* scratch) {
   const int lane = threadIdx.x % TP_WAVE, wave = threadIdx.x / TP_WAVE;
   const int nwaves = (blockDim.x + TP_WAVE - 1) / TP_WAVE;

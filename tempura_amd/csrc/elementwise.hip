@@ -46,9 +46,38 @@ extern "C" int tp_embed(const int* tokens, const void* table, int table_dt, floa
 
 // ---- RMSNorm ---------------------------------------------------------------------
 // y = x * (1 / sqrt(mean(x^2) + eps)) * w, all in float32; one block per output row.
-// `rows` (optional) picks the input row of each output row.  The row is kept in registers
-// between the two passes when it fits (hidden <= 4 * VEC_ITEMS * threads).
-#define RMS_ITEMS 4
+// `rows` (optional) picks the input row of each output row.
+// A thread keeps NV pieces of four; the norm's weight is requested with the row.
+template <typename TO, int T, int NV>
+__global__ __launch_bounds__(T) void rmsnorm_reg_kernel(const float* __restrict__ x, const float* __restrict__ w,
+                                                           const int* __restrict__ rows, TO* __restrict__ out, int hidden, float eps) {
+  __shared__ __attribute__((aligned(16))) float scratch[T / TP_WAVE];
+  const int r = blockIdx.x;
+  const float* xr = x + (size_t)(rows ? rows[r] : r) * hidden;
+  TO* o = out + (size_t)r * hidden;
+  float4 v[NV], wv[NV];
+#pragma unroll
+  for (int i = 0; i < NV; ++i) {
+    const int j = (threadIdx.x + i * T) * 4;
+    if (j < hidden) {
+      v[i] = *(const float4*)(xr + j);
+      wv[i] = *(const float4*)(w + j);
+    }
+  }
+  float ss = 0.f;
+#pragma unroll
+  for (int i = 0; i < NV; ++i)
+    if ((threadIdx.x + i * T) * 4 < hidden) ss += v[i].x * v[i].x + v[i].y * v[i].y + v[i].z * v[i].z + v[i].w * v[i].w;
+  ss = block_sum_once<T>(ss, scratch);
+  const float scale = 1.0f / sqrtf(ss / (float)hidden + eps);
+#pragma unroll
+  for (int i = 0; i < NV; ++i) {
+    const int j = (threadIdx.x + i * T) * 4;
+    if (j < hidden) from_float4(o + j, v[i].x * scale * wv[i].x, v[i].y * scale * wv[i].y, v[i].z * scale * wv[i].z, v[i].w * scale * wv[i].w);
+  }
+}
+
+// Rows of no whole 16-byte pieces, and very long ones.
 template <typename TO>
 __global__ void rmsnorm_kernel(const float* __restrict__ x, const float* __restrict__ w,
                                const int* __restrict__ rows, TO* __restrict__ out, int hidden, float eps) {
@@ -56,30 +85,6 @@ __global__ void rmsnorm_kernel(const float* __restrict__ x, const float* __restr
   const int r = blockIdx.x;
   const float* xr = x + (size_t)(rows ? rows[r] : r) * hidden;
   TO* o = out + (size_t)r * hidden;
-  const bool vec = (hidden % 4 == 0) && hidden <= 4 * RMS_ITEMS * (int)blockDim.x;
-  if (vec) {
-    float4 v[RMS_ITEMS];
-    float ss = 0.f;
-#pragma unroll
-    for (int i = 0; i < RMS_ITEMS; ++i) {
-      const int j = (threadIdx.x + i * blockDim.x) * 4;
-      if (j < hidden) {
-        v[i] = *(const float4*)(xr + j);
-        ss += v[i].x * v[i].x + v[i].y * v[i].y + v[i].z * v[i].z + v[i].w * v[i].w;
-      }
-    }
-    ss = block_sum(ss, scratch);
-    const float scale = 1.0f / sqrtf(ss / (float)hidden + eps);
-#pragma unroll
-    for (int i = 0; i < RMS_ITEMS; ++i) {
-      const int j = (threadIdx.x + i * blockDim.x) * 4;
-      if (j < hidden) {
-        const float4 wv = *(const float4*)(w + j);
-        from_float4(o + j, v[i].x * scale * wv.x, v[i].y * scale * wv.y, v[i].z * scale * wv.z, v[i].w * scale * wv.w);
-      }
-    }
-    return;
-  }
   float ss = 0.f;
   for (int j = threadIdx.x; j < hidden; j += blockDim.x) {
     const float v = xr[j];
@@ -90,17 +95,31 @@ __global__ void rmsnorm_kernel(const float* __restrict__ x, const float* __restr
   for (int j = threadIdx.x; j < hidden; j += blockDim.x) from_float(o + j, xr[j] * scale * w[j]);
 }
 
+template <typename TO>
+static void launch_rmsnorm(const float* x, const float* w, const int* rows, void* out, int n_out, int hidden, float eps, hipStream_t s) {
+  if (hidden % 4 == 0 && hidden <= 16384 && (((uintptr_t)x | (uintptr_t)w | (uintptr_t)out) & 15) == 0) {
+#define RMS(T_, NV_) hipLaunchKernelGGL((rmsnorm_reg_kernel<TO, T_, NV_>), dim3(n_out), dim3(T_), 0, s, x, w, rows, (TO*)out, hidden, eps)
+    if (hidden <= 1024) RMS(256, 1);
+    else if (hidden <= 2048) RMS(512, 1);
+    else if (hidden <= 4096) RMS(512, 2);
+    else if (hidden <= 8192) RMS(1024, 2);
+    else RMS(1024, 4);
+#undef RMS
+    return;
+  }
+  const int threads = hidden >= 8192 ? 1024 : (hidden >= 1024 ? 256 : 64);
+  hipLaunchKernelGGL(rmsnorm_kernel<TO>, dim3(n_out), dim3(threads), 0, s, x, w, rows, (TO*)out, hidden, eps);
+}
+
 extern "C" int tp_rmsnorm(const float* x, const float* w, const int* rows, void* out, int out_dt,
                           int n_out, int hidden, float eps, hipStream_t s) {
   TP_REQUIRE(n_out >= 0 && hidden > 0, "rmsnorm: bad sizes");
   if (n_out == 0) return 0;
-  const int threads = hidden >= 8192 ? 1024 : (hidden >= 1024 ? 256 : 64);
+  TP_REQUIRE(out_dt == TP_F32 || out_dt == TP_BF16, "rmsnorm: unknown dtype %d", out_dt);
   if (out_dt == TP_F32)
-    hipLaunchKernelGGL(rmsnorm_kernel<float>, dim3(n_out), dim3(threads), 0, s, x, w, rows, (float*)out, hidden, eps);
-  else if (out_dt == TP_BF16)
-    hipLaunchKernelGGL(rmsnorm_kernel<bf16_t>, dim3(n_out), dim3(threads), 0, s, x, w, rows, (bf16_t*)out, hidden, eps);
+    launch_rmsnorm<float>(x, w, rows, out, n_out, hidden, eps, s);
   else
-    TP_REQUIRE(false, "rmsnorm: unknown dtype %d", out_dt);
+    launch_rmsnorm<bf16_t>(x, w, rows, out, n_out, hidden, eps, s);
   TP_CHECK_LAUNCH("rmsnorm");
   return 0;
 }

@@ -621,59 +621,72 @@ __global__ void gemm_splitk_reduce_kernel(const float* __restrict__ partial, voi
 // writes the root-mean-square norm of the updated rows: out = h / sqrt(mean(h^2) + eps) * w.  One block
 // per row; takes the place of the reduction kernel and the norm kernel that would follow it.
 // Each thread owns four neighbouring columns (N % 4 == 0); all its loads are issued before the first sum.
-template <typename TO>
-__global__ __launch_bounds__(1024) void splitk_add_rmsnorm_kernel(const float* __restrict__ partial, int splits,
+// SP: the most splits (2, 4 or 16); T: threads; NV: groups of four columns a thread (N <= 4 T NV).
+template <typename TO, int SP, int T, int NV>
+__global__ __launch_bounds__(T) void splitk_add_rmsnorm_kernel(const float* __restrict__ partial, int splits,
                                                                    float* __restrict__ h, const float* __restrict__ w,
                                                                    float eps, TO* __restrict__ out, int M, int N) {
-  __shared__ float red[32];
+  __shared__ __attribute__((aligned(16))) float red[T / TP_WAVE];
   const int m = blockIdx.x;
   const size_t total = (size_t)M * N;
   float* hr = h + (size_t)m * N;
-  constexpr int MAXC = 4;                       // column groups per thread: N <= 4 * 1024 * MAXC
-  f32x4_t acc[MAXC];
+  f32x4_t acc[NV], wv[NV];
   float ss = 0.f;
 #pragma unroll
-  for (int i = 0; i < MAXC; ++i) {
-    const int n = (threadIdx.x + i * 1024) * 4;
-    acc[i] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+  for (int i = 0; i < NV; ++i) {
+    const int n = (threadIdx.x + i * T) * 4;
     if (n < N) {
-      f32x4_t p[16];
+      const float* pr = partial + (size_t)m * N + n;
+      f32x4_t p[SP];
+      p[0] = *(const f32x4_t*)pr;
 #pragma unroll
-      for (int s = 0; s < 16; ++s)
-        if (s < splits) p[s] = *(const f32x4_t*)(partial + (size_t)s * total + (size_t)m * N + n);
+      for (int s = 1; s < SP; ++s)
+        if (s < splits) p[s] = *(const f32x4_t*)(pr + (size_t)s * total);
       const f32x4_t base = *(const f32x4_t*)(hr + n);
+      wv[i] = *(const f32x4_t*)(w + n);
       f32x4_t add = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+      add += p[0];
 #pragma unroll
-      for (int s = 0; s < 16; ++s)
+      for (int s = 1; s < SP; ++s)
         if (s < splits) add += p[s];
       acc[i] = base + add;
       *(f32x4_t*)(hr + n) = acc[i];
       ss += acc[i][0] * acc[i][0] + acc[i][1] * acc[i][1] + acc[i][2] * acc[i][2] + acc[i][3] * acc[i][3];
     }
   }
-  ss = block_sum(ss, red);
+  ss = block_sum_once<T>(ss, red);
   const float scale = rsqrtf(ss / (float)N + eps);
 #pragma unroll
-  for (int i = 0; i < MAXC; ++i) {
-    const int n = (threadIdx.x + i * 1024) * 4;
-    if (n < N) {
-      const f32x4_t wv = *(const f32x4_t*)(w + n);
-#pragma unroll
-      for (int e = 0; e < 4; ++e) from_float(out + (size_t)m * N + n + e, acc[i][e] * scale * wv[e]);
-    }
+  for (int i = 0; i < NV; ++i) {
+    const int n = (threadIdx.x + i * T) * 4;
+    if (n < N)
+      from_float4(out + (size_t)m * N + n, acc[i][0] * scale * wv[i][0], acc[i][1] * scale * wv[i][1], acc[i][2] * scale * wv[i][2],
+                  acc[i][3] * scale * wv[i][3]);
   }
+}
+
+template <typename TO>
+static void launch_splitk_add_rmsnorm(const float* partial, int splits, float* h, const float* w, float eps, void* out, int M, int N, hipStream_t s) {
+#define SKN(SP_, T_, NV_) hipLaunchKernelGGL((splitk_add_rmsnorm_kernel<TO, SP_, T_, NV_>), dim3(M), dim3(T_), 0, s, partial, splits, h, w, eps, (TO*)out, M, N)
+  if (N > 8192) SKN(16, 1024, 4);
+  else if (N > 4096) SKN(16, 1024, 2);
+  else if (N > 2048 && splits <= 2) SKN(2, 1024, 1);
+  else if (N > 2048 && splits <= 4) SKN(4, 1024, 1);
+  else if (N > 2048) SKN(16, 1024, 1);
+  else if (splits <= 4) SKN(4, 512, 1);
+  else SKN(16, 512, 1);
+#undef SKN
 }
 
 extern "C" int tp_splitk_add_rmsnorm(const float* partial, int splits, float* h, const float* w, float eps, void* out,
                                      int out_dt, int M, int N, hipStream_t s) {
   TP_REQUIRE(M > 0 && N > 0 && splits >= 1 && splits <= 16, "splitk_add_rmsnorm: bad sizes");
   TP_REQUIRE(N % 4 == 0 && N <= 16384, "splitk_add_rmsnorm: width %d must be a multiple of 4, at most 16384", N);
+  TP_REQUIRE(out_dt == TP_F32 || out_dt == TP_BF16, "splitk_add_rmsnorm: unknown dtype %d", out_dt);
   if (out_dt == TP_BF16)
-    hipLaunchKernelGGL(splitk_add_rmsnorm_kernel<bf16_t>, dim3(M), dim3(1024), 0, s, partial, splits, h, w, eps, (bf16_t*)out, M, N);
-  else if (out_dt == TP_F32)
-    hipLaunchKernelGGL(splitk_add_rmsnorm_kernel<float>, dim3(M), dim3(1024), 0, s, partial, splits, h, w, eps, (float*)out, M, N);
+    launch_splitk_add_rmsnorm<bf16_t>(partial, splits, h, w, eps, out, M, N, s);
   else
-    TP_REQUIRE(false, "splitk_add_rmsnorm: unknown dtype %d", out_dt);
+    launch_splitk_add_rmsnorm<float>(partial, splits, h, w, eps, out, M, N, s);
   TP_CHECK_LAUNCH("splitk_add_rmsnorm");
   return 0;
 }

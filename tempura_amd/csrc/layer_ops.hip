@@ -211,78 +211,76 @@ __global__ __launch_bounds__(256) void norm_add_kernel(float* __restrict__ h, co
 // The same with the row in registers: every value is read once, sixteen bytes a load, all loads of a pass in flight
 // together (width a multiple of four, at most 256 * 4 * NV).  The sums are formed in the generic kernel's order of
 // a thread's own elements only where the widths agree; a row's result never depends on other rows either way.
-template <typename TO, int NV, bool GATE>
-__global__ __launch_bounds__(256) void norm_add_reg_kernel(float* __restrict__ h, const float* __restrict__ y,
+template <typename TO, int T, int NV, bool GATE>
+__global__ __launch_bounds__(T) void norm_add_reg_kernel(float* __restrict__ h, const float* __restrict__ y,
                                                            const float* __restrict__ w, float eps,
                                                            const float* __restrict__ w_next, float eps_next,
                                                            TO* __restrict__ x, int width, InputGate gate, int normed, int blocked, int parts) {
-  __shared__ float scratch[32];
+  __shared__ __attribute__((aligned(16))) float scratch[2][T / TP_WAVE];
   const size_t base = (size_t)blockIdx.x * width;
   const int w4 = width / 4;
-  float4 yv[NV], hv[NV], wv[NV];
+  const size_t part = (size_t)gridDim.x * width;
+  const float* gr = GATE ? gate.rows + (size_t)blockIdx.x * gate.stride + gate.col0 : nullptr;
+  float4 yv[NV], y1[NV], y2[NV], y3[NV], hv[NV], wv[NV], gv[GATE ? NV : 1], bv[GATE ? NV : 1], nv[NV];
 #pragma unroll
   for (int k = 0; k < NV; ++k) {
-    const int c = k * 256 + threadIdx.x;
+    const int c = k * T + threadIdx.x;
     if (c < w4) {
-      yv[k] = *(const float4*)(y + base + 4 * c);
-      hv[k] = *(const float4*)(h + base + 4 * c);
-      wv[k] = *(const float4*)(w + 4 * c);
-    }
-  }
-  // (parts > 1: y is that many partial sums of a product, added in ascending order)
-  for (int p = 1; p < parts; ++p) {
-    const float* yp = y + (size_t)p * gridDim.x * width + base;
-    float4 more[NV];
-#pragma unroll
-    for (int k = 0; k < NV; ++k)
-      if (k * 256 + threadIdx.x < w4) more[k] = *(const float4*)(yp + 4 * (k * 256 + threadIdx.x));
-#pragma unroll
-    for (int k = 0; k < NV; ++k)
-      if (k * 256 + threadIdx.x < w4) {
-        yv[k].x += more[k].x;
-        yv[k].y += more[k].y;
-        yv[k].z += more[k].z;
-        yv[k].w += more[k].w;
-      }
-  }
-  if constexpr (GATE) {
-    const float* gr = gate.rows + (size_t)blockIdx.x * gate.stride + gate.col0;
-    float4 gv[NV], bv[NV];
-#pragma unroll
-    for (int k = 0; k < NV; ++k) {
-      const int c = k * 256 + threadIdx.x;
-      if (c < w4) {
+      const float* yp = y + base + 4 * c;
+      yv[k] = *(const float4*)yp;
+      if (parts > 1) y1[k] = *(const float4*)(yp + part);
+      if (parts > 2) y2[k] = *(const float4*)(yp + 2 * part);
+      if (parts > 3) y3[k] = *(const float4*)(yp + 3 * part);
+      if constexpr (GATE) {
         gv[k] = *(const float4*)(gr + 4 * c);
         bv[k] = gate.bias != nullptr ? *(const float4*)(gate.bias + 4 * c) : make_float4(0.f, 0.f, 0.f, 0.f);
       }
+      hv[k] = *(const float4*)(h + base + 4 * c);
+      wv[k] = *(const float4*)(w + 4 * c);
+      if (w_next != nullptr) nv[k] = *(const float4*)(w_next + 4 * c);
     }
+  }
+  // (parts > 1: y is that many partial sums of a product, added in ascending order)
+  auto add = [](float4& a, const float4& b) {
+    a.x += b.x;
+    a.y += b.y;
+    a.z += b.z;
+    a.w += b.w;
+  };
 #pragma unroll
-    for (int k = 0; k < NV; ++k)
-      if (k * 256 + threadIdx.x < w4) {
+  for (int k = 0; k < NV; ++k) {
+    const int c = k * T + threadIdx.x;
+    if (c < w4) {
+      if (parts > 1) add(yv[k], y1[k]);
+      if (parts > 2) add(yv[k], y2[k]);
+      if (parts > 3) add(yv[k], y3[k]);
+      for (int p = 4; p < parts; ++p) add(yv[k], *(const float4*)(y + p * part + base + 4 * c));
+      if constexpr (GATE) {
         yv[k].x *= l_sigmoid(gv[k].x + bv[k].x);
         yv[k].y *= l_sigmoid(gv[k].y + bv[k].y);
         yv[k].z *= l_sigmoid(gv[k].z + bv[k].z);
         yv[k].w *= l_sigmoid(gv[k].w + bv[k].w);
       }
+    }
   }
   float rstd = 1.0f;
   if (normed) {
     float ss = 0.f;
 #pragma unroll
     for (int k = 0; k < NV; ++k)
-      if (k * 256 + threadIdx.x < w4) {
+      if (k * T + threadIdx.x < w4) {
         ss = fmaf(yv[k].x, yv[k].x, ss);
         ss = fmaf(yv[k].y, yv[k].y, ss);
         ss = fmaf(yv[k].z, yv[k].z, ss);
         ss = fmaf(yv[k].w, yv[k].w, ss);
       }
-    ss = block_sum(ss, scratch);
+    ss = block_sum_once<T>(ss, scratch[0]);
     rstd = 1.0f / sqrtf(ss / (float)width + eps);
   }
   float ss2 = 0.f;
 #pragma unroll
   for (int k = 0; k < NV; ++k) {
-    const int c = k * 256 + threadIdx.x;
+    const int c = k * T + threadIdx.x;
     if (c < w4) {
       hv[k].x += yv[k].x * rstd * wv[k].x;
       hv[k].y += yv[k].y * rstd * wv[k].y;
@@ -296,17 +294,12 @@ __global__ __launch_bounds__(256) void norm_add_reg_kernel(float* __restrict__ h
     }
   }
   if (w_next == nullptr) return;
-#pragma unroll
-  for (int k = 0; k < NV; ++k) {
-    const int c = k * 256 + threadIdx.x;
-    if (c < w4) wv[k] = *(const float4*)(w_next + 4 * c);
-  }
-  ss2 = block_sum(ss2, scratch);
+  ss2 = block_sum_once<T>(ss2, scratch[1]);
   const float rstd2 = 1.0f / sqrtf(ss2 / (float)width + eps_next);
 #pragma unroll
   for (int k = 0; k < NV; ++k) {
-    const int c = k * 256 + threadIdx.x;
-    if (c < w4) from_float4(x + (blocked ? ((size_t)(c >> 1) * gridDim.x + blockIdx.x) * 8 + (c & 1) * 4 : base + 4 * c), hv[k].x * rstd2 * wv[k].x, hv[k].y * rstd2 * wv[k].y, hv[k].z * rstd2 * wv[k].z, hv[k].w * rstd2 * wv[k].w);
+    const int c = k * T + threadIdx.x;
+    if (c < w4) from_float4(x + (blocked ? ((size_t)(c >> 1) * gridDim.x + blockIdx.x) * 8 + (c & 1) * 4 : base + 4 * c), hv[k].x * rstd2 * nv[k].x, hv[k].y * rstd2 * nv[k].y, hv[k].z * rstd2 * nv[k].z, hv[k].w * rstd2 * nv[k].w);
   }
 }
 
@@ -326,21 +319,22 @@ extern "C" int tp_norm_add(float* h, const float* y, const float* w, float eps, 
                        (gate_rows == nullptr || (((uintptr_t)gate_rows | (uintptr_t)gate_bias) % 16 == 0 && gate_stride % 4 == 0 && gate_col0 % 4 == 0));
   if (width % 4 == 0 && width >= 1024 && width <= 256 * 4 * 8 && aligned) {
     const bool bf = w_next != nullptr && x_dt == TP_BF16;
-#define NA1(TO, NV, G) \
-  hipLaunchKernelGGL((norm_add_reg_kernel<TO, NV, G>), dim3(n), dim3(256), 0, s, h, y, w, eps, w_next, eps_next, (TO*)x, width, gate, normed, blocked, parts)
-#define NA(NV)                                    \
+#define NA1(TO, T, NV, G) \
+  hipLaunchKernelGGL((norm_add_reg_kernel<TO, T, NV, G>), dim3(n), dim3(T), 0, s, h, y, w, eps, w_next, eps_next, (TO*)x, width, gate, normed, blocked, parts)
+#define NA(T, NV)                                 \
   do {                                            \
     if (gate_rows != nullptr) {                   \
-      if (bf) NA1(bf16_t, NV, true);              \
-      else NA1(float, NV, true);                  \
+      if (bf) NA1(bf16_t, T, NV, true);              \
+      else NA1(float, T, NV, true);                  \
     } else {                                      \
-      if (bf) NA1(bf16_t, NV, false);             \
-      else NA1(float, NV, false);                 \
+      if (bf) NA1(bf16_t, T, NV, false);             \
+      else NA1(float, T, NV, false);                 \
     }                                             \
   } while (0)
-    if (width <= 2048) NA(2);
-    else if (width <= 4096) NA(4);
-    else NA(8);
+    if (width <= 1024) NA(256, 1);
+    else if (width <= 2048) NA(512, 1);
+    else if (width <= 4096) NA(1024, 1);
+    else NA(1024, 2);
 #undef NA
 #undef NA1
     TP_CHECK_LAUNCH("norm_add");

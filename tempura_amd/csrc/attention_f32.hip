@@ -206,27 +206,34 @@ __global__ __launch_bounds__(256) void attn_f32_kernel(AttnF32Args a) {
   }
 }
 
-// Adds the splits of a single token's head in ascending order.  grid: (requests, heads), one wave.
-__global__ __launch_bounds__(64) void attn_f32_combine_kernel(const float* __restrict__ scratch, const int* __restrict__ cu_seqlens,
-                                                              float* __restrict__ out, int n_heads, int D, int splits,
-                                                              const float* __restrict__ sink) {
-  const int r = blockIdx.x, h = blockIdx.y, lane = threadIdx.x;
+// Adds the splits of a single token's head in ascending order.  grid: (requests, heads), a thread for every element in whole waves, each
+// of which works out the splits' factors for itself.  The first splits' values are requested with their maxima and sums, so a head of up to eight splits is
+// one trip to memory: with the attention in front, captured, 24 heads of 128, two requests of 300 / 700 keys 14.2 / 17.1 -> 12.0 / 13.4 us, one of
+// 2,000 22.0 -> 15.6 (a wave a head and the values behind the factors before).
+template <int D>
+__global__ __launch_bounds__((D + 63) / 64 * 64) void attn_f32_combine_kernel(const float* __restrict__ scratch, const int* __restrict__ cu_seqlens,
+                                                                           float* __restrict__ out, int n_heads, int splits,
+                                                                           const float* __restrict__ sink) {
+  constexpr int EARLY = 8;
+  const int r = blockIdx.x, h = blockIdx.y, lane = threadIdx.x % TP_WAVE, d = min((int)threadIdx.x, D - 1);
   const float* base = scratch + ((size_t)r * n_heads + h) * splits * (D + 2);
+  float v[EARLY];
+#pragma unroll
+  for (int s = 0; s < EARLY; ++s) v[s] = base[(size_t)min(s, splits - 1) * (D + 2) + d];
   // (at most 64 splits: a lane holds one's maximum and sum)
   const float ms = lane < splits ? base[(size_t)lane * (D + 2) + D] : -INFINITY;
   const float ls = lane < splits ? base[(size_t)lane * (D + 2) + D + 1] : 0.f;
   const float sk = sink != nullptr ? sink[h] : -INFINITY;
+  const int t = cu_seqlens[r];
   const float mg = fmaxf(wave_max(ms), sk);
   const float f = ms == -INFINITY ? 0.f : expf(ms - mg);
   const float inv = 1.0f / (wave_sum(f * ls) + (sink != nullptr ? expf(sk - mg) : 0.f));
-  // (every lane runs every turn: a lane that left could not hand its split's factor on)
-  for (int d0 = 0; d0 < D; d0 += 64) {
-    const int d = min(d0 + lane, D - 1);
-    float og = 0.f;
-#pragma unroll 8
-    for (int s = 0; s < splits; ++s) og = fmaf(__shfl(f, s, TP_WAVE), base[(size_t)s * (D + 2) + d], og);
-    if (d0 + lane < D) out[((size_t)cu_seqlens[r] * n_heads + h) * D + d] = og * inv;
-  }
+  float og = 0.f;
+#pragma unroll
+  for (int s = 0; s < EARLY; ++s)
+    if (s < splits) og = fmaf(__shfl(f, s, TP_WAVE), v[s], og);
+  for (int s = EARLY; s < splits; ++s) og = fmaf(__shfl(f, s, TP_WAVE), base[(size_t)s * (D + 2) + d], og);
+  if ((int)threadIdx.x < D) out[((size_t)t * n_heads + h) * D + d] = og * inv;
 }
 
 template <int D>
@@ -234,7 +241,8 @@ static void launch_f32(const AttnF32Args& a, int n_req, int max_q_len, hipStream
   const int tiles = (max_q_len * (a.n_heads / a.n_kv) + AF_ROWS - 1) / AF_ROWS;
   hipLaunchKernelGGL((attn_f32_kernel<D>), dim3((unsigned)tiles * a.n_kv, n_req, a.splits), dim3(256), 0, s, a);
   if (a.splits > 1)
-    hipLaunchKernelGGL(attn_f32_combine_kernel, dim3(n_req, a.n_heads), dim3(64), 0, s, a.scratch, a.cu_seqlens, a.out, a.n_heads, D, a.splits, a.sink);
+    hipLaunchKernelGGL((attn_f32_combine_kernel<D>), dim3(n_req, a.n_heads), dim3((D + 63) / 64 * 64), 0, s, a.scratch, a.cu_seqlens, a.out, a.n_heads,
+                       a.splits, a.sink);
 }
 
 // Returns -1 for shapes that the general kernel runs.  num_splits > 1 (every request brings one token): scratch of

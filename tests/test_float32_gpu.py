@@ -215,3 +215,23 @@ def test_float32_attention(heads, kv, d, page, q_lens, ctx_lens, what):
         other = run(inf)
         assert torch.equal(other[: q_lens[0] - 1], got[: q_lens[0] - 1])
         assert not torch.isfinite(other[q_lens[0] - 1]).any()
+
+
+@pytest.mark.parametrize("d", [32, 64, 96, 128])
+@pytest.mark.parametrize("ctx_lens", [[130, 1, 256], [600, 77], [1000], [1300]])
+def test_float32_attention_of_split_keys(d, ctx_lens):
+    """Single tokens whose keys are cut into two, four, eight and more splits, some of them without a key, heads that fill no whole
+    wave: against float64 (2e-6, as above), with and without a sink."""
+    from tempura_amd.kernels import ops
+    heads, kv, page, R = 6, 2, 16, len(ctx_lens)
+    g = torch.Generator().manual_seed(d + sum(ctx_lens))
+    width = -(-max(ctx_lens) // page)
+    bt = torch.randperm(R * width, generator=g).to(torch.int32).view(R, width)
+    kc, vc = torch.randn(R * width, kv, page, d, generator=g), torch.randn(R * width, kv, d, page, generator=g)
+    q, sink = torch.randn(R, heads, d, generator=g), torch.randn(heads, generator=g)
+    cu, cl = torch.arange(R + 1, dtype=torch.int32), torch.tensor(ctx_lens, dtype=torch.int32)
+    for more in ({}, {"sink": sink}):
+        want = emu.paged_attention(q.double(), kc, vc, bt, cu, cl, cu[:R], d ** -0.5, 0, 1, max(ctx_lens), **more)
+        got = ops.paged_attention(*(t.to(DEV) for t in (q, kc, vc, bt, cu, cl, cu[:R].contiguous())), d ** -0.5, 0, 1, max(ctx_lens),
+                                  **{k: v.to(DEV) for k, v in more.items()})
+        assert float((got.double().cpu() - want).abs().max() / want.abs().max()) < 2e-6

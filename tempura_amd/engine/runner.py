@@ -411,8 +411,7 @@ class ModelRunner:
     def _clear_state(self, fresh: Sequence[int]) -> None:
         """A request that starts at position 0 gets a cleared state (also after a recompute)."""
         if fresh:
-            for t in self.pools.state.values():
-                ops.zero_rows(t, fresh)
+            ops.zero_rows(list(self.pools.state.values()), fresh)
 
     def step_chained(self, rids: Sequence, tokens: torch.Tensor) -> torch.Tensor:
         """A step of one token per request whose tokens are still on the device: ``tokens`` int32 [len(rids)],

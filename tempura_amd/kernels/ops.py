@@ -13,6 +13,7 @@ from __future__ import annotations
 
 import ctypes
 import os
+import re
 from typing import Optional
 
 import torch
@@ -31,6 +32,35 @@ class KernelError(RuntimeError):
     pass
 
 
+_C_TYPES = {"int": ctypes.c_int, "unsigned": ctypes.c_uint, "size_t": ctypes.c_size_t, "float": ctypes.c_float, "double": ctypes.c_double,
+            "long": ctypes.c_long, "long long": ctypes.c_longlong, "unsigned long long": ctypes.c_ulonglong}
+
+
+def entry_points() -> dict:
+    """name -> (result type, argument types) of the library's C entry points, from the declarations in the sources that it is built from."""
+    from ..csrc.build import sources
+    out = {}
+    for path in sources():
+        with open(path) as f:
+            text = re.sub(r"//[^\n]*", "", f.read())
+        for result, name, args in re.findall(r'extern "C"\s+([\w\s]+?[\s\*]+)(tp_\w+)\s*\(([^)]*)\)\s*\{', text):
+            result = " ".join(result.split())
+            types = []
+            for arg in args.split(",") if args.strip() not in ("", "void") else ():
+                kind = "*" if "*" in arg or "hipStream_t" in arg else " ".join(w for w in arg.split()[:-1] if w != "const")
+                types.append(ctypes.c_void_p if kind == "*" else _C_TYPES[kind])
+            out[name] = (ctypes.c_char_p if "*" in result else None if result == "void" else _C_TYPES[result], types)
+    return out
+
+
+def _declare(lib) -> None:
+    # (addresses, numbers and None go to a declared entry point as they are; undeclared ones want an object of ctypes for each, which costs a
+    # launch of a dozen tensors more than the launch itself)
+    for name, (result, args) in entry_points().items():
+        fn = getattr(lib, name)
+        fn.restype, fn.argtypes = result, args
+
+
 class _Library:
     """The compiled kernel library, loaded on first use."""
 
@@ -47,10 +77,7 @@ class _Library:
                 lib = ctypes.CDLL(path)
             except OSError as e:
                 raise KernelError(f"cannot load the kernel library {path}: {e}") from e
-            lib.tp_last_error.restype = ctypes.c_char_p
-            lib.tp_linear_f32_scratch.restype = ctypes.c_size_t
-            lib.tp_delta_scan_scratch.restype = ctypes.c_size_t
-            lib.tp_step_prepared_size.restype = ctypes.c_size_t
+            _declare(lib)
             cls._lib = lib
             cls.path = path
         return cls._lib
@@ -126,7 +153,7 @@ def _dtcode(dtype: torch.dtype) -> int:
 
 
 def _ptr(t: Optional[torch.Tensor]):
-    return ctypes.c_void_p(0 if t is None else t.data_ptr())
+    return None if t is None else t.data_ptr()
 
 
 _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
@@ -137,8 +164,8 @@ def _stream():
     """The current stream's handle (of the current device).  Asked for at every launch: the direct call is
     some 8 us cheaper than ``torch.cuda.current_stream()``, a quarter of an eager launch's host time."""
     if _raw_stream is not None:
-        return ctypes.c_void_p(_raw_stream(_raw_device()))
-    return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+        return _raw_stream(_raw_device())
+    return torch.cuda.current_stream().cuda_stream
 
 
 def _need(cond: bool, msg: str) -> None:
@@ -149,12 +176,15 @@ def _need(cond: bool, msg: str) -> None:
 def _dev_ok(*ts) -> None:
     for t in ts:
         if t is not None:
-            _need(t.is_cuda, "operand is not on the GPU")
-            _need(t.is_contiguous(), "operand is not contiguous")
+            if not t.is_cuda:
+                raise KernelError("operand is not on the GPU")
+            if not t.is_contiguous():
+                raise KernelError("operand is not contiguous")
 
 
 def _i32(t: torch.Tensor, n: int, what: str) -> None:
-    _need(t.dtype == torch.int32 and t.numel() >= n and t.dim() >= 1, f"{what}: need int32 with {n} elements")
+    if not (t.dtype == torch.int32 and t.numel() >= n and t.dim() >= 1):
+        raise KernelError(f"{what}: need int32 with {n} elements")
 
 
 # ---------------------------------------------------------------------------------
@@ -208,7 +238,8 @@ def stream_step(h: torch.Tensor, streams: int, y: Optional[torch.Tensor] = None,
     for t, size, what in ((mix, streams * streams, "mix"), (out_coef, streams, "out_coef"), (in_coef, streams, "in_coef"),
                           (norm_weight, width, "norm_weight")):
         if t is not None:
-            _need(t.dtype == torch.float32 and t.numel() == size, f"stream_step: {what} must be float32 with {size} elements")
+            if not (t.dtype == torch.float32 and t.numel() == size):
+                raise KernelError(f"stream_step: {what} must be float32 with {size} elements")
     n_out = n
     if rows is not None:
         n_out = rows.numel()
@@ -221,7 +252,7 @@ def stream_step(h: torch.Tensor, streams: int, y: Optional[torch.Tensor] = None,
             return out          # (a step in which no row is wanted)
     else:
         _need(y is not None and write_back, "stream_step: nothing to do")
-    _call("tp_hc_step", _ptr(h), _ptr(y), _ptr(mix), _ptr(out_coef), _ptr(in_coef), _ptr(norm_weight), ctypes.c_float(eps),
+    _call("tp_hc_step", _ptr(h), _ptr(y), _ptr(mix), _ptr(out_coef), _ptr(in_coef), _ptr(norm_weight), float(eps),
           _ptr(out), _dtcode(out_dtype) if out_dtype is not None else _F32, _ptr(rows), n_out, int(streams), width,
           int(bool(write_back) and y is not None), _stream())
     return out
@@ -233,7 +264,7 @@ def scale_(x: torch.Tensor, scale: float) -> torch.Tensor:
         return _backend.scale_(x, scale)
     _dev_ok(x)
     _need(x.dtype == torch.float32, "scale_: needs float32")
-    _call("tp_scale_f32", _ptr(x), ctypes.c_size_t(x.numel()), ctypes.c_float(scale), _stream())
+    _call("tp_scale_f32", _ptr(x), int(x.numel()), float(scale), _stream())
     return x
 
 
@@ -249,8 +280,8 @@ def gated_act(gu: torch.Tensor, out_dtype: torch.dtype, slope: float = 1.0, limi
     _need(gu.dim() == 2 and gu.shape[1] % 2 == 0, "gated_act: input must be [m, 2i]")
     m, i2 = gu.shape
     out = torch.empty((m, i2 // 2), dtype=out_dtype, device=gu.device)
-    _call("tp_gated_act", _ptr(gu), _dt(gu), _ptr(out), _dtcode(out_dtype), m, i2 // 2, ctypes.c_float(slope),
-          ctypes.c_float(limit), ctypes.c_float(up_offset), int(bool(interleaved)), _stream())
+    _call("tp_gated_act", _ptr(gu), _dt(gu), _ptr(out), _dtcode(out_dtype), m, i2 // 2, float(slope),
+          float(limit), float(up_offset), int(bool(interleaved)), _stream())
     return out
 
 
@@ -267,7 +298,8 @@ def qk_store(rows: torch.Tensor, q_bias: Optional[torch.Tensor], k_bias: Optiona
     _need(rows.dtype == torch.float32 and rows.dim() == 2, "qk_store: rows must be float32 [n, width]")
     n = rows.shape[0]
     width = (num_heads + (num_kv_heads if slots is not None else 0)) * head_dim
-    _need(rows.shape[1] == width, f"qk_store: row width {rows.shape[1]} != {width}")
+    if not (rows.shape[1] == width):
+        raise KernelError(f"qk_store: row width {rows.shape[1]} != {width}")
     for b, size in ((q_bias, num_heads * head_dim), (k_bias, num_kv_heads * head_dim)):
         if b is not None:
             _need(b.dtype == torch.float32 and b.numel() == size, "qk_store: bias must be float32, one value per column")
@@ -314,7 +346,7 @@ def causal_conv(proj: torch.Tensor, col0: int, channels: int, weight: torch.Tens
     _i32(token_req, n, "token_req") if n else None
     out = torch.empty((n, channels), dtype=torch.float32, device=proj.device)
     _call("tp_causal_conv", _ptr(proj), proj.shape[1], int(col0), _ptr(weight), _ptr(bias), _ptr(state),
-          ctypes.c_size_t(state.shape[1]), ctypes.c_size_t(state_off), _ptr(cu_seqlens), _ptr(token_req), _ptr(state_slots), _ptr(out),
+          int(state.shape[1]), int(state_off), _ptr(cu_seqlens), _ptr(token_req), _ptr(state_slots), _ptr(out),
           n, int(num_requests), channels, taps, int(bool(act)), int(max_run), _stream())
     return out
 
@@ -334,7 +366,8 @@ def ssm_scan(xbc: torch.Tensor, proj: torch.Tensor, dt_col0: int, dt_bias: torch
     _dev_ok(xbc, proj, dt_bias, a_log, d_skip, state, cu_seqlens, state_slots)
     inner = num_heads * head_dim
     channels = inner + 2 * groups * state_size
-    _need(xbc.dtype == torch.float32 and xbc.dim() == 2 and xbc.shape[1] == channels, f"ssm_scan: xbc must be float32 [n, {channels}]")
+    if not (xbc.dtype == torch.float32 and xbc.dim() == 2 and xbc.shape[1] == channels):
+        raise KernelError(f"ssm_scan: xbc must be float32 [n, {channels}]")
     n = xbc.shape[0]
     _need(proj.dtype == torch.float32 and proj.dim() == 2 and proj.shape[0] == n and 0 <= dt_col0 and dt_col0 + num_heads <= proj.shape[1],
           "ssm_scan: bad projection rows")
@@ -348,12 +381,11 @@ def ssm_scan(xbc: torch.Tensor, proj: torch.Tensor, dt_col0: int, dt_bias: torch
     y = torch.empty((n, inner), dtype=torch.float32, device=xbc.device)
     max_run = n if max_run is None else min(int(max_run), n)
     lib = _Library.get()
-    lib.tp_ssm_scan_scratch.restype = ctypes.c_size_t
     need = lib.tp_ssm_scan_scratch(int(num_requests), max_run, num_heads, head_dim, state_size, None)
     scratch = torch.empty((need,), dtype=torch.float32, device=xbc.device) if need else None
     _call("tp_ssm_scan", _ptr(xbc), _ptr(proj), proj.shape[1], int(dt_col0), _ptr(dt_bias), _ptr(a_log), _ptr(d_skip), _ptr(state),
-          ctypes.c_size_t(state.shape[1]), ctypes.c_size_t(state_off), _ptr(cu_seqlens), _ptr(state_slots), _ptr(y),
-          int(num_requests), num_heads, head_dim, state_size, groups, max_run, _ptr(scratch), ctypes.c_size_t(need), _stream())
+          int(state.shape[1]), int(state_off), _ptr(cu_seqlens), _ptr(state_slots), _ptr(y),
+          int(num_requests), num_heads, head_dim, state_size, groups, max_run, _ptr(scratch), int(need), _stream())
     return y
 
 
@@ -370,7 +402,7 @@ def gated_group_norm(y: torch.Tensor, proj: torch.Tensor, z_col0: int, weight: t
           "gated_group_norm: bad projection rows")
     _need(weight.dtype == torch.float32 and weight.numel() == inner and groups > 0 and inner % groups == 0, "gated_group_norm: bad weight or groups")
     out = torch.empty((n, inner), dtype=out_dtype, device=y.device)
-    _call("tp_gated_group_norm", _ptr(y), _ptr(proj), proj.shape[1], int(z_col0), _ptr(weight), ctypes.c_float(eps), _ptr(out),
+    _call("tp_gated_group_norm", _ptr(y), _ptr(proj), proj.shape[1], int(z_col0), _ptr(weight), float(eps), _ptr(out),
           _dtcode(out_dtype), n, inner, int(groups), _stream())
     return out
 
@@ -393,11 +425,11 @@ def rmsnorm(h: torch.Tensor, weight: torch.Tensor, eps: float, out_dtype: torch.
     out = torch.empty((n_out, h.shape[1]), dtype=out_dtype, device=h.device)
     if groups != 1:
         _need(groups > 0 and h.shape[1] % groups == 0, "rmsnorm: groups must divide the row")
-        _call("tp_group_rmsnorm", _ptr(h), ctypes.c_size_t(h.shape[1]), 0, _ptr(weight), _ptr(rows), _ptr(out), _dtcode(out_dtype),
-              n_out, h.shape[1], int(groups), ctypes.c_float(eps), _stream())
+        _call("tp_group_rmsnorm", _ptr(h), int(h.shape[1]), 0, _ptr(weight), _ptr(rows), _ptr(out), _dtcode(out_dtype),
+              n_out, h.shape[1], int(groups), float(eps), _stream())
         return out
     _call("tp_rmsnorm", _ptr(h), _ptr(weight), _ptr(rows), _ptr(out), _dtcode(out_dtype), n_out, h.shape[1],
-          ctypes.c_float(eps), _stream())
+          float(eps), _stream())
     return out
 
 
@@ -501,7 +533,8 @@ class TiledWeight:
 
     def rows(self, lo: int, hi: int) -> "TiledWeight":
         """Rows lo..hi (multiples of 16) as a weight of their own; no copy."""
-        _need(lo % 16 == 0 and hi % 16 == 0 and 0 <= lo < hi <= self.n, f"tiled weight: rows {lo}..{hi} of {self.n}")
+        if not (lo % 16 == 0 and hi % 16 == 0 and 0 <= lo < hi <= self.n):
+            raise KernelError(f"tiled weight: rows {lo}..{hi} of {self.n}")
         return TiledWeight(self.data[lo // 16: hi // 16], hi - lo, self.k)
 
     def row_major(self) -> torch.Tensor:
@@ -568,8 +601,8 @@ def _pre_args(x):
         m, k = x.shape
         _need(x.x.dtype == torch.bfloat16 and x.ss.dtype == torch.float32 and x.x.numel() == m * k and
               tuple(x.ss.shape) == ((k + 15) // 16, 16), "linear: malformed handed-over rows")
-        return x.x, (_ptr(x.ss), x.ss.shape[0], ctypes.c_float(x.eps)), (m, k), (1 if x.blocked is not None else 0)
-    return x, (_ptr(None), 0, ctypes.c_float(0.0)), (tuple(x.shape) if x.dim() == 2 else None), 0
+        return x.x, (_ptr(x.ss), x.ss.shape[0], float(x.eps)), (m, k), (1 if x.blocked is not None else 0)
+    return x, (_ptr(None), 0, 0.0), (tuple(x.shape) if x.dim() == 2 else None), 0
 
 
 def linear_swiglu(x, w: torch.Tensor, blocked_out: bool = False, slope: float = 1.0, limit: float = 0.0, up_offset: float = 0.0):
@@ -585,7 +618,8 @@ def linear_swiglu(x, w: torch.Tensor, blocked_out: bool = False, slope: float = 
     x, pre, mk, xl = _pre_args(x)
     wd, wl = _w_args(w)
     _dev_ok(x, wd)
-    _need(mk is not None and w.dim() == 2 and mk[1] == w.shape[1], f"linear_swiglu: shapes {mk} x {tuple(w.shape)}")
+    if not (mk is not None and w.dim() == 2 and mk[1] == w.shape[1]):
+        raise KernelError(f"linear_swiglu: shapes {mk} x {tuple(w.shape)}")
     _need(x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16, "linear_swiglu: operands must be bfloat16")
     m, k = mk
     n = w.shape[0]
@@ -598,8 +632,8 @@ def linear_swiglu(x, w: torch.Tensor, blocked_out: bool = False, slope: float = 
         out = torch.empty((m, n // 2), dtype=torch.bfloat16, device=x.device)
     scratch, nscratch = _splitk_scratch(x, m, n)
     _call("tp_linear_fused", _ptr(x), _ptr(wd), _BF16, _ptr(out.data if blocked_out else out), _BF16, 2, m, n, k, 1,
-          _ptr(scratch), ctypes.c_size_t(nscratch), *pre, _ptr(None), _ptr(None), _ptr(None), (2 if blocked_out else 0) | wl | xl,
-          0, _ptr(None), ctypes.c_float(slope), ctypes.c_float(limit), ctypes.c_float(up_offset), 0, _ptr(None), _stream(), tag=(m, n, k))
+          _ptr(scratch), int(nscratch), *pre, _ptr(None), _ptr(None), _ptr(None), (2 if blocked_out else 0) | wl | xl,
+          0, _ptr(None), float(slope), float(limit), float(up_offset), 0, _ptr(None), _stream(), tag=(m, n, k))
     return out
 
 
@@ -627,7 +661,8 @@ def linear_relu2(x: torch.Tensor, w, act_cols: int, blocked_out: bool = False, k
         _need(x.rows <= 16 and tuple(x.data.shape) == (x.width // 8, x.rows, 8), "linear_relu2: malformed k-blocked rows")
         x, xl = x.data, 1
     _dev_ok(x, wd)
-    _need(len(shape) == 2 and w.dim() == 2 and shape[1] == w.shape[1], f"linear_relu2: shapes {shape} x {tuple(w.shape)}")
+    if not (len(shape) == 2 and w.dim() == 2 and shape[1] == w.shape[1]):
+        raise KernelError(f"linear_relu2: shapes {shape} x {tuple(w.shape)}")
     _need(x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and linear_relu2_ok(act_cols, shape[1], x.dtype)
           and 0 < act_cols <= w.shape[0], "linear_relu2: needs bfloat16 operands, k % 64 == 0 and a multiple of 128 activated columns")
     (m, k), n = shape, w.shape[0]
@@ -639,8 +674,8 @@ def linear_relu2(x: torch.Tensor, w, act_cols: int, blocked_out: bool = False, k
     side = torch.empty((m, n - act_cols), dtype=torch.float32, device=x.device)
     scratch, nscratch = _splitk_scratch(x, m, n)
     _call("tp_linear_fused", _ptr(x), _ptr(wd), _BF16, _ptr(out.data if blocked_out else out), _BF16, 3, m, n, k, 1, _ptr(scratch),
-          ctypes.c_size_t(nscratch), _ptr(None), 0, ctypes.c_float(0.0), _ptr(None), _ptr(None), _ptr(None),
-          (2 if blocked_out else 0) | wl | xl | ((0 if kind == "relu2" else ACTIVATIONS[kind] + 1) << 8), 0, _ptr(None), ctypes.c_float(1.0), ctypes.c_float(0.0), ctypes.c_float(0.0), int(act_cols), _ptr(side), _stream(), tag=(m, n, k))
+          int(nscratch), _ptr(None), 0, 0.0, _ptr(None), _ptr(None), _ptr(None),
+          (2 if blocked_out else 0) | wl | xl | ((0 if kind == "relu2" else ACTIVATIONS[kind] + 1) << 8), 0, _ptr(None), 1.0, 0.0, 0.0, int(act_cols), _ptr(side), _stream(), tag=(m, n, k))
     return out, side
 
 
@@ -680,10 +715,11 @@ def _f32_rows(x, w: torch.Tensor, gate: bool) -> torch.Tensor:
     rows, weight, eps = (x.x, x.weight, x.eps) if isinstance(x, Unnormed) else (x, None, 0.0)
     _dev_ok(rows, weight, w)
     (m, k), n = rows.shape, w.shape[0] // (2 if gate else 1)
-    _need(w.dim() == 2 and w.shape[1] == k and w.dtype == torch.float32, f"linear: shapes {(m, k)} x {tuple(w.shape)}")
+    if not (w.dim() == 2 and w.shape[1] == k and w.dtype == torch.float32):
+        raise KernelError(f"linear: shapes {(m, k)} x {tuple(w.shape)}")
     _need(weight is None or (weight.dtype == torch.float32 and weight.numel() == k), "linear: norm weight must be float32 [k]")
     out = torch.empty((m, n), dtype=torch.float32, device=rows.device)
-    _call("tp_linear_f32_rows", _ptr(rows), _ptr(w), _ptr(out), m, n, k, _ptr(weight), ctypes.c_float(eps), int(gate), _stream(),
+    _call("tp_linear_f32_rows", _ptr(rows), _ptr(w), _ptr(out), m, n, k, _ptr(weight), float(eps), int(gate), _stream(),
           tag=(m, w.shape[0], k))
     return out
 
@@ -725,7 +761,8 @@ def _stream_linear(x, w, close: StreamClose):
         return stream_step(h, close.streams, y, close.mix, close.out_coef, inc, weight, eps, None if weight is None else w.dtype)
     data = x.data if blocked else x
     _dev_ok(data, w.data, h, close.mix, close.out_coef)
-    _need(k == w.shape[1] and (not blocked or tuple(data.shape) == (k // 8, m, 8)), f"linear: shapes {(m, k)} x {tuple(w.shape)}")
+    if not (k == w.shape[1] and (not blocked or tuple(data.shape) == (k // 8, m, 8))):
+        raise KernelError(f"linear: shapes {(m, k)} x {tuple(w.shape)}")
     _need(h.dtype == torch.float32 and tuple(h.shape) == (m, close.streams * n), "linear: the stream must be float32 [m, streams * n]")
     s = close.streams
     inc, weight, eps = close.opening or (None, None, 0.0)
@@ -793,15 +830,18 @@ def linear(x, w: torch.Tensor, out_dtype: torch.dtype, residual: Optional[torch.
         _need(allow_mfma and x.data.dtype == torch.bfloat16 and tuple(x.data.shape) == (x.width // 8, x.rows, 8)
               and x.width % 32 == 0, "linear: malformed k-blocked rows")
         kb, layout = x, 1
-        x, pre = x.data, (_ptr(None), 0, ctypes.c_float(0.0))
+        x, pre = x.data, (_ptr(None), 0, 0.0)
         m, k = kb.rows, kb.width
         _dev_ok(x, wd, residual)
-        _need(w.dim() == 2 and w.shape[1] == k and w.dtype == torch.bfloat16, f"linear: shapes {(m, k)} x {tuple(w.shape)}")
+        if not (w.dim() == 2 and w.shape[1] == k and w.dtype == torch.bfloat16):
+            raise KernelError(f"linear: shapes {(m, k)} x {tuple(w.shape)}")
     else:
         x, pre, mk, layout = _pre_args(x)
         _dev_ok(x, wd, residual)
-        _need(mk is not None and w.dim() == 2 and mk[1] == w.shape[1], f"linear: shapes {mk} x {tuple(w.shape)}")
-        _need(x.dtype == w.dtype, f"linear: operand dtypes differ ({x.dtype}, {w.dtype})")
+        if not (mk is not None and w.dim() == 2 and mk[1] == w.shape[1]):
+            raise KernelError(f"linear: shapes {mk} x {tuple(w.shape)}")
+        if not (x.dtype == w.dtype):
+            raise KernelError(f"linear: operand dtypes differ ({x.dtype}, {w.dtype})")
         m, k = mk
     n = w.shape[0]
     if residual is not None:
@@ -835,8 +875,8 @@ def linear(x, w: torch.Tensor, out_dtype: torch.dtype, residual: Optional[torch.
          (partial_ok and residual is None and out_dtype == torch.float32))
     splits = ctypes.c_int(1)
     _call("tp_linear_fused", _ptr(x), _ptr(wd), _dt(x), _ptr(out), _dt(out), acc, m, n, k, int(allow_mfma), _ptr(scratch),
-          ctypes.c_size_t(nscratch), *pre, *post, layout, int(defer), ctypes.byref(splits), ctypes.c_float(1.0),
-          ctypes.c_float(0.0), ctypes.c_float(0.0), 0, _ptr(None), _stream(), tag=(m, n, k))
+          int(nscratch), *pre, *post, layout, int(defer), ctypes.byref(splits), 1.0,
+          0.0, 0.0, 0, _ptr(None), _stream(), tag=(m, n, k))
     if defer and splits.value > 1:
         if next_norm is None:
             return Partials(scratch[: splits.value * m * n].view(splits.value, m, n))
@@ -844,7 +884,7 @@ def linear(x, w: torch.Tensor, out_dtype: torch.dtype, residual: Optional[torch.
         _dev_ok(weight)
         _need(weight.dtype == torch.float32 and weight.numel() == n, "linear: norm weight must be float32 [n]")
         normed = torch.empty((m, n), dtype=x.dtype, device=x.device)
-        _call("tp_splitk_add_rmsnorm", _ptr(scratch), splits.value, _ptr(residual), _ptr(weight), ctypes.c_float(eps),
+        _call("tp_splitk_add_rmsnorm", _ptr(scratch), splits.value, _ptr(residual), _ptr(weight), float(eps),
               _ptr(normed), _dt(normed), m, n, _stream())
         return out, normed
     return out if next_norm is None else (out, handed)
@@ -879,14 +919,16 @@ def linear_rope_kv(x, w: torch.Tensor, positions: torch.Tensor, slots: torch.Ten
     x, pre, mk, xl = _pre_args(x)
     wd, wl = _w_args(w)
     _dev_ok(x, wd, positions, slots, inv_freq, k_cache, v_cache)
-    _need(mk is not None and w.dim() == 2 and mk[1] == w.shape[1], f"linear_rope_kv: shapes {mk} x {tuple(w.shape)}")
+    if not (mk is not None and w.dim() == 2 and mk[1] == w.shape[1]):
+        raise KernelError(f"linear_rope_kv: shapes {mk} x {tuple(w.shape)}")
     m, k = mk
     n = w.shape[0]
     _need(linear_rope_ok(m, n, k, head_dim, rotary_dim, k_cache.shape[2] if k_cache.dim() == 4 else 0, x.dtype, k_cache.dtype,
                          pre[1] != 0) and w.dtype == torch.bfloat16,
           "linear_rope_kv: sizes or dtypes that the fused projection does not take (see linear_rope_ok)")
     _need(m <= 16 or cos_sin is not None, "linear_rope_kv: a long step needs the table of cosines and sines")
-    _need(n == (num_heads + 2 * num_kv_heads) * head_dim, f"linear_rope_kv: {n} weight rows for {num_heads} + 2 x {num_kv_heads} heads of {head_dim}")
+    if not (n == (num_heads + 2 * num_kv_heads) * head_dim):
+        raise KernelError(f"linear_rope_kv: {n} weight rows for {num_heads} + 2 x {num_kv_heads} heads of {head_dim}")
     _i32(positions, m, "positions")
     _i32(slots, m, "slots")
     _need(k_cache.dim() == 4 and v_cache.dim() == 4 and k_cache.shape[1] == num_kv_heads and k_cache.shape[3] == head_dim
@@ -902,7 +944,7 @@ def linear_rope_kv(x, w: torch.Tensor, positions: torch.Tensor, slots: torch.Ten
               "linear_rope_kv: table must be float32 [m, rotary_dim / 2, 2]")
     q = torch.empty((m, num_heads, head_dim), dtype=torch.bfloat16, device=x.device)
     _call("tp_linear_rope", _ptr(x), _ptr(wd), int(wl != 0) | (2 if xl else 0), m, n, k, *pre, _ptr(positions), _ptr(slots), _ptr(inv_freq), rotary_dim,
-          ctypes.c_float(factor), num_heads, num_kv_heads, head_dim, _ptr(q), _ptr(k_cache), _ptr(v_cache),
+          float(factor), num_heads, num_kv_heads, head_dim, _ptr(q), _ptr(k_cache), _ptr(v_cache),
           k_cache.shape[2], _ptr(cos_sin), _stream(), tag=(m, n, k))
     return q
 
@@ -940,7 +982,8 @@ def rope_kv_write(qkv, positions: torch.Tensor, slots: Optional[torch.Tensor],
     _need(qkv.dtype == torch.float32 and qkv.dim() == 2, "rope_kv_write: rows must be float32 [n, width]")
     n = qkv.shape[0]
     width = (num_heads + (num_kv_heads if slots is not None else 0)) * head_dim + (num_kv_heads * vd if slots is not None else 0)
-    _need(qkv.shape[1] == width, f"rope_kv_write: row width {qkv.shape[1]} != {width}")
+    if not (qkv.shape[1] == width):
+        raise KernelError(f"rope_kv_write: row width {qkv.shape[1]} != {width}")
     _i32(positions, n, "positions") if n else None
     page_size, cache_dt = 1, _F32
     if slots is not None:
@@ -960,7 +1003,7 @@ def rope_kv_write(qkv, positions: torch.Tensor, slots: Optional[torch.Tensor],
     _need(od >= head_dim and od % 2 == 0, "rope_kv_write: pad_dim must be even and at least head_dim")
     q = torch.empty((n, num_heads, od), dtype=q_dtype, device=qkv.device)
     _call("tp_rope_kv_write", _ptr(qkv), qkv.shape[1], _ptr(positions), _ptr(slots), _ptr(inv_freq), rotary_dim,
-          ctypes.c_float(factor), n, num_heads, num_kv_heads, head_dim, _ptr(q), _dtcode(q_dtype),
+          float(factor), n, num_heads, num_kv_heads, head_dim, _ptr(q), _dtcode(q_dtype),
           _ptr(k_cache), _ptr(v_cache), cache_dt, page_size, splits, _ptr(cos_sin), vd, od, _stream())
     return q
 
@@ -976,7 +1019,7 @@ def rope_table(positions: torch.Tensor, inv_freq: torch.Tensor, rotary_dim: int,
     _need(rotary_dim > 0 and inv_freq.dtype == torch.float64 and inv_freq.numel() == rotary_dim // 2,
           "rope_table: inv_freq must be float64 [rotary_dim / 2]")
     table = torch.empty((n, rotary_dim // 2, 2), dtype=torch.float32, device=positions.device)
-    _call("tp_rope_table", _ptr(positions), _ptr(inv_freq), rotary_dim, ctypes.c_float(factor), n, _ptr(table), _stream())
+    _call("tp_rope_table", _ptr(positions), _ptr(inv_freq), rotary_dim, float(factor), n, _ptr(table), _stream())
     return table
 
 
@@ -1202,10 +1245,10 @@ def paged_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tenso
                                and gate_col0 + heads * vd // per <= gate.shape[1]), "paged_attention: bad gate rows")
     _call("tp_paged_attention", _ptr(q), _dt(q), _ptr(k_cache), _ptr(v_cache), _ptr(block_tables), width,
           _ptr(cu_seqlens), _ptr(context_lens), _ptr(token_req), _ptr(dest), n, r, heads, kvh, d, page_size,
-          ctypes.c_float(scale), int(window), int(max_q_len), int(max_context_len), 2 if gated else int(fast or fast_f32),
+          float(scale), int(window), int(max_q_len), int(max_context_len), 2 if gated else int(fast or fast_f32),
           int(num_single), int(splits), _decode_waves(max(1, num_single), heads, kvh, splits), _ptr(scratch), int(parts), max(1, portion_min_keys // 32), _ptr(part_scratch),
           _ptr(dist_bias), 0 if dist_bias is None else dist_bias.shape[1], int(vd), int(keep_first), _ptr(sink), int(chunk),
-          ctypes.c_float(softcap), _ptr(gate), 0 if gate is None else gate.shape[1], int(gate_col0), int(per), ctypes.c_float(factor),
+          float(softcap), _ptr(gate), 0 if gate is None else gate.shape[1], int(gate_col0), int(per), float(factor),
           dest.shape[1], int(dest_col0), _stream())
     if into is None:
         return dest
@@ -1312,14 +1355,14 @@ def attention_rows(rows, col0: int, ctx, group: int, heads: int, kvh: int, dim: 
     else:
         gate, gate_col0, gate_scale, out_col0, per = None, 0, 1.0, 0, 1
         out = torch.empty((n, heads * dim), dtype=torch.bfloat16, device=data.device)
-    _call("tp_attention_rows", ctypes.c_void_p(data.data_ptr() + 4 * col0), ctypes.c_size_t(n * stride), stride, parts,
+    _call("tp_attention_rows", (data.data_ptr() + 4 * col0), int(n * stride), stride, parts,
           _ptr(conv_w), 0 if conv_w is None else conv_w.shape[0], 0 if conv_w is None else conv_w.shape[1], _ptr(state),
-          ctypes.c_size_t(0 if state is None else state.shape[1]), ctypes.c_size_t(state_off), _ptr(ctx.state_slots if conv is not None else None),
-          _ptr(None if norms is None else norms[0]), _ptr(None if norms is None else norms[1]), ctypes.c_float(norm_eps), _ptr(ctx.positions),
-          _ptr(inv_freq), int(rotary_dim), ctypes.c_float(factor), _ptr(cos_sin), _ptr(slots), _ptr(k_cache), _ptr(v_cache), _ptr(bt), bt.shape[1],
-          _ptr(ctx.cu_seqlens), _ptr(ctx.context_lens), _ptr(out), n, heads, kvh, dim, page_size, ctypes.c_float(scale), int(window), int(keep_first),
+          int(0 if state is None else state.shape[1]), int(state_off), _ptr(ctx.state_slots if conv is not None else None),
+          _ptr(None if norms is None else norms[0]), _ptr(None if norms is None else norms[1]), float(norm_eps), _ptr(ctx.positions),
+          _ptr(inv_freq), int(rotary_dim), float(factor), _ptr(cos_sin), _ptr(slots), _ptr(k_cache), _ptr(v_cache), _ptr(bt), bt.shape[1],
+          _ptr(ctx.cu_seqlens), _ptr(ctx.context_lens), _ptr(out), n, heads, kvh, dim, page_size, float(scale), int(window), int(keep_first),
           int(chunk), _ptr(sink), int(splits), 8 if beside is not None else _decode_waves(n, heads, kvh, splits), _ptr(scratch), int(into is not None), _ptr(gate), 0 if gate is None else gate.shape[1], int(gate_col0),
-          int(per), ctypes.c_float(gate_scale), out.shape[1], int(out_col0), beside, _stream())
+          int(per), float(gate_scale), out.shape[1], int(out_col0), beside, _stream())
     return None if into is not None else out
 
 
@@ -1553,19 +1596,26 @@ def take_rows(t: torch.Tensor, rows=None) -> torch.Tensor:
     return out
 
 
-def zero_rows(t: torch.Tensor, rows) -> None:
-    """t[rows] = 0 in place for a float32 or int32 tensor [n, ...] (rows: a list of indices)."""
+def zero_rows(t, rows) -> None:
+    """t[rows] = 0 in place for a float32 or int32 tensor [n, ...], or for each of a list of them (rows: a list of indices, which
+    travels to the device once)."""
+    ts = [t] if isinstance(t, torch.Tensor) else list(t)
     if _backend is not None:
-        return _backend.zero_rows(t, rows)
+        for t in ts:
+            _backend.zero_rows(t, rows)
+        return
     import numpy as np
-    _dev_ok(t)
-    _need(t.dtype in (torch.float32, torch.int32) and t.dim() >= 1, "zero_rows: needs a float32 or int32 tensor")
-    n_in = t.shape[0]
-    width = t[0].numel() if n_in else 0
-    _need(all(0 <= int(r) < n_in for r in rows), "zero_rows: row out of range")
-    if len(rows) and width:
-        idx = _Staging.send([np.asarray(rows, dtype=np.int32)], t.device)[0]
-        _call("tp_zero_rows4", _ptr(t), _ptr(idx), len(rows), width, _stream())
+    _dev_ok(*ts)
+    for t in ts:
+        _need(t.dtype in (torch.float32, torch.int32) and t.dim() >= 1, "zero_rows: needs a float32 or int32 tensor")
+        _need(all(0 <= int(r) < t.shape[0] for r in rows), "zero_rows: row out of range")
+    idx = None
+    for t in ts:
+        width = t[0].numel() if t.shape[0] else 0
+        if len(rows) and width:
+            if idx is None or idx.device != t.device:
+                idx = _Staging.send([np.asarray(rows, dtype=np.int32)], t.device)[0]
+            _call("tp_zero_rows4", _ptr(t), _ptr(idx), len(rows), width, _stream())
 
 
 def fill_normal(out: torch.Tensor, seed: int, mean: float, std: float) -> torch.Tensor:
@@ -1574,7 +1624,7 @@ def fill_normal(out: torch.Tensor, seed: int, mean: float, std: float) -> torch.
     if _backend is not None:
         return _backend.fill_normal(out, seed, mean, std)
     _dev_ok(out)
-    _call("tp_fill_normal", _ptr(out), _dt(out), ctypes.c_size_t(out.numel()), ctypes.c_ulonglong(seed & (2 ** 64 - 1)),
+    _call("tp_fill_normal", _ptr(out), _dt(out), int(out.numel()), ctypes.c_ulonglong(seed & (2 ** 64 - 1)),
           ctypes.c_double(mean), ctypes.c_double(std), _stream())
     return out
 
@@ -1606,7 +1656,8 @@ def embed_bigram(tokens: torch.Tensor, table: torch.Tensor, bigram: Optional[tor
     if bigram is not None:
         _need(bigram.dim() == 2 and bigram.shape[1] == table.shape[1] and bigram.dtype == table.dtype,
               "embed_bigram: tables must be [rows, hidden] of one type")
-        _need(bigram.shape[0] == buckets + 1, f"embed_bigram: the bigram table needs {buckets + 1} rows, has {bigram.shape[0]}")
+        if not (bigram.shape[0] == buckets + 1):
+            raise KernelError(f"embed_bigram: the bigram table needs {buckets + 1} rows, has {bigram.shape[0]}")
         _need(prev_state is not None and prev_state.dtype == torch.int32, "embed_bigram: the state must be int32")
     _i32(tokens, n, "embed tokens") if n else None
     _i32(positions, n, "embed positions") if n else None
@@ -1617,7 +1668,7 @@ def embed_bigram(tokens: torch.Tensor, table: torch.Tensor, bigram: Optional[tor
     out = torch.empty((n, hidden), dtype=torch.float32, device=table.device)
     _call("tp_embed_bigram", _ptr(tokens), _ptr(positions), _ptr(token_req), _ptr(cu_seqlens), _ptr(state_slots), _ptr(prev_state),
           _ptr(table), _ptr(bigram), _dt(table), _ptr(out), n, int(num_requests), hidden, ctypes.c_longlong(mul_prev),
-          ctypes.c_longlong(mul_cur), ctypes.c_longlong(buckets), ctypes.c_float(scale), _ptr(pos_table), _stream())
+          ctypes.c_longlong(mul_cur), ctypes.c_longlong(buckets), float(scale), _ptr(pos_table), _stream())
     return out
 
 
@@ -1637,7 +1688,7 @@ def sigmoid_gate(a: torch.Tensor, proj: Optional[torch.Tensor], gate_col0: int, 
     if proj is not None:
         _need(proj.dtype == torch.float32 and proj.dim() == 2 and proj.shape[0] == n and 0 <= gate_col0 and gate_col0 + width // per <= proj.shape[1],
               "sigmoid_gate: bad gate rows")
-    _call("tp_sigmoid_gate", _ptr(a), _dt(a), _ptr(proj), 0 if proj is None else proj.shape[1], int(gate_col0), ctypes.c_float(scale),
+    _call("tp_sigmoid_gate", _ptr(a), _dt(a), _ptr(proj), 0 if proj is None else proj.shape[1], int(gate_col0), float(scale),
           _ptr(out), out.shape[1], int(out_col0), n, width, int(per), _stream())
 
 
@@ -1660,21 +1711,23 @@ def turn_gate(a: torch.Tensor, positions: torch.Tensor, inv_freq: torch.Tensor, 
         _need(cos_sin.dtype == torch.float32 and tuple(cos_sin.shape) == (n, dim // 2, 2), "turn_gate: table must be float32 [n, dim / 2, 2]")
     out = torch.empty_like(a)
     _call("tp_turn_gate", _ptr(a), _dt(a), _ptr(positions), _ptr(inv_freq), _ptr(cos_sin), _ptr(gate),
-          ctypes.c_size_t(0 if gate is None else gate.shape[1]), int(gate_col0), _ptr(out), n, width // dim, int(dim), _stream())
+          int(0 if gate is None else gate.shape[1]), int(gate_col0), _ptr(out), n, width // dim, int(dim), _stream())
     return out
 
 
 def _cache_pair(k_cache, v_cache, kv_heads, key_dim, value_dim, what):
-    _need(k_cache.dim() == 4 and v_cache.dim() == 4 and k_cache.shape[1] == kv_heads and k_cache.shape[3] == key_dim
-          and tuple(v_cache.shape) == (k_cache.shape[0], kv_heads, value_dim, k_cache.shape[2]) and v_cache.dtype == k_cache.dtype,
-          f"{what}: caches must be k [pages, {kv_heads}, page_size, {key_dim}], v [pages, {kv_heads}, {value_dim}, page_size] of one type")
+    if not (k_cache.dim() == 4 and v_cache.dim() == 4 and k_cache.shape[1] == kv_heads and k_cache.shape[3] == key_dim
+            and tuple(v_cache.shape) == (k_cache.shape[0], kv_heads, value_dim, k_cache.shape[2]) and v_cache.dtype == k_cache.dtype):
+        raise KernelError(f"{what}: caches must be k [pages, {kv_heads}, page_size, {key_dim}], v [pages, {kv_heads}, {value_dim}, page_size] of one type")
 
 
 def _rotation(inv_freq, pairs, cos_sin, n, what):
     if pairs:
-        _need(inv_freq is not None and inv_freq.dtype == torch.float64 and inv_freq.numel() == pairs, f"{what}: frequencies must be float64 [{pairs}]")
+        if not (inv_freq is not None and inv_freq.dtype == torch.float64 and inv_freq.numel() == pairs):
+            raise KernelError(f"{what}: frequencies must be float64 [{pairs}]")
     if cos_sin is not None:
-        _need(cos_sin.dtype == torch.float32 and tuple(cos_sin.shape) == (n, pairs, 2), f"{what}: table must be float32 [n, {pairs}, 2]")
+        if not (cos_sin.dtype == torch.float32 and tuple(cos_sin.shape) == (n, pairs, 2)):
+            raise KernelError(f"{what}: table must be float32 [n, {pairs}, 2]")
 
 
 def qkv_rows(rows: torch.Tensor, positions: torch.Tensor, slots: torch.Tensor, num_heads: int, num_kv_heads: int, head_dim: int,
@@ -1691,7 +1744,8 @@ def qkv_rows(rows: torch.Tensor, positions: torch.Tensor, slots: torch.Tensor, n
     to the cache rows ``slots``.  Returns q in the caches' type as [n, heads, pad_dim or head_dim] (keys are stored as
     wide; zeros behind a head's own elements).  ``col0``: the column at which q | k | v start."""
     od = head_dim if pad_dim is None else int(pad_dim)
-    _need(norm_over in ("projection", "head"), f"qkv_rows: norm over {norm_over!r} unknown")
+    if not (norm_over in ("projection", "head")):
+        raise KernelError(f"qkv_rows: norm over {norm_over!r} unknown")
     per_head = norm_over == "head"
     if _backend is not None:
         if col0 or per_head:
@@ -1708,7 +1762,8 @@ def qkv_rows(rows: torch.Tensor, positions: torch.Tensor, slots: torch.Tensor, n
           "qkv_rows: rows must be float32 [n, an even width of at least q | k | v]")
     for b, size, what in ((qb, widths[0], "q bias"), (kb, widths[1], "k bias"), (vb, widths[2], "v bias"),
                           (qn, head_dim if per_head else widths[0], "q norm"), (kn, head_dim if per_head else widths[1], "k norm")):
-        _need(b is None or (b.dtype == torch.float32 and b.numel() == size), f"qkv_rows: {what} must be float32 with {size} elements")
+        if not (b is None or (b.dtype == torch.float32 and b.numel() == size)):
+            raise KernelError(f"qkv_rows: {what} must be float32 with {size} elements")
     _need((qn is None) == (kn is None), "qkv_rows: the norms of q and k come together")
     if n:
         _i32(positions, n, "positions")
@@ -1720,9 +1775,9 @@ def qkv_rows(rows: torch.Tensor, positions: torch.Tensor, slots: torch.Tensor, n
     if value_inv_freq is not None:
         _rotation(value_inv_freq, value_dim // 2, value_cos_sin, n, "qkv_rows: values")
     q = torch.empty((n, num_heads, od), dtype=k_cache.dtype, device=rows.device)
-    _call("tp_qkv_rows", ctypes.c_void_p(rows.data_ptr() + 4 * int(col0)), ctypes.c_size_t(rows.shape[1]), ctypes.c_size_t(rows.shape[1] - int(col0)),
-          _ptr(qb), _ptr(kb), _ptr(vb), _ptr(qn), _ptr(kn), ctypes.c_float(eps),
-          _ptr(positions), _ptr(slots), _ptr(inv_freq), _ptr(cos_sin), int(rotary_dim), ctypes.c_float(factor), _ptr(value_inv_freq),
+    _call("tp_qkv_rows", (rows.data_ptr() + 4 * int(col0)), int(rows.shape[1]), int(rows.shape[1] - int(col0)),
+          _ptr(qb), _ptr(kb), _ptr(vb), _ptr(qn), _ptr(kn), float(eps),
+          _ptr(positions), _ptr(slots), _ptr(inv_freq), _ptr(cos_sin), int(rotary_dim), float(factor), _ptr(value_inv_freq),
           _ptr(value_cos_sin), n, int(num_heads), int(num_kv_heads), int(head_dim), int(value_dim), od, _ptr(q), _ptr(k_cache),
           _ptr(v_cache), _dt(k_cache), k_cache.shape[2], int(per_head), _stream())
     return q
@@ -1756,8 +1811,8 @@ def latent_rows_write(rows: torch.Tensor, q_col0: int, d_col0: int, weight: torc
         _i32(positions, n, "positions")
         _i32(slots, n, "slots")
     q = torch.empty((n, num_heads, od), dtype=k_cache.dtype, device=rows.device)
-    _call("tp_latent_rows_write", _ptr(rows), ctypes.c_size_t(rows.shape[1]), int(q_col0), int(d_col0), _ptr(weight), ctypes.c_float(eps),
-          _ptr(positions), _ptr(slots), _ptr(inv_freq), _ptr(cos_sin), ctypes.c_float(factor), n, int(num_heads), int(rotary_dim),
+    _call("tp_latent_rows_write", _ptr(rows), int(rows.shape[1]), int(q_col0), int(d_col0), _ptr(weight), float(eps),
+          _ptr(positions), _ptr(slots), _ptr(inv_freq), _ptr(cos_sin), float(factor), n, int(num_heads), int(rotary_dim),
           int(latent_dim), od, vd, _ptr(q), _ptr(k_cache), _ptr(v_cache), _dt(k_cache), k_cache.shape[2], q_head, q_rot,
           int(plain_dim is None), _stream())
     return q
@@ -1785,10 +1840,10 @@ def head_linear(x: torch.Tensor, x_col0: int, x_head: int, w: torch.Tensor, out:
     if gate is not None:
         _need(gate.dtype == torch.float32 and gate.dim() == 2 and gate.shape[0] == m and 0 <= gate_col0 and gate_col0 + H <= gate.shape[1],
               "head_linear: bad gate rows")
-    at = lambda t, col: ctypes.c_void_p(t.data_ptr() + col * t.element_size())
-    _call("tp_head_linear", at(x, x_col0), _dt(x), ctypes.c_size_t(x.shape[1]), int(x_head), _ptr(w), at(out, out_col0),
-          ctypes.c_size_t(out.shape[1]), int(out_head), _ptr(None) if gate is None else at(gate, gate_col0),
-          ctypes.c_size_t(0 if gate is None else gate.shape[1]), ctypes.c_float(scale), m, H, N, K, _stream(), tag=(m, H, N, K))
+    at = lambda t, col: (t.data_ptr() + col * t.element_size())
+    _call("tp_head_linear", at(x, x_col0), _dt(x), int(x.shape[1]), int(x_head), _ptr(w), at(out, out_col0),
+          int(out.shape[1]), int(out_head), _ptr(None) if gate is None else at(gate, gate_col0),
+          int(0 if gate is None else gate.shape[1]), float(scale), m, H, N, K, _stream(), tag=(m, H, N, K))
 
 
 def norm_add(h: torch.Tensor, y: torch.Tensor, weight: torch.Tensor, eps: float, next_weight: Optional[torch.Tensor] = None,
@@ -1820,8 +1875,8 @@ def norm_add(h: torch.Tensor, y: torch.Tensor, weight: torch.Tensor, eps: float,
     if next_weight is not None:
         _need(next_weight.dtype == torch.float32 and next_weight.numel() == width and out_dtype is not None, "norm_add: bad next norm")
         x = torch.empty((width // 8, n, 8) if blocked else (n, width), dtype=out_dtype, device=h.device)
-    _call("tp_norm_add", _ptr(h), _ptr(y), _ptr(weight), ctypes.c_float(eps), _ptr(next_weight), ctypes.c_float(next_eps), _ptr(x),
-          _dtcode(out_dtype) if x is not None else _F32, n, width, _ptr(gate), ctypes.c_size_t(0 if gate is None else gate.shape[1]),
+    _call("tp_norm_add", _ptr(h), _ptr(y), _ptr(weight), float(eps), _ptr(next_weight), float(next_eps), _ptr(x),
+          _dtcode(out_dtype) if x is not None else _F32, n, width, _ptr(gate), int(0 if gate is None else gate.shape[1]),
           int(gate_col0), _ptr(gate_bias), int(normed), int(blocked), parts, _stream())
     return KBlocked(x, n, width) if blocked and x is not None else x
 
@@ -1846,7 +1901,8 @@ def activation(u: torch.Tensor, kind: str, out_dtype: torch.dtype, col0: int = 0
     With ``width`` (``u`` float32 rows [n, wider]): the columns col0 .. col0 + width of every row, and with ``gate_col``
     each row's results times the sigmoid of that column of the row.  ``blocked`` (whole float32 rows, see ``few_rows_ok``):
     the result comes as ``KBlocked``."""
-    _need(kind in ACTIVATIONS, f"activation: {kind!r} unknown (known: {sorted(ACTIVATIONS)})")
+    if not (kind in ACTIVATIONS):
+        raise KernelError(f"activation: {kind!r} unknown (known: {sorted(ACTIVATIONS)})")
     if _backend is not None:
         if width is not None:
             return _backend.activation(u, kind, out_dtype, col0, width, gate_col)
@@ -1857,7 +1913,7 @@ def activation(u: torch.Tensor, kind: str, out_dtype: torch.dtype, col0: int = 0
               "activation: rows must be float32 [n, wider]")
         _need(gate_col is None or 0 <= gate_col < u.shape[1], "activation: gate column outside the rows")
         out = torch.empty((u.shape[0], width), dtype=out_dtype, device=u.device)
-        _call("tp_activation_rows", _ptr(u), ctypes.c_size_t(u.shape[1]), int(col0), int(width), -1 if gate_col is None else int(gate_col),
+        _call("tp_activation_rows", _ptr(u), int(u.shape[1]), int(col0), int(width), -1 if gate_col is None else int(gate_col),
               _ptr(out), _dtcode(out_dtype), u.shape[0], ACTIVATIONS[kind], _stream())
         return out
     if blocked:
@@ -1867,7 +1923,7 @@ def activation(u: torch.Tensor, kind: str, out_dtype: torch.dtype, col0: int = 0
         _call("tp_activation_blocked", _ptr(u), _ptr(out), _dtcode(out_dtype), m, n, ACTIVATIONS[kind], _stream())
         return KBlocked(out, m, n)
     out = torch.empty(u.shape, dtype=out_dtype, device=u.device)
-    _call("tp_activation", _ptr(u), _dt(u), _ptr(out), _dtcode(out_dtype), ctypes.c_size_t(u.numel()), ACTIVATIONS[kind], _stream())
+    _call("tp_activation", _ptr(u), _dt(u), _ptr(out), _dtcode(out_dtype), int(u.numel()), ACTIVATIONS[kind], _stream())
     return out
 
 
@@ -1885,7 +1941,8 @@ def moe_route(logits: torch.Tensor, correction: Optional[torch.Tensor], experts:
     weight and 0 elsewhere, ids int32 [n, top], weights [n, top]).  ``bias`` (float32 [experts]) is added to the logits
     first.  (A softmax over the chosen logits alone is ``normalize`` without ``sum_eps``: the chosen experts' shares of
     the full softmax over their sum.)"""
-    _need(score in ROUTE_SCORES, f"moe_route: score {score!r} unknown")
+    if not (score in ROUTE_SCORES):
+        raise KernelError(f"moe_route: score {score!r} unknown")
     if _backend is not None:
         if bias is not None:
             return _backend.moe_route(logits, correction, experts, top, groups, keep, score, group_best, normalize, sum_eps, scale, bias)
@@ -1902,8 +1959,8 @@ def moe_route(logits: torch.Tensor, correction: Optional[torch.Tensor], experts:
     ids = torch.empty((n, top), dtype=torch.int32, device=logits.device)
     weights = torch.empty((n, top), dtype=torch.float32, device=logits.device)
     _call("tp_moe_route", _ptr(logits), logits.shape[1], _ptr(correction), int(experts), int(top), int(groups), int(keep), _ptr(dense),
-          _ptr(ids), _ptr(weights), n, ROUTE_SCORES[score], int(group_best), int(bool(normalize)), ctypes.c_float(sum_eps),
-          ctypes.c_float(scale), _ptr(bias), _stream())
+          _ptr(ids), _ptr(weights), n, ROUTE_SCORES[score], int(group_best), int(bool(normalize)), float(sum_eps),
+          float(scale), _ptr(bias), _stream())
     return dense, ids, weights
 
 
@@ -1917,13 +1974,15 @@ def lowrank_up(x: torch.Tensor, col0: int, weight_t: torch.Tensor, mode: str = "
     exp(-exp(a_log[c // per_head]) * softplus(sum + bias[c])); ``rate_sigmoid``: exp(-rate * sigmoid(sum + bias[c]));
     ``exp_exp``: exp(-exp(sum + bias[c])); ``root_sigmoid``: sigmoid(sum + bias[c])^rate.
     g: the identity, or tanh with ``in_act`` ``"tanh"``."""
-    _need(in_act in (None, "tanh"), f"lowrank_up: input function {in_act!r} unknown")
+    if not (in_act in (None, "tanh")):
+        raise KernelError(f"lowrank_up: input function {in_act!r} unknown")
     if _backend is not None:
         if mode in ("rate_sigmoid", "exp_exp", "root_sigmoid") or in_act is not None:
             return _backend.lowrank_up(x, col0, weight_t, mode, a_log, bias, per_head, rate, in_act)
         return _backend.lowrank_up(x, col0, weight_t, mode, a_log, bias, per_head)
     _dev_ok(x, weight_t, a_log, bias)
-    _need(mode in LOWRANK_MODES, f"lowrank_up: mode {mode!r} unknown")
+    if not (mode in LOWRANK_MODES):
+        raise KernelError(f"lowrank_up: mode {mode!r} unknown")
     _need(x.dtype == torch.float32 and x.dim() == 2 and weight_t.dtype == torch.float32 and weight_t.dim() == 2, "lowrank_up: float32 operands")
     r, n_out = weight_t.shape
     _need(0 <= col0 and col0 + r <= x.shape[1], "lowrank_up: rows too short")
@@ -1934,7 +1993,7 @@ def lowrank_up(x: torch.Tensor, col0: int, weight_t: torch.Tensor, mode: str = "
         _need(bias is not None and bias.dtype == torch.float32 and bias.numel() == n_out, "lowrank_up: bad decay biases")
     out = torch.empty((x.shape[0], n_out), dtype=torch.float32, device=x.device)
     _call("tp_lowrank_up", _ptr(x), x.shape[1], int(col0), r, _ptr(weight_t), _ptr(out), x.shape[0], n_out, LOWRANK_MODES[mode],
-          _ptr(a_log), _ptr(bias), int(per_head), 1 if in_act == "tanh" else 0, ctypes.c_float(rate), _stream())
+          _ptr(a_log), _ptr(bias), int(per_head), 1 if in_act == "tanh" else 0, float(rate), _stream())
     return out
 
 
@@ -1967,9 +2026,9 @@ def delta_scan(qkv: torch.Tensor, decay: torch.Tensor, proj: torch.Tensor, beta_
     need = library().tp_delta_scan_scratch(n, int(num_requests), max_run, int(heads), int(dim), int(vdim)) if allow_mfma else 0
     scratch = torch.empty((need,), dtype=torch.float32, device=qkv.device) if need else None
     _call("tp_delta_scan", _ptr(qkv), qkv.shape[1], _ptr(decay), _ptr(proj), proj.shape[1], int(beta_col0), _ptr(state),
-          ctypes.c_size_t(state.shape[1]), ctypes.c_size_t(state_off), _ptr(cu_seqlens), _ptr(state_slots), _ptr(y), _ptr(kq), n,
-          int(num_requests), int(heads), int(kv_heads), int(dim), int(vdim), ctypes.c_float(q_scale), ctypes.c_float(unit_eps),
-          max_run, _ptr(scratch), ctypes.c_size_t(need), _stream())
+          int(state.shape[1]), int(state_off), _ptr(cu_seqlens), _ptr(state_slots), _ptr(y), _ptr(kq), n,
+          int(num_requests), int(heads), int(kv_heads), int(dim), int(vdim), float(q_scale), float(unit_eps),
+          max_run, _ptr(scratch), int(need), _stream())
     return y
 
 
@@ -1983,7 +2042,8 @@ def head_norm_gate(o: torch.Tensor, weight: torch.Tensor, gate: Optional[torch.T
     ``o`` float32 [n, heads * vdim]; ``weight`` float32 [vdim] shared by the heads, or [heads * vdim], every head its own;
     ``gate`` float32 like ``o`` or None.  ``gate_rows`` (float32 rows [n, wider], instead of ``gate``): the gate is the
     sigmoid (``gate_act`` ``"silu"``: the SiLU) of their columns gate_col0 .. gate_col0 + heads * vdim."""
-    _need(gate_act in GATE_ACTS, f"head_norm_gate: gate function {gate_act!r} unknown (known: {sorted(GATE_ACTS)})")
+    if not (gate_act in GATE_ACTS):
+        raise KernelError(f"head_norm_gate: gate function {gate_act!r} unknown (known: {sorted(GATE_ACTS)})")
     if _backend is not None:
         if gate_act != "sigmoid":
             return _backend.head_norm_gate(o, weight, gate, eps, scale, heads, out, out_col0, gate_rows, gate_col0, gate_act)
@@ -2003,9 +2063,9 @@ def head_norm_gate(o: torch.Tensor, weight: torch.Tensor, gate: Optional[torch.T
     if gate_rows is not None:
         _need(gate_rows.dtype == torch.float32 and gate_rows.dim() == 2 and gate_rows.shape[0] == n and 0 <= gate_col0
               and gate_col0 + o.shape[1] <= gate_rows.shape[1], "head_norm_gate: bad gate rows")
-        gate_ptr, gate_stride, raw = ctypes.c_void_p(gate_rows.data_ptr() + 4 * int(gate_col0)), gate_rows.shape[1], GATE_ACTS[gate_act]
-    _call("tp_head_norm_gate", _ptr(o), _ptr(weight), gate_ptr, ctypes.c_float(eps), ctypes.c_float(scale), _ptr(out), _dt(out),
-          out.shape[1], int(out_col0), n, int(heads), vdim, per_head, ctypes.c_size_t(gate_stride), raw, _stream())
+        gate_ptr, gate_stride, raw = (gate_rows.data_ptr() + 4 * int(gate_col0)), gate_rows.shape[1], GATE_ACTS[gate_act]
+    _call("tp_head_norm_gate", _ptr(o), _ptr(weight), gate_ptr, float(eps), float(scale), _ptr(out), _dt(out),
+          out.shape[1], int(out_col0), n, int(heads), vdim, per_head, int(gate_stride), raw, _stream())
 
 
 def moe_plan(ids: torch.Tensor, experts: int):
@@ -2109,8 +2169,8 @@ def rmsnorm_cols(x: torch.Tensor, col0: int, width: int, weight: torch.Tensor, e
     _need(x.dtype == torch.float32 and x.dim() == 2 and 0 <= col0 and col0 + width <= x.shape[1], "rmsnorm_cols: bad rows")
     _need(weight.dtype == torch.float32 and weight.numel() == width and groups > 0 and width % groups == 0, "rmsnorm_cols: bad weight or groups")
     out = torch.empty((x.shape[0], width), dtype=out_dtype, device=x.device)
-    _call("tp_group_rmsnorm", _ptr(x), ctypes.c_size_t(x.shape[1]), int(col0), _ptr(weight), _ptr(None), _ptr(out), _dtcode(out_dtype),
-          x.shape[0], int(width), int(groups), ctypes.c_float(eps), _stream())
+    _call("tp_group_rmsnorm", _ptr(x), int(x.shape[1]), int(col0), _ptr(weight), _ptr(None), _ptr(out), _dtcode(out_dtype),
+          x.shape[0], int(width), int(groups), float(eps), _stream())
     return out
 
 
@@ -2137,7 +2197,7 @@ def residual_conv(x: torch.Tensor, weight: torch.Tensor, state: torch.Tensor, st
     _i32(state_slots, num_requests, "state_slots")
     _i32(token_req, n, "token_req") if n else None
     out = torch.empty((subs, n, width), dtype=out_dtype, device=x.device)
-    _call("tp_residual_conv", _ptr(x), _ptr(weight), _ptr(state), ctypes.c_size_t(0 if state is None else state.shape[1]), ctypes.c_size_t(state_off),
+    _call("tp_residual_conv", _ptr(x), _ptr(weight), _ptr(state), int(0 if state is None else state.shape[1]), int(state_off),
           _ptr(cu_seqlens), _ptr(token_req), _ptr(state_slots), _ptr(out), _dtcode(out_dtype), n, int(num_requests), width, taps, subs,
           int(max_run), sum(1 << i for i in blocked), _stream())
     return [KBlocked(out[i].view(width // 8, n, 8), n, width) if i in blocked else out[i] for i in range(subs)]
@@ -2166,8 +2226,8 @@ def norm_residual_conv(h: torch.Tensor, norm_weight: torch.Tensor, eps: float, g
     _i32(token_req, n, "token_req")
     _need(state_slots.dtype == torch.int32, "state_slots must be int32")
     out = torch.empty((subs, n, width), dtype=out_dtype, device=h.device)
-    _call("tp_norm_residual_conv", _ptr(h), _ptr(norm_weight), int(groups), ctypes.c_float(eps), _ptr(weight), _ptr(state),
-          ctypes.c_size_t(state.shape[1]), ctypes.c_size_t(state_off), _ptr(token_req), _ptr(state_slots), _ptr(out), _dtcode(out_dtype), n, width,
+    _call("tp_norm_residual_conv", _ptr(h), _ptr(norm_weight), int(groups), float(eps), _ptr(weight), _ptr(state),
+          int(state.shape[1]), int(state_off), _ptr(token_req), _ptr(state_slots), _ptr(out), _dtcode(out_dtype), n, width,
           taps, subs, sum(1 << i for i in blocked), _stream())
     return [KBlocked(out[i].view(width // 8, n, 8), n, width) if i in blocked else out[i] for i in range(subs)]
 
@@ -2179,7 +2239,7 @@ def add_row(h: torch.Tensor, table: torch.Tensor, row: int) -> None:
     _dev_ok(h, table)
     _need(h.dtype == torch.float32 and h.dim() == 2 and table.dtype == torch.float32 and table.dim() == 2 and table.shape[1] == h.shape[1]
           and 0 <= row < table.shape[0], "add_row: h float32 [n, width], table float32 [rows, width]")
-    _call("tp_add_row", _ptr(h), ctypes.c_void_p(table.data_ptr() + 4 * int(row) * table.shape[1]), h.shape[0], h.shape[1], _stream())
+    _call("tp_add_row", _ptr(h), (table.data_ptr() + 4 * int(row) * table.shape[1]), h.shape[0], h.shape[1], _stream())
 
 
 def general_delta_scan(proj: torch.Tensor, col0: int, decay: torch.Tensor, a_bias: torch.Tensor, state: torch.Tensor, state_off: int,
@@ -2203,9 +2263,9 @@ def general_delta_scan(proj: torch.Tensor, col0: int, decay: torch.Tensor, a_bia
     _i32(state_slots, num_requests, "state_slots")
     y = torch.empty((n, hd), dtype=torch.float32, device=proj.device)
     scratch = torch.empty((max(1, n * 2 * hd + n * heads * 2),), dtype=torch.float32, device=proj.device)
-    _call("tp_gdelta_scan", _ptr(proj), proj.shape[1], int(col0), _ptr(decay), _ptr(a_bias), _ptr(state), ctypes.c_size_t(state.shape[1]),
-          ctypes.c_size_t(state_off), _ptr(cu_seqlens), _ptr(state_slots), _ptr(y), _ptr(scratch), n, int(num_requests), int(heads),
-          int(dim), ctypes.c_float(unit_eps), _stream())
+    _call("tp_gdelta_scan", _ptr(proj), proj.shape[1], int(col0), _ptr(decay), _ptr(a_bias), _ptr(state), int(state.shape[1]),
+          int(state_off), _ptr(cu_seqlens), _ptr(state_slots), _ptr(y), _ptr(scratch), n, int(num_requests), int(heads),
+          int(dim), float(unit_eps), _stream())
     return y
 
 
@@ -2224,7 +2284,7 @@ def latent_rows(proj: torch.Tensor, q_col0: int, rot_col0: int, up: torch.Tensor
     _need(0 <= q_col0 and q_col0 + heads * (rot + dim) <= proj.shape[1] and 0 <= rot_col0 and rot_col0 + rot <= proj.shape[1]
           and up.shape[1] >= heads * (dim + vdim), "latent_rows: rows too short")
     out = torch.empty((n, 2 * heads * (rot + dim) + heads * vdim), dtype=torch.float32, device=proj.device)
-    _call("tp_latent_rows", _ptr(proj), ctypes.c_size_t(proj.shape[1]), int(q_col0), int(rot_col0), _ptr(up), ctypes.c_size_t(up.shape[1]),
+    _call("tp_latent_rows", _ptr(proj), int(proj.shape[1]), int(q_col0), int(rot_col0), _ptr(up), int(up.shape[1]),
           _ptr(out), n, int(heads), int(dim), int(rot), int(vdim), _stream())
     return out
 
@@ -2241,8 +2301,8 @@ def head_rmsnorm(rows: torch.Tensor, col_a: int, heads_a: int, weight_a: Optiona
     for col, heads, w in ((col_a, heads_a, weight_a), (col_b, heads_b, weight_b)):
         _need(heads >= 0 and col >= 0 and col + heads * dim <= rows.shape[1], "head_rmsnorm: heads outside the rows")
         _need(heads == 0 or (w is not None and w.dtype == torch.float32 and w.numel() == dim), "head_rmsnorm: weight must be float32 [dim]")
-    _call("tp_head_rmsnorm", _ptr(rows), ctypes.c_size_t(rows.shape[1]), int(col_a), int(heads_a), _ptr(weight_a), int(col_b), int(heads_b),
-          _ptr(weight_b), int(dim), ctypes.c_float(eps), rows.shape[0], _stream())
+    _call("tp_head_rmsnorm", _ptr(rows), int(rows.shape[1]), int(col_a), int(heads_a), _ptr(weight_a), int(col_b), int(heads_b),
+          _ptr(weight_b), int(dim), float(eps), rows.shape[0], _stream())
 
 
 def vector_store(c: torch.Tensor, slots: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor) -> None:
@@ -2282,8 +2342,8 @@ def latent_norms(rows: torch.Tensor, q_col0: int, q_dim: int, q_weight: torch.Te
     n = rows.shape[0]
     _i32(slots, n, "slots")
     cq = torch.empty((n, q_dim), dtype=k_cache.dtype, device=rows.device)
-    _call("tp_latent_norms", _ptr(rows), ctypes.c_size_t(rows.shape[1]), int(q_col0), int(q_dim), _ptr(q_weight), int(c_col0), int(c_dim),
-          _ptr(c_weight), ctypes.c_float(eps), _ptr(cq), _ptr(slots), _ptr(k_cache), _ptr(v_cache), _dt(k_cache), n, k_cache.shape[2], _stream())
+    _call("tp_latent_norms", _ptr(rows), int(rows.shape[1]), int(q_col0), int(q_dim), _ptr(q_weight), int(c_col0), int(c_dim),
+          _ptr(c_weight), float(eps), _ptr(cq), _ptr(slots), _ptr(k_cache), _ptr(v_cache), _dt(k_cache), n, k_cache.shape[2], _stream())
     return cq
 
 
@@ -2317,9 +2377,9 @@ def mlstm_scan(proj: torch.Tensor, col0: int, i_bias: torch.Tensor, f_bias: torc
     _i32(state_slots, num_requests, "state_slots")
     _need(out.dim() == 2 and out.shape[0] == n and 0 <= out_col0 and out_col0 + heads * vdim <= out.shape[1], "mlstm_scan: output rows too short")
     scratch = torch.empty((max(2, n * heads * (vdim + 4)),), dtype=torch.float32, device=proj.device)
-    _call("tp_mlstm_scan", _ptr(proj), proj.shape[1], int(col0), _ptr(i_bias), _ptr(f_bias), ctypes.c_float(cap), ctypes.c_float(q_scale),
-          _ptr(state), ctypes.c_size_t(state.shape[1]), ctypes.c_size_t(state_off), _ptr(cu_seqlens), _ptr(state_slots), _ptr(scratch),
-          _ptr(norm_weight), ctypes.c_float(eps), ctypes.c_float(scale), _ptr(out), _dt(out), out.shape[1], int(out_col0), n,
+    _call("tp_mlstm_scan", _ptr(proj), proj.shape[1], int(col0), _ptr(i_bias), _ptr(f_bias), float(cap), float(q_scale),
+          _ptr(state), int(state.shape[1]), int(state_off), _ptr(cu_seqlens), _ptr(state_slots), _ptr(scratch),
+          _ptr(norm_weight), float(eps), float(scale), _ptr(out), _dt(out), out.shape[1], int(out_col0), n,
           int(num_requests), int(heads), int(dim), int(vdim), _stream())
 
 
@@ -2346,7 +2406,7 @@ def token_shift(x: torch.Tensor, mu: torch.Tensor, state: torch.Tensor, state_of
     _i32(token_req, n, "token_req") if n else None
     mixes = mu.shape[0]
     out = torch.empty((mixes, width // 8, n, 8) if blocked else (mixes, n, width), dtype=out_dtype, device=x.device)
-    _call("tp_token_shift", _ptr(x), _ptr(mu), _ptr(state), ctypes.c_size_t(state.shape[1]), ctypes.c_size_t(state_off), _ptr(cu_seqlens),
+    _call("tp_token_shift", _ptr(x), _ptr(mu), _ptr(state), int(state.shape[1]), int(state_off), _ptr(cu_seqlens),
           _ptr(token_req), _ptr(state_slots), _ptr(out), _dtcode(out_dtype), n, int(num_requests), width, mixes, int(max_run == 1), int(blocked), _stream())
     return out if blocked else list(out.unbind(0))
 
@@ -2381,8 +2441,8 @@ def linear_scan(q, k, v, decay: torch.Tensor, state: torch.Tensor, state_off: in
     n = decay.shape[0]
     _dev_ok(q[0], k[0], v[0], decay, state, cu_seqlens, state_slots, bonus)
     for (rows, col), width, what in ((q, heads * dim, "q"), (k, heads * dim, "k"), (v, heads * vdim, "v")):
-        _need(rows.dtype == torch.float32 and rows.dim() == 2 and rows.shape[0] == n and 0 <= col and col + width <= rows.shape[1],
-              f"linear_scan: bad {what} rows")
+        if not (rows.dtype == torch.float32 and rows.dim() == 2 and rows.shape[0] == n and 0 <= col and col + width <= rows.shape[1]):
+            raise KernelError(f"linear_scan: bad {what} rows")
     _need(decay.dtype == torch.float32 and tuple(decay.shape) == (n, heads * dim), "linear_scan: decay must be float32 [n, heads * dim]")
     _need(bonus is None or (bonus.dtype == torch.float32 and bonus.numel() == heads * dim), "linear_scan: bonus must be float32 [heads * dim]")
     _need(state.dtype == torch.float32 and state.dim() == 2 and state_off >= 0 and state.shape[1] >= state_off + heads * dim * vdim,
@@ -2396,9 +2456,9 @@ def linear_scan(q, k, v, decay: torch.Tensor, state: torch.Tensor, state_off: in
         # (a request's pieces start at place cu_seqlens[r] // piece + r of the scratch)
         pieces = n // piece + num_requests
         scratch = torch.empty((pieces * heads * dim * (vdim + 1),), dtype=torch.float32, device=decay.device)
-    at = lambda rows: ctypes.c_void_p(rows[0].data_ptr() + 4 * int(rows[1]))
-    _call("tp_linear_scan", at(q), q[0].shape[1], at(k), k[0].shape[1], at(v), v[0].shape[1], _ptr(decay), _ptr(bonus), ctypes.c_float(q_scale),
-          _ptr(state), ctypes.c_size_t(state.shape[1]), ctypes.c_size_t(state_off), _ptr(cu_seqlens), _ptr(state_slots), _ptr(y), n,
+    at = lambda rows: (rows[0].data_ptr() + 4 * int(rows[1]))
+    _call("tp_linear_scan", at(q), q[0].shape[1], at(k), k[0].shape[1], at(v), v[0].shape[1], _ptr(decay), _ptr(bonus), float(q_scale),
+          _ptr(state), int(state.shape[1]), int(state_off), _ptr(cu_seqlens), _ptr(state_slots), _ptr(y), n,
           int(num_requests), int(heads), int(dim), int(vdim), max_run, piece, pieces, _ptr(scratch), _stream())
     return y
 
@@ -2427,8 +2487,9 @@ def mixer_step_ok(n: int, max_run: int, heads: int, dim: int, vdim: int, ranks, 
 
 
 def _step_state(n, state, token_req, state_slots, out, out_col0, columns, what):
-    _need(state.dtype == torch.float32 and state.dim() == 2 and out.dim() == 2 and out.shape[0] == n and 0 <= out_col0
-          and out_col0 + columns <= out.shape[1], f"{what}: bad state or output rows")
+    if not (state.dtype == torch.float32 and state.dim() == 2 and out.dim() == 2 and out.shape[0] == n and 0 <= out_col0
+            and out_col0 + columns <= out.shape[1]):
+        raise KernelError(f"{what}: bad state or output rows")
     _i32(token_req, n, "token_req")
     _i32(state_slots, n, "state_slots")
 
@@ -2455,11 +2516,11 @@ def delta_step(proj: torch.Tensor, col0: int, beta_col0: int, a_col0: int, g_col
     _need(conv_w.dtype == a2_t.dtype == g2_t.dtype == a_log.dtype == dt_bias.dtype == norm_w.dtype == torch.float32
           and conv_w.shape[1] == heads * (2 * dim + vdim) and a2_t.shape[1] == heads * dim and g2_t.shape[1] == heads * vdim
           and a_log.numel() == heads and dt_bias.numel() == heads * dim and norm_w.numel() == vdim, "delta_step: bad weights")
-    _call("tp_delta_step", _ptr(proj), ctypes.c_size_t(proj.shape[1]), int(col0), int(beta_col0), int(a_col0), a2_t.shape[0], int(g_col0),
+    _call("tp_delta_step", _ptr(proj), int(proj.shape[1]), int(col0), int(beta_col0), int(a_col0), a2_t.shape[0], int(g_col0),
           g2_t.shape[0], _ptr(conv_w), taps, _ptr(a2_t), _ptr(g2_t), _ptr(a_log), _ptr(dt_bias), _ptr(norm_w), _ptr(state),
-          ctypes.c_size_t(state.shape[1]), ctypes.c_size_t(conv_off), ctypes.c_size_t(state_off), _ptr(token_req), _ptr(state_slots), _ptr(out),
-          _dt(out), ctypes.c_size_t(out.shape[1]), int(out_col0), n, int(heads), int(dim), int(vdim), ctypes.c_float(q_scale),
-          ctypes.c_float(unit_eps), ctypes.c_float(norm_eps), ctypes.c_float(scale), prepared, _stream())
+          int(state.shape[1]), int(conv_off), int(state_off), _ptr(token_req), _ptr(state_slots), _ptr(out),
+          _dt(out), int(out.shape[1]), int(out_col0), n, int(heads), int(dim), int(vdim), float(q_scale),
+          float(unit_eps), float(norm_eps), float(scale), prepared, _stream())
 
 
 def general_delta_step(proj: torch.Tensor, col0: int, gate_col0: int, w_col0: int, w2_t: torch.Tensor, w0: torch.Tensor, rate: float,
@@ -2475,10 +2536,10 @@ def general_delta_step(proj: torch.Tensor, col0: int, gate_col0: int, w_col0: in
           and gate_col0 + hd <= proj.shape[1] and 0 <= w_col0 and w_col0 + w2_t.shape[0] <= proj.shape[1], "general_delta_step: bad projection rows")
     _need(w2_t.dtype == w0.dtype == a_bias.dtype == norm_w.dtype == torch.float32 and w2_t.shape[1] == hd and w0.numel() == hd
           and a_bias.numel() == hd and norm_w.numel() == hd, "general_delta_step: bad weights")
-    _call("tp_general_delta_step", _ptr(proj), ctypes.c_size_t(proj.shape[1]), int(col0), int(gate_col0), int(w_col0), w2_t.shape[0], _ptr(w2_t),
-          _ptr(w0), ctypes.c_float(rate), _ptr(a_bias), _ptr(norm_w), _ptr(state), ctypes.c_size_t(state.shape[1]), ctypes.c_size_t(state_off),
-          _ptr(token_req), _ptr(state_slots), _ptr(out), _dt(out), ctypes.c_size_t(out.shape[1]), int(out_col0), n, int(heads), int(dim),
-          ctypes.c_float(unit_eps), ctypes.c_float(norm_eps), ctypes.c_float(scale), _stream())
+    _call("tp_general_delta_step", _ptr(proj), int(proj.shape[1]), int(col0), int(gate_col0), int(w_col0), w2_t.shape[0], _ptr(w2_t),
+          _ptr(w0), float(rate), _ptr(a_bias), _ptr(norm_w), _ptr(state), int(state.shape[1]), int(state_off),
+          _ptr(token_req), _ptr(state_slots), _ptr(out), _dt(out), int(out.shape[1]), int(out_col0), n, int(heads), int(dim),
+          float(unit_eps), float(norm_eps), float(scale), _stream())
 
 
 def linear_step(q, k, v, x, w2_t: torch.Tensor, mode: str, bias: torch.Tensor, rate: float, in_act: Optional[str],
@@ -2494,18 +2555,18 @@ def linear_step(q, k, v, x, w2_t: torch.Tensor, mode: str, bias: torch.Tensor, r
     _step_state(n, state, token_req, state_slots, out, out_col0, heads * vdim, "linear_step")
     for (rows, col), width, what in ((q, heads * dim, "q"), (k, heads * dim, "k"), (v, heads * vdim, "v"), (x, w2_t.shape[0], "decay"),
                                      (gate, heads * vdim, "gate")):
-        _need(rows.dtype == torch.float32 and rows.dim() == 2 and rows.shape[0] == n and 0 <= col and col + width <= rows.shape[1],
-              f"linear_step: bad {what} rows")
+        if not (rows.dtype == torch.float32 and rows.dim() == 2 and rows.shape[0] == n and 0 <= col and col + width <= rows.shape[1]):
+            raise KernelError(f"linear_step: bad {what} rows")
     _need(w2_t.dtype == bias.dtype == norm_w.dtype == torch.float32 and w2_t.shape[1] == heads * dim and bias.numel() == heads * dim
           and norm_w.numel() in (vdim, heads * vdim) and (bonus is None or (bonus.dtype == torch.float32 and bonus.numel() == heads * dim)),
           "linear_step: bad weights")
-    at = lambda rows: ctypes.c_void_p(rows[0].data_ptr() + 4 * int(rows[1]))
-    wide = lambda rows: ctypes.c_size_t(rows[0].shape[1])
+    at = lambda rows: (rows[0].data_ptr() + 4 * int(rows[1]))
+    wide = lambda rows: int(rows[0].shape[1])
     _call("tp_linear_step", at(q), wide(q), at(k), wide(k), at(v), wide(v), at(x), wide(x), w2_t.shape[0], _ptr(w2_t), _ptr(bias),
-          LOWRANK_MODES[mode], 1 if in_act == "tanh" else 0, ctypes.c_float(rate), _ptr(bonus), ctypes.c_float(q_scale), at(gate), wide(gate),
-          GATE_ACTS["silu"], _ptr(norm_w), int(norm_w.numel() == heads * vdim and heads > 1), _ptr(state), ctypes.c_size_t(state.shape[1]),
-          ctypes.c_size_t(state_off), _ptr(token_req), _ptr(state_slots), _ptr(out), _dt(out), ctypes.c_size_t(out.shape[1]), int(out_col0), n,
-          int(heads), int(dim), int(vdim), ctypes.c_float(norm_eps), ctypes.c_float(scale), prepared, _stream())
+          LOWRANK_MODES[mode], 1 if in_act == "tanh" else 0, float(rate), _ptr(bonus), float(q_scale), at(gate), wide(gate),
+          GATE_ACTS["silu"], _ptr(norm_w), int(norm_w.numel() == heads * vdim and heads > 1), _ptr(state), int(state.shape[1]),
+          int(state_off), _ptr(token_req), _ptr(state_slots), _ptr(out), _dt(out), int(out.shape[1]), int(out_col0), n,
+          int(heads), int(dim), int(vdim), float(norm_eps), float(scale), prepared, _stream())
 
 
 # ---------------------------------------------------------------------------------
@@ -2581,7 +2642,7 @@ def moe_open(x: KBlocked, w_router, correction: Optional[torch.Tensor], experts:
         a = torch.empty((size // 8, m, 8), dtype=torch.bfloat16, device=dev)
         gate = torch.empty((m,), dtype=torch.float32, device=dev) if gated else None
     _call("tp_moe_open", _ptr(x.data), _ptr(w_router.data), _ptr(correction), _ptr(bias), int(experts), int(top), int(groups), int(keep), _ptr(dense),
-          _ptr(ids), _ptr(weights), m, k, ROUTE_SCORES[score], int(group_best), int(bool(normalize)), ctypes.c_float(sum_eps), ctypes.c_float(scale),
+          _ptr(ids), _ptr(weights), m, k, ROUTE_SCORES[score], int(group_best), int(bool(normalize)), float(sum_eps), float(scale),
           _ptr(None if w_shared is None else w_shared.data), 0 if w_shared is None else w_shared.shape[0], int(size), kind, _ptr(a), _ptr(gate), _stream())
     return dense, ids, weights, None if shared is None else (a, gate)
 

@@ -61,3 +61,23 @@ def test_few_blocks_or_short_streams_of_keys_take_the_projections_rows():
     pays = lambda n, longest, *rest: ops.attention_rows_pays(_step(n, longest), 8, *rest)
     assert pays(32, 100000, 128) and pays(64, 2000, 128) and not pays(64, 3000, 128) and pays(64, 3000, 64) and not pays(64, 5000, 64)
     assert pays(128, 500, 128) and not pays(128, 800, 128) and pays(128, 800, 64) and not pays(128, 1500, 64) and pays(64, 100000, 128, 1024)
+
+
+def test_entry_points_are_called_as_they_are_declared():
+    """Every call into the kernel library names an entry point of its sources and brings as many arguments as that has; a pointer, a size, a
+    number and a flag of one of them are declared as such."""
+    import ast
+    import ctypes
+    import inspect
+    from tempura_amd.kernels import ops
+    declared = ops.entry_points()
+    calls = [c for c in ast.walk(ast.parse(inspect.getsource(ops))) if isinstance(c, ast.Call) and getattr(c.func, "id", "") == "_call"]
+    names = [c.args[0].value for c in calls if isinstance(c.args[0], ast.Constant)]
+    assert len(names) > 50 and set(names) <= set(declared)
+    for c in calls:
+        if isinstance(c.args[0], ast.Constant) and not any(isinstance(a, ast.Starred) for a in c.args):
+            assert len(c.args) - 1 == len(declared[c.args[0].value][1]), c.args[0].value
+    result, args = declared["tp_linear_fused"]
+    assert result is ctypes.c_int and args[0] is args[-1] is ctypes.c_void_p and args[2] is ctypes.c_int
+    assert args[11] is ctypes.c_size_t and args[14] is ctypes.c_float
+    assert declared["tp_last_error"][0] is ctypes.c_char_p and declared["tp_linear_f32_scratch"][0] is ctypes.c_size_t

@@ -191,18 +191,22 @@ __device__ inline float block_sum(float v, float* scratch) {
   return t;
 }
 
-// The same for a block of T threads (64, or a multiple of 256) whose `scratch` (T / 64 floats, aligned to 16 bytes) no earlier sum has used: one barrier, and the
-// waves' sums in 16-byte reads side by side (sixteen dependent reads one after the other take longer than the barrier).
-template <int T>
-__device__ inline float block_sum_once(float v, float* scratch) {
-  static_assert(T == TP_WAVE || T % (4 * TP_WAVE) == 0, "one wave, or whole 16-byte pieces");
-  v = wave_sum(v);
-  if constexpr (T == TP_WAVE) return v;
-  if (threadIdx.x % TP_WAVE == 0) scratch[threadIdx.x / TP_WAVE] = v;
+// The same for a block of T threads whose `scratch` (S * T / 64 floats, aligned to 16 bytes) no earlier sum has used: one barrier, and the
+// waves' sums in 16-byte reads side by side (sixteen dependent reads one after the other take longer than the barrier).  Each thread brings S
+// values, which are added in the order in which a block of S * T threads adds one of each: the same bits.  (S * T: 64, or a multiple of 256.)
+template <int T, int S>
+__device__ inline float block_sum_once(const float (&v)[S], float* scratch) {
+  static_assert(T * S == TP_WAVE || T * S % (4 * TP_WAVE) == 0, "one wave, or whole 16-byte pieces");
+  if constexpr (T * S == TP_WAVE) return wave_sum(v[0]);
+#pragma unroll
+  for (int k = 0; k < S; ++k) {
+    const float sum = wave_sum(v[k]);
+    if (threadIdx.x % TP_WAVE == 0) scratch[k * (T / TP_WAVE) + threadIdx.x / TP_WAVE] = sum;
+  }
   __syncthreads();
   float4 t = *(const float4*)scratch;
 #pragma unroll
-  for (int i = 1; i < T / (4 * TP_WAVE); ++i) {
+  for (int i = 1; i < T * S / (4 * TP_WAVE); ++i) {
     const float4 u = ((const float4*)scratch)[i];
     t.x += u.x;
     t.y += u.y;
@@ -210,6 +214,12 @@ __device__ inline float block_sum_once(float v, float* scratch) {
     t.w += u.w;
   }
   return (t.x + t.y) + (t.z + t.w);
+}
+
+template <int T>
+__device__ inline float block_sum_once(float v, float* scratch) {
+  const float one[1] = {v};
+  return block_sum_once<T, 1>(one, scratch);
 }
 
 __device__ inline float block_max(float v, float* scratch) {

@@ -209,14 +209,16 @@ __global__ __launch_bounds__(256) void norm_add_kernel(float* __restrict__ h, co
 }
 
 // The same with the row in registers: every value is read once, sixteen bytes a load, all loads of a pass in flight
-// together (width a multiple of four, at most 256 * 4 * NV).  The sums are formed in the generic kernel's order of
-// a thread's own elements only where the widths agree; a row's result never depends on other rows either way.
-template <typename TO, int T, int NV, bool GATE>
+// together (width a multiple of four, at most 4 * T * NV).  S: the values a thread brings to a sum, 1 or NV; with NV the sums' order is that of
+// a block of NV * T threads, so a row's bits do not depend on how many rows there are.
+// Few rows wait for one request of all their operands and for the sums, so a thread has as little of a row as can be (one row of 4,096 in two
+// parts 4.14 -> 3.20 us against 256 threads that load in turn, with a gate 5.49 -> 3.73); many rows wait for memory.
+template <typename TO, int T, int NV, bool GATE, int S>
 __global__ __launch_bounds__(T) void norm_add_reg_kernel(float* __restrict__ h, const float* __restrict__ y,
                                                            const float* __restrict__ w, float eps,
                                                            const float* __restrict__ w_next, float eps_next,
                                                            TO* __restrict__ x, int width, InputGate gate, int normed, int blocked, int parts) {
-  __shared__ __attribute__((aligned(16))) float scratch[2][T / TP_WAVE];
+  __shared__ __attribute__((aligned(16))) float scratch[2][S * T / TP_WAVE];
   const size_t base = (size_t)blockIdx.x * width;
   const int w4 = width / 4;
   const size_t part = (size_t)gridDim.x * width;
@@ -265,19 +267,18 @@ __global__ __launch_bounds__(T) void norm_add_reg_kernel(float* __restrict__ h, 
   }
   float rstd = 1.0f;
   if (normed) {
-    float ss = 0.f;
+    float ss[S] = {};
 #pragma unroll
     for (int k = 0; k < NV; ++k)
       if (k * T + threadIdx.x < w4) {
-        ss = fmaf(yv[k].x, yv[k].x, ss);
-        ss = fmaf(yv[k].y, yv[k].y, ss);
-        ss = fmaf(yv[k].z, yv[k].z, ss);
-        ss = fmaf(yv[k].w, yv[k].w, ss);
+        ss[k % S] = fmaf(yv[k].x, yv[k].x, ss[k % S]);
+        ss[k % S] = fmaf(yv[k].y, yv[k].y, ss[k % S]);
+        ss[k % S] = fmaf(yv[k].z, yv[k].z, ss[k % S]);
+        ss[k % S] = fmaf(yv[k].w, yv[k].w, ss[k % S]);
       }
-    ss = block_sum_once<T>(ss, scratch[0]);
-    rstd = 1.0f / sqrtf(ss / (float)width + eps);
+    rstd = 1.0f / sqrtf(block_sum_once<T>(ss, scratch[0]) / (float)width + eps);
   }
-  float ss2 = 0.f;
+  float ss2[S] = {};
 #pragma unroll
   for (int k = 0; k < NV; ++k) {
     const int c = k * T + threadIdx.x;
@@ -287,15 +288,14 @@ __global__ __launch_bounds__(T) void norm_add_reg_kernel(float* __restrict__ h, 
       hv[k].z += yv[k].z * rstd * wv[k].z;
       hv[k].w += yv[k].w * rstd * wv[k].w;
       *(float4*)(h + base + 4 * c) = hv[k];
-      ss2 = fmaf(hv[k].x, hv[k].x, ss2);
-      ss2 = fmaf(hv[k].y, hv[k].y, ss2);
-      ss2 = fmaf(hv[k].z, hv[k].z, ss2);
-      ss2 = fmaf(hv[k].w, hv[k].w, ss2);
+      ss2[k % S] = fmaf(hv[k].x, hv[k].x, ss2[k % S]);
+      ss2[k % S] = fmaf(hv[k].y, hv[k].y, ss2[k % S]);
+      ss2[k % S] = fmaf(hv[k].z, hv[k].z, ss2[k % S]);
+      ss2[k % S] = fmaf(hv[k].w, hv[k].w, ss2[k % S]);
     }
   }
   if (w_next == nullptr) return;
-  ss2 = block_sum_once<T>(ss2, scratch[1]);
-  const float rstd2 = 1.0f / sqrtf(ss2 / (float)width + eps_next);
+  const float rstd2 = 1.0f / sqrtf(block_sum_once<T>(ss2, scratch[1]) / (float)width + eps_next);
 #pragma unroll
   for (int k = 0; k < NV; ++k) {
     const int c = k * T + threadIdx.x;
@@ -319,22 +319,28 @@ extern "C" int tp_norm_add(float* h, const float* y, const float* w, float eps, 
                        (gate_rows == nullptr || (((uintptr_t)gate_rows | (uintptr_t)gate_bias) % 16 == 0 && gate_stride % 4 == 0 && gate_col0 % 4 == 0));
   if (width % 4 == 0 && width >= 1024 && width <= 256 * 4 * 8 && aligned) {
     const bool bf = w_next != nullptr && x_dt == TP_BF16;
-#define NA1(TO, T, NV, G) \
-  hipLaunchKernelGGL((norm_add_reg_kernel<TO, T, NV, G>), dim3(n), dim3(T), 0, s, h, y, w, eps, w_next, eps_next, (TO*)x, width, gate, normed, blocked, parts)
-#define NA(T, NV)                                 \
-  do {                                            \
-    if (gate_rows != nullptr) {                   \
-      if (bf) NA1(bf16_t, T, NV, true);              \
-      else NA1(float, T, NV, true);                  \
-    } else {                                      \
-      if (bf) NA1(bf16_t, T, NV, false);             \
-      else NA1(float, T, NV, false);                 \
-    }                                             \
+#define NA1(TO, T, NV, G, S) \
+  hipLaunchKernelGGL((norm_add_reg_kernel<TO, T, NV, G, S>), dim3(n), dim3(T), 0, s, h, y, w, eps, w_next, eps_next, (TO*)x, width, gate, normed, blocked, parts)
+#define NA(T, NV, S)                      \
+  do {                                    \
+    if (gate_rows != nullptr) {           \
+      if (bf) NA1(bf16_t, T, NV, true, S);   \
+      else NA1(float, T, NV, true, S);       \
+    } else {                              \
+      if (bf) NA1(bf16_t, T, NV, false, S);  \
+      else NA1(float, T, NV, false, S);      \
+    }                                     \
   } while (0)
-    if (width <= 1024) NA(256, 1);
-    else if (width <= 2048) NA(512, 1);
-    else if (width <= 4096) NA(1024, 1);
-    else NA(1024, 2);
+    // A thread for every 16 bytes, and half as many where the CUs' 2,048 threads each no longer hold all rows (from 513 rows of 4,096, 1,025 of
+    // 2,048): more blocks then share a CU and hide one another's barriers.  Width 4,096, blocks of 1,024 / 512: 800 rows 10.7 / 10.2 us, 2,048 rows 25.7 /
+    // 23.7 (5.0 TB/s), with a gate 30.6 / 29.8, 5,000 rows 56.3 / 49.2 (5.8).  Width 2,048, blocks of 512 / 256: 2,048 rows 12.5 / 11.7, but of three parts
+    // 15.9 / 16.3.
+    if (width <= 1024) NA(256, 1, 1);
+    else if (width <= 2048 && n > 1024 && parts == 1) NA(256, 2, 2);
+    else if (width <= 2048) NA(512, 1, 1);
+    else if (width <= 4096 && n > 512) NA(512, 2, 2);
+    else if (width <= 4096) NA(1024, 1, 1);
+    else NA(1024, 2, 1);
 #undef NA
 #undef NA1
     TP_CHECK_LAUNCH("norm_add");

@@ -378,6 +378,29 @@ def test_norm_of_partial_sums(width):
     assert torch.equal(h0, h1) and torch.equal(a, b)
 
 
+@pytest.mark.parametrize("n, width, parts", [(1025, 1028, 1), (1025, 2048, 1), (513, 2052, 1), (513, 2052, 5), (513, 3000, 1), (513, 4096, 1), (513, 4096, 5)])
+def test_norm_of_many_rows(n, width, parts):
+    """Many rows (half as many threads a row) against the same rows a few at a time, bit by bit, and against float64."""
+    from tempura_amd.kernels import ops
+    g = torch.Generator().manual_seed(width + parts)
+    y, h, w = torch.randn(parts, n, width, generator=g).to(DEV), torch.randn(n, width, generator=g).to(DEV), torch.rand(width, generator=g).to(DEV)
+    gates = torch.randn(n, width, generator=g).to(DEV)
+    for gate in (None, gates):
+        def run(lo, hi, out):
+            data = y[:, lo:hi].contiguous()
+            more = dict(gate=gate[lo:hi], gate_col0=0, gate_bias=w) if gate is not None else {}
+            return ops.norm_add(out, ops.Partials(data) if parts > 1 else data[0], w, 1e-5, w, 1e-6, torch.float32, **more)
+        h0, h1, h2 = h.clone(), h[:300].clone(), h[300:].clone()
+        a, b, c = run(0, n, h0), run(0, 300, h1), run(300, n, h2)
+        assert torch.equal(h0, torch.cat([h1, h2])) and torch.equal(a, torch.cat([b, c]))
+        v = y.double().sum(0) * (1 if gate is None else torch.sigmoid(gate.double() + w.double()))
+        t = h.double() + v * torch.rsqrt(v.square().mean(1, keepdim=True) + 1e-5) * w.double()
+        ref = t * torch.rsqrt(t.square().mean(1, keepdim=True) + 1e-6) * w.double()
+        # (a value's own roundings, under twenty of 2^-24, of the largest value; the sums' relative error is smaller)
+        assert float((h0.double() - t).abs().max()) <= 2.0 ** -24 * 20 * float(t.abs().max())
+        assert float((a.double() - ref).abs().max()) <= 2.0 ** -24 * 20 * float(ref.abs().max())
+
+
 @pytest.mark.parametrize("m,experts", [(1, 8), (4, 8), (16, 3)])
 @pytest.mark.parametrize("ff,n,parts", [(2048, 96, 2), (4096, 1024, 4), (2112, 96, 1), (2048, 2064, 1)])
 @pytest.mark.parametrize("size", [0, 512])

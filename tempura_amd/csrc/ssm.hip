@@ -874,6 +874,7 @@ __global__ void gated_group_norm_kernel(const float* __restrict__ y, const float
 }
 
 // The same with a part of at most 4,096 in registers, a thread four neighbouring columns, all loads in front of the sum.
+// 8,192 columns in eight parts, against loads of four bytes: one row 3.30 -> 2.27 us, 2,048 rows 50.5 -> 30.7 (5.4 TB/s).
 template <typename TO, int T>
 __global__ __launch_bounds__(T) void gated_group_norm4_kernel(const float* __restrict__ y, const float* __restrict__ proj, int proj_stride,
                                                                  int z_col0, const float* __restrict__ w, float eps, TO* __restrict__ out,

@@ -68,16 +68,37 @@ def test_float32_products_in_blocks_of_128_and_64(small, large, n, k, parts):
     assert torch.equal(ops.linear(few, w, torch.float32, residual=res[:small].clone()), added[:small])
 
 
-# rows and columns at the edges of a block of 128 and of the 16 x 16 tiles; K: whole stages of 32, an odd number of them, a part of one; in parts
-@pytest.mark.parametrize("m,n,k,parts", [(65, 4097, 1536, 6), (128, 4100, 1540, 6), (129, 2050, 1572, 6), (255, 4096, 1568, 4), (300, 3072, 3072, 3),
-                                         (640, 6500, 1600, 1), (700, 5200, 1536, 1)])
-def test_float32_products_in_pieces(m, n, k, parts):
-    """Operands in bfloat16 pieces, plain and added into rows, against float64 with the bound of the products above: of normal operands, of operands
-    over twelve orders of magnitude, of positive ones, and of tiny ones; the same call gives the same bits; a row's bits are the same when rows are
-    added up to the next whole block of 128."""
+# rows and columns at the edges of the blocks, K: whole stages of 32, an odd number of them, a part of one
+@pytest.mark.parametrize("m,n,k", [(17, 70, 132), (64, 512, 2048), (65, 4097, 1536), (129, 2050, 1572), (300, 3072, 3072), (700, 5200, 1536)])
+def test_float32_products_keep_every_bit(m, n, k):
+    """A sum of one term is the correctly rounded product, whatever the operands' size: ordinary ones, small ones (down to those below the
+    smallest normal number) beside large ones, infinity beside the smallest weights.  (Nothing but that term is rounded: added zeros are exact.)"""
     from tempura_amd.kernels import ops
-    lib = ops.library()
-    assert lib.tp_linear_f32_block(m, n, k) == 128 and lib.tp_linear_f32_scratch(m, n, k) == (parts * m * n if parts > 1 else 0)
+    g = torch.Generator().manual_seed(m + n + k)
+    rows, at = torch.arange(m), torch.randint(0, k, (m,), generator=g)
+    value, w = torch.randn(m, generator=g), torch.randn(n, k, generator=g)
+    value = torch.copysign(value.abs().clamp(2.0 ** -3, 4.0), value)
+    w = torch.copysign(w.abs().clamp(2.0 ** -6, 8.0), w)
+    for low, high in ((0, 0), (-60, 40), (-112, 90), (-118, 110), (-123, 110)):
+        for ex, ew in ((low, high), (high, low)):
+            x, b = torch.zeros(m, k), w * 2.0 ** ew
+            x[rows, at] = value * 2.0 ** ex
+            want = (x[rows, at].double()[:, None] * b[:, at].double().T).float()
+            assert torch.isfinite(want).all() and torch.equal(ops.linear(x.to(DEV), b.to(DEV), torch.float32).cpu(), want)
+    x = torch.zeros(m, k)
+    x[rows, at] = math.inf * torch.sign(value)
+    b = torch.sign(w) * 2.0 ** -140
+    got = ops.linear(x.to(DEV), b.to(DEV), torch.float32).cpu()
+    assert torch.equal(got, math.inf * torch.sign(value)[:, None] * torch.sign(b[:, at].T))
+
+
+@pytest.mark.parametrize("m,n,k", [(65, 4097, 1536), (128, 4100, 1540), (129, 2050, 1572), (255, 4096, 1568), (300, 3072, 3072), (640, 6500, 1600),
+                                   (700, 5200, 1536)])
+def test_float32_products_of_many_kinds(m, n, k):
+    """Plain and added into rows, against float64 with the bound of the products above: of normal operands, of operands over twelve orders of magnitude,
+    of positive ones, and of tiny ones; the same call gives the same bits; a row's bits are the same when rows are added up to the next whole
+    block of 128."""
+    from tempura_amd.kernels import ops
     g = torch.Generator().manual_seed(m + n + k)
     x, w, res = (torch.randn(*s, generator=g).to(DEV) for s in ((m, k), (n, k), (m, n)))
     tol = 2.0 ** -24 * math.sqrt(k)
@@ -93,9 +114,9 @@ def test_float32_products_in_pieces(m, n, k, parts):
     assert torch.equal(ops.linear(padded, w, torch.float32)[:m], got)
 
 
-def test_float32_products_in_pieces_of_extreme_values():
-    """Infinity, NaN and the largest finite values give what the products of whole operands give: infinity of the sign of the factor beside it,
-    NaN for infinity times zero, and finite results of values that bfloat16 would round to infinity."""
+def test_float32_products_of_extreme_values():
+    """Infinity, NaN and the largest finite values: infinity of the sign of the factor beside it, NaN for infinity times zero, and finite
+    results of values that bfloat16 would round to infinity."""
     from tempura_amd.kernels import ops
     m, n, k = 256, 4096, 1536
     g = torch.Generator().manual_seed(5)
@@ -107,7 +128,6 @@ def test_float32_products_in_pieces_of_extreme_values():
     x[4], x[5] = 0.0, 0.0
     x[4, 11], x[5, 12] = top, -top
     w[:, 11], w[:, 12] = 0.25, 0.5
-    assert ops.library().tp_linear_f32_block(m, n, k) == 128
     got = ops.linear(x.to(DEV), w.to(DEV), torch.float32).cpu()
     ref = x.double() @ w.double().T
     odd = ~torch.isfinite(ref)

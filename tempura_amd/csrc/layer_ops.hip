@@ -213,7 +213,8 @@ __global__ __launch_bounds__(256) void norm_add_kernel(float* __restrict__ h, co
 // a block of NV * T threads, so a row's bits do not depend on how many rows there are.
 // Few rows wait for one request of all their operands and for the sums, so a thread has as little of a row as can be (one row of 4,096 in two
 // parts 4.14 -> 3.20 us against 256 threads that load in turn, with a gate 5.49 -> 3.73); many rows wait for memory.
-template <typename TO, int T, int NV, bool GATE, int S>
+// LATE: further parts, the gate and the next norm's weight are requested where they are used, so that fewer registers leave room for more rows.
+template <typename TO, int T, int NV, bool GATE, int S, bool LATE>
 __global__ __launch_bounds__(T) void norm_add_reg_kernel(float* __restrict__ h, const float* __restrict__ y,
                                                            const float* __restrict__ w, float eps,
                                                            const float* __restrict__ w_next, float eps_next,
@@ -224,22 +225,30 @@ __global__ __launch_bounds__(T) void norm_add_reg_kernel(float* __restrict__ h, 
   const size_t part = (size_t)gridDim.x * width;
   const float* gr = GATE ? gate.rows + (size_t)blockIdx.x * gate.stride + gate.col0 : nullptr;
   float4 yv[NV], y1[NV], y2[NV], y3[NV], hv[NV], wv[NV], gv[GATE ? NV : 1], bv[GATE ? NV : 1], nv[NV];
+  auto fetch_gate = [&](int k) {
+    const int c = k * T + threadIdx.x;
+    if (c < w4) {
+      gv[k] = *(const float4*)(gr + 4 * c);
+      bv[k] = gate.bias != nullptr ? *(const float4*)(gate.bias + 4 * c) : make_float4(0.f, 0.f, 0.f, 0.f);
+    }
+  };
+  auto fetch_next = [&](int k) {
+    const int c = k * T + threadIdx.x;
+    if (c < w4) nv[k] = *(const float4*)(w_next + 4 * c);
+  };
 #pragma unroll
   for (int k = 0; k < NV; ++k) {
     const int c = k * T + threadIdx.x;
     if (c < w4) {
       const float* yp = y + base + 4 * c;
       yv[k] = *(const float4*)yp;
-      if (parts > 1) y1[k] = *(const float4*)(yp + part);
-      if (parts > 2) y2[k] = *(const float4*)(yp + 2 * part);
-      if (parts > 3) y3[k] = *(const float4*)(yp + 3 * part);
-      if constexpr (GATE) {
-        gv[k] = *(const float4*)(gr + 4 * c);
-        bv[k] = gate.bias != nullptr ? *(const float4*)(gate.bias + 4 * c) : make_float4(0.f, 0.f, 0.f, 0.f);
-      }
+      if (!LATE && parts > 1) y1[k] = *(const float4*)(yp + part);
+      if (!LATE && parts > 2) y2[k] = *(const float4*)(yp + 2 * part);
+      if (!LATE && parts > 3) y3[k] = *(const float4*)(yp + 3 * part);
+      if constexpr (GATE && !LATE) fetch_gate(k);
       hv[k] = *(const float4*)(h + base + 4 * c);
       wv[k] = *(const float4*)(w + 4 * c);
-      if (w_next != nullptr) nv[k] = *(const float4*)(w_next + 4 * c);
+      if (!LATE && w_next != nullptr) fetch_next(k);
     }
   }
   // (parts > 1: y is that many partial sums of a product, added in ascending order)
@@ -249,14 +258,28 @@ __global__ __launch_bounds__(T) void norm_add_reg_kernel(float* __restrict__ h, 
     a.z += b.z;
     a.w += b.w;
   };
+  if constexpr (LATE) {
+    for (int p = 1; p < parts; ++p) {
+#pragma unroll
+      for (int k = 0; k < NV; ++k)
+        if (k * T + threadIdx.x < w4) y1[k] = *(const float4*)(y + p * part + base + 4 * (k * T + threadIdx.x));
+#pragma unroll
+      for (int k = 0; k < NV; ++k)
+        if (k * T + threadIdx.x < w4) add(yv[k], y1[k]);
+    }
+    if constexpr (GATE) {
+#pragma unroll
+      for (int k = 0; k < NV; ++k) fetch_gate(k);
+    }
+  }
 #pragma unroll
   for (int k = 0; k < NV; ++k) {
     const int c = k * T + threadIdx.x;
     if (c < w4) {
-      if (parts > 1) add(yv[k], y1[k]);
-      if (parts > 2) add(yv[k], y2[k]);
-      if (parts > 3) add(yv[k], y3[k]);
-      for (int p = 4; p < parts; ++p) add(yv[k], *(const float4*)(y + p * part + base + 4 * c));
+      if (!LATE && parts > 1) add(yv[k], y1[k]);
+      if (!LATE && parts > 2) add(yv[k], y2[k]);
+      if (!LATE && parts > 3) add(yv[k], y3[k]);
+      for (int p = LATE ? parts : 4; p < parts; ++p) add(yv[k], *(const float4*)(y + p * part + base + 4 * c));
       if constexpr (GATE) {
         yv[k].x *= l_sigmoid(gv[k].x + bv[k].x);
         yv[k].y *= l_sigmoid(gv[k].y + bv[k].y);
@@ -295,6 +318,10 @@ __global__ __launch_bounds__(T) void norm_add_reg_kernel(float* __restrict__ h, 
     }
   }
   if (w_next == nullptr) return;
+  if constexpr (LATE) {
+#pragma unroll
+    for (int k = 0; k < NV; ++k) fetch_next(k);
+  }
   const float rstd2 = 1.0f / sqrtf(block_sum_once<T>(ss2, scratch[1]) / (float)width + eps_next);
 #pragma unroll
   for (int k = 0; k < NV; ++k) {
@@ -319,28 +346,34 @@ extern "C" int tp_norm_add(float* h, const float* y, const float* w, float eps, 
                        (gate_rows == nullptr || (((uintptr_t)gate_rows | (uintptr_t)gate_bias) % 16 == 0 && gate_stride % 4 == 0 && gate_col0 % 4 == 0));
   if (width % 4 == 0 && width >= 1024 && width <= 256 * 4 * 8 && aligned) {
     const bool bf = w_next != nullptr && x_dt == TP_BF16;
-#define NA1(TO, T, NV, G, S) \
-  hipLaunchKernelGGL((norm_add_reg_kernel<TO, T, NV, G, S>), dim3(n), dim3(T), 0, s, h, y, w, eps, w_next, eps_next, (TO*)x, width, gate, normed, blocked, parts)
-#define NA(T, NV, S)                      \
-  do {                                    \
-    if (gate_rows != nullptr) {           \
-      if (bf) NA1(bf16_t, T, NV, true, S);   \
-      else NA1(float, T, NV, true, S);       \
-    } else {                              \
-      if (bf) NA1(bf16_t, T, NV, false, S);  \
-      else NA1(float, T, NV, false, S);      \
-    }                                     \
+#define NA1(TO, T, NV, G, S, L) \
+  hipLaunchKernelGGL((norm_add_reg_kernel<TO, T, NV, G, S, L>), dim3(n), dim3(T), 0, s, h, y, w, eps, w_next, eps_next, (TO*)x, width, gate, normed, blocked, parts)
+#define NA(T, NV, S, L)                      \
+  do {                                       \
+    if (gate_rows != nullptr) {              \
+      if (bf) NA1(bf16_t, T, NV, true, S, L);   \
+      else NA1(float, T, NV, true, S, L);       \
+    } else {                                 \
+      if (bf) NA1(bf16_t, T, NV, false, S, L);  \
+      else NA1(float, T, NV, false, S, L);      \
+    }                                        \
   } while (0)
     // A thread for every 16 bytes, and half as many where the CUs' 2,048 threads each no longer hold all rows (from 513 rows of 4,096, 1,025 of
     // 2,048): more blocks then share a CU and hide one another's barriers.  Width 4,096, blocks of 1,024 / 512: 800 rows 10.7 / 10.2 us, 2,048 rows 25.7 /
-    // 23.7 (5.0 TB/s), with a gate 30.6 / 29.8, 5,000 rows 56.3 / 49.2 (5.8).  Width 2,048, blocks of 512 / 256: 2,048 rows 12.5 / 11.7, but of three parts
-    // 15.9 / 16.3.
-    if (width <= 1024) NA(256, 1, 1);
-    else if (width <= 2048 && n > 1024 && parts == 1) NA(256, 2, 2);
-    else if (width <= 2048) NA(512, 1, 1);
-    else if (width <= 4096 && n > 512) NA(512, 2, 2);
-    else if (width <= 4096) NA(1024, 1, 1);
-    else NA(1024, 2, 1);
+    // 23.7 (5.0 TB/s), with a gate 30.6 / 29.8.  Width 2,048, blocks of 512 / 256: 2,048 rows 12.5 / 11.7, but of three parts 15.9 / 16.3.
+    // Still more rows of one part wait for memory alone, and what they request is better spread out (LATE).  All operands in front / gate and next weight late,
+    // with a gate: 10,000 rows of 1,280 43.4 / 39.2 us, of 1,536 49.6 / 46.9 (2,048 rows 12.1 / 12.3); 5,000 rows of 2,560 46.6 / 42.7 (800 rows 9.8 /
+    // 10.4), of 4,096 68.2 / 67.5; 2,048 rows of 5,120 (1,024 x 2 threads in front) 44.2 / 35.4, without a gate 30.7 / 29.3.  Beyond 6,144 columns
+    // rows without a gate lose: 1,100 of 8,192 27.9 / 29.3.
+    if (width <= 1024) NA(256, 1, 1, false);
+    else if (width <= 2048 && n > 2048 && parts == 1) NA(256, 2, 2, true);
+    else if (width <= 2048 && n > 1024 && parts == 1) NA(256, 2, 2, false);
+    else if (width <= 2048) NA(512, 1, 1, false);
+    else if (width <= 4096 && n > 1024 && parts == 1) NA(512, 2, 2, true);
+    else if (width <= 4096 && n > 512) NA(512, 2, 2, false);
+    else if (width <= 4096) NA(1024, 1, 1, false);
+    else if (width <= 6144 && n > 512 && parts == 1) NA(512, 3, 2, true);
+    else NA(1024, 2, 1, false);
 #undef NA
 #undef NA1
     TP_CHECK_LAUNCH("norm_add");

@@ -378,9 +378,11 @@ def test_norm_of_partial_sums(width):
     assert torch.equal(h0, h1) and torch.equal(a, b)
 
 
-@pytest.mark.parametrize("n, width, parts", [(1025, 1028, 1), (1025, 2048, 1), (513, 2052, 1), (513, 2052, 5), (513, 3000, 1), (513, 4096, 1), (513, 4096, 5)])
+@pytest.mark.parametrize("n, width, parts", [(1025, 1028, 1), (1025, 2048, 1), (513, 2052, 1), (513, 2052, 5), (513, 3000, 1), (513, 4096, 1), (513, 4096, 5),
+                                             (2049, 1028, 1), (2049, 2048, 1), (1025, 2052, 1), (1025, 4096, 1), (513, 4100, 1), (513, 6144, 1), (513, 6144, 3),
+                                             (513, 6148, 1)])
 def test_norm_of_many_rows(n, width, parts):
-    """Many rows (half as many threads a row) against the same rows a few at a time, bit by bit, and against float64."""
+    """Many rows (half as many threads a row, the gate and the next weight late) against the same rows a few at a time, bit by bit, and against float64."""
     from tempura_amd.kernels import ops
     g = torch.Generator().manual_seed(width + parts)
     y, h, w = torch.randn(parts, n, width, generator=g).to(DEV), torch.randn(n, width, generator=g).to(DEV), torch.rand(width, generator=g).to(DEV)

@@ -278,6 +278,24 @@ def test_gated_group_norm(inner, groups, out_dtype):
     _close(got, emu.gated_group_norm(y, proj, 5, w, 1e-5, groups, out_dtype), 2e-6 if out_dtype == torch.float32 else 1e-2)
 
 
+@pytest.mark.parametrize("part", [4, 60, 64, 68, 256, 260, 1024, 1028, 2048, 2052, 4096, 4100])
+@pytest.mark.parametrize("out_dtype", [torch.float32, torch.bfloat16])
+def test_gated_group_norm_of_every_part(part, out_dtype):
+    """Parts at the edges of the blocks of threads, gates at columns and strides of whole 16-byte pieces and of others, against float64: under twenty
+    roundings of 2^-24 of the largest value, and of bfloat16 results half a unit of their last place more."""
+    ops = _ops()
+    for groups, n, col0, more in ((1, 1, 0, 0), (3, 5, 4, 8), (2, 3, 0, 4), (3, 4, 5, 2), (2, 2, 4, 1)):
+        inner = groups * part
+        g = torch.Generator().manual_seed(part + col0)
+        y, proj, w = torch.randn(n, inner, generator=g), torch.randn(n, col0 + inner + more, generator=g), torch.randn(inner, generator=g)
+        got = ops.gated_group_norm(y.to(DEV), proj.to(DEV), col0, w.to(DEV), 1e-5, groups, out_dtype).double().cpu()
+        z = proj[:, col0: col0 + inner].double()
+        v = (y.double() * z * torch.sigmoid(z)).view(n, groups, part)
+        want = (v * torch.rsqrt(v.square().mean(2, keepdim=True) + 1e-5)).view(n, inner) * w.double()
+        off = (got - want).abs() - (want.abs() * 2.0 ** -8 if out_dtype == torch.bfloat16 else 0.0)
+        assert float(off.max()) <= 2.0 ** -24 * 20 * float(want.abs().max()), (groups, n, col0, more)
+
+
 # ---- the model through the step function --------------------------------------------------------
 def _runner(dirs, name, dtype, max_tokens, page_size=16, max_requests=4, use_graph=False):
     from tempura_amd.engine.loading import load_model

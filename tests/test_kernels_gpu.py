@@ -55,6 +55,19 @@ def test_rmsnorm(out_dtype, n, hidden, eps):
     _close(got, emu.rmsnorm(x, w, eps, torch.float64, rows), _tol(out_dtype), "rmsnorm rows")
 
 
+@pytest.mark.parametrize("n,hidden", [(4097, 4), (4097, 256), (4097, 260), (4097, 512), (16385, 516), (16385, 1024), (3, 8192), (3, 8196), (3, 12288), (2, 16384),
+                                      (2, 16388)])
+def test_rmsnorm_of_many_and_of_long_rows(n, hidden):
+    """The bits of the same rows a few at a time, and float64 within the roundings of a value (twenty of 2^-24 of the largest)."""
+    ops = _ops()
+    g = torch.Generator().manual_seed(hidden)
+    x, w = torch.randn(n, hidden, generator=g).to(DEV), torch.randn(hidden, generator=g).to(DEV)
+    got = ops.rmsnorm(x, w, 1e-5, torch.float32)
+    assert torch.equal(got[-2:], ops.rmsnorm(x[-2:].contiguous(), w, 1e-5, torch.float32))
+    want = x.double() * torch.rsqrt(x.double().square().mean(1, keepdim=True) + 1e-5) * w.double()
+    assert float((got.double() - want).abs().max()) <= 2.0 ** -24 * 20 * float(want.abs().max())
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("m,n,k", [(1, 16, 8), (4, 32, 16), (8, 64, 64), (1, 1024, 512), (3, 96, 320), (9, 12, 96),
                                    (17, 100, 36), (64, 384, 96), (65, 130, 70), (130, 257, 129), (2, 301, 1000)])

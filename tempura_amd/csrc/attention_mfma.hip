@@ -1889,8 +1889,11 @@ static int launch_all(AttnArgs a, int n_tokens, int n_req, int max_q_len, int nu
     // single tokens beside portions: one launch where the portions take 16 query rows a wave whole (see below) and make no more
     // than about 800 blocks; beyond, three blocks a CU instead of two are worth more to them.  24 heads in 8 groups, two launches / one: 700 rows beside
     // 4 / 16 / 40 requests of 900 keys 34.3 / 39.4 / 56.0 against 26.2 / 24.8 / 34.3 us, 1,600 rows 60.6 / 69.3 / 89.1 against 55.7 / 63.2 /
-    // 75.6, 2,000 rows 72.4 / 82.2 / 107.5 against 76.8 / 83.6 / 94.6.  More than 256 blocks of single tokens fill the chip alone; the portions
-    // then come first (48 requests of 3,000 keys beside 700 rows 135.5 / 135.4).
+    // 75.6, 2,000 rows 72.4 / 82.2 / 107.5 against 76.8 / 83.6 / 94.6.  Where somebody sees 2,048 keys or more the portions' keys are split (two
+    // launches), so only kept first keys, with which they never are, bring long keys here: 32 heads in 8 groups of 64, 32 requests of 8,000 keys beside
+    // 700 / 1,100 rows 102.5 / 115.1 against 89.6 / 91.1.
+    // More than 256 blocks of single tokens with few keys fill the chip alone, and the portions come first (64 requests of 1,500 keys beside 700 rows 47.3 ->
+    // 42.7, in two launches 54.0); with many keys the single tokens are what everything waits for (those of 8,000 above: 124.8 / 132.2 behind the portions).
     const int kv_groups = a.n_kv * ((group + 3) / 4), portions = n_req - num_single;
     const long blocks2 = (long)((n_tokens - num_single + 31) / 32 + (portions - 1)) * kv_groups;
     if (num_single > 0 && has_multi && !bias && g_attn_tune == 0 && a.page_shift >= 4 && a.page_size >= 512 / D && blocks2 <= 400 &&
@@ -1903,7 +1906,7 @@ static int launch_all(AttnArgs a, int n_tokens, int n_req, int max_q_len, int nu
       const long single = (long)a.n_kv * ((group + 15) / 16) * n_req * a.num_splits, most = (long)gx * gy * portions;
       if (single + most < 0x7fffffffL) {
         hipLaunchKernelGGL((attn_both_kernel<D, DV, MODE, NB>), dim3((unsigned)(single + most)), dim3(256), 0, s, a, n_req, (int)single,
-                           single > 256 ? (int)most : 0, gx, gy);
+                           single > 256 && a.keep_first == 0 ? (int)most : 0, gx, gy);
         if (a.num_splits > 1) launch_combine(a, n_req, DV, s);
         return 0;
       }

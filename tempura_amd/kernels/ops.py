@@ -41,7 +41,7 @@ def entry_points() -> dict:
     from ..csrc.build import sources
     out = {}
     for path in sources():
-        with open(path) as f:
+        with open(path, encoding="utf-8") as f:
             text = re.sub(r"//[^\n]*", "", f.read())
         for result, name, args in re.findall(r'extern "C"\s+([\w\s]+?[\s\*]+)(tp_\w+)\s*\(([^)]*)\)\s*\{', text):
             result = " ".join(result.split())

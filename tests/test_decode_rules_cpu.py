@@ -81,3 +81,42 @@ def test_entry_points_are_called_as_they_are_declared():
     assert result is ctypes.c_int and args[0] is args[-1] is ctypes.c_void_p and args[2] is ctypes.c_int
     assert args[11] is ctypes.c_size_t and args[14] is ctypes.c_float
     assert declared["tp_last_error"][0] is ctypes.c_char_p and declared["tp_linear_f32_scratch"][0] is ctypes.c_size_t
+
+
+def test_every_argument_of_a_call_has_the_declared_type():
+    """No definition in the sources is overlooked, and each argument whose kind shows in the call (an address, a float, a whole number), those that come
+    as a row scale's or a split norm's three included, stands where one of that kind is declared."""
+    import ast
+    import ctypes
+    import inspect
+    import re
+    from tempura_amd.csrc.build import sources
+    from tempura_amd.kernels import ops
+    declared = ops.entry_points()
+    assert sum(len(re.findall(r'^extern "C"', open(p, encoding="utf-8").read(), re.M)) for p in sources()) == len(declared)
+    address, number = {ctypes.c_void_p}, {ctypes.c_float, ctypes.c_double}
+    whole = {ctypes.c_int, ctypes.c_uint, ctypes.c_size_t, ctypes.c_long, ctypes.c_longlong, ctypes.c_ulonglong}
+    kinds = {"_ptr": address, "_stream": address, "at": address, "byref": address, "float": number, "c_float": number, "c_double": number, "int": whole,
+             "len": whole, "max": whole, "min": whole, "_dt": whole, "_dtcode": whole, "c_size_t": whole, "c_longlong": whole, "c_ulonglong": whole}
+    starred = {"pre": [address, whole, number], "post": [address, address, address]}
+
+    def kind_of(arg):
+        if "data_ptr" in ast.dump(arg):
+            return address
+        if isinstance(arg, ast.Constant) and arg.value is not None:
+            return number if isinstance(arg.value, float) else whole
+        return kinds.get(getattr(arg.func, "id", getattr(arg.func, "attr", ""))) if isinstance(arg, ast.Call) else None
+
+    seen = 0
+    for c in ast.walk(ast.parse(inspect.getsource(ops))):
+        if not (isinstance(c, ast.Call) and getattr(c.func, "id", "") == "_call" and isinstance(c.args[0], ast.Constant)):
+            continue
+        name, got = c.args[0].value, []
+        for a in c.args[1:]:
+            got += starred[a.value.id] if isinstance(a, ast.Starred) else [kind_of(a)]
+        types = declared[name][1]
+        assert len(got) == len(types), name
+        for i, (kind, want) in enumerate(zip(got, types)):
+            assert kind is None or want in kind, (name, i, want)
+            seen += kind is not None
+    assert seen > 600

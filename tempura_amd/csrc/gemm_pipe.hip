@@ -1524,9 +1524,65 @@ extern "C" int tp_moe_linear(const void* x, const void* w, int w_tiled, void* ou
   return 0;
 }
 
+int g_pipe_big = 0;   // tuning: 1 = 256 x 256 tiles for every whole block of 256 columns, 2 = never; 3 = 256 x 192 wherever N allows, 4 = never; 5 = 192 x 256 wherever N allows
+
+// The larger tiles of a product in one part of K (see gemm_pipe_big_kernel).  head_dim: of the rotating epilogue (0: another one).
+struct BigTiles {
+  int nb_big;    // so many blocks of 256 columns take 256 x 256, the columns that are left 256 x 128
+  bool low;      // all columns take 192 x 256
+  bool narrow;   // all columns take 256 x 192
+};
+
+static BigTiles big_tiles(int M, int N, int mode, int head_dim) {
+  BigTiles t = {0, false, false};
+  const int MB = (M + BM - 1) / BM, ldo = mode == OUT_SWIGLU ? N / 2 : N;
+  // (with the rotating epilogue a wave's 128 columns of a big tile have to lie inside one of q, k and v: heads
+  // of a multiple of 128; the strips of the 192-column tile are ordered for heads of 128)
+  if (g_pipe_big == 2 || ldo % 4 != 0 || head_dim % 128 != 0) return t;
+  // How many blocks of 256 columns take the big tiles: all, none, or whole rounds of 256 tiles, whichever
+  // needs the fewest rounds when a big tile is priced at 1.72 small ones (measured: 113 against 65 us at
+  // K = 4096).
+  const long NB2 = N / BNB;
+  auto rounds = [&](long nb) {
+    const long rest = (N - nb * BNB + BN - 1) / BN;
+    return 1.72 * (double)((MB * nb + 255) / 256) + (double)((MB * rest + 255) / 256);
+  };
+  const long whole = ((long)MB * NB2 / 256) * 256 / MB;
+  double best = rounds(0);
+  for (long cand : {NB2, whole})
+    if (cand > 0 && rounds(cand) < best - 1e-9) {
+      best = rounds(cand);
+      t.nb_big = (int)cand;
+    }
+  if (g_pipe_big == 1) t.nb_big = (int)NB2;
+  // Tiles of 192 x 256 for all columns, priced at 1.5 small tiles: where they save a quarter of each round's tile (731 rows of 16,384 x
+  // 3,072 gated are 256 of them in one round instead of 192 of 256 x 256 on three quarters of the CUs: 79.8 -> 75.5 us, 560 rows 77.0 ->
+  // 67.6; 2,048 rows of 5,120 x 3,072 69.0 -> 63.3; at an even number of rounds they lose: 731 rows of 28,672 x 4,096 157 -> 165).
+  if (N % BNB == 0 && g_pipe_big != 1) {
+    const double cost = 1.5 * (double)(((long)((M + 191) / 192) * (N / BNB) + 255) / 256);
+    if (cost < best - 1e-9 || g_pipe_big == 5) {
+      best = cost;
+      t.low = true;
+    }
+  }
+  // Tiles of 256 x 192 where N is a multiple of 192 and that many more tiles fill whole rounds: priced at 1.35
+  // small tiles (the q/k/v projection of 2,048 rows, N = 6,144: 256 tiles in one round instead of 192 of 256 x 256
+  // on three quarters of the CUs, 117 -> 104 us in the model).
+  if (N % 192 == 0 && mode != OUT_SWIGLU && mode != OUT_SPLIT && g_pipe_big != 4 && g_pipe_big != 5 && (head_dim == 0 || head_dim == 128))
+    t.narrow = 1.35 * (double)(((long)MB * (N / 192) + 255) / 256) < best - 1e-9 || g_pipe_big == 3;
+  return t;
+}
+
+// The rows and columns of the larger tile that a product in one part of K takes (0: 256 x 128 or 128 x 128), as 1,000 rows + columns; for tests that mean a
+// certain one.
+extern "C" int tp_linear_big_tile(int M, int N, int gated, int head_dim) {
+  if (M < 1 || N < 1 || head_dim < 0) return 0;
+  const BigTiles t = big_tiles(M, N, gated ? OUT_SWIGLU : OUT_F32, head_dim);
+  return t.narrow ? 256192 : t.low ? 192256 : t.nb_big > 0 ? 256256 : 0;
+}
+
 // Returns 0 when launched, -1 when the sizes are not this kernel's.  `scratch` (optional) is room for
 // float32 partial sums: with few result tiles K is split over blocks until there is work for every CU.
-int g_pipe_big = 0;   // tuning: 1 = 256 x 256 tiles for every whole block of 256 columns, 2 = never; 3 = 256 x 192 wherever N allows, 4 = never; 5 = 192 x 256 wherever N allows
 int tp_linear_pipe(const bf16_t* x, const bf16_t* w, int w_tiled, void* out, int mode, int M, int N, int K, float* scratch,
                    size_t scratch_floats, int tune_splits, const RopeOut* rope, int defer, int* splits_out, GateAct gate,
                    hipStream_t s) {
@@ -1562,60 +1618,22 @@ int tp_linear_pipe(const bf16_t* x, const bf16_t* w, int w_tiled, void* out, int
   RopeOut rp = {};
   if (rope != nullptr) rp = *rope;
   rp.gate = gate;
-  // Whole rounds of 256 x 256 tiles first (see gemm_pipe_big_kernel), the columns that are left as above.
-  // How many blocks of 256 columns take the big tiles: all, none, or whole rounds of 256 tiles, whichever
-  // needs the fewest rounds when a big tile is priced at 1.72 small ones (measured: 113 against 65 us at
-  // K = 4096).
-  int nb_big = 0;
-  bool low = false;    // tiles of 192 rows
-  // (with the rotating epilogue a wave's 128 columns of a big tile have to lie inside one of q, k and v: heads
-  // of a multiple of 128; the strips of the 192-column tile are ordered for heads of 128)
-  const bool big_ok = rope == nullptr || rope->head_dim % 128 == 0;
-  if (splits == 1 && g_pipe_big != 2 && ldo % 4 == 0 && big_ok) {
-    const long NB2 = N / BNB;
-    auto rounds = [&](long nb) {
-      const long rest = (N - nb * BNB + BN - 1) / BN;
-      return 1.72 * (double)((MB * nb + 255) / 256) + (double)((MB * rest + 255) / 256);
-    };
-    const long whole = ((long)MB * NB2 / 256) * 256 / MB;
-    double best = rounds(0);
-    for (long cand : {NB2, whole})
-      if (cand > 0 && rounds(cand) < best - 1e-9) {
-        best = rounds(cand);
-        nb_big = (int)cand;
-      }
-    if (g_pipe_big == 1) nb_big = (int)NB2;
-    // Tiles of 192 x 256 for all columns, priced at 1.5 small tiles: where they save a quarter of each round's tile (731 rows of 16,384 x
-    // 3,072 gated are 256 of them in one round instead of 192 of 256 x 256 on three quarters of the CUs: 79.8 -> 75.5 us, 560 rows 77.0 ->
-    // 67.6; 2,048 rows of 5,120 x 3,072 69.0 -> 63.3; at an even number of rounds they lose: 731 rows of 28,672 x 4,096 157 -> 165).
-    const int MB192 = (M + 191) / 192;
-    if (N % BNB == 0 && g_pipe_big != 1) {
-      const double cost = 1.5 * (double)(((long)MB192 * (N / BNB) + 255) / 256);
-      if (cost < best - 1e-9 || g_pipe_big == 5) {
-        best = cost;
-        low = true;
-      }
-    }
-    // Tiles of 256 x 192 where N is a multiple of 192 and that many more tiles fill whole rounds: priced at 1.35
-    // small tiles (the q/k/v projection of 2,048 rows, N = 6,144: 256 tiles in one round instead of 192 of 256 x 256
-    // on three quarters of the CUs, 109 -> 8x us).
-    if (N % 192 == 0 && mode != OUT_SWIGLU && mode != OUT_SPLIT && g_pipe_big != 4 && (rope == nullptr || rope->head_dim == 128)) {
-      const long t192 = (long)MB * (N / 192);
-      if (1.35 * (double)((t192 + 255) / 256) < best - 1e-9 || g_pipe_big == 3) {
-        const long blocks3 = blocks_for(N / 192);
-        hipLaunchKernelGGL((gemm_pipe_big_kernel<8, 6>), dim3((unsigned)blocks3), dim3(256), 0, s, x, w, out, mode, M, N, K, pm, ldo,
-                           rp, w_tiled);
-        return 0;
-      }
-    }
+  // Whole rounds of larger tiles first, the columns that are left as above.
+  BigTiles big = {0, false, false};
+  if (splits == 1) big = big_tiles(M, N, mode, rope != nullptr ? rope->head_dim : 0);
+  if (big.narrow) {
+    hipLaunchKernelGGL((gemm_pipe_big_kernel<8, 6>), dim3((unsigned)blocks_for(N / 192)), dim3(256), 0, s, x, w, out, mode, M, N, K, pm, ldo,
+                       rp, w_tiled);
+    return 0;
   }
-  if (low) {
+  if (big.low) {
     const int MB192 = (M + 191) / 192, strips192 = (MB192 + 7) / 8;
     const long blocks4 = 8L * (((long)MB192 * (N / BNB) + 7) / 8);
     hipLaunchKernelGGL((gemm_pipe_big_kernel<6, 8>), dim3((unsigned)blocks4), dim3(256), 0, s, x, w, out, mode, M, N, K,
                        (MB192 + strips192 - 1) / strips192, ldo, rp, w_tiled);
     return 0;
   }
+  const int nb_big = big.nb_big;
   if (nb_big > 0) {
     const long blocks2 = blocks_for(nb_big);
     hipLaunchKernelGGL((gemm_pipe_big_kernel<8, 8>), dim3((unsigned)blocks2), dim3(256), 0, s, x, w, out, mode, M, nb_big * BNB, K,

@@ -558,11 +558,8 @@ def test_linear_big_tiles(m, n, k):
             lib.tp_linear_tune_tile(0)
 
 
-@pytest.mark.parametrize("m,heads,kv,k", [(191, 4, 2, 64), (192, 6, 1, 128), (193, 12, 2, 192), (577, 12, 4, 320), (1153, 14, 9, 256)])
-def test_linear_tiles_of_192_rows(m, heads, kv, k):
-    """192 x 256 tiles asked for, and the choice that the library makes by itself, at rows that fill no whole tile: the bits of the 256 x 128
-    tiles (every sum runs over K in ascending order) in every output mode, row-major and tiled weights, and through the rotating epilogue."""
-    ops = _ops()
+def _every_linear(ops, m, heads, kv, k, modes):
+    """Each mode's results of every output mode, row-major and tiled weights, and the rotating epilogue, n = (heads + 2 kv) * 128 columns."""
     lib = ops.library()
     from tempura_amd.parts.rope import rotary_inv_freq
     d, page, n = 128, 16, (heads + 2 * kv) * 128
@@ -586,7 +583,7 @@ def test_linear_tiles_of_192_rows(m, heads, kv, k):
         return out
 
     got = {}
-    for mode in (6, 9, 0):
+    for mode in modes:
         lib.tp_linear_tune_tile(mode)
         lib.tp_linear_tune_mid_tile(2)
         try:
@@ -594,8 +591,37 @@ def test_linear_tiles_of_192_rows(m, heads, kv, k):
         finally:
             lib.tp_linear_tune_tile(0)
             lib.tp_linear_tune_mid_tile(0)
+    return got
+
+
+@pytest.mark.parametrize("m,heads,kv,k", [(191, 4, 2, 64), (192, 6, 1, 128), (193, 12, 2, 192), (577, 12, 4, 320), (1153, 14, 9, 256), (385, 4, 1, 128),
+                                          (577, 8, 2, 192)])
+def test_linear_tiles_of_192_rows(m, heads, kv, k):
+    """192 x 256 tiles asked for, at rows that fill no whole tile and columns that 192 divides too: the bits of the 256 x 128 tiles (every
+    sum runs over K in ascending order)."""
+    ops = _ops()
+    lib = ops.library()
+    lib.tp_linear_tune_tile(9)
+    try:
+        assert lib.tp_linear_big_tile(m, (heads + 2 * kv) * 128, 0, 0) == 192256
+    finally:
+        lib.tp_linear_tune_tile(0)
+    got = _every_linear(ops, m, heads, kv, k, (6, 9, 0))
     for mode in (9, 0):
         assert all(torch.equal(a, b) for a, b in zip(got[mode], got[6])), mode
+
+
+@pytest.mark.parametrize("m,heads,kv,k", [(560, 96, 16, 64), (731, 96, 16, 128), (1153, 48, 8, 192), (2047, 24, 8, 64), (2304, 24, 8, 128), (3900, 16, 2, 64),
+                                          (1046, 126, 14, 64)])
+def test_linear_tiles_of_192_rows_by_the_rule(m, heads, kv, k):
+    """Sizes at which the rule itself takes 192 x 256 tiles: rows that fill no whole tile, a whole number of them, more than eight row blocks,
+    more than one round of tiles."""
+    ops = _ops()
+    n = (heads + 2 * kv) * 128
+    assert ops.library().tp_linear_big_tile(m, n, 0, 0) == ops.library().tp_linear_big_tile(m, n, 1, 0) == 192256
+    assert ops.library().tp_linear_big_tile(m, n, 0, 128) == 192256
+    got = _every_linear(ops, m, heads, kv, k, (6, 0))
+    assert all(torch.equal(a, b) for a, b in zip(got[0], got[6]))
 
 
 @pytest.mark.parametrize("m,hidden,kp,nc", [(1, 64, 32, 48), (8, 4096, 4096, 6144), (16, 160, 96, 272), (5, 4096, 14336, 1024),

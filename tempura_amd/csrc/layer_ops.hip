@@ -209,11 +209,11 @@ __global__ __launch_bounds__(256) void norm_add_kernel(float* __restrict__ h, co
 }
 
 // The same with the row in registers: every value is read once, sixteen bytes a load, all loads of a pass in flight
-// together (width a multiple of four, at most 4 * T * NV).  S: the values a thread brings to a sum, 1 or NV; with NV the sums' order is that of
-// a block of NV * T threads, so a row's bits do not depend on how many rows there are.
+// together (width a multiple of four, at most 4 * T * NV).  S: the values a thread brings to a sum, whose order is that of a block of S * T threads
+// whatever T is, so a row's bits do not depend on how many rows there are.
 // Few rows wait for one request of all their operands and for the sums, so a thread has as little of a row as can be (one row of 4,096 in two
 // parts 4.14 -> 3.20 us against 256 threads that load in turn, with a gate 5.49 -> 3.73); many rows wait for memory.
-// LATE: further parts, the gate and the next norm's weight are requested where they are used, so that fewer registers leave room for more rows.
+// LATE (y in one part): the gate and the next norm's weight are requested where they are used, so that fewer registers leave room for more rows.
 template <typename TO, int T, int NV, bool GATE, int S, bool LATE>
 __global__ __launch_bounds__(T) void norm_add_reg_kernel(float* __restrict__ h, const float* __restrict__ y,
                                                            const float* __restrict__ w, float eps,
@@ -258,19 +258,9 @@ __global__ __launch_bounds__(T) void norm_add_reg_kernel(float* __restrict__ h, 
     a.z += b.z;
     a.w += b.w;
   };
-  if constexpr (LATE) {
-    for (int p = 1; p < parts; ++p) {
+  if constexpr (GATE && LATE) {
 #pragma unroll
-      for (int k = 0; k < NV; ++k)
-        if (k * T + threadIdx.x < w4) y1[k] = *(const float4*)(y + p * part + base + 4 * (k * T + threadIdx.x));
-#pragma unroll
-      for (int k = 0; k < NV; ++k)
-        if (k * T + threadIdx.x < w4) add(yv[k], y1[k]);
-    }
-    if constexpr (GATE) {
-#pragma unroll
-      for (int k = 0; k < NV; ++k) fetch_gate(k);
-    }
+    for (int k = 0; k < NV; ++k) fetch_gate(k);
   }
 #pragma unroll
   for (int k = 0; k < NV; ++k) {
@@ -279,7 +269,7 @@ __global__ __launch_bounds__(T) void norm_add_reg_kernel(float* __restrict__ h, 
       if (!LATE && parts > 1) add(yv[k], y1[k]);
       if (!LATE && parts > 2) add(yv[k], y2[k]);
       if (!LATE && parts > 3) add(yv[k], y3[k]);
-      for (int p = LATE ? parts : 4; p < parts; ++p) add(yv[k], *(const float4*)(y + p * part + base + 4 * c));
+      for (int p = 4; !LATE && p < parts; ++p) add(yv[k], *(const float4*)(y + p * part + base + 4 * c));
       if constexpr (GATE) {
         yv[k].x *= l_sigmoid(gv[k].x + bv[k].x);
         yv[k].y *= l_sigmoid(gv[k].y + bv[k].y);

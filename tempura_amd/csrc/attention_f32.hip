@@ -231,8 +231,8 @@ __global__ __launch_bounds__((D + 63) / 64 * 64) void attn_f32_combine_kernel(co
   float og = 0.f;
 #pragma unroll
   for (int s = 0; s < EARLY; ++s)
-    if (s < splits) og = fmaf(__shfl(f, s, TP_WAVE), v[s], og);
-  for (int s = EARLY; s < splits; ++s) og = fmaf(__shfl(f, s, TP_WAVE), base[(size_t)s * (D + 2) + d], og);
+    if (s < splits) og = fmaf(lane_value(f, s), v[s], og);
+  for (int s = EARLY; s < splits; ++s) og = fmaf(lane_value(f, s), base[(size_t)s * (D + 2) + d], og);
   if ((int)threadIdx.x < D) out[((size_t)t * n_heads + h) * D + d] = og * inv;
 }
 

@@ -1751,22 +1751,22 @@ __global__ __launch_bounds__(256, 2) void attn_both_kernel(AttnArgs a, int n_req
 __device__ inline void combine_request(float (&early)[COMBINE_EARLY], const float* values, size_t stride, int splits) {
 #pragma unroll
   for (int s = 0; s < COMBINE_EARLY; ++s)
-    if (s < splits) early[s] = values[(size_t)s * stride];
+    early[s] = values[(size_t)min(s, splits - 1) * stride];   // (a branch for each takes longer than a value asked for twice)
 }
 __device__ inline float combine_sum(const float (&early)[COMBINE_EARLY], const float* values, size_t stride, int splits, float ws) {
   float acc = 0.f;
 #pragma unroll
   for (int s = 0; s < COMBINE_EARLY; ++s)
-    if (s < splits) acc = fmaf(__shfl(ws, s, 64), early[s], acc);
+    if (s < splits) acc = fmaf(lane_value(ws, s), early[s], acc);
   int s = COMBINE_EARLY;
   for (; s + 8 <= splits; s += 8) {   // eight independent loads in flight
     float v[8];
 #pragma unroll
     for (int u = 0; u < 8; ++u) v[u] = values[(size_t)(s + u) * stride];
 #pragma unroll
-    for (int u = 0; u < 8; ++u) acc = fmaf(__shfl(ws, s + u, 64), v[u], acc);
+    for (int u = 0; u < 8; ++u) acc = fmaf(lane_value(ws, s + u), v[u], acc);
   }
-  for (; s < splits; ++s) acc = fmaf(__shfl(ws, s, 64), values[(size_t)s * stride], acc);
+  for (; s < splits; ++s) acc = fmaf(lane_value(ws, s), values[(size_t)s * stride], acc);
   return acc;
 }
 
@@ -1774,7 +1774,8 @@ __device__ inline float combine_sum(const float (&early)[COMBINE_EARLY], const f
 // grid: (requests, heads); block: whole waves for the head's elements, up to 256 at a time, each wave working out the splits' weights for itself
 // (its lane s holds split s's statistics, num_splits <= 64).  cu_seqlens null: every request brings one token.
 // Bound by one trip to memory, the statistics and the first eight splits' values together.  With the attention in front, captured, against a wave a head that
-// asked for the values behind the statistics: 32 heads of 128, one request of 3,072 keys 11.1 -> 10.1 us, sixteen of 3,000 37.8 -> 37.0; heads of 64 alike.
+// asked for the values behind the statistics: 24 heads of 128, one request of 523 keys 7.5 -> 7.1 us, fourteen of 2,373 25.5 -> 24.5; 16 of 64, two of 732 6.4 -> 6.3, fourteen of
+// 2,373 11.3 -> 11.3 (the weights by instructions: with __shfl 6.5 and 11.5).
 // (Combining inside the decode kernel by whichever block finishes last was tried and is far
 // slower: the L2 caches of the eight XCDs are not coherent with each other, so partial results
 // would have to travel through memory with device-scope fences.)

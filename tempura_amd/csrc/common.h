@@ -146,6 +146,8 @@ template <int N>
 __device__ inline float row_rotated(float v) {
   return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x120 + N, 0xf, 0xf, false));
 }
+// v of one lane, the same for all: by an instruction instead of a trip through LDS (__shfl).
+__device__ inline float lane_value(float v, int lane) { return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), lane)); }
 __device__ inline float row_sum(float v) {
   v += row_rotated<8>(v);
   v += row_rotated<4>(v);

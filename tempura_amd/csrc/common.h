@@ -132,16 +132,18 @@ struct LanePair {
   float a, b;
 };
 // (written out: of the builtins' two results this compiler hands on the first twice; a wave's own writes need two states before the swap)
-__device__ inline LanePair lanes_32(float v) {
-  LanePair p = {v, v};
+__device__ inline LanePair halves_swapped(float a, float b) {   // a: the lower halves of both, b: the upper ones
+  LanePair p = {a, b};
   asm volatile("s_nop 1\n\tv_permlane32_swap_b32_e32 %0, %1" : "+v"(p.a), "+v"(p.b));
   return p;
 }
-__device__ inline LanePair lanes_16(float v) {
-  LanePair p = {v, v};
+__device__ inline LanePair rows_swapped(float a, float b) {     // a: rows 0 and 2 of 16 lanes, each followed by b's; b: rows 1 and 3
+  LanePair p = {a, b};
   asm volatile("s_nop 1\n\tv_permlane16_swap_b32_e32 %0, %1" : "+v"(p.a), "+v"(p.b));
   return p;
 }
+__device__ inline LanePair lanes_32(float v) { return halves_swapped(v, v); }
+__device__ inline LanePair lanes_16(float v) { return rows_swapped(v, v); }
 template <int N>
 __device__ inline float row_rotated(float v) {
   return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x120 + N, 0xf, 0xf, false));
@@ -165,6 +167,24 @@ __device__ inline float wave_sum(float v) {
   LanePair p = lanes_32(v);
   p = lanes_16(p.a + p.b);
   return row_sum(p.a + p.b);
+}
+
+// The sums of S (1, 2 or 4) values, sum k in the lanes from 64 / S * k on, each with wave_sum's bits: the swaps bring halves of two values
+// (rows of two pairs) together instead of twice the same, so four sums are ten steps instead of four times eight.
+template <int S>
+__device__ inline float wave_sums(const float (&v)[S]) {
+  static_assert(S == 1 || S == 2 || S == 4, "values");
+  if constexpr (S == 1) {
+    return wave_sum(v[0]);
+  } else if constexpr (S == 2) {
+    LanePair p = halves_swapped(v[0], v[1]);
+    p = lanes_16(p.a + p.b);
+    return row_sum(p.a + p.b);
+  } else {
+    const LanePair p = halves_swapped(v[0], v[2]), q = halves_swapped(v[1], v[3]);
+    const LanePair r = rows_swapped(p.a + p.b, q.a + q.b);
+    return row_sum(r.a + r.b);
+  }
 }
 
 // Sum over `lanes` (a power of two) neighbouring lanes, from a multiple of `lanes` on; every lane gets it.
@@ -200,11 +220,9 @@ template <int T, int S>
 __device__ inline float block_sum_once(const float (&v)[S], float* scratch) {
   static_assert(T * S == TP_WAVE || T * S % (4 * TP_WAVE) == 0, "one wave, or whole 16-byte pieces");
   if constexpr (T * S == TP_WAVE) return wave_sum(v[0]);
-#pragma unroll
-  for (int k = 0; k < S; ++k) {
-    const float sum = wave_sum(v[k]);
-    if (threadIdx.x % TP_WAVE == 0) scratch[k * (T / TP_WAVE) + threadIdx.x / TP_WAVE] = sum;
-  }
+  const float sum = wave_sums<S>(v);
+  const int lane = threadIdx.x % TP_WAVE;
+  if (lane % (TP_WAVE / S) == 0) scratch[lane / (TP_WAVE / S) * (T / TP_WAVE) + threadIdx.x / TP_WAVE] = sum;
   __syncthreads();
   float4 t = *(const float4*)scratch;
 #pragma unroll

@@ -99,13 +99,17 @@ template <typename TO>
 static void launch_rmsnorm(const float* x, const float* w, const int* rows, void* out, int n_out, int hidden, float eps, hipStream_t s) {
   if (hidden % 4 == 0 && hidden <= 16384 && (((uintptr_t)x | (uintptr_t)w | (uintptr_t)out) & 15) == 0) {
     // (up to 1,024 columns a wave a row where there are several rows for every wave the chip holds: blocks of 256 / 64, 40,000 rows of 128 columns 16.8 /
-    // 11.7 us, 5,000 rows of 512 5.4 / 5.0, of 1,000 7.2 / 8.0, 40,000 of them 44.0 / 39.2; a row of 1,000 alone 2.2 / 2.9)
+    // 11.7 us, 5,000 rows of 512 5.4 / 5.0, of 1,000 7.2 / 8.0, 40,000 of them 44.0 / 39.2; a row of 1,000 alone 2.2 / 2.9; from 1,025 to 3,072 columns half as
+    // many threads where a CU has more than four rows: 512x1 / 256x2, 1,024 rows of 2,048 4.1 / 3.9 us, 2,048 rows 5.9 / 5.3, 600 of 1,028 3.1 / 3.3; 512x2 / 256x3, 800 of
+    // 3,072 4.4 / 4.6, 2,048 7.6 / 7.2, but 8,000 of 4,096 29.6 / 30.1)
 #define RMS(T_, NV_, ...) hipLaunchKernelGGL((rmsnorm_reg_kernel<TO, T_, NV_, ##__VA_ARGS__>), dim3(n_out), dim3(T_), 0, s, x, w, rows, (TO*)out, hidden, eps)
     if (hidden <= 256) RMS(64, 1);
     else if (hidden <= 512 && n_out > 4096) RMS(64, 2, 4);
     else if (hidden <= 1024 && n_out > 16384) RMS(64, 4, 4);
     else if (hidden <= 1024) RMS(256, 1);
+    else if (hidden <= 2048 && n_out > 1024) RMS(256, 2, 2);
     else if (hidden <= 2048) RMS(512, 1);
+    else if (hidden <= 3072 && n_out > 1024) RMS(256, 3, 2);
     else if (hidden <= 4096) RMS(512, 2);
     else if (hidden <= 8192) RMS(1024, 2);
     else RMS(1024, 4);

@@ -338,33 +338,41 @@ extern "C" int tp_norm_add(float* h, const float* y, const float* w, float eps, 
     const bool bf = w_next != nullptr && x_dt == TP_BF16;
 #define NA1(TO, T, NV, G, S, L) \
   hipLaunchKernelGGL((norm_add_reg_kernel<TO, T, NV, G, S, L>), dim3(n), dim3(T), 0, s, h, y, w, eps, w_next, eps_next, (TO*)x, width, gate, normed, blocked, parts)
+#define NAP(T, NV, S, L)                     \
+  do {                                       \
+    if (bf) NA1(bf16_t, T, NV, false, S, L);  \
+    else NA1(float, T, NV, false, S, L);      \
+  } while (0)
 #define NA(T, NV, S, L)                      \
   do {                                       \
-    if (gate_rows != nullptr) {              \
-      if (bf) NA1(bf16_t, T, NV, true, S, L);   \
-      else NA1(float, T, NV, true, S, L);       \
-    } else {                                 \
-      if (bf) NA1(bf16_t, T, NV, false, S, L);  \
-      else NA1(float, T, NV, false, S, L);      \
-    }                                        \
+    if (gate_rows == nullptr) NAP(T, NV, S, L);  \
+    else if (bf) NA1(bf16_t, T, NV, true, S, L); \
+    else NA1(float, T, NV, true, S, L);       \
   } while (0)
-    // A thread for every 16 bytes, and half as many where the CUs' 2,048 threads each no longer hold all rows (from 513 rows of 4,096, 1,025 of
-    // 2,048): more blocks then share a CU and hide one another's barriers.  Width 4,096, blocks of 1,024 / 512: 800 rows 10.7 / 10.2 us, 2,048 rows 25.7 /
-    // 23.7 (5.0 TB/s), with a gate 30.6 / 29.8.  Width 2,048, blocks of 512 / 256: 2,048 rows 12.5 / 11.7, but of three parts 15.9 / 16.3.
-    // Still more rows of one part wait for memory alone, and what they request is better spread out (LATE).  All operands in front / gate and next weight late,
-    // with a gate: 10,000 rows of 1,280 43.4 / 39.2 us, of 1,536 49.6 / 46.9 (2,048 rows 12.1 / 12.3); 5,000 rows of 2,560 46.6 / 42.7 (800 rows 9.8 /
-    // 10.4), of 4,096 68.2 / 67.5; 2,048 rows of 5,120 (1,024 x 2 threads in front) 44.2 / 35.4, without a gate 30.7 / 29.3.  Beyond 6,144 columns
-    // rows without a gate lose: 1,100 of 8,192 27.9 / 29.3.
+    // A thread for every 16 bytes, and fewer from two rows a CU on: more blocks then share a CU and hide one another's barriers.  Rows of many
+    // parts need their registers and keep more threads for longer (2,048 rows of 2,048 in three parts 15.9 us, with 256 threads 16.3).
+    // From there on rows of one part request their gate and the next norm's weight late (LATE), which leaves room for more of them.  Without a gate still fewer threads
+    // take a row where there are many, whose sums cost fewer instructions.  us, threads x pieces (l: late), without a gate:
+    //   1,408 columns   512x1 / 256x2 / 256x2l / 128x4l   200 rows 3.2 / 3.5 / 3.6 / 3.9, 560 4.5 / 4.3 / 4.3 / 4.7, 1,100 6.2 / 6.0 / 5.5 / 5.6, 3,033 11.8 / 10.8 / 10.9 / 9.3
+    //   3,072           1,024x1 / 512x2 / 512x2l / 256x4l  256 rows 4.2 / 4.2 / 4.3 / 4.7, 400 5.4 / 5.0 / 5.0 / 5.4, 640 7.3 / 6.4 / 6.3 / 6.3, 1,500 13.0 / 11.5 / 11.9 / 10.5
+    //   5,120           1,024x2 / 1,024x2l / 512x3 / 512x3l  200 rows 4.8 / 4.8 / 4.9 / 4.9, 400 6.9 / 6.7 / 6.5 / 6.4, 640 9.2 / 9.1 / 9.4 / 8.1, 2,337 28.0 / 28.8 / 29.8 / 26.4
+    // and with one, 2,048: 1,500 rows 10.5 / 10.4 / 10.1 / 12.4; 3,072: 256 rows 4.8 / 4.9 / 5.0 / 5.5, 640 8.7 / 8.3 / 8.4 / 8.6, 1,024 11.8 / 11.2 / 10.4 / 10.9; 5,120: 400 rows
+    // 9.4 / 8.6 / 8.6 / 8.7, 2,337 41.6 / 34.9 / 37.1 / 34.3; 8,192 (1,024x2 / 512x4l): 1,100 rows 35.3 / 28.8.
     if (width <= 1024) NA(256, 1, 1, false);
-    else if (width <= 2048 && n > 2048 && parts == 1) NA(256, 2, 2, true);
-    else if (width <= 2048 && n > 1024 && parts == 1) NA(256, 2, 2, false);
+    else if (width < 2048 && n > 2048 && parts == 1 && gate_rows == nullptr) NAP(128, 4, 4, true);
+    else if (width <= 2048 && n > 512 && parts == 1) NA(256, 2, 2, true);
     else if (width <= 2048) NA(512, 1, 1, false);
-    else if (width <= 4096 && n > 1024 && parts == 1) NA(512, 2, 2, true);
+    else if (width <= 4096 && n > 768 && parts == 1 && gate_rows == nullptr) NAP(256, 4, 4, true);
+    else if (width <= 4096 && n > (gate_rows != nullptr ? 768 : 256) && parts == 1) NA(512, 2, 2, true);
+    else if (width <= 4096 && n > 256 && parts == 1) NA(512, 2, 2, false);
     else if (width <= 4096 && n > 512) NA(512, 2, 2, false);
     else if (width <= 4096) NA(1024, 1, 1, false);
     else if (width <= 6144 && n > 512 && parts == 1) NA(512, 3, 2, true);
+    else if (n > 512 && parts == 1) NA(512, 4, 2, true);
+    else if (n > 256 && parts == 1) NA(1024, 2, 1, true);
     else NA(1024, 2, 1, false);
 #undef NA
+#undef NAP
 #undef NA1
     TP_CHECK_LAUNCH("norm_add");
     return 0;

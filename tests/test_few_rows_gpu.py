@@ -380,7 +380,8 @@ def test_norm_of_partial_sums(width):
 
 @pytest.mark.parametrize("n, width, parts", [(1025, 1028, 1), (1025, 2048, 1), (513, 2052, 1), (513, 2052, 5), (513, 3000, 1), (513, 4096, 1), (513, 4096, 5),
                                              (2049, 1028, 1), (2049, 2048, 1), (1025, 2052, 1), (1025, 4096, 1), (513, 4100, 1), (513, 6144, 1), (513, 6144, 3),
-                                             (513, 6148, 1)])
+                                             (513, 6148, 1), (513, 8192, 1), (513, 1028, 1), (513, 2048, 1), (2049, 2044, 1), (301, 2052, 1), (301, 4096, 1),
+                                             (769, 2052, 1), (769, 4096, 1), (301, 4100, 1), (301, 8192, 1)])
 def test_norm_of_many_rows(n, width, parts):
     """Many rows (half as many threads a row, the gate and the next weight late) against the same rows a few at a time, bit by bit, and against float64."""
     from tempura_amd.kernels import ops

@@ -56,7 +56,7 @@ def test_rmsnorm(out_dtype, n, hidden, eps):
 
 
 @pytest.mark.parametrize("n,hidden", [(4097, 4), (4097, 256), (4097, 260), (4097, 512), (16385, 516), (16385, 1024), (3, 8192), (3, 8196), (3, 12288), (2, 16384),
-                                      (2, 16388)])
+                                      (2, 16388), (1025, 1028), (1025, 2048), (1025, 2052), (1025, 3072)])
 def test_rmsnorm_of_many_and_of_long_rows(n, hidden):
     """The bits of the same rows a few at a time, and float64 within the roundings of a value (twenty of 2^-24 of the largest)."""
     ops = _ops()

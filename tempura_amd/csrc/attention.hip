@@ -118,7 +118,7 @@ int tp_paged_attention_fast(const void* q, const void* k_cache, const void* v_ca
                             int portion_splits, int portion_min_steps, float* portion_scratch, const float* dist_bias,
                             int bias_len, int keep_first, const float* sink, int value_dim, int chunk, float softcap,
                             int gated, const float* gate, int gate_stride, int gate_col0, int gate_per, float gate_scale, int out_stride,
-                            int out_col0, hipStream_t s);
+                            int out_col0, const int* order, hipStream_t s);
 
 // Defined in attention_f32.hip; -1 for shapes that are not its own.
 int tp_paged_attention_f32(const float* q, const float* k_cache, const float* v_cache, const int* block_tables, int table_width,
@@ -135,7 +135,7 @@ extern "C" int tp_paged_attention(const void* q, int dt, const void* k_cache, co
                                   int num_splits, int decode_waves, float* scratch, int portion_splits, int portion_min_steps,
                                   float* portion_scratch, const float* dist_bias, int bias_len, int value_dim,
                                   int keep_first, const float* sink, int chunk, float softcap, const float* gate, int gate_stride,
-                                  int gate_col0, int gate_per, float gate_scale, int out_stride, int out_col0, hipStream_t s) {
+                                  int gate_col0, int gate_per, float gate_scale, int out_stride, int out_col0, const int* order, hipStream_t s) {
   // value_dim: the size of a value head (0: head_dim): v_cache is [page, kv_head, value_dim, page_size] and out
   // [n, heads * value_dim]; the matrix-core kernels take equal sizes and a few pairs with wider keys.
   if (value_dim <= 0) value_dim = head_dim;
@@ -146,6 +146,7 @@ extern "C" int tp_paged_attention(const void* q, int dt, const void* k_cache, co
   // allow_fast 2 (single tokens only, sizes that the matrix-core kernels take): `out` is rows of out_stride columns, and the heads'
   // outputs go to its columns from out_col0 on, rounded to bfloat16, times sigmoid(gate[:, gate_col0 + column / gate_per]) (gate
   // float32 rows of gate_stride; nullptr: none) and gate_scale.
+  // order: of the requests among the blocks (tp_decode_order; used where every request brings one token), or nullptr.
   TP_REQUIRE(n_tokens >= 0 && n_req >= 0 && n_heads > 0 && n_kv > 0 && head_dim > 0 && page_size > 0,
              "paged_attention: bad sizes");
   TP_REQUIRE(n_heads % n_kv == 0, "paged_attention: %d heads is not a multiple of %d kv heads", n_heads, n_kv);
@@ -173,7 +174,7 @@ extern "C" int tp_paged_attention(const void* q, int dt, const void* k_cache, co
                                            context_lens, out, n_tokens, n_req, n_heads, n_kv, head_dim,
                                            page_size, scale, window, max_q_len, num_single, num_splits, decode_waves, scratch, token_req,
                                            portion_splits, portion_min_steps, portion_scratch, dist_bias, bias_len, keep_first, sink, value_dim, chunk,
-                                           softcap, allow_fast == 2, gate, gate_stride, gate_col0, gate_per, gate_scale, out_stride, out_col0, s);
+                                           softcap, allow_fast == 2, gate, gate_stride, gate_col0, gate_per, gate_scale, out_stride, out_col0, order, s);
     if (rc >= 0) return rc;
   }
   TP_REQUIRE(allow_fast != 2, "paged_attention: no gate over the heads' outputs for these sizes");

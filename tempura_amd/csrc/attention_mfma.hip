@@ -109,6 +109,7 @@ struct AttnArgs {
   float* portion_scratch;
   const int* token_req;
   int decode_waves;  // of a block of single tokens whose keys go to LDS, 4 or 8
+  const int* order;  // of their requests among the blocks (decode_order_kernel), or nullptr: as they are
   bool all_single;  // (every request brings one token: request r's row is row r)
   bool gated;       // (every request brings one token: the rows go through `gate`)
   CombineGate gate;
@@ -1403,13 +1404,16 @@ __global__ __launch_bounds__(256) void attn_decode_kernel(AttnArgs a) {
 // kilobytes (a key fragment loaded into its registers is 64-byte pieces of sixteen rows, which the address path of a CU takes at
 // half the rate) and emptied without a barrier: a step's keys go on their way NB steps ahead, as soon as the fragments of the keys
 // they replace are in registers, its values likewise, its pages before that.
+#define DECODE_ORDER_ROWS 512
 // (a wait that stays in its place among the assembly that reads LDS behind it)
 #define ATTN_WAIT_VM_ORDERED(n) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(n) : "memory")
 // ROWS: q, k and v come as the projection's float32 rows (RowsIn): a wave takes a head (of q, or the new key, or the new value), the
 // block's heads go to LDS, the new key and value to the cache and, since the cache's own copy may not have arrived when the step
 // that holds it is read, into that step's place in LDS.  The rows travel beside the first keys; a launch or two between the
 // projection and the attention are gone: Bomotar's decode step, four layers with a convolution, 377 -> 361 us; 28 layers of the 3B
-// shape with 48 requests, three parts of K, 3,219 -> 3,187.
+// shape with 48 requests, three parts of K, 3,219 -> 3,187.  What a block does before its first step costs every block of a launch: two items a wave
+// requested in front of the keys, the cache's new key and value stored behind the last step instead of in front of the first wait, 48 requests of 1,100 keys
+// 41.0 -> 39.8 us, with the step's table of cosines and sines instead of its own 39.5.
 // (stages: WAVES * NB * (D + DV) * 64 bytes of LDS; bx: key head and block of heads, r: request, split: its part of the keys)
 template <int D, int DV, int MODE, int WAVES, int NB, bool ROWS>
 __device__ inline void attn_decode_lds_block(const AttnArgs& a, const RowsIn& in, unsigned char* stages, int bx, int r, int split) {
@@ -1440,9 +1444,9 @@ __device__ inline void attn_decode_lds_block(const AttnArgs& a, const RowsIn& in
   }
   // (ROWS; r is the token's row) item i: head i of q, then the new key, then the new value; a lane has the elements 2 lane, 2 lane + 1
   const int items = ncols + 2;
-  float2 raw[ROWS ? ROWS_PARTS : 1], turn = make_float2(1.f, 0.f);
-  int place = 0;
-  auto fetch_row = [&](int i) __attribute__((always_inline)) {
+  // (a wave's first two items are requested in front of its keys: a row asked for behind them comes when they have come)
+  float2 raw[ROWS ? 2 : 1][ROWS ? ROWS_PARTS : 1], turn[2] = {make_float2(1.f, 0.f), make_float2(1.f, 0.f)};
+  auto fetch_row = [&](int i, int s) __attribute__((always_inline)) {
     if constexpr (ROWS) {
       const int e = 2 * lane;
       if (e >= (i == ncols + 1 ? DV : D)) return;
@@ -1450,24 +1454,25 @@ __device__ inline void attn_decode_lds_block(const AttnArgs& a, const RowsIn& in
       const int col = (i < ncols ? (kvh * group + i) * D : i == ncols ? qd + kvh * D : qd + kd + kvh * DV) + e;
       const float* row = in.rows + (size_t)r * in.stride + col;
       if (in.conv_w != nullptr) {     // this token's input, the carried ones, the weights
-        raw[0] = *(const float2*)row;
+        raw[s][0] = *(const float2*)row;
         const float* st = in.state + (size_t)in.state_slots[r] * in.state_stride + in.state_off + col;
 #pragma unroll
         for (int t = 0; t < ROWS_TAPS - 1; ++t)
-          if (t < in.taps - 1) raw[1 + t] = *(const float2*)(st + (size_t)t * in.channels);
+          if (t < in.taps - 1) raw[s][1 + t] = *(const float2*)(st + (size_t)t * in.channels);
 #pragma unroll
         for (int t = 0; t < ROWS_TAPS; ++t)
-          if (t < in.taps) raw[ROWS_TAPS + t] = *(const float2*)(in.conv_w + (size_t)t * in.channels + col);
+          if (t < in.taps) raw[s][ROWS_TAPS + t] = *(const float2*)(in.conv_w + (size_t)t * in.channels + col);
       } else {
 #pragma unroll
         for (int t = 0; t < ROWS_PARTS; ++t)
-          if (t < in.parts) raw[t] = *(const float2*)(row + (size_t)t * in.part_stride);
+          if (t < in.parts) raw[s][t] = *(const float2*)(row + (size_t)t * in.part_stride);
       }
-      if (i <= ncols && e < in.rotary_dim && in.cos_sin != nullptr) turn = in.cos_sin[(size_t)r * (in.rotary_dim >> 1) + lane];
-      if (i >= ncols) place = in.slots[r];
+      if (i <= ncols && e < in.rotary_dim && in.cos_sin != nullptr) turn[s] = in.cos_sin[(size_t)r * (in.rotary_dim >> 1) + lane];
     }
   };
-  if (ROWS && wave < items) fetch_row(wave);
+  const int place = ROWS ? in.slots[r] : 0;
+  if (ROWS && wave < items) fetch_row(wave, 0);
+  if (ROWS && wave + WAVES < items) fetch_row(wave + WAVES, 1);
   // this lane's offset in each load of a step, and its addresses in LDS (see attn_prefill_lds_kernel)
   const int ps = a.page_size, psh = a.page_shift, pmask = ps - 1;
   unsigned koff[KI];
@@ -1546,11 +1551,10 @@ __device__ inline void attn_decode_lds_block(const AttnArgs& a, const RowsIn& in
     }
   if (NB < n) pages_of(NB);
   const unsigned hl0 = (unsigned)(size_t)(__attribute__((address_space(3))) const bf16_t*)heads_lds;
+  const bool newest = ROWS && s_begin < s_end && s_end == steps;      // this block's keys end with the token's own
   if constexpr (ROWS) {
-    const bool newest = s_begin < s_end && s_end == steps;      // this block's keys end with the token's own
-    for (int i = wave; i < items; i += WAVES) {
-      if (i != wave) fetch_row(i);
-      if (i >= ncols && !newest) continue;
+    auto finish_row = [&](int i, int s) __attribute__((always_inline)) {
+      if (i >= ncols && !newest) return;
       const int e = 2 * lane, width = i == ncols + 1 ? DV : D;
       float x0 = 0.f, x1 = 0.f;
       if (e < width) {
@@ -1561,17 +1565,17 @@ __device__ inline void attn_decode_lds_block(const AttnArgs& a, const RowsIn& in
 #pragma unroll
           for (int t = 0; t < ROWS_TAPS; ++t)
             if (t < in.taps) {
-              const float2 v = t == in.taps - 1 ? raw[0] : raw[1 + t];
+              const float2 v = t == in.taps - 1 ? raw[s][0] : raw[s][1 + t];
               if (t > 0) *(float2*)(st + (size_t)(t - 1) * in.channels) = v;
-              x0 = fmaf(raw[ROWS_TAPS + t].x, v.x, x0);
-              x1 = fmaf(raw[ROWS_TAPS + t].y, v.y, x1);
+              x0 = fmaf(raw[s][ROWS_TAPS + t].x, v.x, x0);
+              x1 = fmaf(raw[s][ROWS_TAPS + t].y, v.y, x1);
             }
         } else {
 #pragma unroll
           for (int t = 0; t < ROWS_PARTS; ++t)
             if (t < in.parts) {
-              x0 += raw[t].x;
-              x1 += raw[t].y;
+              x0 += raw[s][t].x;
+              x1 += raw[s][t].y;
             }
         }
       }
@@ -1583,9 +1587,9 @@ __device__ inline void attn_decode_lds_block(const AttnArgs& a, const RowsIn& in
           x1 = x1 * rstd * w[e + 1];
         }
       }
-      if (e >= width) continue;
+      if (e >= width) return;
       if (i <= ncols && e < in.rotary_dim) {
-        float2 cs = turn;
+        float2 cs = turn[s];
         if (in.cos_sin == nullptr) rope_cos_sin(in.positions[r], in.inv_freq[lane], in.factor, cs.x, cs.y);
         const float y0 = x0, y1 = x1;
         x0 = y0 * cs.x - y1 * cs.y;
@@ -1594,16 +1598,12 @@ __device__ inline void attn_decode_lds_block(const AttnArgs& a, const RowsIn& in
       const unsigned pk = pack_bf16(x0, x1);
       const unsigned to = hl0 + (i < ncols ? i : 16 + i - ncols) * (D * 2) + e * 2;
       asm volatile("ds_write_b32 %0, %1" ::"v"(to), "v"(pk) : "memory");
-      if (i >= ncols) {
-        const size_t page = (size_t)(place >> psh), off = (size_t)(place & pmask);
-        if (i == ncols) {
-          *(unsigned*)(in.k_cache + ((page * a.n_kv + kvh) * ps + off) * D + e) = pk;
-        } else {
-          bf16_t* o = in.v_cache + ((page * a.n_kv + kvh) * DV + e) * ps + off;
-          o[0] = bf16_t{(uint16_t)(pk & 0xffff)};
-          o[ps] = bf16_t{(uint16_t)(pk >> 16)};
-        }
-      }
+    };
+    if (wave < items) finish_row(wave, 0);
+    if (wave + WAVES < items) finish_row(wave + WAVES, 1);
+    for (int i = wave + 2 * WAVES; i < items; i += WAVES) {
+      fetch_row(i, 0);
+      finish_row(i, 0);
     }
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     __builtin_amdgcn_s_barrier();
@@ -1628,10 +1628,9 @@ __device__ inline void attn_decode_lds_block(const AttnArgs& a, const RowsIn& in
     const unsigned base = lds0 + st * STAGE;
     const bool behind = NB > 1 && i + 1 < n;      // (a whole step on its way behind this one)
     const bool more = i + NB < n;
-    // (ROWS: the stores of the new key, value and carried inputs are behind the first loads, and the waits count them as well: a
-    // step that should have waited for its loads alone waits for less than it could, never for less than it needs, so the first
+    // (ROWS with a convolution: the stores of the carried inputs are behind the first loads, and the waits count them as well: the first
     // steps wait for everything)
-    if (ROWS && i < NB) ATTN_WAIT_VM_ORDERED(0);
+    if (ROWS && i < NB && in.conv_w != nullptr) ATTN_WAIT_VM_ORDERED(0);
     else if (behind) ATTN_WAIT_VM_ORDERED(VI + KI + VI);
     else ATTN_WAIT_VM_ORDERED(VI);
     const int j0 = key0(i);
@@ -1706,6 +1705,21 @@ __device__ inline void attn_decode_lds_block(const AttnArgs& a, const RowsIn& in
     attn_pv<DV, 1>(vf, pf, alpha, moved, o);
     st = st + 1 == NB ? 0 : st + 1;
   }
+  if (newest && wave < 2) {      // the new key and value into the cache, behind the steps: their waits would count these stores
+    const int e = 2 * lane;
+    if (e < (wave == 0 ? D : DV)) {
+      unsigned pk;
+      asm volatile("ds_read_b32 %0, %1\n\ts_waitcnt lgkmcnt(0)" : "=v"(pk) : "v"(hl0 + (16 + wave) * (D * 2) + e * 2) : "memory");
+      const size_t page = (size_t)(place >> psh), off = (size_t)(place & pmask);
+      if (wave == 0) {
+        *(unsigned*)(in.k_cache + ((page * a.n_kv + kvh) * ps + off) * D + e) = pk;
+      } else {
+        bf16_t* o = in.v_cache + ((page * a.n_kv + kvh) * DV + e) * ps + off;
+        o[0] = bf16_t{(uint16_t)(pk & 0xffff)};
+        o[ps] = bf16_t{(uint16_t)(pk >> 16)};
+      }
+    }
+  }
   __syncthreads();     // (every wave's ring is empty)
   decode_merge<DV, WAVES>(a, (float*)stages, wave, lane, m[0], l[0], o[0], r, q_start, split, kvh * group + h0, ncols);
 }
@@ -1713,7 +1727,30 @@ __device__ inline void attn_decode_lds_block(const AttnArgs& a, const RowsIn& in
 template <int D, int DV, int MODE, int WAVES, int NB, bool ROWS = false>
 __global__ __launch_bounds__(WAVES * 64) void attn_decode_lds_kernel(AttnArgs a, RowsIn in) {
   __shared__ __attribute__((aligned(1024))) unsigned char stages[WAVES * NB * (D + DV) * 64];
-  attn_decode_lds_block<D, DV, MODE, WAVES, NB, ROWS>(a, in, stages, blockIdx.x, blockIdx.y, blockIdx.z);
+  attn_decode_lds_block<D, DV, MODE, WAVES, NB, ROWS>(a, in, stages, blockIdx.x, a.order != nullptr ? a.order[blockIdx.y] : blockIdx.y, blockIdx.z);
+}
+
+// The order of n requests of one token each among the blocks of an attention whose blocks of four waves are more than the CUs: a CU gets its
+// first block in the order of the launch, then a second one in the same order, and from then on whoever is done first.  A CU pulls at most 55 to 60 GB/s, which
+// one block of four waves reaches, so what counts is how many keys a CU has: of up to two blocks a CU the longest requests stay alone, and the
+// others are paired, the longest with the shortest; of more the longest come first.  places: CUs a head and group of heads.  Requests of one
+// length stay in their order.  No request is computed otherwise than without an order.  24 heads in 8 groups of 128, a captured chain over ten layers'
+// caches, requests of a fifth of the mean to twice it, as they come (the longest last) / ordered: 48 of 1,100 keys 43.0 / 39.5 us (of one length 39.5 / 39.6),
+// 64 of them 52.3 / 48.8 (48.5 / 48.5), 128 99.4 / 93.2 (94.2 / 94.3), 200 of 500 79.6 / 73.9; this launch 2.4 us a step.
+__global__ __launch_bounds__(DECODE_ORDER_ROWS) void decode_order_kernel(AttnArgs a, int n, int places, int* __restrict__ order) {
+  __shared__ int steps[DECODE_ORDER_ROWS];
+  const int t = threadIdx.x;
+  int mine = 0, first, kept;
+  if (t < n) mine = decode_steps(a, a.context_lens[t], first, kept);
+  steps[t] = mine;
+  __syncthreads();
+  if (t >= n) return;
+  int rank = 0;
+  for (int i = 0; i < n; ++i) rank += steps[i] > mine || (steps[i] == mine && i < t);
+  const int alone = 2 * places - n;
+  int at = rank;
+  if (alone >= 0) at = rank < alone ? n - places + rank : rank < places ? rank - alone : places + n - 1 - rank;
+  order[at] = t;
 }
 
 // The attention of single tokens and the recurrent mixer that stands beside it in one launch: neither fills the chip (32 and 64 blocks
@@ -2077,9 +2114,20 @@ static AttnArgs decode_args(const bf16_t* k_cache, const bf16_t* v_cache, const 
   return a;
 }
 
+// order [n]: see decode_order_kernel.  The mask's arguments as of tp_paged_attention.
+extern "C" int tp_decode_order(const int* context_lens, int n, int window, int keep_first, int chunk, int places, int* order, hipStream_t s) {
+  TP_REQUIRE(n > 0 && n <= DECODE_ORDER_ROWS && places > 0 && places < n, "decode_order: bad sizes (%d requests, %d places)", n, places);
+  TP_REQUIRE(window >= 0 && keep_first >= 0 && chunk >= 0 && chunk != 1 && (chunk == 0 || window == 0), "decode_order: bad mask");
+  const AttnArgs a = decode_args(nullptr, nullptr, nullptr, 0, nullptr, context_lens, nullptr, 1, 1, 16, 1.f, window, 1, 4, nullptr, keep_first, nullptr, chunk);
+  hipLaunchKernelGGL(decode_order_kernel, dim3(1), dim3(DECODE_ORDER_ROWS), 0, s, a, n, places, order);
+  TP_CHECK_LAUNCH("decode_order");
+  return 0;
+}
+
 // Single tokens from their projection's rows (see RowsIn and attn_decode_lds_kernel): n requests of one token each, heads of 64 or 128
 // elements, values alike, at most 16 heads a key head, pages of a power of two from 16 on.  beside: a step that tp_delta_step or
-// tp_linear_step wrote down, of the same requests, to run in the same launch (nullptr: none; then decode_waves is 8).  With num_splits > 1 scratch of n * n_heads *
+// tp_linear_step wrote down, of the same requests, to run in the same launch (nullptr: none; then decode_waves is 8).  order: of the requests
+// among the blocks (tp_decode_order), or nullptr.  With num_splits > 1 scratch of n * n_heads *
 // num_splits * (dim + 2) floats, and no convolution (a channel's carried inputs have one block).  gated: out as of tp_paged_attention
 // with allow_fast 2.
 extern "C" int tp_attention_rows(const float* rows, size_t part_stride, int stride, int parts, const float* conv_w, int taps, int channels,
@@ -2089,7 +2137,7 @@ extern "C" int tp_attention_rows(const float* rows, size_t part_stride, int stri
                                  const int* cu_seqlens, const int* context_lens, void* out, int n, int n_heads, int n_kv, int dim, int page_size,
                                  float scale, int window, int keep_first, int chunk, const float* sink, int num_splits, int decode_waves, float* scratch, int gated,
                                  const float* gate, int gate_stride, int gate_col0, int gate_per, float gate_scale, int out_stride, int out_col0,
-                                 const void* beside, hipStream_t s) {
+                                 const void* beside, const int* order, hipStream_t s) {
   TP_REQUIRE(n >= 0 && n <= 65535 && n_kv > 0 && n_heads > 0 && n_heads <= 65535 && n_heads % n_kv == 0 && n_heads / n_kv <= 16 && (dim == 64 || dim == 128),
              "attention_rows: bad heads (%d of %d, %d key heads)", n_heads, dim, n_kv);
   TP_REQUIRE(page_size >= 16 && (page_size & (page_size - 1)) == 0 && parts >= 1 && parts <= ROWS_PARTS && stride % 2 == 0 && part_stride % 2 == 0 &&
@@ -2113,6 +2161,7 @@ extern "C" int tp_attention_rows(const float* rows, size_t part_stride, int stri
   AttnArgs a = decode_args((const bf16_t*)k_cache, (const bf16_t*)v_cache, block_tables, table_width, cu_seqlens, context_lens, (bf16_t*)out, n_heads,
                            n_kv, page_size, scale, window, num_splits, decode_waves, scratch, keep_first, sink, chunk);
   a.all_single = true;
+  a.order = order;
   a.gated = gated != 0;
   a.gate = CombineGate{gate, gate_stride, gate_col0, gate_per, out_stride, out_col0, gate_scale};
   const RowsIn in = {rows, part_stride, stride, parts, conv_w, state, state_stride, state_off, state_slots, taps, channels, q_norm, k_norm, norm_eps,
@@ -2153,7 +2202,7 @@ int tp_paged_attention_fast(const void* q, const void* k_cache, const void* v_ca
                             int portion_splits, int portion_min_steps, float* portion_scratch, const float* dist_bias,
                             int bias_len, int keep_first, const float* sink, int value_dim, int chunk, float softcap,
                             int gated, const float* gate, int gate_stride, int gate_col0, int gate_per, float gate_scale, int out_stride,
-                            int out_col0, hipStream_t s) {
+                            int out_col0, const int* order, hipStream_t s) {
   if (head_dim % 32 != 0 || page_size % 8 != 0) return -1;
   if (dist_bias != nullptr && (value_dim != head_dim || softcap > 0.f)) return -1;
   if (chunk < 0 || chunk == 1 || (chunk > 0 && (window > 0 || keep_first > 0))) return -1;
@@ -2170,6 +2219,7 @@ int tp_paged_attention_fast(const void* q, const void* k_cache, const void* v_ca
                            n_kv, page_size, scale, window, num_splits, decode_waves, scratch, keep_first, sink, chunk);
   a.q = (const bf16_t*)q;
   a.all_single = num_single == n_req;
+  a.order = a.all_single ? order : nullptr;
   a.gated = gated != 0;
   a.gate = CombineGate{gate, gate_stride, gate_col0, gate_per, out_stride, out_col0, gate_scale};
   a.portion_splits = portion_splits;

@@ -1130,12 +1130,31 @@ def _decode_waves(requests: int, heads: int, kvh: int, splits: int) -> int:
     return 8 if splits == 1 and decode_rows_padded(requests) * kvh * ((heads // kvh + 15) // 16) <= 256 else 4
 
 
+def decode_order(shared: Optional[dict], context_lens: torch.Tensor, n: int, heads: int, kvh: int, splits: int, window: int, keep_first: int,
+                 chunk: int) -> Optional[torch.Tensor]:
+    """The order of a step's single tokens among the blocks of the kernel of ``decode_rings`` (int32 [n]), or None: as they are.  ``shared``: the
+    step's (``StepContext.shared``; without it no order is made): its layers with the same mask and heads share one."""
+    # (one launch a step, 2.4 us, and 0.2 us a layer; up to as many blocks as CUs there is nothing to choose)
+    per = kvh * ((heads // kvh + 15) // 16)
+    places = 256 // per
+    if shared is None or splits != 1 or not 0 < places < n <= 512 or _decode_waves(n, heads, kvh, splits) != 4:
+        return None
+    key = ("decode_order", n, places, int(window), int(keep_first), int(chunk))
+    if key not in shared:
+        _dev_ok(context_lens)
+        _i32(context_lens, n, "context_lens")
+        order = torch.empty((n,), dtype=torch.int32, device=context_lens.device)
+        _call("tp_decode_order", _ptr(context_lens), n, int(window), int(keep_first), int(chunk), places, _ptr(order), _stream())
+        shared[key] = order
+    return shared[key]
+
+
 def paged_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, block_tables: torch.Tensor,
                     cu_seqlens: torch.Tensor, context_lens: torch.Tensor, token_req: torch.Tensor,
                     scale: float, window: int, max_q_len: int, max_context_len: int,
                     num_single: Optional[int] = None, dist_bias: Optional[torch.Tensor] = None,
                     sink: Optional[torch.Tensor] = None, keep_first: int = 0, chunk: int = 0, softcap: float = 0.0,
-                    into: Optional[tuple] = None) -> Optional[torch.Tensor]:
+                    into: Optional[tuple] = None, shared: Optional[dict] = None) -> Optional[torch.Tensor]:
     """q [n, heads, head_dim] over k [pages, kv_heads, page_size, head_dim] and transposed
     v [pages, kv_heads, value_dim, page_size] -> [n, heads * value_dim] (value_dim is the value cache's own; the
     matrix-core kernels take the pairs of sizes in ``FAST_PAIRS``, other sizes run the general kernel).
@@ -1146,7 +1165,7 @@ def paged_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tenso
     ``chunk`` (instead of a window): a query sees the keys of its own aligned chunk of that many positions only.
     ``softcap`` > 0: a scaled score s becomes softcap * tanh(s / softcap) before the softmax (no distance bias then).
     ``into``: the last six arguments of ``sigmoid_gate`` (gate rows or None, their column, scale, output rows, their column, columns
-    that share a gate): the result goes there and None comes back."""
+    that share a gate): the result goes there and None comes back.  ``shared``: the step's (``StepContext.shared``, see ``decode_order``)."""
     if into is not None and not (_backend is None and num_single == block_tables.shape[0] == q.shape[0]):
         sigmoid_gate(paged_attention(q, k_cache, v_cache, block_tables, cu_seqlens, context_lens, token_req, scale, window, max_q_len,
                                      max_context_len, num_single, dist_bias, sink, keep_first, chunk, softcap), *into)
@@ -1202,11 +1221,13 @@ def paged_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tenso
     fast = allow_fast_attention and q.dtype == torch.bfloat16 and (d, vd) in FAST_PAIRS and page_size % 8 == 0
     fast = fast and (dist_bias is None or d == vd)
     fast = fast and fast_attention_takes(sink is not None, keep_first) and not (keep_first and dist_bias is not None)
-    splits, scratch = 1, None
+    splits, scratch, order = 1, None, None
     if fast and num_single > 0:
         splits = _decode_splits(num_single, heads, kvh, max_context_len, window, keep_first, chunk, dist_bias is None and decode_rings(d, vd, page_size))
         if splits > 1:
             scratch = torch.empty((r * heads * splits * (vd + 2),), dtype=torch.float32, device=q.device)
+        if num_single == r == n and dist_bias is None and decode_rings(d, vd, page_size):
+            order = decode_order(shared, context_lens, n, heads, kvh, splits, window, keep_first, chunk)
     fast_f32 = allow_fast_attention and q.dtype == torch.float32 and d == vd and d in (32, 64, 96, 128) and page_size % 16 == 0
     if fast_f32 and max_q_len == 1 and n == r:
         # (float32: at least 128 keys a block of four waves, by the same bound on the context as above, until there are
@@ -1249,7 +1270,7 @@ def paged_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tenso
           int(num_single), int(splits), _decode_waves(max(1, num_single), heads, kvh, splits), _ptr(scratch), int(parts), max(1, portion_min_keys // 32), _ptr(part_scratch),
           _ptr(dist_bias), 0 if dist_bias is None else dist_bias.shape[1], int(vd), int(keep_first), _ptr(sink), int(chunk),
           float(softcap), _ptr(gate), 0 if gate is None else gate.shape[1], int(gate_col0), int(per), float(factor),
-          dest.shape[1], int(dest_col0), _stream())
+          dest.shape[1], int(dest_col0), _ptr(order), _stream())
     if into is None:
         return dest
     if not gated:
@@ -1345,6 +1366,8 @@ def attention_rows(rows, col0: int, ctx, group: int, heads: int, kvh: int, dim: 
         chunk, window = 0, 1
     splits = _rows_splits(ctx, heads, kvh, window, keep_first, chunk, conv is not None, beside is not None)
     scratch = torch.empty((n * heads * splits * (dim + 2),), dtype=torch.float32, device=data.device) if splits > 1 else None
+    order = None if beside is not None else decode_order(getattr(ctx, "shared", None), ctx.context_lens, n, heads, kvh, splits, window,
+                                                         keep_first if window else 0, chunk)
     if into is not None:
         gate, gate_col0, gate_scale, out, out_col0, per = into
         _dev_ok(gate, out)
@@ -1362,7 +1385,7 @@ def attention_rows(rows, col0: int, ctx, group: int, heads: int, kvh: int, dim: 
           _ptr(inv_freq), int(rotary_dim), float(factor), _ptr(cos_sin), _ptr(slots), _ptr(k_cache), _ptr(v_cache), _ptr(bt), bt.shape[1],
           _ptr(ctx.cu_seqlens), _ptr(ctx.context_lens), _ptr(out), n, heads, kvh, dim, page_size, float(scale), int(window), int(keep_first),
           int(chunk), _ptr(sink), int(splits), 8 if beside is not None else _decode_waves(n, heads, kvh, splits), _ptr(scratch), int(into is not None), _ptr(gate), 0 if gate is None else gate.shape[1], int(gate_col0),
-          int(per), float(gate_scale), out.shape[1], int(out_col0), beside, _stream())
+          int(per), float(gate_scale), out.shape[1], int(out_col0), beside, _ptr(order), _stream())
     return None if into is not None else out
 
 

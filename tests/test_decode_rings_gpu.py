@@ -311,3 +311,42 @@ def test_portions_and_single_tokens_in_one_launch(heads, kv, d, vd, page, q_lens
         a, b = a.double().cpu(), b.double().cpu()
         assert float((a - b)[single].norm() / b[single].norm()) < 2.0 ** -8
         assert float((a - b).abs().max() / b.abs().max()) < 2.0 ** -6
+
+
+@pytest.mark.parametrize("n,places", [(33, 32), (48, 32), (64, 32), (65, 32), (130, 64), (2, 1), (512, 8)])
+def test_order_of_requests_among_blocks(n, places):
+    """Every request once; up to two a place: the longest alone, the others in pairs (place p and p + places), the longest with the shortest; else longest first."""
+    ops = _ops()
+    g = torch.Generator().manual_seed(n)
+    lens = torch.randint(1, 900, (n,), generator=g).to(torch.int32)
+    shared, kvh = {}, 256 // places
+    got = ops.decode_order(shared, lens.to(DEV), n, kvh, kvh, 1, 0, 0, 0).cpu().tolist()
+    assert len(shared) == 1 and sorted(got) == list(range(n))
+    rank = sorted(range(n), key=lambda i: (-((int(lens[i]) + 31) // 32), i))
+    if n > 2 * places:
+        assert got == rank
+        return
+    alone = 2 * places - n
+    assert got[n - places: places] == rank[:alone]
+    assert [(got[p], got[p + places]) for p in range(n - places)] == [(rank[alone + i], rank[n - 1 - i]) for i in range(n - places)]
+
+
+@pytest.mark.parametrize("heads,kv,d,n,longest", [(16, 8, 64, 33, 700), (16, 8, 128, 48, 1300), (5, 5, 128, 110, 300)])
+@pytest.mark.parametrize("mask", [{}, {"window": 100}, {"sink": True, "chunk": 200}])
+def test_ordered_requests_give_the_same_bits(heads, kv, d, n, longest, mask):
+    """With an order among the blocks and without: outputs and caches, from rows and from q."""
+    ops = _ops()
+    g = torch.Generator().manual_seed(n + d)
+    ctx, k, v = _step([1 + (i * 37 % n) * (longest - 1) // (n - 1) for i in range(n)], kv, d, 16, g)
+    rows = torch.randn(n, (heads + 2 * kv) * d, generator=g).to(DEV)
+    q = torch.randn(n, heads, d, generator=g).to(DEV).bfloat16()
+    if "sink" in mask:
+        mask = {**mask, "sink": torch.randn(heads, generator=g).to(DEV)}
+    outs = []
+    for shared in (None, {}):
+        ctx.shared, kk, vv = shared, k.clone(), v.clone()
+        a = ops.attention_rows(rows, 0, ctx, 0, heads, kv, d, kk, vv, d ** -0.5, None, 0, 1.0, None, **mask)
+        b = ops.paged_attention(q, kk, vv, ctx.block_tables[0], ctx.cu_seqlens, ctx.context_lens, ctx.token_req, d ** -0.5, mask.get("window", 0), 1,
+                                ctx.max_context_len, n, sink=mask.get("sink"), chunk=mask.get("chunk", 0), shared=shared)
+        outs.append((a, b, kk, vv))
+    assert len(ctx.shared) == 1 and all(torch.equal(x, y) for x, y in zip(*outs))

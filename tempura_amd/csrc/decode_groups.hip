@@ -24,24 +24,22 @@ __device__ inline f32x4_t dg_mfma(u32x4_t w, u32x4_t x, f32x4_t acc) {
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, w), __builtin_bit_cast(bf16x8_t, x), acc, 0, 0, 0);
 }
 
-// acc += the wave's runs of one 16-row tile of a weight: wp this lane's first piece of the tile, xp of the rows; steps of 32 k
+// acc += the wave's runs of one 16-row tile of a weight: wp this lane's first piece of the tile, xp of the rows; steps of 32 k.  One run on its way at a
+// time (see gemm_few_kernel in gemm_mfma.hip).  A decode step of Zemarax at width 4,096 494 -> 473 us with both, Golavik's 701 -> 675, Makisun's 461 -> 444.
 __device__ inline f32x4_t dg_tile(const u32x4_t* wp, const u32x4_t* xp, int xstep, int steps, int wave, f32x4_t acc) {
-  for (int s0 = wave * 4; s0 < steps; s0 += DG_WAVES * 8) {
-    u32x4_t a[2][4], b[2][4];
+  const int runs = steps / 4;      // (whole ones)
+  for (int run = wave; run < runs; run += DG_WAVES) {
+    u32x4_t a[4], b[4];
 #pragma unroll
-    for (int d = 0; d < 2; ++d)
+    for (int u = 0; u < 4; ++u) a[u] = __builtin_nontemporal_load(wp + (size_t)(run * 4 + u) * 64);
 #pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const int s = min(s0 + d * DG_WAVES * 4 + u, steps - 1);   // (steps past the end repeat the last one and are dropped below)
-        a[d][u] = __builtin_nontemporal_load(wp + (size_t)s * 64);
-        b[d][u] = xp[(size_t)s * xstep];
-      }
+    for (int u = 0; u < 4; ++u) b[u] = xp[(size_t)(run * 4 + u) * xstep];
+    __builtin_amdgcn_sched_barrier(0);      // (all of a run's loads in front of its first product)
 #pragma unroll
-    for (int d = 0; d < 2; ++d)
-#pragma unroll
-      for (int u = 0; u < 4; ++u)
-        if (s0 + d * DG_WAVES * 4 + u < steps) acc = dg_mfma(a[d][u], b[d][u], acc);
+    for (int u = 0; u < 4; ++u) acc = dg_mfma(a[u], b[u], acc);
   }
+  if (wave == runs % DG_WAVES)     // what is left of K, fewer than four steps
+    for (int s = runs * 4; s < steps; ++s) acc = dg_mfma(__builtin_nontemporal_load(wp + (size_t)s * 64), xp[(size_t)s * xstep], acc);
   return acc;
 }
 
@@ -131,7 +129,7 @@ extern "C" int tp_split_linear(const void* x, const void* w, float* out, int M, 
 // ---- a product that closes a sublayer over several copies of the stream ---------------------------
 // y = x w^T, then per row and column, in the order of hc_step_reg_kernel: h'[b] = sum_a mix[a, b] h[a] + outc[b] y, written back into
 // h [M, S, N]; with norm_w also u = sum_a inc[a] h'[a], handed over as xg = bfloat16(u * norm_w), k-blocked [N / 8, M, 8], and ss
-// [N / 16, 16], each block's sums of u^2 per row, for the next product to finish the norm (RowScale in gemm_mfma.hip).  The copies mix
+// [M, N / 16], each block's sums of u^2 per row, for the next product to finish the norm (RowScale in gemm_mfma.hip).  The copies mix
 // column by column, so the block that has a column's sum has all it needs; what it reads besides is requested before the weights.
 // Bound by the weights' stream, as the product alone.  Four copies, a captured chain, product and closing kernel / together, one row and
 // eight: 4,096 x 4,096 11.4 / 8.4 and 12.8 / 8.9 us, 4,096 x 14,336 25.2 / 22.1 and 26.5 / 22.8, 2,048 x 7,168 13.7 / 11.5 and 15.2 / 12.2,
@@ -195,12 +193,12 @@ __global__ __launch_bounds__(DG_WAVES * 64) void stream_linear_kernel(const bf16
   }
   if (e.norm_w == nullptr) return;   // (the same for every thread)
   __syncthreads();
-  if (threadIdx.x < 16)
-    e.ss[blockIdx.x * 16 + threadIdx.x] = part[0][threadIdx.x] + part[1][threadIdx.x] + part[2][threadIdx.x] + part[3][threadIdx.x];
+  if ((int)threadIdx.x < M)
+    e.ss[threadIdx.x * gridDim.x + blockIdx.x] = part[0][threadIdx.x] + part[1][threadIdx.x] + part[2][threadIdx.x] + part[3][threadIdx.x];
 }
 
 // x: bfloat16 [K / 8, M, 8] (blocked) or [M, K]; w: tiled [N, K]; h float32 [M, streams, N]; mix float32 [streams, streams], outc and inc
-// [streams], norm_w [N] (each may be nullptr); xg bfloat16 [N / 8, M, 8] and ss [N / 16, 16] with norm_w
+// [streams], norm_w [N] (each may be nullptr); xg bfloat16 [N / 8, M, 8] and ss [M, N / 16] with norm_w
 extern "C" int tp_stream_linear(const void* x, int blocked, const void* w, float* h, int streams, const float* mix, const float* outc,
                                 const float* inc, const float* norm_w, void* xg, float* ss, int M, int N, int K, hipStream_t s) {
   TP_REQUIRE(M > 0 && M <= 16 && N > 0 && N % 16 == 0 && K > 0 && K % 64 == 0, "stream_linear: sizes M %d N %d K %d", M, N, K);
@@ -378,29 +376,25 @@ __global__ __launch_bounds__(DG_WAVES * 64) void moe_down_kernel(const bf16_t* _
   // run r of expert e goes to wave (e * runs + r) % 8: `per` turns an expert
   const int per = (runs + DG_WAVES - 1) / DG_WAVES;
   f32x4_t acc = (f32x4_t){0.f, 0.f, 0.f, 0.f};
-  for (int it = 0; it < total * per; it += 2) {
-    u32x4_t av[2][4], bv[2][4];
-    int left[2];
+  for (int it = 0; it < total * per; ++it) {
+    const int e = __builtin_amdgcn_readfirstlane(list[it / per]);
+    const int run = it % per * DG_WAVES + ((wave - e * runs) & (DG_WAVES - 1));
+    if (run >= runs) continue;
+    const u32x4_t* wp = w_lane + (size_t)e * w_expert + (size_t)run * 256;
+    const u32x4_t* xp = x_lane + (size_t)e * x_expert + (size_t)run * 4 * xstep;
+    const int left = steps - run * 4;
+    if (left >= 4) {
+      u32x4_t av[4], bv[4];
 #pragma unroll
-    for (int d = 0; d < 2; ++d) {
-      const int i = min(it + d, total * per - 1);
-      const int e = __builtin_amdgcn_readfirstlane(list[i / per]);
-      const int run = i % per * DG_WAVES + ((wave - e * runs) & (DG_WAVES - 1));
-      left[d] = it + d < total * per && run < runs ? min(4, steps - run * 4) : 0;
-      const u32x4_t* wp = w_lane + (size_t)e * w_expert;
-      const u32x4_t* xp = x_lane + (size_t)e * x_expert;
+      for (int u = 0; u < 4; ++u) av[u] = __builtin_nontemporal_load(wp + u * 64);
 #pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const int s = min(run * 4 + u, steps - 1);
-        av[d][u] = __builtin_nontemporal_load(wp + (size_t)s * 64);
-        bv[d][u] = xp[(size_t)s * xstep];
-      }
+      for (int u = 0; u < 4; ++u) bv[u] = xp[(size_t)u * xstep];
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int u = 0; u < 4; ++u) acc = dg_mfma(av[u], bv[u], acc);
+    } else {
+      for (int u = 0; u < left; ++u) acc = dg_mfma(__builtin_nontemporal_load(wp + u * 64), xp[(size_t)u * xstep], acc);
     }
-#pragma unroll
-    for (int d = 0; d < 2; ++d)
-#pragma unroll
-      for (int u = 0; u < 4; ++u)
-        if (u < left[d]) acc = dg_mfma(av[d][u], bv[d][u], acc);
   }
 #pragma unroll
   for (int r = 0; r < 4; ++r) red[wave][lane * 4 + r] = acc[r];

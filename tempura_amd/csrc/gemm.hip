@@ -181,8 +181,8 @@ extern "C" int tp_linear_rope(const void* x, const void* w, int w_tiled, int M, 
 //
 // The split norm (bfloat16, at most 16 rows, K % 32 == 0): with `post_w` (a float32 norm weight [N]; accumulate
 // must be 1) the product also writes post_xg [M, N] = bfloat16(out * post_w) and post_ss
-// [ceil(N / 16), 16], per block of 16 columns and row the sum of squares of `out`.  With `pre_ss`
-// ([pre_count, 16], as written by such a product whose N is this product's K) the result rows are
+// [M, ceil(N / 16)], per row and block of 16 columns the sum of squares of `out`.  With `pre_ss`
+// ([M, pre_count], as written by such a product whose N is this product's K) the result rows are
 // multiplied by rsqrt(sum of squares / K + pre_eps): x is then that product's post_xg.
 //
 // `layout` (bfloat16, at most 16 rows): bit 0, x is k-blocked [K / 8, M, 8] instead of [M, K]; bit 1, the

@@ -1,14 +1,12 @@
 // bfloat16 products on the gfx950 matrix cores: out[M, N] (+)= x[M, K] * w[N, K]^T,
 // float32 accumulation (v_mfma_f32_16x16x32_bf16).
 //
-// Two kernels:
-//  * skinny (M <= 64, decode): weight-bandwidth bound.  A block owns 16 output columns
-//    (16 weight rows); its waves split K in interleaved 32-wide steps and each lane pulls
-//    its 16 bytes of a weight row straight from global memory into the MFMA operand
-//    registers (no LDS: a weight is used by exactly one wave).  The activations are the
-//    other operand, read through the caches.  Partial tiles are summed through LDS in a
-//    fixed order, so results are deterministic and a row's value does not depend on the
-//    other rows of the batch.
+// Three kernels:
+//  * few (M <= 16, a decode step): bound by the weights' stream from memory.  A block owns 16 output columns (16 weight rows); its eight
+//    waves split K in runs of 128 and each lane pulls its 16 bytes of a weight row straight from global memory into the MFMA operand
+//    registers (no LDS: a weight is used by exactly one wave).  Partial tiles are summed through LDS in the order of the waves, so results
+//    are deterministic and a row's value does not depend on the other rows of the batch.
+//  * skinny (17 to 64 rows without scratch): the same with two to four tiles of rows.
 //  * tiled (M > 64, prefill): 128x128 block tile, 64x64 per wave, K in steps of 64 (or
 //    32), operands staged through padded LDS tiles; the next tile is fetched into
 //    registers while the current one is multiplied.
@@ -80,19 +78,25 @@ __device__ inline void store_split(void* out, int layout, const GateAct& ga, int
     ga.side[(size_t)m * ga.side_ld + n - ga.act_cols] = v;
 }
 
+// What the rotation of one column of one row reads besides its sums, requested before the weights.
+struct RopeIn {
+  float2 cs;
+  int slot;
+};
+__device__ inline RopeIn rope_request(const RopeOut& rp, int m, int n) {
+  RopeIn in = {make_float2(1.f, 0.f), rp.slots[m]};
+  const int d = n % rp.head_dim;
+  if (rp.cos_sin != nullptr) in.cs = rp.cos_sin[(size_t)m * (rp.rotary_dim >> 1) + min(d, max(rp.rotary_dim - 1, 0)) / 2];
+  return in;
+}
+
 // v: this lane's sum of column n of row m; other: the sum of column n ^ 1 (the partner of a rotary pair)
-__device__ inline void rope_store(const RopeOut& rp, int m, int n, float v, float other) {
+__device__ inline void rope_store(const RopeOut& rp, const RopeIn& in, int m, int n, float v, float other) {
   const int h = n / rp.head_dim, d = n % rp.head_dim;
   float y = v;
   if (h < rp.n_heads + rp.n_kv && d < rp.rotary_dim) {
-    float c, sn;
-    if (rp.cos_sin != nullptr) {
-      const float2 cs = rp.cos_sin[(size_t)m * (rp.rotary_dim >> 1) + (d >> 1)];
-      c = cs.x;
-      sn = cs.y;
-    } else {
-      rope_cos_sin(rp.positions[m], rp.inv_freq[d >> 1], rp.factor, c, sn);
-    }
+    float c = in.cs.x, sn = in.cs.y;
+    if (rp.cos_sin == nullptr) rope_cos_sin(rp.positions[m], rp.inv_freq[d >> 1], rp.factor, c, sn);
     // the pair is (x0, x1) = (even column, odd column): x0 c - x1 s and x0 s + x1 c
     y = (d & 1) ? other * sn + v * c : v * c - other * sn;
   }
@@ -100,8 +104,7 @@ __device__ inline void rope_store(const RopeOut& rp, int m, int n, float v, floa
     rp.q_out[((size_t)m * rp.n_heads + h) * rp.head_dim + d] = float_to_bf16(y);
     return;
   }
-  const int slot = rp.slots[m];
-  const size_t page = (size_t)(slot / rp.page_size), off = (size_t)(slot % rp.page_size);
+  const size_t page = (size_t)(in.slot / rp.page_size), off = (size_t)(in.slot % rp.page_size);
   if (h < rp.n_heads + rp.n_kv)
     rp.k_cache[((page * rp.n_kv + (h - rp.n_heads)) * rp.page_size + off) * rp.head_dim + d] = float_to_bf16(y);
   else
@@ -117,108 +120,206 @@ __device__ inline void rope_store(const RopeOut& rp, int m, int n, float v, floa
 struct NormPrep {
   const float* w;    // norm weight [N]; nullptr: no preparation
   bf16_t* xg;        // [M, N]
-  float* ss;         // [blocks, 16]
+  float* ss;         // [M, blocks]
 };
 struct RowScale {
-  const float* ss;   // [count, 16] partial sums of squares; nullptr: no scaling
+  const float* ss;   // [M, count] partial sums of squares; nullptr: no scaling
   int count;
   float inv_k, eps;
 };
 
-// RowScale, first half: every thread fetches its share of the partial sums of one row.  The loads are
-// issued together, early (before the main loop), and nothing waits for them until the second half.
-struct RowScaleLoads {
-  float v[8];
+// ---- few rows ---------------------------------------------------------------------------
+// What happens to the sums: stored (float32, bfloat16, added into float32), the gated SiLU, added into the stream with the next norm prepared,
+// rotation and cache, the split epilogue (mode OUT_SPLIT, or a gate with constants).  Each is a kernel of its own: what one of them
+// needs of constants and branches costs every other half a microsecond.  (The split epilogue: an activation's own launch and trip through memory, 4.9 us behind
+// a product of one row, is gone.)
+enum { FEW_STORE, FEW_SWIGLU, FEW_POST, FEW_ROPE, FEW_SPLIT };
+#define FEW_WAVES 8
+#define FEW_RED 80      // floats between the four column groups of a wave's tile: a thread a (row, column) then reads without more conflicts than 64 lanes have anyway
+
+// The wave's share of K: runs of four steps of 32 (256 contiguous bytes of each weight row), run r to wave r % 8, one run on its way at a
+// time, and nothing between the loads but their addresses: a loop whose loads stand behind conditions (a second run only where there is one, a chunk of rows
+// only for the threads that copy it) waits for every load on its way at each join, and what the epilogue reads of the kernel's arguments must not
+// stand in front of the first load either.  From memory, a captured chain, float32 results, against two runs at a time with such conditions
+// (plain reads of the same bytes: 4.5, 6.1, 16.7, 6.5, 9.2, 19.5 us): one row of K x N 3,072 x 3,072 6.6 -> 5.0 us, 3,072 x 5,120 10.2 -> 7.4, 3,072 x 16,384 20.0 -> 16.4,
+// 4,096 x 4,096 7.9 -> 6.9, 8,192 x 3,072 11.5 -> 9.7, 14,336 x 4,096 21.1 -> 18.9; eight rows 6.2 -> 5.2, 9.4 -> 8.3, 18.6 -> 16.8, 8.8 -> 6.9,
+// 13.5 -> 10.4, 21.8 -> 18.9.  Sixteen waves with a run each: the same within 3 %.
+// P > 0: row-major rows through LDS, P pieces of 16 bytes a thread (padded rows: 16-byte reads of 16 rows then hit different banks); 0: straight from memory.
+// PRE: the norm of the rows is finished here (RowScale).
+// What the end reads of the arguments stands in one structure behind those that arrive in registers.  It is read through few_end(), behind the first
+// requests: the compiler asks for a structure's members at the start of a kernel and waits for them at its first branch.
+struct FewEnd {
+  RowScale pre;
+  NormPrep post;
+  RopeOut rp;
 };
-__device__ inline RowScaleLoads row_scale_begin(const RowScale& pre, int nthreads) {
-  RowScaleLoads ld;
+#define FEW_END_AT 48      // x, w, out and five numbers are 44 bytes
+template <typename T>
+using constant_ptr = const __attribute__((address_space(4))) T*;
+__device__ inline constant_ptr<FewEnd> few_end() {
+  constant_ptr<char> args = (constant_ptr<char>)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(args)::"memory");
+  return (constant_ptr<FewEnd>)(args + FEW_END_AT);
+}
+
+template <int P, int KIND, bool PRE, bool WT>
+__global__ __launch_bounds__(FEW_WAVES * 64) void gemm_few_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w, void* __restrict__ out, int M,
+                                                                  int N, int K, int mode, int layout, FewEnd) {
+  constexpr int T = FEW_WAVES * 64;
+  extern __shared__ __attribute__((aligned(16))) unsigned char rows_lds[];
+  __shared__ __attribute__((aligned(16))) float red[FEW_WAVES][4 * FEW_RED];
+  __shared__ float rstd[16];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int g = lane >> 4, row = min(lane & 15, M - 1), n0 = blockIdx.x * 16;
+  const int steps = K / 32, ld = K * 2 + 16;
+  u32x4_t xv[P > 0 ? P : 1];
+  if constexpr (P > 0) {
+    const int total = M * (K / 8);
 #pragma unroll
-  for (int i = 0; i < 8; ++i) ld.v[i] = 0.f;
-  if (pre.ss == nullptr) return ld;
-  const int t = threadIdx.x, nparts = min(nthreads / 16, 32);
-  if (t < nparts * 16) {
-    const int m = t & 15, p = t >> 4;
+    for (int i = 0; i < P; ++i) xv[i] = ((const u32x4_t*)x)[min(i * T + tid, total - 1)];
+  }
+  const u32x4_t* wp = WT ? (const u32x4_t*)(w + (size_t)n0 * K) + lane : (const u32x4_t*)(w + (size_t)min(n0 + (lane & 15), N - 1) * K) + g;
+  constexpr int wstep = WT ? 64 : 4;   // u32x4 units per 32 of k
+  const bool blocked = (layout & X_KBLOCKED) != 0;
+  const u32x4_t* xp = (const u32x4_t*)x + (blocked ? g * M + row : row * (K / 8) + g);
+  const int xstep = blocked ? 4 * M : 4;
+  u32x4_t a[4], b[4];
+  auto request = [&](int run) __attribute__((always_inline)) {
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const int b = p + i * nparts;
-      if (b < pre.count) ld.v[i] = pre.ss[b * 16 + m];
+    for (int u = 0; u < 4; ++u) a[u] = TP_WLOAD(wp + (size_t)(run * 4 + u) * wstep);
+    if constexpr (P == 0) {
+#pragma unroll
+      for (int u = 0; u < 4; ++u) b[u] = xp[(size_t)(run * 4 + u) * xstep];
+    }
+  };
+  f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
+  auto multiply = [&](int run) __attribute__((always_inline)) {
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const u32x4_t bv = P == 0 ? b[u] : *(const u32x4_t*)(rows_lds + (size_t)row * ld + (run * 4 + u) * 64 + g * 16);
+      acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_frag(a[u]), as_frag(bv), acc, 0, 0, 0);
+    }
+  };
+  const int runs = steps / 4;      // (whole ones)
+  if (wave < runs) request(wave);
+  const constant_ptr<FewEnd> end = few_end();
+  const RowScale pre = {end->pre.ss, end->pre.count, end->pre.inv_k, end->pre.eps};
+  const NormPrep post = {end->post.w, end->post.xg, end->post.ss};
+  RopeOut rp;
+  if constexpr (KIND == FEW_ROPE || KIND == FEW_SPLIT) __builtin_memcpy(&rp, (const void*)(uintptr_t)&end->rp, sizeof(rp));
+  // what the end needs besides the sums.  A thread of the first four waves has row m, column n; the others repeat them.
+  const int m = (tid >> 4) & 15, n = n0 + (tid & 15), mc = min(m, M - 1), nc = min(n, N - 1);
+  float held = 0.f, wn = 0.f;
+  if constexpr (KIND == FEW_POST) {
+    held = ((const float*)out)[(size_t)mc * N + nc];
+    wn = post.w[nc];
+  }
+  RopeIn turn;
+  if constexpr (KIND == FEW_ROPE) turn = rope_request(rp, mc, nc);
+  float parts[2][4] = {};      // wave v adds up rows v and v + 8: a lane has every 64th partial sum
+  if constexpr (PRE) {
+    const int last = pre.count - 1;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) parts[0][j] = pre.ss[min(wave, M - 1) * pre.count + min(lane + 64 * j, last)];
+    if (M > 8) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) parts[1][j] = pre.ss[min(wave + 8, M - 1) * pre.count + min(lane + 64 * j, last)];
     }
   }
-  return ld;
-}
-// Second half: call after a barrier and follow with one; afterwards rstd[m] is valid for every thread.
-__device__ inline void row_scale_finish(const RowScale& pre, const RowScaleLoads& ld, float (*part)[16], float* rstd,
-                                        int nthreads) {
-  const int t = threadIdx.x, nparts = min(nthreads / 16, 32);
-  if (pre.ss == nullptr) {
-    if (t < 16) rstd[t] = 1.0f;
-    return;
-  }
-  if (t < nparts * 16) {
-    const int m = t & 15, p = t >> 4;
-    float sum = 0.f;
+  if constexpr (P > 0) {
+    const int kc = K / 8, total = M * kc;
 #pragma unroll
-    for (int i = 0; i < 8; ++i) sum += ld.v[i];
-    for (int b = p + 8 * nparts; b < pre.count; b += nparts) sum += pre.ss[b * 16 + m];   // more than 8 each: rare
-    part[p][m] = sum;
+    for (int i = 0; i < P; ++i) {
+      const int e = min(i * T + tid, total - 1), r = M == 1 ? 0 : e / kc;
+      *(u32x4_t*)(rows_lds + (size_t)r * ld + (e - r * kc) * 16) = xv[i];
+    }
+    // (not __syncthreads: it would wait for the weights as well)
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+  }
+  if (wave < runs) multiply(wave);
+  for (int run = wave + FEW_WAVES; run < runs; run += FEW_WAVES) {
+    request(run);
+    __builtin_amdgcn_sched_barrier(0);      // (all of a run's loads in front of its first product)
+    multiply(run);
+  }
+  if (wave == runs % FEW_WAVES) {      // what is left of K, fewer than four steps
+    for (int st = runs * 4; st < steps; ++st) {
+      const u32x4_t av = TP_WLOAD(wp + (size_t)st * wstep);
+      const u32x4_t bv = P == 0 ? xp[(size_t)st * xstep] : *(const u32x4_t*)(rows_lds + (size_t)row * ld + st * 64 + g * 16);
+      acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_frag(av), as_frag(bv), acc, 0, 0, 0);
+    }
+  }
+  *(f32x4_t*)(&red[wave][g * FEW_RED + (lane & 15) * 4]) = acc;
+  if constexpr (PRE) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      if (wave + 8 * i >= M) break;
+      float sum = 0.f;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) sum += lane + 64 * j < pre.count ? parts[i][j] : 0.f;
+      for (int c = lane + 256; c < pre.count; c += 64) sum += pre.ss[(wave + 8 * i) * pre.count + c];
+      sum = wave_sum(sum);
+      if (lane == 0) rstd[wave + 8 * i] = rsqrtf(sum * pre.inv_k + pre.eps);
+    }
   }
   __syncthreads();
-  if (t < 16) {
-    float sum = 0.f;
-    for (int p = 0; p < nparts; ++p) sum += part[p][t];
-    rstd[t] = rsqrtf(sum * pre.inv_k + pre.eps);
+  if (wave >= 4 || wave * 4 >= M) return;
+  // the waves' partial tiles in wave order
+  const int at = ((tid & 15) >> 2) * FEW_RED + m * 4 + (tid & 3);
+  float v = 0.f;
+#pragma unroll
+  for (int i = 0; i < FEW_WAVES; ++i) v += red[i][at];
+  if constexpr (PRE) v *= rstd[mc];
+  const bool mine = n < N && m < M;
+  const bool gated = KIND == FEW_SWIGLU || (KIND == FEW_SPLIT && mode == OUT_SWIGLU);
+  if (gated) {
+    const float up = row_rotated<8>(v);      // a gate row's up row is eight further on
+    if ((tid & 15) < 8 && n + 8 < N && m < M)
+      store_gated(out, layout, M, N / 2, m, n0 / 2 + (tid & 15), KIND == FEW_SPLIT ? gated_few(v, up, rp.gate) : silu_mul(v, up));
+  } else if constexpr (KIND == FEW_SPLIT) {
+    if (mine) store_split(out, layout, rp.gate, M, m, n, v);
+  } else if constexpr (KIND == FEW_POST) {
+    // residual add, and the next norm's preparation
+    const float h = held + v;
+    if (mine) {
+      ((float*)out)[(size_t)m * N + n] = h;
+      // (k-blocked on request: the product that consumes these rows then reads them straight from memory as operands)
+      post.xg[(layout & XG_KBLOCKED) ? ((size_t)(n >> 3) * M + m) * 8 + (n & 7) : (size_t)m * N + n] = float_to_bf16(h * wn);
+    }
+    const float sq = row_sum(mine ? h * h : 0.f);
+    if ((tid & 15) == 0 && m < M) post.ss[m * gridDim.x + blockIdx.x] = sq;
+  } else if constexpr (KIND == FEW_ROPE) {
+    const float other = __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0xB1, 0xf, 0xf, false));   // column n ^ 1
+    if (mine) rope_store(rp, turn, m, n, v, other);
+  } else if (mine) {
+    store_out(out, mode, (size_t)m * N + n, v);
   }
 }
 
-// ---- skinny ---------------------------------------------------------------------------
-// MT: 16-row tiles of activations; NT: 16-row tiles of weights per block; WAVES: waves that
-// split K.  A wave takes K in runs of four consecutive 32-wide steps (256 contiguous bytes of
-// each weight row), run r going to wave r % WAVES.
-// SPLIT: mode OUT_SPLIT, or OUT_SWIGLU with a gate that has constants, in kernels of their own (these branches in the others' epilogue
-// cost every short product half a microsecond).  The activation's own launch and trip through memory, 4.9 us behind a product of one
-// row, is gone: both products of a feed-forward, 16,384 x 4,096, one row 48.1 -> 46.0 us (gate with constants 66.9 -> 64.8), 16 rows
-// 56.4 -> 53.5 (83.9 -> 74.7: the down product takes k-blocked rows as well).
-template <int MT, int NT, int WAVES, int DEPTH, bool WT, bool SPLIT>
-__global__ __launch_bounds__(WAVES * 64) void gemm_skinny_mfma_kernel(const bf16_t* __restrict__ x,
-                                                                      const bf16_t* __restrict__ w,
-                                                                      void* __restrict__ out, int mode, int M,
-                                                                      int N, int K, int layout, RowScale pre,
-                                                                      NormPrep post, RopeOut rp) {
-  __shared__ float red[WAVES][NT * MT][256];
-  __shared__ float rs_part[32][16], rstd[16], ss_lds[NT][4][16];
+// ---- 17 to 64 rows ------------------------------------------------------------------------
+// The same without scratch for the pipelined kernels: MT 16-row tiles of activations; WAVES waves split K, DEPTH runs on their way.
+// SPLIT: mode OUT_SPLIT, or OUT_SWIGLU with a gate that has constants.
+template <int MT, int WAVES, int DEPTH, bool WT, bool SPLIT>
+__global__ __launch_bounds__(WAVES * 64) void gemm_skinny_mfma_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w,
+                                                                      void* __restrict__ out, int mode, int M, int N, int K, GateAct gate) {
+  __shared__ float red[WAVES][MT][256];
   const int lane = threadIdx.x % 64, wave = threadIdx.x / 64;
-  const int n0 = blockIdx.x * 16 * NT;
+  const int n0 = blockIdx.x * 16;
   const int kofs = (lane >> 4) * 8;
-  const u32x4_t* wp[NT];
-#pragma unroll
-  for (int j = 0; j < NT; ++j) {
-    const int wrow = min(n0 + j * 16 + (lane & 15), N - 1);
-    wp[j] = WT ? (const u32x4_t*)(w + (size_t)min(n0 + j * 16, N - 16) * K) + lane
-                               : (const u32x4_t*)(w + (size_t)wrow * K + kofs);
-  }
+  const int wrow = min(n0 + (lane & 15), N - 1);
+  const u32x4_t* wp = WT ? (const u32x4_t*)(w + (size_t)min(n0, N - 16) * K) + lane : (const u32x4_t*)(w + (size_t)wrow * K + kofs);
   constexpr int wstep = WT ? 64 : 4;   // u32x4 units per 32 of k (a compile-time stride: the four loads of a run share one address)
-  // x is [M, K] row-major, or (xblocked, M <= 16) [K / 8, M, 8]: eight consecutive k of all rows side by
-  // side, so that the 16 bytes the lanes of a wave fetch lie next to each other
   const u32x4_t* xp[MT];
-  const bool xblocked = (layout & X_KBLOCKED) != 0;
-  const int xstep = xblocked ? 4 * M : 4;   // u32x4 units per 32 of k
 #pragma unroll
-  for (int t = 0; t < MT; ++t) {
-    const int xrow = min(t * 16 + (lane & 15), M - 1);
-    xp[t] = xblocked ? (const u32x4_t*)(x + ((size_t)(lane >> 4) * M + xrow) * 8) : (const u32x4_t*)(x + (size_t)xrow * K + kofs);
-  }
-  f32x4_t acc[NT][MT];
+  for (int t = 0; t < MT; ++t) xp[t] = (const u32x4_t*)(x + (size_t)min(t * 16 + (lane & 15), M - 1) * K + kofs);
+  f32x4_t acc[MT];
 #pragma unroll
-  for (int j = 0; j < NT; ++j)
-#pragma unroll
-    for (int t = 0; t < MT; ++t) acc[j][t] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
-
-  const RowScaleLoads rs_loads = row_scale_begin(pre, WAVES * 64);
+  for (int t = 0; t < MT; ++t) acc[t] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
   const int steps = K / 32;  // a step is 32 k = 4 u32x4 per row
-  // DEPTH runs of four steps are fetched before any of them is multiplied: 4 * DEPTH * NT loads
-  // of 16 bytes per lane are in flight, which is what keeps the memory system busy.
   for (int s0 = wave * 4; s0 < steps; s0 += WAVES * 4 * DEPTH) {
-    u32x4_t a[DEPTH][NT][4];
+    u32x4_t a[DEPTH][4];
     u32x4_t b[DEPTH][MT][4];
 #pragma unroll
     for (int d = 0; d < DEPTH; ++d)
@@ -226,10 +327,9 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_mfma_kernel(const bf16
       for (int u = 0; u < 4; ++u) {
         // steps past the end repeat the last one; their products are dropped below
         const int sidx = min(s0 + d * WAVES * 4 + u, steps - 1);
+        a[d][u] = TP_WLOAD(wp + (size_t)sidx * wstep);
 #pragma unroll
-        for (int j = 0; j < NT; ++j) a[d][j][u] = TP_WLOAD(wp[j] + (size_t)sidx * wstep);
-#pragma unroll
-        for (int t = 0; t < MT; ++t) b[d][t][u] = xp[t][(size_t)sidx * xstep];
+        for (int t = 0; t < MT; ++t) b[d][t][u] = xp[t][(size_t)sidx * 4];
       }
 #pragma unroll
     for (int d = 0; d < DEPTH; ++d)
@@ -237,231 +337,35 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_mfma_kernel(const bf16
       for (int u = 0; u < 4; ++u) {
         if (s0 + d * WAVES * 4 + u < steps) {
 #pragma unroll
-          for (int t = 0; t < MT; ++t)
-#pragma unroll
-            for (int j = 0; j < NT; ++j)
-              acc[j][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_frag(a[d][j][u]), as_frag(b[d][t][u]), acc[j][t], 0, 0, 0);
+          for (int t = 0; t < MT; ++t) acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_frag(a[d][u]), as_frag(b[d][t][u]), acc[t], 0, 0, 0);
         }
       }
   }
   // sum the waves' partial tiles in wave order
 #pragma unroll
-  for (int j = 0; j < NT; ++j)
+  for (int t = 0; t < MT; ++t)
 #pragma unroll
-    for (int t = 0; t < MT; ++t)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) red[wave][j * MT + t][lane * 4 + r] = acc[j][t][r];
+    for (int r = 0; r < 4; ++r) red[wave][t][lane * 4 + r] = acc[t][r];
   __syncthreads();
-  row_scale_finish(pre, rs_loads, rs_part, rstd, WAVES * 64);
-  __syncthreads();
-  for (int e = threadIdx.x; e < NT * MT * 256; e += WAVES * 64) {
-    const int jt = e / 256, q = e % 256;
-    const int j = jt / MT, t = jt % MT;
+  for (int e = threadIdx.x; e < MT * 256; e += WAVES * 64) {
+    const int t = e / 256, q = e % 256;
     float v = 0.f;
 #pragma unroll
-    for (int i = 0; i < WAVES; ++i) v += red[i][jt][q];
+    for (int i = 0; i < WAVES; ++i) v += red[i][t][q];
     const int l = q / 4, r = q % 4;
-    const int n = n0 + j * 16 + (l >> 4) * 4 + r;   // weight row = output column
+    const int n = n0 + (l >> 4) * 4 + r;   // weight row = output column
     const int m = t * 16 + (l & 15);
-    if (MT == 1) v *= rstd[l & 15];
     if (SPLIT && mode == OUT_SPLIT) {
-      if (n < N && m < M) store_split(out, layout, rp.gate, M, m, n, v);
+      if (n < N && m < M) store_split(out, 0, gate, M, m, n, v);
     } else if (SPLIT || mode == OUT_SWIGLU) {
       if ((l >> 4) < 2 && n + 8 < N && m < M) {       // a gate row: its up row is eight further on
         float u = 0.f;
 #pragma unroll
-        for (int i = 0; i < WAVES; ++i) u += red[i][jt][q + 128];
-        if (MT == 1) u *= rstd[l & 15];
-        store_gated(out, layout, M, N / 2, m, (n0 + j * 16) / 2 + (l >> 4) * 4 + r, SPLIT ? gated_few(v, u, rp.gate) : silu_mul(v, u));
+        for (int i = 0; i < WAVES; ++i) u += red[i][t][q + 128];
+        store_gated(out, 0, M, N / 2, m, n0 / 2 + (l >> 4) * 4 + r, SPLIT ? gated_few(v, u, gate) : silu_mul(v, u));
       }
-    } else if (MT == 1 && post.w != nullptr) {
-      // residual add, and the next norm's preparation (mode is OUT_ACC_F32)
-      float sq = 0.f;
-      if (n < N && m < M) {
-        float* o = (float*)out + (size_t)m * N + n;
-        const float h = *o + v;
-        *o = h;
-        // (k-blocked on request: the product that consumes these rows then reads them straight from memory as operands)
-        post.xg[(layout & XG_KBLOCKED) ? ((size_t)(n >> 3) * M + m) * 8 + (n & 7) : (size_t)m * N + n] = float_to_bf16(h * post.w[n]);
-        sq = h * h;
-      }
-      sq += __shfl_xor(sq, 1, 64);      // the four columns r = 0..3 of this row
-      sq += __shfl_xor(sq, 2, 64);
-      if (r == 0) ss_lds[j][l >> 4][l & 15] = sq;
-    } else if (mode == OUT_ROPE) {
-      const float other = __shfl_xor(v, 1, 64);   // r and r ^ 1 are neighbouring lanes
-      if (n < N && m < M) rope_store(rp, m, n, v, other);
     } else if (n < N && m < M) {
       store_out(out, mode, (size_t)m * N + n, v);
-    }
-  }
-  if (MT == 1 && post.w != nullptr) {
-    __syncthreads();
-    if (threadIdx.x < 16) {
-      float sum = 0.f;
-#pragma unroll
-      for (int j = 0; j < NT; ++j)
-#pragma unroll
-        for (int c = 0; c < 4; ++c) sum += ss_lds[j][c][threadIdx.x];
-      post.ss[blockIdx.x * 16 + threadIdx.x] = sum;
-    }
-  }
-}
-
-// ---- skinny, activations through LDS (M <= 16) ------------------------------------------
-// With more than one activation row the second operand is a gather of short pieces of several
-// rows, and the address path, not HBM, limits the kernel.  Here the block copies the
-// activations of one K chunk (1,024 wide) into LDS with wide coalesced loads and every wave
-// reads its operand fragments from there; the weight stream is as above, one run of four steps
-// per wave and chunk, the next chunk's weights and activations already in flight while this
-// chunk is multiplied.  Two LDS buffers, one barrier per chunk.  The LDS row is padded by 8 elements:
-// 16-byte reads of 16 rows then hit 64 different banks.
-#define LKC 1024            // K elements per chunk with eight waves
-
-// A wave's weights of four chunks (one run per chunk) and the activations of two chunks are requested
-// before anything is multiplied, and again as soon as their registers are free, always in the order in
-// which they are consumed (loads return in order): a block has 256 bytes per lane in flight from its
-// first cycle.  (Measured against one chunk of prefetch: 5-10 % faster at 8 and 16 rows.)
-template <int NT, int WAVES, bool WT, bool SPLIT>
-__global__ __launch_bounds__(WAVES * 64) void gemm_skinny_lds_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w,
-                                                               void* __restrict__ out, int mode, int M, int N, int K,
-                                                               int layout, RowScale pre, NormPrep post, RopeOut rp) {
-  constexpr int THREADS = WAVES * 64, G = 1;
-  constexpr int KC = WAVES * 128;        // K elements per chunk: one run of four steps per wave
-  constexpr int LD = KC + 8;             // padded LDS row
-  constexpr int TPR = THREADS / 16;      // threads that copy one activation row, 16 bytes each, four passes
-  __shared__ __attribute__((aligned(16))) uint16_t xs[2][16 * LD];
-  __shared__ float red[WAVES][NT][256];
-  __shared__ float rs_part[32][16], rstd[16], ss_lds[NT][4][16];
-  const int tid = threadIdx.x, lane = tid % 64, wave = tid / 64;
-  const int kw = wave;
-  const int n0 = blockIdx.x * 16 * NT;
-  const int kofs = (lane >> 4) * 8;
-  const u32x4_t* wp[NT];
-#pragma unroll
-  for (int j = 0; j < NT; ++j) {
-    const int wrow = min(n0 + j * 16 + (lane & 15), N - 1);
-    wp[j] = WT ? (const u32x4_t*)(w + (size_t)min(n0 + j * 16, N - 16) * K) + lane
-                               : (const u32x4_t*)(w + (size_t)wrow * K + kofs);
-  }
-  constexpr int wstep = WT ? 64 : 4;
-  const int xrow = tid / TPR, xcol = (tid % TPR) * 8;
-  const bool xload = xrow < M;
-  const bf16_t* xsrc = x + (size_t)min(xrow, M - 1) * K + xcol;
-  f32x4_t acc[NT];
-#pragma unroll
-  for (int j = 0; j < NT; ++j) acc[j] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
-  const int steps = K / 32;
-  const int chunks = (K + KC - 1) / KC;
-
-  u32x4_t a[4][NT][4], xr[2][4];
-  auto load_w = [&](int ch, int slot) {
-    const int s0 = ch * (KC / 32) + kw * 4;
-#pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      const int sidx = min(s0 + u, steps - 1);
-#pragma unroll
-      for (int j = 0; j < NT; ++j) a[slot][j][u] = TP_WLOAD(wp[j] + (size_t)sidx * wstep);
-    }
-  };
-  auto load_x = [&](int ch, int slot) {
-    if (xload) {
-#pragma unroll
-      for (int p = 0; p < 4; ++p) {
-        const int k = ch * KC + p * TPR * 8 + xcol;
-        xr[slot][p] = (k < K) ? *(const u32x4_t*)(xsrc + (size_t)ch * KC + p * TPR * 8) : (u32x4_t){0u, 0u, 0u, 0u};
-      }
-    }
-  };
-  load_x(0, 0);
-  load_w(0, 0);
-  if (chunks > 1) { load_x(1, 1); load_w(1, 1); }
-  if (chunks > 2) load_w(2, 2);
-  if (chunks > 3) load_w(3, 3);
-  const RowScaleLoads rs_loads = row_scale_begin(pre, THREADS);
-  for (int ch0 = 0; ch0 < chunks; ch0 += 4) {
-#pragma unroll
-    for (int c = 0; c < 4; ++c) {
-      const int ch = ch0 + c;
-      if (ch < chunks) {
-        const int buf = c & 1;
-        if (xload) {
-#pragma unroll
-          for (int p = 0; p < 4; ++p) *(u32x4_t*)(&xs[buf][xrow * LD + p * TPR * 8 + xcol]) = xr[c & 1][p];
-        }
-        __syncthreads();
-        if (ch + 2 < chunks) load_x(ch + 2, c & 1);
-        const int s0 = ch * (KC / 32) + kw * 4;
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-          if (s0 + u < steps) {
-            const u32x4_t b = *(const u32x4_t*)(&xs[buf][(lane & 15) * LD + (kw * 4 + u) * 32 + kofs]);
-#pragma unroll
-            for (int j = 0; j < NT; ++j)
-              acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_frag(a[c][j][u]), as_frag(b), acc[j], 0, 0, 0);
-          }
-        }
-        if (ch + 4 < chunks) load_w(ch + 4, c);
-      }
-    }
-  }
-#pragma unroll
-  for (int j = 0; j < NT; ++j)
-#pragma unroll
-    for (int r = 0; r < 4; ++r) red[wave][j][lane * 4 + r] = acc[j][r];
-  __syncthreads();
-  row_scale_finish(pre, rs_loads, rs_part, rstd, THREADS);
-  __syncthreads();
-  for (int e = tid; e < G * NT * 256; e += THREADS) {
-    const int gj = e / 256, q = e % 256;
-    const int ge = gj / NT, j = gj % NT;            // the group and tile this element belongs to
-    const int nt0 = ((blockIdx.x * G + ge) * NT + j) * 16;
-    float v = 0.f;
-#pragma unroll
-    for (int i = 0; i < WAVES; ++i) v += red[ge * WAVES + i][j][q];
-    const int l = q / 4, r = q % 4;
-    const int n = nt0 + (l >> 4) * 4 + r;
-    const int m = l & 15;
-    v *= rstd[m];
-    if (SPLIT && mode == OUT_SPLIT) {
-      if (n < N && m < M) store_split(out, layout, rp.gate, M, m, n, v);
-    } else if (SPLIT || mode == OUT_SWIGLU) {
-      if ((l >> 4) < 2 && n + 8 < N && m < M) {
-        float u = 0.f;
-#pragma unroll
-        for (int i = 0; i < WAVES; ++i) u += red[ge * WAVES + i][j][q + 128];
-        u *= rstd[m];
-        store_gated(out, layout, M, N / 2, m, nt0 / 2 + (l >> 4) * 4 + r, SPLIT ? gated_few(v, u, rp.gate) : silu_mul(v, u));
-      }
-    } else if (post.w != nullptr) {
-      float sq = 0.f;
-      if (n < N && m < M) {
-        float* o = (float*)out + (size_t)m * N + n;
-        const float h = *o + v;
-        *o = h;
-        // (k-blocked on request: the product that consumes these rows then reads them straight from memory as operands)
-        post.xg[(layout & XG_KBLOCKED) ? ((size_t)(n >> 3) * M + m) * 8 + (n & 7) : (size_t)m * N + n] = float_to_bf16(h * post.w[n]);
-        sq = h * h;
-      }
-      sq += __shfl_xor(sq, 1, 64);
-      sq += __shfl_xor(sq, 2, 64);
-      if (r == 0) ss_lds[gj][l >> 4][m] = sq;
-    } else if (mode == OUT_ROPE) {
-      const float other = __shfl_xor(v, 1, 64);
-      if (n < N && m < M) rope_store(rp, m, n, v, other);
-    } else if (n < N && m < M) {
-      store_out(out, mode, (size_t)m * N + n, v);
-    }
-  }
-  if (post.w != nullptr) {
-    __syncthreads();
-    if (tid < 16 * G * NT) {
-      const int gj = tid / 16, m = tid % 16;
-      const int tile = blockIdx.x * G * NT + gj;
-      float sum = 0.f;
-#pragma unroll
-      for (int c = 0; c < 4; ++c) sum += ss_lds[gj][c][m];
-      if (tile * 16 < N) post.ss[tile * 16 + m] = sum;
     }
   }
 }
@@ -691,11 +595,9 @@ extern "C" int tp_splitk_add_rmsnorm(const float* partial, int splits, float* h,
   return 0;
 }
 
-// In the skinny kernel x is the second operand, so the result lane holds weight rows
+// In the few and skinny kernels x is the second operand, so the result lane holds weight rows
 // (l / 16) * 4 + r and activation row l % 16; see the index arithmetic there.
 
-// Tuning knobs of the skinny kernel (0 = choose by shape); set through tp_linear_tune.
-static int g_tune_waves = 0, g_tune_nt = 0, g_tune_depth = 0;   // depth 9 selects the LDS kernel
 static int g_tune_splits = 0, g_tune_mid = 0;                    // mid = 1: 17..64 rows stay on the skinny kernel
 static int g_tune_order = 0;   // large products: 1 tiled kernel, plain block order; 2 tiled, XCD patches; 3 pipelined kernel
 
@@ -728,101 +630,81 @@ extern "C" void tp_linear_tune_mid(int mid, int splits) {
   g_tune_splits = splits;
 }
 
-extern "C" void tp_linear_tune(int waves, int nt, int depth) {
-  g_tune_waves = waves;
-  g_tune_nt = nt;
-  g_tune_depth = depth;
-}
-
 static bool gate_has_constants(const GateAct& g) { return g.extra_slope != 0.f || g.limit > 0.f || g.offset != 0.f; }
 // whether a product of a few rows takes the kernels of the split epilogue (see SPLIT)
 static bool split_epilogue(int mode, const GateAct& g) { return mode == OUT_SPLIT || (mode == OUT_SWIGLU && gate_has_constants(g)); }
 
-template <int MT, int NT, int WAVES, int DEPTH>
-static void launch_skinny4(const bf16_t* x, const bf16_t* w, void* out, int mode, int M, int N, int K, int layout,
-                           RowScale pre, NormPrep post, const RopeOut& rp, hipStream_t s) {
-  const int blocks = (N + 16 * NT - 1) / (16 * NT);
-#define SKINNY(WT_, SPLIT_)                                                                                                              \
-  hipLaunchKernelGGL((gemm_skinny_mfma_kernel<MT, NT, WAVES, DEPTH, WT_, SPLIT_>), dim3(blocks), dim3(WAVES * 64), 0, s, x, w, out, mode, \
-                     M, N, K, layout, pre, post, rp)
-  if (split_epilogue(mode, rp.gate)) {
-    if (layout & W_TILED) SKINNY(true, true);
-    else SKINNY(false, true);
-  } else if (layout & W_TILED) {
-    SKINNY(true, false);
-  } else {
-    SKINNY(false, false);
-  }
-#undef SKINNY
+template <int P, int KIND, bool PRE, bool WT>
+static void launch_few3(const bf16_t* x, const bf16_t* w, void* out, int mode, int M, int N, int K, int layout, const RowScale& pre, const NormPrep& post,
+                        const RopeOut& rp, hipStream_t s) {
+  const size_t rows = P > 0 ? (size_t)M * (K * 2 + 16) : 0;
+  hipLaunchKernelGGL((gemm_few_kernel<P, KIND, PRE, WT>), dim3((N + 15) / 16), dim3(FEW_WAVES * 64), rows, s, x, w, out, M, N, K, mode, layout, FewEnd{pre, post, rp});
+}
+
+template <int KIND, bool PRE>
+static void launch_few2(const bf16_t* x, const bf16_t* w, void* out, int mode, int M, int N, int K, int layout, const RowScale& pre, const NormPrep& post,
+                        const RopeOut& rp, hipStream_t s) {
+#define FEW(P_, WT_) return launch_few3<P_, KIND, PRE, WT_>(x, w, out, mode, M, N, K, layout, pre, post, rp, s)
+  if (!(layout & W_TILED)) FEW(0, false);
+  const int blocks = N / 16, pieces = (M * (K / 8) + FEW_WAVES * 64 - 1) / (FEW_WAVES * 64);
+  const bool blocked = M == 1 || (layout & X_KBLOCKED) != 0;
+  // Row-major rows of several requests go through LDS while they are few enough for two blocks a CU to have theirs (up to 32 KB: four rows
+  // 4,096 x 4,096 7.6 us, straight from memory 8.3), and so does a single row where some CUs have two blocks and others one: those share what a CU can pull, and
+  // the rows' own loads are in their way (3,072 x 5,120 8.3 us from memory, 7.4 through LDS, 4,096 x 6,144 11.0 and 9.9; elsewhere the wait for the
+  // copy is what counts, 4,096 x 4,096 6.9 and 7.0, 14,336 x 4,096 18.9 and 19.3).
+  const bool staged = pieces <= 4 && (M == 1 ? blocks > 256 && blocks <= 512 : !blocked);
+  if (!staged) FEW(0, true);
+  if (pieces <= 1) FEW(1, true);
+  if (pieces <= 2) FEW(2, true);
+  FEW(4, true);
+#undef FEW
+}
+
+template <int KIND>
+static void launch_few1(const bf16_t* x, const bf16_t* w, void* out, int mode, int M, int N, int K, int layout, const RowScale& pre, const NormPrep& post,
+                        const RopeOut& rp, hipStream_t s) {
+  if (pre.ss != nullptr) launch_few2<KIND, true>(x, w, out, mode, M, N, K, layout, pre, post, rp, s);
+  else launch_few2<KIND, false>(x, w, out, mode, M, N, K, layout, pre, post, rp, s);
+}
+
+// at most 16 rows
+static void launch_few(const bf16_t* x, const bf16_t* w, void* out, int mode, int M, int N, int K, int layout, const RowScale& pre, const NormPrep& post,
+                       const RopeOut& rp, hipStream_t s) {
+#define FEW(KIND_) return launch_few1<KIND_>(x, w, out, mode, M, N, K, layout, pre, post, rp, s)
+  if (split_epilogue(mode, rp.gate)) FEW(FEW_SPLIT);
+  if (mode == OUT_SWIGLU) FEW(FEW_SWIGLU);
+  if (mode == OUT_ROPE) FEW(FEW_ROPE);
+  if (post.w != nullptr) FEW(FEW_POST);
+  FEW(FEW_STORE);
+#undef FEW
 }
 
 template <int MT>
-static void launch_skinny(const bf16_t* x, const bf16_t* w, void* out, int mode, int M, int N, int K, int layout,
-                          RowScale pre, NormPrep post, const RopeOut& rp, hipStream_t s) {
-  // every wave should get at least one run of four steps; small N wants many waves per block
-  // (one block per 16 columns is all the parallelism there is), large N fewer and two row tiles
-  // Measured on MI355X at Llama-8B shapes: eight waves with two runs in flight each stream
-  // fastest (5.7-6.3 TB/s with one activation row); wider blocks or two row tiles never won.
+static void launch_skinny(const bf16_t* x, const bf16_t* w, void* out, int mode, int M, int N, int K, int w_tiled, const GateAct& gate, hipStream_t s) {
+  // every wave should get at least one run of four steps
   const int runs = K / 128;
-  int waves = runs >= 8 ? 8 : (runs >= 4 ? 4 : 2);
-  int nt = 1;
-  int depth = (runs >= 2 * waves && MT <= 2) ? 2 : 1;
-  if (g_tune_waves) waves = g_tune_waves;
-  if (g_tune_nt) nt = g_tune_nt;
-  if (g_tune_depth) depth = g_tune_depth;
-  if (post.w != nullptr) nt = 1;   // the consumer counts one partial sum per 16 columns
-  if constexpr (MT == 1) {
-    // several activation rows: feed them through LDS, unless K is so long that the barrier per
-    // chunk costs more than the gather (measured: K = 14336 is faster without)
-    bool lds = M > 1 && K >= 2 * LKC && K <= 8 * LKC && !(layout & X_KBLOCKED);
-    if (g_tune_depth && !(layout & X_KBLOCKED)) lds = g_tune_depth == 9;
-    if (lds) {
-      if (nt > 2) nt = 2;
-      const int blocks = (N + 16 * nt - 1) / (16 * nt);
-      const bool wt = (layout & W_TILED) != 0;
-#define LDS_CASE(NT_, WT_)                                                                                                                     \
-  do {                                                                                                                                         \
-    if (split_epilogue(mode, rp.gate))                                                                                                         \
-      hipLaunchKernelGGL((gemm_skinny_lds_kernel<NT_, 8, WT_, true>), dim3(blocks), dim3(512), 0, s, x, w, out, mode, M, N, K, layout, pre,    \
-                         post, rp);                                                                                                            \
-    else                                                                                                                                       \
-      hipLaunchKernelGGL((gemm_skinny_lds_kernel<NT_, 8, WT_, false>), dim3(blocks), dim3(512), 0, s, x, w, out, mode, M, N, K, layout, pre,   \
-                         post, rp);                                                                                                            \
-  } while (0)
-      if (nt == 2 && wt) LDS_CASE(2, true);
-      else if (nt == 2) LDS_CASE(2, false);
-      else if (wt) LDS_CASE(1, true);
-      else LDS_CASE(1, false);
-#undef LDS_CASE
-      return;
-    }
+  const int waves = runs >= 8 ? 8 : (runs >= 4 ? 4 : 2);
+  const int depth = runs >= 2 * waves && MT <= 2 ? 2 : 1;           // (more tiles: registers)
+  const bool split = split_epilogue(mode, gate);
+#define SKINNY(W_, D_, WT_, SPLIT_) \
+  hipLaunchKernelGGL((gemm_skinny_mfma_kernel<MT, W_, D_, WT_, SPLIT_>), dim3((N + 15) / 16), dim3(W_ * 64), 0, s, x, w, out, mode, M, N, K, gate)
+#define CASE(W_, D_)                                                  \
+  if (waves == W_ && depth == D_) {                                   \
+    if (split && w_tiled) SKINNY(W_, D_, true, true);                 \
+    else if (split) SKINNY(W_, D_, false, true);                      \
+    else if (w_tiled) SKINNY(W_, D_, true, false);                    \
+    else SKINNY(W_, D_, false, false);                                \
+    return;                                                           \
   }
-  if (MT > 2 && waves > 8) waves = 8;       // LDS for the partial tiles
-  if (MT > 1) nt = 1;
-  if (MT > 2 || nt > 2) depth = 1;           // registers
-#define CASE(NT_, W_, D_) \
-  if (nt == NT_ && waves == W_ && depth == D_) return launch_skinny4<MT, NT_, W_, D_>(x, w, out, mode, M, N, K, layout, pre, post, rp, s)
-  CASE(1, 16, 1);
-  CASE(1, 8, 1);
-  CASE(1, 4, 1);
-  CASE(1, 2, 1);
+  CASE(8, 1)
+  CASE(4, 1)
+  CASE(2, 1)
   if constexpr (MT <= 2) {
-    CASE(1, 16, 2);
-    CASE(1, 8, 2);
-    CASE(1, 4, 2);
-  }
-  if constexpr (MT == 1) {
-    CASE(2, 16, 1);
-    CASE(2, 8, 1);
-    CASE(2, 4, 1);
-    CASE(2, 16, 2);
-    CASE(2, 8, 2);
-    CASE(2, 4, 2);
-    CASE(4, 8, 1);
-    CASE(4, 4, 1);
+    CASE(8, 2)
+    CASE(4, 2)
   }
 #undef CASE
-  launch_skinny4<MT, 1, 8, 1>(x, w, out, mode, M, N, K, layout, pre, post, rp, s);
+#undef SKINNY
 }
 
 // The q/k/v projection of at most 16 rows with rotation and cache write in its epilogue (see RopeOut).
@@ -848,8 +730,8 @@ int tp_linear_rope_mfma(const void* x, const void* w, int w_tiled, int M, int N,
     if (head_dim % 64 != 0 || rotary_dim % 8 != 0 || cos_sin == nullptr || pre_ss != nullptr || page_size % 8 != 0) return -1;
     return tp_linear_pipe((const bf16_t*)x, (const bf16_t*)w, w_tiled & 1, nullptr, OUT_ROPE, M, N, K, nullptr, 0, 0, &rp, 0, nullptr, GateAct{}, s);
   }
-  launch_skinny<1>((const bf16_t*)x, (const bf16_t*)w, nullptr, OUT_ROPE, M, N, K, (w_tiled & 1 ? W_TILED : 0) | (w_tiled & 2 ? X_KBLOCKED : 0),
-                   pre, post, rp, s);
+  launch_few((const bf16_t*)x, (const bf16_t*)w, nullptr, OUT_ROPE, M, N, K, (w_tiled & 1 ? W_TILED : 0) | (w_tiled & 2 ? X_KBLOCKED : 0), pre, post, rp,
+             s);
   return 0;
 }
 
@@ -882,13 +764,13 @@ int tp_linear_mfma(const void* x, const void* w, void* out, int out_dt, int accu
   no_rope.gate = gate;      // (the kernels read the gated epilogue's constants from here)
   if (M <= 16 || (M <= 64 && !mid_ok)) {
     if (M <= 16)
-      launch_skinny<1>(xb, wb, out, mode, M, N, K, layout, pre, post, no_rope, s);
+      launch_few(xb, wb, out, mode, M, N, K, layout, pre, post, no_rope, s);
     else if (M <= 32)
-      launch_skinny<2>(xb, wb, out, mode, M, N, K, layout, pre, post, no_rope, s);
+      launch_skinny<2>(xb, wb, out, mode, M, N, K, w_tiled, gate, s);
     else if (M <= 48)
-      launch_skinny<3>(xb, wb, out, mode, M, N, K, layout, pre, post, no_rope, s);
+      launch_skinny<3>(xb, wb, out, mode, M, N, K, w_tiled, gate, s);
     else
-      launch_skinny<4>(xb, wb, out, mode, M, N, K, layout, pre, post, no_rope, s);
+      launch_skinny<4>(xb, wb, out, mode, M, N, K, w_tiled, gate, s);
   } else {
     // large products: 128 x 128 tiles.  Between 17 and 128 rows the weights are still the traffic:
     // 64 x 128 tiles, and K split over blockIdx.z until there are blocks for every CU.

@@ -451,7 +451,7 @@ def interleave_gate_up(gate: torch.Tensor, up: torch.Tensor) -> torch.Tensor:
 
 class Prenormed:
     """Rows whose root-mean-square norm is finished by the product that consumes them: ``x`` is
-    bfloat16(h * norm weight) [m, k]; ``ss`` [ceil(k / 16), 16] float32 holds, per block of 16 columns
+    bfloat16(h * norm weight) [m, k]; ``ss`` [ceil(k / 16), m] float32 (each row's values side by side in memory) holds, per block of 16 columns
     and row, the sum of squares of h; the consumer multiplies its float32 result rows by
     rsqrt(sum(ss) / k + eps).  Made by ``linear(..., residual=h, next_norm=(weight, eps))``."""
     __slots__ = ("x", "ss", "eps", "blocked")
@@ -597,10 +597,10 @@ def _pre_args(x):
     """(the tensor a product reads, the arguments of its row scale, its rows and columns, layout bit 1 when the
     tensor is k-blocked) of plain rows or of ``Prenormed`` rows."""
     if isinstance(x, Prenormed):
-        _dev_ok(x.x, x.ss)
+        _dev_ok(x.x, x.ss.t())
         m, k = x.shape
         _need(x.x.dtype == torch.bfloat16 and x.ss.dtype == torch.float32 and x.x.numel() == m * k and
-              tuple(x.ss.shape) == ((k + 15) // 16, 16), "linear: malformed handed-over rows")
+              tuple(x.ss.shape) == ((k + 15) // 16, m), "linear: malformed handed-over rows")
         return x.x, (_ptr(x.ss), x.ss.shape[0], float(x.eps)), (m, k), (1 if x.blocked is not None else 0)
     return x, (_ptr(None), 0, 0.0), (tuple(x.shape) if x.dim() == 2 else None), 0
 
@@ -773,7 +773,7 @@ def _stream_linear(x, w, close: StreamClose):
     handed = None
     if weight is not None:
         handed = Prenormed(torch.empty((n // 8, m, 8), dtype=torch.bfloat16, device=h.device),
-                           torch.empty((n // 16, 16), dtype=torch.float32, device=h.device), eps, (m, n))
+                           torch.empty((m, n // 16), dtype=torch.float32, device=h.device).t(), eps, (m, n))
     _call("tp_stream_linear", _ptr(data), int(blocked), _ptr(w.data), _ptr(h), s, _ptr(close.mix), _ptr(close.out_coef), _ptr(inc),
           _ptr(weight), _ptr(None if handed is None else handed.x), _ptr(None if handed is None else handed.ss), m, n, k, _stream(), tag=(m, n, k))
     return handed
@@ -859,7 +859,7 @@ def linear(x, w: torch.Tensor, out_dtype: torch.dtype, residual: Optional[torch.
         # activations straight from memory as operands instead of staging them through LDS)
         hand_blocked = handoff_blocked and n % 32 == 0
         handed = Prenormed(torch.empty((n // 8, m, 8) if hand_blocked else (m, n), dtype=torch.bfloat16, device=x.device),
-                           torch.empty(((n + 15) // 16, 16), dtype=torch.float32, device=x.device), eps,
+                           torch.empty((m, (n + 15) // 16), dtype=torch.float32, device=x.device).t(), eps,
                            (m, n) if hand_blocked else None)
         post = (_ptr(weight), _ptr(handed.x), _ptr(handed.ss))
         if hand_blocked:

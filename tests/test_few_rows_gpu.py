@@ -542,3 +542,44 @@ def test_latent_norms_and_store(n, q_dim, c_dim, dtype):
     assert ops.latent_norms_ok(rows, 4, q_dim, 4 + q_dim, c_dim, dtype, dtype) and not ops.latent_norms_ok(rows, 2, q_dim, 4, c_dim, dtype, dtype)
     got = ops.latent_norms(rows, 4, q_dim, qw, 4 + q_dim, c_dim, cw, 1e-5, slots, k1, v1)
     assert torch.equal(got, want) and torch.equal(k0, k1) and torch.equal(v0, v1)
+
+
+@pytest.mark.parametrize("m,k,n", [(1, 64, 16), (1, 192, 4128), (1, 4096, 4128), (1, 4160, 8192), (1, 8256, 4112), (1, 16448, 4128), (2, 4160, 64), (3, 960, 544),
+                                   (4, 4096, 48), (5, 4160, 96), (8, 1024, 8224), (9, 320, 288), (16, 2112, 272), (16, 1088, 8192)])
+@pytest.mark.parametrize("tiled", [True, False])
+def test_products_of_few_rows_at_the_edges_of_their_variants(m, k, n, tiled):
+    """Rows through LDS (one to four pieces a thread, one and several rows) and straight from memory, whole and partial runs of K, waves without
+    a run, more column blocks than CUs; every kind of end.  Bounds: k products of exact bfloat16 factors summed in float32 are within k * 2^-24 of
+    the sum of their magnitudes; a result in bfloat16 within 2^-8 of itself besides; the norm's scale adds 2^-22 (its own sum and root)."""
+    from tempura_amd.kernels import ops
+    g = torch.Generator().manual_seed(m + k + n)
+    x = torch.randn(m, k, generator=g).to(torch.bfloat16)
+    w = (torch.randn(n, k, generator=g) * k ** -0.5).to(torch.bfloat16)
+    ref, mag = x.double() @ w.double().T, x.double().abs() @ w.double().abs().T
+    slack = k * 2.0 ** -24 * mag
+    wd = ops.tile_weight(w.to(DEV)) if tiled else w.to(DEV)
+    assert not tiled or isinstance(wd, ops.TiledWeight)
+    blocked = ops.KBlocked(x.view(m, k // 8, 8).transpose(0, 1).contiguous().to(DEV), m, k)
+    for given in (x.to(DEV), blocked):
+        assert bool(((ops.linear(given, wd, torch.float32).cpu().double() - ref).abs() <= slack).all())
+    low = ops.linear(x.to(DEV), wd, torch.bfloat16).cpu().double()
+    assert bool(((low - ref).abs() <= slack + 2.0 ** -8 * ref.abs() + 1e-30).all())
+    # added into the stream, the next norm prepared, and a product that finishes it
+    h = torch.randn(m, n, generator=g)
+    nw = torch.rand(n, generator=g) + 0.5
+    hd = h.to(DEV)
+    out, pre = ops.linear(x.to(DEV), wd, torch.float32, residual=hd, next_norm=(nw.to(DEV), 1e-6))
+    assert out is hd and bool(((hd.cpu().double() - h.double() - ref).abs() <= slack + 2.0 ** -23 * (h.double() + ref).abs()).all())
+    if pre is None:
+        assert n % 32 != 0
+        return
+    assert torch.equal(pre.rows().cpu(), (hd.cpu() * nw).to(torch.bfloat16))
+    sums = (hd.cpu().double() ** 2).sum(1)
+    assert bool(((pre.ss.cpu().double().sum(0)[:m] - sums).abs() <= n * 2.0 ** -24 * sums).all())
+    w2 = (torch.randn(32, n, generator=g) * n ** -0.5).to(torch.bfloat16)
+    rows = pre.rows().cpu().double()
+    rstd = torch.rsqrt(sums / n + 1e-6)[:, None]
+    want, most = rows @ w2.double().T * rstd, rows.abs() @ w2.double().abs().T * rstd
+    for weight in (ops.tile_weight(w2.to(DEV)), w2.to(DEV)) if n % 64 == 0 else (w2.to(DEV),) if n % 32 == 0 else ():
+        got = ops.linear(pre, weight, torch.float32).cpu().double()
+        assert bool(((got - want).abs() <= (n * 2.0 ** -24 + 2.0 ** -22) * most + n * 2.0 ** -25 * want.abs()).all())

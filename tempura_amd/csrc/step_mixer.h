@@ -52,6 +52,14 @@ __device__ inline float step_lowrank_f(const LowRank& l, float v, float a_log, f
   return expf(-l.rate * s_softplus(-(v + b)));
 }
 
+// what the waves exchange here lies in LDS: __syncthreads would wait for the state on its way as well
+#define STEP_BARRIER()                                  \
+  do {                                                  \
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); \
+    __builtin_amdgcn_s_barrier();                       \
+    asm volatile("" ::: "memory");                      \
+  } while (0)
+
 // t: the token's row, h: the head
 template <int KIND, int KS, typename TO>
 __device__ inline void mixer_step_block(const StepArgs& a, int t, int h) {
@@ -64,39 +72,61 @@ __device__ inline void mixer_step_block(const StepArgs& a, int t, int h) {
   const int tid = threadIdx.x, lane = tid % TP_WAVE;
   const int ks = tid % KS, jl = tid / KS;
   const int dim = a.dim, vdim = a.vdim;
+  constexpr bool LR_GATE = KIND == STEP_DELTA;      // the gate comes from a low-rank product of its own, not as raw columns
   // ---- everything that depends on no other load is requested before anything is waited for: in a decode step nothing of this
-  // is in a cache near the CU, and each trip that starts only behind a barrier would add its whole latency
+  // is in a cache near the CU, and each trip that starts only behind a barrier would add its whole latency.  No load stands behind a condition
+  // (places are clamped, values past the end replaced where they are used): at a join behind one, and at a store into the state in front of
+  // a load from it, all loads on their way are waited for.
+  const int req = a.token_req[t];
   // low-rank products: column tid % 256 (decay, then gate), its sum in eight shares of the rank, half of them a thread
-  const int lr = tid % 256, half = tid / 256, lc = lr % 128;
-  const LowRank& l = lr < 128 ? a.decay : a.gate_lr;
-  const bool have = l.x != nullptr && lc < (lr < 128 ? dim : vdim);
-  const int lcol = h * (lr < 128 ? dim : vdim) + lc;
-  const float* wt = l.wt + lcol;
+  const int lr = tid % 256, lc = lr % 128;
+  const int part_of = __builtin_amdgcn_readfirstlane(tid / 128), half = part_of / 2;
+  const bool to_gate = LR_GATE && (part_of & 1);
+  const LowRank& l = to_gate ? a.gate_lr : a.decay;
+  const int lwidth = to_gate ? vdim : dim, lat = min(lc, lwidth - 1);
+  const bool have = (LR_GATE || lr < 128) && lc < lwidth;
+  const float* wt = l.wt + (size_t)h * lwidth;      // (one for the wave; the lane's column is an offset)
+  // the head's inputs.  Thread c: element c % 128 of q, k, v or (general) the removal rates
+  const int i = tid % 128;
+  const int width = part_of == 2 || (part_of == 3 && KIND != STEP_GENERAL) ? vdim : dim;
+  const size_t col = (size_t)h * width + min(i, width - 1);
+  const float* in = part_of == 0 ? a.q + (size_t)t * a.q_stride : part_of == 1 ? a.k + (size_t)t * a.k_stride
+                    : part_of == 3 && KIND == STEP_GENERAL ? a.a + (size_t)t * a.q_stride : a.v + (size_t)t * a.v_stride;
+  float elem = in[col];
+  const float inner = l.x[(size_t)t * a.x_stride + min(lc, l.rank - 1)];
+  float cw[4];
+  size_t ch = 0;
+  const int channels = 2 * a.heads * dim + a.heads * vdim;
+  if constexpr (KIND == STEP_DELTA) {
+    ch = (size_t)min(part_of, 2) * a.heads * dim + col;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) cw[j] = a.conv_w[(size_t)min(j, a.taps - 1) * channels + ch];
+  }
+  const int slot = a.state_slots[req];
   float lw[2][4][4];       // the first 64 of the rank
 #pragma unroll
   for (int b = 0; b < 2; ++b)
 #pragma unroll
     for (int p = 0; p < 4; ++p)
 #pragma unroll
-      for (int d = 0; d < 4; ++d) {
-        const int i = b * 32 + (half * 4 + p) * 4 + d;
-        lw[b][p][d] = have && i < l.rank ? wt[(size_t)i * l.columns] : 0.f;
-      }
-  float lb = 0.f, la = 0.f;
-  if (have && half == 0 && l.mode >= 2) {
-    lb = l.bias[lcol];
-    if (l.mode == 2) la = l.a_log[lcol / dim];
-  }
-  float* st = a.state + (size_t)a.state_slots[a.token_req[t]] * a.state_stride;
+      for (int d = 0; d < 4; ++d) lw[b][p][d] = (wt + (size_t)min(b * 32 + (half * 4 + p) * 4 + d, l.rank - 1) * l.columns)[lat];
+  const float lb = a.decay.bias[(size_t)h * dim + min(lc, dim - 1)];
+  const float la = KIND == STEP_DELTA ? a.decay.a_log[h] : 0.f;
+  float* st = a.state + (size_t)slot * a.state_stride;
   float* S_mem = st + a.state_off + (size_t)h * a.vdim * a.dim;
+  float* cs = a.taps > 1 ? st + a.conv_off + ch : S_mem;
+  float carried[3];
+  if constexpr (KIND == STEP_DELTA) {
+#pragma unroll
+    for (int j = 0; j < 3; ++j) carried[j] = cs[(size_t)max(0, min(j, a.taps - 2)) * channels];
+  }
   float S[NP][PER];
 #pragma unroll
   for (int p = 0; p < NP; ++p) {
     const int j = p * C + jl;
 #pragma unroll
     for (int e4 = 0; e4 < PER / 4; ++e4) {
-      const int i = ks * PER + e4 * 4;
-      const float4 f = j < a.vdim && i < a.dim ? *(const float4*)(S_mem + (size_t)j * a.dim + i) : make_float4(0.f, 0.f, 0.f, 0.f);
+      const float4 f = *(const float4*)(S_mem + (size_t)min(j, vdim - 1) * dim + min(ks * PER + e4 * 4, dim - 4));
       S[p][e4 * 4] = f.x; S[p][e4 * 4 + 1] = f.y; S[p][e4 * 4 + 2] = f.z; S[p][e4 * 4 + 3] = f.w;
     }
   }
@@ -104,54 +134,55 @@ __device__ inline void mixer_step_block(const StepArgs& a, int t, int h) {
   int group = 1;
   while (group < 64 && group * 4 < vdim) group *= 2;
   const int d4 = lane % group * 4;
-  float4 wv = make_float4(0.f, 0.f, 0.f, 0.f), gv = make_float4(1.f, 1.f, 1.f, 1.f);
-  if (tid < TP_WAVE && d4 < vdim) {
-    wv = *(const float4*)(a.norm_w + (size_t)h * a.norm_stride + d4);
-    if (a.gate != nullptr) gv = *(const float4*)(a.gate + (size_t)t * a.gate_stride + (size_t)h * vdim + d4);
-  }
+  const float4 wv = *(const float4*)(a.norm_w + (size_t)h * a.norm_stride + min(d4, vdim - 4));
+  float4 gv = make_float4(1.f, 1.f, 1.f, 1.f);
+  if constexpr (!LR_GATE) gv = *(const float4*)(a.gate + (size_t)t * a.gate_stride + (size_t)h * vdim + min(d4, vdim - 4));
   const float beta_raw = KIND == STEP_DELTA ? a.beta[(size_t)t * a.x_stride + h] : 0.f;
-  float bonus[PER];
+  float rate_bias[2];
+  if constexpr (KIND == STEP_GENERAL) {
 #pragma unroll
-  for (int e = 0; e < PER; ++e)
-    bonus[e] = KIND == STEP_LINEAR && a.bonus != nullptr && ks * PER + e < dim ? a.bonus[(size_t)h * dim + ks * PER + e] : 0.f;
-  // ---- the head's inputs
-  {
-    // thread c: element c % 128 of q, k, v or (general) the removal rates
-    const int i = tid % 128, part_of = tid / 128;
-    const int width = part_of == 2 ? vdim : dim;
-    const size_t col = (size_t)h * width + i;
-    float x = 0.f;
-    if (i < width) {
-      if (part_of == 0) x = a.q[(size_t)t * a.q_stride + col];
-      else if (part_of == 1) x = a.k[(size_t)t * a.k_stride + col];
-      else if (part_of == 2) x = a.v[(size_t)t * a.v_stride + col];
-      else if (KIND == STEP_GENERAL) x = a.a[(size_t)t * a.q_stride + col];
-      if (KIND == STEP_DELTA && part_of < 3) {
-        const int channels = 2 * a.heads * dim + a.heads * vdim;
-        const size_t ch = (size_t)part_of * a.heads * dim + col;
-        float* cs = st + a.conv_off + ch;
-        float acc = 0.f;
-        for (int j = 0; j < a.taps; ++j) {
-          const float y = j < a.taps - 1 ? cs[(size_t)j * channels] : x;
-          if (j > 0) cs[(size_t)(j - 1) * channels] = y;
-          acc = fmaf(a.conv_w[(size_t)j * channels + ch], y, acc);
-        }
-        x = s_silu(acc);
-      }
-      if (KIND == STEP_LINEAR && part_of == 0) x *= a.q_scale;
-    }
-    if (part_of == 0) qs[i] = x;
-    else if (part_of == 1) kk[i] = x;
-    else if (part_of == 2) vs[i] = x;
-    else as[i] = x;
-    if (tid < 128) {
-      const float y = tid < a.decay.rank ? a.decay.x[(size_t)t * a.x_stride + tid] : 0.f;
-      xa[tid] = a.decay.in_act ? tanhf(y) : y;
-    } else if (tid < 256 && a.gate_lr.x != nullptr) {
-      xg[i] = i < a.gate_lr.rank ? a.gate_lr.x[(size_t)t * a.x_stride + i] : 0.f;
-    }
+    for (int e = 0; e < 2; ++e) rate_bias[e] = a.a_bias[(size_t)h * dim + min(lane + e * TP_WAVE, dim - 1)];
   }
-  __syncthreads();
+  float bonus[PER];
+  if constexpr (KIND == STEP_LINEAR) {
+    const float* from = (a.bonus != nullptr ? a.bonus : a.decay.bias) + (size_t)h * dim;      // (without a bonus: not used)
+#pragma unroll
+    for (int e = 0; e < PER; ++e) bonus[e] = from[min(ks * PER + e, dim - 1)];
+  }
+  // ---- the head's inputs, on their way above
+  {
+    if constexpr (KIND == STEP_DELTA) {
+      if (part_of < 3 && i < width) {
+        float acc = 0.f;
+        if (a.taps <= 4) {
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            if (j >= a.taps) break;
+            const float y = j < 3 && j < a.taps - 1 ? carried[j < 3 ? j : 0] : elem;
+            if (j > 0) cs[(size_t)(j - 1) * channels] = y;
+            acc = fmaf(cw[j], y, acc);
+          }
+        } else {
+          for (int j = 0; j < a.taps; ++j) {
+            const float y = j < a.taps - 1 ? cs[(size_t)j * channels] : elem;
+            if (j > 0) cs[(size_t)(j - 1) * channels] = y;
+            acc = fmaf(a.conv_w[(size_t)j * channels + ch], y, acc);
+          }
+        }
+        elem = s_silu(acc);
+      }
+    }
+    if (KIND == STEP_LINEAR && part_of == 0) elem *= a.q_scale;
+    if (i >= width) elem = 0.f;
+    if (part_of == 0) qs[i] = elem;
+    else if (part_of == 1) kk[i] = elem;
+    else if (part_of == 2) vs[i] = elem;
+    else as[i] = elem;
+    const float y = lc < l.rank ? inner : 0.f;
+    if (tid < 128) xa[lc] = a.decay.in_act ? tanhf(y) : y;
+    else if (LR_GATE && tid < 256) xg[lc] = y;
+  }
+  STEP_BARRIER();
   // ---- low-rank products
   float acc[4] = {0.f, 0.f, 0.f, 0.f};
   if (have) {
@@ -161,13 +192,16 @@ __device__ inline void mixer_step_block(const StepArgs& a, int t, int h) {
 #pragma unroll
       for (int p = 0; p < 4; ++p)
 #pragma unroll
-        for (int d = 0; d < 4; ++d) acc[p] = fmaf(xs[b * 32 + (half * 4 + p) * 4 + d], lw[b][p][d], acc[p]);
+        for (int d = 0; d < 4; ++d) {
+          const int e = b * 32 + (half * 4 + p) * 4 + d;
+          acc[p] = fmaf(xs[e], e < l.rank ? lw[b][p][d] : 0.f, acc[p]);
+        }
     for (int i0 = 64; i0 < l.rank; i0 += 32) {
 #pragma unroll
       for (int p = 0; p < 4; ++p) {
         const int i = i0 + (half * 4 + p) * 4;
 #pragma unroll
-        for (int d = 0; d < 4; ++d) acc[p] = fmaf(xs[i + d], i + d < l.rank ? wt[(size_t)(i + d) * l.columns] : 0.f, acc[p]);
+        for (int d = 0; d < 4; ++d) acc[p] = fmaf(xs[i + d], i + d < l.rank ? wt[(size_t)(i + d) * l.columns + lat] : 0.f, acc[p]);
       }
     }
     if (half == 1)
@@ -200,9 +234,11 @@ __device__ inline void mixer_step_block(const StepArgs& a, int t, int h) {
       sk = wave_sum(sk);
       const float rk = 1.0f / sqrtf(sk + a.unit_eps);
       float d1 = 0.f, d2 = 0.f;
-      for (int i = lane; i < 128; i += TP_WAVE) {
+#pragma unroll
+      for (int e = 0; e < 2; ++e) {
+        const int i = lane + e * TP_WAVE;
         const float u = i < dim ? kk[i] * rk : 0.f;
-        const float au = i < dim ? s_sigmoid(as[i] + a.a_bias[(size_t)h * dim + i]) * u : 0.f;
+        const float au = i < dim ? s_sigmoid(as[i] + rate_bias[e]) * u : 0.f;
         us[i] = u;
         as[i] = au;
         if (i < dim) {
@@ -218,7 +254,7 @@ __device__ inline void mixer_step_block(const StepArgs& a, int t, int h) {
       }
     }
   }
-  __syncthreads();
+  STEP_BARRIER();
   if (half == 0) {
     float v = 0.f;
 #pragma unroll
@@ -233,8 +269,13 @@ __device__ inline void mixer_step_block(const StepArgs& a, int t, int h) {
     if (lr < 128) ws[lc] = v;
     else gs[lc] = v;
   }
-  __syncthreads();
+  STEP_BARRIER();
   // ---- the step
+#pragma unroll
+  for (int p = 0; p < NP; ++p)
+#pragma unroll
+    for (int e = 0; e < PER; ++e)
+      if (p * C + jl >= vdim || ks * PER + e >= dim) S[p][e] = 0.f;
   const float beta = KIND == STEP_DELTA ? s_sigmoid(beta_raw) : 0.f;
   const int o8 = ks * PER;
   float qa[PER], ka[PER], wa[PER], ua[PER], aa[PER];
@@ -247,7 +288,7 @@ __device__ inline void mixer_step_block(const StepArgs& a, int t, int h) {
       ua[e] = us[o8 + e];
       aa[e] = as[o8 + e];
     } else if (KIND == STEP_LINEAR) {
-      ua[e] = bonus[e];
+      ua[e] = o8 + e < dim ? bonus[e] : 0.f;
     }
   }
 #pragma unroll
@@ -309,7 +350,7 @@ __device__ inline void mixer_step_block(const StepArgs& a, int t, int h) {
       if (j < vdim && i < dim) *(float4*)(S_mem + (size_t)j * dim + i) = make_float4(S[p][e4 * 4], S[p][e4 * 4 + 1], S[p][e4 * 4 + 2], S[p][e4 * 4 + 3]);
     }
   }
-  __syncthreads();
+  STEP_BARRIER();
   // ---- norm and gate: four elements a lane, `group` lanes
   if (tid >= TP_WAVE) return;
   const float4 x = d4 < vdim ? *(const float4*)(ys + d4) : make_float4(0.f, 0.f, 0.f, 0.f);
@@ -323,10 +364,10 @@ __device__ inline void mixer_step_block(const StepArgs& a, int t, int h) {
   const float rstd = 1.0f / sqrtf(ss / (float)vdim + a.norm_eps);
   float v[4] = {x.x * rstd * wv.x, x.y * rstd * wv.y, x.z * rstd * wv.z, x.w * rstd * wv.w};
   float4 g = gv;
-  if (a.gate != nullptr) {
+  if constexpr (!LR_GATE) {
     if (a.gate_act == 2) g = make_float4(g.x * s_sigmoid(g.x), g.y * s_sigmoid(g.y), g.z * s_sigmoid(g.z), g.w * s_sigmoid(g.w));
     else g = make_float4(s_sigmoid(g.x), s_sigmoid(g.y), s_sigmoid(g.z), s_sigmoid(g.w));
-  } else if (a.gate_lr.x != nullptr) {
+  } else {
     g = *(const float4*)(gs + d4);
   }
   from_float4((TO*)a.out + (size_t)t * a.out_stride + a.out_col0 + (size_t)h * vdim + d4, v[0] * g.x * a.scale, v[1] * g.y * a.scale,

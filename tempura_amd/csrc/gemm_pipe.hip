@@ -27,6 +27,7 @@
 // Further down: the same pipeline on 256 x 256 block tiles (gemm_pipe_big_kernel; the host mixes both tile
 // sizes so that whole rounds of tiles fill the CUs) and on 64 x 128 tiles for 17..64 rows (gemm_pipe64_kernel).
 #include <algorithm>
+#include <cmath>
 
 #include "common.h"
 
@@ -1186,55 +1187,75 @@ __global__ __launch_bounds__(256, NST == NS ? 2 : 1) void gemm_pipe64_kernel(con
 // fewer than 128 tiles, K has to be split over blocks, and a kernel has to add the partial sums.  Here a block
 // owns 128 x 128 (a wave 64 x 64: sixteen MFMAs per eight fragment reads), three stages of (128 + 128) rows
 // (96 KB).  The row blocks of a column block run side by side (they share its weights in L2); K is split only when
-// even these tiles are too few.  Epilogues as above, the rotating one included (a wave's 64 columns lie in one head).
+// even these tiles are too few.  Bound by the operands' way from L2 and memory into the CU (32 KB a step: 0.37 us on 40 CUs, 0.48 on 240 with
+// weights in L2, 0.51 from memory), not by LDS: with a quarter of K a wave, weights from memory to registers and a ring of LDS a wave, which halves the
+// LDS reads and needs no barrier, 0.43, 0.45 and 0.58 us.  Epilogues as above, the rotating one included (a wave's 64 columns lie in one head).
 namespace {
 
-constexpr int BM128 = 128, BN128 = 128, STAGE128 = (BM128 + BN128) * ROWB, LPW128 = 8;
+constexpr int BM128 = 128, BN128 = 128;
+// NJ: 16-column tiles a wave, four (blocks of 128 columns) or eight (256).
 // five stages of 32 KB: a step of 128 x 128 x 64 is short (512 cycles of MFMA a wave), and a load has to be four
-// steps ahead to have arrived from L2 when its turn comes
-constexpr int NS128 = 5;
-
-struct Frags128 {
-  u32x4_t a[4], b[4];
+// steps ahead to have arrived from L2 when its turn comes; three of 48 KB at 256 columns
+template <int NJ>
+struct Tile128 {
+  static constexpr int COLUMNS = 32 * NJ, STAGE = (BM128 + COLUMNS) * ROWB, STAGES = NJ == 4 ? 5 : 3, LOADS = 4 + NJ;
 };
-__device__ inline void wait_frags128(Frags128& f) {
+
+template <int NJ>
+struct Frags128 {
+  u32x4_t a[4], b[NJ];
+};
+template <int NJ>
+__device__ inline void wait_frags128(Frags128<NJ>& f) {
   asm volatile("s_waitcnt lgkmcnt(0)"
                : "+v"(f.a[0]), "+v"(f.a[1]), "+v"(f.a[2]), "+v"(f.a[3]), "+v"(f.b[0]), "+v"(f.b[1]), "+v"(f.b[2]), "+v"(f.b[3]));
+  if constexpr (NJ == 8) asm volatile("" : "+v"(f.b[4]), "+v"(f.b[5]), "+v"(f.b[6]), "+v"(f.b[7]));
 }
-// read R (0..7) of a half step: the four w fragments, then the four x fragments
-template <int R>
-__device__ inline void read_one128(Frags128& f, unsigned aaddr, unsigned baddr) {
-  if constexpr (R < 4)
+// read R of a half step: the NJ w fragments, then the four x fragments
+template <int R, int NJ>
+__device__ inline void read_one128(Frags128<NJ>& f, unsigned aaddr, unsigned baddr) {
+  if constexpr (R < NJ)
     f.b[R] = lds_read16<R * 16 * ROWB>(baddr);
   else
-    f.a[R - 4] = lds_read16<(R - 4) * 16 * ROWB>(aaddr);
+    f.a[R - NJ] = lds_read16<(R - NJ) * 16 * ROWB>(aaddr);
 }
-// load I (0..7) of this wave: 0..3 are x rows, 4..7 w rows; one load covers 8 rows
-template <int I>
+// load I of this wave: 0..3 are x rows, the NJ others w rows; one load covers 8 rows
+template <int I, int NJ>
 __device__ inline void issue_one128(unsigned char* buf, const unsigned char* xk, const unsigned char* wk,
-                                    const unsigned (&voff)[LPW128], int wave) {
-  const int t = I < 4 ? wave * 4 + I : 16 + wave * 4 + (I - 4);
-  load_lds16(I < 4 ? xk : wk, voff[I], buf + t * 1024);
+                                    const unsigned (&voff)[4 + NJ], int wave) {
+  if constexpr (I < 4 + NJ) {
+    const int t = I < 4 ? wave * 4 + I : 16 + wave * NJ + (I - 4);
+    load_lds16(I < 4 ? xk : wk, voff[I], buf + t * 1024);
+  }
 }
-template <bool READ, bool LOAD>
-__device__ inline void half_step128(f32x4_t (&acc)[4][4], const Frags128& cur, Frags128& nxt, unsigned aaddr, unsigned baddr,
+template <bool READ, bool LOAD, int NJ>
+__device__ inline void half_step128(f32x4_t (&acc)[4][NJ], const Frags128<NJ>& cur, Frags128<NJ>& nxt, unsigned aaddr, unsigned baddr,
                                     unsigned char* buf, const unsigned char* xk, const unsigned char* wk,
-                                    const unsigned (&voff)[LPW128], int wave) {
+                                    const unsigned (&voff)[4 + NJ], int wave) {
 #define SB() __builtin_amdgcn_sched_barrier(0)
 #define RD(R) \
-  if (READ) read_one128<R>(nxt, aaddr, baddr); \
+  if (READ) read_one128<R, NJ>(nxt, aaddr, baddr); \
   SB()
 #define LD(I) \
-  if (LOAD) issue_one128<I>(buf, xk, wk, voff, wave); \
+  if (LOAD) issue_one128<I, NJ>(buf, xk, wk, voff, wave); \
   SB()
 // (assembly with the accumulator as an AGPR operand that is read and written in place: left to the compiler,
 // the sixteen accumulators were moved between register files around every MFMA)
 #define M1(I, J) \
   asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc[I][J]) : "v"(cur.a[I]), "v"(cur.b[J])); \
   SB()
-  RD(0); M1(0, 0); LD(0); RD(1); M1(0, 1); LD(1); RD(2); M1(0, 2); LD(2); RD(3); M1(0, 3); LD(3);
-  RD(4); M1(1, 0); LD(4); RD(5); M1(1, 1); LD(5); RD(6); M1(1, 2); LD(6); RD(7); M1(1, 3); LD(7);
-  M1(2, 0); M1(2, 1); M1(2, 2); M1(2, 3); M1(3, 0); M1(3, 1); M1(3, 2); M1(3, 3);
+  if constexpr (NJ == 4) {
+    RD(0); M1(0, 0); LD(0); RD(1); M1(0, 1); LD(1); RD(2); M1(0, 2); LD(2); RD(3); M1(0, 3); LD(3);
+    RD(4); M1(1, 0); LD(4); RD(5); M1(1, 1); LD(5); RD(6); M1(1, 2); LD(6); RD(7); M1(1, 3); LD(7);
+    M1(2, 0); M1(2, 1); M1(2, 2); M1(2, 3); M1(3, 0); M1(3, 1); M1(3, 2); M1(3, 3);
+  } else {
+    static_assert(NJ == 4 || NJ == 8, "w tiles a wave");
+    RD(0); M1(0, 0); LD(0); RD(1); M1(0, 1); LD(1); RD(2); M1(0, 2); LD(2); RD(3); M1(0, 3); LD(3);
+    RD(4); M1(0, 4); LD(4); RD(5); M1(0, 5); LD(5); RD(6); M1(0, 6); LD(6); RD(7); M1(0, 7); LD(7);
+    RD(8); M1(1, 0); LD(8); RD(9); M1(1, 1); LD(9); RD(10); M1(1, 2); LD(10); RD(11); M1(1, 3); LD(11);
+    M1(1, 4); M1(1, 5); M1(1, 6); M1(1, 7); M1(2, 0); M1(2, 1); M1(2, 2); M1(2, 3); M1(2, 4); M1(2, 5); M1(2, 6); M1(2, 7);
+    M1(3, 0); M1(3, 1); M1(3, 2); M1(3, 3); M1(3, 4); M1(3, 5); M1(3, 6); M1(3, 7);
+  }
 #undef RD
 #undef LD
 #undef M1
@@ -1253,12 +1274,14 @@ struct ExpertRows {
 // GROUPED: one launch for all experts of a routed layer.  The offsets are read here, so the host waits for nothing, and the list of
 // tiles is (expert, column block, row block), row blocks fastest: the blocks that share an expert's weights run side by side on
 // one XCD.  The grid holds the most tiles that any split of the rows can make; the ones too many are the last of each XCD's share.
-template <bool GROUPED>
+template <bool GROUPED, int NJ>
 __global__ __launch_bounds__(256) void gemm_pipe128_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w,
                                                            void* __restrict__ out, float* __restrict__ partial, int mode,
                                                            int M, int N, int K, int ldo, RopeOut rp, int wt, int splits,
                                                            ExpertRows ex) {
-  __shared__ __attribute__((aligned(1024))) unsigned char stages[NS128 * STAGE128];
+  using T = Tile128<NJ>;
+  constexpr int BNT = T::COLUMNS, NST = T::STAGES, LPWT = T::LOADS;
+  __shared__ __attribute__((aligned(1024))) unsigned char stages[NST * T::STAGE];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave >> 1, wn = wave & 1;
   // Blocks go to the 8 XCDs in turn, and each XCD has an L2 of its own: XCD j takes the j-th eighth of the list
@@ -1266,7 +1289,7 @@ __global__ __launch_bounds__(256) void gemm_pipe128_kernel(const bf16_t* __restr
   // blocks of the weights and the rows of x over one part of K, and the weights cross the fabric once.
   int MB, split, tile;
   if constexpr (GROUPED) {
-    const int NB = (N + BN128 - 1) / BN128;
+    const int NB = (N + BNT - 1) / BNT;
     int total = 0;
     for (int e = 0; e < ex.experts; ++e) total += (ex.offsets[e + 1] - ex.offsets[e] + BM128 - 1) / BM128;
     total *= NB;
@@ -1288,7 +1311,7 @@ __global__ __launch_bounds__(256) void gemm_pipe128_kernel(const bf16_t* __restr
     out = (char*)out + (size_t)first * ldo * (mode == OUT_F32 ? 4 : 2);
   } else {
     MB = (M + BM128 - 1) / BM128;
-    const int tiles = MB * ((N + BN128 - 1) / BN128);
+    const int tiles = MB * ((N + BNT - 1) / BNT);
     const int total = tiles * splits;
     const int per_xcd = (total + 7) / 8;
     const int item = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
@@ -1297,12 +1320,12 @@ __global__ __launch_bounds__(256) void gemm_pipe128_kernel(const bf16_t* __restr
     tile = item - split * tiles;
   }
   const int bm = tile % MB, bn = tile / MB;
-  const int m0 = bm * BM128, n0 = bn * BN128;
-  f32x4_t acc[4][4];
+  const int m0 = bm * BM128, n0 = bn * BNT;
+  f32x4_t acc[4][NJ];
 #pragma unroll
   for (int i = 0; i < 4; ++i)
 #pragma unroll
-    for (int j = 0; j < 4; ++j) acc[i][j] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+    for (int j = 0; j < NJ; ++j) acc[i][j] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
   const int kt_per = (K / BK + splits - 1) / splits;
   const int kt_first = split * kt_per;
   const int KT = min(K / BK, kt_first + kt_per) - kt_first;
@@ -1315,16 +1338,16 @@ __global__ __launch_bounds__(256) void gemm_pipe128_kernel(const bf16_t* __restr
   const unsigned lds0 = (unsigned)(size_t)(__attribute__((address_space(3))) const unsigned char*)&stages[0];
   const unsigned off0 = c * ROWB + (((0 * 4 + g) ^ ((c >> 1) & 7)) << 4);
   const unsigned off1 = c * ROWB + (((1 * 4 + g) ^ ((c >> 1) & 7)) << 4);
-  const unsigned arow = wm * 64 * ROWB, brow = (BM128 + wn * 64) * ROWB;
-  unsigned voff[LPW128];
+  const unsigned arow = wm * 64 * ROWB, brow = (BM128 + wn * 16 * NJ) * ROWB;
+  unsigned voff[LPWT];
 #pragma unroll
-  for (int i = 0; i < LPW128; ++i) {
-    const int row = (wave * 4 + (i & 3)) * 8 + (lane >> 3);
+  for (int i = 0; i < LPWT; ++i) {
+    const int row = (i < 4 ? wave * 4 + i : wave * NJ + (i - 4)) * 8 + (lane >> 3);
     const int chunk = (lane & 7) ^ ((row >> 1) & 7);
     const int grow = i < 4 ? min(row, M - 1 - m0) : min(row, N - 1 - n0);
     voff[i] = (unsigned)grow * (unsigned)K * 2u + chunk * 16;
     if (wt && i >= 4) {   // block u of the stage's weights: row group u / 2 of the block tile, first or second 32 of k
-      const int u = wave * 4 + (i - 4);
+      const int u = wave * NJ + (i - 4);
       const int grp = min(u / 2, (N - n0) / 16 - 1);
       voff[i] = ((unsigned)grp * (unsigned)(K / 32) + (u & 1)) * 1024u + lane * 16;
     }
@@ -1334,56 +1357,62 @@ __global__ __launch_bounds__(256) void gemm_pipe128_kernel(const bf16_t* __restr
   const unsigned char* xk = (const unsigned char*)x + ((size_t)m0 * K + (size_t)kt_first * BK) * 2;
   const unsigned char* wk = (const unsigned char*)w + (size_t)n0 * K * 2 + (size_t)kt_first * wkstep;
   auto issue_stage = [&](unsigned char* buf, const unsigned char* xs, const unsigned char* ws) {
-    issue_one128<0>(buf, xs, ws, voff, wave); issue_one128<1>(buf, xs, ws, voff, wave);
-    issue_one128<2>(buf, xs, ws, voff, wave); issue_one128<3>(buf, xs, ws, voff, wave);
-    issue_one128<4>(buf, xs, ws, voff, wave); issue_one128<5>(buf, xs, ws, voff, wave);
-    issue_one128<6>(buf, xs, ws, voff, wave); issue_one128<7>(buf, xs, ws, voff, wave);
+    issue_one128<0, NJ>(buf, xs, ws, voff, wave); issue_one128<1, NJ>(buf, xs, ws, voff, wave);
+    issue_one128<2, NJ>(buf, xs, ws, voff, wave); issue_one128<3, NJ>(buf, xs, ws, voff, wave);
+    issue_one128<4, NJ>(buf, xs, ws, voff, wave); issue_one128<5, NJ>(buf, xs, ws, voff, wave);
+    issue_one128<6, NJ>(buf, xs, ws, voff, wave); issue_one128<7, NJ>(buf, xs, ws, voff, wave);
+    issue_one128<8, NJ>(buf, xs, ws, voff, wave); issue_one128<9, NJ>(buf, xs, ws, voff, wave);
+    issue_one128<10, NJ>(buf, xs, ws, voff, wave); issue_one128<11, NJ>(buf, xs, ws, voff, wave);
   };
 #pragma unroll
-  for (int p = 0; p < NS128; ++p)
-    if (p < KT) issue_stage(stages + p * STAGE128, xk + p * BK * 2, wk + p * wkstep);
-  xk += NS128 * BK * 2;
-  wk += NS128 * wkstep;
-  Frags128 fa, fb;
-  if (KT >= NS128) WAIT_VM((NS128 - 1) * LPW128); else WAIT_VM(0);
+  for (int p = 0; p < NST; ++p)
+    if (p < KT) issue_stage(stages + p * T::STAGE, xk + p * BK * 2, wk + p * wkstep);
+  xk += NST * BK * 2;
+  wk += NST * wkstep;
+  Frags128<NJ> fa, fb;
+  if (KT >= NST) WAIT_VM((NST - 1) * LPWT); else WAIT_VM(0);
   __builtin_amdgcn_s_barrier();
-  auto read_all = [&](Frags128& f, unsigned aaddr, unsigned baddr) {
-    read_one128<0>(f, aaddr, baddr); read_one128<1>(f, aaddr, baddr); read_one128<2>(f, aaddr, baddr);
-    read_one128<3>(f, aaddr, baddr); read_one128<4>(f, aaddr, baddr); read_one128<5>(f, aaddr, baddr);
-    read_one128<6>(f, aaddr, baddr); read_one128<7>(f, aaddr, baddr);
+  auto read_all = [&](Frags128<NJ>& f, unsigned aaddr, unsigned baddr) {
+    read_one128<0, NJ>(f, aaddr, baddr); read_one128<1, NJ>(f, aaddr, baddr); read_one128<2, NJ>(f, aaddr, baddr);
+    read_one128<3, NJ>(f, aaddr, baddr); read_one128<4, NJ>(f, aaddr, baddr); read_one128<5, NJ>(f, aaddr, baddr);
+    read_one128<6, NJ>(f, aaddr, baddr); read_one128<7, NJ>(f, aaddr, baddr);
+    if constexpr (NJ == 8) {
+      read_one128<8, NJ>(f, aaddr, baddr); read_one128<9, NJ>(f, aaddr, baddr);
+      read_one128<10, NJ>(f, aaddr, baddr); read_one128<11, NJ>(f, aaddr, baddr);
+    }
   };
   read_all(fa, lds0 + arow + off0, lds0 + brow + boff0);
-  wait_frags128(fa);
+  wait_frags128<NJ>(fa);
   int st = 0, kt = 0;
-  for (; kt + NS128 < KT; ++kt) {
-    const int sn = st + 1 == NS128 ? 0 : st + 1;
-    const unsigned cur = lds0 + st * STAGE128, nxt = lds0 + sn * STAGE128;
-    half_step128<true, false>(acc, fa, fb, cur + arow + off1, cur + brow + boff1, nullptr, nullptr, nullptr, voff, wave);
-    wait_frags128(fb);
-    WAIT_VM((NS128 - 2) * LPW128);
+  for (; kt + NST < KT; ++kt) {
+    const int sn = st + 1 == NST ? 0 : st + 1;
+    const unsigned cur = lds0 + st * T::STAGE, nxt = lds0 + sn * T::STAGE;
+    half_step128<true, false, NJ>(acc, fa, fb, cur + arow + off1, cur + brow + boff1, nullptr, nullptr, nullptr, voff, wave);
+    wait_frags128<NJ>(fb);
+    WAIT_VM((NST - 2) * LPWT);
     __builtin_amdgcn_s_barrier();
-    half_step128<true, true>(acc, fb, fa, nxt + arow + off0, nxt + brow + boff0, stages + st * STAGE128, xk, wk, voff, wave);
-    wait_frags128(fa);
+    half_step128<true, true, NJ>(acc, fb, fa, nxt + arow + off0, nxt + brow + boff0, stages + st * T::STAGE, xk, wk, voff, wave);
+    wait_frags128<NJ>(fa);
     xk += BK * 2;
     wk += wkstep;
     st = sn;
   }
   for (; kt + 1 < KT; ++kt) {   // nothing left to load
-    const int sn = st + 1 == NS128 ? 0 : st + 1;
-    const unsigned cur = lds0 + st * STAGE128, nxt = lds0 + sn * STAGE128;
-    half_step128<true, false>(acc, fa, fb, cur + arow + off1, cur + brow + boff1, nullptr, nullptr, nullptr, voff, wave);
-    wait_frags128(fb);
+    const int sn = st + 1 == NST ? 0 : st + 1;
+    const unsigned cur = lds0 + st * T::STAGE, nxt = lds0 + sn * T::STAGE;
+    half_step128<true, false, NJ>(acc, fa, fb, cur + arow + off1, cur + brow + boff1, nullptr, nullptr, nullptr, voff, wave);
+    wait_frags128<NJ>(fb);
     WAIT_VM(0);
     __builtin_amdgcn_s_barrier();
-    half_step128<true, false>(acc, fb, fa, nxt + arow + off0, nxt + brow + boff0, nullptr, nullptr, nullptr, voff, wave);
-    wait_frags128(fa);
+    half_step128<true, false, NJ>(acc, fb, fa, nxt + arow + off0, nxt + brow + boff0, nullptr, nullptr, nullptr, voff, wave);
+    wait_frags128<NJ>(fa);
     st = sn;
   }
   {
-    const unsigned cur = lds0 + st * STAGE128;
-    half_step128<true, false>(acc, fa, fb, cur + arow + off1, cur + brow + boff1, nullptr, nullptr, nullptr, voff, wave);
-    wait_frags128(fb);
-    half_step128<false, false>(acc, fb, fa, 0, 0, nullptr, nullptr, nullptr, voff, wave);
+    const unsigned cur = lds0 + st * T::STAGE;
+    half_step128<true, false, NJ>(acc, fa, fb, cur + arow + off1, cur + brow + boff1, nullptr, nullptr, nullptr, voff, wave);
+    wait_frags128<NJ>(fb);
+    half_step128<false, false, NJ>(acc, fb, fa, 0, 0, nullptr, nullptr, nullptr, voff, wave);
   }
   // The MFMAs are assembly, so the compiler does not know that their results take time: wait out the last ones,
   // tied to their accumulators, and pass every other accumulator through an ordered statement after the wait.
@@ -1391,25 +1420,36 @@ __global__ __launch_bounds__(256) void gemm_pipe128_kernel(const bf16_t* __restr
                : "+a"(acc[3][0]), "+a"(acc[3][1]), "+a"(acc[3][2]), "+a"(acc[3][3])
                :
                : "memory");
+  if constexpr (NJ == 8) asm volatile("" : "+a"(acc[3][4]), "+a"(acc[3][5]), "+a"(acc[3][6]), "+a"(acc[3][7]));
 #pragma unroll
-  for (int i = 0; i < 3; ++i) asm volatile("" : "+a"(acc[i][0]), "+a"(acc[i][1]), "+a"(acc[i][2]), "+a"(acc[i][3]));
-  // the result leaves through LDS: 64 x 64 per wave
+  for (int i = 0; i < 3; ++i) {
+    asm volatile("" : "+a"(acc[i][0]), "+a"(acc[i][1]), "+a"(acc[i][2]), "+a"(acc[i][3]));
+    if constexpr (NJ == 8) asm volatile("" : "+a"(acc[i][4]), "+a"(acc[i][5]), "+a"(acc[i][6]), "+a"(acc[i][7]));
+  }
+  // the result leaves through LDS: 64 x 64 per wave at a time
   __syncthreads();
   float* ct = (float*)stages + wave * (64 * CLD);
-  const int mw = m0 + wm * 64, nw = n0 + wn * 64;
-  RopeFetch<64, 64> fetched;
-  if (mode == OUT_ROPE) rope_fetch(fetched, lane, mw, nw, rp, M);
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) ct[(i * 16 + g * 4 + r) * CLD + j * 16 + c] = acc[i][j][r];
-  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-  if (mode == OUT_ROPE)
-    emit_tile_rope<64, 64, CLD>(ct, lane, mw, nw, rp, M, fetched);
-  else
-    emit_tile<64, 64, CLD>(ct, lane, mw, nw, out, mode, M, N, ldo, rp.gate);
+  const int mw = m0 + wm * 64;
+  // (written out for each half, as the accumulators are indexed by constants only)
+#define HALF(H)                                                                                                 \
+  {                                                                                                             \
+    const int nw = n0 + wn * 16 * NJ + (H) * 64;                                                                \
+    RopeFetch<64, 64> fetched;                                                                                  \
+    if (mode == OUT_ROPE) rope_fetch(fetched, lane, mw, nw, rp, M);                                             \
+    _Pragma("unroll") for (int i = 0; i < 4; ++i) _Pragma("unroll") for (int j = 0; j < 4; ++j)                 \
+        _Pragma("unroll") for (int r = 0; r < 4; ++r) ct[(i * 16 + g * 4 + r) * CLD + j * 16 + c] = acc[i][(H) * 4 + j][r]; \
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");                                                          \
+    if (mode == OUT_ROPE)                                                                                       \
+      emit_tile_rope<64, 64, CLD>(ct, lane, mw, nw, rp, M, fetched);                                            \
+    else                                                                                                        \
+      emit_tile<64, 64, CLD>(ct, lane, mw, nw, out, mode, M, N, ldo, rp.gate);                                  \
+  }
+  HALF(0)
+  if constexpr (NJ == 8) {
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    HALF(1)
+  }
+#undef HALF
 }
 
 // Defined in gemm_mfma.hip.
@@ -1484,7 +1524,7 @@ static int tp_linear_pipe128(const bf16_t* x, const bf16_t* w, int w_tiled, void
   const int ldo = mode == OUT_SWIGLU ? N / 2 : N;
   const long per_xcd = (tiles * splits + 7) / 8;
   if (8 * per_xcd > 0x7fffffffL) return -1;
-  hipLaunchKernelGGL(gemm_pipe128_kernel<false>, dim3((unsigned)(8 * per_xcd)), dim3(256), 0, s, x, w, out,
+  hipLaunchKernelGGL((gemm_pipe128_kernel<false, 4>), dim3((unsigned)(8 * per_xcd)), dim3(256), 0, s, x, w, out,
                      splits > 1 ? scratch : nullptr, mode, M, N, K, ldo, rp, w_tiled, splits, ExpertRows{});
   if (splits > 1 && defer && splits_out != nullptr && mode != OUT_SWIGLU && mode != OUT_SPLIT) {
     *splits_out = splits;   // the parts stay unadded for the caller's next kernel
@@ -1495,6 +1535,21 @@ static int tp_linear_pipe128(const bf16_t* x, const bf16_t* w, int w_tiled, void
   }
   return 0;
 }
+
+// Whether the experts' products take blocks of 128 x 256 instead of 128 x 128 (the same bits): a quarter less traffic from L2 into LDS, which is what
+// bounds the smaller ones (32 KB a step of 64 of K and CU, 0.5 to 0.58 us where all CUs run), and half as many starts and ends; but a step takes 1.5 to
+// 1.9 times as long, so they pay where they need clearly fewer rounds of the CUs.  The rows of each expert are not known here: half a block of each is
+// taken as padding.  Eight experts, choice of two, 128 / 256 columns: 7,168 x 4,096 gated 512 / 1,024 / 2,048 rows 134.6 / 133.7, 204 / 194, 335 / 302 us;
+// 4,096 x 3,584 81 / 69, 117 / 119.5 (three rounds against two), 192 / 178; 4,096 x 2,048 gated 48.6 / 40.2, 69.4 / 70.6, 106.6 / 103.5;
+// 1,024 x 1,024 25.4 / 22.6 at 2,048 rows; 3,584 x 4,096 at 200 rows (one round either way) 50 / 72.
+static bool moe_wide(int pairs, int experts, int N) {
+  if (N % 256 != 0) return false;
+  const double row_blocks = (double)pairs / BM128 + 0.5 * std::min(pairs, experts);
+  auto rounds = [&](int columns) { return std::ceil(row_blocks * (N / columns) / 256.0); };
+  return 1.6 * rounds(256) < rounds(128);
+}
+// For tests that mean a certain tile: the columns of a block.
+extern "C" int tp_moe_linear_columns(int pairs, int experts, int N) { return moe_wide(pairs, experts, N) ? 256 : 128; }
 
 // Rows sorted by expert (x [pairs, K], offsets [experts + 1] on the device) times the experts' weights w [experts, N, K] (w_tiled: each
 // in the tiled layout): out [pairs, N] float32 (mode 0), the gated activation [pairs, N / 2] (mode 2, interleaved rows) or max(v, 0)^2
@@ -1510,16 +1565,21 @@ extern "C" int tp_moe_linear(const void* x, const void* w, int w_tiled, void* ou
   TP_REQUIRE(x && w && out && offsets && (((uintptr_t)x | (uintptr_t)w | (uintptr_t)out) & 15) == 0, "moe_linear: missing or misaligned operand");
   TP_REQUIRE((size_t)(BM128 - 1) * K * 2 + 128 < ((size_t)1 << 31), "moe_linear: K too large");
   if (pairs == 0) return 0;
-  const long blocks = ((long)((N + BN128 - 1) / BN128) * (pairs / BM128 + experts) + 7) / 8 * 8;
+  const bool wide = moe_wide(pairs, experts, N);
+  const long blocks = ((long)(wide ? N / 256 : (N + BN128 - 1) / BN128) * (pairs / BM128 + experts) + 7) / 8 * 8;
   TP_REQUIRE(blocks < 0x7fffffffL, "moe_linear: too many tiles");
   RopeOut rp = {};
   if (mode == 3) {
     rp.gate.act_cols = N;
     rp.gate.act_ld = N;
   }
-  hipLaunchKernelGGL(gemm_pipe128_kernel<true>, dim3((unsigned)blocks), dim3(256), 0, s, (const bf16_t*)x, (const bf16_t*)w, out, (float*)nullptr,
-                     mode == 0 ? OUT_F32 : mode == 2 ? OUT_SWIGLU : OUT_SPLIT, 0, N, K, mode == 2 ? N / 2 : N, rp, w_tiled, 1,
-                     ExpertRows{offsets, experts});
+#define MOE_LINEAR(NJ_)                                                                                                                       \
+  hipLaunchKernelGGL((gemm_pipe128_kernel<true, NJ_>), dim3((unsigned)blocks), dim3(256), 0, s, (const bf16_t*)x, (const bf16_t*)w, out,        \
+                     (float*)nullptr, mode == 0 ? OUT_F32 : mode == 2 ? OUT_SWIGLU : OUT_SPLIT, 0, N, K, mode == 2 ? N / 2 : N, rp, w_tiled, 1, \
+                     ExpertRows{offsets, experts})
+  if (wide) MOE_LINEAR(8);
+  else MOE_LINEAR(4);
+#undef MOE_LINEAR
   TP_CHECK_LAUNCH("moe_linear");
   return 0;
 }

@@ -583,3 +583,36 @@ def test_products_of_few_rows_at_the_edges_of_their_variants(m, k, n, tiled):
     for weight in (ops.tile_weight(w2.to(DEV)), w2.to(DEV)) if n % 64 == 0 else (w2.to(DEV),) if n % 32 == 0 else ():
         got = ops.linear(pre, weight, torch.float32).cpu().double()
         assert bool(((got - want).abs() <= (n * 2.0 ** -24 + 2.0 ** -22) * most + n * 2.0 ** -25 * want.abs()).all())
+
+
+@pytest.mark.parametrize("counts,n,k", [([0, 5, 1121, 300, 128, 641], 2048, 64), ([129, 1850, 0, 127], 2048, 128), ([1, 2047, 255, 257, 0, 0], 1792, 320),
+                                        ([4097], 1024, 192)])
+@pytest.mark.parametrize("tiled", [True, False])
+@pytest.mark.parametrize("output", ["float32", "swiglu", "relu2"])
+def test_moe_linear_of_256_columns(counts, n, k, tiled, output):
+    """Blocks of 128 x 256: fewer steps of K than stages and more, experts without rows, tiles that end inside an expert.  Bounds as of
+    ``test_moe_linear``; a product for each expert alone, in blocks of 128 x 128, gives the same bits."""
+    from tempura_amd.kernels import ops
+    g = torch.Generator().manual_seed(sum(counts) + n + k)
+    E, pairs = len(counts), sum(counts)
+    assert ops.library().tp_moe_linear_columns(pairs, E, n) == 256
+    x, w = torch.randn(pairs, k, generator=g).to(torch.bfloat16), (torch.randn(E * n, k, generator=g) * 0.2).to(torch.bfloat16)
+    offsets = torch.tensor([0] + list(torch.tensor(counts).cumsum(0)), dtype=torch.int32)
+    wd = ops.tile_weight(w.to(DEV)) if tiled else w.to(DEV)
+    got = ops.moe_linear(x.to(DEV), wd, offsets.to(DEV), E, output)
+    want = torch.cat([x[offsets[e]: offsets[e + 1]].double() @ w[e * n: (e + 1) * n].double().T for e in range(E)])
+    if output == "float32":
+        _close(got, want, 2e-6)
+    elif output == "relu2":
+        _close(got, want.clamp(min=0.0) ** 2, 8e-3)
+    else:
+        pair = want.view(pairs, -1, 2, 8)
+        gate, up = pair[:, :, 0].reshape(pairs, -1), pair[:, :, 1].reshape(pairs, -1)
+        _close(got, gate * torch.sigmoid(gate) * up, 8e-3)
+    for e in range(E):
+        for a in range(int(offsets[e]), int(offsets[e + 1]), 512):
+            b = min(a + 512, int(offsets[e + 1]))
+            assert ops.library().tp_moe_linear_columns(b - a, 1, n) == 128
+            we = w[e * n: (e + 1) * n].to(DEV).contiguous()
+            one = ops.moe_linear(x[a:b].to(DEV), ops.tile_weight(we) if tiled else we, torch.tensor([0, b - a], dtype=torch.int32, device=DEV), 1, output)
+            assert torch.equal(got[a:b], one)

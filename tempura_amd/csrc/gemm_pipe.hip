@@ -1185,8 +1185,8 @@ __global__ __launch_bounds__(256, NST == NS ? 2 : 1) void gemm_pipe64_kernel(con
 // ---- the same pipeline on 128 x 128 blocks ------------------------------------------------------------
 // For steps of a few hundred rows (a prompt portion of 512) times a narrow weight: 256 x 128 blocks then make
 // fewer than 128 tiles, K has to be split over blocks, and a kernel has to add the partial sums.  Here a block
-// owns 128 x 128 (a wave 64 x 64: sixteen MFMAs per eight fragment reads), three stages of (128 + 128) rows
-// (96 KB).  The row blocks of a column block run side by side (they share its weights in L2); K is split only when
+// owns 128 x 128 (a wave 64 x 64: sixteen MFMAs per eight fragment reads), five stages of (128 + 128) rows
+// (160 KB).  The row blocks of a column block run side by side (they share its weights in L2); K is split only when
 // even these tiles are too few.  Bound by the operands' way from L2 and memory into the CU (32 KB a step: 0.37 us on 40 CUs, 0.48 on 240 with
 // weights in L2, 0.51 from memory), not by LDS: with a quarter of K a wave, weights from memory to registers and a ring of LDS a wave, which halves the
 // LDS reads and needs no barrier, 0.43, 0.45 and 0.58 us.  Epilogues as above, the rotating one included (a wave's 64 columns lie in one head).

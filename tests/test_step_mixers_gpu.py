@@ -77,3 +77,10 @@ def test_linear_step(n, heads, dim, vdim, rank, bonus):
         assert ops.mixer_step_ok(n, 1, heads, dim, vdim, (rank,), s1, 8, fused, 0, gate[1], proj.shape[1])
         ops.linear_step(q, k, v, x, w2, mode, b, 0.06, act, u, 0.3, gate, nw, 1e-6, 1.0, s1, 8, req, slots, heads, dim, vdim, fused, 0)
         assert torch.equal(plain, fused) and torch.equal(s0, s1)
+
+
+@pytest.mark.parametrize("taps", [2, 3, 5, 6])
+@pytest.mark.parametrize("n,heads,dim,vdim,rank", SIZES[:2])
+def test_delta_step_of_other_convolutions(n, heads, dim, vdim, rank, taps):
+    """Fewer taps than are requested in front, and more: the same bits as the separate kernels."""
+    test_delta_step(n, heads, dim, vdim, rank, taps)

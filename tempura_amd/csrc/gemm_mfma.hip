@@ -14,6 +14,10 @@
 // and 8 consecutive k at (l / 16) * 8; the result lane l holds rows (l / 16) * 4 + r,
 // r = 0..3, of column l % 16.
 #include "activations.h"
+#include <cstddef>
+#include <tuple>
+#include <type_traits>
+
 #include "common.h"
 
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
@@ -153,7 +157,15 @@ struct FewEnd {
   NormPrep post;
   RopeOut rp;
 };
-#define FEW_END_AT 48      // x, w, out and five numbers are 44 bytes
+// (the kernel's arguments as they lie in memory: each on its own alignment, in their order.  A parameter of another type or order, here or there,
+// does not compile: see the types that gemm_few_kernel is compared with)
+struct FewArgs {
+  const bf16_t *x, *w;
+  void* out;
+  int M, N, K, mode, layout;
+  FewEnd end;
+};
+#define FEW_END_AT offsetof(FewArgs, end)
 template <typename T>
 using constant_ptr = const __attribute__((address_space(4))) T*;
 __device__ inline constant_ptr<FewEnd> few_end() {
@@ -634,9 +646,18 @@ static bool gate_has_constants(const GateAct& g) { return g.extra_slope != 0.f |
 // whether a product of a few rows takes the kernels of the split epilogue (see SPLIT)
 static bool split_epilogue(int mode, const GateAct& g) { return mode == OUT_SPLIT || (mode == OUT_SWIGLU && gate_has_constants(g)); }
 
+// whether a kernel's parameters are the members of FewArgs (whose offsets few_end() goes by)
+template <typename... T>
+constexpr bool few_args_are(void (*)(T...)) {
+  FewArgs* a = nullptr;
+  return std::is_same_v<std::tuple<T...>, std::tuple<decltype(a->x), decltype(a->w), decltype(a->out), decltype(a->M), decltype(a->N), decltype(a->K),
+                                                     decltype(a->mode), decltype(a->layout), decltype(a->end)>>;
+}
+
 template <int P, int KIND, bool PRE, bool WT>
 static void launch_few3(const bf16_t* x, const bf16_t* w, void* out, int mode, int M, int N, int K, int layout, const RowScale& pre, const NormPrep& post,
                         const RopeOut& rp, hipStream_t s) {
+  static_assert(few_args_are(&gemm_few_kernel<P, KIND, PRE, WT>), "few_end() reads another structure than the kernel is given");
   const size_t rows = P > 0 ? (size_t)M * (K * 2 + 16) : 0;
   hipLaunchKernelGGL((gemm_few_kernel<P, KIND, PRE, WT>), dim3((N + 15) / 16), dim3(FEW_WAVES * 64), rows, s, x, w, out, M, N, K, mode, layout, FewEnd{pre, post, rp});
 }

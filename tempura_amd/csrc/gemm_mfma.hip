@@ -132,6 +132,12 @@ struct RowScale {
   float inv_k, eps;
 };
 
+// v of another lane of the same four, by the order of a DPP quad_perm (0xB1: neighbours swapped, 0x4E: pairs swapped)
+template <int ORDER>
+__device__ inline float quad_swapped(float v) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), ORDER, 0xf, 0xf, false));
+}
+
 // ---- few rows ---------------------------------------------------------------------------
 // What happens to the sums: stored (float32, bfloat16, added into float32), the gated SiLU, added into the stream with the next norm prepared,
 // rotation and cache, the split epilogue (mode OUT_SPLIT, or a gate with constants).  Each is a kernel of its own: what one of them
@@ -251,6 +257,26 @@ __global__ __launch_bounds__(FEW_WAVES * 64) void gemm_few_kernel(const bf16_t* 
     asm volatile("" ::: "memory");
   }
   if (wave < runs) multiply(wave);
+  if constexpr (PRE) {
+    // The order is part of the result: 32 sums of every 32nd partial sum, then these in ascending order.  (The same time as a sum in pairs: one row of the
+    // 3B shape 1,462.1 and 1,461.5 us, eight of the 8B shape 3,262 and 3,269.  What costs is asking for the partial sums in front of the weights, 1,476,
+    // and this work in waves that have no row, 1,489.)
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      if (wave + 8 * i >= M) break;
+      float sum = 0.f, total = 0.f;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const LanePair both = lanes_32(lane + 64 * j < pre.count ? parts[i][j] : 0.f);
+        sum += both.a;
+        sum += both.b;
+      }
+      for (int c = (lane & 31) + 256; c < pre.count; c += 32) sum += pre.ss[(wave + 8 * i) * pre.count + c];
+#pragma unroll
+      for (int c = 0; c < 32; ++c) total += lane_value(sum, c);
+      if (lane == 0) rstd[wave + 8 * i] = rsqrtf(total * pre.inv_k + pre.eps);
+    }
+  }
   for (int run = wave + FEW_WAVES; run < runs; run += FEW_WAVES) {
     request(run);
     __builtin_amdgcn_sched_barrier(0);      // (all of a run's loads in front of its first product)
@@ -264,18 +290,6 @@ __global__ __launch_bounds__(FEW_WAVES * 64) void gemm_few_kernel(const bf16_t* 
     }
   }
   *(f32x4_t*)(&red[wave][g * FEW_RED + (lane & 15) * 4]) = acc;
-  if constexpr (PRE) {
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      if (wave + 8 * i >= M) break;
-      float sum = 0.f;
-#pragma unroll
-      for (int j = 0; j < 4; ++j) sum += lane + 64 * j < pre.count ? parts[i][j] : 0.f;
-      for (int c = lane + 256; c < pre.count; c += 64) sum += pre.ss[(wave + 8 * i) * pre.count + c];
-      sum = wave_sum(sum);
-      if (lane == 0) rstd[wave + 8 * i] = rsqrtf(sum * pre.inv_k + pre.eps);
-    }
-  }
   __syncthreads();
   if (wave >= 4 || wave * 4 >= M) return;
   // the waves' partial tiles in wave order
@@ -300,10 +314,14 @@ __global__ __launch_bounds__(FEW_WAVES * 64) void gemm_few_kernel(const bf16_t* 
       // (k-blocked on request: the product that consumes these rows then reads them straight from memory as operands)
       post.xg[(layout & XG_KBLOCKED) ? ((size_t)(n >> 3) * M + m) * 8 + (n & 7) : (size_t)m * N + n] = float_to_bf16(h * wn);
     }
-    const float sq = row_sum(mine ? h * h : 0.f);
+    // (in this order: pairs, fours, then the fours in ascending order)
+    float sq = mine ? h * h : 0.f;
+    sq += quad_swapped<0xB1>(sq);
+    sq += quad_swapped<0x4E>(sq);
+    sq = ((sq + row_rotated<12>(sq)) + row_rotated<8>(sq)) + row_rotated<4>(sq);
     if ((tid & 15) == 0 && m < M) post.ss[m * gridDim.x + blockIdx.x] = sq;
   } else if constexpr (KIND == FEW_ROPE) {
-    const float other = __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0xB1, 0xf, 0xf, false));   // column n ^ 1
+    const float other = quad_swapped<0xB1>(v);   // column n ^ 1
     if (mine) rope_store(rp, turn, m, n, v, other);
   } else if (mine) {
     store_out(out, mode, (size_t)m * N + n, v);

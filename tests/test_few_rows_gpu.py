@@ -616,3 +616,38 @@ def test_moe_linear_of_256_columns(counts, n, k, tiled, output):
             we = w[e * n: (e + 1) * n].to(DEV).contiguous()
             one = ops.moe_linear(x[a:b].to(DEV), ops.tile_weight(we) if tiled else we, torch.tensor([0, b - a], dtype=torch.int32, device=DEV), 1, output)
             assert torch.equal(got[a:b], one)
+
+
+def _in_order(values, group):
+    """float32 sums of ``group`` neighbours along the last axis, added in ascending order."""
+    v = values.reshape(*values.shape[:-1], -1, group)
+    total = torch.zeros_like(v[..., 0])
+    for i in range(group):
+        total = total + v[..., i]
+    return total
+
+
+@pytest.mark.parametrize("m,k", [(1, 1024), (2, 3072), (8, 4096), (9, 4128), (16, 5120), (1, 16384)])
+def test_handed_over_norms_add_in_a_stated_order(m, k):
+    """The order in which a norm's sums of squares are added is part of the result.  A block's sum: neighbours, fours, then the fours in ascending
+    order; a row's: 32 sums of every 32nd block, then those in ascending order.  The same bits as these additions in float32."""
+    from tempura_amd.kernels import ops
+    g = torch.Generator().manual_seed(m + k)
+    h = torch.randn(m, k, generator=g)
+    nw = torch.rand(k, generator=g) + 0.5
+    x, w = torch.zeros(m, 64, dtype=torch.bfloat16, device=DEV), torch.zeros(k, 64, dtype=torch.bfloat16, device=DEV)
+    hd = h.to(DEV)
+    _, pre = ops.linear(x, ops.tile_weight(w), torch.float32, residual=hd, next_norm=(nw.to(DEV), 1e-5))
+    fours = _in_order(_in_order(h * h, 2), 2)
+    assert torch.equal(hd.cpu(), h) and torch.equal(pre.ss.t().cpu(), _in_order(fours, 4))
+    # the same scale as of sums that are the expected total and zeros
+    ss = torch.rand(m, k // 16, generator=g) ** 8 * 64.0
+    lanes = torch.zeros(m, 32)
+    for at in torch.cat([ss, torch.zeros(m, -ss.shape[1] % 32)], 1).view(m, -1, 32).unbind(1):
+        lanes = lanes + at
+    alone = torch.zeros_like(ss)
+    alone[:, 0] = _in_order(lanes, 32)[:, 0]
+    w2 = torch.randn(64, k, generator=g).to(torch.bfloat16)
+    for weight in (ops.tile_weight(w2.to(DEV)), w2.to(DEV)) if k % 64 == 0 else (w2.to(DEV),):
+        got, want = (ops.linear(ops.Prenormed(pre.x, t.to(DEV).t(), 1e-5, pre.blocked), weight, torch.float32) for t in (ss, alone))
+        assert torch.equal(got, want)

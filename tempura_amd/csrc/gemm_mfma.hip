@@ -180,6 +180,9 @@ __device__ inline constant_ptr<FewEnd> few_end() {
   return (constant_ptr<FewEnd>)(args + FEW_END_AT);
 }
 
+// P < 0: row-major rows through LDS in chunks of 1,024 of K, two of them in LDS, the weights of four and the rows of two on their way.
+#define FEW_CHUNK 1024
+#define FEW_CHUNK_LD (FEW_CHUNK * 2 + 16)
 template <int P, int KIND, bool PRE, bool WT>
 __global__ __launch_bounds__(FEW_WAVES * 64) void gemm_few_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w, void* __restrict__ out, int M,
                                                                   int N, int K, int mode, int layout, FewEnd) {
@@ -201,25 +204,48 @@ __global__ __launch_bounds__(FEW_WAVES * 64) void gemm_few_kernel(const bf16_t* 
   const bool blocked = (layout & X_KBLOCKED) != 0;
   const u32x4_t* xp = (const u32x4_t*)x + (blocked ? g * M + row : row * (K / 8) + g);
   const int xstep = blocked ? 4 * M : 4;
-  u32x4_t a[4], b[4];
-  auto request = [&](int run) __attribute__((always_inline)) {
+  u32x4_t a[P < 0 ? 4 : 1][4], b[P < 0 ? 2 : 1][4];
+  auto request = [&](int d, int run) __attribute__((always_inline)) {
 #pragma unroll
-    for (int u = 0; u < 4; ++u) a[u] = TP_WLOAD(wp + (size_t)(run * 4 + u) * wstep);
+    for (int u = 0; u < 4; ++u) a[d][u] = TP_WLOAD(wp + (size_t)(run * 4 + u) * wstep);
     if constexpr (P == 0) {
 #pragma unroll
-      for (int u = 0; u < 4; ++u) b[u] = xp[(size_t)(run * 4 + u) * xstep];
+      for (int u = 0; u < 4; ++u) b[d][u] = xp[(size_t)(run * 4 + u) * xstep];
     }
   };
   f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
-  auto multiply = [&](int run) __attribute__((always_inline)) {
+  auto multiply = [&](int d, int run) __attribute__((always_inline)) {
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
-      const u32x4_t bv = P == 0 ? b[u] : *(const u32x4_t*)(rows_lds + (size_t)row * ld + (run * 4 + u) * 64 + g * 16);
-      acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_frag(a[u]), as_frag(bv), acc, 0, 0, 0);
+      const u32x4_t bv = P == 0 ? b[d][u] : *(const u32x4_t*)(rows_lds + (size_t)row * ld + (run * 4 + u) * 64 + g * 16);
+      acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_frag(a[d][u]), as_frag(bv), acc, 0, 0, 0);
     }
   };
+  // (P < 0) run `wave` of a chunk, and the chunk's rows: 32 threads a row, four pieces of 16 bytes each.  What lies behind the end of K repeats its last
+  // pieces and is not multiplied.
+  const int chunks = (K + FEW_CHUNK - 1) / FEW_CHUNK, copy_row = tid / 32, copy_at = tid % 32;
+  auto request_weights = [&](int d, int chunk) __attribute__((always_inline)) {
+#pragma unroll
+    for (int u = 0; u < 4; ++u) a[d][u] = TP_WLOAD(wp + (size_t)min(chunk * (FEW_CHUNK / 32) + wave * 4 + u, steps - 1) * wstep);
+  };
+  auto request_rows = [&](int d, int chunk) __attribute__((always_inline)) {
+    if (copy_row >= M) return;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) b[d][i] = ((const u32x4_t*)x)[copy_row * (K / 8) + min(chunk * (FEW_CHUNK / 8) + i * 32 + copy_at, K / 8 - 1)];
+  };
   const int runs = steps / 4;      // (whole ones)
-  if (wave < runs) request(wave);
+  if constexpr (P < 0) {
+    request_rows(0, 0);
+    request_weights(0, 0);
+    if (chunks > 1) {
+      request_rows(1, 1);
+      request_weights(1, 1);
+    }
+    if (chunks > 2) request_weights(2, 2);
+    if (chunks > 3) request_weights(3, 3);
+  } else {
+    if (wave < runs) request(0, wave);
+  }
   const constant_ptr<FewEnd> end = few_end();
   const RowScale pre = {end->pre.ss, end->pre.count, end->pre.inv_k, end->pre.eps};
   const NormPrep post = {end->post.w, end->post.xg, end->post.ss};
@@ -256,7 +282,34 @@ __global__ __launch_bounds__(FEW_WAVES * 64) void gemm_few_kernel(const bf16_t* 
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
   }
-  if (wave < runs) multiply(wave);
+  if constexpr (P < 0) {
+    for (int chunk0 = 0; chunk0 < chunks; chunk0 += 4) {
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        const int chunk = chunk0 + c;
+        if (chunk < chunks) {
+          unsigned char* rows = rows_lds + (c & 1) * 16 * FEW_CHUNK_LD;
+          if (copy_row < M) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) *(u32x4_t*)(rows + copy_row * FEW_CHUNK_LD + (i * 32 + copy_at) * 16) = b[c & 1][i];
+          }
+          asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+          __builtin_amdgcn_s_barrier();
+          asm volatile("" ::: "memory");
+          if (chunk + 2 < chunks) request_rows(c & 1, chunk + 2);
+          const int s0 = chunk * (FEW_CHUNK / 32) + wave * 4;
+#pragma unroll
+          for (int u = 0; u < 4; ++u)
+            if (s0 + u < steps)
+              acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_frag(a[c][u]), as_frag(*(const u32x4_t*)(rows + row * FEW_CHUNK_LD + (wave * 4 + u) * 64 + g * 16)),
+                                                            acc, 0, 0, 0);
+          if (chunk + 4 < chunks) request_weights(c, chunk + 4);
+        }
+      }
+    }
+  } else {
+    if (wave < runs) multiply(0, wave);
+  }
   if constexpr (PRE) {
     // The order is part of the result: 32 sums of every 32nd partial sum, then these in ascending order.  (The same time as a sum in pairs: one row of the
     // 3B shape 1,462.1 and 1,461.5 us, eight of the 8B shape 3,262 and 3,269.  What costs is asking for the partial sums in front of the weights, 1,476,
@@ -277,12 +330,12 @@ __global__ __launch_bounds__(FEW_WAVES * 64) void gemm_few_kernel(const bf16_t* 
       if (lane == 0) rstd[wave + 8 * i] = rsqrtf(total * pre.inv_k + pre.eps);
     }
   }
-  for (int run = wave + FEW_WAVES; run < runs; run += FEW_WAVES) {
-    request(run);
+  for (int run = wave + FEW_WAVES; P >= 0 && run < runs; run += FEW_WAVES) {
+    request(0, run);
     __builtin_amdgcn_sched_barrier(0);      // (all of a run's loads in front of its first product)
-    multiply(run);
+    multiply(0, run);
   }
-  if (wave == runs % FEW_WAVES) {      // what is left of K, fewer than four steps
+  if (P >= 0 && wave == runs % FEW_WAVES) {      // what is left of K, fewer than four steps
     for (int st = runs * 4; st < steps; ++st) {
       const u32x4_t av = TP_WLOAD(wp + (size_t)st * wstep);
       const u32x4_t bv = P == 0 ? xp[(size_t)st * xstep] : *(const u32x4_t*)(rows_lds + (size_t)row * ld + st * 64 + g * 16);
@@ -676,7 +729,7 @@ template <int P, int KIND, bool PRE, bool WT>
 static void launch_few3(const bf16_t* x, const bf16_t* w, void* out, int mode, int M, int N, int K, int layout, const RowScale& pre, const NormPrep& post,
                         const RopeOut& rp, hipStream_t s) {
   static_assert(few_args_are(&gemm_few_kernel<P, KIND, PRE, WT>), "few_end() reads another structure than the kernel is given");
-  const size_t rows = P > 0 ? (size_t)M * (K * 2 + 16) : 0;
+  const size_t rows = P < 0 ? 2 * 16 * FEW_CHUNK_LD : P > 0 ? M * (K * 2 + 16) : 0;
   hipLaunchKernelGGL((gemm_few_kernel<P, KIND, PRE, WT>), dim3((N + 15) / 16), dim3(FEW_WAVES * 64), rows, s, x, w, out, M, N, K, mode, layout, FewEnd{pre, post, rp});
 }
 
@@ -684,14 +737,25 @@ template <int KIND, bool PRE>
 static void launch_few2(const bf16_t* x, const bf16_t* w, void* out, int mode, int M, int N, int K, int layout, const RowScale& pre, const NormPrep& post,
                         const RopeOut& rp, hipStream_t s) {
 #define FEW(P_, WT_) return launch_few3<P_, KIND, PRE, WT_>(x, w, out, mode, M, N, K, layout, pre, post, rp, s)
-  if (!(layout & W_TILED)) FEW(0, false);
-  const int blocks = N / 16, pieces = (M * (K / 8) + FEW_WAVES * 64 - 1) / (FEW_WAVES * 64);
-  const bool blocked = M == 1 || (layout & X_KBLOCKED) != 0;
-  // Row-major rows of several requests go through LDS while they are few enough for two blocks a CU to have theirs (up to 32 KB: four rows
-  // 4,096 x 4,096 7.6 us, straight from memory 8.3), and so does a single row where some CUs have two blocks and others one: those share what a CU can pull, and
+  const bool tiled = (layout & W_TILED) != 0, major = M > 1 && (layout & X_KBLOCKED) == 0;
+  const int blocks = (N + 15) / 16, pieces = (M * (K / 8) + FEW_WAVES * 64 - 1) / (FEW_WAVES * 64);
+  // Row-major rows of wide products go through LDS in chunks: read from memory as operands, 64-byte pieces of up to sixteen rows, their way into the CU is as
+  // long as the weights' where there are many column blocks.  From memory (to 32 KB through LDS) / in chunks, tiled weight, 128,256 columns, K 3,072: two rows
+  // 117.0 / 115.4 us, eight 124.0 / 120.8, sixteen 156.4 / 138.7; K 4,096: ten 171.3 / 177.3, twelve 183.9 / 180.4, sixteen 201.9 / 183.1; 16,384 columns, K 3,072: 14 rows 19.7 / 19.8,
+  // sixteen 20.9 / 20.3; 28,672, K 4,096: 14 rows 42.5 / 43.6, sixteen 45.4 / 44.0; 8,192 columns, K 2,048, sixteen rows 8.4 / 8.6.  A row-major weight takes that
+  // way twice over: 4,096 x 128,256 eight rows 227 / 206, sixteen 270 / 230; 4,096 x 6,144 16.1 / 15.5 and 18.6 / 17.0; 2,048 x 8,192 9.6 / 9.5 and 10.9 / 10.5;
+  // 8,192 x 4,096 six rows 18.2 / 19.2, eight 19.3 / 19.4, sixteen 21.4 / 20.7.  (Chunks are of use from two on, and to 8,192: 14,336 x 4,096 eight rows
+  // 21.6 / 26.0.)
+  if (major && K >= 2 * FEW_CHUNK && K <= 8 * FEW_CHUNK) {
+    if (tiled && blocks >= 1024 && (M > 14 || (blocks >= 4096 && (M >= 12 || K <= 3 * FEW_CHUNK)))) FEW(-1, true);
+    if (!tiled && (K <= 4 * FEW_CHUNK || M >= 8)) FEW(-1, false);
+  }
+  if (!tiled) FEW(0, false);
+  // Row-major rows of several requests go through LDS whole while they are few enough (up to 32 KB: four rows 4,096 x 4,096 7.6 us, straight from memory
+  // 8.3), and so does a single row where some CUs have two blocks and others one: those share what a CU can pull, and
   // the rows' own loads are in their way (3,072 x 5,120 8.3 us from memory, 7.4 through LDS, 4,096 x 6,144 11.0 and 9.9; elsewhere the wait for the
   // copy is what counts, 4,096 x 4,096 6.9 and 7.0, 14,336 x 4,096 18.9 and 19.3).
-  const bool staged = pieces <= 4 && (M == 1 ? blocks > 256 && blocks <= 512 : !blocked);
+  const bool staged = pieces <= 4 && (M == 1 ? blocks > 256 && blocks <= 512 : major);
   if (!staged) FEW(0, true);
   if (pieces <= 1) FEW(1, true);
   if (pieces <= 2) FEW(2, true);

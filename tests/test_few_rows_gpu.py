@@ -651,3 +651,53 @@ def test_handed_over_norms_add_in_a_stated_order(m, k):
     for weight in (ops.tile_weight(w2.to(DEV)), w2.to(DEV)) if k % 64 == 0 else (w2.to(DEV),):
         got, want = (ops.linear(ops.Prenormed(pre.x, t.to(DEV).t(), 1e-5, pre.blocked), weight, torch.float32) for t in (ss, alone))
         assert torch.equal(got, want)
+
+
+def _every_end(ops, plain, normed, w, g):
+    """What a product of these rows (plain ones, and ones whose norm it finishes) gives at every kind of end."""
+    m, n = plain.shape[0], w.shape[0]
+    slots = torch.randperm(32, generator=g)[:m].to(torch.int32).to(DEV)
+    positions = torch.randint(0, 4000, (m,), generator=g).to(torch.int32).to(DEV)
+    freq = (10000.0 ** (-torch.arange(0, 16, 2, dtype=torch.float64) / 16)).to(DEV)
+    h, nw = torch.randn(m, n, generator=g).to(DEV), (torch.rand(n, generator=g) + 0.5).to(DEV)
+    out = []
+    for x in (plain, normed):
+        out += [ops.linear(x, w, torch.float32), ops.linear(x, w, torch.bfloat16)]
+        stream = h.clone()
+        _, handed = ops.linear(x, w, torch.float32, residual=stream, next_norm=(nw, 1e-6))
+        out += [stream] + ([] if handed is None else [handed.x, handed.ss])
+    out += [ops.linear_swiglu(normed, w), ops.linear_swiglu(normed, w, slope=1.5, limit=4.0, up_offset=1.0)]
+    if n > 128 and w.shape[1] % 64 == 0:
+        out += ops.linear_relu2(plain, w, 128)
+    for table in (None, ops.rope_table(positions, freq, 16, 1.0)):
+        k_cache, v_cache = (torch.zeros(2, 1, *s, dtype=torch.bfloat16, device=DEV) for s in ((16, 16), (16, 16)))
+        out += [ops.linear_rope_kv(normed, w, positions, slots, freq, 16, 1.0, n // 16 - 2, 1, 16, k_cache, v_cache, table), k_cache, v_cache]
+    return out
+
+
+@pytest.mark.parametrize("m,k,n,tiled", [(2, 2048, 65536, True), (16, 4160, 16384, True), (15, 8192, 16400, True), (14, 8192, 16400, True), (12, 4096, 65536, True), (11, 4096, 65536, True),
+                                         (2, 2048, 48, False), (16, 3104, 64, False), (9, 4128, 160, False), (8, 8192, 48, False), (7, 8192, 48, False), (16, 8224, 48, False)])
+def test_row_major_rows_of_wide_products(m, k, n, tiled):
+    """Rows through LDS in chunks of K, whole and partial ones, and sizes beside theirs: the bits of k-blocked rows at every end."""
+    from tempura_amd.kernels import ops
+    g = torch.Generator().manual_seed(m + k + n)
+    x, ss = torch.randn(m, k, generator=g).to(torch.bfloat16).to(DEV), torch.rand(m, k // 16, generator=g).to(DEV).t()
+    w = (torch.randn(n, k, generator=g) * k ** -0.5).to(torch.bfloat16).to(DEV)
+    w = ops.tile_weight(w) if tiled else w
+    assert isinstance(w, ops.TiledWeight) == tiled
+    xb = x.view(m, k // 8, 8).transpose(0, 1).contiguous()
+    got = _every_end(ops, x, ops.Prenormed(x, ss, 1e-6), w, torch.Generator().manual_seed(n))
+    want = _every_end(ops, ops.KBlocked(xb, m, k), ops.Prenormed(xb, ss, 1e-6, (m, k)), w, torch.Generator().manual_seed(n))
+    assert len(got) == len(want) and all(torch.equal(a, b) for a, b in zip(got, want))
+
+
+@pytest.mark.parametrize("k,n", [(1024, 4112), (4096, 5120), (4160, 8192), (8256, 4128), (16384, 4112)])
+def test_one_row_through_lds(k, n):
+    """One row of more column blocks than CUs with a tiled weight, one to four pieces a thread, up to 1,024 sums of a norm: the bits of the row-major
+    weight, whose product reads the row from memory, at every end."""
+    from tempura_amd.kernels import ops
+    g = torch.Generator().manual_seed(k + n)
+    x, ss = torch.randn(1, k, generator=g).to(torch.bfloat16).to(DEV), torch.rand(1, k // 16, generator=g).to(DEV).t()
+    w = (torch.randn(n, k, generator=g) * k ** -0.5).to(torch.bfloat16).to(DEV)
+    got, want = (_every_end(ops, x, ops.Prenormed(x, ss, 1e-6), weight, torch.Generator().manual_seed(n)) for weight in (ops.tile_weight(w), w))
+    assert len(got) == len(want) and all(torch.equal(a, b) for a, b in zip(got, want))

@@ -180,10 +180,11 @@ __device__ inline constant_ptr<FewEnd> few_end() {
   return (constant_ptr<FewEnd>)(args + FEW_END_AT);
 }
 
-// P < 0: row-major rows through LDS in chunks of 1,024 of K, two of them in LDS, the weights of four and the rows of two on their way.
+// P < 0: row-major rows through LDS in chunks of 1,024 of K, two of them in LDS, the weights of four and the rows of two on their way.  DEEP: two runs on
+// their way (K of at least 16 runs).
 #define FEW_CHUNK 1024
 #define FEW_CHUNK_LD (FEW_CHUNK * 2 + 16)
-template <int P, int KIND, bool PRE, bool WT>
+template <int P, int KIND, bool PRE, bool WT, bool DEEP>
 __global__ __launch_bounds__(FEW_WAVES * 64) void gemm_few_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w, void* __restrict__ out, int M,
                                                                   int N, int K, int mode, int layout, FewEnd) {
   constexpr int T = FEW_WAVES * 64;
@@ -204,7 +205,7 @@ __global__ __launch_bounds__(FEW_WAVES * 64) void gemm_few_kernel(const bf16_t* 
   const bool blocked = (layout & X_KBLOCKED) != 0;
   const u32x4_t* xp = (const u32x4_t*)x + (blocked ? g * M + row : row * (K / 8) + g);
   const int xstep = blocked ? 4 * M : 4;
-  u32x4_t a[P < 0 ? 4 : 1][4], b[P < 0 ? 2 : 1][4];
+  u32x4_t a[P < 0 ? 4 : DEEP ? 2 : 1][4], b[P < 0 || DEEP ? 2 : 1][4];
   auto request = [&](int d, int run) __attribute__((always_inline)) {
 #pragma unroll
     for (int u = 0; u < 4; ++u) a[d][u] = TP_WLOAD(wp + (size_t)(run * 4 + u) * wstep);
@@ -243,6 +244,9 @@ __global__ __launch_bounds__(FEW_WAVES * 64) void gemm_few_kernel(const bf16_t* 
     }
     if (chunks > 2) request_weights(2, 2);
     if (chunks > 3) request_weights(3, 3);
+  } else if constexpr (DEEP) {
+    request(0, wave);
+    request(1, wave + FEW_WAVES);
   } else {
     if (wave < runs) request(0, wave);
   }
@@ -307,6 +311,9 @@ __global__ __launch_bounds__(FEW_WAVES * 64) void gemm_few_kernel(const bf16_t* 
         }
       }
     }
+  } else if constexpr (DEEP) {
+    multiply(0, wave);
+    multiply(1, wave + FEW_WAVES);
   } else {
     if (wave < runs) multiply(0, wave);
   }
@@ -330,7 +337,17 @@ __global__ __launch_bounds__(FEW_WAVES * 64) void gemm_few_kernel(const bf16_t* 
       if (lane == 0) rstd[wave + 8 * i] = rsqrtf(total * pre.inv_k + pre.eps);
     }
   }
-  for (int run = wave + FEW_WAVES; P >= 0 && run < runs; run += FEW_WAVES) {
+  int run = wave + (DEEP ? 2 : 1) * FEW_WAVES;
+  if constexpr (DEEP) {
+    for (; run + FEW_WAVES < runs; run += 2 * FEW_WAVES) {
+      request(0, run);
+      request(1, run + FEW_WAVES);
+      __builtin_amdgcn_sched_barrier(0);
+      multiply(0, run);
+      multiply(1, run + FEW_WAVES);
+    }
+  }
+  for (; P >= 0 && run < runs; run += FEW_WAVES) {
     request(0, run);
     __builtin_amdgcn_sched_barrier(0);      // (all of a run's loads in front of its first product)
     multiply(0, run);
@@ -725,18 +742,20 @@ constexpr bool few_args_are(void (*)(T...)) {
                                                      decltype(a->mode), decltype(a->layout), decltype(a->end)>>;
 }
 
-template <int P, int KIND, bool PRE, bool WT>
+template <int P, int KIND, bool PRE, bool WT, bool DEEP = false>
 static void launch_few3(const bf16_t* x, const bf16_t* w, void* out, int mode, int M, int N, int K, int layout, const RowScale& pre, const NormPrep& post,
                         const RopeOut& rp, hipStream_t s) {
-  static_assert(few_args_are(&gemm_few_kernel<P, KIND, PRE, WT>), "few_end() reads another structure than the kernel is given");
-  const size_t rows = P < 0 ? 2 * 16 * FEW_CHUNK_LD : P > 0 ? M * (K * 2 + 16) : 0;
-  hipLaunchKernelGGL((gemm_few_kernel<P, KIND, PRE, WT>), dim3((N + 15) / 16), dim3(FEW_WAVES * 64), rows, s, x, w, out, M, N, K, mode, layout, FewEnd{pre, post, rp});
+  static_assert(few_args_are(&gemm_few_kernel<P, KIND, PRE, WT, DEEP>), "few_end() reads another structure than the kernel is given");
+  // (DEEP: two blocks a CU, by their LDS; with more of them, 32,000 columns of one row, K 4,096 41.9 -> 42.1 us, K 8,192 78.6 -> 78.8)
+  const size_t rows = P < 0 ? 2 * 16 * FEW_CHUNK_LD : P > 0 ? std::max((size_t)M * (K * 2 + 16), (size_t)(DEEP ? 56 << 10 : 0)) : 0;
+  hipLaunchKernelGGL((gemm_few_kernel<P, KIND, PRE, WT, DEEP>), dim3((N + 15) / 16), dim3(FEW_WAVES * 64), rows, s, x, w, out, M, N, K, mode, layout, FewEnd{pre, post, rp});
 }
 
 template <int KIND, bool PRE>
 static void launch_few2(const bf16_t* x, const bf16_t* w, void* out, int mode, int M, int N, int K, int layout, const RowScale& pre, const NormPrep& post,
                         const RopeOut& rp, hipStream_t s) {
 #define FEW(P_, WT_) return launch_few3<P_, KIND, PRE, WT_>(x, w, out, mode, M, N, K, layout, pre, post, rp, s)
+#define FEW_DEEP(P_) return launch_few3<P_, KIND, PRE, true, true>(x, w, out, mode, M, N, K, layout, pre, post, rp, s)
   const bool tiled = (layout & W_TILED) != 0, major = M > 1 && (layout & X_KBLOCKED) == 0;
   const int blocks = (N + 15) / 16, pieces = (M * (K / 8) + FEW_WAVES * 64 - 1) / (FEW_WAVES * 64);
   // Row-major rows of wide products go through LDS in chunks: read from memory as operands, 64-byte pieces of up to sixteen rows, their way into the CU is as
@@ -752,15 +771,27 @@ static void launch_few2(const bf16_t* x, const bf16_t* w, void* out, int mode, i
   }
   if (!tiled) FEW(0, false);
   // Row-major rows of several requests go through LDS whole while they are few enough (up to 32 KB: four rows 4,096 x 4,096 7.6 us, straight from memory
-  // 8.3), and so does a single row where some CUs have two blocks and others one: those share what a CU can pull, and
-  // the rows' own loads are in their way (3,072 x 5,120 8.3 us from memory, 7.4 through LDS, 4,096 x 6,144 11.0 and 9.9; elsewhere the wait for the
-  // copy is what counts, 4,096 x 4,096 6.9 and 7.0, 14,336 x 4,096 18.9 and 19.3).
-  const bool staged = pieces <= 4 && (M == 1 ? blocks > 256 && blocks <= 512 : major);
-  if (!staged) FEW(0, true);
+  // 8.3), and so does a single row of more blocks than there are CUs, up to 64 KB: blocks that follow or share a CU are bound by what it can pull, and the
+  // row's own loads, four as wide as the weights' a run, are in their way; with up to one block a CU the wait for the copy is what counts.  From memory / through
+  // LDS: K 4,096, 256 blocks 7.4 / 7.6 us, 257 9.7 / 8.6, 384 11.8 / 10.4, 512 13.0 / 12.5; K 2,048 4.7 / 5.0, 5.6 / 5.1, 6.6 / 6.1 and 7.5 / 7.1; K 8,192
+  // 12.6 / 12.9, 17.8 / 16.0, 21.6 / 18.9 and 24.0 / 23.0.
+  if (M > 1 ? !major || pieces > 4 : blocks <= 256 || pieces > 8) FEW(0, true);
+  // From three blocks a CU on, or with more than 32 KB, a row of 4,096 and more also has two runs on their way and no more than two blocks a CU (56 KB of LDS).
+  // One run from memory / two through LDS: K 4,096, 576 blocks 15.4 / 14.6 us, 1,024 22.7 / 22.5, 8,016 153.0 / 153.5; K 8,192, 768 blocks 33.8 / 33.0, 1,792 72.5 / 71.1,
+  // 8,016 300.8 / 302.9; K 14,336, 576 48.6 / 45.7, 1,792 123.9 / 120.7, 4,000 270.7 / 263.9; K 28,672, 512 75.9 / 72.1; but K 2,048, 1,280 blocks 14.7 / 15.3, and K 3,072,
+  // 384 blocks, one and two through LDS 8.0 / 8.3.
+  if (M == 1 && (blocks > 512 || pieces > 4)) {
+    if (K < 4 * FEW_CHUNK || (K <= 8 * FEW_CHUNK && blocks > 2048)) FEW(0, true);
+    if (pieces <= 1) FEW_DEEP(1);
+    if (pieces <= 2) FEW_DEEP(2);
+    if (pieces <= 4) FEW_DEEP(4);
+    FEW_DEEP(8);
+  }
   if (pieces <= 1) FEW(1, true);
   if (pieces <= 2) FEW(2, true);
   FEW(4, true);
 #undef FEW
+#undef FEW_DEEP
 }
 
 template <int KIND>

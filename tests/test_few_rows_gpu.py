@@ -691,9 +691,11 @@ def test_row_major_rows_of_wide_products(m, k, n, tiled):
     assert len(got) == len(want) and all(torch.equal(a, b) for a, b in zip(got, want))
 
 
-@pytest.mark.parametrize("k,n", [(1024, 4112), (4096, 5120), (4160, 8192), (8256, 4128), (16384, 4112)])
+@pytest.mark.parametrize("k,n", [(1024, 4112), (4096, 5120), (4160, 8192), (8256, 4128), (16384, 4112), (4032, 8208), (4096, 8208), (4160, 32784), (5184, 8208),
+                                 (9280, 8208), (16448, 4112), (32768, 4112), (32832, 4112)])
 def test_one_row_through_lds(k, n):
-    """One row of more column blocks than CUs with a tiled weight, one to four pieces a thread, up to 1,024 sums of a norm: the bits of the row-major
+    """One row of more column blocks than CUs with a tiled weight, one to eight pieces a thread, one run of K on its way and two, up to
+    2,052 sums of a norm: the bits of the row-major
     weight, whose product reads the row from memory, at every end."""
     from tempura_amd.kernels import ops
     g = torch.Generator().manual_seed(k + n)

@@ -1548,8 +1548,11 @@ static bool moe_wide(int pairs, int experts, int N) {
   auto rounds = [&](int columns) { return std::ceil(row_blocks * (N / columns) / 256.0); };
   return 1.6 * rounds(256) < rounds(128);
 }
+// (the loads of a block's weights go by 32-bit offsets into 2 GiB: see load_lds16)
+static bool moe_wide_fits(int K) { return (size_t)(Tile128<8>::COLUMNS - 1) * K * 2 + 128 < ((size_t)1 << 31); }
 // For tests that mean a certain tile: the columns of a block.
-extern "C" int tp_moe_linear_columns(int pairs, int experts, int N) { return moe_wide(pairs, experts, N) ? 256 : 128; }
+extern "C" int tp_moe_tile_columns(int pairs, int experts, int N, int K) { return moe_wide_fits(K) && moe_wide(pairs, experts, N) ? 256 : 128; }
+extern "C" int tp_moe_linear_columns(int pairs, int experts, int N) { return tp_moe_tile_columns(pairs, experts, N, BK); }
 
 // Rows sorted by expert (x [pairs, K], offsets [experts + 1] on the device) times the experts' weights w [experts, N, K] (w_tiled: each
 // in the tiled layout): out [pairs, N] float32 (mode 0), the gated activation [pairs, N / 2] (mode 2, interleaved rows) or max(v, 0)^2
@@ -1565,7 +1568,7 @@ extern "C" int tp_moe_linear(const void* x, const void* w, int w_tiled, void* ou
   TP_REQUIRE(x && w && out && offsets && (((uintptr_t)x | (uintptr_t)w | (uintptr_t)out) & 15) == 0, "moe_linear: missing or misaligned operand");
   TP_REQUIRE((size_t)(BM128 - 1) * K * 2 + 128 < ((size_t)1 << 31), "moe_linear: K too large");
   if (pairs == 0) return 0;
-  const bool wide = moe_wide(pairs, experts, N);
+  const bool wide = moe_wide_fits(K) && moe_wide(pairs, experts, N);
   const long blocks = ((long)(wide ? N / 256 : (N + BN128 - 1) / BN128) * (pairs / BM128 + experts) + 7) / 8 * 8;
   TP_REQUIRE(blocks < 0x7fffffffL, "moe_linear: too many tiles");
   RopeOut rp = {};

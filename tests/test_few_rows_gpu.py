@@ -703,3 +703,11 @@ def test_one_row_through_lds(k, n):
     w = (torch.randn(n, k, generator=g) * k ** -0.5).to(torch.bfloat16).to(DEV)
     got, want = (_every_end(ops, x, ops.Prenormed(x, ss, 1e-6), weight, torch.Generator().manual_seed(n)) for weight in (ops.tile_weight(w), w))
     assert len(got) == len(want) and all(torch.equal(a, b) for a, b in zip(got, want))
+
+
+def test_moe_linear_of_256_columns_keeps_within_its_offsets():
+    """A block of 256 columns reaches 255 rows of its weight by offsets into 2 GiB: longer rows, which blocks of 128 columns take, are left to those."""
+    from tempura_amd.kernels import ops
+    longest = (2 ** 31 - 129) // 510 // 64 * 64
+    columns = lambda k: ops.library().tp_moe_tile_columns(2195, 6, 2048, k)
+    assert columns(64) == columns(longest) == 256 and columns(longest + 64) == columns((2 ** 31 - 129) // 254 // 64 * 64) == 128

@@ -27,7 +27,6 @@
 // Further down: the same pipeline on 256 x 256 block tiles (gemm_pipe_big_kernel; the host mixes both tile
 // sizes so that whole rounds of tiles fill the CUs) and on 64 x 128 tiles for 17..64 rows (gemm_pipe64_kernel).
 #include <algorithm>
-#include <cmath>
 
 #include "common.h"
 
@@ -1271,17 +1270,23 @@ struct ExpertRows {
   int experts;
 };
 
+// Blocks of 128 rows that the experts' rows make.
+__device__ inline int expert_row_blocks(const ExpertRows& ex) {
+  int blocks = 0;
+  for (int e = 0; e < ex.experts; ++e) blocks += (ex.offsets[e + 1] - ex.offsets[e] + BM128 - 1) / BM128;
+  return blocks;
+}
+
 // GROUPED: one launch for all experts of a routed layer.  The offsets are read here, so the host waits for nothing, and the list of
 // tiles is (expert, column block, row block), row blocks fastest: the blocks that share an expert's weights run side by side on
 // one XCD.  The grid holds the most tiles that any split of the rows can make; the ones too many are the last of each XCD's share.
+// (stages: Tile128<NJ>::STAGES * STAGE bytes of LDS; row_blocks: expert_row_blocks)
 template <bool GROUPED, int NJ>
-__global__ __launch_bounds__(256) void gemm_pipe128_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w,
-                                                           void* __restrict__ out, float* __restrict__ partial, int mode,
-                                                           int M, int N, int K, int ldo, RopeOut rp, int wt, int splits,
-                                                           ExpertRows ex) {
+__device__ __attribute__((always_inline)) inline void pipe128_block(unsigned char* stages, const bf16_t* __restrict__ x, const bf16_t* __restrict__ w,
+                                                                    void* __restrict__ out, float* __restrict__ partial, int mode, int M, int N, int K,
+                                                                    int ldo, const RopeOut& rp, int wt, int splits, const ExpertRows& ex, int row_blocks) {
   using T = Tile128<NJ>;
   constexpr int BNT = T::COLUMNS, NST = T::STAGES, LPWT = T::LOADS;
-  __shared__ __attribute__((aligned(1024))) unsigned char stages[NST * T::STAGE];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave >> 1, wn = wave & 1;
   // Blocks go to the 8 XCDs in turn, and each XCD has an L2 of its own: XCD j takes the j-th eighth of the list
@@ -1290,9 +1295,7 @@ __global__ __launch_bounds__(256) void gemm_pipe128_kernel(const bf16_t* __restr
   int MB, split, tile;
   if constexpr (GROUPED) {
     const int NB = (N + BNT - 1) / BNT;
-    int total = 0;
-    for (int e = 0; e < ex.experts; ++e) total += (ex.offsets[e + 1] - ex.offsets[e] + BM128 - 1) / BM128;
-    total *= NB;
+    const int total = row_blocks * NB;
     const int per_xcd = (total + 7) / 8;
     int item = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
     if ((int)(blockIdx.x >> 3) >= per_xcd || item >= total) return;
@@ -1452,6 +1455,36 @@ __global__ __launch_bounds__(256) void gemm_pipe128_kernel(const bf16_t* __restr
 #undef HALF
 }
 
+__global__ __launch_bounds__(256) void gemm_pipe128_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w, void* __restrict__ out,
+                                                           float* __restrict__ partial, int mode, int M, int N, int K, int ldo, RopeOut rp, int wt,
+                                                           int splits) {
+  __shared__ __attribute__((aligned(1024))) unsigned char stages[Tile128<4>::STAGES * Tile128<4>::STAGE];
+  pipe128_block<false, 4>(stages, x, w, out, partial, mode, M, N, K, ldo, rp, wt, splits, ExpertRows{}, 0);
+}
+
+// Whether the experts' products take blocks of 128 x 256 instead of 128 x 128 (the same bits): a quarter less traffic from L2 into LDS, which is what
+// bounds the smaller ones (32 KB a step of 64 of K and CU, 0.5 to 0.58 us where all CUs run), and half as many starts and ends; but a step takes 1.5 to
+// 1.9 times as long, so they pay where they need clearly fewer rounds of the CUs.  How many blocks of rows there are hangs on the routing: the kernel counts
+// them and chooses.  Eight experts, 128 / 256 columns / as chosen, us.  4,096 x 3,584, 1,024 pairs spread evenly 49 / 65 / 49, at random 82 / 68 / 67, all in one
+// expert 34 / 50 / 34; 2,048 x 2,048, 2,048 pairs 28 / 36 / 28, 46 / 37 / 38 and 25 / 34 / 25; 1,024 x 1,024, 4,096 pairs 16.0 / 21.2 / 16.4, 28 / 21 / 22 and
+// 17.6 / 20.6 / 18.0; 7,168 x 4,096 gated, 400 pairs in one expert 36 / 54 / 35, 4,096 pairs at random 313 / 280 / 283, 8,192 pairs 563 / 460 / 467;
+// 4,096 x 2,048 gated, 3,000 pairs (three rounds against two, spread evenly) 69.4 / 68.6 / 69.5.
+__host__ __device__ inline bool moe_wide(int row_blocks, int N) {
+  if (N % 256 != 0) return false;
+  const long rounds_256 = ((long)row_blocks * (N / 256) + 255) / 256, rounds_128 = ((long)row_blocks * (N / 128) + 255) / 256;
+  return 8 * rounds_256 < 5 * rounds_128;
+}
+
+// wide: blocks of 256 columns may be chosen.  (Both bodies in one kernel: a block has a CU to itself either way, by its LDS.)
+__global__ __launch_bounds__(256) void gemm_pipe128_experts_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w, void* __restrict__ out, int mode,
+                                                                   int N, int K, int ldo, int wt, int wide, RopeOut rp, ExpertRows ex) {
+  __shared__ __attribute__((aligned(1024))) unsigned char stages[Tile128<4>::STAGES * Tile128<4>::STAGE];
+  static_assert(Tile128<8>::STAGES * Tile128<8>::STAGE <= Tile128<4>::STAGES * Tile128<4>::STAGE, "stages of both tiles");
+  const int row_blocks = expert_row_blocks(ex);
+  if (wide && moe_wide(row_blocks, N)) pipe128_block<true, 8>(stages, x, w, out, nullptr, mode, 0, N, K, ldo, rp, wt, 1, ex, row_blocks);
+  else pipe128_block<true, 4>(stages, x, w, out, nullptr, mode, 0, N, K, ldo, rp, wt, 1, ex, row_blocks);
+}
+
 // Defined in gemm_mfma.hip.
 __global__ void gemm_splitk_reduce_kernel(const float* __restrict__ partial, void* __restrict__ out, int mode,
                                           int splits, int M, int N, GateAct ga);
@@ -1524,8 +1557,8 @@ static int tp_linear_pipe128(const bf16_t* x, const bf16_t* w, int w_tiled, void
   const int ldo = mode == OUT_SWIGLU ? N / 2 : N;
   const long per_xcd = (tiles * splits + 7) / 8;
   if (8 * per_xcd > 0x7fffffffL) return -1;
-  hipLaunchKernelGGL((gemm_pipe128_kernel<false, 4>), dim3((unsigned)(8 * per_xcd)), dim3(256), 0, s, x, w, out,
-                     splits > 1 ? scratch : nullptr, mode, M, N, K, ldo, rp, w_tiled, splits, ExpertRows{});
+  hipLaunchKernelGGL(gemm_pipe128_kernel, dim3((unsigned)(8 * per_xcd)), dim3(256), 0, s, x, w, out,
+                     splits > 1 ? scratch : nullptr, mode, M, N, K, ldo, rp, w_tiled, splits);
   if (splits > 1 && defer && splits_out != nullptr && mode != OUT_SWIGLU && mode != OUT_SPLIT) {
     *splits_out = splits;   // the parts stay unadded for the caller's next kernel
   } else if (splits > 1) {
@@ -1536,23 +1569,13 @@ static int tp_linear_pipe128(const bf16_t* x, const bf16_t* w, int w_tiled, void
   return 0;
 }
 
-// Whether the experts' products take blocks of 128 x 256 instead of 128 x 128 (the same bits): a quarter less traffic from L2 into LDS, which is what
-// bounds the smaller ones (32 KB a step of 64 of K and CU, 0.5 to 0.58 us where all CUs run), and half as many starts and ends; but a step takes 1.5 to
-// 1.9 times as long, so they pay where they need clearly fewer rounds of the CUs.  The rows of each expert are not known here: half a block of each is
-// taken as padding.  Eight experts, choice of two, 128 / 256 columns: 7,168 x 4,096 gated 512 / 1,024 / 2,048 rows 134.6 / 133.7, 204 / 194, 335 / 302 us;
-// 4,096 x 3,584 81 / 69, 117 / 119.5 (three rounds against two), 192 / 178; 4,096 x 2,048 gated 48.6 / 40.2, 69.4 / 70.6, 106.6 / 103.5;
-// 1,024 x 1,024 25.4 / 22.6 at 2,048 rows; 3,584 x 4,096 at 200 rows (one round either way) 50 / 72.
-static bool moe_wide(int pairs, int experts, int N) {
-  if (N % 256 != 0) return false;
-  const double row_blocks = (double)pairs / BM128 + 0.5 * std::min(pairs, experts);
-  auto rounds = [&](int columns) { return std::ceil(row_blocks * (N / columns) / 256.0); };
-  return 1.6 * rounds(256) < rounds(128);
-}
 // (the loads of a block's weights go by 32-bit offsets into 2 GiB: see load_lds16)
 static bool moe_wide_fits(int K) { return (size_t)(Tile128<8>::COLUMNS - 1) * K * 2 + 128 < ((size_t)1 << 31); }
-// For tests that mean a certain tile: the columns of a block.
-extern "C" int tp_moe_tile_columns(int pairs, int experts, int N, int K) { return moe_wide_fits(K) && moe_wide(pairs, experts, N) ? 256 : 128; }
-extern "C" int tp_moe_linear_columns(int pairs, int experts, int N) { return tp_moe_tile_columns(pairs, experts, N, BK); }
+// For tests that mean a certain tile: the columns of a block with so many blocks of 128 rows, and where half a block of every expert is padding.
+extern "C" int tp_moe_tile_columns(int row_blocks, int N, int K) { return moe_wide_fits(K) && moe_wide(row_blocks, N) ? 256 : 128; }
+extern "C" int tp_moe_linear_columns(int pairs, int experts, int N) {
+  return tp_moe_tile_columns((2 * pairs + BM128 * std::min(pairs, experts) + 2 * BM128 - 1) / (2 * BM128), N, BK);
+}
 
 // Rows sorted by expert (x [pairs, K], offsets [experts + 1] on the device) times the experts' weights w [experts, N, K] (w_tiled: each
 // in the tiled layout): out [pairs, N] float32 (mode 0), the gated activation [pairs, N / 2] (mode 2, interleaved rows) or max(v, 0)^2
@@ -1568,21 +1591,22 @@ extern "C" int tp_moe_linear(const void* x, const void* w, int w_tiled, void* ou
   TP_REQUIRE(x && w && out && offsets && (((uintptr_t)x | (uintptr_t)w | (uintptr_t)out) & 15) == 0, "moe_linear: missing or misaligned operand");
   TP_REQUIRE((size_t)(BM128 - 1) * K * 2 + 128 < ((size_t)1 << 31), "moe_linear: K too large");
   if (pairs == 0) return 0;
-  const bool wide = moe_wide_fits(K) && moe_wide(pairs, experts, N);
-  const long blocks = ((long)(wide ? N / 256 : (N + BN128 - 1) / BN128) * (pairs / BM128 + experts) + 7) / 8 * 8;
+  // Where every routing of so many pairs takes blocks of 256 columns the grid has no more; else as many as blocks of 128 need, of which those of 256 leave half
+  // without work (8,192 pairs, 2,048 x 1,024 gated, 42.8 us and, with twice the grid, 44.3).
+  const int most = pairs / BM128 + experts;
+  const bool wide = moe_wide_fits(K);
+  bool all_wide = wide;
+  for (int rows = (pairs + BM128 - 1) / BM128; all_wide && rows <= most; ++rows) all_wide = moe_wide(rows, N);
+  const long blocks = ((long)(all_wide ? N / 256 : (N + BN128 - 1) / BN128) * most + 7) / 8 * 8;
   TP_REQUIRE(blocks < 0x7fffffffL, "moe_linear: too many tiles");
   RopeOut rp = {};
   if (mode == 3) {
     rp.gate.act_cols = N;
     rp.gate.act_ld = N;
   }
-#define MOE_LINEAR(NJ_)                                                                                                                       \
-  hipLaunchKernelGGL((gemm_pipe128_kernel<true, NJ_>), dim3((unsigned)blocks), dim3(256), 0, s, (const bf16_t*)x, (const bf16_t*)w, out,        \
-                     (float*)nullptr, mode == 0 ? OUT_F32 : mode == 2 ? OUT_SWIGLU : OUT_SPLIT, 0, N, K, mode == 2 ? N / 2 : N, rp, w_tiled, 1, \
-                     ExpertRows{offsets, experts})
-  if (wide) MOE_LINEAR(8);
-  else MOE_LINEAR(4);
-#undef MOE_LINEAR
+  hipLaunchKernelGGL(gemm_pipe128_experts_kernel, dim3((unsigned)blocks), dim3(256), 0, s, (const bf16_t*)x, (const bf16_t*)w, out,
+                     mode == 0 ? OUT_F32 : mode == 2 ? OUT_SWIGLU : OUT_SPLIT, N, K, mode == 2 ? N / 2 : N, w_tiled, (int)wide, rp,
+                     ExpertRows{offsets, experts});
   TP_CHECK_LAUNCH("moe_linear");
   return 0;
 }

@@ -709,5 +709,39 @@ def test_moe_linear_of_256_columns_keeps_within_its_offsets():
     """A block of 256 columns reaches 255 rows of its weight by offsets into 2 GiB: longer rows, which blocks of 128 columns take, are left to those."""
     from tempura_amd.kernels import ops
     longest = (2 ** 31 - 129) // 510 // 64 * 64
-    columns = lambda k: ops.library().tp_moe_tile_columns(2195, 6, 2048, k)
+    columns = lambda k: ops.library().tp_moe_tile_columns(20, 2048, k)
     assert columns(64) == columns(longest) == 256 and columns(longest + 64) == columns((2 ** 31 - 129) // 254 // 64 * 64) == 128
+
+
+def test_moe_linear_chooses_its_blocks_by_the_rows_there_are():
+    """Blocks of 256 columns where they need clearly fewer rounds of 256 CUs, by the blocks of rows that the routing makes: as many pairs of rows need one
+    round or two.  (Blocks of rows and columns, and rounds of 128 / 256 columns.)"""
+    from tempura_amd.kernels import ops
+    for row_blocks, n, wide in ((16, 2048, False), (17, 2048, True), (8, 4096, False), (9, 4096, True), (16, 4096, True), (17, 4096, False), (24, 4096, False),
+                                (25, 4096, True), (1, 2048, False), (300, 128, False), (300, 384, False), (300, 256, False), (500, 256, True), (4000, 8192, True), (7, 7168, True),
+                                (10, 7168, False), (4, 7168, False)):
+        rounds = lambda columns: -(-row_blocks * (n // columns) // 256)
+        assert wide == (n % 256 == 0 and 8 * rounds(256) < 5 * rounds(128)), (row_blocks, n)
+        assert ops.library().tp_moe_tile_columns(row_blocks, n, 64) == (256 if wide else 128), (row_blocks, n)
+
+
+@pytest.mark.parametrize("counts", [[256] * 8, [2048] + [0] * 7, [0, 1024, 0, 0, 1024, 0, 0, 0], [300, 212, 129, 383, 255, 257, 1, 511], [2049, 0, 0, 0, 0, 0, 0, 0],
+                                    [512] * 8, [4096, 0, 0, 0, 0, 0, 0, 0], [1] * 7 + [8000]])
+@pytest.mark.parametrize("output", ["float32", "swiglu", "relu2"])
+def test_moe_linear_of_any_routing(counts, output):
+    """As many rows in one, two and eight experts, which take blocks of 128 and of 256 columns, and rows that always take those of 256: the bits of a product
+    for each expert alone."""
+    from tempura_amd.kernels import ops
+    g = torch.Generator().manual_seed(counts[0] + len(output))
+    E, pairs, n, k = len(counts), sum(counts), 2048, 192
+    row_blocks = sum(-(-c // 128) for c in counts)
+    assert ops.library().tp_moe_tile_columns(row_blocks, n, k) == (128 if row_blocks == 16 else 256)
+    x, w = torch.randn(pairs, k, generator=g).to(torch.bfloat16).to(DEV), (torch.randn(E * n, k, generator=g) * 0.2).to(torch.bfloat16).to(DEV)
+    first = [0] + torch.tensor(counts).cumsum(0).tolist()
+    got = ops.moe_linear(x, ops.tile_weight(w), torch.tensor(first, dtype=torch.int32, device=DEV), E, output)
+    for e in range(E):
+        for a in range(first[e], first[e + 1], 512):
+            b = min(a + 512, first[e + 1])
+            we = ops.tile_weight(w[e * n: (e + 1) * n].contiguous())
+            one = ops.moe_linear(x[a:b], we, torch.tensor([0, b - a], dtype=torch.int32, device=DEV), 1, output)
+            assert torch.equal(got[a:b], one)

@@ -282,7 +282,8 @@ class PagedAttention(Mixer):
         if self.gate and self.value_position is None:
             gated = torch.empty((x.shape[0], self.num_heads * self.value_dim), dtype=self.dtype, device=self.device)
             into = {"into": (gates, self.gate_col0, 1.0, gated, 0, 1)}
-        step = {**into, "shared": ctx.shared}
+        shared = getattr(ctx, "shared", None)      # (a context that a program made itself may share nothing)
+        step = {**into, "shared": shared}
         a, attended = None, False
         if q is None:
             rows = self._project(x, cache, rot)
@@ -291,7 +292,7 @@ class PagedAttention(Mixer):
                     and ops.attention_rows_pays(ctx, self.num_kv_heads, self.head_dim, int(self.window or 0), self.keep_first, self.chunk):
                 # single tokens: the attention takes the projection's rows itself
                 inv_freq, rotary_dim, factor = rot if rot is not None else (None, 0, 1.0)
-                table = self.position.table(ctx, always=True) if hasattr(self.position, "table") else None
+                table = self.position.table(ctx, always=shared is not None) if hasattr(self.position, "table") else None
                 norms = {} if self.qk_norm is None else {"norms": (self.q_norm_w, self.k_norm_w), "norm_eps": float(self.qk_norm["eps"])}
                 a = ops.attention_rows(rows, 0, ctx, cache.group, self.num_heads, self.num_kv_heads, self.head_dim, cache.k, cache.v, self.scale,
                                        inv_freq, rotary_dim, factor, table, int(self.window or 0), self.keep_first, self.chunk, self.sink_w,
@@ -549,7 +550,7 @@ class ConvAttention(BranchMixer):
                                   self.num_kv_heads, self.head_dim, cache.k, cache.v, self.dtype, table, value_dim=self.value_dim,
                                   pad_dim=self.key_dim)
         ops.paged_attention(q, cache.k, cache.v, ctx.block_tables[cache.group], ctx.cu_seqlens, ctx.context_lens,
-                            ctx.token_req, self.scale, int(self.window or 0), ctx.max_q_len, ctx.max_context_len, ctx.num_single, into=into, shared=ctx.shared)
+                            ctx.token_req, self.scale, int(self.window or 0), ctx.max_q_len, ctx.max_context_len, ctx.num_single, into=into, shared=getattr(ctx, "shared", None))
 
 
 register_part("mixer", "conv_attention", ConvAttention)
@@ -640,7 +641,7 @@ class LatentAttention(BranchMixer):
                               cache.k, cache.v, self.dtype, table, value_dim=self.value_dim)
         ops.paged_attention(q, cache.k, cache.v, ctx.block_tables[cache.group], ctx.cu_seqlens, ctx.context_lens,
                             ctx.token_req, self.scale, int(self.window or 0), ctx.max_q_len, ctx.max_context_len, ctx.num_single,
-                            into=(proj if self.gate else None, col0 + self.q_dim + self.down_dim, scale, out, out_col0, 1), shared=ctx.shared)
+                            into=(proj if self.gate else None, col0 + self.q_dim + self.down_dim, scale, out, out_col0, 1), shared=getattr(ctx, "shared", None))
 
 
 register_part("mixer", "latent_attention", LatentAttention)
@@ -742,7 +743,7 @@ class LatentCacheAttention(BranchMixer):
         q = ops.linear(cq, self.w_q, self.dtype).view(n, self.num_heads, self.latent_dim)
         ops.paged_attention(q, cache.k, cache.v, ctx.block_tables[cache.group], ctx.cu_seqlens, ctx.context_lens, ctx.token_req,
                             self.scale, int(self.window or 0), ctx.max_q_len, ctx.max_context_len, ctx.num_single, sink=self.sink_w,
-                            into=(None, 0, scale, out, out_col0, 1), shared=ctx.shared)
+                            into=(None, 0, scale, out, out_col0, 1), shared=getattr(ctx, "shared", None))
 
 
 register_part("mixer", "latent_cache_attention", LatentCacheAttention)

@@ -250,3 +250,22 @@ def test_command_line_inspects_and_writes_random_folders(dirs, tmp_path, capsys)
     assert model.layers[2].mixer.dist_table.shape[0] == 6 and model.streams == 1
     # connection tensors are drawn around the plain residual sum
     assert abs(float(model.layers[0].mixer_link.mix[0, 0]) - 1.0) < 1.5
+
+
+@pytest.mark.parametrize("name", ["attn", "mix"])
+def test_a_context_without_shared_values(dirs, name, monkeypatch):
+    """Steps whose context shares nothing between its layers: the same logits."""
+    from tempura_amd.engine.runner import StepContext, StepEntry
+    first = list(cases.requests(name).values())[1]
+
+    def logits():
+        runner = _runner(dirs, name, 64)
+        runner.add_request("r")
+        return [runner.step([StepEntry("r", part, [len(part) - 1])]) for part in (first[:-2], first[-2:-1], first[-1:])]
+    want, plain_init = logits(), StepContext.__init__
+
+    def init(self):
+        plain_init(self)
+        del self.shared
+    monkeypatch.setattr(StepContext, "__init__", init)
+    assert all(torch.equal(a, b) for a, b in zip(logits(), want))

@@ -28,8 +28,10 @@ ARCH = "gfx950"
 # instructions from ordinary float code.
 # The first 16 dwords of a kernel's arguments arrive in scalar registers with its waves instead of by a load from
 # memory that every wave's first address waits for: a decode step is 40 to 200 dependent launches, each of which
-# began with that trip (steps of 8 requests of the 8B shape 3,508 -> 3,474 us, 2,048 rows' designs 0.4 to 0.9 % a
-# request, prompts 0.6 %; the same instructions otherwise).  Pointers and sizes in front, structures behind them.
+# began with that trip (one request of the 3B shape 1,477 -> 1,459 us a step, eight of the 8B shape 3,308 -> 3,263, 48 of
+# the 3B shape 2,962 -> 2,931, 700 tokens beside 31 requests 6,400 -> 6,342, whole requests of the designs 0.6 to 0.9 %
+# but for one with none; a prompt of 5,000 tokens 71,439 and 71,364, float32 none beyond its noise; the same
+# instructions otherwise).  Pointers and sizes in front, structures behind them.
 FLAGS = ["-O3", "-std=c++17", "-fPIC", f"--offload-arch={ARCH}", "-ffp-contract=off",
          "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops", "-Wno-unused-result",
          "-mllvm", "-amdgpu-kernarg-preload-count=16"]

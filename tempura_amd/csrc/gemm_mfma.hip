@@ -776,13 +776,13 @@ static void launch_few2(const bf16_t* x, const bf16_t* w, void* out, int mode, i
   // LDS: K 4,096, 256 blocks 7.4 / 7.6 us, 257 9.7 / 8.6, 384 11.8 / 10.4, 512 13.0 / 12.5; K 2,048 4.7 / 5.0, 5.6 / 5.1, 6.6 / 6.1 and 7.5 / 7.1; K 8,192
   // 12.6 / 12.9, 17.8 / 16.0, 21.6 / 18.9 and 24.0 / 23.0.
   if (M > 1 ? !major || pieces > 4 : blocks <= 256 || pieces > 8) FEW(0, true);
-  // From three blocks a CU on, or with more than 32 KB, a row of 4,096 and more also has two runs on their way and no more than two blocks a CU (56 KB of LDS).
-  // One run from memory / two through LDS: K 4,096, 576 blocks 15.4 / 14.6 us, 1,024 22.7 / 22.5, 8,016 153.0 / 153.5; K 8,192, 768 blocks 33.8 / 33.0, 1,792 72.5 / 71.1,
-  // 8,016 300.8 / 302.9; K 14,336, 576 48.6 / 45.7, 1,792 123.9 / 120.7, 4,000 270.7 / 263.9; K 28,672, 512 75.9 / 72.1; but K 2,048, 1,280 blocks 14.7 / 15.3, and K 3,072,
-  // 384 blocks, one and two through LDS 8.0 / 8.3.
+  // From three blocks a CU on, or with more than 32 KB, a row of more than 4,096 also has two runs on their way and no more than two blocks a CU (56 KB of LDS).
+  // One run from memory / two through LDS: K 8,192, 768 blocks 33.8 / 33.0 us, 1,792 72.5 / 71.1, 8,016 300.8 / 302.9; K 14,336, 576 48.6 / 45.7, 1,792
+  // 123.9 / 120.7, 4,000 270.7 / 263.9; K 28,672, 512 75.9 / 72.1; six layers of the 70B shape, one row, 1,983 / 1,963.  Shorter rows gain alone what they lose
+  // behind other kernels, where the wait for the copy counts: K 4,096, 576 blocks 15.4 / 14.6 and 1,024 22.7 / 22.5, but four layers with products of
+  // 1,100 to 1,800 blocks 16,330 / 16,490 us for 24 steps; K 2,048, 1,280 blocks 14.7 / 15.3; K 3,072, 384 blocks, one and two through LDS 8.0 / 8.3.
   if (M == 1 && (blocks > 512 || pieces > 4)) {
-    if (K < 4 * FEW_CHUNK || (K <= 8 * FEW_CHUNK && blocks > 2048)) FEW(0, true);
-    if (pieces <= 1) FEW_DEEP(1);
+    if (K <= 4 * FEW_CHUNK || (K <= 8 * FEW_CHUNK && blocks > 2048)) FEW(0, true);
     if (pieces <= 2) FEW_DEEP(2);
     if (pieces <= 4) FEW_DEEP(4);
     FEW_DEEP(8);

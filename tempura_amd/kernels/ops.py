@@ -2108,10 +2108,12 @@ def moe_plan(ids: torch.Tensor, experts: int):
 
 def moe_linear_ok(experts: int, n: int, k: int, w, pairs: int = 0) -> bool:
     """Whether ``moe_linear`` takes the experts' stacked weight ``w`` (each [n, k]) and is the better way for ``pairs`` rows."""
-    # (its tiles are 128 x 128 or 128 x 256; from some thousand rows an expert on, a product for each with tiles of 256 x 256 is faster.  Both
-    # products of eight experts, 8,192 / 16,384 / 32,768 pairs, a product an expert against one launch: 4,096 x 4,096 gated and 4,096 x
-    # 2,048 533 / 773 / 1,303 us against 439 / 827 / 1,831; 4,096 x 2,048 and 2,048 x 2,048 334 / 476 / 768 against 213 / 440 / 955; 7,168 x
-    # 4,096 and 4,096 x 3,584 785 / 1,270 / 2,271 against 655 / 1,320 / 2,977)
+    # (its tiles are 128 x 128 or 128 x 256; from some thousand rows an expert on, a product for each with tiles of 256 x 256 is the faster
+    # product.  Both products of eight experts alone, 8,192 / 16,384 / 32,768 pairs, a product an expert against one launch: 4,096 x 4,096 gated
+    # and 4,096 x 2,048 533 / 773 / 1,303 us against 439 / 827 / 1,831; 4,096 x 2,048 and 2,048 x 2,048 334 / 476 / 768 against 213 / 440 / 955; 7,168 x
+    # 4,096 and 4,096 x 3,584 785 / 1,270 / 2,271 against 655 / 1,320 / 2,977.  But a product an expert waits on the host for the rows' counts and is
+    # sixteen launches: the whole layer, routing and gathering included, 8,192 / 16,384 / 24,576 pairs at random, 744 / 1,236 / 1,593 us against 548 /
+    # 1,070 / 1,489; 459 / 722 / 957 against 317 / 592 / 816; 1,050 / 1,638 / 2,320 against 828 / 1,615 / 2,331.  So up to 2,048 rows an expert go in one.)
     if pairs > 2048 * experts:
         return False
     return _backend is None and allow_mfma and w is not None and w.dtype == torch.bfloat16 and 0 < experts <= 64 and n % 16 == 0 and k % 64 == 0 and \

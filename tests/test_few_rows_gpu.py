@@ -549,7 +549,8 @@ def test_latent_norms_and_store(n, q_dim, c_dim, dtype):
 @pytest.mark.parametrize("tiled", [True, False])
 def test_products_of_few_rows_at_the_edges_of_their_variants(m, k, n, tiled):
     """Rows through LDS (one to four pieces a thread, one and several rows) and straight from memory, whole and partial runs of K, waves without
-    a run, more column blocks than CUs; every kind of end.  Bounds: k products of exact bfloat16 factors summed in float32 are within k * 2^-24 of
+    a run, more column blocks than CUs; sums that are stored, or added into the stream with the next norm prepared, and a product that finishes it (all other
+    ends: ``test_row_major_rows`` and ``test_one_row_through_lds``).  Bounds: k products of exact bfloat16 factors summed in float32 are within k * 2^-24 of
     the sum of their magnitudes; a result in bfloat16 within 2^-8 of itself besides; the norm's scale adds 2^-22 (its own sum and root)."""
     from tempura_amd.kernels import ops
     g = torch.Generator().manual_seed(m + k + n)
@@ -676,9 +677,11 @@ def _every_end(ops, plain, normed, w, g):
 
 
 @pytest.mark.parametrize("m,k,n,tiled", [(2, 2048, 65536, True), (16, 4160, 16384, True), (15, 8192, 16400, True), (14, 8192, 16400, True), (12, 4096, 65536, True), (11, 4096, 65536, True),
-                                         (2, 2048, 48, False), (16, 3104, 64, False), (9, 4128, 160, False), (8, 8192, 48, False), (7, 8192, 48, False), (16, 8224, 48, False)])
-def test_row_major_rows_of_wide_products(m, k, n, tiled):
-    """Rows through LDS in chunks of K, whole and partial ones, and sizes beside theirs: the bits of k-blocked rows at every end."""
+                                         (2, 2048, 48, False), (16, 3104, 64, False), (9, 4128, 160, False), (8, 8192, 48, False), (7, 8192, 48, False), (16, 8224, 48, False),
+                                         (2, 1024, 64, True), (16, 512, 4128, True), (3, 2112, 48, True), (4, 4096, 160, True), (5, 4096, 160, True), (16, 2048, 4112, True)])
+def test_row_major_rows(m, k, n, tiled):
+    """Rows through LDS in chunks of K, whole and partial ones, rows that go there whole (one to four pieces a thread), and sizes beside theirs: the bits of
+    k-blocked rows at every end."""
     from tempura_amd.kernels import ops
     g = torch.Generator().manual_seed(m + k + n)
     x, ss = torch.randn(m, k, generator=g).to(torch.bfloat16).to(DEV), torch.rand(m, k // 16, generator=g).to(DEV).t()

@@ -758,15 +758,24 @@ static void launch_few2(const bf16_t* x, const bf16_t* w, void* out, int mode, i
 #define FEW_DEEP(P_) return launch_few3<P_, KIND, PRE, true, true>(x, w, out, mode, M, N, K, layout, pre, post, rp, s)
   const bool tiled = (layout & W_TILED) != 0, major = M > 1 && (layout & X_KBLOCKED) == 0;
   const int blocks = (N + 15) / 16, pieces = (M * (K / 8) + FEW_WAVES * 64 - 1) / (FEW_WAVES * 64);
-  // Row-major rows of wide products go through LDS in chunks: read from memory as operands, 64-byte pieces of up to sixteen rows, their way into the CU is as
-  // long as the weights' where there are many column blocks.  From memory (to 32 KB through LDS) / in chunks, tiled weight, 128,256 columns, K 3,072: two rows
-  // 117.0 / 115.4 us, eight 124.0 / 120.8, sixteen 156.4 / 138.7; K 4,096: ten 171.3 / 177.3, twelve 183.9 / 180.4, sixteen 201.9 / 183.1; 16,384 columns, K 3,072: 14 rows 19.7 / 19.8,
-  // sixteen 20.9 / 20.3; 28,672, K 4,096: 14 rows 42.5 / 43.6, sixteen 45.4 / 44.0; 8,192 columns, K 2,048, sixteen rows 8.4 / 8.6.  A row-major weight takes that
+  // Row-major rows of products with more column blocks than CUs go through LDS in chunks: read from memory as operands, 64-byte pieces of up to sixteen rows,
+  // their way into the CU is as long as the weights' where blocks follow or share a CU.  From memory (to 32 KB through LDS) / in chunks, tiled weight, us; first
+  // float32 results, then the sums added into the stream with the next norm prepared.  Sixteen rows: K 2,048, 272 blocks 7.5 / 7.4 and 8.1 / 7.7, 512 8.5 / 8.6 and
+  // 9.5 / 9.2, 1,792 25.5 / 23.5; K 4,096, 272 13.6 / 12.8 and 13.7 / 12.9, 512 15.9 / 15.4 and 16.5 / 15.8, 896 27.5 / 25.3 and 28.6 / 25.9; K 8,192, 272 24.4 / 22.9
+  // and 25.0 / 23.2, 512 27.9 / 26.9 and 29.0 / 27.1, 896 50.2 / 45.4 and 51.8 / 46.2, 1,792 88.0 / 81.2; but with a CU a block the latter K 2,048 6.0 / 6.1, K 4,096
+  // 8.9 / 9.5, K 8,192 16.0 / 17.0.  Fourteen: K 2,048, 512 8.3 / 8.6 and 9.0 / 8.9; K 4,096, 384 13.8 / 14.1 and 14.6 / 14.6, 1,792 44.2 / 43.4 and 46.8 / 45.5; K 6,144,
+  // 384 19.9 / 19.6 and 20.5 / 20.0, 768 30.0 / 30.8 and 30.9 / 31.2; K 8,192, 272 23.0 / 22.3 and 23.7 / 22.9, 512 26.4 / 26.4 and 27.2 / 26.7, 896 47.8 / 45.2 and 48.8 / 46.0.  Thirteen: K 8,192, 768 36.8 / 38.5 and 37.8 / 39.0, 896
+  // 46.4 / 44.9 and 47.4 / 45.6, 1,792 80.5 / 81.5 and 84.4 / 83.8; K 5,120, 1,728 53.6 / 50.8 and 55.4 / 52.2; K 6,144, 1,792 62.9 / 63.6 and 65.3 / 65.8.  Twelve: K 3,072, 512
+  // the latter 12.0 / 11.8, 1,792 32.7 / 32.3 and 34.6 / 33.2; K 2,048, 4,000 52.9 / 52.1; K 4,096, 1,280 32.3 / 33.0, 1,792 42.2 / 43.1; K 6,144, 1,792 61.9 / 62.7 and
+  // 63.2 / 64.3; K 8,192, 896 45.5 / 43.9 and 46.4 / 45.0, 1,792 79.2 / 81.0.  Float32 results of 128,256 columns: K 3,072, two rows 117.0 / 115.4, eight 124.0 / 120.8,
+  // sixteen 156.4 / 138.7; K 4,096, ten 171.3 / 177.3, twelve 183.9 / 180.4, sixteen 201.9 / 183.1.  A row-major weight takes that
   // way twice over: 4,096 x 128,256 eight rows 227 / 206, sixteen 270 / 230; 4,096 x 6,144 16.1 / 15.5 and 18.6 / 17.0; 2,048 x 8,192 9.6 / 9.5 and 10.9 / 10.5;
   // 8,192 x 4,096 six rows 18.2 / 19.2, eight 19.3 / 19.4, sixteen 21.4 / 20.7.  (Chunks are of use from two on, and to 8,192: 14,336 x 4,096 eight rows
   // 21.6 / 26.0.)
   if (major && K >= 2 * FEW_CHUNK && K <= 8 * FEW_CHUNK) {
-    if (tiled && blocks >= 1024 && (M > 14 || (blocks >= 4096 && (M >= 12 || K <= 3 * FEW_CHUNK)))) FEW(-1, true);
+    const bool short_k = K <= 3 * FEW_CHUNK;
+    const int from = blocks <= 256 ? 17 : blocks < 896 ? (blocks <= 512 && K > 4 * FEW_CHUNK ? 14 : 15) : blocks < 4096 ? (short_k ? 12 : 13) : short_k ? 2 : 12;      // rows
+    if (tiled && M >= from) FEW(-1, true);
     if (!tiled && (K <= 4 * FEW_CHUNK || M >= 8)) FEW(-1, false);
   }
   if (!tiled) FEW(0, false);

@@ -678,7 +678,8 @@ def _every_end(ops, plain, normed, w, g):
 
 @pytest.mark.parametrize("m,k,n,tiled", [(2, 2048, 65536, True), (16, 4160, 16384, True), (15, 8192, 16400, True), (14, 8192, 16400, True), (12, 4096, 65536, True), (11, 4096, 65536, True),
                                          (2, 2048, 48, False), (16, 3104, 64, False), (9, 4128, 160, False), (8, 8192, 48, False), (7, 8192, 48, False), (16, 8224, 48, False),
-                                         (2, 1024, 64, True), (16, 512, 4128, True), (3, 2112, 48, True), (4, 4096, 160, True), (5, 4096, 160, True), (16, 2048, 4112, True)])
+                                         (2, 1024, 64, True), (16, 512, 4128, True), (3, 2112, 48, True), (4, 4096, 160, True), (5, 4096, 160, True), (16, 2048, 4096, True),
+                                         (15, 2048, 4112, True), (14, 8192, 8192, True), (14, 8192, 8208, True), (13, 8192, 4112, True), (13, 3136, 14336, True), (13, 3136, 14320, True), (12, 3072, 14336, True), (12, 3136, 14336, True)])
 def test_row_major_rows(m, k, n, tiled):
     """Rows through LDS in chunks of K, whole and partial ones, rows that go there whole (one to four pieces a thread), and sizes beside theirs: the bits of
     k-blocked rows at every end."""

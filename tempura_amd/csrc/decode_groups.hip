@@ -24,24 +24,49 @@ __device__ inline f32x4_t dg_mfma(u32x4_t w, u32x4_t x, f32x4_t acc) {
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, w), __builtin_bit_cast(bf16x8_t, x), acc, 0, 0, 0);
 }
 
-// acc += the wave's runs of one 16-row tile of a weight: wp this lane's first piece of the tile, xp of the rows; steps of 32 k.  One run on its way at a
-// time (see gemm_few_kernel in gemm_mfma.hip).  A decode step of Zemarax at width 4,096 494 -> 473 us with both, Golavik's 701 -> 675, Makisun's 461 -> 444.
+// acc += the wave's runs of one 16-row tile of a weight: wp this lane's first piece of the tile, xp of the rows; steps of 32 k.  DEPTH runs on their way at
+// a time (see gemm_few_kernel in gemm_mfma.hip and dg_deep).  One run: a decode step of Zemarax at width 4,096 494 -> 473 us with both, Golavik's 701 -> 675, Makisun's 461 -> 444.
+template <int DEPTH = 1>
 __device__ inline f32x4_t dg_tile(const u32x4_t* wp, const u32x4_t* xp, int xstep, int steps, int wave, f32x4_t acc) {
   const int runs = steps / 4;      // (whole ones)
-  for (int run = wave; run < runs; run += DG_WAVES) {
-    u32x4_t a[4], b[4];
+  u32x4_t a[DEPTH][4], b[DEPTH][4];
+  auto request = [&](int d, int run) __attribute__((always_inline)) {
 #pragma unroll
-    for (int u = 0; u < 4; ++u) a[u] = __builtin_nontemporal_load(wp + (size_t)(run * 4 + u) * 64);
+    for (int u = 0; u < 4; ++u) a[d][u] = __builtin_nontemporal_load(wp + (size_t)(run * 4 + u) * 64);
 #pragma unroll
-    for (int u = 0; u < 4; ++u) b[u] = xp[(size_t)(run * 4 + u) * xstep];
+    for (int u = 0; u < 4; ++u) b[d][u] = xp[(size_t)(run * 4 + u) * xstep];
+  };
+  auto multiply = [&](int d) __attribute__((always_inline)) {
+#pragma unroll
+    for (int u = 0; u < 4; ++u) acc = dg_mfma(a[d][u], b[d][u], acc);
+  };
+  int run = wave;
+  if constexpr (DEPTH == 2) {
+    for (; run + DG_WAVES < runs; run += 2 * DG_WAVES) {
+      request(0, run);
+      request(1, run + DG_WAVES);
+      __builtin_amdgcn_sched_barrier(0);
+      multiply(0);
+      multiply(1);
+    }
+  }
+  for (; run < runs; run += DG_WAVES) {
+    request(0, run);
     __builtin_amdgcn_sched_barrier(0);      // (all of a run's loads in front of its first product)
-#pragma unroll
-    for (int u = 0; u < 4; ++u) acc = dg_mfma(a[u], b[u], acc);
+    multiply(0);
   }
   if (wave == runs % DG_WAVES)     // what is left of K, fewer than four steps
     for (int s = runs * 4; s < steps; ++s) acc = dg_mfma(__builtin_nontemporal_load(wp + (size_t)s * 64), xp[(size_t)s * xstep], acc);
   return acc;
 }
+
+// Whether the waves of a product have two runs on their way: one or two rows with a long K and more blocks than CUs.  These are bound by the weights alone, and a
+// block that comes to its end leaves a CU with one run a wave (more rows' own loads fill that, and with up to one block a CU the second run's place costs
+// more than it gives).  One run / two, one row and two, us: four copies' closing product 13,824 x 5,120 32.5 / 31.2 and 32.5 / 31.2, 14,336 x 8,192 40.6 / 39.4 and 40.4 / 39.3,
+// 28,672 x 8,192 77.4 / 74.6 and 76.8 / 74.7 (four rows 74.9 / 74.8), but 14,336 x 4,096 21.7 / 21.9 and 21.5 / 21.9, 8,192 x 2,048 11.3 / 11.5; groups 14,336 x
+// 8,192 39.3 / 38.5, 4,096 x 8,192 13.2 / 13.1, but 2,048 x 4,096 4.9 / 5.0; experts, choice of two of eight, width 4,096 with 3,584 38.2 / 37.0 and 63.5 / 61.5, 6,144
+// with 16,384 205 / 197 and 390 / 374, 8,192 with 4,096 72.1 / 70.0 and 133.8 / 127.7, but width 2,048 with 1,408 (six of 64) 35.8 / 37.6 and 54.1 / 57.4.
+static bool dg_deep(int M, int K, int blocks) { return M <= 2 && K >= 4096 && blocks > 256; }
 
 // the waves' sums of element q (lane q / 4, register q % 4) in wave order
 __device__ inline float dg_sum(const float (*red)[256], int q) {
@@ -57,6 +82,7 @@ struct GroupEnds {
   int end[DG_MAX_GROUPS];
 };
 
+template <int DEPTH>
 __global__ __launch_bounds__(DG_WAVES * 64) void group_linear_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w,
                                                                       float* __restrict__ out, GroupEnds ends, int M, int N, int K) {
   __shared__ float red[DG_WAVES][256];
@@ -68,7 +94,7 @@ __global__ __launch_bounds__(DG_WAVES * 64) void group_linear_kernel(const bf16_
   const u32x4_t* wp = (const u32x4_t*)(w + (size_t)n0 * K) + lane;
   const int row = min(lane & 15, M - 1);
   const u32x4_t* xp = (const u32x4_t*)(x + (size_t)g * M * K + ((size_t)(lane >> 4) * M + row) * 8);
-  const f32x4_t acc = dg_tile(wp, xp, 4 * M, K / 32, wave, (f32x4_t){0.f, 0.f, 0.f, 0.f});
+  const f32x4_t acc = dg_tile<DEPTH>(wp, xp, 4 * M, K / 32, wave, (f32x4_t){0.f, 0.f, 0.f, 0.f});
 #pragma unroll
   for (int r = 0; r < 4; ++r) red[wave][lane * 4 + r] = acc[r];
   __syncthreads();
@@ -89,7 +115,7 @@ extern "C" int tp_group_linear(const void* x, const void* w, float* out, const i
     e.end[i] = i < groups ? ends[i] : N;
     TP_REQUIRE(e.end[i] % 16 == 0 && e.end[i] <= N && e.end[i] > (i > 0 && i < groups ? e.end[i - 1] : 0), "group_linear: bad group borders");
   }
-  hipLaunchKernelGGL(group_linear_kernel, dim3(N / 16), dim3(DG_WAVES * 64), 0, s, (const bf16_t*)x, (const bf16_t*)w, out, e, M, N, K);
+  hipLaunchKernelGGL(dg_deep(M, K, N / 16) ? group_linear_kernel<2> : group_linear_kernel<1>, dim3(N / 16), dim3(DG_WAVES * 64), 0, s, (const bf16_t*)x, (const bf16_t*)w, out, e, M, N, K);
   TP_CHECK_LAUNCH("group_linear");
   return 0;
 }
@@ -140,6 +166,7 @@ struct StreamEnd {
   float* ss;
 };
 
+template <int DEPTH>
 __global__ __launch_bounds__(DG_WAVES * 64) void stream_linear_kernel(const bf16_t* __restrict__ x, int blocked, const bf16_t* __restrict__ w,
                                                                        float* __restrict__ h, StreamEnd e, int M, int N, int K) {
   __shared__ float red[DG_WAVES][256];
@@ -166,7 +193,7 @@ __global__ __launch_bounds__(DG_WAVES * 64) void stream_linear_kernel(const bf16
   const u32x4_t* wp = (const u32x4_t*)(w + (size_t)n0 * K) + lane;
   const int row = min(lane & 15, M - 1);
   const u32x4_t* xp = blocked ? (const u32x4_t*)x + (size_t)(lane >> 4) * M + row : (const u32x4_t*)(x + (size_t)row * K) + (lane >> 4);
-  const f32x4_t acc = dg_tile(wp, xp, blocked ? 4 * M : 4, K / 32, wave, (f32x4_t){0.f, 0.f, 0.f, 0.f});
+  const f32x4_t acc = dg_tile<DEPTH>(wp, xp, blocked ? 4 * M : 4, K / 32, wave, (f32x4_t){0.f, 0.f, 0.f, 0.f});
 #pragma unroll
   for (int r = 0; r < 4; ++r) red[wave][lane * 4 + r] = acc[r];
   __syncthreads();
@@ -206,7 +233,7 @@ extern "C" int tp_stream_linear(const void* x, int blocked, const void* w, float
   TP_REQUIRE(norm_w == nullptr || (xg != nullptr && ss != nullptr), "stream_linear: no room for the rows of the next norm");
   const StreamEnd e = {mix, outc, inc, norm_w, (bf16_t*)xg, ss};
   TP_REQUIRE(streams == 4, "stream_linear: %d copies of the stream (takes 4)", streams);
-  hipLaunchKernelGGL(stream_linear_kernel, dim3(N / 16), dim3(DG_WAVES * 64), 0, s, (const bf16_t*)x, blocked, (const bf16_t*)w, h, e, M, N, K);
+  hipLaunchKernelGGL(dg_deep(M, K, N / 16) ? stream_linear_kernel<2> : stream_linear_kernel<1>, dim3(N / 16), dim3(DG_WAVES * 64), 0, s, (const bf16_t*)x, blocked, (const bf16_t*)w, h, e, M, N, K);
   TP_CHECK_LAUNCH("stream_linear");
   return 0;
 }
@@ -215,7 +242,7 @@ extern "C" int tp_stream_linear(const void* x, int blocked, const void* w, float
 // Up: a[m][e * ff + c] = f(x_m . up_e[c]) * dense[m][e] as bfloat16, k-blocked over the columns of all experts; experts whose
 // column of `dense` is zero for all rows are skipped (their columns stay unwritten).  GATED: the weight's rows alternate
 // eight gate rows and eight up rows, and f is silu(gate) * up.
-template <bool GATED>
+template <bool GATED, int DEPTH>
 __global__ __launch_bounds__(DG_WAVES * 64) void moe_up_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w,
                                                                 const float* __restrict__ dense, bf16_t* __restrict__ a, int M, int experts,
                                                                 int rows, int K, int kind) {
@@ -227,7 +254,7 @@ __global__ __launch_bounds__(DG_WAVES * 64) void moe_up_kernel(const bf16_t* __r
   const u32x4_t* wp = (const u32x4_t*)(w + (size_t)n0 * K) + lane;
   const int row = min(lane & 15, M - 1);
   const u32x4_t* xp = (const u32x4_t*)(x + ((size_t)(lane >> 4) * M + row) * 8);
-  const f32x4_t acc = dg_tile(wp, xp, 4 * M, K / 32, wave, (f32x4_t){0.f, 0.f, 0.f, 0.f});
+  const f32x4_t acc = dg_tile<DEPTH>(wp, xp, 4 * M, K / 32, wave, (f32x4_t){0.f, 0.f, 0.f, 0.f});
 #pragma unroll
   for (int r = 0; r < 4; ++r) red[wave][lane * 4 + r] = acc[r];
   __syncthreads();
@@ -342,6 +369,7 @@ extern "C" int tp_moe_open(const void* x, const void* w_router, const float* cor
 // behind the other.  gridDim.y > 1: every expert's K in that many equal parts of whole runs, y [parts, M, N] (see split_linear_kernel).
 // ws: then the shared expert's tiled [N, size] (nullptr: none) times a_shared, its sum added on its own, times
 // sigmoid(gate[m]) where there is a gate.
+template <int DEPTH>
 __global__ __launch_bounds__(DG_WAVES * 64) void moe_down_kernel(const bf16_t* __restrict__ a, const bf16_t* __restrict__ w,
                                                                   const float* __restrict__ dense, float* __restrict__ y, int M, int experts,
                                                                   int ff, int N, int accumulate, const bf16_t* __restrict__ ws,
@@ -376,7 +404,29 @@ __global__ __launch_bounds__(DG_WAVES * 64) void moe_down_kernel(const bf16_t* _
   // run r of expert e goes to wave (e * runs + r) % 8: `per` turns an expert
   const int per = (runs + DG_WAVES - 1) / DG_WAVES;
   f32x4_t acc = (f32x4_t){0.f, 0.f, 0.f, 0.f};
-  for (int it = 0; it < total * per; ++it) {
+  int it = 0;
+  if constexpr (DEPTH == 2) {      // (every expert's runs are whole and a multiple of the waves)
+    for (; it + 1 < total * per; it += 2) {
+      u32x4_t av[2][4], bv[2][4];
+#pragma unroll
+      for (int d = 0; d < 2; ++d) {
+        const int e = __builtin_amdgcn_readfirstlane(list[(it + d) / per]);
+        const int run = (it + d) % per * DG_WAVES + ((wave - e * runs) & (DG_WAVES - 1));
+        const u32x4_t* wp = w_lane + (size_t)e * w_expert + (size_t)run * 256;
+        const u32x4_t* xp = x_lane + (size_t)e * x_expert + (size_t)run * 4 * xstep;
+#pragma unroll
+        for (int u = 0; u < 4; ++u) av[d][u] = __builtin_nontemporal_load(wp + u * 64);
+#pragma unroll
+        for (int u = 0; u < 4; ++u) bv[d][u] = xp[(size_t)u * xstep];
+      }
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int d = 0; d < 2; ++d)
+#pragma unroll
+        for (int u = 0; u < 4; ++u) acc = dg_mfma(av[d][u], bv[d][u], acc);
+    }
+  }
+  for (; it < total * per; ++it) {
     const int e = __builtin_amdgcn_readfirstlane(list[it / per]);
     const int run = it % per * DG_WAVES + ((wave - e * runs) & (DG_WAVES - 1));
     if (run >= runs) continue;
@@ -439,11 +489,13 @@ extern "C" int tp_moe_few(const void* x, const void* w_up, const void* w_down, c
   const int rows = gated ? 2 * ff : ff;
   TP_REQUIRE((long)experts * rows < 0x7fffffffL, "moe_few: too many rows");
   const dim3 up(experts * rows / 16), block(DG_WAVES * 64);
+  const bool deep = dg_deep(M, K, experts * rows / 16);
   if (gated)
-    hipLaunchKernelGGL(moe_up_kernel<true>, up, block, 0, s, (const bf16_t*)x, (const bf16_t*)w_up, dense, (bf16_t*)a, M, experts, rows, K, 0);
+    hipLaunchKernelGGL((deep ? moe_up_kernel<true, 2> : moe_up_kernel<true, 1>), up, block, 0, s, (const bf16_t*)x, (const bf16_t*)w_up, dense, (bf16_t*)a, M, experts, rows, K, 0);
   else
-    hipLaunchKernelGGL(moe_up_kernel<false>, up, block, 0, s, (const bf16_t*)x, (const bf16_t*)w_up, dense, (bf16_t*)a, M, experts, rows, K, kind);
-  hipLaunchKernelGGL(moe_down_kernel, dim3(N / 16, parts), block, 0, s, (const bf16_t*)a, (const bf16_t*)w_down, dense, y, M, experts, ff, N, accumulate,
+    hipLaunchKernelGGL((deep ? moe_up_kernel<false, 2> : moe_up_kernel<false, 1>), up, block, 0, s, (const bf16_t*)x, (const bf16_t*)w_up, dense, (bf16_t*)a, M, experts, rows, K, kind);
+  const bool deep_down = dg_deep(M, ff / parts, N / 16 * parts) && ff / parts % (DG_WAVES * 128) == 0;
+  hipLaunchKernelGGL(deep_down ? moe_down_kernel<2> : moe_down_kernel<1>, dim3(N / 16, parts), block, 0, s, (const bf16_t*)a, (const bf16_t*)w_down, dense, y, M, experts, ff, N, accumulate,
                      (const bf16_t*)w_shared, (const bf16_t*)a_shared, gate, size);
   TP_CHECK_LAUNCH("moe_few");
   return 0;

@@ -749,3 +749,33 @@ def test_moe_linear_of_any_routing(counts, output):
             we = ops.tile_weight(w[e * n: (e + 1) * n].contiguous())
             one = ops.moe_linear(x[a:b], we, torch.tensor([0, b - a], dtype=torch.int32, device=DEV), 1, output)
             assert torch.equal(got[a:b], one)
+
+
+@pytest.mark.parametrize("k,n", [(4096, 4128), (4096, 4096), (4032, 4128), (4160, 4128), (8192, 4128)])
+def test_one_and_two_rows_with_two_runs_on_their_way(k, n):
+    """Products in groups, that close a sublayer over four copies, and of routed experts: one and two rows, long K and more blocks than CUs, and sizes
+    beside these, have the bits that they have among three rows (whose products are within k * 2^-24 of the sum of their magnitudes)."""
+    from tempura_amd.kernels import ops
+    g = torch.Generator().manual_seed(k + n)
+    draw = lambda *s: (torch.randn(*s, generator=g) * k ** -0.5).to(torch.bfloat16).to(DEV)
+    plain, experts = draw(n, k), 3
+    w = ops.tile_weight(plain)
+    w_up, w_down = ops.tile_weight(draw(experts * 2 * k, 1024)), ops.tile_weight(draw(experts * n, k))
+    w_up_long, w_down_short = ops.tile_weight(draw(experts * 2816, k)), ops.tile_weight(draw(experts * 64, 1408))
+    rows, inner = draw(3, k), draw(3, 1024)
+    h = torch.randn(3, 4 * n, generator=g).to(DEV)
+    mix, coef, nw = torch.randn(4, 4, generator=g).to(DEV), torch.randn(4, generator=g).to(DEV), torch.ones(n, device=DEV)
+    dense = torch.tensor([[0.3, 0.0, 0.7], [0.0, 1.0, 0.0], [0.5, 0.5, 0.0]], device=DEV)
+
+    def results(m):
+        x, y, d, copies = ops.block_rows(rows[:m].contiguous()), ops.block_rows(inner[:m].contiguous()), dense[:m].contiguous(), h[:m].clone()
+        out = [ops.group_linear(torch.stack([x.data, x.data]), w, [16, n])]
+        handed = ops.linear(x, w, torch.float32, residual=ops.StreamClose(copies, 4, mix, coef, (coef, nw, 1e-6)))
+        out += [copies, handed.rows(), handed.ss.t()]
+        return out + [ops.moe_few(y, w_up, w_down, d, k, None), ops.moe_few(x, w_up_long, w_down_short, d, 1408, None)]
+    want = results(3)
+    ref, mag = rows.double() @ plain.double().T, rows.double().abs() @ plain.double().abs().T
+    assert bool(((want[0].double() - ref).abs() <= k * 2.0 ** -24 * mag).all())
+    for m in (1, 2):
+        for got, all_rows in zip(results(m), want):
+            assert torch.equal(got, all_rows[:m])

@@ -64,8 +64,8 @@ __device__ inline f32x4_t dg_tile(const u32x4_t* wp, const u32x4_t* xp, int xste
 // block that comes to its end leaves a CU with one run a wave (more rows' own loads fill that, and with up to one block a CU the second run's place costs
 // more than it gives).  One run / two, one row and two, us: four copies' closing product 13,824 x 5,120 32.5 / 31.2 and 32.5 / 31.2, 14,336 x 8,192 40.6 / 39.4 and 40.4 / 39.3,
 // 28,672 x 8,192 77.4 / 74.6 and 76.8 / 74.7 (four rows 74.9 / 74.8), but 14,336 x 4,096 21.7 / 21.9 and 21.5 / 21.9, 8,192 x 2,048 11.3 / 11.5; groups 14,336 x
-// 8,192 39.3 / 38.5, 4,096 x 8,192 13.2 / 13.1, but 2,048 x 4,096 4.9 / 5.0; experts, choice of two of eight, width 4,096 with 3,584 38.2 / 37.0 and 63.5 / 61.5, 6,144
-// with 16,384 205 / 197 and 390 / 374, 8,192 with 4,096 72.1 / 70.0 and 133.8 / 127.7, but width 2,048 with 1,408 (six of 64) 35.8 / 37.6 and 54.1 / 57.4.
+// 8,192 39.3 / 38.5, 4,096 x 8,192 13.2 / 13.1, but 2,048 x 4,096 4.9 / 5.0; experts, choice of two of eight, width 4,096 with 3,584 38.2 / 37.9 and 63.5 / 62.7, 6,144
+// with 16,384 205 / 200 and 390 / 381, 8,192 with 4,096 72.1 / 71.1 and 133.8 / 129.0, but width 2,048 with 1,408 (six of 64) 35.8 / 37.6 and 54.1 / 57.4.
 static bool dg_deep(int M, int K, int blocks) { return M <= 2 && K >= 4096 && blocks > 256; }
 
 // the waves' sums of element q (lane q / 4, register q % 4) in wave order

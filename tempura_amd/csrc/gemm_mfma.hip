@@ -317,27 +317,56 @@ __global__ __launch_bounds__(FEW_WAVES * 64) void gemm_few_kernel(const bf16_t* 
   } else {
     if (wave < runs) multiply(0, wave);
   }
+  int run = wave + (DEEP ? 2 : 1) * FEW_WAVES;
   if constexpr (PRE) {
     // The order is part of the result: 32 sums of every 32nd partial sum, then these in ascending order.  (The same time as a sum in pairs: one row of the
     // 3B shape 1,462.1 and 1,461.5 us, eight of the 8B shape 3,262 and 3,269.  What costs is asking for the partial sums in front of the weights, 1,476,
-    // and this work in waves that have no row, 1,489.)
+    // and this work in waves that have no row, 1,489.)  Those behind the first 256, of a K of more than 4,096, are asked for with a run of weights each 256, which
+    // every wave has (asked for one after the other / so: K x N 8,192 x 3,072 one row 14.2 / 11.1 us, nine 16.1 / 12.8, 14,336 x 4,096 26.9 / 20.8 and 29.5 / 22.1,
+    // 8,192 x 28,672 76.6 / 70.7 and 74.8 / 70.7, 28,672 x 8,192 76.7 / 72.1 and 85.2 / 73.3; 6,144 x 6,144 16.1 / 14.9, but three rows 16.2 / 16.8).
+    float sums[2] = {0.f, 0.f};
+    auto add_parts = [&](int c0) __attribute__((always_inline)) {
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        if (wave + 8 * i >= M) break;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const LanePair both = lanes_32(c0 + lane + 64 * j < pre.count ? parts[i][j] : 0.f);
+          sums[i] += both.a;
+          sums[i] += both.b;
+        }
+      }
+    };
+    auto request_parts = [&](int c0) __attribute__((always_inline)) {
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) parts[i][j] = pre.ss[min(wave + 8 * i, M - 1) * pre.count + min(c0 + lane + 64 * j, pre.count - 1)];
+    };
+    add_parts(0);
+    if (wave < M) {
+      int c0 = 256;
+      for (; P >= 0 && c0 < pre.count && run < runs; c0 += 256, run += FEW_WAVES) {
+        request(0, run);
+        request_parts(c0);
+        __builtin_amdgcn_sched_barrier(0);
+        multiply(0, run);
+        add_parts(c0);
+      }
+      for (; c0 < pre.count; c0 += 256) {
+        request_parts(c0);
+        add_parts(c0);
+      }
+    }
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
       if (wave + 8 * i >= M) break;
-      float sum = 0.f, total = 0.f;
+      float total = 0.f;
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const LanePair both = lanes_32(lane + 64 * j < pre.count ? parts[i][j] : 0.f);
-        sum += both.a;
-        sum += both.b;
-      }
-      for (int c = (lane & 31) + 256; c < pre.count; c += 32) sum += pre.ss[(wave + 8 * i) * pre.count + c];
-#pragma unroll
-      for (int c = 0; c < 32; ++c) total += lane_value(sum, c);
+      for (int c = 0; c < 32; ++c) total += lane_value(sums[i], c);
       if (lane == 0) rstd[wave + 8 * i] = rsqrtf(total * pre.inv_k + pre.eps);
     }
   }
-  int run = wave + (DEEP ? 2 : 1) * FEW_WAVES;
   if constexpr (DEEP) {
     for (; run + FEW_WAVES < runs; run += 2 * FEW_WAVES) {
       request(0, run);
